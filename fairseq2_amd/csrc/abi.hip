@@ -190,9 +190,8 @@ int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_
   if (T == 0) return FS2MOE_OK;
 
   // rows are read through the permutation where the expert kernels can (see fs2moe_grouped_swiglu)
-  const int64_t widest = (int64_t)FS2MOE_MAX_ROWS(T, K, E, tile_m) * (D > F ? D : F) * 2;
-  const bool fused = !scale_input && fs2moe_grouped_swiglu_fuses_gather(D, F, act_dtype, w_dtype) &&
-                     (w_dtype == FS2MOE_FP8_E4M3 || widest <= 0xffffffffll);
+  const bool fused = !scale_input && fs2moe::swiglu_gathers_rows(act_dtype, w_dtype, D, F,
+                                                                 FS2MOE_MAX_ROWS(T, K, E, tile_m));
   if (act_q) {
     FS2_REQUIRE(w_dtype == FS2MOE_FP8_E4M3 && act_dtype == FS2MOE_BF16 && s_gate && s_up && s_down,
                 "forward: FS2MOE_ACT_MXFP8 goes with e4m3 weights, their scales and bf16 rows");

@@ -220,6 +220,8 @@ int dispatch_with_row_weights(const int32_t* topk_idx, const float* topk_w, int3
                               int32_t E, int32_t tile_m, int64_t max_rows, int32_t* counts,
                               int32_t* offsets, int32_t* perm, int32_t* inv_perm, float* row_w,
                               void* stream);
+// Whether the grouped SwiGLU pair of these sizes reads its rows through a row map (no gathered copy).
+bool swiglu_gathers_rows(int32_t act_dtype, int32_t w_dtype, int32_t D, int32_t F, int64_t max_rows);
 // Whether the grouped SwiGLU pair of these sizes runs on the kernels that stream the weights past a
 // few staged rows (at most rows_per_expert of any expert), which can scale each row by row_w as
 // they stage it; and that pair: fs2moe_grouped_swiglu_rows with rows read through row_map and

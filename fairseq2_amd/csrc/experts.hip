@@ -26,7 +26,8 @@
 
 namespace fs2moe {
 
-// ------------------------------------------------------------------------------------ bf16, 128-row tiles (any D, F multiple of 8)
+// ------------------------------------------------------------------ bf16, 128-row tiles (64-bit addresses)
+// For activation matrices of 4 GB and more, which the throughput kernel's 32-bit offsets do not reach.
 namespace bf16k {
 constexpr int BM = 128, BN = 128, BK = 64;
 constexpr int LDA = BK + 8;    // sA row stride (elements): 144 B, conflict-free 16-byte reads
@@ -324,71 +325,77 @@ static int cu_count_by_xcd() {
 #endif
 constexpr int64_t kFp8GemmMinRowsPerExpert = FS2MOE_FP8_GEMM_MIN_ROWS;
 
-static bool dma_path_applies(int act_dtype, int D, int F) {
+// The bf16 throughput kernel takes any D and F that are multiples of 8 (its KTAIL variants where a K is
+// not a multiple of the unit's 64).  The entry points that exist for whole units only (the fused
+// gather of the stage calls, the kept products, the two-source product) say so with this.
+static bool whole_units(int act_dtype, int D, int F) {
   return act_dtype == FS2MOE_BF16 && D % (2 * dma::BK) == 0 && F % (2 * dma::BK) == 0;
 }
 
-// The bf16 throughput kernel pair (gate/up, then down) on persistent blocks; BLAYOUT as the kernel
-// takes it, scales only with dma::W_FP8_TILED.  The caller has checked that the path applies.
+// One launch of the bf16 throughput kernel on persistent blocks, one per CU (the 128 KB ring allows no
+// more), a multiple of the 8 XCDs.  `b1`, `s0` and `s1` as the kernel's variants take them.
+template <bool DUAL, int BLAYOUT, bool KEEP_GU = false, bool TWO_SRC = false>
+static int launch_dma(const void* a, const int32_t* row_map, int K, const void* b0, const void* b1,
+                      const void* s0, const void* s1, void* c, int N, const Groups& g,
+                      int64_t rows_bound, const char* what, hipStream_t stream) {
+  using namespace dma;
+  constexpr bool CAN_TAIL = BLAYOUT != W_FP8_TILED;
+  auto whole = glu_gemm_bf16_dma_kernel<DUAL, BLAYOUT, KEEP_GU, TWO_SRC>;
+  auto tail = glu_gemm_bf16_dma_kernel<DUAL, BLAYOUT, KEEP_GU, TWO_SRC, CAN_TAIL>;
+  static bool attr_set = false;  // benign race: setting the attribute is idempotent
+  if (!attr_set) {
+    for (const void* k : {reinterpret_cast<const void*>(whole), reinterpret_cast<const void*>(tail)}) {
+      hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_BYTES);
+      if (e != hipSuccess) {
+        set_error("%s: cannot reserve %d bytes of LDS: %s", what, SMEM_BYTES, hipGetErrorString(e));
+        return FS2MOE_ERR_LAUNCH;
+      }
+    }
+    attr_set = true;
+  }
+  const int num_blocks = cu_count_by_xcd();
+  if (num_blocks == 0) {
+    set_error("%s: cannot query the compute-unit count", what);
+    return FS2MOE_ERR_LAUNCH;
+  }
+  const int groups = g.counts ? g.E : 0;
+  const int nt = (N + (DUAL ? 127 : 255)) / (DUAL ? 128 : 256);
+  if ((rows_bound / BM + groups + 1) * nt > 0x7fffffffll) {
+    set_error("%s: too many tiles", what);
+    return FS2MOE_ERR_UNSUPPORTED;
+  }
+  hipLaunchKernelGGL(K % (2 * BK) == 0 ? whole : tail, dim3((unsigned)num_blocks), dim3(NWAVES * 64),
+                     SMEM_BYTES, stream, static_cast<const uint16_t*>(a), row_map, K,
+                     static_cast<const uint16_t*>(b0), static_cast<const uint16_t*>(b1),
+                     static_cast<const float*>(s0), static_cast<const float*>(s1),
+                     static_cast<uint16_t*>(c), N, K, N, g, nt);
+  return check_launch(what);
+}
+
+// The bf16 throughput kernel pair (gate/up, then down); BLAYOUT as the kernel takes it, scales only
+// with dma::W_FP8_TILED.  With g_keep and u_keep the gate/up kernel also stores the two products (their
+// destinations travel in the two scale arguments).
 template <int BLAYOUT>
 static int launch_dma_pair(const void* x, const int32_t* row_map, const Groups& g,
                            int64_t rows_bound, const void* w_gate, const void* w_up,
                            const void* w_down, const float* s_gate, const float* s_up,
                            const float* s_down, int D, int F, void* h, void* y,
                            hipStream_t stream, void* g_keep = nullptr, void* u_keep = nullptr) {
-  using namespace dma;
-  const int groups = g.counts ? g.E : 0;
-  // the gate/up kernel, or its variant that also stores the two products (plain bf16 weights only)
   constexpr bool CAN_KEEP = BLAYOUT != dma::W_FP8_TILED;
-  auto k1 = glu_gemm_bf16_dma_kernel<true, BLAYOUT>;
-  auto k1k = glu_gemm_bf16_dma_kernel<true, BLAYOUT, CAN_KEEP>;
-  auto k2 = glu_gemm_bf16_dma_kernel<false, BLAYOUT>;
   if (g_keep != nullptr && !CAN_KEEP) {
     set_error("experts: the products are kept with bf16 weights only");
     return FS2MOE_ERR_UNSUPPORTED;
   }
-  static bool attr_set = false;  // benign race: setting the attribute is idempotent
-  if (!attr_set) {
-    const void* ks[3] = {reinterpret_cast<const void*>(k1), reinterpret_cast<const void*>(k1k),
-                         reinterpret_cast<const void*>(k2)};
-    for (const void* k : ks) {
-      hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_BYTES);
-      if (e != hipSuccess) {
-        set_error("experts: cannot reserve %d bytes of LDS: %s", SMEM_BYTES, hipGetErrorString(e));
-        return FS2MOE_ERR_LAUNCH;
-      }
-    }
-    attr_set = true;
-  }
-  // Persistent blocks: one per CU (the 128 KB ring allows no more), a multiple of the 8 XCDs.
-  const int num_blocks = cu_count_by_xcd();
-  if (num_blocks == 0) {
-    set_error("experts: cannot query the compute-unit count");
-    return FS2MOE_ERR_LAUNCH;
-  }
-  const int nt1 = (F + 127) / 128, nt2 = (D + 255) / 256;
-  {
-    const int64_t m_tiles = rows_bound / BM + groups + 1;
-    if (m_tiles * nt1 > 0x7fffffffll || m_tiles * nt2 > 0x7fffffffll) {
-      set_error("experts: too many tiles");
-      return FS2MOE_ERR_UNSUPPORTED;
-    }
-  }
-  const unsigned g1 = (unsigned)num_blocks, g2 = (unsigned)num_blocks;
-  // (the variant that keeps the products takes their destinations in the two scale arguments)
-  hipLaunchKernelGGL(g_keep != nullptr ? k1k : k1, dim3(g1), dim3(NWAVES * 64), SMEM_BYTES, stream,
-                     static_cast<const uint16_t*>(x), row_map, D,
-                     static_cast<const uint16_t*>(w_gate), static_cast<const uint16_t*>(w_up),
-                     g_keep != nullptr ? static_cast<const float*>(g_keep) : s_gate,
-                     g_keep != nullptr ? static_cast<const float*>(u_keep) : s_up,
-                     static_cast<uint16_t*>(h), F, D, F, g, nt1);
-  if (int rc = check_launch("glu_gemm_bf16_dma<gate,up>")) return rc;
-  hipLaunchKernelGGL(k2, dim3(g2), dim3(NWAVES * 64), SMEM_BYTES, stream,
-                     static_cast<const uint16_t*>(h), static_cast<const int32_t*>(nullptr), F,
-                     static_cast<const uint16_t*>(w_down), static_cast<const uint16_t*>(nullptr),
-                     s_down, static_cast<const float*>(nullptr), static_cast<uint16_t*>(y), D, F, D, g,
-                     nt2);
-  return check_launch("glu_gemm_bf16_dma<down>");
+  int rc;
+  if (g_keep != nullptr)
+    rc = launch_dma<true, BLAYOUT, CAN_KEEP>(x, row_map, D, w_gate, w_up, g_keep, u_keep, h, F, g,
+                                             rows_bound, "glu_gemm_bf16_dma<gate,up>", stream);
+  else
+    rc = launch_dma<true, BLAYOUT>(x, row_map, D, w_gate, w_up, s_gate, s_up, h, F, g, rows_bound,
+                                   "glu_gemm_bf16_dma<gate,up>", stream);
+  if (rc) return rc;
+  return launch_dma<false, BLAYOUT>(h, nullptr, F, w_down, nullptr, s_down, nullptr, y, D, g, rows_bound,
+                                    "glu_gemm_bf16_dma<down>", stream);
 }
 
 // The throughput kernel addresses activations and one expert's weights with 32-bit byte offsets.
@@ -551,12 +558,11 @@ static int launch_glu(const void* x, const int32_t* row_map, const Groups& g, in
     set_error("experts: internal: row weights given to kernels that do not scale rows");
     return FS2MOE_ERR_UNSUPPORTED;
   }
-  if (dma_path_applies(act_dtype, D, F) && dma_offsets_fit(rows_bound, D, F))
+  if (act_dtype == FS2MOE_BF16 && dma_offsets_fit(rows_bound, D, F))
     return launch_dma_pair<BLAYOUT>(x, row_map, g, rows_bound, w_gate, w_up, w_down, nullptr, nullptr,
                                     nullptr, D, F, h, y, stream);
   if (row_map != nullptr) {
-    set_error("experts: the fused gather needs bf16, D and F multiples of 64 and activation "
-              "matrices below 4 GB");
+    set_error("experts: the fused gather needs bf16 and activation matrices below 4 GB");
     return FS2MOE_ERR_UNSUPPORTED;
   }
   if (act_dtype == FS2MOE_BF16) {
@@ -605,13 +611,13 @@ extern "C" int fs2moe_grouped_swiglu_fuses_gather(int32_t D, int32_t F, int32_t 
                                                   int32_t w_dtype) {
   if (D <= 0 || F <= 0) return 0;
   if (w_dtype == FS2MOE_FP8_E4M3) return (act_dtype == FS2MOE_BF16 && D % 64 == 0 && F % 64 == 0) ? 1 : 0;
-  return (w_dtype == act_dtype && dma_path_applies(act_dtype, D, F)) ? 1 : 0;
+  return (w_dtype == act_dtype && whole_units(act_dtype, D, F)) ? 1 : 0;
 }
 
 extern "C" int fs2moe_grouped_swiglu_keeps(int32_t D, int32_t F, int64_t max_rows,
                                            int32_t act_dtype) {
   if (D <= 0 || F <= 0 || max_rows < 0) return 0;
-  return (dma_path_applies(act_dtype, D, F) && dma_offsets_fit(max_rows, D, F)) ? 1 : 0;
+  return (whole_units(act_dtype, D, F) && dma_offsets_fit(max_rows, D, F)) ? 1 : 0;
 }
 
 extern "C" int fs2moe_grouped_swiglu_keep(const void* xe, const int32_t* row_map,
@@ -744,6 +750,13 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
                                      h, ye, static_cast<hipStream_t>(stream), rows_hint, row_w);
 }
 
+bool fs2moe::swiglu_gathers_rows(int32_t act_dtype, int32_t w_dtype, int32_t D, int32_t F,
+                                 int64_t max_rows) {
+  if (act_dtype != FS2MOE_BF16 || D < 8 || F < 8 || D % 8 || F % 8) return false;
+  if (w_dtype == FS2MOE_FP8_E4M3) return D % 64 == 0 && F % 64 == 0;
+  return w_dtype == FS2MOE_BF16 && dma_offsets_fit(max_rows, D, F);
+}
+
 bool fs2moe::swiglu_streams_rows(int32_t act_dtype, int32_t w_dtype, int32_t D, int32_t F, int32_t E,
                                  int32_t rows_per_expert) {
   if (act_dtype != FS2MOE_BF16 || w_dtype != FS2MOE_BF16 || D < 8 || F < 8 || D % 8 || F % 8) return false;
@@ -792,37 +805,11 @@ template <int BLAYOUT>
 static int launch_gemm(const void* a, const int32_t* row_map, const Groups& g, int64_t rows_bound,
                        const void* b, int K, int N, int dtype, void* c, hipStream_t stream) {
   const int groups = g.counts ? g.E : 0;
-  if (dtype == FS2MOE_BF16 && K % (2 * dma::BK) == 0 && dma_offsets_fit(rows_bound, K, N)) {
-    using namespace dma;
-    auto k = glu_gemm_bf16_dma_kernel<false, BLAYOUT>;
-    static bool attr_set = false;  // benign race: setting the attribute is idempotent
-    if (!attr_set) {
-      hipError_t e1 = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_BYTES);
-      if (e1 != hipSuccess) {
-        set_error("gemm: cannot reserve %d bytes of LDS: %s", SMEM_BYTES, hipGetErrorString(e1));
-        return FS2MOE_ERR_LAUNCH;
-      }
-      attr_set = true;
-    }
-    const int num_blocks = cu_count_by_xcd();
-    if (num_blocks == 0) {
-      set_error("gemm: cannot query the compute-unit count");
-      return FS2MOE_ERR_LAUNCH;
-    }
-    const int nt = (N + 255) / 256;
-    if ((rows_bound / BM + groups + 1) * nt > 0x7fffffffll) {
-      set_error("gemm: too many tiles");
-      return FS2MOE_ERR_UNSUPPORTED;
-    }
-    hipLaunchKernelGGL(k, dim3((unsigned)num_blocks), dim3(NWAVES * 64), SMEM_BYTES, stream,
-                       static_cast<const uint16_t*>(a), row_map, K, static_cast<const uint16_t*>(b),
-                       static_cast<const uint16_t*>(nullptr), static_cast<const float*>(nullptr),
-                       static_cast<const float*>(nullptr), static_cast<uint16_t*>(c), N, K, N, g, nt);
-    return check_launch("glu_gemm_bf16_dma<single>");
-  }
+  if (dtype == FS2MOE_BF16 && dma_offsets_fit(rows_bound, K, N))
+    return launch_dma<false, BLAYOUT>(a, row_map, K, b, nullptr, nullptr, nullptr, c, N, g, rows_bound,
+                                      "glu_gemm_bf16_dma<single>", stream);
   if (row_map != nullptr) {
-    set_error("gemm: a row map needs bf16, K a multiple of 64 and matrices below 4 GB");
+    set_error("gemm: a row map needs bf16 and matrices below 4 GB");
     return FS2MOE_ERR_UNSUPPORTED;
   }
   if (dtype == FS2MOE_BF16) {
@@ -924,38 +911,10 @@ extern "C" int fs2moe_grouped_gemm_sum(const void* a1, const void* b1, const voi
   FS2_REQUIRE(aligned16(a1) && aligned16(b1) && aligned16(a2) && aligned16(b2) && aligned16(c),
               "grouped_gemm_sum: buffers must be 16-byte aligned");
   if (max_rows == 0) return FS2MOE_OK;
-  using namespace dma;
-  Groups g{counts, offsets, E, (int)max_rows};
-  auto k = glu_gemm_bf16_dma_kernel<false, FS2MOE_W_OUT_IN, false, true>;
-  static bool attr_set = false;  // benign race: setting the attribute is idempotent
-  if (!attr_set) {
-    hipError_t e1 = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_BYTES);
-    if (e1 != hipSuccess) {
-      set_error("grouped_gemm_sum: cannot reserve %d bytes of LDS: %s", SMEM_BYTES,
-                hipGetErrorString(e1));
-      return FS2MOE_ERR_LAUNCH;
-    }
-    attr_set = true;
-  }
-  const int num_blocks = cu_count_by_xcd();
-  if (num_blocks == 0) {
-    set_error("grouped_gemm_sum: cannot query the compute-unit count");
-    return FS2MOE_ERR_LAUNCH;
-  }
-  const int groups = counts ? E : 0;
-  const int nt = (N + 255) / 256;
-  if ((max_rows / BM + groups + 1) * nt > 0x7fffffffll) {
-    set_error("grouped_gemm_sum: too many tiles");
-    return FS2MOE_ERR_UNSUPPORTED;
-  }
   // (the second activation matrix travels in the first scale argument, the second weights in B1)
-  hipLaunchKernelGGL(k, dim3((unsigned)num_blocks), dim3(NWAVES * 64), SMEM_BYTES,
-                     static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(a1),
-                     static_cast<const int32_t*>(nullptr), K, static_cast<const uint16_t*>(b1),
-                     static_cast<const uint16_t*>(b2), static_cast<const float*>(a2),
-                     static_cast<const float*>(nullptr), static_cast<uint16_t*>(c), N, K, N, g, nt);
-  return check_launch("glu_gemm_bf16_dma<two sources>");
+  return launch_dma<false, FS2MOE_W_OUT_IN, false, true>(
+      a1, nullptr, K, b1, b2, a2, nullptr, c, N, Groups{counts, offsets, E, (int)max_rows}, max_rows,
+      "glu_gemm_bf16_dma<two sources>", static_cast<hipStream_t>(stream));
 }
 
 extern "C" int fs2moe_dense_swiglu(const void* x, const void* w_gate, const void* w_up,

@@ -130,7 +130,14 @@ struct TileOrder {
 // TWO_SRC (single matrix, (out, in) bf16 weights): C = A @ B0_e^T + A2 @ B1_e^T, the second pair
 // walked after the first into the same accumulators (Kdim is one pair's).  A2 arrives in S0, for the
 // reason given above.
-template <bool DUAL, int BLAYOUT, bool KEEP_GU = false, bool TWO_SRC = false>
+// KTAIL (bf16 weights): Kdim is a multiple of 8 but not of the unit's 64.  A tile's last unit then
+// ends inside its 64 k: the producers load zeros for the 16-byte pieces past Kdim, of both operands,
+// since what lies there may be anything.  Variants of their own, so that the kernels for whole units
+// compile to what they were.  Against the 128-row kernel that such sizes took before (its blocks wait
+// for every k-step's loads) and the gathered copy it needed: D 1088, F 1392, 8 experts, 8364 rows, whole
+// layer 179 -> 134 us; D 1664, F 1312, 32 experts and a shared one, 7092 rows 339 -> 275 us; the bits
+// are the same.
+template <bool DUAL, int BLAYOUT, bool KEEP_GU = false, bool TWO_SRC = false, bool KTAIL = false>
 __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
     const uint16_t* __restrict__ A, const int32_t* __restrict__ row_map, int lda,
     const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1,
@@ -139,6 +146,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
   using namespace dma;
   constexpr bool FP8 = BLAYOUT == W_FP8_TILED;
   static_assert(!KEEP_GU || (DUAL && !FP8), "the products are kept by the bf16 gate/up kernel only");
+  static_assert(!KTAIL || !FP8, "e4m3 weight tiles hold whole units");
   static_assert(!TWO_SRC || (!DUAL && BLAYOUT == FS2MOE_W_OUT_IN), "two sources: one (out, in) matrix each");
   constexpr int BN = DUAL ? 128 : 256;    // real channels per tile
   constexpr int BROW = DUAL ? 256 : 512;  // bytes per LDS row of a weight sub-tile (in x out)
@@ -228,8 +236,8 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
   // of which heavy: the block's j-th tile (in list order) is heavy for j < my_heavy
   const int my_heavy = slot < heavy_end ? (heavy_end - slot + grid - 1) / grid : 0;
 
-  // units per tile; the host guarantees Kdim % 64 == 0
-  const int nu = (TWO_SRC ? 2 : 1) * (Kdim / (2 * BK));
+  // units per tile; without KTAIL the host guarantees Kdim % 64 == 0
+  const int nu = (TWO_SRC ? 2 : 1) * ((Kdim + (KTAIL ? 2 * BK - 1 : 0)) / (2 * BK));
   const int total_units = my_tiles * nu;
 
   // Wave-uniform parameters of a tile: expert, first row, end row, first channel.
@@ -398,6 +406,29 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
     int stage_pieces = 0;  // a_pieces of the unit held in `stage`
     int stage_scale_slot = -1;  // e4m3: the unit in `stage` is the first of a tile with this slot
     float stage_scale = 0.f;
+    // KTAIL: the piece at base + off, or zeros where it lies past Kdim: a buffer load, whose range check
+    // turns an offset outside the buffer into zeros (one select per piece, and no branch around the
+    // loads).  In the activation block and in (out, in) weights every piece of a lane holds the same
+    // chunk of its row's 128 bytes (the swizzle key of row 8 (q + 4 jj) + lane / 8 does not depend on
+    // jj), k from 8 tail_kc on; in (in, out) weights a piece lies in one k row, tail_row(i) of the
+    // sub-stage for piece register i.
+    const int tail_kc = (lane & 7) ^ ((4 * q + (lane >> 4)) & 7);
+    auto tail_row = [&](int i) {
+      constexpr int ROWS = 1024 / BROW, CHUNKS = BROW / 16;
+      const int p = q + 4 * i;
+      return ROWS * (DUAL ? (p & 7) : p) + lane / CHUNKS;
+    };
+    auto piece = [&](bool in_k, const uint8_t* base, uint32_t off) -> u32x4 {
+      if constexpr (KTAIL) {
+        // (the host keeps every valid offset below 2^32 - 16)
+        const __amdgpu_buffer_rsrc_t rsrc =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), 0, 0xfffffff0u, 0x00020000);
+        return __builtin_amdgcn_raw_buffer_load_b128(rsrc, in_k ? off : 0xfffffff0u, 0, 0);
+      } else {
+        return *reinterpret_cast<const u32x4*>(base + off);
+      }
+    };
+    auto k_left = [&](int ku) { return Kdim - ku * (2 * BK); };  // k of unit ku and those after it
     // Unit ku of the tile set up last -> registers.
     auto load_unit = [&](int ku) {
       // with two sources the second half of a tile's units comes from the second pair
@@ -405,9 +436,11 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
       if constexpr (TWO_SRC) ku = second ? ku - nu / 2 : ku;
       const uint16_t* a_src = second ? reinterpret_cast<const uint16_t*>(S0) : A;
       const uint8_t* abase = reinterpret_cast<const uint8_t*>(a_src + (size_t)ku * (2 * BK));
+      const int left = k_left(ku);
+      const bool kc_ok = tail_kc * 8 < left;
 #pragma unroll
       for (int jj = 0; jj < 8; ++jj)
-        if (jj < a_pieces) stage[jj] = *reinterpret_cast<const u32x4*>(abase + pa[jj]);
+        if (jj < a_pieces) stage[jj] = piece(kc_ok, abase, pa[jj]);
       if constexpr (FP8) {
         const uint8_t* bg = reinterpret_cast<const uint8_t*>(ld_bg) + (size_t)ku * 1024;
         const uint8_t* bu = reinterpret_cast<const uint8_t*>(ld_bu) + (size_t)ku * 1024;
@@ -423,10 +456,9 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
           const uint8_t* bg = reinterpret_cast<const uint8_t*>(ld_bg + k0);
           const uint8_t* bu = reinterpret_cast<const uint8_t*>(ld_bu + k0);
           // pieces q, q+4 (gate when DUAL) and q+8, q+12 (up when DUAL)
-          stage[8 + 4 * h + 0] = *reinterpret_cast<const u32x4*>(bg + pb[0]);
-          stage[8 + 4 * h + 1] = *reinterpret_cast<const u32x4*>(bg + pb[1]);
-          stage[8 + 4 * h + 2] = *reinterpret_cast<const u32x4*>(bu + pb[2]);
-          stage[8 + 4 * h + 3] = *reinterpret_cast<const u32x4*>(bu + pb[3]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            stage[8 + 4 * h + i] = piece(h * BK + tail_row(i) < left, i < 2 ? bg : bu, pb[i]);
         }
       } else {
         const uint8_t* bg =
@@ -435,8 +467,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
             TWO_SRC ? bg : reinterpret_cast<const uint8_t*>(ld_bu + (size_t)ku * (2 * BK));
         // pieces q + 4 jj: jj < 4 lie in rows 0..127 (gate when DUAL), the rest in rows 128..255
 #pragma unroll
-        for (int jj = 0; jj < 8; ++jj)
-          stage[8 + jj] = *reinterpret_cast<const u32x4*>((jj < 4 ? bg : bu) + pb[jj]);
+        for (int jj = 0; jj < 8; ++jj) stage[8 + jj] = piece(kc_ok, jj < 4 ? bg : bu, pb[jj]);
       }
       stage_pieces = a_pieces;
     };
@@ -510,11 +541,13 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
         if constexpr (TWO_SRC) ku = second ? ku - nu / 2 : ku;
         const uint16_t* a_src = second ? reinterpret_cast<const uint16_t*>(S0) : A;
         const uint8_t* abase = reinterpret_cast<const uint8_t*>(a_src + (size_t)ku * (2 * BK));
+        const int left = k_left(ku);
+        const bool kc_ok = tail_kc * 8 < left;
         uint8_t* dst = smem_raw + half * UNIT_BYTES + q * 1024 + lane * 16;
 #pragma unroll
         for (int jj = 0; jj < 8; ++jj) {
           if (jj < stage_pieces) *reinterpret_cast<u32x4*>(dst + jj * 4096) = stage[jj];
-          if (jj < a_pieces) stage[jj] = *reinterpret_cast<const u32x4*>(abase + pa[jj]);
+          if (jj < a_pieces) stage[jj] = piece(kc_ok, abase, pa[jj]);
         }
         if constexpr (KN) {
 #pragma unroll
@@ -525,7 +558,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               *reinterpret_cast<u32x4*>(dst + A_BYTES + (4 * h + i) * 4096) = stage[8 + 4 * h + i];
-              stage[8 + 4 * h + i] = *reinterpret_cast<const u32x4*>((i < 2 ? bg : bu) + pb[i]);
+              stage[8 + 4 * h + i] = piece(h * BK + tail_row(i) < left, i < 2 ? bg : bu, pb[i]);
             }
           }
         } else {
@@ -536,7 +569,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
 #pragma unroll
           for (int jj = 0; jj < 8; ++jj) {
             *reinterpret_cast<u32x4*>(dst + A_BYTES + jj * 4096) = stage[8 + jj];
-            stage[8 + jj] = *reinterpret_cast<const u32x4*>((jj < 4 ? bg : bu) + pb[jj]);
+            stage[8 + jj] = piece(kc_ok, jj < 4 ? bg : bu, pb[jj]);
           }
         }
         stage_pieces = a_pieces;

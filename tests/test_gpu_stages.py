@@ -552,6 +552,41 @@ def test_grouped_swiglu_fp8_row_map_equals_gathered_rows(gpu_device, t, d, e, k,
     assert torch.equal(ye_a[valid], ye_b[valid])
 
 
+# K off the throughput kernel's units of 64 (8 mod 64 up to 56 mod 64), N off its tiles of 128 and 256
+@pytest.mark.parametrize("d,f", [(8, 56), (1032, 8), (120, 184), (200, 1368), (952, 264)])
+def test_grouped_swiglu_with_a_k_tail(gpu_device, d, f):
+    """bf16 sizes that end inside a unit: every expert against the oracle, the rows through a map bit
+    for bit like the copy, and an expert full of NaN, whose weights lie right behind its neighbour's
+    last rows of k, reaches no other expert."""
+    _say("grouped_swiglu k tail", d, f)
+    rows_per_expert = [257, 0, 40, 3, 300, 128]
+    counts, offsets, xe, wg, wu, wd = _expert_case("bf16", rows_per_expert, d, f, seed=d + f)
+    e, bf, dev = len(rows_per_expert), torch.bfloat16, gpu_device
+    args = [v.to(bf).to(dev) for v in (wg, wu, wd)]
+    groups = (counts.to(dev), offsets.to(dev))
+    ye, h = _abi.grouped_swiglu(xe.to(bf).to(dev), *groups, *args, e)
+    for ex in range(e):
+        lo, n = int(offsets[ex]), int(counts[ex])
+        if n == 0:
+            continue
+        u = xe[lo : lo + n].double()
+        h_ref = torch.nn.functional.silu(u @ wg[ex * d : (ex + 1) * d].double()) * (u @ wu[ex * d : (ex + 1) * d].double())
+        assert_output_close(h[lo : lo + n], h_ref, "bf16", f"h of expert {ex}")
+        y_ref = h[lo : lo + n].double().cpu() @ wd[ex * f : (ex + 1) * f].double()
+        assert_output_close(ye[lo : lo + n], y_ref, "bf16", f"ye of expert {ex}")
+    order = torch.randperm(xe.shape[0], generator=torch.Generator().manual_seed(d))
+    scattered = torch.empty_like(xe)
+    scattered[order] = xe
+    ye_map, _ = _abi.grouped_swiglu(scattered.to(bf).to(dev), *groups, *args, e, row_map=order.to(torch.int32).to(dev))
+    for w, k in zip(args, (d, d, f)):
+        w[3 * k : 4 * k] = float("nan")
+    ye_nan, _ = _abi.grouped_swiglu(xe.to(bf).to(dev), *groups, *args, e)
+    for ex in range(e):
+        sl = slice(int(offsets[ex]), int(offsets[ex]) + int(counts[ex]))
+        assert torch.equal(ye_map[sl], ye[sl]), f"expert {ex} through the map"
+        assert ex == 3 or torch.equal(ye_nan[sl], ye[sl]), f"expert {ex} next to NaN weights"
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
 @pytest.mark.parametrize(
     "t,d,f",
