@@ -13,20 +13,21 @@
 #include <type_traits>
 
 #include "common.h"
+#include "experts_f32.h"
 #include "tile_map.h"
 
 namespace fs2moe {
 
 // ---------------------------------------------------------------------------------- weight gradient
-// C_e [M, N] = sum over the rows r of expert e of A[r, :M]^T B[r, :N].  A block owns a 256 x 256 tile
-// of one expert's gradient and walks the expert's rows RK at a time (32 for bf16, 16 for f32).  Eight
-// consumer waves multiply (a wave 128 x 64: 4 x 2 MFMA tiles); four producer waves, one per SIMD,
-// move the data: a wave that waits for memory issues nothing else, so loads issued by the waves that
-// multiply cost matrix-pipe time.  Both chunks go to LDS as they lie in memory (row = contraction
-// index, columns contiguous) and come back through the transposing LDS read (bf16) or as single
-// floats (f32), each already in MFMA operand order.  LDS holds two chunks: while one is multiplied
-// the producers write the next from registers and the two after that are on their way from memory
-// in two sets of registers, so there is one barrier per chunk, which orders LDS traffic only.
+// C_e [M, N] = sum over the rows r of expert e of A[r, :M]^T B[r, :N], bf16 (f32:
+// grouped_wgrad_f32_kernel in experts_f32.h).  A block owns a 256 x 256 tile of one expert's gradient and
+// walks the expert's rows 32 at a time.  Eight consumer waves multiply (a wave 128 x 64: 4 x 2 MFMA
+// tiles); four producer waves, one per SIMD, move the data: a wave that waits for memory issues nothing
+// else, so loads issued by the waves that multiply cost matrix-pipe time.  Both chunks go to LDS as they
+// lie in memory (row = contraction index, columns contiguous) and come back through the transposing LDS
+// read, in MFMA operand order.  LDS holds two chunks: while one is multiplied the producers write the
+// next from registers and the two after that are on their way from memory in two sets of registers, so
+// there is one barrier per chunk, which orders LDS traffic only.
 // (Chunks of twice the rows, a half per register set and one barrier per chunk, were slower: 277
 // against 244 us on 8 experts of 8192 rows.)  Rows past the expert's count are zero-filled,
 // experts without rows get a zero gradient.
@@ -40,19 +41,19 @@ __device__ __attribute__((aligned(16))) uint32_t kZero16[4] = {0u, 0u, 0u, 0u}; 
 // MAPPED: A's rows are read through a_map.  A template parameter, not a test of the pointer: behind
 // a condition the map entry's load is waited for with every other load of the wave (the counter
 // cannot tell them apart at the join), which serialises a chunk's loads into round trips.
-template <typename T, bool MAPPED>
+template <bool MAPPED>
 __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
-    const T* __restrict__ A, const int32_t* __restrict__ a_map, int lda, const T* __restrict__ B,
-    int ldb, T* __restrict__ C, int M, int N, Groups g, int m_tiles, int n_tiles, int seg_rows,
-    float* __restrict__ partial, int paired) {
+    const uint16_t* __restrict__ A, const int32_t* __restrict__ a_map, int lda,
+    const uint16_t* __restrict__ B, int ldb, uint16_t* __restrict__ C, int M, int N, Groups g,
+    int m_tiles, int n_tiles, int seg_rows, float* __restrict__ partial, int paired) {
   using namespace wgk;
-  constexpr bool BF16 = sizeof(T) == 2;
-  constexpr int RK = BF16 ? 32 : 16;              // rows per chunk
-  constexpr int VEC = 16 / sizeof(T);             // elements per 16-byte chunk
-  constexpr int ROW_CHUNKS = TM / VEC;            // 16-byte chunks per LDS row (32 or 64)
+  using T = uint16_t;
+  constexpr int RK = 32;                          // rows per chunk
+  constexpr int VEC = 8;                          // elements per 16-byte chunk
+  constexpr int ROW_CHUNKS = TM / VEC;            // 16-byte chunks per LDS row (32)
   constexpr int PLANES = PRODUCERS * 64;          // lanes that move data
   constexpr int PER_THREAD = RK * ROW_CHUNKS / PLANES;  // chunks per producer lane and operand (4)
-  constexpr int ROWB = TM * sizeof(T);            // bytes per LDS row (512 or 1024)
+  constexpr int ROWB = TM * sizeof(T);            // bytes per LDS row (512)
   constexpr int OPB = RK * ROWB;                  // bytes per operand chunk (16 KB)
   static_assert(4 * OPB == SMEM_BYTES, "two chunks of two operands");
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -177,15 +178,15 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     for (int i = 0; i < PER_THREAD; ++i) {
       const int c = ptid + PLANES * i;
       const int k = c / ROW_CHUNKS, ch = c % ROW_CHUNKS;
-      // bf16: chunk ch of row k sits in slot ch ^ ((k & 3) << 2), so that the four consecutive rows
-      // a transposing read touches lie 64 bytes apart
-      const int slot = BF16 ? (ch ^ ((k & 3) << 2)) : ch;
+      // chunk ch of row k sits in slot ch ^ ((k & 3) << 2), so that the four consecutive rows a
+      // transposing read touches lie 64 bytes apart
+      const int slot = ch ^ ((k & 3) << 2);
       *reinterpret_cast<u32x4*>(sA + k * ROWB + slot * 16) = ra[set][i];
       *reinterpret_cast<u32x4*>(sB + k * ROWB + slot * 16) = rb[set][i];
     }
   };
 
-  // bf16 fragment address of the 32 columns from cbase on, rows 8 lk .. 8 lk + 3 (+4 for the upper half)
+  // fragment address of the 32 columns from cbase on, rows 8 lk .. 8 lk + 3 (+4 for the upper half)
   auto tr_addr = [&](int cbase) {
     const int s = lane & 15, half = (lane >> 4) & 1;
     const int k = lk * 8 + (s >> 2);
@@ -195,53 +196,35 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
   int fa[4], fb[2];
 #pragma unroll
   for (int t = 0; t < 4; ++t)
-    fa[t] = BF16 ? tr_addr(wm * 128 + t * 32) : (wm * 128 + t * 32 + lr) * 4;
+    fa[t] = tr_addr(wm * 128 + t * 32);
 #pragma unroll
   for (int t = 0; t < 2; ++t)
-    fb[t] = BF16 ? tr_addr(wn * 64 + t * 32) : (wn * 64 + t * 32 + lr) * 4;
+    fb[t] = tr_addr(wn * 64 + t * 32);
 
   auto compute_chunk = [&](int buf) {
     const uint8_t* sA = smem + buf * 2 * OPB;
     const uint8_t* sB = sA + OPB;
-    if constexpr (BF16) {
 #pragma unroll
-      for (int ks = 0; ks < RK / 16; ++ks) {
-        bf16x8 af[4], bfr[2];
+    for (int ks = 0; ks < RK / 16; ++ks) {
+      bf16x8 af[4], bfr[2];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const uint8_t* pa = sA + fa[t] + ks * 16 * ROWB;
-          af[t] = lds_read_frag_tr(reinterpret_cast<const uint16_t*>(pa),
-                                   reinterpret_cast<const uint16_t*>(pa + 4 * ROWB));
-        }
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const uint8_t* pb = sB + fb[t] + ks * 16 * ROWB;
-          bfr[t] = lds_read_frag_tr(reinterpret_cast<const uint16_t*>(pb),
-                                    reinterpret_cast<const uint16_t*>(pb + 4 * ROWB));
-        }
-#pragma unroll
-        for (int tn = 0; tn < 2; ++tn)
-#pragma unroll
-          for (int tm = 0; tm < 4; ++tm)
-            acc[tn][tm] =
-                __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[tn], af[tm], acc[tn][tm], 0, 0, 0);
+      for (int t = 0; t < 4; ++t) {
+        const uint8_t* pa = sA + fa[t] + ks * 16 * ROWB;
+        af[t] = lds_read_frag_tr(reinterpret_cast<const uint16_t*>(pa),
+                                 reinterpret_cast<const uint16_t*>(pa + 4 * ROWB));
       }
-    } else {
-#pragma unroll 2
-      for (int ks = 0; ks < RK / 2; ++ks) {
-        float af[4], bfr[2];
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-          af[t] = *reinterpret_cast<const float*>(sA + (2 * ks + lk) * ROWB + fa[t]);
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-          bfr[t] = *reinterpret_cast<const float*>(sB + (2 * ks + lk) * ROWB + fb[t]);
-#pragma unroll
-        for (int tn = 0; tn < 2; ++tn)
-#pragma unroll
-          for (int tm = 0; tm < 4; ++tm)
-            acc[tn][tm] = __builtin_amdgcn_mfma_f32_32x32x2f32(bfr[tn], af[tm], acc[tn][tm], 0, 0, 0);
+      for (int t = 0; t < 2; ++t) {
+        const uint8_t* pb = sB + fb[t] + ks * 16 * ROWB;
+        bfr[t] = lds_read_frag_tr(reinterpret_cast<const uint16_t*>(pb),
+                                  reinterpret_cast<const uint16_t*>(pb + 4 * ROWB));
       }
+#pragma unroll
+      for (int tn = 0; tn < 2; ++tn)
+#pragma unroll
+        for (int tm = 0; tm < 4; ++tm)
+          acc[tn][tm] =
+              __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[tn], af[tm], acc[tn][tm], 0, 0, 0);
     }
   };
 
@@ -285,43 +268,41 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
   // fragment tn in registers 4 q .. 4 q + 3.
   T* Ce = C + (size_t)e * M * N;
   float* Pe = partial != nullptr ? partial + (size_t)slot * M * N : nullptr;
-  if constexpr (BF16) {
-    if (Pe == nullptr) {
-      // Through LDS (free after the loop's last barrier), so that a store instruction writes 8 rows
-      // of 128 contiguous bytes instead of 32 rows of 16: the wave puts a 32 (m) x 64 (n) fragment
-      // row into its own 4.25 KB as bf16, rows 136 bytes apart, and reads it back 16 bytes per lane.
-      constexpr int LDE = 136;
-      uint8_t* sw = smem + wave * 8192;
-      const int rrow = lane >> 3, rcol = lane & 7;
+  if (Pe == nullptr) {
+    // Through LDS (free after the loop's last barrier), so that a store instruction writes 8 rows
+    // of 128 contiguous bytes instead of 32 rows of 16: the wave puts a 32 (m) x 64 (n) fragment
+    // row into its own 4.25 KB as bf16, rows 136 bytes apart, and reads it back 16 bytes per lane.
+    constexpr int LDE = 136;
+    uint8_t* sw = smem + wave * 8192;
+    const int rrow = lane >> 3, rcol = lane & 7;
 #pragma unroll
-      for (int tm = 0; tm < 4; ++tm) {
+    for (int tm = 0; tm < 4; ++tm) {
 #pragma unroll
-        for (int tn = 0; tn < 2; ++tn)
+      for (int tn = 0; tn < 2; ++tn)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            u32x2 o = {pack_bf16x2(acc[tn][tm][4 * q], acc[tn][tm][4 * q + 1]),
-                       pack_bf16x2(acc[tn][tm][4 * q + 2], acc[tn][tm][4 * q + 3])};
-            *reinterpret_cast<u32x2*>(sw + lr * LDE + (tn * 32 + 8 * q + 4 * lk) * 2) = o;
-          }
-        // the wave's own LDS traffic runs in order; the compiler must not move the reads (other
-        // lanes' data) above the writes, nor the next round's writes above these reads
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        const int n = n0 + wn * 64 + rcol * 8;
-#pragma unroll
-        for (int p8 = 0; p8 < 4; ++p8) {
-          const int row = p8 * 8 + rrow;
-          const u32x2 lo = *reinterpret_cast<const u32x2*>(sw + row * LDE + rcol * 16);
-          const u32x2 hi = *reinterpret_cast<const u32x2*>(sw + row * LDE + rcol * 16 + 8);
-          const int m = m0 + wm * 128 + tm * 32 + row;
-          if (m < M && n < N) {  // N is a multiple of 8: the eight columns are in or out together
-            u32x4 o = {lo[0], lo[1], hi[0], hi[1]};
-            *reinterpret_cast<u32x4*>(Ce + (size_t)m * N + n) = o;
-          }
+        for (int q = 0; q < 4; ++q) {
+          u32x2 o = {pack_bf16x2(acc[tn][tm][4 * q], acc[tn][tm][4 * q + 1]),
+                     pack_bf16x2(acc[tn][tm][4 * q + 2], acc[tn][tm][4 * q + 3])};
+          *reinterpret_cast<u32x2*>(sw + lr * LDE + (tn * 32 + 8 * q + 4 * lk) * 2) = o;
         }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      // the wave's own LDS traffic runs in order; the compiler must not move the reads (other
+      // lanes' data) above the writes, nor the next round's writes above these reads
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      const int n = n0 + wn * 64 + rcol * 8;
+#pragma unroll
+      for (int p8 = 0; p8 < 4; ++p8) {
+        const int row = p8 * 8 + rrow;
+        const u32x2 lo = *reinterpret_cast<const u32x2*>(sw + row * LDE + rcol * 16);
+        const u32x2 hi = *reinterpret_cast<const u32x2*>(sw + row * LDE + rcol * 16 + 8);
+        const int m = m0 + wm * 128 + tm * 32 + row;
+        if (m < M && n < N) {  // N is a multiple of 8: the eight columns are in or out together
+          u32x4 o = {lo[0], lo[1], hi[0], hi[1]};
+          *reinterpret_cast<u32x4*>(Ce + (size_t)m * N + n) = o;
+        }
       }
-      return;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
+    return;
   }
 #pragma unroll
   for (int tm = 0; tm < 4; ++tm) {
@@ -335,16 +316,8 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
         if (n >= N) continue;  // N is a multiple of 4: the four columns are in or out together
         const float v0 = acc[tn][tm][4 * q], v1 = acc[tn][tm][4 * q + 1];
         const float v2 = acc[tn][tm][4 * q + 2], v3 = acc[tn][tm][4 * q + 3];
-        if (Pe != nullptr) {
-          f32x4 o = {v0, v1, v2, v3};
-          *reinterpret_cast<f32x4*>(Pe + (size_t)m * N + n) = o;
-        } else if constexpr (BF16) {
-          u32x2 o = {pack_bf16x2(v0, v1), pack_bf16x2(v2, v3)};
-          *reinterpret_cast<u32x2*>(Ce + (size_t)m * N + n) = o;
-        } else {
-          f32x4 o = {v0, v1, v2, v3};
-          *reinterpret_cast<f32x4*>(Ce + (size_t)m * N + n) = o;
-        }
+        f32x4 o = {v0, v1, v2, v3};
+        *reinterpret_cast<f32x4*>(Pe + (size_t)m * N + n) = o;
       }
     }
   }
@@ -742,6 +715,11 @@ extern "C" int fs2moe_grouped_wgrad(const void* a, const int32_t* a_row_map, con
   int segments = 1;
   if (counts == nullptr) {
     segments = wgrad_segments(max_rows, M, N);
+    if (dtype == FS2MOE_F32) {
+      // (the f32 tiles are smaller: enough segments for two blocks to a CU)
+      const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64), enough = (511 + tiles) / tiles;
+      if (segments > enough) segments = (int)enough;
+    }
     if (workspace == nullptr || workspace_bytes < (int64_t)segments * M * N * 4) segments = 1;
   }
   const int slots = counts != nullptr ? E : segments;
@@ -756,33 +734,36 @@ extern "C" int fs2moe_grouped_wgrad(const void* a, const int32_t* a_row_map, con
   Groups g{counts, offsets, E, (int)max_rows};
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool mapped = a_row_map != nullptr;
-  auto kb = mapped ? grouped_wgrad_kernel<uint16_t, true> : grouped_wgrad_kernel<uint16_t, false>;
-  auto kf = mapped ? grouped_wgrad_kernel<float, true> : grouped_wgrad_kernel<float, false>;
-  static bool attr_set = false;  // benign race: setting the attribute is idempotent
-  if (!attr_set) {
-    const void* ks[4] = {reinterpret_cast<const void*>(grouped_wgrad_kernel<uint16_t, false>),
-                         reinterpret_cast<const void*>(grouped_wgrad_kernel<uint16_t, true>),
-                         reinterpret_cast<const void*>(grouped_wgrad_kernel<float, false>),
-                         reinterpret_cast<const void*>(grouped_wgrad_kernel<float, true>)};
-    for (const void* k : ks) {
-      hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, wgk::SMEM_BYTES);
-      if (e != hipSuccess) {
-        set_error("grouped_wgrad: cannot reserve %d bytes of LDS: %s", wgk::SMEM_BYTES,
-                  hipGetErrorString(e));
-        return FS2MOE_ERR_LAUNCH;
+  if (dtype == FS2MOE_BF16) {
+    auto k = mapped ? grouped_wgrad_kernel<true> : grouped_wgrad_kernel<false>;
+    static bool attr_set = false;  // benign race: setting the attribute is idempotent
+    if (!attr_set) {
+      for (const void* p : {reinterpret_cast<const void*>(grouped_wgrad_kernel<false>),
+                            reinterpret_cast<const void*>(grouped_wgrad_kernel<true>)}) {
+        hipError_t e = hipFuncSetAttribute(p, hipFuncAttributeMaxDynamicSharedMemorySize, wgk::SMEM_BYTES);
+        if (e != hipSuccess) {
+          set_error("grouped_wgrad: cannot reserve %d bytes of LDS: %s", wgk::SMEM_BYTES,
+                    hipGetErrorString(e));
+          return FS2MOE_ERR_LAUNCH;
+        }
       }
+      attr_set = true;
     }
-    attr_set = true;
-  }
-  if (dtype == FS2MOE_BF16)
-    hipLaunchKernelGGL(kb, dim3((unsigned)blocks), dim3(wgk::WAVES * 64), wgk::SMEM_BYTES, st,
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(wgk::WAVES * 64), wgk::SMEM_BYTES, st,
                        static_cast<const uint16_t*>(a), a_row_map, M,
                        static_cast<const uint16_t*>(b), N, static_cast<uint16_t*>(dw), M, N, g,
                        m_tiles, n_tiles, seg_rows, partial, paired);
-  else
-    hipLaunchKernelGGL(kf, dim3((unsigned)blocks), dim3(wgk::WAVES * 64), wgk::SMEM_BYTES, st,
-                       static_cast<const float*>(a), a_row_map, M, static_cast<const float*>(b), N,
-                       static_cast<float*>(dw), M, N, g, m_tiles, n_tiles, seg_rows, partial, paired);
+  } else {
+    const int64_t big = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
+    const bool small = f32t::small_tiles(big * slots, 128);
+    const int t = small ? 64 : 128, mt = (M + t - 1) / t, nt = (N + t - 1) / t;
+    FS2_REQUIRE((int64_t)slots * mt * nt <= 0x7fffffffll, "grouped_wgrad: too many tiles");
+    auto k = small ? (mapped ? grouped_wgrad_f32_kernel<1, true> : grouped_wgrad_f32_kernel<1, false>)
+                   : (mapped ? grouped_wgrad_f32_kernel<2, true> : grouped_wgrad_f32_kernel<2, false>);
+    hipLaunchKernelGGL(k, dim3((unsigned)(slots * mt * nt)), dim3(f32t::THREADS), 0, st,
+                       static_cast<const float*>(a), a_row_map, static_cast<const float*>(b),
+                       static_cast<float*>(dw), M, N, g, mt, nt, seg_rows, partial);
+  }
   if (int rc = check_launch("grouped_wgrad")) return rc;
   if (segments > 1) {
     const int64_t n = (int64_t)M * N;

@@ -21,6 +21,7 @@
 #include "common.h"
 #include "tile_map.h"
 #include "experts_dma.h"
+#include "experts_f32.h"
 #include "experts_fp8.h"
 #include "experts_gemv.h"
 
@@ -187,123 +188,6 @@ __global__ __launch_bounds__(256, 2) void glu_gemm_bf16_kernel(
   }
 }
 
-// ------------------------------------------------------------------------------------- f32
-// Same schedule with v_mfma_f32_32x32x2_f32 (true f32 FMA); tiles are smaller because the
-// operands are four bytes wide.  This path serves the fp32 reference configuration.
-namespace f32k {
-constexpr int BM = 64, BN = 64, BK = 16;
-constexpr int LDA = BK + 4;
-constexpr int LDB_KN = BN + 4;
-constexpr int LDB_NK = BK + 4;
-}  // namespace f32k
-
-template <bool DUAL, int BLAYOUT>
-__global__ __launch_bounds__(256) void glu_gemm_f32_kernel(
-    const float* __restrict__ A, int lda, const float* __restrict__ B0,
-    const float* __restrict__ B1, float* __restrict__ C, int ldc, int Kdim, int N, Groups g,
-    int n_tiles) {
-  using namespace f32k;
-  constexpr int NB = DUAL ? 2 : 1;
-  constexpr bool KN = BLAYOUT == FS2MOE_W_IN_OUT;
-  constexpr int SB_ELEMS = KN ? BK * LDB_KN : BN * LDB_NK;
-  __shared__ __attribute__((aligned(16))) float sA[BM * LDA];
-  __shared__ __attribute__((aligned(16))) float sB[NB][SB_ELEMS];
-
-  const int tid = threadIdx.x;
-  const int mt = blockIdx.x / n_tiles, nt = blockIdx.x - mt * n_tiles;
-  int e, row0, row_end;
-  if (!locate_tile<BM>(g, mt, e, row0, row_end)) return;
-  const int n0 = nt * BN;
-  const size_t wstride = (size_t)Kdim * N;
-  const float* Bp[2] = {B0 + (size_t)e * wstride, DUAL ? B1 + (size_t)e * wstride : nullptr};
-
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int lr = lane & 31, lk = lane >> 5;
-
-  f32x16 acc[NB];
-#pragma unroll
-  for (int b = 0; b < NB; ++b)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[b][i] = 0.f;
-
-  f32x4 ra, rb[NB];
-  const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
-  auto load_global = [&](int k0) {
-    {
-      const int row = tid >> 2, kc = tid & 3;
-      int grow = row0 + row;
-      grow = grow < row_end ? grow : row_end - 1;
-      const int k = k0 + kc * 4;
-      ra = k < Kdim ? *reinterpret_cast<const f32x4*>(A + (size_t)grow * lda + k) : zero4;
-    }
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      if (KN) {
-        const int k = k0 + (tid >> 4), n = n0 + (tid & 15) * 4;
-        rb[b] = (k < Kdim && n < N) ? *reinterpret_cast<const f32x4*>(Bp[b] + (size_t)k * N + n)
-                                    : zero4;
-      } else {
-        const int n = n0 + (tid >> 2), k = k0 + (tid & 3) * 4;
-        rb[b] = (k < Kdim && n < N)
-                    ? *reinterpret_cast<const f32x4*>(Bp[b] + (size_t)n * Kdim + k)
-                    : zero4;
-      }
-    }
-  };
-  auto store_lds = [&]() {
-    *reinterpret_cast<f32x4*>(&sA[(tid >> 2) * LDA + (tid & 3) * 4]) = ra;
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      if (KN)
-        *reinterpret_cast<f32x4*>(&sB[b][(tid >> 4) * LDB_KN + (tid & 15) * 4]) = rb[b];
-      else
-        *reinterpret_cast<f32x4*>(&sB[b][(tid >> 2) * LDB_NK + (tid & 3) * 4]) = rb[b];
-    }
-  };
-
-  const bool active = row0 + wm * 32 < row_end;
-  const int nk = (Kdim + BK - 1) / BK;
-  load_global(0);
-  for (int kt = 0; kt < nk; ++kt) {
-    store_lds();
-    __syncthreads();
-    if (kt + 1 < nk) load_global((kt + 1) * BK);
-    if (active) {
-#pragma unroll
-      for (int ks = 0; ks < BK / 2; ++ks) {
-        const int k = ks * 2 + lk;
-        const float xf = sA[(wm * 32 + lr) * LDA + k];
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          const float wf = KN ? sB[b][k * LDB_KN + wn * 32 + lr] : sB[b][(wn * 32 + lr) * LDB_NK + k];
-          acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(wf, xf, acc[b], 0, 0, 0);
-        }
-      }
-    }
-    __syncthreads();
-  }
-
-  const int m = row0 + wm * 32 + lr;
-  if (m >= row_end) return;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int n = n0 + wn * 32 + 8 * q + 4 * lk;
-    if (n >= N) continue;
-    f32x4 v;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (DUAL) {
-        const float gte = acc[0][4 * q + j];
-        v[j] = (gte / (1.0f + expf(-gte))) * acc[NB - 1][4 * q + j];
-      } else {
-        v[j] = acc[0][4 * q + j];
-      }
-    }
-    *reinterpret_cast<f32x4*>(C + (size_t)m * ldc + n) = v;
-  }
-}
-
 // ------------------------------------------------------------------------------------ host
 // Compute units of the current device, rounded down to a multiple of its 8 XCDs (0 on failure).
 static int cu_count_by_xcd() {
@@ -317,6 +201,31 @@ static int cu_count_by_xcd() {
     cached = cus / 8 * 8;
   }
   return cached;
+}
+
+// One launch of the f32 kernel; a2, g_keep, u_keep may be null.
+template <bool DUAL, int BLAYOUT>
+static int launch_f32(const void* a, const void* b0, const void* b1, const void* a2, void* c,
+                      void* g_keep, void* u_keep, int K, int N, const Groups& g, int64_t rows_bound,
+                      const char* what, hipStream_t stream) {
+  const int groups = g.counts ? g.E : 0;
+  const int big_n = DUAL ? 64 : 128;
+  const bool small = f32t::small_tiles((rows_bound / 128 + groups + 1) * ((N + big_n - 1) / big_n),
+                                       groups ? rows_bound / groups : rows_bound);
+  const int bm = small ? 64 : 128, bn = small ? 64 : big_n;
+  const int64_t m_tiles = rows_bound / bm + groups + 1;
+  const int nt = (N + bn - 1) / bn;
+  if (m_tiles * nt > 0x7ffffff0ll) {
+    set_error("%s: grid too large", what);
+    return FS2MOE_ERR_UNSUPPORTED;
+  }
+  auto k = small ? glu_gemm_f32_kernel<DUAL, 1, 1, BLAYOUT> : glu_gemm_f32_kernel<DUAL, 2, DUAL ? 1 : 2, BLAYOUT>;
+  hipLaunchKernelGGL(k, dim3((unsigned)((m_tiles * nt + 7) / 8 * 8)), dim3(f32t::THREADS), 0, stream,
+                     static_cast<const float*>(a), static_cast<const float*>(b0),
+                     static_cast<const float*>(b1), static_cast<const float*>(a2),
+                     static_cast<float*>(c), static_cast<float*>(g_keep), static_cast<float*>(u_keep), K,
+                     N, g, nt);
+  return check_launch(what);
 }
 
 // e4m3 weights go to the throughput kernel from this many rows per expert on (mean over all experts)
@@ -584,23 +493,11 @@ static int launch_glu(const void* x, const int32_t* row_map, const Groups& g, in
                        static_cast<uint16_t*>(y), D, F, D, g, nt2);
     return check_launch("glu_gemm_bf16<down>");
   }
-  using namespace f32k;
-  const int64_t m_tiles = rows_bound / BM + groups + 1;
-  const int nt1 = (F + BN - 1) / BN, nt2 = (D + BN - 1) / BN;
-  if (m_tiles * nt1 > 0x7fffffffll || m_tiles * nt2 > 0x7fffffffll) {
-    set_error("experts: grid too large");
-    return FS2MOE_ERR_UNSUPPORTED;
-  }
-  hipLaunchKernelGGL((glu_gemm_f32_kernel<true, BLAYOUT>), dim3((unsigned)(m_tiles * nt1)),
-                     dim3(256), 0, stream, static_cast<const float*>(x), D,
-                     static_cast<const float*>(w_gate), static_cast<const float*>(w_up),
-                     static_cast<float*>(h), F, D, F, g, nt1);
-  if (int rc = check_launch("glu_gemm_f32<gate,up>")) return rc;
-  hipLaunchKernelGGL((glu_gemm_f32_kernel<false, BLAYOUT>), dim3((unsigned)(m_tiles * nt2)),
-                     dim3(256), 0, stream, static_cast<const float*>(h), F,
-                     static_cast<const float*>(w_down), static_cast<const float*>(nullptr),
-                     static_cast<float*>(y), D, F, D, g, nt2);
-  return check_launch("glu_gemm_f32<down>");
+  if (int rc = launch_f32<true, BLAYOUT>(x, w_gate, w_up, nullptr, h, nullptr, nullptr, D, F, g, rows_bound,
+                                         "glu_gemm_f32<gate,up>", stream))
+    return rc;
+  return launch_f32<false, BLAYOUT>(h, w_down, nullptr, nullptr, y, nullptr, nullptr, F, D, g, rows_bound,
+                                    "glu_gemm_f32<down>", stream);
 }
 
 }  // namespace fs2moe
@@ -826,17 +723,8 @@ static int launch_gemm(const void* a, const int32_t* row_map, const Groups& g, i
                        static_cast<uint16_t*>(c), N, K, N, g, nt);
     return check_launch("glu_gemm_bf16<single>");
   }
-  using namespace f32k;
-  const int64_t m_tiles = rows_bound / BM + groups + 1;
-  const int nt = (N + BN - 1) / BN;
-  if (m_tiles * nt > 0x7fffffffll) {
-    set_error("gemm: grid too large");
-    return FS2MOE_ERR_UNSUPPORTED;
-  }
-  hipLaunchKernelGGL((glu_gemm_f32_kernel<false, BLAYOUT>), dim3((unsigned)(m_tiles * nt)), dim3(256),
-                     0, stream, static_cast<const float*>(a), K, static_cast<const float*>(b),
-                     static_cast<const float*>(nullptr), static_cast<float*>(c), N, K, N, g, nt);
-  return check_launch("glu_gemm_f32<single>");
+  return launch_f32<false, BLAYOUT>(a, b, nullptr, nullptr, c, nullptr, nullptr, K, N, g, rows_bound,
+                                    "glu_gemm_f32<single>", stream);
 }
 
 extern "C" int fs2moe_grouped_gemm(const void* a, const int32_t* row_map, const int32_t* counts,

@@ -1,0 +1,405 @@
+// f32 GEMMs of the expert networks and of their backward pass, on v_mfma_f32_32x32x2_f32 (true f32
+// products and sums).
+//
+// What bounds them: the matrix pipe (64 clocks per instruction and SIMD, 157 TFLOP/s nominal, 154 in a
+// large product of the vendor's library), and, with few tiles, their number against 256 CUs.  A chunk is
+// 32 k; two chunks are on their way from memory in two register sets while a third is multiplied, LDS
+// holds two (one barrier per chunk), and a block is 4 waves on a 64 x 64 or 128 x 128 tile: the small one,
+// several blocks to a CU, where 128 x 128 tiles would not fill the chip twice (f32t::small_tiles).  What a
+// wave does besides multiplying is dealt out one instruction behind each product (Walk::run): as phases,
+// i.e. stores, barrier, loads, reads, products, the same tiles reach 132 TFLOP/s with every SIMD full
+// and 95 with one wave on each, whether one chunk or four are in flight; dealt out 149-154 and 107.
+// 8192 x 2048 by 2048 x 4096: 1012 -> 949 us (the library's product 923); the kernels before these, 64 x 64
+// tiles of 16 k one chunk ahead and 256 x 256 tiles for the weight gradients: 512 x 1408 by 8 experts of
+// 250 rows on average 52 -> 36 us a product and 83 -> 28 us a weight gradient.
+//
+// k slots.  Lanes 0..31 carry one k of an instruction and lanes 32..63 the other, and which k they are is
+// free as long as both operands agree: instruction j of step s takes k 8 s + j and 8 s + 4 + j, so that a
+// lane's four values of a k-contiguous operand are one 16-byte LDS read.
+//
+// LDS layouts (16-byte chunks).  k-contiguous operand: rows of 128 bytes, chunk c of row r in slot
+// c ^ ((r >> 1) & 7).  k-major operand: a row per k, chunk c of row k in slot c ^ (((k >> 2) & 1) << 3), so
+// that the two half waves, which read rows 4 apart, use different banks.
+#pragma once
+
+#include <type_traits>
+
+#include "common.h"
+#include "tile_map.h"
+
+namespace fs2moe {
+namespace f32t {
+constexpr int BK = 32, THREADS = 256;
+
+// Tiles of 64 x 64 while 128 x 128 ones would give a CU fewer than two blocks (big_tiles of them in the
+// launch), or where the groups have so few rows on average that half of a 128-row tile would be padding.
+inline bool small_tiles(int64_t big_tiles, int64_t rows_per_group) {
+  return big_tiles < 512 || rows_per_group <= 96;
+}
+
+// what a load through a row map reads past the end (not const: a global address)
+static __device__ __attribute__((aligned(16))) uint32_t zero16[4] = {0u, 0u, 0u, 0u};
+
+// A chunk (32 k) of one operand: ROWS rows (or columns) x 32 k.  `base` points at the operand's first row
+// (column) of the tile in k 0; ld is the stride in floats of a row (k-contiguous) or of a k (k-major).
+template <int ROWS, bool KMAJOR>
+struct Operand {
+  static constexpr int BYTES = ROWS * BK * 4;
+  static constexpr int PER = ROWS * BK / 4 / THREADS;  // 16-byte chunks per thread
+  static constexpr int CPK = ROWS / 4;                 // k-major: chunks per k
+  uint32_t off[PER];
+  bool ok[KMAJOR ? PER : 1];  // k-major: the chunk's columns exist
+
+  // rows: how many of the tile's rows (columns) exist, at least 1.  Rows past them repeat the last one
+  // (their results are not stored), columns past them are zeros.
+  __device__ __forceinline__ void setup(int tid, int ld, int rows) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int c = tid + THREADS * i;
+      if constexpr (KMAJOR) {
+        off[i] = (uint32_t)((c / CPK) * ld + (c % CPK) * 4) * 4u;
+        ok[i] = (c % CPK) * 4 < rows;
+      } else {
+        const int r = c >> 3;
+        off[i] = (uint32_t)((r < rows ? r : rows - 1) * ld + (c & 7) * 4) * 4u;
+      }
+    }
+  }
+  // The pieces of k from k0 on, `left` of them (what lies past the end loads zeros and touches no memory):
+  // where they come from, then piece by piece.
+  struct From {
+    __amdgpu_buffer_rsrc_t rsrc;
+    int left;
+  };
+  static __device__ __forceinline__ From from(const float* base, int ld, int k0, int left) {
+    const float* p = KMAJOR ? base + (size_t)k0 * ld : base + k0;
+    return From{__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, 0xfffffff0u, 0x00020000), left};
+  }
+  __device__ __forceinline__ u32x4 load(const From& f, int tid, int i) const {
+    const bool in = KMAJOR ? ok[i] && (tid + THREADS * i) / CPK < f.left : (tid & 7) * 4 < f.left;
+    return __builtin_amdgcn_raw_buffer_load_b128(f.rsrc, in ? off[i] : 0xfffffff0u, 0, 0);
+  }
+  // the same of a k-major operand whose row k is row map[k] of `base`
+  __device__ __forceinline__ void load_mapped(u32x4 (&reg)[PER], int tid, const float* base, int ld,
+                                              const int32_t* map, int k0, int left) const {
+    static_assert(KMAJOR, "the rows of the contraction are mapped");
+    int row[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int k = (tid + THREADS * i) / CPK;
+      row[i] = map[left > 0 ? k0 + (k < left ? k : left - 1) : 0];
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int c = tid + THREADS * i;
+      const float* p = base + (size_t)row[i] * ld + (c % CPK) * 4;
+      if (!(ok[i] && c / CPK < left)) p = reinterpret_cast<const float*>(zero16);
+      reg[i] = *reinterpret_cast<const u32x4*>(p);
+    }
+  }
+  static __device__ __forceinline__ void store(u32x4 reg, int tid, int i, uint8_t* lds) {
+    const int c = tid + THREADS * i;
+    const int at = KMAJOR ? (c / CPK) * CPK + ((c % CPK) ^ (((c / CPK) >> 2 & 1) << 3))
+                          : (c >> 3) * 8 + ((c & 7) ^ ((c >> 4) & 7));
+    *reinterpret_cast<u32x4*>(lds + at * 16) = reg;
+  }
+  // the lane's four values of step s (k 8 s + 4 (lane / 32) + 0..3) of the 32 rows from r0 on
+  static __device__ __forceinline__ f32x4 frag(const uint8_t* lds, int lane, int r0, int s) {
+    const int lr = lane & 31, lk = lane >> 5;
+    if constexpr (KMAJOR) {
+      const float* p = reinterpret_cast<const float*>(lds) + (8 * s + 4 * lk) * ROWS + ((r0 + lr) ^ (lk << 5));
+      return f32x4{p[0], p[ROWS], p[2 * ROWS], p[3 * ROWS]};
+    } else {
+      const int r = r0 + lr;
+      return *reinterpret_cast<const f32x4*>(lds + r * 128 + (((2 * s + lk) ^ ((r >> 1) & 7)) << 4));
+    }
+  }
+};
+
+// The walk over k of one tile: waves 2 x 2, each 32 FM rows x 32 FN channels of each of NB matrices.
+// acc[b][fn][fm] is the transposed 32 x 32 tile (lane: row lr, channels 8 q + 4 lk + 0..3 in 4 q ..).
+// With two sources the second pair follows the first in the same accumulators.
+// A_MAPPED: a_map gives the rows of the k-major A.
+template <int NB, int FM, int FN, bool A_KMAJOR, bool B_KMAJOR, bool A_MAPPED = false>
+struct Walk {
+  static constexpr int BM = 64 * FM, BN = 64 * FN;
+  using OpA = Operand<BM, A_KMAJOR>;
+  using OpB = Operand<BN, B_KMAJOR>;
+  static constexpr int BUF_BYTES = OpA::BYTES + NB * OpB::BYTES;
+  static constexpr int SMEM_BYTES = 2 * BUF_BYTES;
+  static constexpr int PIECES = OpA::PER + NB * OpB::PER;  // 16-byte pieces of a chunk per thread
+  static constexpr int PRODUCTS = BK / 2 * NB * FM * FN;    // MFMAs of a chunk per wave
+
+  struct Source {
+    const float* a;
+    const float* b[NB];
+  };
+  // m_rows, n_cols: how many of the tile's rows and channels exist; `active`: this wave's rows do
+  static __device__ __forceinline__ void run(f32x16 (&acc)[NB][FN][FM], uint8_t* smem, const Source& s0,
+                                             const Source& s1, int sources, int lda, int ldb, int K,
+                                             int m_rows, int n_cols, bool active,
+                                             const int32_t* a_map = nullptr) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 1, wn = wave >> 1;
+    OpA opa;
+    OpB opb;
+    opa.setup(tid, lda, m_rows);
+    opb.setup(tid, ldb, n_cols);
+    const int nk = (K + BK - 1) / BK, steps = sources * nk;
+    u32x4 ra[2][OpA::PER], rb[2][NB][OpB::PER];
+    // piece p of a chunk's PIECES: A's first, then each matrix's
+    struct Chunk {
+      typename OpA::From a;
+      typename OpB::From b[NB];
+      int k0, left;
+    };
+    auto chunk_at = [&](int step) {
+      const bool second = step >= nk;
+      const int k0 = (second ? step - nk : step) * BK;
+      const int left = step < steps ? K - k0 : 0;
+      Chunk c;
+      c.k0 = k0;
+      c.left = left;
+      c.a = OpA::from(second ? s1.a : s0.a, lda, k0, left);
+#pragma unroll
+      for (int i = 0; i < NB; ++i) c.b[i] = OpB::from(second ? s1.b[i] : s0.b[i], ldb, k0, left);
+      return c;
+    };
+    auto load = [&](auto& a, auto& b, const Chunk& c, int p) {
+      if (p < OpA::PER) {
+        if constexpr (A_MAPPED) {
+          if (p == 0) opa.load_mapped(a, tid, s0.a, lda, a_map, c.k0, c.left);
+        } else {
+          a[p] = opa.load(c.a, tid, p);
+        }
+      } else {
+        const int i = (p - OpA::PER) / OpB::PER, j = (p - OpA::PER) % OpB::PER;
+        b[i][j] = opb.load(c.b[i], tid, j);
+      }
+    };
+    auto store = [&](const auto& a, const auto& b, int buf, int p) {
+      uint8_t* at = smem + buf * BUF_BYTES;
+      if (p < OpA::PER) {
+        OpA::store(a[p], tid, p, at);
+      } else {
+        const int i = (p - OpA::PER) / OpB::PER, j = (p - OpA::PER) % OpB::PER;
+        OpB::store(b[i][j], tid, j, at + OpA::BYTES + i * OpB::BYTES);
+      }
+    };
+    f32x4 xf[2][FM], wf[2][NB][FN];
+    auto read = [&](int set, int buf, int s) {
+      const uint8_t* at = smem + buf * BUF_BYTES;
+#pragma unroll
+      for (int fm = 0; fm < FM; ++fm) xf[set][fm] = OpA::frag(at, lane, (wm * FM + fm) * 32, s);
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int fn = 0; fn < FN; ++fn)
+          wf[set][b][fn] = OpB::frag(at + OpA::BYTES + b * OpB::BYTES, lane, (wn * FN + fn) * 32, s);
+    };
+    // Chunk st is multiplied from buffer st & 1, while chunk st + 1 is stored from register set
+    // (st + 1) & 1 into the other buffer (read last in chunk st - 1, whose barrier has passed) and the
+    // loads of chunk st + 3 go into the registers that frees.  A wave issues in order, and a 16-byte store
+    // takes its turn for about 80 clocks and a load for about 40: they go out one at a time, each behind
+    // a product that takes the matrix pipe 64 clocks, and each step's fragments are read a step ahead.
+    // (The fences keep that order: left alone, the compiler moves the reads to their first use.  A wave
+    // without rows walks a loop of its own: a condition around the products would make every one of them
+    // wait for all LDS traffic in flight.)
+    auto chunk = [&](auto multiply, auto& a, auto& b, int buf, int st) {
+      const Chunk next = chunk_at(st + 3);
+      if constexpr (decltype(multiply)::value) {
+        constexpr int EVERY = PRODUCTS / (2 * PIECES);
+        static_assert(EVERY >= 1 && EVERY * 2 * PIECES <= PRODUCTS, "a product per store and load");
+        read(0, buf, 0);
+#pragma unroll
+        for (int s = 0; s < BK / 8; ++s) {
+          if (s + 1 < BK / 8) read((s + 1) & 1, buf, s + 1);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int m = 0; m < NB; ++m)
+#pragma unroll
+              for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+                for (int fm = 0; fm < FM; ++fm) {
+                  __builtin_amdgcn_sched_barrier(0);
+                  acc[m][fn][fm] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                      wf[s & 1][m][fn][j], xf[s & 1][fm][j], acc[m][fn][fm], 0, 0, 0);
+                  const int done = (((s * 4 + j) * NB + m) * FN + fn) * FM + fm;
+                  if (done % EVERY == 0) {
+                    const int o = done / EVERY;
+                    if (o < PIECES)
+                      store(a, b, buf ^ 1, o);
+                    else if (o < 2 * PIECES)
+                      load(a, b, next, o - PIECES);
+                  }
+                }
+        }
+      } else {
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) store(a, b, buf ^ 1, p);
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) load(a, b, next, p);
+      }
+      lds_barrier();
+    };
+    auto load_all = [&](auto& a, auto& b, int step) {
+      const Chunk c = chunk_at(step);
+#pragma unroll
+      for (int p = 0; p < PIECES; ++p) load(a, b, c, p);
+      __builtin_amdgcn_sched_barrier(0);  // oldest first, as in the loop
+    };
+    load_all(ra[0], rb[0], 0);
+    load_all(ra[1], rb[1], 1);
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) store(ra[0], rb[0], 0, p);
+    load_all(ra[0], rb[0], 2);
+    lds_barrier();
+    auto walk = [&](auto multiply) {
+      int st = 0;
+      for (; st + 1 < steps; st += 2) {
+        chunk(multiply, ra[1], rb[1], 0, st);
+        chunk(multiply, ra[0], rb[0], 1, st + 1);
+      }
+      if (st < steps) chunk(multiply, ra[1], rb[1], 0, st);
+    };
+    if (active)
+      walk(std::integral_constant<bool, true>{});
+    else
+      walk(std::integral_constant<bool, false>{});
+  }
+};
+}  // namespace f32t
+
+// C = A B_e (+ A2 B2_e), or with DUAL C = SiLU(A B0_e) * (A B1_e), the two products left in g_keep and
+// u_keep where those are given.  A block per tile; BLAYOUT as for the bf16 kernels.
+template <bool DUAL, int FM, int FN, int BLAYOUT>
+__global__ __launch_bounds__(f32t::THREADS, 2) void glu_gemm_f32_kernel(
+    const float* __restrict__ A, const float* __restrict__ B0, const float* __restrict__ B1,
+    const float* __restrict__ A2, float* __restrict__ C, float* __restrict__ g_keep,
+    float* __restrict__ u_keep, int K, int N, Groups g, int n_tiles) {
+  constexpr int NB = DUAL ? 2 : 1;
+  constexpr bool KN = BLAYOUT == FS2MOE_W_IN_OUT;
+  using W = f32t::Walk<NB, FM, FN, false, KN>;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[W::SMEM_BYTES];
+  int e, row0, row_end, nt;
+  if (!locate_tile_by_xcd<W::BM>(g, n_tiles, e, row0, row_end, nt)) return;
+  e = __builtin_amdgcn_readfirstlane(e);
+  row0 = __builtin_amdgcn_readfirstlane(row0);
+  row_end = __builtin_amdgcn_readfirstlane(row_end);
+  const int n0 = nt * W::BN;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave & 1, wn = wave >> 1, lr = lane & 31, lk = lane >> 5;
+
+  f32x16 acc[NB][FN][FM];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+      for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[b][fn][fm][i] = 0.f;
+
+  const size_t at = (size_t)e * K * N + (KN ? (size_t)n0 : (size_t)n0 * K);
+  typename W::Source s0, s1;
+  s0.a = A + (size_t)row0 * K;
+  s0.b[0] = B0 + at;
+  s1 = s0;
+  if constexpr (DUAL) {
+    s0.b[1] = B1 + at;
+  } else if (A2 != nullptr) {
+    s1.a = A2 + (size_t)row0 * K;
+    s1.b[0] = B1 + at;
+  }
+  const int m_wave = row0 + wm * 32 * FM;
+  W::run(acc, smem, s0, s1, !DUAL && A2 != nullptr ? 2 : 1, K, KN ? N : K, K, row_end - row0, N - n0,
+         m_wave < row_end);
+
+#pragma unroll
+  for (int fm = 0; fm < FM; ++fm) {
+    const int m = m_wave + fm * 32 + lr;
+    if (m >= row_end) continue;
+#pragma unroll
+    for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = n0 + (wn * FN + fn) * 32 + 8 * q + 4 * lk;
+        if (n >= N) continue;
+        const size_t to = (size_t)m * N + n;
+        f32x4 v, u;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v[j] = acc[0][fn][fm][4 * q + j];
+          u[j] = acc[NB - 1][fn][fm][4 * q + j];
+        }
+        if constexpr (DUAL) {
+          if (g_keep != nullptr) {
+            *reinterpret_cast<f32x4*>(g_keep + to) = v;
+            *reinterpret_cast<f32x4*>(u_keep + to) = u;
+          }
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = (v[j] / (1.0f + expf(-v[j]))) * u[j];
+        }
+        *reinterpret_cast<f32x4*>(C + to) = v;
+      }
+  }
+}
+
+// dW_e = A_e^T B_e over the rows of an expert (slots: the experts), or over seg_rows rows each of one
+// group (slots: segments, whose sums go to `partial` where there are several).
+// MAPPED: A's rows are read through a_map.
+template <int F, bool MAPPED>
+__global__ __launch_bounds__(f32t::THREADS, 2) void grouped_wgrad_f32_kernel(
+    const float* __restrict__ A, const int32_t* __restrict__ a_map, const float* __restrict__ B,
+    float* __restrict__ C, int M, int N, Groups g, int m_tiles, int n_tiles, int seg_rows,
+    float* __restrict__ partial) {
+  using W = f32t::Walk<1, F, F, true, true, MAPPED>;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[W::SMEM_BYTES];
+  const int per = m_tiles * n_tiles;
+  const int slot = blockIdx.x / per, rem = blockIdx.x - slot * per;
+  const int mt = rem / n_tiles, nt = rem - mt * n_tiles;
+  int off, cnt;
+  if (g.counts == nullptr) {
+    off = slot * seg_rows;
+    cnt = g.dense_rows - off < seg_rows ? g.dense_rows - off : seg_rows;
+  } else {
+    off = __builtin_amdgcn_readfirstlane(g.offsets[slot]);
+    cnt = __builtin_amdgcn_readfirstlane(g.counts[slot]);
+  }
+  const int m0 = mt * W::BM, n0 = nt * W::BN;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave & 1, wn = wave >> 1, lr = lane & 31, lk = lane >> 5;
+  f32x16 acc[1][F][F];
+#pragma unroll
+  for (int fn = 0; fn < F; ++fn)
+#pragma unroll
+    for (int fm = 0; fm < F; ++fm)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[0][fn][fm][i] = 0.f;
+  typename W::Source s;
+  s.a = (MAPPED ? A : A + (size_t)off * M) + m0;
+  s.b[0] = B + (size_t)off * N + n0;
+  const int m_wave = m0 + wm * 32 * F;
+  if (cnt > 0) W::run(acc, smem, s, s, 1, M, N, cnt, M - m0, N - n0, m_wave < M,
+                     MAPPED ? a_map + off : nullptr);
+  float* to = partial != nullptr ? partial : C;
+  to += (size_t)slot * M * N;
+#pragma unroll
+  for (int fm = 0; fm < F; ++fm) {
+    const int m = m_wave + fm * 32 + lr;
+    if (m >= M) continue;
+#pragma unroll
+    for (int fn = 0; fn < F; ++fn)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = n0 + (wn * F + fn) * 32 + 8 * q + 4 * lk;
+        if (n >= N) continue;
+        const f32x16& a = acc[0][fn][fm];
+        *reinterpret_cast<f32x4*>(to + (size_t)m * N + n) = f32x4{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+      }
+  }
+}
+
+}  // namespace fs2moe

@@ -121,6 +121,39 @@ def test_grouped_gemm_both_orientations(gpu_device, dtype, layout, rows, k, n):
     assert_grad_close(d, a.double() @ b[0].double(), dtype, "dense")
 
 
+# Both tile sizes of the f32 kernels (128 x 128 from 512 such tiles on), their edges in rows and channels,
+# K (for the weight gradient: rows) below, at and off its chunks of 32.
+@pytest.mark.parametrize("rows,k,n", [
+    ([63, 64, 65, 0, 1], 8, 56), ([129, 31, 32, 33], 40, 64), ([97], 96, 136),
+    ([700, 127, 128, 1, 1300], 40, 4104), ([400] * 6, 1000, 1032),
+])
+def test_f32_products_at_the_edges_of_their_tiles(gpu_device, rows, k, n):
+    _say("f32 products", rows, k, n)
+    dev = gpu_device
+    g = torch.Generator().manual_seed(k + n)
+    e = len(rows)
+    counts, offsets = _groups(rows)
+    c, o = counts.to(dev), offsets.to(dev)
+    total = int(offsets[-1])
+    a, d = torch.randn(total, k, generator=g).to(dev), torch.randn(total, n, generator=g).to(dev)
+    w = (0.1 * torch.randn(e, k, n, generator=g)).to(dev)
+    y1 = _abi.grouped_gemm(a, w.reshape(e * k, n), _abi.W_IN_OUT, c, o, e)
+    y2 = _abi.grouped_gemm(a, w.transpose(1, 2).contiguous().reshape(e * n, k), _abi.W_OUT_IN, c, o, e)
+    order = torch.randperm(total, generator=g)
+    scattered = torch.empty_like(a)
+    scattered[order.to(dev)] = a
+    dw = _abi.grouped_wgrad(a, d, c, o, e).reshape(e, k, n)
+    dw_map = _abi.grouped_wgrad(scattered, d, c, o, e, a_row_map=order.to(torch.int32).to(dev)).reshape(e, k, n)
+    assert torch.equal(dw, dw_map)
+    for ex in range(e):
+        sl = slice(int(offsets[ex]), int(offsets[ex]) + int(counts[ex]))
+        ref = a[sl].cpu().double() @ w[ex].cpu().double()
+        if rows[ex]:
+            assert_grad_close(y1[sl], ref, "fp32", f"expert {ex}, (in, out)")
+            assert_grad_close(y2[sl], ref, "fp32", f"expert {ex}, (out, in)")
+        assert_grad_close(dw[ex], a[sl].cpu().double().t() @ d[sl].cpu().double(), "fp32", f"expert {ex}, weight gradient")
+
+
 @pytest.mark.parametrize("rows,k,n", [([5, 0, 300, 64, 1, 700], 192, 128), ([130, 257], 64, 72), ([0, 0, 9], 128, 256)])
 def test_grouped_gemm_sum_adds_two_products(gpu_device, rows, k, n):
     """``a1 @ B1^T + a2 @ B2^T`` in one kernel against f64, and against the two products apart."""
