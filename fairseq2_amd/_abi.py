@@ -24,6 +24,24 @@ ACT_MXFP8 = 0x100  # OR-ed into a whole-layer call's w_dtype next to e4m3 weight
 W_IN_OUT, W_OUT_IN = 0, 1
 MAX_EXPERTS, MAX_TOP_K = 512, 32
 
+
+
+class TrainArgs(ctypes.Structure):
+    """``fs2moe_train_args`` of include/fs2moe.h, field by field."""
+
+    _fields_ = (
+        [(n, c_int32) for n in ("T", "D", "E", "K", "F", "F_shared", "tile_m", "act_dtype",
+                                "score_fn", "renormalize", "scale_input", "normed")]
+        + [("norm_eps", c_float), ("reserved", c_int32)]
+        + [(n, c_void_p) for n in ("x", "norm_weight", "residual", "router", "router_read", "router_bias",
+                                   "w_gate", "w_up", "w_down", "shared_gate", "shared_up", "shared_down",
+                                   "saved", "workspace")]
+        + [("saved_bytes", c_int64), ("workspace_bytes", c_int64)]
+        + [(n, c_void_p) for n in ("out", "dout", "dx", "d_router", "d_gate", "d_up", "d_down",
+                                   "d_shared_gate", "d_shared_up", "d_shared_down", "d_norm_weight")]
+    )
+
+
 # name -> (restype, argtypes); mirrors include/fs2moe.h one to one
 _PROTOTYPES = {
     "fs2moe_abi_version": (c_int32, []),
@@ -130,6 +148,10 @@ _PROTOTYPES = {
         [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32,
          c_int32, c_void_p, c_void_p],
     ),
+    "fs2moe_train_saved_bytes": (c_int64, [ctypes.POINTER(TrainArgs)]),
+    "fs2moe_train_workspace_bytes": (c_int64, [ctypes.POINTER(TrainArgs), c_int32]),
+    "fs2moe_train_forward": (c_int32, [ctypes.POINTER(TrainArgs), c_void_p]),
+    "fs2moe_train_backward": (c_int32, [ctypes.POINTER(TrainArgs), c_void_p]),
     "fs2moe_rms_norm_backward_workspace_bytes": (c_int64, [c_int32, c_int32]),
     "fs2moe_rms_norm_backward": (
         c_int32,
@@ -1026,3 +1048,68 @@ def forward(
         _check_norm_weight(norm[0], x)
         _check(lib.fs2moe_forward_norm(_ptr(x), _ptr(norm[0]), float(norm[1]), *tail), "fs2moe_forward_norm")
     return out
+
+
+def _train_args(x, router, wg, wu, wd, shared, norm_w, cfg) -> TrainArgs:
+    a = TrainArgs()
+    a.T, a.D = x.shape
+    a.E, a.K, a.tile_m = cfg["num_experts"], cfg["top_k"], cfg["tile_m"]
+    a.F = wd.shape[0] // a.E
+    a.act_dtype = dtype_code(x.dtype)
+    a.score_fn, a.renormalize, a.scale_input = cfg["score_fn"], int(cfg["renormalize"]), int(cfg["scale_input"])
+    if cfg.get("norm_eps") is not None:
+        a.normed, a.norm_eps = 1, cfg["norm_eps"]
+        a.norm_weight = _ptr(norm_w)
+    a.x, a.router, a.router_bias = _ptr(x), _ptr(router), _ptr(cfg["router_bias"])
+    a.w_gate, a.w_up, a.w_down = _ptr(wg), _ptr(wu), _ptr(wd)
+    if shared[0] is not None:
+        a.F_shared = shared[0].shape[0]
+        a.shared_gate, a.shared_up, a.shared_down = map(_ptr, shared)
+    return a
+
+
+def train_forward(x: Tensor, residual: Tensor | None, router: Tensor, wg: Tensor, wu: Tensor, wd: Tensor,
+                  shared: tuple, norm_w: Tensor | None, cfg: dict) -> tuple[Tensor, Tensor] | None:
+    """``(out, saved)`` of the layer's forward pass in training (``fs2moe_train_forward``), ``saved``
+    the opaque buffer that :func:`train_backward` reads; None at sizes the call does not take.  ``cfg``
+    as for :class:`fairseq2_amd.autograd.MoEFunction`; the arguments are those that
+    :func:`check_layer_arguments` has passed."""
+    lib = load()
+    a = _train_args(x, router, wg, wu, wd, shared, norm_w, cfg)
+    saved_bytes = lib.fs2moe_train_saved_bytes(a)
+    if saved_bytes < 0:
+        return None
+    if cfg.get("norm_eps") is not None:
+        _check_norm_weight(norm_w, x)
+    if residual is not None:
+        _same("residual", residual, x.shape, x.dtype, x.device)
+        a.residual = _ptr(residual)
+    mat, a.score_fn = router_operand(lib, x, router, cfg.get("router_t"), a.score_fn)
+    a.router_read = _ptr(mat)
+    a.workspace_bytes, a.saved_bytes = lib.fs2moe_train_workspace_bytes(a, 0), saved_bytes
+    saved = torch.empty(saved_bytes, dtype=torch.uint8, device=x.device)
+    workspace = torch.empty(a.workspace_bytes, dtype=torch.uint8, device=x.device)
+    out = torch.empty_like(x)
+    a.saved, a.workspace, a.out = saved.data_ptr(), workspace.data_ptr(), out.data_ptr()
+    _check(lib.fs2moe_train_forward(a, _stream()), "fs2moe_train_forward")
+    return out, saved
+
+
+def train_backward(x: Tensor, router: Tensor, wg: Tensor, wu: Tensor, wd: Tensor, shared: tuple,
+                   norm_w: Tensor | None, cfg: dict, saved: Tensor, dout: Tensor, need: tuple) -> tuple:
+    """Gradients ``(dx, d_router, d_wg, d_wu, d_wd, d_sg, d_su, d_sd, d_norm_w)`` from the output
+    gradient and what :func:`train_forward` saved (``fs2moe_train_backward``); None where ``need`` -- in
+    that order -- says so or where there is no such operand."""
+    lib = load()
+    a = _train_args(x, router, wg, wu, wd, shared, norm_w, cfg)
+    _same("dout", dout, x.shape, x.dtype, x.device)
+    a.dout, a.saved, a.saved_bytes = dout.data_ptr(), saved.data_ptr(), saved.numel()
+    operands = (x, router, wg, wu, wd, *shared, norm_w if cfg.get("norm_eps") is not None else None)
+    grads = tuple(torch.empty_like(t) if n and t is not None else None for t, n in zip(operands, need))
+    (a.dx, a.d_router, a.d_gate, a.d_up, a.d_down, a.d_shared_gate, a.d_shared_up, a.d_shared_down,
+     a.d_norm_weight) = (None if g is None else g.data_ptr() for g in grads)
+    a.workspace_bytes = lib.fs2moe_train_workspace_bytes(a, 1)
+    workspace = torch.empty(a.workspace_bytes, dtype=torch.uint8, device=x.device)
+    a.workspace = workspace.data_ptr()
+    _check(lib.fs2moe_train_backward(a, _stream()), "fs2moe_train_backward")
+    return grads

@@ -25,6 +25,11 @@ With the layer's RMS normalisation in front (``decoder_layer.py:187-191``) ``x``
 normalised rows ``xn`` that the router kernel wrote, and one more step turns their gradient into
 that of the raw rows and of the norm's weight                                  -> fs2moe_rms_norm_backward
 
+The layer as a whole runs these stages inside the library, a call per pass (``fs2moe_train_forward``,
+``fs2moe_train_backward``), with the weight gradients in one launch: called one by one from here, a
+step of 1000 to 3000 rows took the host longer than the GPU.  The stage-by-stage functions below serve
+what those calls do not take (another gate activation, matrices of 4 GB and more).
+
 The discrete selection (``torch.topk``) has no gradient, as in the reference.  Intermediates are
 rounded to the activation dtype between kernels, as autograd's would be.
 """
@@ -191,13 +196,40 @@ def backward_from(x, router, wg, wu, wd, sg, su, sd, saved, cfg, dout, need):
     return dx, d_router, d_wg, d_wu, d_wd, d_sg, d_su, d_sd
 
 
+def layer_forward(x, residual, router, wg, wu, wd, sg, su, sd, norm_w, cfg):
+    """``(out, saved)``: the whole forward pass in one library call (``saved`` then holds one buffer);
+    stage by stage for a gate activation other than SiLU and at the sizes that call does not take."""
+    if cfg.get("activation") is None:
+        done = _abi.train_forward(x, residual, router, wg, wu, wd, (sg, su, sd), norm_w, cfg)
+        if done is not None:
+            return done[0], (done[1],)
+    return forward_saving(x, residual, router, wg, wu, wd, sg, su, sd, cfg, norm_w)
+
+
+def layer_backward(x, router, wg, wu, wd, sg, su, sd, norm_w, cfg, saved, dout, need):
+    """Gradients ``(dx, d_router, d_wg, d_wu, d_wd, d_sg, d_su, d_sd, d_norm_w)`` (None where ``need``
+    says so) from what :func:`layer_forward` saved."""
+    dout = dout.contiguous()
+    if len(saved) == 1:
+        return _abi.train_backward(x, router, wg, wu, wd, (sg, su, sd), norm_w, cfg, saved[0], dout, need)
+    normed = cfg.get("norm_eps") is not None
+    # through the normalisation the rows' gradient is needed for the weight's as well
+    need_x = need[0] or (normed and need[8])
+    dx, *rest = backward_from(saved[12] if normed else x, router, wg, wu, wd, sg, su, sd, saved, cfg, dout,
+                              (need_x, *need[1:8]))
+    d_norm_w = None
+    if normed and dx is not None:
+        dx, d_norm_w = _abi.rms_norm_backward(x, norm_w, cfg["norm_eps"], dx, want_weight_grad=bool(need[8]))
+    return (dx if need[0] else None, *rest, d_norm_w)
+
+
 class MoEFunction(torch.autograd.Function):
     """``forward(x, residual, router, wg, wu, wd, sg, su, sd, norm_w, cfg)``; ``cfg`` carries the
     integers (and ``norm_eps`` when the rows are normalised first; ``norm_w`` may then still be None)."""
 
     @staticmethod
     def forward(ctx, x, residual, router, wg, wu, wd, sg, su, sd, norm_w, cfg):  # noqa: D102
-        out, saved = forward_saving(x, residual, router, wg, wu, wd, sg, su, sd, cfg, norm_w)
+        out, saved = layer_forward(x, residual, router, wg, wu, wd, sg, su, sd, norm_w, cfg)
         ctx.cfg = cfg
         ctx.has_residual = residual is not None
         ctx.save_for_backward(x, router, wg, wu, wd, sg, su, sd, norm_w, *saved)
@@ -208,20 +240,10 @@ class MoEFunction(torch.autograd.Function):
     def backward(ctx, dout):  # noqa: D102
         x, router, wg, wu, wd, sg, su, sd, norm_w, *saved = ctx.saved_tensors
         n = ctx.needs_input_grad
-        normed = ctx.cfg.get("norm_eps") is not None
-        # through the normalisation the rows' gradient is needed for the weight's as well
-        need = (n[0] or (normed and n[9]), n[2], n[3], n[4], n[5], n[6], n[7], n[8])
-        xn = saved[12]
-        dx, d_router, d_wg, d_wu, d_wd, d_sg, d_su, d_sd = backward_from(
-            xn if normed else x, router, wg, wu, wd, sg, su, sd, tuple(saved), ctx.cfg, dout, need)
-        d_norm_w = None
-        if normed and dx is not None:
-            dx, d_norm_w = _abi.rms_norm_backward(x, norm_w, ctx.cfg["norm_eps"], dx,
-                                                  want_weight_grad=bool(n[9]))
-            if not n[0]:
-                dx = None
+        need = (n[0], *n[2:10])
+        grads = layer_backward(x, router, wg, wu, wd, sg, su, sd, norm_w, ctx.cfg, tuple(saved), dout, need)
         d_res = dout if ctx.has_residual and n[1] else None
-        return dx, d_res, d_router, d_wg, d_wu, d_wd, d_sg, d_su, d_sd, d_norm_w, None
+        return grads[0], d_res, *grads[1:], None
 
 
 def _sum_rounded_once(a: Tensor, b: Tensor | None) -> Tensor:

@@ -31,161 +31,465 @@ namespace fs2moe {
 // (Chunks of twice the rows, a half per register set and one barrier per chunk, were slower: 277
 // against 244 us on 8 experts of 8192 rows.)  Rows past the expert's count are zero-filled,
 // experts without rows get a zero gradient.
+//
+// Blocks are persistent, one per CU, and a launch may hold several gradients (WgradJobs).  Their tiles
+// form one list: the gradients of one group (each slot a segment of its rows), then expert by expert all
+// grouped gradients, inside a gradient bands of BAND row blocks of C, row block minor.  A tile costs its
+// chunks and kTileCost more.  How the list is dealt depends on the largest tile:
+//   * at most a quarter of a block's fair share: eight equal shares by cost, one per XCD; the blocks of the
+//     XCD (block b runs on XCD b % 8) take the share's tiles in turn, so that at any time they work on
+//     neighbours, which share operand slabs in the XCD's L2 (shares of neighbours per block instead: 2170
+//     against 1750 us at 8 experts of 2048 rows, M 4096, N 14336);
+//   * larger (a few experts or one group hold most rows): the experts are sorted by their rows, the tiles
+//     above that quarter go out one per block in rounds that reverse direction, and the rest are cut into
+//     shares that fill each block up to a common level.
+// The chunks of a block's tiles form one stream: while the consumers write a tile out, the producers have
+// the next one's first three chunks on their way.  (A block per tile, started by the hardware, paid about
+// 10 us around its chunks.)
 namespace wgk {
 constexpr int TM = 256, TN = 256, CONSUMERS = 8, PRODUCERS = 4, WAVES = CONSUMERS + PRODUCERS;
-constexpr int SMEM_BYTES = 65536;  // two chunks of both operands
-}
-// what a load past the end of an operand reads
-__device__ __attribute__((aligned(16))) uint32_t kZero16[4] = {0u, 0u, 0u, 0u};  // (not const: a global address, so the loads stay global loads)
+constexpr int RK = 32;                                  // rows per chunk
+constexpr int ROWB = TM * 2;                            // bytes per LDS row
+constexpr int OPB = RK * ROWB;                          // bytes per operand chunk (16 KB)
+constexpr int RING_BYTES = 4 * OPB;                     // two chunks of both operands
+constexpr int LDE = 136;                                // epilogue: bytes between rows
+constexpr int EPI_BYTES = CONSUMERS * 32 * LDE;         // a 32 x 64 piece per consumer
+constexpr int MAX_BLOCKS = 512;
+constexpr int TABLE_INTS = 4 * FS2MOE_MAX_EXPERTS + 4 + MAX_BLOCKS;
+constexpr int SMEM_BYTES = RING_BYTES + EPI_BYTES + TABLE_INTS * 4;
+// What a tile costs besides its chunks, in chunks: starting its accumulators and writing 128 KB.
+constexpr int kTileCost = 5;
+constexpr int BAND = 8;
+constexpr int MAX_JOBS = 8;
+constexpr int kNonTemporal = 2;                         // in a buffer instruction's cache policy
+}  // namespace wgk
+// what a load through a row map reads past the end (not const: a global address, so the loads stay global
+// loads)
+static __device__ __attribute__((aligned(16))) uint32_t kZero16[4] = {0u, 0u, 0u, 0u};
 
-// MAPPED: A's rows are read through a_map.  A template parameter, not a test of the pointer: behind
-// a condition the map entry's load is waited for with every other load of the wave (the counter
+// One gradient: slots of rows, one per expert (grouped), or segments of seg_rows rows of one group, whose
+// f32 sums go to `partial` [slots, M, N] when it is not null.
+struct WgradJob {
+  const uint16_t *A, *B;
+  uint16_t* C;
+  float* partial;
+  int M, N, m_tiles, tiles;  // tiles: per slot
+  int grouped, slots, seg_rows, rows;
+  int past_cache;  // store C past the caches (see nt_stores)
+};
+struct WgradJobs {
+  WgradJob job[wgk::MAX_JOBS];
+  int n;
+};
+
+// MAPPED: A's rows are read through a_map (one job).  A template parameter, not a test of the pointer:
+// behind a condition the map entry's load is waited for with every other load of the wave (the counter
 // cannot tell them apart at the join), which serialises a chunk's loads into round trips.
 template <bool MAPPED>
 __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
-    const uint16_t* __restrict__ A, const int32_t* __restrict__ a_map, int lda,
-    const uint16_t* __restrict__ B, int ldb, uint16_t* __restrict__ C, int M, int N, Groups g,
-    int m_tiles, int n_tiles, int seg_rows, float* __restrict__ partial, int paired) {
+    const WgradJobs jobs, const int32_t* __restrict__ a_map, const int32_t* __restrict__ counts,
+    const int32_t* __restrict__ offsets, int E) {
   using namespace wgk;
-  using T = uint16_t;
-  constexpr int RK = 32;                          // rows per chunk
-  constexpr int VEC = 8;                          // elements per 16-byte chunk
-  constexpr int ROW_CHUNKS = TM / VEC;            // 16-byte chunks per LDS row (32)
+  constexpr int ROW_CHUNKS = TM / 8;              // 16-byte chunks per LDS row (32)
   constexpr int PLANES = PRODUCERS * 64;          // lanes that move data
   constexpr int PER_THREAD = RK * ROW_CHUNKS / PLANES;  // chunks per producer lane and operand (4)
-  constexpr int ROWB = TM * sizeof(T);            // bytes per LDS row (512)
-  constexpr int OPB = RK * ROWB;                  // bytes per operand chunk (16 KB)
-  static_assert(4 * OPB == SMEM_BYTES, "two chunks of two operands");
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  int32_t* s_cnt = reinterpret_cast<int32_t*>(smem + RING_BYTES + EPI_BYTES);
+  int32_t* s_off = s_cnt + FS2MOE_MAX_EXPERTS;
+  int32_t* s_exp = s_off + FS2MOE_MAX_EXPERTS;    // expert of list position
+  int32_t* s_pre = s_exp + FS2MOE_MAX_EXPERTS;    // [E + 1]: chunks + kTileCost of the positions before
+  int32_t* s_cap = s_pre + FS2MOE_MAX_EXPERTS + 4;
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // Which tile: slots (an expert, by rank as below, or a segment of the one group's rows) in launch
-  // order, and within a slot row block minor: blocks reach the 8 XCDs round-robin (block b runs on
-  // XCD b % 8, each with its own L2), so with 8 row blocks the tiles of a slot that share an XCD
-  // share their block of A's columns.
-  const int per_e = m_tiles * n_tiles;
-  int slot, mt, nt;
-  if (paired) {
-    // Two slots share 2 per_e consecutive blocks, i.e. (per_e being a multiple of 4) whole rounds
-    // of the 8 XCDs: four XCDs per slot, each taking a quarter of the row blocks (or of the column
-    // blocks) with all blocks of the other kind, so that a slot's operand slabs are fetched by 4
-    // L2s with 5 slabs each instead of by 8 with 4 each.  Which half of the XCDs takes the pair's
-    // larger slot alternates from pair to pair.
-    const int pair = blockIdx.x / (2 * per_e);
-    const int i = blockIdx.x - pair * 2 * per_e;
-    const int xcd = i & 7, j = i >> 3, x4 = xcd & 3;
-    slot = 2 * pair + (((xcd >> 2) ^ pair) & 1);
-    if (m_tiles % 4 == 0) {
-      const int q = m_tiles / 4;
-      mt = x4 * q + j % q;
-      nt = j / q;
-    } else {
-      const int q = n_tiles / 4;
-      nt = x4 * q + j % q;
-      mt = j / q;
-    }
-    if (slot >= g.E) return;  // the partner of the last of an odd number of slots
-  } else {
-    slot = blockIdx.x / per_e;
-    const int rem = blockIdx.x - slot * per_e;
-    nt = rem / m_tiles;
-    mt = rem - nt * m_tiles;
-  }
-  const int m0 = mt * TM, n0 = nt * TN;
-  const bool dense = g.counts == nullptr;
-  // Grouped: the experts are taken in descending order of their row counts (ties: lower index
-  // first), so that the longest chains of chunks start first and the short ones fill the end of the
-  // launch.  Every block finds the expert of its rank itself: a thread per expert, one comparison loop over
-  // the E counts (the block has 768 threads, the library's limit is 512 experts).
-  // One group: the rows are cut into segments of seg_rows, one slot each, whose partial sums go to
-  // `partial` [segments, M, N] in f32 for wgrad_reduce_kernel to add in order.
-  int e = 0, off, cnt;
-  if (dense) {
-    off = slot * seg_rows;
-    cnt = g.dense_rows - off < seg_rows ? g.dense_rows - off : seg_rows;
-  } else {
-    __shared__ int s_expert, s_cnt[FS2MOE_MAX_EXPERTS], s_off[FS2MOE_MAX_EXPERTS];
-    const int mine = tid < g.E ? g.counts[tid] : 0;
-    if (tid < g.E) {
-      s_cnt[tid] = mine;
-      s_off[tid] = g.offsets[tid];  // with the counts: not a second round trip once the expert is known
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  __shared__ int s_wave_tot[WAVES], s_wave_max[WAVES];
+  // The experts' tables in the order of `pos` (position of expert tid), and the prefix sums of their costs.
+  const int my_cnt = counts != nullptr && tid < E ? counts[tid] : 0;
+  const int my_off = counts != nullptr && tid < E ? offsets[tid] : 0;
+  auto tables = [&](int pos) {
+    if (tid < E) {
+      s_cnt[pos] = my_cnt;
+      s_off[pos] = my_off;
+      s_exp[pos] = tid;
     }
     __syncthreads();
-    if (tid < g.E) {
-      int rank = 0;
-      for (int j = 0; j < g.E; ++j) {
-        const int cj = s_cnt[j];
-        rank += (cj > mine || (cj == mine && j < tid)) ? 1 : 0;
+    const int cost = tid < E ? (s_cnt[tid] + RK - 1) / RK + kTileCost : 0;
+    int incl = cost, most = cost;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int v = __shfl_up(incl, off, kWave);
+      if (lane >= off) incl += v;
+    }
+    most = (int)wave_max_u32((uint32_t)most);
+    if (lane == 63) {
+      s_wave_tot[wave] = incl;
+      s_wave_max[wave] = most;
+    }
+    __syncthreads();
+    int base = 0;
+    for (int w = 0; w < wave; ++w) base += s_wave_tot[w];
+    if (tid < E) {
+      s_pre[tid] = base + incl - cost;
+      if (tid == E - 1) s_pre[E] = base + incl;
+    }
+    __syncthreads();
+  };
+  if (counts != nullptr) tables(tid);
+  // (a 64-bit division is some 150 instructions, and nearly every cost fits 32 bits)
+  auto divide = [](int64_t n, int64_t d) -> int64_t {
+    if (((n | d) >> 31) == 0) return (uint32_t)n / (uint32_t)d;
+    return n / d;
+  };
+  // ---- the list: `dense` tiles of the gradients of one group, then those of the experts: gradient by
+  // gradient (expert by expert the rows of three gradients, rather than two operands of one, would compete
+  // for L2: 958 against 880 us for the gradients of 128 experts of 512 rows, 2048 x 768), or `per` tiles
+  // for each expert where the experts are taken in the order of their sizes
+  // (all segments of a gradient but the last have seg_rows rows)
+  auto seg_cost = [&](const WgradJob& j, int slot) {
+    const int left = j.rows - slot * j.seg_rows;
+    return ((left < j.seg_rows ? left : j.seg_rows) + RK - 1) / RK + kTileCost;
+  };
+  int dense = 0, per = 0, most = 0;
+  int64_t dense_cost = 0;
+  for (int i = 0; i < jobs.n; ++i) {
+    const WgradJob& j = jobs.job[i];
+    if (j.grouped) {
+      per += j.tiles;
+      continue;
+    }
+    const int c = seg_cost(j, 0);
+    dense += j.slots * j.tiles;
+    dense_cost += ((int64_t)(j.slots - 1) * c + seg_cost(j, j.slots - 1)) * j.tiles;
+    most = c > most ? c : most;
+  }
+  if (per > 0)
+    for (int w = 0; w < WAVES; ++w) most = s_wave_max[w] > most ? s_wave_max[w] : most;
+  const int64_t total = dense_cost + (per > 0 ? (int64_t)s_pre[E] * per : 0);
+  bool by_expert = false;
+  // The number of tiles whose middle lies before cost x of the list: where a share from x on begins.
+  auto tiles_before = [&](int64_t x) -> int {
+    int tiles = 0, tiles_of = per, cost;
+    if (x < dense_cost) {
+      for (int i = 0;; ++i) {
+        const WgradJob& j = jobs.job[i];
+        if (j.grouped) continue;
+        const int c = seg_cost(j, 0), last = seg_cost(j, j.slots - 1);
+        const int64_t all = ((int64_t)(j.slots - 1) * c + last) * j.tiles;
+        if (x >= all) {
+          x -= all;
+          tiles += j.slots * j.tiles;
+          continue;
+        }
+        int slot = (int)divide(x, (int64_t)c * j.tiles);
+        slot = slot < j.slots - 1 ? slot : j.slots - 1;
+        x -= (int64_t)slot * c * j.tiles;
+        tiles += slot * j.tiles;
+        tiles_of = j.tiles;
+        cost = slot < j.slots - 1 ? c : last;
+        break;
       }
-      if (rank == slot) s_expert = tid;
+    } else {
+      x -= dense_cost;
+      tiles = dense;
+      if (per == 0 || x >= (int64_t)s_pre[E] * per) return dense + E * per;
+      if (!by_expert)
+        for (int i = 0;; ++i) {
+          const WgradJob& j = jobs.job[i];
+          if (!j.grouped) continue;
+          tiles_of = j.tiles;
+          const int64_t all = (int64_t)s_pre[E] * tiles_of;
+          if (x < all) break;
+          x -= all;
+          tiles += E * tiles_of;
+        }
+      const int col = (int)divide(x, tiles_of);  // s_pre[pos] * tiles_of <= x  <=>  s_pre[pos] <= col
+      int pos = 0;
+      for (int e0 = 0; e0 < E; e0 += 64) {
+        const int e = e0 + lane;
+        const unsigned long long m = __ballot(e < E && s_pre[e] <= col && col < s_pre[e + 1]);
+        if (m) pos = e0 + (int)__builtin_ctzll(m);
+      }
+      pos = __builtin_amdgcn_readfirstlane(pos);
+      x -= (int64_t)s_pre[pos] * tiles_of;
+      tiles += pos * tiles_of;
+      cost = s_pre[pos + 1] - s_pre[pos];
+    }
+    // tile t of these begins at t cost; its middle lies before x for 2 t + 1 < 2 x / cost
+    const int64_t t = divide(2 * x + cost - 1, 2 * (int64_t)cost);
+    return tiles + (int)(t < tiles_of ? t : tiles_of);
+  };
+  // The block's tiles: `rounds` of one of the first `big` tiles each, then first, first + stride, ..
+  struct Deal {
+    int slot, grid, rounds, big, round, next_t, end, stride;
+    __device__ int next() {  // -1: no more
+      while (round < rounds) {
+        const int r = round++, p = r * grid + ((r & 1) ? grid - 1 - slot : slot);
+        if (p < big) return p;
+      }
+      if (next_t >= end) return -1;
+      const int t = next_t;
+      next_t += stride;
+      return t;
+    }
+  };
+  Deal deal;
+  deal.grid = (int)gridDim.x;
+  const int xcd = blockIdx.x & 7;
+  deal.slot = xcd * (deal.grid >> 3) + (int)(blockIdx.x >> 3);
+  deal.round = deal.rounds = deal.big = 0;
+  const int64_t fair = divide(total, deal.grid);
+  if (dense + (int64_t)E * per <= deal.grid) {
+    deal.big = dense + E * per;  // at most one tile each
+    deal.rounds = 1;
+    deal.next_t = deal.end = 0;
+    deal.stride = 1;
+  } else if (most * 4ll <= fair) {
+    deal.next_t = tiles_before(total * xcd / 8) + (int)(blockIdx.x >> 3);
+    deal.end = tiles_before(total * (xcd + 1) / 8);
+    deal.stride = deal.grid >> 3;
+  } else {
+    by_expert = true;
+    if (per > 0) {
+      // sort the experts by their rows, largest first (ties: lower index first)
+      int rank = 0;
+      for (int j = 0; j < E; ++j) {
+        const int cj = s_cnt[j];
+        rank += (cj > my_cnt || (cj == my_cnt && j < tid)) ? 1 : 0;
+      }
+      __syncthreads();
+      tables(rank);
+    }
+    // the large tiles: all of one group (as large as any expert's, mostly), and the experts whose tiles
+    // are above a quarter of the fair share
+    int large = 0;
+    if (per > 0) {
+      for (int e0 = 0; e0 < E; e0 += 64) {
+        const int e = e0 + lane;
+        large += __popcll(__ballot(e < E && (s_pre[e + 1] - s_pre[e]) * 4ll > fair));
+      }
+    }
+    deal.big = dense + large * per;
+    deal.rounds = (deal.big + deal.grid - 1) / deal.grid;
+    const int64_t big_cost = dense_cost + (large > 0 ? (int64_t)s_pre[large] * per : 0);
+    // the load of every block (by slot) after the rounds
+    for (int sl = tid; sl < deal.grid; sl += WAVES * 64) {
+      int load = 0;
+      for (int r = 0; r < deal.rounds; ++r) {
+        const int p = r * deal.grid + ((r & 1) ? deal.grid - 1 - sl : sl);
+        if (p >= deal.big) continue;
+        if (p >= dense) {
+          const int pos = (p - dense) / per;
+          load += s_pre[pos + 1] - s_pre[pos];
+        } else {
+          int q = p, i = 0;
+          for (;; ++i) {
+            const WgradJob& j = jobs.job[i];
+            if (j.grouped) continue;
+            if (q < j.slots * j.tiles) {
+              load += seg_cost(j, q / j.tiles);
+              break;
+            }
+            q -= j.slots * j.tiles;
+          }
+        }
+      }
+      s_cap[sl] = load;
     }
     __syncthreads();
-    e = s_expert;
-    off = s_off[e];
-    cnt = s_cnt[e];
+    // The level L that the remaining cost fills the blocks to, L = (rest + loads below L) / (blocks below
+    // L): from all blocks on, dropping those above, until none is; then this block's part of what lies
+    // between the loads and L.  Every wave for itself, lane l holding the loads of slots 8 l .. 8 l + 7.
+    const int64_t rest = total - big_cost;
+    constexpr int PL = MAX_BLOCKS / 64;
+    int load[PL];
+#pragma unroll
+    for (int i = 0; i < PL; ++i) load[i] = PL * lane + i < deal.grid ? s_cap[PL * lane + i] : 0x7fffffff;
+    int level = 0x7ffffffe;
+    for (int below = deal.grid + 1;;) {
+      int n = 0, sum = 0;
+#pragma unroll
+      for (int i = 0; i < PL; ++i)
+        if (load[i] <= level) {
+          ++n;
+          sum += load[i];
+        }
+      n = wave_sum_i32(n);
+      if (n == below) break;
+      below = n;
+      level = (int)divide(rest + wave_sum_i32(sum) + n - 1, n);
+    }
+    int mine = 0, before = 0;  // room of this lane's slots, and of those before this block's
+#pragma unroll
+    for (int i = 0; i < PL; ++i) {
+      const int r = load[i] <= level ? level - load[i] : 0;
+      if (PL * lane + i < deal.slot) before += r;
+      if (PL * lane + i == deal.slot) mine = r;
+    }
+    const int64_t from = wave_sum_i32(before), to = from + wave_sum_i32(mine);
+    deal.next_t = tiles_before(big_cost + (from < rest ? from : rest));
+    deal.end = tiles_before(big_cost + (to < rest ? to : rest));
+    deal.stride = 1;
   }
+  deal.next_t = __builtin_amdgcn_readfirstlane(deal.next_t);
+  deal.end = __builtin_amdgcn_readfirstlane(deal.end);
+
+  // Wave-uniform parameters of a tile.
+  struct Tile {
+    int job, slot, off, cnt, m0, n0;
+  };
+  auto locate = [&](int t) {
+    Tile r;
+    int pos = 0;
+    const bool grouped = t >= dense;
+    if (grouped) {
+      t -= dense;
+      if (by_expert) {
+        pos = t / per;
+        t -= pos * per;
+      }
+    }
+    for (r.job = 0;; ++r.job) {
+      const WgradJob& j = jobs.job[r.job];
+      if ((j.grouped != 0) != grouped) continue;
+      const int n = grouped && by_expert ? j.tiles : j.slots * j.tiles;
+      if (t < n) break;
+      t -= n;
+    }
+    const WgradJob& j = jobs.job[r.job];
+    if (grouped && !by_expert) {
+      pos = t / j.tiles;
+      t -= pos * j.tiles;
+    }
+    if (grouped) {
+      r.slot = __builtin_amdgcn_readfirstlane(s_exp[pos]);
+      r.off = __builtin_amdgcn_readfirstlane(s_off[pos]);
+      r.cnt = __builtin_amdgcn_readfirstlane(s_cnt[pos]);
+    } else {
+      r.slot = t / j.tiles;
+      t -= r.slot * j.tiles;
+      r.off = r.slot * j.seg_rows;
+      r.cnt = j.rows - r.off < j.seg_rows ? j.rows - r.off : j.seg_rows;
+    }
+    const int n_tiles = j.tiles / j.m_tiles, band = t / (BAND * n_tiles);
+    const int i = t - band * BAND * n_tiles, left = j.m_tiles - band * BAND;
+    const int high = left < BAND ? left : BAND, nt = i / high;
+    r.m0 = (band * BAND + i - nt * high) * TM;
+    r.n0 = nt * TN;
+    return r;
+  };
+
+  if (wave >= CONSUMERS) {
+    // ---- producers: chunk g of the block's stream goes to LDS buffer g & 1 through register set g & 1;
+    // while chunk g is multiplied, chunk g + 1 goes into the other buffer (read last during chunk g - 1:
+    // the barrier that ended it has passed), chunk g + 3 is loaded into the set this frees, and chunk
+    // g + 2 is still on its way in the other set.  Every load and store is unconditional (what lies past
+    // a tile's rows or columns, or past the stream's end, loads zeros: an offset outside the buffer):
+    // behind a condition the compiler cannot count the loads in flight, and waits for all of them, the
+    // other set's included, before a store.
+    const int ptid = tid - CONSUMERS * 64;
+    const int kr = ptid / ROW_CHUNKS, ch = ptid % ROW_CHUNKS;  // rows kr + 8 i, chunk ch
+    u32x4 ra[2][PER_THREAD], rb[2][PER_THREAD];
+    // the chunk to load next: rows [ld_off, ld_off + ld_left) of the tile's operands
+    const uint16_t* ld_a = nullptr;
+    const uint16_t* ld_b = nullptr;
+    const int32_t* ld_map = a_map;
+    int ld_left = 0, ld_lda = 0, ld_ldb = 0;
+    Deal ld_deal = deal;
+    uint32_t oa[PER_THREAD], ob[PER_THREAD];
+    int loaded = 0;  // chunks so far (those past the stream's end do not count)
+    auto next_tile = [&]() {
+      // (tiles without rows have no chunks)
+      ld_left = 0;
+      for (int n; ld_left == 0 && (n = ld_deal.next()) >= 0;) {
+        const Tile t = locate(n);
+        if (t.cnt == 0) continue;
+        const WgradJob& j = jobs.job[t.job];
+        ld_lda = j.M;
+        ld_ldb = j.N;
+        ld_a = (MAPPED ? j.A : j.A + (size_t)t.off * j.M) + t.m0;
+        ld_b = j.B + (size_t)t.off * j.N + t.n0;
+        if (MAPPED) ld_map = a_map + t.off;
+        ld_left = t.cnt;
+        const bool a_ok = t.m0 + ch * 8 < j.M, b_ok = t.n0 + ch * 8 < j.N;
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i) {
+          oa[i] = a_ok ? (uint32_t)(((kr + 8 * i) * j.M + ch * 8) * 2) : 0xfffffff0u;
+          ob[i] = b_ok ? (uint32_t)(((kr + 8 * i) * j.N + ch * 8) * 2) : 0xfffffff0u;
+        }
+      }
+    };
+    auto load_chunk = [&](auto set_c) {
+      constexpr int set = decltype(set_c)::value;
+      if (ld_left <= 0) next_tile();
+      loaded += ld_left > 0 ? 1 : 0;
+      const __amdgpu_buffer_rsrc_t b_rsrc =
+          __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(ld_b), 0, 0xfffffff0u, 0x00020000);
+      if constexpr (MAPPED) {  // all the map entries first, then all the rows
+        int row[PER_THREAD];
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i) {
+          const int k = kr + 8 * i;
+          row[i] = ld_left > 0 ? ld_map[k < ld_left ? k : ld_left - 1] : 0;
+        }
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i) {
+          const bool in = kr + 8 * i < ld_left;
+          const uint16_t* p = in && oa[i] != 0xfffffff0u ? ld_a + (size_t)row[i] * ld_lda + ch * 8
+                                                         : reinterpret_cast<const uint16_t*>(kZero16);
+          ra[set][i] = *reinterpret_cast<const u32x4*>(p);
+          rb[set][i] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, in ? ob[i] : 0xfffffff0u, 0, 0);
+        }
+        ld_map += RK;
+      } else {
+        const __amdgpu_buffer_rsrc_t a_rsrc =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(ld_a), 0, 0xfffffff0u, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i) {
+          const bool in = kr + 8 * i < ld_left;
+          ra[set][i] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, in ? oa[i] : 0xfffffff0u, 0, 0);
+          rb[set][i] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, in ? ob[i] : 0xfffffff0u, 0, 0);
+        }
+        ld_a += (size_t)RK * ld_lda;
+      }
+      ld_b += (size_t)RK * ld_ldb;
+      ld_left -= RK;
+    };
+    auto store_chunk = [&](auto set_c, int buf) {
+      constexpr int set = decltype(set_c)::value;
+      uint8_t* sA = smem + buf * 2 * OPB;
+      uint8_t* sB = sA + OPB;
+#pragma unroll
+      for (int i = 0; i < PER_THREAD; ++i) {
+        // chunk ch of row k sits in slot ch ^ ((k & 3) << 2), so that the four consecutive rows a
+        // transposing read touches lie 64 bytes apart
+        const int k = kr + 8 * i, at = k * ROWB + ((ch ^ ((k & 3) << 2)) * 16);
+        *reinterpret_cast<u32x4*>(sA + at) = ra[set][i];
+        *reinterpret_cast<u32x4*>(sB + at) = rb[set][i];
+      }
+    };
+    using Set0 = std::integral_constant<int, 0>;
+    using Set1 = std::integral_constant<int, 1>;
+    load_chunk(Set0{});
+    if (loaded == 0) return;  // no tile with rows: nothing for the consumers to wait for
+    load_chunk(Set1{});
+    store_chunk(Set0{}, 0);
+    load_chunk(Set0{});
+    lds_barrier();
+    auto step = [&](int g, auto next_set) {
+      store_chunk(next_set, (g + 1) & 1);
+      load_chunk(next_set);
+      lds_barrier();  // the loads of the next chunks stay in flight
+    };
+    for (int g = 0; g < loaded; g += 2) {  // (a step's load is three chunks ahead: `loaded` is final in time)
+      step(g, Set1{});
+      if (g + 1 < loaded) step(g + 1, Set0{});
+    }
+    return;  // the consumers write the tiles
+  }
+
+  // ---- consumers
   const int wm = wave & 1, wn = (wave >> 1) & 3;  // a consumer's 128 (m) x 64 (n) part of the tile
-  const bool producer = wave >= CONSUMERS;
-  const int ptid = tid - CONSUMERS * 64;  // a producer lane's index among the PLANES
   const int lr = lane & 31, lk = lane >> 5;
-
-  f32x16 acc[2][4];  // [tn][tm]
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
-
-  // Loads are unconditional; what lies past the expert's rows or the matrix's columns is read from
-  // 16 zero bytes instead (the address is selected, not the data: any instruction on the loaded
-  // registers other than the LDS store gets scheduled early and waits for the load there).
-  // Two sets of registers in the producers, so that two chunks are on their way from memory at any
-  // time (one chunk's loads take about as long as its MFMAs do: with a single set every chunk waited
-  // for its loads).
-  u32x4 ra[2][PER_THREAD], rb[2][PER_THREAD];
-  const T* zero_src = reinterpret_cast<const T*>(kZero16);
-  auto load_chunk = [&](auto set_c, int r0) {
-    constexpr int set = decltype(set_c)::value;
-    int rr[PER_THREAD], arow[PER_THREAD];
-#pragma unroll
-    for (int i = 0; i < PER_THREAD; ++i) {
-      const int r = r0 + (ptid + PLANES * i) / ROW_CHUNKS;
-      rr[i] = off + (r < cnt ? r : cnt - 1);  // cnt > 0 here
-      arow[i] = rr[i];
-    }
-    if constexpr (MAPPED) {  // all the map entries first, then all the rows
-#pragma unroll
-      for (int i = 0; i < PER_THREAD; ++i) arow[i] = a_map[rr[i]];
-    }
-#pragma unroll
-    for (int i = 0; i < PER_THREAD; ++i) {
-      const int c = ptid + PLANES * i;
-      const int k = c / ROW_CHUNKS, ch = c % ROW_CHUNKS;
-      const bool row_ok = r0 + k < cnt;
-      const bool a_ok = row_ok && m0 + ch * VEC < M, b_ok = row_ok && n0 + ch * VEC < N;
-      const T* pa = a_ok ? A + (size_t)arow[i] * lda + m0 + ch * VEC : zero_src;
-      const T* pb = b_ok ? B + (size_t)rr[i] * ldb + n0 + ch * VEC : zero_src;
-      ra[set][i] = *reinterpret_cast<const u32x4*>(pa);
-      rb[set][i] = *reinterpret_cast<const u32x4*>(pb);
-    }
-  };
-  auto store_chunk = [&](auto set_c, int buf) {
-    constexpr int set = decltype(set_c)::value;
-    uint8_t* sA = smem + buf * 2 * OPB;
-    uint8_t* sB = sA + OPB;
-#pragma unroll
-    for (int i = 0; i < PER_THREAD; ++i) {
-      const int c = ptid + PLANES * i;
-      const int k = c / ROW_CHUNKS, ch = c % ROW_CHUNKS;
-      // chunk ch of row k sits in slot ch ^ ((k & 3) << 2), so that the four consecutive rows a
-      // transposing read touches lie 64 bytes apart
-      const int slot = ch ^ ((k & 3) << 2);
-      *reinterpret_cast<u32x4*>(sA + k * ROWB + slot * 16) = ra[set][i];
-      *reinterpret_cast<u32x4*>(sB + k * ROWB + slot * 16) = rb[set][i];
-    }
-  };
-
   // fragment address of the 32 columns from cbase on, rows 8 lk .. 8 lk + 3 (+4 for the upper half)
   auto tr_addr = [&](int cbase) {
     const int s = lane & 15, half = (lane >> 4) & 1;
@@ -195,12 +499,11 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
   };
   int fa[4], fb[2];
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
-    fa[t] = tr_addr(wm * 128 + t * 32);
+  for (int t = 0; t < 4; ++t) fa[t] = tr_addr(wm * 128 + t * 32);
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
-    fb[t] = tr_addr(wn * 64 + t * 32);
+  for (int t = 0; t < 2; ++t) fb[t] = tr_addr(wn * 64 + t * 32);
 
+  f32x16 acc[2][4];  // [tn][tm]
   auto compute_chunk = [&](int buf) {
     const uint8_t* sA = smem + buf * 2 * OPB;
     const uint8_t* sB = sA + OPB;
@@ -227,99 +530,92 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
               __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[tn], af[tm], acc[tn][tm], 0, 0, 0);
     }
   };
-
-  // Chunk i is multiplied from LDS buffer i & 1 while chunk i + 1 goes from register set (i + 1) & 1
-  // into the other buffer (read last during chunk i - 1: the barrier that ended it has passed), chunk
-  // i + 3 is loaded into the set this frees, and chunk i + 2 is still on its way in the other set.
-  const int chunks = (cnt + RK - 1) / RK;
-  using Set0 = std::integral_constant<int, 0>;
-  using Set1 = std::integral_constant<int, 1>;
-  // Every load and store of the loop is unconditional (chunks past the last one load clamped rows
-  // and store zeros into the buffer nobody reads any more): behind a condition the compiler cannot
-  // count the loads in flight, and waits for all of them, the other set's included, before a store.
-  if (producer) {
-    if (chunks > 0) {
-      load_chunk(Set0{}, 0);
-      load_chunk(Set1{}, RK);
-      store_chunk(Set0{}, 0);
-      load_chunk(Set0{}, 2 * RK);
-      lds_barrier();
-    }
-    auto step = [&](int i, auto next_set) {
-      store_chunk(next_set, (i + 1) & 1);
-      load_chunk(next_set, (i + 3) * RK);
-      lds_barrier();  // the loads of the next chunks stay in flight
-    };
-    int ci = 0;
-    for (; ci + 1 < chunks; ci += 2) {
-      step(ci, Set1{});
-      step(ci + 1, Set0{});
-    }
-    if (ci < chunks) step(ci, Set1{});
-    return;  // the consumers write the tile
-  }
-  if (chunks > 0) lds_barrier();
-  for (int i = 0; i < chunks; ++i) {
-    compute_chunk(i & 1);
-    lds_barrier();
-  }
-
   // Accumulator layout: the lane holds row m = lr of fragment tm and columns 8 q + 4 lk + {0..3} of
   // fragment tn in registers 4 q .. 4 q + 3.
-  T* Ce = C + (size_t)e * M * N;
-  float* Pe = partial != nullptr ? partial + (size_t)slot * M * N : nullptr;
-  if (Pe == nullptr) {
-    // Through LDS (free after the loop's last barrier), so that a store instruction writes 8 rows
-    // of 128 contiguous bytes instead of 32 rows of 16: the wave puts a 32 (m) x 64 (n) fragment
-    // row into its own 4.25 KB as bf16, rows 136 bytes apart, and reads it back 16 bytes per lane.
-    constexpr int LDE = 136;
-    uint8_t* sw = smem + wave * 8192;
-    const int rrow = lane >> 3, rcol = lane & 7;
+  auto write_tile = [&](const Tile& tl) {
+    const WgradJob& j = jobs.job[tl.job];
+    const int M = j.M, N = j.N;
+    if (j.partial == nullptr) {
+      // Through the wave's own piece of LDS, so that a store instruction writes 8 rows of 128 contiguous
+      // bytes instead of 32 rows of 16: a 32 (m) x 64 (n) fragment row as bf16, rows 136 bytes apart,
+      // read back 16 bytes per lane.
+      const __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          j.C + (size_t)tl.slot * M * N + (size_t)tl.m0 * N + tl.n0, 0, 0xfffffff0u, 0x00020000);
+      uint8_t* sw = smem + RING_BYTES + wave * 32 * LDE;
+      const int rrow = lane >> 3, rcol = lane & 7;
+#pragma unroll
+      for (int tm = 0; tm < 4; ++tm) {
+#pragma unroll
+        for (int tn = 0; tn < 2; ++tn)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            u32x2 o = {pack_bf16x2(acc[tn][tm][4 * q], acc[tn][tm][4 * q + 1]),
+                       pack_bf16x2(acc[tn][tm][4 * q + 2], acc[tn][tm][4 * q + 3])};
+            *reinterpret_cast<u32x2*>(sw + lr * LDE + (tn * 32 + 8 * q + 4 * lk) * 2) = o;
+          }
+        // the wave's own LDS traffic runs in order; the compiler must not move the reads (other
+        // lanes' data) above the writes, nor the next round's writes above these reads
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        const int n = tl.n0 + wn * 64 + rcol * 8;
+#pragma unroll
+        for (int p8 = 0; p8 < 4; ++p8) {
+          const int row = p8 * 8 + rrow;
+          const u32x2 lo = *reinterpret_cast<const u32x2*>(sw + row * LDE + rcol * 16);
+          const u32x2 hi = *reinterpret_cast<const u32x2*>(sw + row * LDE + rcol * 16 + 8);
+          const int m = tl.m0 + wm * 128 + tm * 32 + row;
+          if (m < M && n < N) {  // N is a multiple of 8: the eight columns are in or out together
+            u32x4 o = {lo[0], lo[1], hi[0], hi[1]};
+            // (two plain stores of which one is marked non-temporal the compiler merges into one that is not)
+            const int at = ((m - tl.m0) * N + n - tl.n0) * 2;
+            if (j.past_cache)
+              __builtin_amdgcn_raw_buffer_store_b128(o, c_rsrc, at, 0, kNonTemporal);
+            else
+              __builtin_amdgcn_raw_buffer_store_b128(o, c_rsrc, at, 0, 0);
+          }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+      return;
+    }
+    float* Pe = j.partial + (size_t)tl.slot * M * N;
 #pragma unroll
     for (int tm = 0; tm < 4; ++tm) {
+      const int m = tl.m0 + wm * 128 + tm * 32 + lr;
+      if (m >= M) continue;
 #pragma unroll
-      for (int tn = 0; tn < 2; ++tn)
+      for (int tn = 0; tn < 2; ++tn) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          u32x2 o = {pack_bf16x2(acc[tn][tm][4 * q], acc[tn][tm][4 * q + 1]),
-                     pack_bf16x2(acc[tn][tm][4 * q + 2], acc[tn][tm][4 * q + 3])};
-          *reinterpret_cast<u32x2*>(sw + lr * LDE + (tn * 32 + 8 * q + 4 * lk) * 2) = o;
-        }
-      // the wave's own LDS traffic runs in order; the compiler must not move the reads (other
-      // lanes' data) above the writes, nor the next round's writes above these reads
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      const int n = n0 + wn * 64 + rcol * 8;
-#pragma unroll
-      for (int p8 = 0; p8 < 4; ++p8) {
-        const int row = p8 * 8 + rrow;
-        const u32x2 lo = *reinterpret_cast<const u32x2*>(sw + row * LDE + rcol * 16);
-        const u32x2 hi = *reinterpret_cast<const u32x2*>(sw + row * LDE + rcol * 16 + 8);
-        const int m = m0 + wm * 128 + tm * 32 + row;
-        if (m < M && n < N) {  // N is a multiple of 8: the eight columns are in or out together
-          u32x4 o = {lo[0], lo[1], hi[0], hi[1]};
-          *reinterpret_cast<u32x4*>(Ce + (size_t)m * N + n) = o;
+          const int n = tl.n0 + wn * 64 + tn * 32 + 8 * q + 4 * lk;
+          if (n >= N) continue;  // N is a multiple of 4: the four columns are in or out together
+          f32x4 o = {acc[tn][tm][4 * q], acc[tn][tm][4 * q + 1], acc[tn][tm][4 * q + 2],
+                     acc[tn][tm][4 * q + 3]};
+          *reinterpret_cast<f32x4*>(Pe + (size_t)m * N + n) = o;
         }
       }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
-    return;
-  }
+  };
+  bool started = false;
+  int buf = 0;
+  for (int n; (n = deal.next()) >= 0;) {
+    const Tile tl = locate(n);
 #pragma unroll
-  for (int tm = 0; tm < 4; ++tm) {
-    const int m = m0 + wm * 128 + tm * 32 + lr;
-    if (m >= M) continue;
+    for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int tn = 0; tn < 2; ++tn) {
+      for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = n0 + wn * 64 + tn * 32 + 8 * q + 4 * lk;
-        if (n >= N) continue;  // N is a multiple of 4: the four columns are in or out together
-        const float v0 = acc[tn][tm][4 * q], v1 = acc[tn][tm][4 * q + 1];
-        const float v2 = acc[tn][tm][4 * q + 2], v3 = acc[tn][tm][4 * q + 3];
-        f32x4 o = {v0, v1, v2, v3};
-        *reinterpret_cast<f32x4*>(Pe + (size_t)m * N + n) = o;
-      }
+        for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
+    const int chunks = (tl.cnt + RK - 1) / RK;
+    if (chunks > 0 && !started) {
+      lds_barrier();
+      started = true;
     }
+    for (int i = 0; i < chunks; ++i) {
+      compute_chunk(buf);
+      buf ^= 1;
+      lds_barrier();
+    }
+    write_tile(tl);
   }
 }
 
@@ -619,7 +915,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void router_backward_kernel(
     const float* __restrict__ logits, const int32_t* __restrict__ topk_idx,
     const float* __restrict__ topk_w, const float* __restrict__ d_w, int Tn, int E, int K,
-    int score_fn, int renormalize, T* __restrict__ dlogits) {
+    int score_fn, int renormalize, T* __restrict__ dlogits, int ld) {
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= Tn) return;
   const int lane = threadIdx.x & 63;
@@ -668,8 +964,9 @@ __global__ __launch_bounds__(256) void router_backward_kernel(
       const float p = __expf(l[e] - mx) / den;
       dl = p * ((sel ? dw : 0.f) - dot);
     }
-    Elem<T>::store(dlogits + (size_t)t * E + e, dl);
+    Elem<T>::store(dlogits + (size_t)t * ld + e, dl);
   }
+  for (int e = E + lane; e < ld; e += 64) Elem<T>::store(dlogits + (size_t)t * ld + e, 0.f);
 }
 
 }  // namespace fs2moe
@@ -684,6 +981,61 @@ static int wgrad_segments(int64_t rows, int M, int N) {
   const int64_t most = rows / 256;  // at least 256 rows per segment
   s = s < most ? s : most;
   return s >= 2 ? (int)s : 1;
+}
+
+// A gradient is written once and not read here, and as ordinary stores its lines push the operands' rows,
+// which other tiles read again, out of L2: 128 experts of 256 rows, 2048 x 768, 207 us with ordinary and
+// 186 us with non-temporal stores (bf16).  Rows that do not begin on a 128-byte line leave parts of lines,
+// which are better merged in the caches unless the gradient is larger than these (16 experts, 1024 x 1368:
+// 43 against 50 us).
+static int nt_stores(int64_t slots, int64_t M, int64_t N) {
+  return N % 64 == 0 || slots * M * N * 2 > (256ll << 20);
+}
+
+// Rows of each of (at most) *segments segments, a multiple of 16; *segments becomes how many that makes,
+// none of them empty.
+static int segment_rows(int64_t rows, int* segments) {
+  const int64_t per = ((rows + *segments - 1) / *segments + 15) / 16 * 16;
+  if (rows > 0) *segments = (int)((rows + per - 1) / per);
+  return (int)per;
+}
+
+static int launch_wgrad_reduce(const float* partial, int segments, int64_t n, int dtype, void* dw,
+                               hipStream_t st) {
+  const unsigned blocks = (unsigned)((n / 4 + 255) / 256);
+  if (dtype == FS2MOE_BF16)
+    hipLaunchKernelGGL(wgrad_reduce_kernel<uint16_t>, dim3(blocks), dim3(256), 0, st, partial, segments, n,
+                       static_cast<uint16_t*>(dw));
+  else
+    hipLaunchKernelGGL(wgrad_reduce_kernel<float>, dim3(blocks), dim3(256), 0, st, partial, segments, n,
+                       static_cast<float*>(dw));
+  return check_launch("wgrad_reduce");
+}
+
+// One launch for all gradients of `jobs`; the grouped ones share counts and offsets.
+static int launch_wgrad(const WgradJobs& jobs, const int32_t* a_map, const int32_t* counts,
+                        const int32_t* offsets, int E, hipStream_t st) {
+  auto k = a_map != nullptr ? grouped_wgrad_kernel<true> : grouped_wgrad_kernel<false>;
+  static bool attr_set = false;  // benign race: setting the attribute is idempotent
+  if (!attr_set) {
+    for (const void* p : {reinterpret_cast<const void*>(grouped_wgrad_kernel<false>),
+                          reinterpret_cast<const void*>(grouped_wgrad_kernel<true>)}) {
+      hipError_t e = hipFuncSetAttribute(p, hipFuncAttributeMaxDynamicSharedMemorySize, wgk::SMEM_BYTES);
+      if (e != hipSuccess) {
+        set_error("grouped_wgrad: cannot reserve %d bytes of LDS: %s", wgk::SMEM_BYTES, hipGetErrorString(e));
+        return FS2MOE_ERR_LAUNCH;
+      }
+    }
+    attr_set = true;
+  }
+  const int cus = cu_count_by_xcd(), blocks = cus < wgk::MAX_BLOCKS ? cus : wgk::MAX_BLOCKS;
+  if (blocks == 0) {
+    set_error("grouped_wgrad: cannot query the compute-unit count");
+    return FS2MOE_ERR_LAUNCH;
+  }
+  hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(wgk::WAVES * 64), wgk::SMEM_BYTES, st, jobs, a_map,
+                     counts, offsets, E);
+  return check_launch("grouped_wgrad");
 }
 
 extern "C" int64_t fs2moe_grouped_wgrad_workspace_bytes(int32_t grouped, int32_t M, int32_t N,
@@ -722,37 +1074,20 @@ extern "C" int fs2moe_grouped_wgrad(const void* a, const int32_t* a_row_map, con
     }
     if (workspace == nullptr || workspace_bytes < (int64_t)segments * M * N * 4) segments = 1;
   }
+  const int seg_rows = segment_rows(max_rows, &segments);
   const int slots = counts != nullptr ? E : segments;
-  const int seg_rows = (int)(((max_rows + segments - 1) / segments + 15) / 16 * 16);
   float* partial = segments > 1 ? static_cast<float*>(workspace) : nullptr;
-  // grouped, the tile grid divides over four XCDs, and there are enough experts for the two halves
-  // of the XCDs to get the same work over all pairs (with 8 skewed experts they did not: Mixtral's
-  // gradients took 9 % longer): slots in pairs (see the kernel)
-  const int paired = counts != nullptr && E >= 32 && (m_tiles % 4 == 0 || n_tiles % 4 == 0) ? 1 : 0;
-  const int64_t blocks = (int64_t)(paired ? (slots + 1) / 2 * 2 : slots) * m_tiles * n_tiles;
-  FS2_REQUIRE(blocks <= 0x7fffffffll, "grouped_wgrad: too many tiles");
+  FS2_REQUIRE((int64_t)slots * m_tiles * n_tiles <= 0x7fffffffll, "grouped_wgrad: too many tiles");
   Groups g{counts, offsets, E, (int)max_rows};
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool mapped = a_row_map != nullptr;
   if (dtype == FS2MOE_BF16) {
-    auto k = mapped ? grouped_wgrad_kernel<true> : grouped_wgrad_kernel<false>;
-    static bool attr_set = false;  // benign race: setting the attribute is idempotent
-    if (!attr_set) {
-      for (const void* p : {reinterpret_cast<const void*>(grouped_wgrad_kernel<false>),
-                            reinterpret_cast<const void*>(grouped_wgrad_kernel<true>)}) {
-        hipError_t e = hipFuncSetAttribute(p, hipFuncAttributeMaxDynamicSharedMemorySize, wgk::SMEM_BYTES);
-        if (e != hipSuccess) {
-          set_error("grouped_wgrad: cannot reserve %d bytes of LDS: %s", wgk::SMEM_BYTES,
-                    hipGetErrorString(e));
-          return FS2MOE_ERR_LAUNCH;
-        }
-      }
-      attr_set = true;
-    }
-    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(wgk::WAVES * 64), wgk::SMEM_BYTES, st,
-                       static_cast<const uint16_t*>(a), a_row_map, M,
-                       static_cast<const uint16_t*>(b), N, static_cast<uint16_t*>(dw), M, N, g,
-                       m_tiles, n_tiles, seg_rows, partial, paired);
+    WgradJobs jobs;
+    jobs.n = 1;
+    jobs.job[0] = {static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b),
+                   static_cast<uint16_t*>(dw), partial, M, N, m_tiles, m_tiles * n_tiles,
+                   counts != nullptr, slots, seg_rows, (int)max_rows, nt_stores(slots, M, N)};
+    if (int rc = launch_wgrad(jobs, a_row_map, counts, offsets, E, st)) return rc;
   } else {
     const int64_t big = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
     const bool small = f32t::small_tiles(big * slots, 128);
@@ -765,17 +1100,82 @@ extern "C" int fs2moe_grouped_wgrad(const void* a, const int32_t* a_row_map, con
                        static_cast<float*>(dw), M, N, g, mt, nt, seg_rows, partial);
   }
   if (int rc = check_launch("grouped_wgrad")) return rc;
-  if (segments > 1) {
-    const int64_t n = (int64_t)M * N;
-    const unsigned rblocks = (unsigned)((n / 4 + 255) / 256);
-    if (dtype == FS2MOE_BF16)
-      hipLaunchKernelGGL(wgrad_reduce_kernel<uint16_t>, dim3(rblocks), dim3(256), 0, st, partial,
-                         segments, n, static_cast<uint16_t*>(dw));
-    else
-      hipLaunchKernelGGL(wgrad_reduce_kernel<float>, dim3(rblocks), dim3(256), 0, st, partial,
-                         segments, n, static_cast<float*>(dw));
-    return check_launch("wgrad_reduce");
+  return segments > 1 ? launch_wgrad_reduce(partial, segments, (int64_t)M * N, dtype, dw, st) : FS2MOE_OK;
+}
+
+int64_t fs2moe::wgrad_plan(WgradRequest* r, int n, int32_t E, int64_t grouped_rows, int64_t rows,
+                           int32_t dtype) {
+  if (dtype == FS2MOE_F32) {  // (one launch each: every single group is cut as in fs2moe_grouped_wgrad)
+    int64_t most = 0;
+    for (int i = 0; i < n; ++i) {
+      const int64_t b = r[i].grouped ? 0 : fs2moe_grouped_wgrad_workspace_bytes(0, r[i].M, r[i].N, rows);
+      most = b > most ? b : most;
+    }
+    return most;
   }
+  auto tiles = [](const WgradRequest& q) {
+    return (int64_t)((q.M + wgk::TM - 1) / wgk::TM) * ((q.N + wgk::TN - 1) / wgk::TN);
+  };
+  const int64_t one = rows / wgk::RK + wgk::kTileCost;
+  int64_t total = 0;
+  for (int i = 0; i < n; ++i)
+    total += tiles(r[i]) * (r[i].grouped ? grouped_rows / wgk::RK + (int64_t)E * wgk::kTileCost : one);
+  const int64_t fair = total / 256 + 1;
+  int64_t bytes = 0;
+  for (int i = 0; i < n; ++i) {
+    r[i].segments = 1;
+    if (r[i].grouped || one <= fair) continue;
+    // at least 256 rows each, and no more than gives every CU a tile of this gradient
+    int64_t s = (one + fair - 1) / fair;
+    const int64_t by_rows = rows / 256, by_cus = 256 / tiles(r[i]) + 1;
+    s = s < by_rows ? s : by_rows;
+    s = s < by_cus ? s : by_cus;
+    if (s < 2) continue;
+    r[i].segments = (int)s;
+    bytes += s * r[i].M * r[i].N * 4;
+  }
+  return bytes;
+}
+
+int fs2moe::wgrad_all(const WgradRequest* r, int n, const int32_t* counts, const int32_t* offsets,
+                      int32_t E, int64_t grouped_rows, int64_t rows, int32_t dtype, void* scratch,
+                      void* stream) {
+  if (dtype == FS2MOE_F32) {
+    for (int i = 0; i < n; ++i) {
+      const bool g = r[i].grouped;
+      const int64_t ws = g ? 0 : fs2moe_grouped_wgrad_workspace_bytes(0, r[i].M, r[i].N, rows);
+      if (int rc = fs2moe_grouped_wgrad(r[i].a, nullptr, r[i].b, g ? counts : nullptr, g ? offsets : nullptr,
+                                        g ? E : 1, r[i].M, r[i].N, g ? grouped_rows : rows, dtype, r[i].dw,
+                                        ws > 0 ? scratch : nullptr, ws, stream))
+        return rc;
+    }
+    return FS2MOE_OK;
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  FS2_REQUIRE(n <= wgk::MAX_JOBS, "wgrad: internal: %d gradients", n);
+  WgradJobs jobs;
+  jobs.n = n;
+  float* part = static_cast<float*>(scratch);
+  bool any_grouped = false;
+  for (int i = 0; i < n; ++i) {
+    const WgradRequest& q = r[i];
+    const int mt = (q.M + wgk::TM - 1) / wgk::TM, nt = (q.N + wgk::TN - 1) / wgk::TN;
+    any_grouped = any_grouped || q.grouped;
+    int segments = q.grouped ? 1 : q.segments;
+    const int seg = segment_rows(rows, &segments), slots = q.grouped ? E : segments;
+    jobs.job[i] = {static_cast<const uint16_t*>(q.a), static_cast<const uint16_t*>(q.b),
+                   static_cast<uint16_t*>(q.dw), !q.grouped && slots > 1 ? part : nullptr, q.M, q.N, mt, mt * nt,
+                   q.grouped ? 1 : 0, slots, q.grouped ? 0 : seg, (int)rows, nt_stores(slots, q.M, q.N)};
+    if (!q.grouped && slots > 1) part += (int64_t)slots * q.M * q.N;
+  }
+  if (int rc = launch_wgrad(jobs, nullptr, any_grouped ? counts : nullptr, any_grouped ? offsets : nullptr,
+                            any_grouped ? E : 0, st))
+    return rc;
+  for (int i = 0; i < n; ++i)
+    if (jobs.job[i].partial != nullptr)
+      if (int rc = launch_wgrad_reduce(jobs.job[i].partial, jobs.job[i].slots, (int64_t)r[i].M * r[i].N, dtype,
+                                       r[i].dw, st))
+        return rc;
   return FS2MOE_OK;
 }
 
@@ -846,16 +1246,24 @@ extern "C" int fs2moe_router_backward(const float* logits, const int32_t* topk_i
   FS2_REQUIRE(score_fn == FS2MOE_SCORE_SIGMOID || score_fn == FS2MOE_SCORE_SOFTMAX,
               "router_backward: score_fn %d", score_fn);
   if (T == 0) return FS2MOE_OK;
+  return router_backward_ld(logits, topk_idx, topk_w, d_w, T, E, K, score_fn, renormalize, dtype, dlogits, E,
+                            stream);
+}
+
+int fs2moe::router_backward_ld(const float* logits, const int32_t* topk_idx, const float* topk_w,
+                               const float* d_w, int32_t T, int32_t E, int32_t K, int32_t score_fn,
+                               int32_t renormalize, int32_t dtype, void* dlogits, int32_t ld,
+                               void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
   const unsigned blocks = (unsigned)((T + 3) / 4);
   if (dtype == FS2MOE_BF16)
     hipLaunchKernelGGL(router_backward_kernel<uint16_t>, dim3(blocks), dim3(256), 0, st, logits,
                        topk_idx, topk_w, d_w, T, E, K, score_fn, renormalize,
-                       static_cast<uint16_t*>(dlogits));
+                       static_cast<uint16_t*>(dlogits), ld);
   else
     hipLaunchKernelGGL(router_backward_kernel<float>, dim3(blocks), dim3(256), 0, st, logits,
                        topk_idx, topk_w, d_w, T, E, K, score_fn, renormalize,
-                       static_cast<float*>(dlogits));
+                       static_cast<float*>(dlogits), ld);
   return check_launch("router_backward");
 }
 

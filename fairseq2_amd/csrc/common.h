@@ -128,6 +128,20 @@ __device__ __forceinline__ float wave_sum_f32(float v) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ int dpp_add_step_i32(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROW_MASK, 0xf, false);
+}
+__device__ __forceinline__ int wave_sum_i32(int v) {
+  v = dpp_add_step_i32<kDppXor1, 0xf>(v);
+  v = dpp_add_step_i32<kDppXor2, 0xf>(v);
+  v = dpp_add_step_i32<kDppHalfMirror, 0xf>(v);
+  v = dpp_add_step_i32<kDppMirror, 0xf>(v);
+  v = dpp_add_step_i32<kDppBcast15, 0xa>(v);
+  v = dpp_add_step_i32<kDppBcast31, 0xc>(v);
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 // ---- MFMA operand fragments from LDS ---------------------------------------------------------------
 // Plain: the lane's 8 consecutive k values lie contiguously (k-contiguous tile).
 // Transposing: the tile is n-contiguous; ds_read_tr16_b64 hands lane i of each 16-lane group element
@@ -172,6 +186,20 @@ void set_error(const char* fmt, ...);
 int check_launch(const char* what);
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+// Compute units of the current device, rounded down to a multiple of its 8 XCDs (0 on failure).
+inline int cu_count_by_xcd() {
+  static int cached = 0;  // benign race: every thread computes the same value
+  if (cached == 0) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        cus < 8)
+      return 0;
+    cached = cus / 8 * 8;
+  }
+  return cached;
+}
+
 inline int elem_size(int dtype) { return dtype == FS2MOE_F32 ? 4 : dtype == FS2MOE_BF16 ? 2 : 1; }
 
 // Where the whole-layer call wants its dispatch (no rows copied): with at most 32 bf16 tokens the
@@ -233,6 +261,36 @@ int grouped_swiglu_scaled_rows(const void* x, const int32_t* row_map, const floa
                                const void* w_up, const void* w_down, int32_t E, int32_t D, int32_t F,
                                int64_t max_rows, void* h, void* ye, int32_t rows_per_expert,
                                void* stream);
+
+// ---- pieces of a training step (fs2moe_train_forward / fs2moe_train_backward)
+// Whether the SwiGLU pair keeps its two products at these sizes, and that pair (E 0: one group of `rows`
+// rows with nn.Linear-oriented weights).
+bool swiglu_train_applies(int32_t dtype, int32_t D, int32_t F, int64_t rows);
+int swiglu_train(const void* x, const int32_t* counts, const int32_t* offsets, int32_t E,
+                 const void* w_gate, const void* w_up, const void* w_down, int32_t D, int32_t F,
+                 int64_t rows, int32_t dtype, void* g, void* u, void* h, void* y, void* stream);
+// c = a1 @ B1 + a2 @ B2 (fs2moe_grouped_gemm's layouts and groups; E 0: one group), one rounding.
+int gemm_sum(const void* a1, const void* b1, const void* a2, const void* b2, int32_t layout,
+             const int32_t* counts, const int32_t* offsets, int32_t E, int32_t K, int32_t N,
+             int64_t rows, int32_t dtype, void* c, void* stream);
+// One of several weight gradients taken together: grouped (over the experts' rows) or over all `rows` of
+// one group.
+struct WgradRequest {
+  const void *a, *b;
+  void* dw;
+  int32_t M, N;
+  bool grouped;
+  int segments;  // set by wgrad_plan: of a group's rows, each with its own partial sums
+};
+// Cuts the rows of single groups whose tiles would take longer than the others together; returns the
+// bytes of scratch that the partial sums need.
+int64_t wgrad_plan(WgradRequest* r, int n, int32_t E, int64_t grouped_rows, int64_t rows, int32_t dtype);
+int wgrad_all(const WgradRequest* r, int n, const int32_t* counts, const int32_t* offsets, int32_t E,
+              int64_t grouped_rows, int64_t rows, int32_t dtype, void* scratch, void* stream);
+// fs2moe_router_backward into rows of ld >= E elements, those past E zero
+int router_backward_ld(const float* logits, const int32_t* topk_idx, const float* topk_w,
+                       const float* d_w, int32_t T, int32_t E, int32_t K, int32_t score_fn,
+                       int32_t renormalize, int32_t dtype, void* dlogits, int32_t ld, void* stream);
 
 }  // namespace fs2moe
 

@@ -189,20 +189,6 @@ __global__ __launch_bounds__(256, 2) void glu_gemm_bf16_kernel(
 }
 
 // ------------------------------------------------------------------------------------ host
-// Compute units of the current device, rounded down to a multiple of its 8 XCDs (0 on failure).
-static int cu_count_by_xcd() {
-  static int cached = 0;  // benign race: every thread computes the same value
-  if (cached == 0) {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        cus < 8)
-      return 0;
-    cached = cus / 8 * 8;
-  }
-  return cached;
-}
-
 // One launch of the f32 kernel; a2, g_keep, u_keep may be null.
 template <bool DUAL, int BLAYOUT>
 static int launch_f32(const void* a, const void* b0, const void* b1, const void* a2, void* c,
@@ -803,6 +789,53 @@ extern "C" int fs2moe_grouped_gemm_sum(const void* a1, const void* b1, const voi
   return launch_dma<false, FS2MOE_W_OUT_IN, false, true>(
       a1, nullptr, K, b1, b2, a2, nullptr, c, N, Groups{counts, offsets, E, (int)max_rows}, max_rows,
       "glu_gemm_bf16_dma<two sources>", static_cast<hipStream_t>(stream));
+}
+
+bool fs2moe::swiglu_train_applies(int32_t dtype, int32_t D, int32_t F, int64_t rows) {
+  return dtype == FS2MOE_F32 || dma_offsets_fit(rows, D, F);
+}
+
+int fs2moe::swiglu_train(const void* x, const int32_t* counts, const int32_t* offsets, int32_t E,
+                         const void* w_gate, const void* w_up, const void* w_down, int32_t D,
+                         int32_t F, int64_t rows, int32_t dtype, void* g, void* u, void* h, void* y,
+                         void* stream) {
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const Groups grp{E > 0 ? counts : nullptr, E > 0 ? offsets : nullptr, E > 0 ? E : 1, (int)rows};
+  if (dtype == FS2MOE_BF16) {
+    if (E > 0)
+      return launch_dma_pair<FS2MOE_W_IN_OUT>(x, nullptr, grp, rows, w_gate, w_up, w_down, nullptr, nullptr,
+                                              nullptr, D, F, h, y, st, g, u);
+    return launch_dma_pair<FS2MOE_W_OUT_IN>(x, nullptr, grp, rows, w_gate, w_up, w_down, nullptr, nullptr,
+                                            nullptr, D, F, h, y, st, g, u);
+  }
+  int rc = E > 0 ? launch_f32<true, FS2MOE_W_IN_OUT>(x, w_gate, w_up, nullptr, h, g, u, D, F, grp, rows,
+                                                     "glu_gemm_f32<gate,up>", st)
+                 : launch_f32<true, FS2MOE_W_OUT_IN>(x, w_gate, w_up, nullptr, h, g, u, D, F, grp, rows,
+                                                     "glu_gemm_f32<gate,up>", st);
+  if (rc) return rc;
+  return E > 0 ? launch_f32<false, FS2MOE_W_IN_OUT>(h, w_down, nullptr, nullptr, y, nullptr, nullptr, F, D,
+                                                    grp, rows, "glu_gemm_f32<down>", st)
+               : launch_f32<false, FS2MOE_W_OUT_IN>(h, w_down, nullptr, nullptr, y, nullptr, nullptr, F, D,
+                                                    grp, rows, "glu_gemm_f32<down>", st);
+}
+
+int fs2moe::gemm_sum(const void* a1, const void* b1, const void* a2, const void* b2, int32_t layout,
+                     const int32_t* counts, const int32_t* offsets, int32_t E, int32_t K, int32_t N,
+                     int64_t rows, int32_t dtype, void* c, void* stream) {
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const Groups g{E > 0 ? counts : nullptr, E > 0 ? offsets : nullptr, E > 0 ? E : 1, (int)rows};
+  // (the second activation matrix travels in the first scale argument, the second weights in B1)
+  if (dtype == FS2MOE_BF16)
+    return layout == FS2MOE_W_IN_OUT
+               ? launch_dma<false, FS2MOE_W_IN_OUT, false, true>(a1, nullptr, K, b1, b2, a2, nullptr, c, N, g,
+                                                                 rows, "glu_gemm_bf16_dma<two sources>", st)
+               : launch_dma<false, FS2MOE_W_OUT_IN, false, true>(a1, nullptr, K, b1, b2, a2, nullptr, c, N, g,
+                                                                 rows, "glu_gemm_bf16_dma<two sources>", st);
+  return layout == FS2MOE_W_IN_OUT
+             ? launch_f32<false, FS2MOE_W_IN_OUT>(a1, b1, b2, a2, c, nullptr, nullptr, K, N, g, rows,
+                                                  "glu_gemm_f32<two sources>", st)
+             : launch_f32<false, FS2MOE_W_OUT_IN>(a1, b1, b2, a2, c, nullptr, nullptr, K, N, g, rows,
+                                                  "glu_gemm_f32<two sources>", st);
 }
 
 extern "C" int fs2moe_dense_swiglu(const void* x, const void* w_gate, const void* w_up,

@@ -127,7 +127,7 @@ struct TileOrder {
 // to bf16 and laid out like C, for a backward pass that would otherwise compute them again.  Their
 // destinations arrive in S0 and S1, which bf16 weights leave unused: two more arguments cost every
 // other variant of the kernel registers in its main loop (1-2.5 % of the layer, measured).
-// TWO_SRC (single matrix, (out, in) bf16 weights): C = A @ B0_e^T + A2 @ B1_e^T, the second pair
+// TWO_SRC (single matrix, bf16 weights): C = A @ B0_e + A2 @ B1_e, the second pair
 // walked after the first into the same accumulators (Kdim is one pair's).  A2 arrives in S0, for the
 // reason given above.
 // KTAIL (bf16 weights): Kdim is a multiple of 8 but not of the unit's 64.  A tile's last unit then
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
   constexpr bool FP8 = BLAYOUT == W_FP8_TILED;
   static_assert(!KEEP_GU || (DUAL && !FP8), "the products are kept by the bf16 gate/up kernel only");
   static_assert(!KTAIL || !FP8, "e4m3 weight tiles hold whole units");
-  static_assert(!TWO_SRC || (!DUAL && BLAYOUT == FS2MOE_W_OUT_IN), "two sources: one (out, in) matrix each");
+  static_assert(!TWO_SRC || (!DUAL && !FP8), "two sources: one bf16 matrix each");
   constexpr int BN = DUAL ? 128 : 256;    // real channels per tile
   constexpr int BROW = DUAL ? 256 : 512;  // bytes per LDS row of a weight sub-tile (in x out)
   constexpr bool KN = BLAYOUT == FS2MOE_W_IN_OUT;
@@ -453,8 +453,8 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const size_t k0 = ((size_t)ku * 2 + h) * BK * N;
-          const uint8_t* bg = reinterpret_cast<const uint8_t*>(ld_bg + k0);
-          const uint8_t* bu = reinterpret_cast<const uint8_t*>(ld_bu + k0);
+          const uint8_t* bg = reinterpret_cast<const uint8_t*>((second ? ld_bu : ld_bg) + k0);
+          const uint8_t* bu = TWO_SRC ? bg : reinterpret_cast<const uint8_t*>(ld_bu + k0);
           // pieces q, q+4 (gate when DUAL) and q+8, q+12 (up when DUAL)
 #pragma unroll
           for (int i = 0; i < 4; ++i)
@@ -553,8 +553,8 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
             const size_t k0 = ((size_t)ku * 2 + h) * BK * N;
-            const uint8_t* bg = reinterpret_cast<const uint8_t*>(ld_bg + k0);
-            const uint8_t* bu = reinterpret_cast<const uint8_t*>(ld_bu + k0);
+            const uint8_t* bg = reinterpret_cast<const uint8_t*>((second ? ld_bu : ld_bg) + k0);
+            const uint8_t* bu = TWO_SRC ? bg : reinterpret_cast<const uint8_t*>(ld_bu + k0);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               *reinterpret_cast<u32x4*>(dst + A_BYTES + (4 * h + i) * 4096) = stage[8 + 4 * h + i];

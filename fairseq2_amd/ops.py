@@ -90,18 +90,14 @@ def moe_backward(
 ) -> list[Tensor]:
     """Gradients of ``moe_forward`` for ``x``, ``router``, the three expert weights, (when given)
     the three shared-expert weights and (when given) the norm's weight, in that order."""
-    from fairseq2_amd.autograd import backward_from, forward_saving
+    from fairseq2_amd.autograd import layer_backward, layer_forward
 
     cfg = dict(num_experts=num_experts, top_k=top_k, tile_m=tile_m, score_fn=score_fn,
                renormalize=renormalize, scale_input=scale_input, router_bias=router_bias,
                norm_eps=norm_eps if normed else None, router_t=_abi.router_expert_major(router))
-    _, saved = forward_saving(x, None, router, w_gate, w_up, w_down, shared_gate, shared_up,
-                              shared_down, cfg, norm_weight)
-    grads = list(backward_from(saved[12] if normed else x, router, w_gate, w_up, w_down, shared_gate,
-                               shared_up, shared_down, saved, cfg, grad_out, (True,) * 8))
-    if normed:
-        grads[0], d_norm_w = _abi.rms_norm_backward(x, norm_weight, norm_eps, grads[0])
-        grads.append(d_norm_w)
+    weights = (router, w_gate, w_up, w_down, shared_gate, shared_up, shared_down, norm_weight, cfg)
+    _, saved = layer_forward(x, None, *weights)
+    grads = layer_backward(x, *weights, saved, grad_out, (True,) * 9)
     return [g for g in grads if g is not None]
 
 

@@ -455,6 +455,47 @@ int fs2moe_rms_norm_backward(const void* x, const void* weight, float eps, const
                              int32_t T, int32_t D, int32_t dtype, void* dx, void* dweight,
                              void* workspace, int64_t workspace_bytes, void* stream);
 
+/*
+ * A training step of the layer in two calls, one per pass: the stages above in their order, on two
+ * buffers of the caller's (what autograd would keep between the passes, and scratch).  SiLU gate,
+ * weights in the activation dtype.  What the stage calls do one at a time is done together where that
+ * saves a launch or a pass over memory: all weight gradients in one launch (bf16), the gather of the
+ * output gradients with the gradients of the combine weights, the two halves of each input gradient
+ * into one result; and the gate and up products are kept for every size and type.
+ *
+ * `saved` is written by the forward call and read by the backward call (which leaves it as it is);
+ * `workspace` is scratch of either.  Both 256-byte aligned, of the bytes that
+ * fs2moe_train_saved_bytes / fs2moe_train_workspace_bytes return for the sizes in the struct and, for
+ * the backward pass (backward 1, else 0), the gradients whose pointers are set (-1: sizes these calls do not take -- bf16 matrices of 4 GB and more).
+ *   normed       the rows are RMS-normalised first (norm_weight [D] or NULL, norm_eps)
+ *   router       (D, E); router_read: what the forward pass reads, the same or, with
+ *                FS2MOE_ROUTER_OUT_IN or-ed into score_fn, its (E, D) copy
+ *   shared_*     NULL without a shared expert (F_shared 0)
+ *   forward:     out [T, D] = [residual +] MoE([RMSNorm](x))
+ *   backward:    dout [T, D] -> dx [T, D] (through the normalisation), d_router (D, E), d_gate / d_up
+ *                (E*D, F), d_down (E*F, D), d_shared_* and d_norm_weight; a NULL one is not computed.
+ *                The residual's gradient is dout itself and is not added to dx.
+ */
+typedef struct fs2moe_train_args {
+  int32_t T, D, E, K, F, F_shared, tile_m, act_dtype;
+  int32_t score_fn, renormalize, scale_input, normed;
+  float norm_eps;
+  int32_t reserved;
+  const void *x, *norm_weight, *residual, *router, *router_read;
+  const float* router_bias;
+  const void *w_gate, *w_up, *w_down, *shared_gate, *shared_up, *shared_down;
+  void *saved, *workspace;
+  int64_t saved_bytes, workspace_bytes;
+  void* out;
+  const void* dout;
+  void *dx, *d_router, *d_gate, *d_up, *d_down, *d_shared_gate, *d_shared_up, *d_shared_down,
+      *d_norm_weight;
+} fs2moe_train_args;
+int64_t fs2moe_train_saved_bytes(const fs2moe_train_args* sizes);
+int64_t fs2moe_train_workspace_bytes(const fs2moe_train_args* sizes, int32_t backward);
+int fs2moe_train_forward(const fs2moe_train_args* args, void* stream);
+int fs2moe_train_backward(const fs2moe_train_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

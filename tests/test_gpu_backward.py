@@ -154,6 +154,47 @@ def test_f32_products_at_the_edges_of_their_tiles(gpu_device, rows, k, n):
         assert_grad_close(dw[ex], a[sl].cpu().double().t() @ d[sl].cpu().double(), "fp32", f"expert {ex}, weight gradient")
 
 
+# The step in two library calls against the same step stage by stage: sizes at which the weight gradients'
+# tiles are dealt in each of the three ways (no more tiles than CUs; many, of similar cost; some experts
+# much larger), with the shared expert's and the router's rows cut into segments, and without.
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("t,d,e,k,f,f_shared,skew,scale_input,normed", [
+    (17, 64, 3, 1, 40, 0, 0.0, True, False), (700, 256, 6, 2, 128, 264, 0.0, True, True),
+    (1500, 512, 64, 4, 520, 0, 0.0, False, False), (2500, 520, 60, 4, 256, 512, 2.0, False, True),
+    (1100, 1024, 4, 2, 1032, 1024, 3.0, True, False),
+])
+def test_step_in_two_calls_against_its_stages(gpu_device, dtype, t, d, e, k, f, f_shared, skew, scale_input, normed):
+    from fairseq2_amd import autograd as A
+
+    _say("two calls", dtype, t, d, e, k, f, f_shared, skew, scale_input, normed)
+    g = torch.Generator().manual_seed(t + e)
+    mk = lambda *s, scale=1.0: (scale * torch.randn(*s, generator=g)).to(TORCH_DTYPE[dtype]).to(gpu_device)  # noqa: E731
+    x, res, dout, router = mk(t, d), mk(t, d), mk(t, d), mk(d, e, scale=d**-0.5)
+    ws = [mk(e * d, f, scale=d**-0.5), mk(e * d, f, scale=d**-0.5), mk(e * f, d, scale=f**-0.5)]
+    ws += [mk(f_shared, d, scale=d**-0.5), mk(f_shared, d, scale=d**-0.5), mk(d, f_shared, scale=f_shared**-0.5)] \
+        if f_shared else [None] * 3
+    norm_w = mk(d) if normed else None
+    bias = (-skew * torch.log(1.0 + torch.arange(e))).to(gpu_device) if skew else None
+    cfg = dict(num_experts=e, top_k=k, tile_m=16, score_fn=_abi.SCORE_SOFTMAX, renormalize=False,
+               scale_input=scale_input, router_bias=bias, norm_eps=1e-6 if normed else None)
+    out, saved = A.layer_forward(x, res, router, *ws, norm_w, cfg)
+    assert len(saved) == 1
+    grads = A.layer_backward(x, router, *ws, norm_w, cfg, saved, dout, (True,) * 9)
+    out_ref, saved_ref = A.forward_saving(x, res, router, *ws, cfg, norm_w)
+    refs = A.layer_backward(x, router, *ws, norm_w, cfg, saved_ref, dout, (True,) * 9)
+    assert torch.equal(out, out_ref)
+    names = ("x", "router", "gate", "up", "down", "shared gate", "shared up", "shared down", "norm weight")
+    for name, got, ref in zip(names, grads, refs):
+        assert (got is None) == (ref is None), name
+        if got is not None:
+            assert_grad_close(got, ref.cpu(), dtype, f"d {name}", blocks=e if name in ("gate", "up", "down") else 1)
+    # a subset: the same numbers, whatever else is asked for
+    some = A.layer_backward(x, router, *ws, norm_w, cfg, saved, dout, (False, True, False, False, True) + (False,) * 4)
+    assert [n for n, v in zip(names, some) if v is not None] == ["router", "down"]
+    assert_grad_close(some[1], grads[1].cpu(), dtype, "d router alone")
+    assert torch.equal(some[4], grads[4])
+
+
 @pytest.mark.parametrize("rows,k,n", [([5, 0, 300, 64, 1, 700], 192, 128), ([130, 257], 64, 72), ([0, 0, 9], 128, 256)])
 def test_grouped_gemm_sum_adds_two_products(gpu_device, rows, k, n):
     """``a1 @ B1^T + a2 @ B2^T`` in one kernel against f64, and against the two products apart."""
