@@ -353,6 +353,38 @@ extern "C" int fs2moe_forward_norm(const void* x, const void* norm_weight, float
                       workspace, workspace_bytes, out, stream);
 }
 
+extern "C" int fs2moe_forward_call(const fs2moe_forward_args* a, void* stream) {
+  FS2_REQUIRE(a != nullptr, "forward_call: null pointer");
+  return forward_impl(true, a->normed != 0, a->x, a->norm_weight, a->norm_eps, a->residual, a->router,
+                      a->router_bias, a->w_gate, a->w_up, a->w_down, a->s_gate, a->s_up, a->s_down,
+                      a->shared_gate, a->shared_up, a->shared_down, a->T, a->D, a->E, a->K, a->F, a->F_shared,
+                      a->tile_m, a->act_dtype, a->w_dtype, a->score_fn, a->renormalize, a->scale_input,
+                      a->workspace, a->workspace_bytes, a->out, stream);
+}
+
+// A kernel, where a device-to-device hipMemcpyAsync is a blit kernel between barriers of its own: in
+// front of a graph's first kernel 2.3 us instead of 5.4.
+namespace {
+__global__ __launch_bounds__(256) void copy_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
+                                                   int64_t vec, int64_t bytes) {
+  const int64_t stride = (int64_t)gridDim.x * 256, first = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  for (int64_t i = first; i < vec; i += stride)
+    reinterpret_cast<fs2moe::u32x4*>(dst)[i] = reinterpret_cast<const fs2moe::u32x4*>(src)[i];
+  for (int64_t i = vec * 16 + first; i < bytes; i += stride) dst[i] = src[i];
+}
+}  // namespace
+
+extern "C" int fs2moe_copy(const void* src, void* dst, int64_t bytes, void* stream) {
+  FS2_REQUIRE(bytes >= 0 && (bytes == 0 || (src && dst)), "copy: bad arguments");
+  if (bytes == 0 || src == dst) return FS2MOE_OK;
+  const int64_t vec = fs2moe::aligned16(src) && fs2moe::aligned16(dst) ? bytes / 16 : 0;
+  const int64_t items = vec > 0 ? vec : bytes, blocks = (items + 255) / 256;
+  hipLaunchKernelGGL(copy_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), static_cast<const uint8_t*>(src),
+                     static_cast<uint8_t*>(dst), vec, bytes);
+  return fs2moe::check_launch("copy");
+}
+
 // ---- the whole layer for callers that cannot allocate ----------------------------------------------
 // Every intermediate of fs2moe_forward lives in one array inside the library's own device image, so
 // the call needs no workspace from the caller and never touches an allocator.  Every device the

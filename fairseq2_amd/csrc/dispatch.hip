@@ -319,20 +319,20 @@ __global__ __launch_bounds__(256) void dispatch_index_scan_kernel(
 // from L2: thread (slice, group of 8 experts) takes every S-th tile, 8 bytes a load, all of a
 // round's loads issued before any is looked at), block 0 writes counts and offsets, and the blocks
 // past the tiles fill the padding rows of perm.  Same integers as the other dispatch kernels.
-// E a multiple of 8 and at most 256 (one thread per expert in the scan).
+// E at most 256 (one thread per expert in the scan); a tile's counts are Ep bytes, E up to a multiple of 8.
 constexpr int kTileSumLoads = 8;
 __global__ __launch_bounds__(256) void dispatch_index_tiles_kernel(
-    const int32_t* __restrict__ topk_idx, int T, int K, int E, int tile_m, int64_t max_rows,
+    const int32_t* __restrict__ topk_idx, int T, int K, int E, int tile_tok, int tile_m, int64_t max_rows,
     unsigned tile_blocks, const uint8_t* __restrict__ tile_counts, int num_tiles,
     const int32_t* __restrict__ tile_rank, int32_t* __restrict__ counts,
     int32_t* __restrict__ offsets, int32_t* __restrict__ perm, int32_t* __restrict__ inv_perm) {
-  __shared__ int32_t s_part[2][2048];  // [all tiles | tiles before mine][slice][expert]: S E <= 2048
+  __shared__ int32_t s_part[2][2048];  // [all tiles | tiles before mine][slice][expert]: S Ep <= 2048
   __shared__ int32_t s_off[257], s_cnt[256], s_pre[256];
   __shared__ int32_t s_wave_tot[4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const bool tile_block = blockIdx.x < tile_blocks;
   const int mine = tile_block ? (int)blockIdx.x : 0;
-  const int G = E >> 3, S = 256 / G;
+  const int Ep = (E + 7) & ~7, G = Ep >> 3, S = 256 / G;
   const int g = tid % G, sl = tid / G;
   if (sl < S) {
     int tot[8], pre[8];
@@ -343,7 +343,7 @@ __global__ __launch_bounds__(256) void dispatch_index_tiles_kernel(
 #pragma unroll
       for (int i = 0; i < kTileSumLoads; ++i) {
         const int tile = t0 + i * S;
-        c[i] = *reinterpret_cast<const uint2*>(tile_counts + (size_t)(tile < num_tiles ? tile : 0) * E +
+        c[i] = *reinterpret_cast<const uint2*>(tile_counts + (size_t)(tile < num_tiles ? tile : 0) * Ep +
                                                g * 8);
       }
 #pragma unroll
@@ -360,8 +360,8 @@ __global__ __launch_bounds__(256) void dispatch_index_tiles_kernel(
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      s_part[0][sl * E + g * 8 + j] = tot[j];
-      s_part[1][sl * E + g * 8 + j] = pre[j];
+      s_part[0][sl * Ep + g * 8 + j] = tot[j];
+      s_part[1][sl * Ep + g * 8 + j] = pre[j];
     }
   }
   __syncthreads();
@@ -369,8 +369,8 @@ __global__ __launch_bounds__(256) void dispatch_index_tiles_kernel(
   if (tid < E) {
     int run = 0, pre = 0;
     for (int i = 0; i < S; ++i) {
-      run += s_part[0][i * E + tid];
-      pre += s_part[1][i * E + tid];
+      run += s_part[0][i * Ep + tid];
+      pre += s_part[1][i * Ep + tid];
     }
     s_cnt[tid] = run;
     s_pre[tid] = pre;
@@ -407,8 +407,8 @@ __global__ __launch_bounds__(256) void dispatch_index_tiles_kernel(
     }
     return;
   }
-  const int64_t p0 = (int64_t)mine * kRouterTileTok * K, pairs = (int64_t)T * K;
-  for (int i = tid; i < kRouterTileTok * K; i += 256) {
+  const int64_t p0 = (int64_t)mine * tile_tok * K, pairs = (int64_t)T * K;
+  for (int i = tid; i < tile_tok * K; i += 256) {
     const int64_t p = p0 + i;
     if (p >= pairs) break;
     const int e = topk_idx[p];
@@ -490,18 +490,18 @@ __global__ __launch_bounds__(kDispTok) void dispatch_small_copy_kernel(
 using namespace fs2moe;
 
 int fs2moe::dispatch_index_tiles(const int32_t* topk_idx, int32_t T, int32_t K, int32_t E,
-                                 int32_t tile_m, int64_t max_rows, const uint8_t* tile_counts,
+                                 int tile_tok, int32_t tile_m, int64_t max_rows, const uint8_t* tile_counts,
                                  const int32_t* tile_rank, int32_t* counts, int32_t* offsets,
                                  int32_t* perm, int32_t* inv_perm, void* stream) {
-  const int nt = (T + kRouterTileTok - 1) / kRouterTileTok;
-  FS2_REQUIRE(E % 8 == 0 && E <= 256 && nt >= 1 && nt <= kIndexTilesMax,
+  const int nt = (T + tile_tok - 1) / tile_tok;
+  FS2_REQUIRE(E <= 256 && nt >= 1 && nt <= kIndexTilesMax,
               "dispatch: internal: E=%d, %d tiles given to the tile form", E, nt);
   FS2_REQUIRE(max_rows >= FS2MOE_MAX_ROWS(T, K, E, tile_m) && max_rows < (1ll << 31),
               "dispatch: max_rows=%lld outside [%lld, 2^31)", (long long)max_rows,
               (long long)FS2MOE_MAX_ROWS(T, K, E, tile_m));
   const unsigned tail_blocks = (unsigned)((max_rows - (int64_t)T * K + 255) / 256);
   hipLaunchKernelGGL(dispatch_index_tiles_kernel, dim3((unsigned)nt + (unsigned)E + tail_blocks),
-                     dim3(256), 0, static_cast<hipStream_t>(stream), topk_idx, T, K, E, tile_m,
+                     dim3(256), 0, static_cast<hipStream_t>(stream), topk_idx, T, K, E, tile_tok, tile_m,
                      max_rows, (unsigned)nt, tile_counts, nt, tile_rank, counts, offsets, perm,
                      inv_perm);
   return check_launch("dispatch_index_tiles");
@@ -534,10 +534,10 @@ int fs2moe::dispatch_with_row_weights(const int32_t* topk_idx, const float* topk
 extern "C" int64_t fs2moe_dispatch_workspace_bytes(int32_t T, int32_t K, int32_t E) {
   if (T < 0 || K < 1 || E < 1) return -1;
   const int64_t nb = (T + kDispTok - 1) / kDispTok;
-  // per-block counts and per-pair ranks; twice the counts' room so that the same bytes also hold
-  // the form a tile-counting router leaves (a byte per expert and tile of 32 tokens, then the
+  // per-block counts and per-pair ranks; eight times the counts' room so that the same bytes also hold
+  // the form a tile-counting router leaves (a byte per expert and tile of 8 or more tokens, then the
   // ranks from the next multiple of 256 bytes on: tile_rank_of)
-  int64_t bytes = (2 * nb * E + (int64_t)T * K) * (int64_t)sizeof(int32_t);
+  int64_t bytes = (8 * nb * ((E + 7) / 8 * 8) + (int64_t)T * K) * (int64_t)sizeof(int32_t);
   return (bytes + 255) / 256 * 256 + 256;
 }
 

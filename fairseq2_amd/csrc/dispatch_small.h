@@ -1,7 +1,6 @@
 // All of dispatch for at most 256 tokens when no rows are copied: count, scan and index by one block.
-// A device function, because two kernels end with it: dispatch_small_kernel (fs2moe_dispatch) and
-// the router's finishing kernel for a few tokens, which selects the experts and dispatches in one
-// launch.
+// A device function, because two kernels begin with it: dispatch_small_kernel, and the form that goes on
+// to copy the rows.
 #pragma once
 
 #include "common.h"

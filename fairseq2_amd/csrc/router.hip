@@ -13,7 +13,6 @@
 #include <cstring>
 
 #include "common.h"
-#include "dispatch_small.h"
 
 namespace fs2moe {
 
@@ -141,75 +140,94 @@ struct Pack16<uint16_t> {
 // row); w may be null (no elementwise weight).  A wave takes two rows at a time so that their loads
 // are in flight together; rows of up to 256 16-byte chunks stay in registers between the sum of
 // squares and the product, longer ones are read a second time (from cache).
-template <typename TA>
+// H rows at a time of at most CACHE chunks a lane, held in registers between the two passes.
+template <int CACHE, int H, typename TA>
+__device__ __forceinline__ void rms_norm_cached_rows(const TA* x, const TA* w, float eps, TA* xn, int t0, int rows,
+                                                     int D, int k_lo, int k_hi) {
+  using P = Pack16<TA>;
+  constexpr int V = P::N;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave, nwaves = blockDim.x / kWave;
+  const float inv_d = 1.0f / (float)D;
+  const int nchunk = D / V, c_lo = k_lo / V, c_hi = (k_hi + V - 1) / V;
+  const u32x4 zero4 = {0u, 0u, 0u, 0u};
+  constexpr bool HOLD_W = CACHE <= 4;  // (longer rows: the weight's chunks are fetched where they are used)
+  u32x4 g[HOLD_W ? CACHE : 1];
+  if (HOLD_W && w != nullptr) {
+#pragma unroll
+    for (int i = 0; i < (HOLD_W ? CACHE : 0); ++i) {
+      const int c = lane + kWave * i;
+      g[i] = (c >= c_lo && c < c_hi && c < nchunk)
+                 ? *reinterpret_cast<const u32x4*>(w + (size_t)c * V) : zero4;
+    }
+  }
+  for (int r0 = wave; r0 < rows; r0 += H * nwaves) {
+    const int r1 = H == 2 && r0 + nwaves < rows ? r0 + nwaves : r0;  // a missing partner repeats r0
+    const int row[2] = {r0, r1};
+    u32x4 q[H][CACHE];
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+      for (int i = 0; i < CACHE; ++i) {
+        const int c = lane + kWave * i;
+        q[h][i] = c < nchunk ? *reinterpret_cast<const u32x4*>(x + (size_t)(t0 + row[h]) * D + (size_t)c * V) : zero4;
+      }
+    float rstd[H];
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < CACHE; ++i) {
+        float v[V];
+        P::unpack(q[h][i], v);
+#pragma unroll
+        for (int j = 0; j < V; ++j) ss += v[j] * v[j];
+      }
+      rstd[h] = 1.0f / sqrtf(wave_sum_f32(ss) * inv_d + eps);
+    }
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const bool row_on = h == 0 || r1 != r0;  // wave-uniform
+      TA* yr = xn + (size_t)(t0 + row[h]) * D;
+#pragma unroll
+      for (int i = 0; i < CACHE; ++i) {
+        const int c = lane + kWave * i;
+        if (!row_on || c < c_lo || c >= c_hi || c >= nchunk) continue;
+        float v[V], gv[V];
+        P::unpack(q[h][i], v);
+        if (w != nullptr) P::unpack(HOLD_W ? g[HOLD_W ? i : 0] : *reinterpret_cast<const u32x4*>(w + (size_t)c * V), gv);
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+          v[j] = v[j] * rstd[h];
+          if (w != nullptr) v[j] = v[j] * gv[j];
+        }
+        *reinterpret_cast<u32x4*>(yr + (size_t)c * V) = P::pack(v);
+      }
+    }
+  }
+}
+
+// LONG: rows of up to 12 chunks a lane in registers as well (for a kernel with registers to spare).
+template <typename TA, bool LONG = false>
 __device__ __forceinline__ void rms_norm_block_rows(const TA* x, const TA* w, float eps, TA* xn, int t0, int rows,
                                     int D, int k_lo, int k_hi) {
   using P = Pack16<TA>;
   constexpr int V = P::N;
-  constexpr int CACHE = 4;  // chunks per lane held in registers
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave, nwaves = blockDim.x / kWave;
   const uintptr_t bases = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(xn) |
                           reinterpret_cast<uintptr_t>(w);
   const bool vec = D % V == 0 && (bases & 15u) == 0 && k_lo % V == 0;
   const float inv_d = 1.0f / (float)D;
-  if (vec && D / V <= CACHE * kWave) {
-    const int nchunk = D / V, c_lo = k_lo / V, c_hi = (k_hi + V - 1) / V;
-    const u32x4 zero4 = {0u, 0u, 0u, 0u};
-    u32x4 g[CACHE];
-    if (w != nullptr) {
-#pragma unroll
-      for (int i = 0; i < CACHE; ++i) {
-        const int c = lane + kWave * i;
-        g[i] = (c >= c_lo && c < c_hi && c < nchunk)
-                   ? *reinterpret_cast<const u32x4*>(w + (size_t)c * V) : zero4;
-      }
-    }
-    for (int r0 = wave; r0 < rows; r0 += 2 * nwaves) {
-      const int r1 = r0 + nwaves < rows ? r0 + nwaves : r0;  // a missing partner repeats r0
-      const TA* xr[2] = {x + (size_t)(t0 + r0) * D, x + (size_t)(t0 + r1) * D};
-      u32x4 q[2][CACHE];
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int i = 0; i < CACHE; ++i) {
-          const int c = lane + kWave * i;
-          q[h][i] = c < nchunk ? *reinterpret_cast<const u32x4*>(xr[h] + (size_t)c * V) : zero4;
-        }
-      float rstd[2];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        float ss = 0.f;
-#pragma unroll
-        for (int i = 0; i < CACHE; ++i) {
-          float v[V];
-          P::unpack(q[h][i], v);
-#pragma unroll
-          for (int j = 0; j < V; ++j) ss += v[j] * v[j];
-        }
-        rstd[h] = 1.0f / sqrtf(wave_sum_f32(ss) * inv_d + eps);
-      }
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const bool row_on = h == 0 || r1 != r0;  // wave-uniform
-        TA* yr = xn + (size_t)(t0 + (h == 0 ? r0 : r1)) * D;
-#pragma unroll
-        for (int i = 0; i < CACHE; ++i) {
-          const int c = lane + kWave * i;
-          if (!row_on || c < c_lo || c >= c_hi || c >= nchunk) continue;
-          float v[V], gv[V];
-          P::unpack(q[h][i], v);
-          if (w != nullptr) P::unpack(g[i], gv);
-#pragma unroll
-          for (int j = 0; j < V; ++j) {
-            v[j] = v[j] * rstd[h];
-            if (w != nullptr) v[j] = v[j] * gv[j];
-          }
-          *reinterpret_cast<u32x4*>(yr + (size_t)c * V) = P::pack(v);
-        }
-      }
-    }
+  if (vec && D / V <= 4 * kWave) {
+    rms_norm_cached_rows<4, 2>(x, w, eps, xn, t0, rows, D, k_lo, k_hi);
     return;
+  }
+  if constexpr (LONG) {
+    if (vec && D / V <= 12 * kWave) {
+      rms_norm_cached_rows<12, 1>(x, w, eps, xn, t0, rows, D, k_lo, k_hi);
+      return;
+    }
   }
   for (int r = wave; r < rows; r += nwaves) {
     const TA* xr = x + (size_t)(t0 + r) * D;
@@ -253,6 +271,62 @@ __device__ __forceinline__ void rms_norm_block_rows(const TA* x, const TA* w, fl
   }
 }
 
+// The bf16 rows of a 32-token tile for a block that reads only a share of their columns, at most 32 chunks
+// (16 waves, two rows each; same arithmetic).  The share is loaded before the sums are taken and kept, a
+// half wave to a row, and goes to xn and, by `emit(row, chunk, value)`, to where the block reads it.
+template <typename Emit>
+__device__ __forceinline__ void rms_norm_tile_share(const uint16_t* x, const uint16_t* w, float eps, uint16_t* xn,
+                                                    int t0, int rows, int D, int c_lo, int c_hi, Emit emit) {
+  using P = Pack16<uint16_t>;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  if (wave >= rows) return;
+  const int other = wave + 16 < rows ? wave + 16 : wave;
+  const int my_row = lane < 32 ? wave : other, chunk = c_lo + (lane & 31);
+  const bool mine = chunk < c_hi && (lane < 32 || other != wave);
+  const uint16_t* xr[2] = {x + (size_t)(t0 + wave) * D, x + (size_t)(t0 + other) * D};
+  const int at = (chunk < c_hi ? chunk : c_lo) * 8;
+  const u32x4 keep = *reinterpret_cast<const u32x4*>(x + (size_t)(t0 + my_row) * D + at);
+  u32x4 g = {0u, 0u, 0u, 0u};
+  if (w != nullptr) g = *reinterpret_cast<const u32x4*>(w + at);
+  float ss[2] = {0.f, 0.f};
+  const int nchunk = D / 8;
+  for (int c0 = 0; c0 < nchunk; c0 += 4 * kWave) {
+    u32x4 q[2][4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int c = c0 + lane + kWave * i;
+        q[h][i] = c < nchunk ? *reinterpret_cast<const u32x4*>(xr[h] + (size_t)c * 8) : u32x4{0u, 0u, 0u, 0u};
+      }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float v[8];
+        P::unpack(q[h][i], v);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) ss[h] += v[j] * v[j];
+      }
+  }
+  const float inv_d = 1.0f / (float)D;
+  const float r0 = 1.0f / sqrtf(wave_sum_f32(ss[0]) * inv_d + eps), r1 = 1.0f / sqrtf(wave_sum_f32(ss[1]) * inv_d + eps);
+  if (!mine) return;
+  const float rstd = lane < 32 ? r0 : r1;
+  float v[8], gv[8];
+  P::unpack(keep, v);
+  P::unpack(g, gv);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    v[j] = v[j] * rstd;
+    if (w != nullptr) v[j] = v[j] * gv[j];
+  }
+  const u32x4 y = P::pack(v);
+  *reinterpret_cast<u32x4*>(xn + (size_t)(t0 + my_row) * D + at) = y;
+  emit(my_row, chunk, y);
+}
+
 // The same normalisation as a kernel of its own, four rows per block.  Used in front of the router
 // when there are so few 32-token blocks that the CUs running them would do the normalisation one
 // after the other while the rest of the chip idles.
@@ -262,7 +336,7 @@ __global__ __launch_bounds__(kNormRows* kWave) void rms_norm_kernel(const TA* x,
                                                                     float eps, TA* xn, int T,
                                                                     int D) {
   const int t0 = blockIdx.x * kNormRows;
-  rms_norm_block_rows<TA>(x, w, eps, xn, t0, T - t0 < kNormRows ? T - t0 : kNormRows, D, 0, D);
+  rms_norm_block_rows<TA, true>(x, w, eps, xn, t0, T - t0 < kNormRows ? T - t0 : kNormRows, D, 0, D);
 }
 
 constexpr int kRouterTok = 8;     // tokens per wave
@@ -379,7 +453,13 @@ struct Shape {
 // step while most CUs idle.  Then gridDim.y blocks share a token tile, block y taking a contiguous
 // range of chunks, and write their sums to `partial` [gridDim.y][T][E] instead of selecting;
 // router_finish_kernel adds the ranges in ascending order and selects.
-template <int NF, bool SPLIT>
+//
+// STEP: SPLIT with one chunk to a group (the whole of a decode step's router).  The router's chunk is
+// then on its way while the rows are normalised, and the normalised columns go straight to the tile in
+// LDS: loading them back from xn, and the router after that, were two more round trips (8 tokens of
+// 2048 features, 128 experts: 8.1 -> 6.0 us).  With xn: D a multiple of 64, NF = 1, norm_w aligned.
+enum class RouterMode { WHOLE, SPLIT, STEP };
+template <int NF, RouterMode MODE>
 __global__ __launch_bounds__(rmfma::Shape<NF>::THREADS) void router_mfma_kernel(
     const uint16_t* x, const uint16_t* norm_w, float norm_eps, uint16_t* xn,
     const uint16_t* __restrict__ router, const float* __restrict__ bias, int T, int D, int E, int K,
@@ -387,6 +467,7 @@ __global__ __launch_bounds__(rmfma::Shape<NF>::THREADS) void router_mfma_kernel(
     float* __restrict__ logits, float* __restrict__ partial) {
   using namespace rmfma;
   using S = Shape<NF>;
+  constexpr bool SPLIT = MODE != RouterMode::WHOLE, STEP = MODE == RouterMode::STEP;
   constexpr int BK = S::BK, LDX = S::LDX, EP = S::EP, LDR = S::LDR, LDL = S::LDL;
   constexpr int GROUPS = S::GROUPS;
   constexpr int J = EP / 64;
@@ -402,23 +483,6 @@ __global__ __launch_bounds__(rmfma::Shape<NF>::THREADS) void router_mfma_kernel(
   const int t0 = blockIdx.x * BT;
   uint16_t* sX = reinterpret_cast<uint16_t*>(smem + group * S::GROUP_BYTES);
   uint16_t* sR = sX + BT * LDX;
-  if (xn != nullptr) {
-    // the columns this block goes on to read: all of them, or (SPLIT, a single token tile: the host
-    // sends more tiles than that through rms_norm_kernel first) the chunks of its share, which the
-    // blocks of the tile write between them
-    int k_lo = 0, k_hi = D;
-    if constexpr (SPLIT) {
-      const int nk_all = (D + BK - 1) / BK;
-      const int share = (nk_all + (int)gridDim.y - 1) / (int)gridDim.y;
-      k_lo = (int)blockIdx.y * share * BK;
-      k_hi = k_lo + share * BK < D ? k_lo + share * BK : D;
-    }
-    if (k_lo < k_hi)
-      rms_norm_block_rows<uint16_t>(x, norm_w, norm_eps, xn, t0, T - t0 < BT ? T - t0 : BT, D, k_lo, k_hi);
-    __syncthreads();  // the block's part of xn is written and visible to all its waves
-    x = xn;
-  }
-
   f32x16 acc[NF];
 #pragma unroll
   for (int f = 0; f < NF; ++f)
@@ -448,7 +512,7 @@ __global__ __launch_bounds__(rmfma::Shape<NF>::THREADS) void router_mfma_kernel(
   // only when the registers are stored to LDS: with no branch around the loads and no use of their
   // results before that, the compiler can count them, and waiting for one register set leaves the
   // other in flight.
-  auto load_global = [&](int set, int step) {
+  auto load_x = [&](int set, int step) {
     const int kt = kt_lo + step * GROUPS + group;
     const int k0 = (kt < kt_hi ? kt : 0) * BK;
 #pragma unroll
@@ -460,16 +524,32 @@ __global__ __launch_bounds__(rmfma::Shape<NF>::THREADS) void router_mfma_kernel(
       const int k = k0 + kc * 8;
       rx[set][i] = *reinterpret_cast<const u32x4*>(x + (size_t)t * D + (k < D ? k : D - 8));
     }
+  };
+  // With E not a multiple of 8 a row's last chunk runs on into the next row (columns past E, which
+  // nothing looks at), and rows begin wherever they do: 16-byte loads at 2-byte alignment.  The very
+  // last chunk would end past the matrix: it is read from the last place that does not, and shifted.
+  struct __attribute__((packed, aligned(2))) Unaligned16 {
+    u32x4 v;
+  };
+  auto router_at = [&](int k0, int c) -> int64_t {
+    const int k = k0 + c / (EP / 8), e = (c % (EP / 8)) * 8;
+    return (int64_t)(k < D ? k : D - 1) * E + (e < E ? e : 0);
+  };
+  const int64_t router_last = (int64_t)D * E - 8;  // (D >= 8)
+  auto load_r = [&](int set, int step) {
+    const int kt = kt_lo + step * GROUPS + group;
+    const int k0 = (kt < kt_hi ? kt : 0) * BK;
 #pragma unroll
     for (int i = 0; i < R_CHUNKS; ++i) {
-      const int c = tid + 256 * i;
-      const int kr = c / (EP / 8), ec = c % (EP / 8);
-      const int k = k0 + kr, e = ec * 8;
-      rr[set][i] = *reinterpret_cast<const u32x4*>(router + (size_t)(k < D ? k : D - 1) * E +
-                                                   (e < E ? e : E - 8));
+      const int64_t at = router_at(k0, tid + 256 * i);
+      rr[set][i] = reinterpret_cast<const Unaligned16*>(router + (at < router_last ? at : router_last))->v;
     }
   };
-  auto store_lds = [&](int set, int step) {
+  auto load_global = [&](int set, int step) {
+    load_x(set, step);
+    load_r(set, step);
+  };
+  auto store_x = [&](int set, int step) {
     const int kt = kt_lo + step * GROUPS + group;
     const bool live = kt < kt_hi;
     const int k0 = (live ? kt : 0) * BK;
@@ -480,14 +560,32 @@ __global__ __launch_bounds__(rmfma::Shape<NF>::THREADS) void router_mfma_kernel(
       const bool in = live && k0 + kc * 8 < D;
       *reinterpret_cast<u32x4*>(&sX[row * LDX + kc * 8]) = in ? rx[set][i] : zero4;
     }
+  };
+  auto store_r = [&](int set, int step) {
+    const int kt = kt_lo + step * GROUPS + group;
+    const bool live = kt < kt_hi;
+    const int k0 = (live ? kt : 0) * BK;
 #pragma unroll
     for (int i = 0; i < R_CHUNKS; ++i) {
       const int c = tid + 256 * i;
       const int kr = c / (EP / 8), ec = c % (EP / 8);
-      // E is a multiple of 8 on this path, so a chunk is entirely inside or outside.
       const bool in = live && k0 + kr < D && ec * 8 < E;
-      *reinterpret_cast<u32x4*>(&sR[kr * LDR + ec * 8]) = in ? rr[set][i] : zero4;
+      u32x4 v = in ? rr[set][i] : zero4;
+      const int64_t over = router_at(k0, c) - router_last;
+      if (over > 0) {  // (at most one chunk of the matrix, and none with E a multiple of 8)
+        uint64_t lo = (uint64_t)v[1] << 32 | v[0], hi = (uint64_t)v[3] << 32 | v[2];
+        for (int j = 0; j < (int)over; ++j) {
+          lo = lo >> 16 | hi << 48;
+          hi >>= 16;
+        }
+        v = u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+      }
+      *reinterpret_cast<u32x4*>(&sR[kr * LDR + ec * 8]) = v;
     }
+  };
+  auto store_lds = [&](int set, int step) {
+    store_x(set, step);
+    store_r(set, step);
   };
   const int s = lane & 15, half = (lane >> 4) & 1;
   auto compute = [&]() {
@@ -504,7 +602,39 @@ __global__ __launch_bounds__(rmfma::Shape<NF>::THREADS) void router_mfma_kernel(
     }
   };
 
-  // Both groups run the same number of steps (a group with one chunk fewer multiplies zeros in its
+  const int tile_rows = T - t0 < BT ? T - t0 : BT;
+  // the columns this block goes on to read: all of them, or (SPLIT) the chunks of its share, which the
+  // blocks of the tile write between them
+  const int k_lo = kt_lo * BK, k_hi = kt_hi * BK < D ? kt_hi * BK : D;
+  if constexpr (STEP) {
+    load_r(0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (NF == 1 && xn != nullptr) {
+      if (k_lo < k_hi)
+        rms_norm_tile_share(x, norm_w, norm_eps, xn, t0, tile_rows, D, k_lo / 8, k_hi / 8,
+                            [&](int row, int c, u32x4 y) {
+                              const int g2 = c / (BK / 8) - kt_lo;
+                              uint16_t* to = reinterpret_cast<uint16_t*>(smem + g2 * S::GROUP_BYTES);
+                              *reinterpret_cast<u32x4*>(&to[row * LDX + (c % (BK / 8)) * 8]) = y;
+                            });
+    } else {
+      load_x(0, 0);
+      store_x(0, 0);
+    }
+    store_r(0, 0);
+    lds_barrier();
+    // (rows of the tile past T are never looked at, and may hold anything; so may the rows of a group
+    // without a chunk, which must not be multiplied)
+    if (kt_lo + group < kt_hi) compute();
+    lds_barrier();
+  } else {
+  if (xn != nullptr) {
+    if (k_lo < k_hi)
+      rms_norm_block_rows<uint16_t>(x, norm_w, norm_eps, xn, t0, tile_rows, D, k_lo, k_hi);
+    __syncthreads();  // the block's part of xn is written and visible to all its waves
+    x = xn;
+  }
+  // All groups run the same number of steps (a group with one chunk fewer multiplies zeros in its
   // last step), so the barriers below are common to the block.
   load_global(0, 0);
   // keep set 0 the older one here as it is in the loop: a wait for it then leaves set 1 in flight
@@ -522,6 +652,7 @@ __global__ __launch_bounds__(rmfma::Shape<NF>::THREADS) void router_mfma_kernel(
     if (st + 1 < steps) compute();
     lds_barrier();
   }
+  }
 
   // Partial logits of each group -> its own LDS region (the stage is no longer needed).
   // Accumulator layout: lane holds token lr and experts 32 F + 8 q + 4 lk + j (F = wave + 4 f).
@@ -537,9 +668,9 @@ __global__ __launch_bounds__(rmfma::Shape<NF>::THREADS) void router_mfma_kernel(
   __syncthreads();
 
   if constexpr (SPLIT) {
-    for (int i = tid_all; i < BT * EP; i += S::THREADS) {
+    for (int i = tid_all; i < tile_rows * EP; i += S::THREADS) {
       const int tl = i / EP, e = i - tl * EP;
-      if (t0 + tl >= T || e >= E) continue;
+      if (e >= E) continue;
       float sum = 0.f;
 #pragma unroll
       for (int g2 = 0; g2 < GROUPS; ++g2)
@@ -771,18 +902,16 @@ __global__ __launch_bounds__(1024) void router_mfma_t_kernel(
   if (tid < E) tile_counts[(size_t)blockIdx.x * E + tid] = (uint8_t)__popc(s_bits[tid]);
 }
 
-constexpr int kMaxSlices = 8;  // blocks sharing a token tile, at most
+constexpr int kMaxSlices = 20;  // blocks sharing a token tile, at most
 
 // Second half of the split router: one wave per token adds the `slices` partial logits in
 // ascending order, then the bias, and selects.
 template <int J>
-__global__ __launch_bounds__(4 * kWave) void router_finish_kernel(
-    const float* __restrict__ partial, int slices, const float* __restrict__ bias, int T, int E,
-    int K, int score_fn, int renorm, int32_t* __restrict__ topk_idx, float* __restrict__ topk_w,
-    float* __restrict__ logits) {
+__device__ __forceinline__ void finish_token(const float* __restrict__ partial, int slices,
+                                             const float* __restrict__ bias, int t, int T, int E, int K,
+                                             int score_fn, int renorm, int32_t* topk_idx, float* topk_w,
+                                             float* logits, int* chosen) {
   const int lane = lane_id();
-  const int t = blockIdx.x * 4 + threadIdx.x / kWave;
-  if (t >= T) return;  // wave-uniform
   // all loads first (at most kMaxSlices of them per expert), then the sums in ascending order
   float p[kMaxSlices][J], b[J];
 #pragma unroll
@@ -803,47 +932,114 @@ __global__ __launch_bounds__(4 * kWave) void router_finish_kernel(
     v[j] = sum + b[j];
     if (logits != nullptr && e < E) logits[(size_t)t * E + e] = v[j];
   }
-  select_topk<J>(v, lane, t, E, K, score_fn, renorm, topk_idx, topk_w);
+  select_topk<J>(v, lane, t, E, K, score_fn, renorm, topk_idx, topk_w, chosen);
 }
 
-// The same for a few tokens in one block, which then goes on to dispatch them (dispatch_small_block:
-// no rows copied): a decode step of a few sequences spends more on starting its kernels than on
-// their work, and this is one start fewer.  A wave takes the tokens wave, wave + 16, ..  Same
-// arithmetic as router_finish_kernel followed by dispatch_small_kernel, so the results are identical.
-constexpr int kFinishDispatchThreads = 1024;
-constexpr int kFinishDispatchTokens = 2 * kFinishDispatchThreads / kWave;
 template <int J>
-__global__ __launch_bounds__(kFinishDispatchThreads) void router_finish_dispatch_kernel(
+__global__ __launch_bounds__(4 * kWave) void router_finish_kernel(
     const float* __restrict__ partial, int slices, const float* __restrict__ bias, int T, int E,
-    int K, int score_fn, int renorm, int32_t* topk_idx, float* topk_w, int tile_m, int64_t max_rows,
-    int32_t* counts, int32_t* offsets, int32_t* perm, int32_t* inv_perm, float* row_w) {
-  extern __shared__ uint32_t s_mem[];
-  __shared__ int32_t s_wave_tot[4];
-  const int lane = lane_id();
-  for (int t = threadIdx.x / kWave; t < T; t += kFinishDispatchThreads / kWave) {  // wave-uniform
-    float p[kMaxSlices][J], b[J];
+    int K, int score_fn, int renorm, int32_t* __restrict__ topk_idx, float* __restrict__ topk_w,
+    float* __restrict__ logits) {
+  const int t = blockIdx.x * 4 + threadIdx.x / kWave;
+  if (t >= T) return;  // wave-uniform
+  int chosen;
+  finish_token<J>(partial, slices, bias, t, T, E, K, score_fn, renorm, topk_idx, topk_w, logits, &chosen);
+}
+
+// The same with dispatch's bookkeeping (no rows copied), for tiles of TOK tokens, one or two tokens to
+// a wave: lane k of a token's wave knows the token's k-th expert, so that a word per expert with a bit
+// per token of the tile holds the tile's membership, and a pair's rank among its expert's pairs is a
+// population count.
+//
+// ALL: the tile is all there is (T <= 32), and the block goes on to the counts, the offsets and the
+// permutation itself: a decode step of a few sequences spends more on starting its kernels than on
+// their work.  Else it leaves its counts and ranks to dispatch_index_tiles_kernel.  Both instead of a
+// selection kernel and one or two that read the selection back from memory (8 tokens, 128 experts:
+// 9.1 -> 5.2 us; 777 tokens, 64 experts: 16.5 -> 10.5 us with the index kernel).  The partial logits of a
+// tile are one CU's reads, which favours small tiles (48 tokens in tiles of 32: 11.3 us, of 8: 5.4),
+// while the index kernel's every block adds up all tiles' counts, which favours few of them.
+constexpr int kFinishTok = 8, kFinishTokMax = 1024;  // tokens per tile up to so many tokens, then kRouterTileTok
+template <int TOK>
+constexpr int finish_tile_threads() { return TOK <= 16 ? TOK * kWave : 1024; }
+template <int J, bool ALL, int TOK>
+__global__ __launch_bounds__(finish_tile_threads<TOK>()) void router_finish_tile_kernel(
+    const float* __restrict__ partial, int slices, const float* __restrict__ bias, int T, int E,
+    int K, int score_fn, int renorm, int32_t* __restrict__ topk_idx, float* __restrict__ topk_w,
+    uint8_t* __restrict__ tile_counts, int32_t* __restrict__ tile_rank, int tile_m, int64_t max_rows,
+    int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ perm,
+    int32_t* __restrict__ inv_perm, float* __restrict__ row_w) {
+  constexpr int THREADS = finish_tile_threads<TOK>(), NW = THREADS / kWave, TPW = TOK / NW;
+  __shared__ uint32_t s_bits[64 * J];
+  __shared__ int32_t s_off[64 * J + 1], s_wave_tot[J];
+  const int tid = threadIdx.x, lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int t0 = blockIdx.x * TOK;
+  static_assert(64 * J <= THREADS, "a thread per expert");
+  if (tid < 64 * J) s_bits[tid] = 0u;
+  __syncthreads();
+  int chosen[TPW];
 #pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int e = lane + 64 * j;
-      b[j] = (bias != nullptr && e < E) ? bias[e] : 0.f;
-#pragma unroll
-      for (int s = 0; s < kMaxSlices; ++s)
-        p[s][j] = (s < slices && e < E) ? partial[((size_t)s * T + t) * E + e] : 0.f;
-    }
-    float v[J];
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      float sum = p[0][j];
-#pragma unroll
-      for (int s = 1; s < kMaxSlices; ++s) sum += p[s][j];
-      v[j] = sum + b[j];
-    }
-    select_topk<J>(v, lane, t, E, K, score_fn, renorm, topk_idx, topk_w);
+  for (int i = 0; i < TPW; ++i) {
+    const int tl = wave + NW * i;
+    chosen[i] = 0;
+    if (t0 + tl >= T) continue;  // wave-uniform
+    finish_token<J>(partial, slices, bias, t0 + tl, T, E, K, score_fn, renorm, topk_idx, topk_w, nullptr,
+                    &chosen[i]);
+    if (lane < K) atomicOr(&s_bits[chosen[i]], 1u << tl);
   }
-  __syncthreads();  // the tokens' experts are written and visible to the block
-  // (the host sends K > 16 through router_finish_kernel and the dispatch kernels instead)
-  dispatch_small_block<16>(topk_idx, T, K, E, tile_m, max_rows, counts, offsets, perm, inv_perm,
-                           s_mem, s_wave_tot, threadIdx.x, kFinishDispatchThreads, true, topk_w, row_w);
+  __syncthreads();
+  if constexpr (!ALL) {
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+      const int tl = wave + NW * i;
+      if (t0 + tl < T && lane < K)
+        tile_rank[(size_t)(t0 + tl) * K + lane] = __popc(s_bits[chosen[i]] & ((1u << tl) - 1u));
+    }
+    const int Ep = (E + 7) & ~7;  // (experts past E have no pairs)
+    if (tid < Ep) tile_counts[(size_t)blockIdx.x * Ep + tid] = (uint8_t)__popc(s_bits[tid]);
+    return;
+  }
+  // counts and tile-padded offsets: a thread per expert, a scan over the J waves that hold them
+  int cnt = 0, padded = 0, incl = 0;
+  if (wave < J) {
+    cnt = __popc(s_bits[tid]);
+    padded = (cnt + tile_m - 1) / tile_m * tile_m;
+    incl = padded;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int v = __shfl_up(incl, off, kWave);
+      if (lane >= off) incl += v;
+    }
+    if (lane == 63) s_wave_tot[wave] = incl;
+  }
+  __syncthreads();
+  if (wave < J) {
+    int base = 0;
+    for (int w = 0; w < wave; ++w) base += s_wave_tot[w];
+    s_off[tid] = base + incl - padded;
+    if (tid == 64 * J - 1) s_off[64 * J] = base + incl;
+    if (tid < E) {
+      counts[tid] = cnt;
+      offsets[tid] = base + incl - padded;
+      if (tid == E - 1) offsets[E] = base + incl;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < TPW; ++i) {
+    const int tl = wave + NW * i;
+    if (tl >= T || lane >= K) continue;
+    const int row = s_off[chosen[i]] + __popc(s_bits[chosen[i]] & ((1u << tl) - 1u));
+    inv_perm[(size_t)tl * K + lane] = row;
+    perm[row] = tl;
+    // (for kernels that scale a row by its routing weight while they read it through perm: lane k
+    // reads what it has written)
+    if (row_w != nullptr) row_w[row] = topk_w[(size_t)tl * K + lane];
+  }
+  // padding rows, then the rows beyond the last expert's
+  if (tid < E)
+    for (int r = s_off[tid] + cnt; r < s_off[tid + 1]; ++r) perm[r] = -1;
+  for (int64_t r = (int64_t)s_off[64 * J] + tid; r < max_rows; r += THREADS) perm[r] = -1;
 }
 
 // ------------------------------------------------------------------------------------ f32 / MFMA
@@ -1067,14 +1263,14 @@ static int launch_router_fma(const void* x, const void* norm_w, float norm_eps, 
 
 using namespace fs2moe;
 
-// Token counts up to this are normalised by rms_norm_kernel in front of the router, larger ones by
-// the router blocks themselves.  It covers every token count the split router takes.
+// Token counts up to this are normalised by rms_norm_kernel in front of the router where one block has a
+// token tile to itself (unless it is the only tile), larger ones by the router blocks themselves.
 constexpr int kNormAloneMaxTokens = 4096;
 
 // How many blocks share a 32-token tile of the bf16 MFMA router: enough to put about 256 blocks on
-// the chip, each with at least one step of its k-groups, at most 8.  1 = no split.
+// the chip, each with at least one step of its k-groups, at most kMaxSlices.  1 = no split.
 static int router_slices(int T, int D, int E, int act_dtype) {
-  if (act_dtype != FS2MOE_BF16 || D % 8 != 0 || E % 8 != 0 || E > 256 || T < 1) return 1;
+  if (act_dtype != FS2MOE_BF16 || D % 8 != 0 || E > 256 || T < 1) return 1;
   const int tiles = (T + rmfma::BT - 1) / rmfma::BT;
   const int groups = E <= 128 ? rmfma::Shape<1>::GROUPS : rmfma::Shape<2>::GROUPS;
   const int nk = (D + 63) / 64;
@@ -1126,11 +1322,17 @@ static int router_entry(const void* x, const void* norm_w, float norm_eps, void*
               "(T=%d D=%d E=%d), from 16-byte aligned operands", T, D, E);
   if (T == 0) return FS2MOE_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // (a single token tile of the bf16 MFMA router normalises in its own blocks, also when several
-  // blocks share the tile: one launch fewer for a decode step)
-  const bool one_tile = act_dtype == FS2MOE_BF16 && T <= rmfma::BT && D % 8 == 0 && E % 8 == 0 && E <= 256 &&
-                        aligned16(x) && aligned16(router) && aligned16(xn);
-  if (xn != nullptr && T <= kNormAloneMaxTokens && !one_tile) {
+  // (a single token tile of the bf16 MFMA router, and the tiles of blocks that take one step each, are
+  // normalised by their blocks: each reads its 32 rows, which costs less than a launch in front)
+  const int slices = router_slices(T, D, E, act_dtype);
+  const bool split = slices > 1 && workspace != nullptr && workspace_bytes >= (int64_t)slices * T * E * 4 &&
+                     aligned16(x) && aligned16(router);
+  const int k_groups = E <= 128 ? rmfma::Shape<1>::GROUPS : rmfma::Shape<2>::GROUPS;
+  const bool one_step = split && ((D + 63) / 64 + slices - 1) / slices <= k_groups;
+  const bool step_norms = one_step && D % 64 == 0 && E <= 128 && aligned16(norm_w);
+  const bool in_blocks = act_dtype == FS2MOE_BF16 && (T <= rmfma::BT || step_norms) && D % 8 == 0 && E <= 256 &&
+                         aligned16(x) && aligned16(router) && aligned16(xn);
+  if (xn != nullptr && T <= kNormAloneMaxTokens && !in_blocks) {
     // few token blocks: normalise with the whole chip first, then route xn as it is
     dim3 grid((T + kNormRows - 1) / kNormRows), block(kNormRows * kWave);
     if (act_dtype == FS2MOE_F32)
@@ -1171,7 +1373,7 @@ static int router_entry(const void* x, const void* norm_w, float norm_eps, void*
     const bool counting = disp != nullptr && disp->ws != nullptr && (int)grid.x <= kIndexTilesMax &&
                           disp->ws_bytes >= fs2moe_dispatch_workspace_bytes(T, K, E);
     uint8_t* tile_counts = counting ? tile_counts_of(disp->ws) : nullptr;
-    int32_t* tile_rank = counting ? tile_rank_of(disp->ws, T, E) : nullptr;
+    int32_t* tile_rank = counting ? tile_rank_of(disp->ws, T, E, kRouterTileTok) : nullptr;
     if (E <= 128)
       hipLaunchKernelGGL(k1, grid, threads, rmfma_t::Shape<1>::SMEM_BYTES, s, xp, wp, norm_eps, xnp,
                          static_cast<const uint16_t*>(router), bias, T, D, E, K, score_fn, renormalize,
@@ -1182,8 +1384,8 @@ static int router_entry(const void* x, const void* norm_w, float norm_eps, void*
                          topk_idx, topk_w, logits, tile_counts, tile_rank);
     if (int rc = check_launch("router_mfma (E, D)")) return rc;
     if (counting) {
-      if (int rc = dispatch_index_tiles(topk_idx, T, K, E, disp->tile_m, disp->max_rows, tile_counts,
-                                        tile_rank, disp->counts, disp->offsets, disp->perm,
+      if (int rc = dispatch_index_tiles(topk_idx, T, K, E, kRouterTileTok, disp->tile_m, disp->max_rows,
+                                        tile_counts, tile_rank, disp->counts, disp->offsets, disp->perm,
                                         disp->inv_perm, stream))
         return rc;
       disp->done = true;
@@ -1210,26 +1412,32 @@ static int router_entry(const void* x, const void* norm_w, float norm_eps, void*
     return launch_router_fma<float>(x, norm_w, norm_eps, xn, router, bias, T, D, E, K, score_fn, renormalize, topk_idx,
                                     topk_w, logits, s);
   }
-  // The MFMA path moves 16-byte chunks (D and E multiples of 8, aligned bases) and holds up to 256
+  // The MFMA path moves 16-byte chunks of rows (D a multiple of 8, aligned bases) and holds up to 256
   // experts; anything else takes the FMA kernel.
-  if (D % 8 == 0 && E % 8 == 0 && E <= 256 && aligned16(x) && aligned16(router)) {
+  if (D % 8 == 0 && E <= 256 && aligned16(x) && aligned16(router)) {
     dim3 grid((T + rmfma::BT - 1) / rmfma::BT);
     const uint16_t* xp = static_cast<const uint16_t*>(x);
     const uint16_t* rp = static_cast<const uint16_t*>(router);
     const uint16_t* wp = static_cast<const uint16_t*>(norm_w);
     uint16_t* xnp = static_cast<uint16_t*>(xn);
-    auto k1 = router_mfma_kernel<1, false>;
-    auto k2 = router_mfma_kernel<2, false>;
-    auto k1s = router_mfma_kernel<1, true>;
-    auto k2s = router_mfma_kernel<2, true>;
+    using M = RouterMode;
+    auto k1 = router_mfma_kernel<1, M::WHOLE>;
+    auto k2 = router_mfma_kernel<2, M::WHOLE>;
+    const bool step = one_step && (xn == nullptr || step_norms);
+    auto k1s = step ? router_mfma_kernel<1, M::STEP> : router_mfma_kernel<1, M::SPLIT>;
+    auto k2s = step ? router_mfma_kernel<2, M::STEP> : router_mfma_kernel<2, M::SPLIT>;
     static bool attr_set = false;  // benign race: setting the attribute is idempotent
     if (!attr_set) {
-      const void* kernels[4] = {reinterpret_cast<const void*>(k1), reinterpret_cast<const void*>(k1s),
-                                reinterpret_cast<const void*>(k2), reinterpret_cast<const void*>(k2s)};
-      for (int i = 0; i < 4; ++i) {
+      const void* kernels[6] = {reinterpret_cast<const void*>(k1),
+                                reinterpret_cast<const void*>(router_mfma_kernel<1, M::SPLIT>),
+                                reinterpret_cast<const void*>(router_mfma_kernel<1, M::STEP>),
+                                reinterpret_cast<const void*>(k2),
+                                reinterpret_cast<const void*>(router_mfma_kernel<2, M::SPLIT>),
+                                reinterpret_cast<const void*>(router_mfma_kernel<2, M::STEP>)};
+      for (int i = 0; i < 6; ++i) {
         hipError_t e = hipFuncSetAttribute(
             kernels[i], hipFuncAttributeMaxDynamicSharedMemorySize,
-            i < 2 ? rmfma::Shape<1>::SMEM_BYTES : rmfma::Shape<2>::SMEM_BYTES);
+            i < 3 ? rmfma::Shape<1>::SMEM_BYTES : rmfma::Shape<2>::SMEM_BYTES);
         if (e != hipSuccess) {
           set_error("router: cannot reserve LDS: %s", hipGetErrorString(e));
           return FS2MOE_ERR_LAUNCH;
@@ -1237,13 +1445,9 @@ static int router_entry(const void* x, const void* norm_w, float norm_eps, void*
       }
       attr_set = true;
     }
-    const int slices = router_slices(T, D, E, act_dtype);
     const dim3 threads(E <= 128 ? rmfma::Shape<1>::THREADS : rmfma::Shape<2>::THREADS);
     const int lds = E <= 128 ? rmfma::Shape<1>::SMEM_BYTES : rmfma::Shape<2>::SMEM_BYTES;
-    if (slices > 1 && workspace != nullptr && workspace_bytes >= (int64_t)slices * T * E * 4) {
-      // (several tiles were normalised by the kernel in front, T being within kNormAloneMaxTokens;
-      // a single tile is normalised by its blocks, each the columns it reads)
-      static_assert(256 * rmfma::BT / 2 <= kNormAloneMaxTokens, "split tiles are normalised in front");
+    if (split) {
       float* partial = static_cast<float*>(workspace);
       grid.y = slices;
       hipLaunchKernelGGL(E <= 128 ? k1s : k2s, grid, threads, lds, s, xp, wp, norm_eps, xnp, rp, bias,
@@ -1251,15 +1455,24 @@ static int router_entry(const void* x, const void* norm_w, float norm_eps, void*
       if (int rc = check_launch("router_mfma (split)")) return rc;
       const dim3 fgrid((T + 3) / 4), fblock(4 * kWave);
       const int j = (E + 63) / 64;
-      if (disp != nullptr && logits == nullptr && T <= kFinishDispatchTokens && K <= 16) {
-        const size_t dlds = dispatch_small_lds_words(E) * sizeof(uint32_t);
-#define FS2_FINISH_CASE(JJ)                                                                       \
-  case JJ:                                                                                        \
-    hipLaunchKernelGGL((router_finish_dispatch_kernel<JJ>), dim3(1),                                \
-                       dim3(kFinishDispatchThreads), dlds, s,                                     \
-                       partial, slices, bias, T, E, K, score_fn, renormalize, topk_idx, topk_w,   \
-                       disp->tile_m, disp->max_rows, disp->counts, disp->offsets, disp->perm,     \
-                       disp->inv_perm, disp->row_w);                                              \
+      const bool all = T <= kRouterTileTok;
+      const int tok = all || T > kFinishTokMax ? kRouterTileTok : kFinishTok, tiles = (T + tok - 1) / tok;
+      if (disp != nullptr && logits == nullptr &&
+          (all || (disp->row_w == nullptr && disp->ws != nullptr && tiles <= kIndexTilesMax &&
+                   disp->ws_bytes >= fs2moe_dispatch_workspace_bytes(T, K, E)))) {
+        uint8_t* tile_counts = all ? nullptr : tile_counts_of(disp->ws);
+        int32_t* tile_rank = all ? nullptr : tile_rank_of(disp->ws, T, E, tok);
+#define FS2_FINISH_CASE(JJ)                                                                        \
+  case JJ:                                                                                         \
+    hipLaunchKernelGGL((all                 ? router_finish_tile_kernel<JJ, true, kRouterTileTok>  \
+                        : tok == kFinishTok ? router_finish_tile_kernel<JJ, false, kFinishTok>     \
+                                            : router_finish_tile_kernel<JJ, false, kRouterTileTok>), \
+                       dim3(tiles), dim3(tok == kFinishTok ? finish_tile_threads<kFinishTok>()     \
+                                                           : finish_tile_threads<kRouterTileTok>()), \
+                       0, s, partial, slices, bias, T, E, K, \
+                       score_fn, renormalize, topk_idx, topk_w, tile_counts, tile_rank, disp->tile_m, \
+                       disp->max_rows, disp->counts, disp->offsets, disp->perm, disp->inv_perm,    \
+                       disp->row_w);                                                               \
     break;
         switch (j) {
           FS2_FINISH_CASE(1)
@@ -1268,7 +1481,11 @@ static int router_entry(const void* x, const void* norm_w, float norm_eps, void*
           FS2_FINISH_CASE(4)
         }
 #undef FS2_FINISH_CASE
-        if (int rc = check_launch("router_finish_dispatch")) return rc;
+        if (int rc = check_launch("router_finish_tile")) return rc;
+        if (!all)
+          if (int rc = dispatch_index_tiles(topk_idx, T, K, E, tok, disp->tile_m, disp->max_rows, tile_counts,
+                                            tile_rank, disp->counts, disp->offsets, disp->perm, disp->inv_perm, stream))
+            return rc;
         disp->done = true;
         return FS2MOE_OK;
       }

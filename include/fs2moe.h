@@ -456,6 +456,28 @@ int fs2moe_rms_norm_backward(const void* x, const void* weight, float eps, const
                              void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * fs2moe_forward (normed 0) or fs2moe_forward_norm (normed 1) with their arguments in a struct, for
+ * callers that prepare them once and change a few pointers from call to call.
+ */
+typedef struct fs2moe_forward_args {
+  int32_t T, D, E, K, F, F_shared, tile_m, act_dtype, w_dtype;
+  int32_t score_fn, renormalize, scale_input, normed;
+  float norm_eps;
+  const void *x, *norm_weight, *residual, *router;
+  const float* router_bias;
+  const void *w_gate, *w_up, *w_down;
+  const float *s_gate, *s_up, *s_down;
+  const void *shared_gate, *shared_up, *shared_down;
+  void* workspace;
+  int64_t workspace_bytes;
+  void* out;
+} fs2moe_forward_args;
+int fs2moe_forward_call(const fs2moe_forward_args* args, void* stream);
+
+/* Copies bytes from src to dst (device memory that does not overlap) by a kernel. */
+int fs2moe_copy(const void* src, void* dst, int64_t bytes, void* stream);
+
+/*
  * A training step of the layer in two calls, one per pass: the stages above in their order, on two
  * buffers of the caller's (what autograd would keep between the passes, and scratch).  SiLU gate,
  * weights in the activation dtype.  What the stage calls do one at a time is done together where that

@@ -924,3 +924,45 @@ def test_layer_arguments_are_validated_before_the_gpu_reads_them(gpu_device):
     assert ex.gate_q.dtype == torch.float8_e4m3fn and ex.gate_scale.dtype == torch.float32
     with torch.no_grad():
         m(x)
+
+
+def test_repeated_calls_follow_the_module(gpu_device):
+    """A call in the state of an earlier one reuses its arguments: what changes between calls is seen."""
+    import copy
+
+    from fairseq2_amd import MoE
+
+    torch.manual_seed(3)
+    with torch.device(gpu_device):
+        layer, other = (MoE(128, 64, True, 8, 1.0, 2, inner_dim_scale=1.0, auto_scale=False).bfloat16()
+                        for _ in range(2))
+        norm = torch.nn.RMSNorm(128, eps=1e-6).bfloat16()
+        for p in (*layer.parameters(), *other.parameters()):
+            torch.nn.init.normal_(p, 0.0, 0.05)
+        x, y = (torch.randn(2, 40, 128).bfloat16() for _ in range(2))
+
+    def staged(m, rows):
+        r = rows.reshape(-1, 128)
+        return m._stages(r, r, m._norm_args(norm, r))[0].view(rows.shape)
+
+    with torch.inference_mode(), torch.no_grad():
+        call = lambda m, rows: m(rows, residual=rows, norm=norm)  # noqa: E731
+        first = call(layer, x)
+        assert torch.equal(call(layer, x), first) and torch.equal(first, staged(layer, x))
+        assert torch.equal(call(layer, y), staged(layer, y))
+        twin = copy.deepcopy(layer)
+        assert torch.equal(call(twin, x), first)
+    with torch.no_grad():
+        layer.router.data = other.router.data
+        assert torch.equal(call(layer, x), staged(layer, x)) and not torch.equal(call(layer, x), first)
+        layer.experts.gate_proj.mul_(0.5)
+        assert torch.equal(call(layer, x), staged(layer, x))
+        layer.top_k = 3
+        assert torch.equal(call(layer, x), staged(layer, x))
+        layer.experts = other.experts
+        layer.shared_expert = None
+        assert torch.equal(call(layer, x), staged(layer, x))
+        norm.eps = 0.5
+        assert torch.equal(call(layer, x), staged(layer, x))
+        assert torch.equal(call(layer, x[:1]), staged(layer, x[:1]))
+        assert torch.equal(call(twin, x.transpose(0, 1)), staged(twin, x.transpose(0, 1).contiguous()))

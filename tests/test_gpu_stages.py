@@ -75,6 +75,42 @@ def test_router_matches_oracle(gpu_device, dtype, tokens, d, e, k, mode, zipf):
         assert torch.equal(gl, sl) and torch.equal(gw, sw)
 
 
+# Numbers of experts that are no multiple of 8 on the matrix-pipe router (rows of the matrix begin anywhere, the
+# last chunk ends past it), and the bookkeeping that the router's kernels leave to the whole-layer call: in one
+# block (up to 32 tokens), in tiles of 8 (up to 1024) and of 32, with one step of the model dimension to a
+# block (normalised on the way) and with several.
+@pytest.mark.parametrize("tokens,d,e,k", [
+    (1, 512, 60, 6), (32, 2048, 132, 32), (33, 1024, 60, 8), (257, 2048, 250, 5), (1024, 320, 9, 2),
+    (1025, 2048, 60, 4), (40, 5120, 7, 3), (8200, 128, 60, 6),
+])
+@pytest.mark.parametrize("normed", [False, True])
+def test_router_and_bookkeeping_in_the_whole_layer_call(gpu_device, tokens, d, e, k, normed):
+    from fairseq2_amd import MoE
+
+    _say("router and bookkeeping", tokens, d, e, k, normed)
+    g = torch.Generator().manual_seed(tokens + e)
+    x = torch.randn(tokens, d, generator=g).bfloat16().to(gpu_device)
+    with torch.device(gpu_device):
+        layer = MoE(d, 64, False, e, 1.0, k, inner_dim_scale=1.0, auto_scale=False, score_fn="softmax", scale_on="output")
+        norm = torch.nn.RMSNorm(d, eps=1e-6) if normed else None
+    layer.bfloat16().requires_grad_(False)
+    for p in layer.parameters():
+        p.normal_(0.0, 0.05)
+    if normed:
+        norm.bfloat16().requires_grad_(False).weight.normal_(1.0, 0.1)
+    router = layer.router.detach()
+    idx, _, logits = _abi.router_topk(x, router, None, k, _abi.SCORE_SOFTMAX, want_logits=True)
+    ref = x.double().cpu() @ router.double().cpu()
+    np.testing.assert_allclose(logits.cpu().double().numpy(), ref.numpy(), rtol=1e-5, atol=1e-4)
+    host, _ = _abi.cpu_router_select(logits, k, _abi.SCORE_SOFTMAX)
+    assert torch.equal(idx.cpu(), host)
+    with torch.inference_mode():
+        whole = layer(x, norm=norm)
+        again = layer(x, norm=norm)
+        staged = layer._stages(x, None, layer._norm_args(norm, x))[0]
+    assert torch.equal(whole, again) and torch.equal(whole, staged)
+
+
 @pytest.mark.parametrize(
     "tokens,d,e,k,mode,zipf",
     [
