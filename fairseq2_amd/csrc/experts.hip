@@ -313,7 +313,17 @@ static bool gemv_applies(int act_dtype, int D, int F, const Groups& g, int rows_
       rows_hint > FS2MOE_GEMV_MAX_ROWS)
     return false;
   const int r = rows_hint <= 1 ? 1 : rows_hint <= 2 ? 2 : 4;
-  return gemv::fits(D > F ? D : F, r);
+  return gemv::offsets_fit(D, F) && gemv::fits(D > F ? D : F, r);
+}
+
+// How many experts' blocks are launched at a time, of about `blocks` in all.  More than run at once (two to
+// a CU), since blocks that the hardware starts as others end balance better than blocks that go on to
+// another expert (16 tokens, 81 experts: the down projection 60 us with 768, 57 with 2048); but a token or
+// two reach a few experts only, and the blocks that find none take their time too (one token, the down
+// projection: 7.2 us with 512 blocks, 10.6 with 2048).
+static unsigned stream_experts(int blocks, int col_blocks, int E) {
+  const int n = (blocks + col_blocks - 1) / col_blocks;
+  return (unsigned)(n < E ? n : E);
 }
 
 template <int R>
@@ -339,17 +349,18 @@ static int launch_gemv_pair_r(const void* x, const int32_t* row_map, const float
     attr_set = true;
   }
   const uint16_t* xp = static_cast<const uint16_t*>(x);
-  hipLaunchKernelGGL(k1, dim3((unsigned)((F + COLS - 1) / COLS), (unsigned)g.E), dim3(threads(R)),
+  const int f_blocks = (F + COLS - 1) / COLS, d_blocks = (D + COLS - 1) / COLS;
+  hipLaunchKernelGGL(k1, dim3((unsigned)f_blocks, stream_experts(256 * (R + 1), f_blocks, g.E)), dim3(threads(R)),
                      (size_t)R * D * 2, stream, xp, row_map, row_w, D, static_cast<const uint16_t*>(w_gate),
                      static_cast<const uint16_t*>(w_up), static_cast<uint16_t*>(h), F, D, F,
-                     g.counts, g.offsets);
+                     g.counts, g.offsets, g.E);
   if (int rc = check_launch("glu_gemv_bf16<gate,up>")) return rc;
-  hipLaunchKernelGGL(deep_applies(F, R) ? k2d : k2, dim3((unsigned)((D + COLS - 1) / COLS), (unsigned)g.E),
+  hipLaunchKernelGGL(deep_applies(F, R) ? k2d : k2, dim3((unsigned)d_blocks, stream_experts(256 * (R + 1), d_blocks, g.E)),
                      dim3(threads(R)), (size_t)R * F * 2, stream, static_cast<const uint16_t*>(h),
                      static_cast<const int32_t*>(nullptr), static_cast<const float*>(nullptr), F,
                      static_cast<const uint16_t*>(w_down),
                      static_cast<const uint16_t*>(nullptr), static_cast<uint16_t*>(y), D, F, D,
-                     g.counts, g.offsets);
+                     g.counts, g.offsets, g.E);
   return check_launch("glu_gemv_bf16<down>");
 }
 
@@ -365,7 +376,7 @@ static bool gemv16_applies(int act_dtype, int D, int F, const Groups& g, int row
   if (act_dtype != FS2MOE_BF16 || g.counts == nullptr || g.E > 256 ||
       rows_hint <= FS2MOE_GEMV_MAX_ROWS || rows_hint > FS2MOE_GEMV16_MAX_ROWS)
     return false;
-  return gemv16::offsets_fit(D, F) && gemv16::fits(D > F ? D : F, 8);
+  return gemv::offsets_fit(D, F) && gemv16::fits(D > F ? D : F, 8);
 }
 // rows staged per pass: 16 when the bound asks for it and rows that long fit LDS, else 8 (an expert
 // with more rows is walked again)
@@ -392,17 +403,18 @@ static int launch_gemv16_pair(const void* x, const int32_t* row_map, const float
     }
     attr_set = true;
   }
-  hipLaunchKernelGGL(k1, dim3((unsigned)((F + COLS - 1) / COLS), (unsigned)g.E), dim3(THREADS),
+  const int f_blocks = (F + COLS - 1) / COLS, d_blocks = (D + COLS - 1) / COLS;
+  hipLaunchKernelGGL(k1, dim3((unsigned)f_blocks, stream_experts(2048, f_blocks, g.E)), dim3(THREADS),
                      lds_bytes(D, XR, true), stream, static_cast<const uint16_t*>(x), row_map, row_w, D,
                      static_cast<const uint16_t*>(w_gate), static_cast<const uint16_t*>(w_up),
-                     static_cast<uint16_t*>(h), F, D, F, g.counts, g.offsets);
+                     static_cast<uint16_t*>(h), F, D, F, g.counts, g.offsets, g.E);
   if (int rc = check_launch("glu_gemv16_bf16<gate,up>")) return rc;
-  hipLaunchKernelGGL(k2, dim3((unsigned)((D + COLS - 1) / COLS), (unsigned)g.E), dim3(THREADS),
+  hipLaunchKernelGGL(k2, dim3((unsigned)d_blocks, stream_experts(2048, d_blocks, g.E)), dim3(THREADS),
                      lds_bytes(F, XR, false), stream, static_cast<const uint16_t*>(h),
                      static_cast<const int32_t*>(nullptr), static_cast<const float*>(nullptr), F,
                      static_cast<const uint16_t*>(w_down),
                      static_cast<const uint16_t*>(nullptr), static_cast<uint16_t*>(y), D, F, D,
-                     g.counts, g.offsets);
+                     g.counts, g.offsets, g.E);
   return check_launch("glu_gemv16_bf16<down>");
 }
 

@@ -19,6 +19,8 @@
 // expert on the arithmetic no longer hides behind the stream and the GEMM tiles are faster.
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace fs2moe {
@@ -30,15 +32,25 @@ constexpr int waves(int R) { return 8; }
 constexpr int threads(int R) { return 64 * waves(R); }
 constexpr int MAX_LDS_BYTES = 144 * 1024;  // (160 KB less the kernel's own partial sums, 16 KB at most)
 inline bool fits(int K, int R) { return (int64_t)K * R * 2 <= MAX_LDS_BYTES; }
-// Steps of K (256 rows a block) whose loads a wave issues before it multiplies any: 4 with one or
-// two rows, 2 with four (registers).  DEEP: 8, for the single product with one or two rows over a
+// Steps of K (256 rows a block) whose loads a wave has in flight: 4 with one or two rows, 2 with four
+// (registers).  DEEP: 8, for the single product with one or two rows over a
 // long K, where a block is a chain of K / 256 / U round trips (Mixtral's down projection, K 14336:
 // the layer at one token 225 -> 178 us, at two 286 -> 251; a short K would only issue loads that it
 // then masks: Qwen3's K of 768 is three steps, and two tokens took 54 instead of 48 us with 8).
 // The sums do not depend on it: a lane adds its products in the same order.
 constexpr int steps_in_flight(bool dual, int R, bool deep) { return R > 2 ? 2 : (deep && !dual) ? 8 : 4; }
 inline bool deep_applies(int K, int R) { return R <= 2 && K >= 4096; }
+// (one expert's matrix is addressed with 32-bit byte offsets, by up to 4096 rows past its end)
+inline bool offsets_fit(int D, int F) {
+  const int64_t lo = D < F ? D : F, hi = D < F ? F : D;
+  return (lo + 4096) * hi * 2 < 0xffffffffll && (hi + 4096) * lo * 2 < 0xffffffffll;
+}
 }  // namespace gemv
+// One expert's matrix as a buffer: a row past its end reads as zeros, without memory traffic.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t expert_matrix(const uint16_t* B, int e, int K, int N) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(B + (size_t)e * K * N), 0,
+                                           (int)((uint32_t)K * (uint32_t)N * 2u), 0x00020000);
+}
 
 // The n-th expert that has rows, -1 when there are fewer (wave-uniform; every wave works it out for
 // itself from the counts, without LDS or a barrier: E <= 256 is four ballots).  A block takes the
@@ -46,9 +58,12 @@ inline bool deep_applies(int K, int R) { return R <= 2 && K >= 4096; }
 // once wherever they are, but numbered this way the blocks that work are contiguous in launch order
 // whatever the experts' numbers, and consecutive blocks go to consecutive XCDs.  With the real routing
 // of 12 tokens (24 experts active, scattered over 128) the blocks of the block-per-CU kernel below
-// crowded on some XCDs and its pair of launches took 73 instead of 54 us.
+// crowded on some XCDs and its pair of launches took 73 instead of 54 us.  The grid holds about as many
+// blocks as run at once, and a block goes on to the expert gridDim.y further: with a block for every
+// expert there may be, the last of those without rows began a microsecond or two after the others' end.
 __device__ __forceinline__ int nth_active_expert(const int32_t* __restrict__ counts, int E, int n) {
-  const int lane = threadIdx.x & 63;
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));  // (nothing of this is kept from one expert to the next)
   int c[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -71,14 +86,14 @@ __device__ __forceinline__ int nth_active_expert(const int32_t* __restrict__ cou
 // A rows are read through row_map when it is given (row r of the expert is A[row_map[offset + r]]),
 // and multiplied by row_w[offset + r] on the way into LDS when that is given (rounded to bf16: the
 // bits dispatch's scaled row copy would have held).
-// grid: (ceil(N / 64), E).  K a multiple of 4, N a multiple of 8.
+// grid: (ceil(N / 64), as many experts at a time as fill the chip).  K a multiple of 4, N a multiple of 8.
 template <bool DUAL, int R, bool DEEP = false>
 __global__ __launch_bounds__(gemv::threads(R)) void glu_gemv_bf16_kernel(
     const uint16_t* __restrict__ A, const int32_t* __restrict__ row_map,
     const float* __restrict__ row_w, int lda,
     const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1, uint16_t* __restrict__ C,
     int ldc, int K, int N, const int32_t* __restrict__ counts,
-    const int32_t* __restrict__ offsets) {
+    const int32_t* __restrict__ offsets, int E) {
   using namespace gemv;
   constexpr int M = DUAL ? 2 : 1;
   constexpr int NW = waves(R), THREADS = threads(R);
@@ -87,41 +102,98 @@ __global__ __launch_bounds__(gemv::threads(R)) void glu_gemv_bf16_kernel(
   uint16_t* xs = reinterpret_cast<uint16_t*>(gemv_smem);  // [R][K]
   __shared__ float red[NW][M][R][COLS];
 
-  const int e = blockIdx.y;
-  const int cnt = counts[e];
-  if (cnt == 0) return;
-  const int off = offsets[e];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ks = lane >> 3, cc = lane & 7;
   const int col = blockIdx.x * COLS + cc * 8;
   const bool col_ok = col < N;  // N is a multiple of 8: the lane's eight channels are in or out together
-  const size_t wbase = (size_t)e * K * N + (col_ok ? col : 0);
-  const uint16_t* w0 = B0 + wbase;
-  const uint16_t* w1 = DUAL ? B1 + wbase : w0;
+  for (int nth = blockIdx.y;; nth += (int)gridDim.y) {
+  const int e = nth_active_expert(counts, E, nth);
+  if (e < 0) return;
+  const int cnt = counts[e], off = offsets[e];
+  const __amdgpu_buffer_rsrc_t w_rsrc[2] = {expert_matrix(B0, e, K, N), expert_matrix(DUAL ? B1 : B0, e, K, N)};
+  // U steps of K are in flight, each loaded into the registers of the one U before it as soon as that has
+  // been multiplied.  The first of them are issued before the rows are even looked up: they need only the
+  // expert's number, and a decode step's block is a chain of round trips (one token, D 2048 / F 768: the
+  // pair 23.1 -> 20.4 us).
+  constexpr int U = gemv::steps_in_flight(DUAL, R, DEEP);
+  u32x4 wv[U][M][4];
+  // (a lane's four rows of a step are in or out of the matrix together, so that the first one's offset
+  // decides; the others add a scalar to it)
+  uint32_t at;  // the lane's place in the next step
+  auto rewind = [&]() {
+    uint32_t row = (uint32_t)(wave * 32 + ks * 4);
+    asm volatile("" : "+v"(row));  // (else addresses are computed in front of the passes and kept)
+    at = (row * (uint32_t)N + (uint32_t)(col_ok ? col : 0)) * 2u;
+  };
+  auto load_step = [&](int set) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int m = 0; m < M; ++m) wv[set][m][j] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc[m], at, j * N * 2, 0);
+    at += (uint32_t)KSTEP * (uint32_t)N * 2u;
+  };
+  const int steps = (K + KSTEP - 1) / KSTEP;
 
   for (int r0 = 0; r0 < cnt; r0 += R) {
+    // (where rows are looked up, half of the steps go in front of that and half behind the rows' loads;
+    // the down projection's rows lie in order and come from L2: they go first)
+    constexpr int FRONT = DUAL ? U / 2 : 0;
+    rewind();
+#pragma unroll
+    for (int u = 0; u < FRONT; ++u) load_step(u);
+    __builtin_amdgcn_sched_barrier(0);
     // ---- the pass's rows -> LDS (rows past the expert's count as zeros) ---------------------------
-    if (r0 > 0) __syncthreads();  // the previous pass's reads of xs and red are over
+    __syncthreads();  // the previous pass's reads of xs and red are over
     const int kchunks = K / 4;    // 8-byte pieces per row
-    for (int i = tid; i < R * kchunks; i += THREADS) {
-      const int r = i / kchunks, c = i - r * kchunks;
-      u32x2 v = {0u, 0u};
-      if (r0 + r < cnt) {
-        const int row = off + r0 + r;
-        const size_t src = (size_t)(row_map != nullptr ? row_map[row] : row) * lda;
-        v = *reinterpret_cast<const u32x2*>(A + src + 4 * c);
-        if (row_w != nullptr) {
-          const float w = row_w[row];
-          v = u32x2{scale_bf16x2(v[0], w), scale_bf16x2(v[1], w)};
-        }
-      }
-      *reinterpret_cast<u32x2*>(xs + (size_t)r * K + 4 * c) = v;
+    // (rows the expert does not have are skipped, block-uniformly: R only bounds the registers; where
+    // a row lies is wave-uniform, and looked up by scalar loads, which do not wait for the vector ones)
+    const int rcnt = __builtin_amdgcn_readfirstlane(cnt - r0 < R ? cnt - r0 : R);
+    size_t src[R];
+    float rw[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int row = off + r0 + (r < rcnt ? r : 0);
+      src[r] = (size_t)(row_map != nullptr ? row_map[row] : row) * lda;
+      rw[r] = row_w != nullptr ? row_w[row] : 1.f;
     }
-    __syncthreads();
+    constexpr int AHEAD = R > 2 ? 1 : 2;  // pieces of each row in flight per thread
+    u32x2 v[R][AHEAD];
+    auto load_rows = [&](int c0) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+          const int c = c0 + i * THREADS;
+          v[r][i] = *reinterpret_cast<const u32x2*>(A + src[r] + 4 * (c < kchunks ? c : 0));
+        }
+    };
+    auto store_rows = [&](int c0) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+          const int c = c0 + i * THREADS;
+          u32x2 q = v[r][i];
+          if (r >= rcnt) q = u32x2{0u, 0u};
+          if (row_w != nullptr) q = u32x2{scale_bf16x2(q[0], rw[r]), scale_bf16x2(q[1], rw[r])};
+          if (c < kchunks) *reinterpret_cast<u32x2*>(xs + (size_t)r * K + 4 * c) = q;
+        }
+    };
+    load_rows(tid);
+    // (behind the first of the rows, which are waited for first)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = FRONT; u < U; ++u) load_step(u);
+    __builtin_amdgcn_sched_barrier(0);
+    store_rows(tid);
+    for (int c0 = tid + AHEAD * THREADS; c0 < kchunks; c0 += AHEAD * THREADS) {
+      load_rows(c0);
+      store_rows(c0);
+    }
+    lds_barrier();
 
     // ---- the stream over K --------------------------------------------------------------------------
-    // (rows the expert does not have are skipped, block-uniformly: R only bounds the registers)
-    const int rcnt = __builtin_amdgcn_readfirstlane(cnt - r0 < R ? cnt - r0 : R);
     float acc[M][R][8];
 #pragma unroll
     for (int m = 0; m < M; ++m)
@@ -129,61 +201,54 @@ __global__ __launch_bounds__(gemv::threads(R)) void glu_gemv_bf16_kernel(
       for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int c = 0; c < 8; ++c) acc[m][r][c] = 0.f;
-    // U steps of K per iteration, all their loads issued before any arithmetic: a step is one round
-    // trip to memory and little else, so the steps' round trips overlap
-    constexpr int U = gemv::steps_in_flight(DUAL, R, DEEP);
-    for (int kb0 = 0; kb0 < K; kb0 += U * KSTEP) {
-      u32x4 wvu[U][M][4];
+    // (the last U steps load nothing: loads past K's end cost as much of the CU's load path as others)
+    auto multiply = [&](int s0, auto more) {
 #pragma unroll
-      for (int uu = 0; uu < U; ++uu) {
-        const int k0 = kb0 + uu * KSTEP + wave * 32 + ks * 4;
-        const int kk = k0 < K ? k0 : 0;
+      for (int u = 0; u < U; ++u) {
+        const int k0 = (s0 + u) * KSTEP + wave * 32 + ks * 4;
+        const bool k_ok = k0 < K;  // K is a multiple of 4: the lane's four rows are in or out together
+        const int kk = k_ok ? k0 : 0;
+        float xv[R][4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          wvu[uu][0][j] = *reinterpret_cast<const u32x4*>(w0 + (size_t)(kk + j) * N);
-          if (DUAL) wvu[uu][M - 1][j] = *reinterpret_cast<const u32x4*>(w1 + (size_t)(kk + j) * N);
-        }
-      }
-      // (without the fence the compiler moves every load down to its first use and waits for each
-      // one there: one round trip per load instead of one per iteration)
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int uu = 0; uu < U; ++uu) {
-      const int k0 = kb0 + uu * KSTEP + wave * 32 + ks * 4;
-      const bool k_ok = k0 < K;  // K is a multiple of 4: the lane's four rows are in or out together
-      const int kk = k_ok ? k0 : 0;
-      const u32x4 (&wv)[M][4] = wvu[uu];
-      float xv[R][4];
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if (r < rcnt) {
-          const u32x2 q = *reinterpret_cast<const u32x2*>(xs + (size_t)r * K + kk);
-          xv[r][0] = k_ok ? __uint_as_float(q[0] << 16) : 0.f;
-          xv[r][1] = k_ok ? __uint_as_float(q[0] & 0xffff0000u) : 0.f;
-          xv[r][2] = k_ok ? __uint_as_float(q[1] << 16) : 0.f;
-          xv[r][3] = k_ok ? __uint_as_float(q[1] & 0xffff0000u) : 0.f;
-        }
-      }
-#pragma unroll
-      for (int m = 0; m < M; ++m)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float wf[8];
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            wf[2 * c] = __uint_as_float(wv[m][j][c] << 16);
-            wf[2 * c + 1] = __uint_as_float(wv[m][j][c] & 0xffff0000u);
+        for (int r = 0; r < R; ++r) {
+          if (r < rcnt) {
+            const u32x2 q = *reinterpret_cast<const u32x2*>(xs + (size_t)r * K + kk);
+            xv[r][0] = k_ok ? __uint_as_float(q[0] << 16) : 0.f;
+            xv[r][1] = k_ok ? __uint_as_float(q[0] & 0xffff0000u) : 0.f;
+            xv[r][2] = k_ok ? __uint_as_float(q[1] << 16) : 0.f;
+            xv[r][3] = k_ok ? __uint_as_float(q[1] & 0xffff0000u) : 0.f;
           }
+        }
 #pragma unroll
-          for (int r = 0; r < R; ++r) {
-            if (r < rcnt) {
+        for (int m = 0; m < M; ++m)
 #pragma unroll
-              for (int c = 0; c < 8; ++c) acc[m][r][c] += xv[r][j] * wf[c];
+          for (int j = 0; j < 4; ++j) {
+            float wf[8];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              wf[2 * c] = __uint_as_float(wv[u][m][j][c] << 16);
+              wf[2 * c + 1] = __uint_as_float(wv[u][m][j][c] & 0xffff0000u);
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              if (r < rcnt) {
+#pragma unroll
+                for (int c = 0; c < 8; ++c) acc[m][r][c] += xv[r][j] * wf[c];
+              }
             }
           }
+        // (without the fences the compiler moves every load down to its first use and waits for each
+        // one there: one round trip per load)
+        if constexpr (decltype(more)::value) {
+          __builtin_amdgcn_sched_barrier(0);
+          load_step(u);
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
-    }
+    };
+    int s0 = 0;
+    for (; s0 + U < steps; s0 += U) multiply(s0, std::true_type{});
+    multiply(s0, std::false_type{});
 
     // ---- lane groups (fixed order: exchange distances 8, 16, 32), then waves through LDS ------------
 #pragma unroll
@@ -224,6 +289,7 @@ __global__ __launch_bounds__(gemv::threads(R)) void glu_gemv_bf16_kernel(
       C[(size_t)(off + r0 + r) * ldc + n] = f32_to_bf16_bits(g);
     }
   }
+  }
 }
 
 
@@ -256,11 +322,9 @@ inline size_t lds_bytes(int K, int XR, bool dual) {
   return xs > red ? xs : red;
 }
 inline bool fits(int K, int XR) { return lds_bytes(K, XR, true) <= (size_t)MAX_LDS_BYTES; }
-// (one expert's matrix is addressed with 32-bit byte offsets)
-inline bool offsets_fit(int D, int F) { return (int64_t)D * F * 2 <= 0xffffffffll; }
 }  // namespace gemv16
 
-// Arguments as glu_gemv_bf16_kernel.  grid: (ceil(N / 128), E).  K and N multiples of 8.
+// Arguments as glu_gemv_bf16_kernel.  grid: (ceil(N / 128), experts at a time).  K and N multiples of 8.
 // (The second launch bound is waves per SIMD: the single product is held to 128 registers so that
 // two blocks share a CU -- the down projection of 20 active experts is 320 blocks, which at one block
 // per CU ran as a full round and a quarter-full one: 4 us of 75 at 8 tokens.)
@@ -270,73 +334,116 @@ __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16
     const float* __restrict__ row_w, int lda,
     const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1, uint16_t* __restrict__ C,
     int ldc, int K, int N, const int32_t* __restrict__ counts,
-    const int32_t* __restrict__ offsets) {
+    const int32_t* __restrict__ offsets, int E) {
   using namespace gemv16;
   constexpr int M = DUAL ? 2 : 1;
-  constexpr int PAIRS = DUAL ? 1 : 2;  // pairs of steps per iteration: 16 loads in flight per lane
+  constexpr int SETS = 2;  // pairs of steps in flight: 32 (DUAL) or 16 loads per lane
   extern __shared__ __attribute__((aligned(16))) uint8_t gemv16_smem[];
   uint16_t* xs = reinterpret_cast<uint16_t*>(gemv16_smem);  // [XR][K + 4], then 4 zeros
   float* red = reinterpret_cast<float*>(gemv16_smem);       // [4][M][32][64], after the stream
 
-  const int e = nth_active_expert(counts, (int)gridDim.y, (int)blockIdx.y);
-  if (e < 0) return;
-  const int cnt = counts[e];
-  const int off = offsets[e];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ldx = stride(K);
-  const int col = blockIdx.x * COLS + c16 * 8;
-  const bool col_ok = col < N;  // N is a multiple of 8: the lane's eight channels are in or out together
-  // the expert's matrices as uniform bases, a lane's place in them as a 32-bit byte offset (one
-  // register per address, shared by gate and up)
-  const uint8_t* w0 = reinterpret_cast<const uint8_t*>(B0 + (size_t)e * K * N);
-  const uint8_t* w1 = DUAL ? reinterpret_cast<const uint8_t*>(B1 + (size_t)e * K * N) : w0;
-  const uint32_t lane_col = (uint32_t)(col_ok ? col : 0);
-  const uint16_t* xzero = xs + (size_t)XR * ldx;
-  const uint16_t* xrow = xs + (size_t)c16 * ldx;  // row m = c16 of the pass, if it is staged
-  const bool row_ok = c16 < XR;
+  for (int nth = blockIdx.y;; nth += (int)gridDim.y) {
+  const int e = nth_active_expert(counts, E, nth);
+  if (e < 0) return;
+  const int cnt = counts[e], off = offsets[e];
+  // the expert's matrices as buffers, a lane's place in them as a 32-bit byte offset (one register per
+  // address, shared by gate and up)
+  const __amdgpu_buffer_rsrc_t w_rsrc[2] = {expert_matrix(B0, e, K, N), expert_matrix(DUAL ? B1 : B0, e, K, N)};
+  const int pairs = (K + 2 * KSTEP - 1) / (2 * KSTEP);
 
   for (int r0 = 0; r0 < cnt; r0 += XR) {
+    // (everything a lane derives from its number, anew for each pass: kept across the passes it costs
+    // the registers that the loads need, and a value spilled to memory is read back behind those loads)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, c16 = lane & 15, g = lane >> 4;
+    const int col = blockIdx.x * COLS + c16 * 8;
+    // (N is a multiple of 8: the lane's eight channels are in or out together)
+    const uint32_t lane_col = (uint32_t)(col < N ? col : 0);
+    const bool row_ok = c16 < XR;  // row m = c16 of the pass, if it is staged; else, and past K, zeros
+    const int xzero = XR * ldx, xrow = c16 * ldx, xend = row_ok ? K : 0;
+    // A pair of steps is loaded into the registers of the one SETS before it as soon as that has been
+    // multiplied; the first is issued before the rows are looked up (see glu_gemv_bf16_kernel; 8 tokens,
+    // D 2048 / F 768: 50.3 -> 46.5 us for the pair of launches).
+    u32x4 wq[SETS][2][M][4];
+    uint32_t at = ((uint32_t)(wave * 16 + g * 4) * (uint32_t)N + lane_col) * 2u;  // as in glu_gemv_bf16_kernel
+    auto load_pair = [&](int set) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int m = 0; m < M; ++m)
+            wq[set][h][m][j] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc[m], at, j * N * 2, 0);
+        at += (uint32_t)KSTEP * (uint32_t)N * 2u;
+      }
+    };
+    if (DUAL) load_pair(0);
+    __builtin_amdgcn_sched_barrier(0);
     // ---- the pass's rows -> LDS (rows past the expert's count as zeros) ---------------------------
-    if (r0 > 0) __syncthreads();  // the previous pass's sums have left LDS
+    __syncthreads();  // the previous pass's sums have left LDS
     // (a row per group of threads, so that the row's place is looked up once and a thread's loads
     // are all in flight together; K is a multiple of 8 here: 16-byte pieces)
     {
-      constexpr int TPR = THREADS / XR, INFLIGHT = 4;
-      const int r = tid / TPR, c0 = tid - r * TPR;
+      constexpr int TPR = THREADS / XR, INFLIGHT = DUAL ? 8 : 4;
+      const int r = tid / TPR;
+      const int c0 = tid - r * TPR;
       const int kchunks = K / 8;
       const bool has = r0 + r < cnt;
-      size_t src = 0;
-      float w = 1.f;
-      if (has) {
-        const int row = off + r0 + r;
-        src = (size_t)(row_map != nullptr ? row_map[row] : row) * lda;
-        if (row_w != nullptr) w = row_w[row];
+      // (the places of the rows of a wave, one or two, are uniform: scalar loads, which do not wait for
+      // the vector ones)
+      constexpr int RPW = XR / WAVES;
+      size_t place[RPW];
+      float weight[RPW];
+#pragma unroll
+      for (int i = 0; i < RPW; ++i) {
+        const int rr = r0 + wave * RPW + i, row = off + (rr < cnt ? rr : 0);
+        place[i] = (size_t)(row_map != nullptr ? row_map[row] : row) * lda;
+        weight[i] = row_w != nullptr ? row_w[row] : 1.f;
       }
-      for (int cb = c0; cb < kchunks; cb += TPR * INFLIGHT) {
-        u32x4 v[INFLIGHT];
+      const size_t src = RPW > 1 && lane >= 32 ? place[RPW - 1] : place[0];
+      const float w = RPW > 1 && lane >= 32 ? weight[RPW - 1] : weight[0];
+      u32x4 v[INFLIGHT];
+      auto load_rows = [&](int cb) {
 #pragma unroll
         for (int u = 0; u < INFLIGHT; ++u) {
           const int c = cb + u * TPR;
           v[u] = *reinterpret_cast<const u32x4*>(A + src + 8 * (c < kchunks ? c : 0));
         }
+      };
+      auto store_rows = [&](int cb) {
+        if (row_w != nullptr) {  // (block-uniform; as dispatch's scaled copy rounds)
+#pragma unroll
+          for (int u = 0; u < INFLIGHT; ++u)
+            v[u] = u32x4{scale_bf16x2(v[u][0], w), scale_bf16x2(v[u][1], w), scale_bf16x2(v[u][2], w),
+                         scale_bf16x2(v[u][3], w)};
+        }
 #pragma unroll
         for (int u = 0; u < INFLIGHT; ++u) {
           const int c = cb + u * TPR;
-          if (c >= kchunks) continue;
           if (!has) v[u] = u32x4{0u, 0u, 0u, 0u};
-          if (row_w != nullptr)  // (block-uniform; as dispatch's scaled copy rounds)
-            v[u] = u32x4{scale_bf16x2(v[u][0], w), scale_bf16x2(v[u][1], w), scale_bf16x2(v[u][2], w),
-                         scale_bf16x2(v[u][3], w)};
+          if (c >= kchunks) continue;
           u32x2* dst = reinterpret_cast<u32x2*>(xs + (size_t)r * ldx + 8 * c);  // 8-byte aligned
           dst[0] = u32x2{v[u][0], v[u][1]};
           dst[1] = u32x2{v[u][2], v[u][3]};
         }
+      };
+      load_rows(c0);
+      // (behind the first of the rows, which are waited for first)
+      __builtin_amdgcn_sched_barrier(0);
+      if (!DUAL) load_pair(0);
+      load_pair(1);
+      __builtin_amdgcn_sched_barrier(0);
+      store_rows(c0);
+      for (int cb = c0 + TPR * INFLIGHT; cb < kchunks; cb += TPR * INFLIGHT) {
+        load_rows(cb);
+        store_rows(cb);
       }
     }
     if (tid < 4) xs[(size_t)XR * ldx + tid] = 0;
-    __syncthreads();
+    lds_barrier();
 
     // ---- the stream over K --------------------------------------------------------------------------
     f32x4 acc[M][8];
@@ -344,29 +451,19 @@ __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16
     for (int m = 0; m < M; ++m)
 #pragma unroll
       for (int c = 0; c < 8; ++c) acc[m][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int kb0 = 0; kb0 < K; kb0 += 2 * PAIRS * KSTEP) {
-      u32x4 wq[2 * PAIRS][M][4];
-      u32x2 xq[2 * PAIRS];
+    int xk = wave * 16 + g * 4;  // the lane's first k of the next step
+    auto multiply = [&](auto more) {  // (as in glu_gemv_bf16_kernel)
 #pragma unroll
-      for (int s = 0; s < 2 * PAIRS; ++s) {
-        const int k0 = kb0 + s * KSTEP + wave * 16 + g * 4;
-        const bool k_ok = k0 < K;  // K is a multiple of 4: the lane's four rows are in or out together
-        const int kk = k_ok ? k0 : 0;
+      for (int p = 0; p < SETS; ++p) {
+        u32x2 xq[2];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t at = ((uint32_t)(kk + j) * (uint32_t)N + lane_col) * 2u;
-          wq[s][0][j] = *reinterpret_cast<const u32x4*>(w0 + at);
-          if (DUAL) wq[s][M - 1][j] = *reinterpret_cast<const u32x4*>(w1 + at);
+        for (int h = 0; h < 2; ++h) {
+          // (k rows past K, four together as K is a multiple of 4, meet zeros: chosen by address, a
+          // select on the value would become a branch)
+          xq[h] = *reinterpret_cast<const u32x2*>(xs + (xk < xend ? xrow + xk : xzero));
+          xk += KSTEP;
         }
-        // (k rows past K meet zeros: chosen by address, a select on the value would become a branch)
-        xq[s] = *reinterpret_cast<const u32x2*>(k_ok && row_ok ? xrow + k0 : xzero);
-      }
-      // (without the fence the compiler moves every load down to its first use and waits for each
-      // one there: one round trip per load instead of one per iteration)
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int p = 0; p < PAIRS; ++p) {
-        const u32x4 xo = {xq[2 * p][0], xq[2 * p][1], xq[2 * p + 1][0], xq[2 * p + 1][1]};
+        const u32x4 xo = {xq[0][0], xq[0][1], xq[1][0], xq[1][1]};
         const bf16x8 xop = __builtin_bit_cast(bf16x8, xo);
 #pragma unroll
         for (int m = 0; m < M; ++m)
@@ -374,8 +471,8 @@ __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16
           for (int c = 0; c < 8; ++c) {
             // channel c of the lane: the low (c even) or high (c odd) half of dword c / 2 of each row
             const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;
-            const u32x4(&a)[4] = wq[2 * p][m];
-            const u32x4(&b)[4] = wq[2 * p + 1][m];
+            const u32x4(&a)[4] = wq[p][0][m];
+            const u32x4(&b)[4] = wq[p][1][m];
             const u32x4 wo = {__builtin_amdgcn_perm(a[1][c >> 1], a[0][c >> 1], sel),
                               __builtin_amdgcn_perm(a[3][c >> 1], a[2][c >> 1], sel),
                               __builtin_amdgcn_perm(b[1][c >> 1], b[0][c >> 1], sel),
@@ -384,10 +481,16 @@ __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16
                                                                  acc[m][c], 0, 0, 0);
             // (operands are formed four channels ahead at most: formed all at once they cost 64
             // registers and the kernel spills)
-            if ((c & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+            if ((c & (DUAL ? 3 : 1)) == (DUAL ? 3 : 1)) __builtin_amdgcn_sched_barrier(0);
           }
+        if constexpr (decltype(more)::value) {
+          load_pair(p);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
-    }
+    };
+    for (int p0 = SETS; p0 < pairs; p0 += SETS) multiply(std::true_type{});
+    multiply(std::false_type{});
 
     // ---- the waves' sums meet in LDS: (w + 4) onto w, then (w + 2) onto w, then 1 onto 0 ------------
     __syncthreads();  // every wave is done reading the rows: the sums take their place
@@ -434,6 +537,7 @@ __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16
         *reinterpret_cast<u32x4*>(C + (size_t)(off + r0 + c16) * ldc + n) = o;
       }
     }
+  }
   }
 }
 
