@@ -76,18 +76,22 @@ struct WgradJob {
   int M, N, m_tiles, tiles;  // tiles: per slot
   int grouped, slots, seg_rows, rows;
   int past_cache;  // store C past the caches (see nt_stores)
+  int map_a, map_b;  // MAPPED: this operand's rows are read through the row map
 };
 struct WgradJobs {
   WgradJob job[wgk::MAX_JOBS];
   int n;
 };
 
-// MAPPED: A's rows are read through a_map (one job).  A template parameter, not a test of the pointer:
-// behind a condition the map entry's load is waited for with every other load of the wave (the counter
-// cannot tell them apart at the join), which serialises a chunk's loads into round trips.
+// MAPPED: operands of some gradients are read through the row map (rows of the layer's input, or of its
+// output gradient, that no one has copied into expert order).  The map's entries are scalar loads, two rows
+// per wave and load, asked for before the chunk ahead is stored: vector loads would be waited for with every
+// other load of the wave, a round trip per chunk.  128 experts of about 256 rows, 2048 x 768, the three
+// gradients of a step: 594 us on copied rows, 570 through the map (fewer distinct rows to fetch).  The map
+// holds at least one entry, and one for every row of a gradient in the same launch that does not use it.
 template <bool MAPPED>
 __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
-    const WgradJobs jobs, const int32_t* __restrict__ a_map, const int32_t* __restrict__ counts,
+    const WgradJobs jobs, const int32_t* __restrict__ row_map, const int32_t* __restrict__ counts,
     const int32_t* __restrict__ offsets, int E) {
   using namespace wgk;
   constexpr int ROW_CHUNKS = TM / 8;              // 16-byte chunks per LDS row (32)
@@ -392,8 +396,14 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     // the chunk to load next: rows [ld_off, ld_off + ld_left) of the tile's operands
     const uint16_t* ld_a = nullptr;
     const uint16_t* ld_b = nullptr;
-    const int32_t* ld_map = a_map;
     int ld_left = 0, ld_lda = 0, ld_ldb = 0;
+    // MAPPED: the chunk's first row in expert order, which operands go through the map, and the rows of the
+    // wave's eight pieces (two to a load instruction) in expert order and behind the map
+    typedef u32x4 __attribute__((address_space(1))) GlobalVec;
+    uint64_t zero = (uint64_t)kZero16;
+    asm volatile("" : "+s"(zero));  // (read once)
+    const int kr0 = (wave - CONSUMERS) * 2;
+    int ld_row = 0, ld_map_a = 0, ld_map_b = 0, place[PER_THREAD][2], entry[PER_THREAD][2];
     Deal ld_deal = deal;
     uint32_t oa[PER_THREAD], ob[PER_THREAD];
     int loaded = 0;  // chunks so far (those past the stream's end do not count)
@@ -407,8 +417,10 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
         ld_lda = j.M;
         ld_ldb = j.N;
         ld_a = (MAPPED ? j.A : j.A + (size_t)t.off * j.M) + t.m0;
-        ld_b = j.B + (size_t)t.off * j.N + t.n0;
-        if (MAPPED) ld_map = a_map + t.off;
+        ld_b = (MAPPED ? j.B : j.B + (size_t)t.off * j.N) + t.n0;
+        ld_row = t.off;
+        ld_map_a = j.map_a;
+        ld_map_b = j.map_b;
         ld_left = t.cnt;
         const bool a_ok = t.m0 + ch * 8 < j.M, b_ok = t.n0 + ch * 8 < j.N;
 #pragma unroll
@@ -418,31 +430,40 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
         }
       }
     };
+    auto look_up = [&]() {
+      if (ld_left <= 0) next_tile();
+      if constexpr (MAPPED) {
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i)
+#pragma unroll
+          for (int r = 0; r < 2; ++r) {
+            const int k = kr0 + 8 * i + r, last = ld_left - 1;
+            place[i][r] = last >= 0 ? ld_row + (k < last ? k : last) : 0;
+            entry[i][r] = row_map[place[i][r]];
+          }
+      }
+    };
     auto load_chunk = [&](auto set_c) {
       constexpr int set = decltype(set_c)::value;
-      if (ld_left <= 0) next_tile();
       loaded += ld_left > 0 ? 1 : 0;
-      const __amdgpu_buffer_rsrc_t b_rsrc =
-          __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(ld_b), 0, 0xfffffff0u, 0x00020000);
-      if constexpr (MAPPED) {  // all the map entries first, then all the rows
-        int row[PER_THREAD];
-#pragma unroll
-        for (int i = 0; i < PER_THREAD; ++i) {
-          const int k = kr + 8 * i;
-          row[i] = ld_left > 0 ? ld_map[k < ld_left ? k : ld_left - 1] : 0;
-        }
+      if constexpr (MAPPED) {
 #pragma unroll
         for (int i = 0; i < PER_THREAD; ++i) {
           const bool in = kr + 8 * i < ld_left;
-          const uint16_t* p = in && oa[i] != 0xfffffff0u ? ld_a + (size_t)row[i] * ld_lda + ch * 8
-                                                         : reinterpret_cast<const uint16_t*>(kZero16);
-          ra[set][i] = *reinterpret_cast<const u32x4*>(p);
-          rb[set][i] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, in ? ob[i] : 0xfffffff0u, 0, 0);
+          const uint32_t a0 = ld_map_a ? entry[i][0] : place[i][0], a1 = ld_map_a ? entry[i][1] : place[i][1];
+          const uint32_t b0 = ld_map_b ? entry[i][0] : place[i][0], b1 = ld_map_b ? entry[i][1] : place[i][1];
+          const uint64_t pa = (uint64_t)ld_a + ((uint64_t)(lane < 32 ? a0 : a1) * (uint32_t)ld_lda + ch * 8) * 2;
+          const uint64_t pb = (uint64_t)ld_b + ((uint64_t)(lane < 32 ? b0 : b1) * (uint32_t)ld_ldb + ch * 8) * 2;
+          // (the address chosen, by its bits: as pointers the two sides become branches)
+          ra[set][i] = *(const GlobalVec*)((in & (oa[i] != 0xfffffff0u)) ? pa : zero);
+          rb[set][i] = *(const GlobalVec*)((in & (ob[i] != 0xfffffff0u)) ? pb : zero);
         }
-        ld_map += RK;
+        ld_row += RK;
       } else {
         const __amdgpu_buffer_rsrc_t a_rsrc =
             __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(ld_a), 0, 0xfffffff0u, 0x00020000);
+        const __amdgpu_buffer_rsrc_t b_rsrc =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(ld_b), 0, 0xfffffff0u, 0x00020000);
 #pragma unroll
         for (int i = 0; i < PER_THREAD; ++i) {
           const bool in = kr + 8 * i < ld_left;
@@ -450,8 +471,8 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
           rb[set][i] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, in ? ob[i] : 0xfffffff0u, 0, 0);
         }
         ld_a += (size_t)RK * ld_lda;
+        ld_b += (size_t)RK * ld_ldb;
       }
-      ld_b += (size_t)RK * ld_ldb;
       ld_left -= RK;
     };
     auto store_chunk = [&](auto set_c, int buf) {
@@ -469,13 +490,17 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     };
     using Set0 = std::integral_constant<int, 0>;
     using Set1 = std::integral_constant<int, 1>;
+    look_up();
     load_chunk(Set0{});
     if (loaded == 0) return;  // no tile with rows: nothing for the consumers to wait for
+    look_up();
     load_chunk(Set1{});
+    look_up();
     store_chunk(Set0{}, 0);
     load_chunk(Set0{});
     lds_barrier();
     auto step = [&](int g, auto next_set) {
+      look_up();
       store_chunk(next_set, (g + 1) & 1);
       load_chunk(next_set);
       lds_barrier();  // the loads of the next chunks stay in flight
@@ -1013,9 +1038,9 @@ static int launch_wgrad_reduce(const float* partial, int segments, int64_t n, in
 }
 
 // One launch for all gradients of `jobs`; the grouped ones share counts and offsets.
-static int launch_wgrad(const WgradJobs& jobs, const int32_t* a_map, const int32_t* counts,
+static int launch_wgrad(const WgradJobs& jobs, const int32_t* row_map, const int32_t* counts,
                         const int32_t* offsets, int E, hipStream_t st) {
-  auto k = a_map != nullptr ? grouped_wgrad_kernel<true> : grouped_wgrad_kernel<false>;
+  auto k = row_map != nullptr ? grouped_wgrad_kernel<true> : grouped_wgrad_kernel<false>;
   static bool attr_set = false;  // benign race: setting the attribute is idempotent
   if (!attr_set) {
     for (const void* p : {reinterpret_cast<const void*>(grouped_wgrad_kernel<false>),
@@ -1033,7 +1058,7 @@ static int launch_wgrad(const WgradJobs& jobs, const int32_t* a_map, const int32
     set_error("grouped_wgrad: cannot query the compute-unit count");
     return FS2MOE_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(wgk::WAVES * 64), wgk::SMEM_BYTES, st, jobs, a_map,
+  hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(wgk::WAVES * 64), wgk::SMEM_BYTES, st, jobs, row_map,
                      counts, offsets, E);
   return check_launch("grouped_wgrad");
 }
@@ -1086,8 +1111,9 @@ extern "C" int fs2moe_grouped_wgrad(const void* a, const int32_t* a_row_map, con
     jobs.n = 1;
     jobs.job[0] = {static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b),
                    static_cast<uint16_t*>(dw), partial, M, N, m_tiles, m_tiles * n_tiles,
-                   counts != nullptr, slots, seg_rows, (int)max_rows, nt_stores(slots, M, N)};
-    if (int rc = launch_wgrad(jobs, a_row_map, counts, offsets, E, st)) return rc;
+                   counts != nullptr, slots, seg_rows, (int)max_rows, nt_stores(slots, M, N), mapped, 0};
+    // (without rows nothing is read, and the map may be empty)
+    if (int rc = launch_wgrad(jobs, max_rows > 0 ? a_row_map : nullptr, counts, offsets, E, st)) return rc;
   } else {
     const int64_t big = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
     const bool small = f32t::small_tiles(big * slots, 128);
@@ -1137,9 +1163,9 @@ int64_t fs2moe::wgrad_plan(WgradRequest* r, int n, int32_t E, int64_t grouped_ro
   return bytes;
 }
 
-int fs2moe::wgrad_all(const WgradRequest* r, int n, const int32_t* counts, const int32_t* offsets,
-                      int32_t E, int64_t grouped_rows, int64_t rows, int32_t dtype, void* scratch,
-                      void* stream) {
+int fs2moe::wgrad_all(const WgradRequest* r, int n, const int32_t* row_map, const int32_t* counts,
+                      const int32_t* offsets, int32_t E, int64_t grouped_rows, int64_t rows, int32_t dtype,
+                      void* scratch, void* stream) {
   if (dtype == FS2MOE_F32) {
     for (int i = 0; i < n; ++i) {
       const bool g = r[i].grouped;
@@ -1156,19 +1182,21 @@ int fs2moe::wgrad_all(const WgradRequest* r, int n, const int32_t* counts, const
   WgradJobs jobs;
   jobs.n = n;
   float* part = static_cast<float*>(scratch);
-  bool any_grouped = false;
+  bool any_grouped = false, any_mapped = false;
   for (int i = 0; i < n; ++i) {
     const WgradRequest& q = r[i];
     const int mt = (q.M + wgk::TM - 1) / wgk::TM, nt = (q.N + wgk::TN - 1) / wgk::TN;
     any_grouped = any_grouped || q.grouped;
+    any_mapped = any_mapped || q.map_a || q.map_b;
     int segments = q.grouped ? 1 : q.segments;
     const int seg = segment_rows(rows, &segments), slots = q.grouped ? E : segments;
     jobs.job[i] = {static_cast<const uint16_t*>(q.a), static_cast<const uint16_t*>(q.b),
                    static_cast<uint16_t*>(q.dw), !q.grouped && slots > 1 ? part : nullptr, q.M, q.N, mt, mt * nt,
-                   q.grouped ? 1 : 0, slots, q.grouped ? 0 : seg, (int)rows, nt_stores(slots, q.M, q.N)};
+                   q.grouped ? 1 : 0, slots, q.grouped ? 0 : seg, (int)rows, nt_stores(slots, q.M, q.N),
+                   q.map_a, q.map_b};
     if (!q.grouped && slots > 1) part += (int64_t)slots * q.M * q.N;
   }
-  if (int rc = launch_wgrad(jobs, nullptr, any_grouped ? counts : nullptr, any_grouped ? offsets : nullptr,
+  if (int rc = launch_wgrad(jobs, any_mapped ? row_map : nullptr, any_grouped ? counts : nullptr, any_grouped ? offsets : nullptr,
                             any_grouped ? E : 0, st))
     return rc;
   for (int i = 0; i < n; ++i)

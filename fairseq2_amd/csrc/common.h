@@ -264,9 +264,9 @@ int grouped_swiglu_scaled_rows(const void* x, const int32_t* row_map, const floa
 
 // ---- pieces of a training step (fs2moe_train_forward / fs2moe_train_backward)
 // Whether the SwiGLU pair keeps its two products at these sizes, and that pair (E 0: one group of `rows`
-// rows with nn.Linear-oriented weights).
+// rows with nn.Linear-oriented weights; bf16: rows read through row_map where it is not null).
 bool swiglu_train_applies(int32_t dtype, int32_t D, int32_t F, int64_t rows);
-int swiglu_train(const void* x, const int32_t* counts, const int32_t* offsets, int32_t E,
+int swiglu_train(const void* x, const int32_t* row_map, const int32_t* counts, const int32_t* offsets, int32_t E,
                  const void* w_gate, const void* w_up, const void* w_down, int32_t D, int32_t F,
                  int64_t rows, int32_t dtype, void* g, void* u, void* h, void* y, void* stream);
 // c = a1 @ B1 + a2 @ B2 (fs2moe_grouped_gemm's layouts and groups; E 0: one group), one rounding.
@@ -281,12 +281,13 @@ struct WgradRequest {
   int32_t M, N;
   bool grouped;
   int segments;  // set by wgrad_plan: of a group's rows, each with its own partial sums
+  bool map_a = false, map_b = false;  // bf16: the operand's rows are read through the row map
 };
 // Cuts the rows of single groups whose tiles would take longer than the others together; returns the
 // bytes of scratch that the partial sums need.
 int64_t wgrad_plan(WgradRequest* r, int n, int32_t E, int64_t grouped_rows, int64_t rows, int32_t dtype);
-int wgrad_all(const WgradRequest* r, int n, const int32_t* counts, const int32_t* offsets, int32_t E,
-              int64_t grouped_rows, int64_t rows, int32_t dtype, void* scratch, void* stream);
+int wgrad_all(const WgradRequest* r, int n, const int32_t* row_map, const int32_t* counts, const int32_t* offsets,
+              int32_t E, int64_t grouped_rows, int64_t rows, int32_t dtype, void* scratch, void* stream);
 // fs2moe_router_backward into rows of ld >= E elements, those past E zero
 int router_backward_ld(const float* logits, const int32_t* topk_idx, const float* topk_w,
                        const float* d_w, int32_t T, int32_t E, int32_t K, int32_t score_fn,

@@ -807,7 +807,8 @@ bool fs2moe::swiglu_train_applies(int32_t dtype, int32_t D, int32_t F, int64_t r
   return dtype == FS2MOE_F32 || dma_offsets_fit(rows, D, F);
 }
 
-int fs2moe::swiglu_train(const void* x, const int32_t* counts, const int32_t* offsets, int32_t E,
+int fs2moe::swiglu_train(const void* x, const int32_t* row_map, const int32_t* counts,
+                         const int32_t* offsets, int32_t E,
                          const void* w_gate, const void* w_up, const void* w_down, int32_t D,
                          int32_t F, int64_t rows, int32_t dtype, void* g, void* u, void* h, void* y,
                          void* stream) {
@@ -815,7 +816,7 @@ int fs2moe::swiglu_train(const void* x, const int32_t* counts, const int32_t* of
   const Groups grp{E > 0 ? counts : nullptr, E > 0 ? offsets : nullptr, E > 0 ? E : 1, (int)rows};
   if (dtype == FS2MOE_BF16) {
     if (E > 0)
-      return launch_dma_pair<FS2MOE_W_IN_OUT>(x, nullptr, grp, rows, w_gate, w_up, w_down, nullptr, nullptr,
+      return launch_dma_pair<FS2MOE_W_IN_OUT>(x, row_map, grp, rows, w_gate, w_up, w_down, nullptr, nullptr,
                                               nullptr, D, F, h, y, st, g, u);
     return launch_dma_pair<FS2MOE_W_OUT_IN>(x, nullptr, grp, rows, w_gate, w_up, w_down, nullptr, nullptr,
                                             nullptr, D, F, h, y, st, g, u);

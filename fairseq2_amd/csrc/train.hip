@@ -4,7 +4,8 @@
 // Python with its own buffers took the host longer (10 to 15 us a launch) than a layer of a few
 // thousand rows takes the GPU.  Both calls therefore carve every intermediate out of two buffers and
 // launch the whole pass.  What is new on the device is small: the gather of the output gradients, which
-// also takes the dot products that are the combine weights' gradients, and the padding of a router matrix
+// also takes the dot products that are the combine weights' gradients, the activation's derivative of a step
+// whose rows stay in token order, and the padding of a router matrix
 // whose number of experts is not a multiple of 8.
 #include "common.h"
 
@@ -59,6 +60,60 @@ __global__ __launch_bounds__(256) void gather_backward_kernel(
   if (lane == 0) d_w[p] = s;
 }
 
+// The same for a step whose rows stay in token order (in_token_order below): one wave per pair p with row
+// r = inv_perm[p].  dh holds the products of the token's output gradient, not yet weighted, with the expert's
+// down projection; from the kept g and u come h (weighted: the left operand of that projection's gradient,
+// whose right one is the unweighted output gradient), dg and du, and from the forward pass' h the combine
+// weight's gradient d_w[p] = <ye[r], dout[t]> = <h[r], dh[r]>, which so needs neither ye nor dout.  (With an
+// h from the rounded g and u the router's gradient is 15% further from 64 bits: three roundings instead of
+// two.)  Bound by memory: seven passes over [rows, F].  h may be dh's buffer.
+__global__ __launch_bounds__(256) void swiglu_backward_pairs_kernel(
+    const uint16_t* __restrict__ g, const uint16_t* __restrict__ u, const uint16_t* __restrict__ h_fwd,
+    const uint16_t* dh, const int32_t* __restrict__ inv_perm, const float* __restrict__ topk_w, int pairs, int F, uint16_t* h,
+    uint16_t* __restrict__ dg, uint16_t* __restrict__ du, float* __restrict__ d_w) {
+  const int p = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (p >= pairs) return;
+  const int lane = threadIdx.x & 63;
+  const int row = __builtin_amdgcn_readfirstlane(inv_perm[p]);
+  if (row < 0) {
+    if (lane == 0) d_w[p] = 0.f;
+    return;
+  }
+  const float w = topk_w[p];
+  const size_t base = (size_t)row * F;
+  float dot = 0.f;
+  for (int c = lane * 8; c < F; c += 512) {
+    const u32x4 gv = *reinterpret_cast<const u32x4*>(g + base + c);
+    const u32x4 uv = *reinterpret_cast<const u32x4*>(u + base + c);
+    const u32x4 fv = *reinterpret_cast<const u32x4*>(h_fwd + base + c);
+    const u32x4 dv = *reinterpret_cast<const u32x4*>(dh + base + c);
+    u32x4 hv, gov, uov;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float ho[2], go[2], uo[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const float gf = __uint_as_float(q ? gv[j] & 0xffff0000u : gv[j] << 16);
+        const float uf = __uint_as_float(q ? uv[j] & 0xffff0000u : uv[j] << 16);
+        const float df = __uint_as_float(q ? dv[j] & 0xffff0000u : dv[j] << 16);
+        const float s = 1.0f / (1.0f + __expf(-gf)), silu = gf * s, dw = df * w;
+        dot += __uint_as_float(q ? fv[j] & 0xffff0000u : fv[j] << 16) * df;
+        ho[q] = silu * uf * w;
+        go[q] = dw * uf * (s * (1.0f + gf * (1.0f - s)));
+        uo[q] = dw * silu;
+      }
+      hv[j] = pack_bf16x2(ho[0], ho[1]);
+      gov[j] = pack_bf16x2(go[0], go[1]);
+      uov[j] = pack_bf16x2(uo[0], uo[1]);
+    }
+    *reinterpret_cast<u32x4*>(h + base + c) = hv;
+    *reinterpret_cast<u32x4*>(dg + base + c) = gov;
+    *reinterpret_cast<u32x4*>(du + base + c) = uov;
+  }
+  dot = wave_sum_f32(dot);
+  if (lane == 0) d_w[p] = dot;
+}
+
 // out[r, 0..cols_out) = in[r, 0..cols_in), cut or padded with zeros
 template <typename T>
 __global__ __launch_bounds__(256) void copy_columns_kernel(const T* __restrict__ in, int cols_in,
@@ -103,10 +158,17 @@ bool streams(const Args& a) {
   return a.T <= 16 && swiglu_streams_rows(a.act_dtype, a.act_dtype, a.D, a.F, a.E, a.T);
 }
 
+// Whether the rows stay where they are: every product and weight gradient reads the tokens' rows (x, and in
+// the backward pass dout) through the permutation, and nothing of K rows a token is copied, kept or gathered.
+// Needs rows that enter the experts unscaled, and the bf16 kernels, which take a row map.  A step of 4096
+// tokens, D 2048 / F 768, 128 experts, top-8: 1804 -> 1672 us (the copy of x 28 us and the gather of dout
+// 49 us gone, 17 us less in the first down product and 24 us in the weight gradients), 220 MB less kept.
+bool in_token_order(const Args& a) { return a.act_dtype == FS2MOE_BF16 && !a.scale_input && !streams(a); }
+
 struct Saved {
   int32_t *idx, *counts, *offsets, *perm, *inv_perm;
   float *w, *logits;
-  void *xn, *xe, *ye, *g, *u, *gs, *us;
+  void *xn, *xe, *ye, *g, *u, *h, *gs, *us;
   int64_t total;
 };
 Saved carve_saved(const Args& a, void* base) {
@@ -121,11 +183,12 @@ Saved carve_saved(const Args& a, void* base) {
   s.perm = static_cast<int32_t*>(c.take(R * 4));
   s.inv_perm = static_cast<int32_t*>(c.take((int64_t)a.T * a.K * 4));
   s.xn = a.normed ? c.take((int64_t)a.T * a.D * sz) : nullptr;
-  s.xe = c.take(R * a.D * sz);
-  s.ye = c.take(R * a.D * sz);
+  s.xe = in_token_order(a) ? nullptr : c.take(R * a.D * sz);
+  s.ye = in_token_order(a) ? nullptr : c.take(R * a.D * sz);
   const bool keep = !streams(a);
   s.g = keep ? c.take(R * a.F * sz) : nullptr;
   s.u = keep ? c.take(R * a.F * sz) : nullptr;
+  s.h = in_token_order(a) ? c.take(R * a.F * sz) : nullptr;
   s.gs = a.F_shared > 0 ? c.take((int64_t)a.T * a.F_shared * sz) : nullptr;
   s.us = a.F_shared > 0 ? c.take((int64_t)a.T * a.F_shared * sz) : nullptr;
   s.total = c.used;
@@ -133,7 +196,7 @@ Saved carve_saved(const Args& a, void* base) {
 }
 
 struct ForwardScratch {
-  void *disp, *router, *h, *hs;
+  void *disp, *router, *h, *hs, *ye;
   int64_t disp_bytes, router_bytes, total;
 };
 ForwardScratch carve_forward(const Args& a, void* base) {
@@ -144,8 +207,9 @@ ForwardScratch carve_forward(const Args& a, void* base) {
   f.disp = c.take(f.disp_bytes);
   f.router_bytes = fs2moe_router_workspace_bytes(a.T, a.D, a.E, a.act_dtype);
   f.router = f.router_bytes > 0 ? c.take(f.router_bytes) : nullptr;
-  f.h = c.take(rows_of(a) * a.F * sz);
+  f.h = in_token_order(a) ? nullptr : c.take(rows_of(a) * a.F * sz);
   f.hs = a.F_shared > 0 ? c.take((int64_t)a.T * a.F_shared * sz) : nullptr;
+  f.ye = in_token_order(a) ? c.take(rows_of(a) * a.D * sz) : nullptr;
   f.total = c.used;
   return f;
 }
@@ -162,12 +226,14 @@ int requests(const Args& a, const Saved& s, const BackwardScratch& b, WgradReque
   const void* x = a.normed ? s.xn : a.x;
   int n = 0;
   // (wanted or not goes by the caller's pointer: the buffers' are null while the sizes are taken)
-  auto add = [&](void* dw, const void* left, const void* right, int M, int N, bool grouped) {
-    if (dw != nullptr) r[n++] = WgradRequest{left, right, dw, M, N, grouped, 1};
+  auto add = [&](void* dw, const void* left, const void* right, int M, int N, bool grouped, bool map_a = false,
+                 bool map_b = false) {
+    if (dw != nullptr) r[n++] = WgradRequest{left, right, dw, M, N, grouped, 1, map_a, map_b};
   };
-  add(a.d_gate, s.xe, b.dg, a.D, a.F, true);
-  add(a.d_up, s.xe, b.du, a.D, a.F, true);
-  add(a.d_down, b.dh, b.dye, a.F, a.D, true);  // (dh holds h by then)
+  const bool mapped = in_token_order(a);
+  add(a.d_gate, mapped ? x : s.xe, b.dg, a.D, a.F, true, mapped);
+  add(a.d_up, mapped ? x : s.xe, b.du, a.D, a.F, true, mapped);
+  add(a.d_down, b.dh, mapped ? a.dout : b.dye, a.F, a.D, true, false, mapped);  // (dh holds h by then)
   if (a.F_shared > 0) {
     add(a.d_shared_gate, b.dgs, x, a.F_shared, a.D, false);
     add(a.d_shared_up, b.dus, x, a.F_shared, a.D, false);
@@ -182,7 +248,7 @@ BackwardScratch carve_backward(const Args& a, void* base) {
   const int64_t R = rows_of(a), sz = elem_size(a.act_dtype), T = a.T;
   const int Ep = padded_experts(a);
   BackwardScratch b;
-  b.dye = c.take(R * a.D * sz);
+  b.dye = in_token_order(a) ? nullptr : c.take(R * a.D * sz);
   b.dh = c.take(R * a.F * sz);
   b.dg = c.take(R * a.F * sz);
   b.du = c.take(R * a.F * sz);
@@ -261,25 +327,27 @@ extern "C" int fs2moe_train_forward(const fs2moe_train_args* a, void* stream) {
   rc = fs2moe_dispatch(s.idx, s.w, x, a->T, a->K, a->E, a->D, a->tile_m, a->act_dtype, a->scale_input, R, s.counts,
                        s.offsets, s.perm, s.inv_perm, s.xe, f.disp, f.disp_bytes, stream);
   if (rc) return rc;
+  const bool mapped = in_token_order(*a);
+  void* ye = mapped ? f.ye : s.ye;
   if (s.g == nullptr)
     rc = fs2moe_grouped_swiglu_rows(s.xe, nullptr, s.counts, s.offsets, a->w_gate, a->w_up, a->w_down, nullptr,
                                     nullptr, nullptr, a->E, a->D, a->F, R, a->act_dtype, a->act_dtype, f.h, s.ye,
                                     a->T, stream);
   else
-    rc = swiglu_train(s.xe, s.counts, s.offsets, a->E, a->w_gate, a->w_up, a->w_down, a->D, a->F, R, a->act_dtype,
-                      s.g, s.u, f.h, s.ye, stream);
+    rc = swiglu_train(mapped ? x : s.xe, mapped ? s.perm : nullptr, s.counts, s.offsets, a->E, a->w_gate, a->w_up,
+                      a->w_down, a->D, a->F, R, a->act_dtype, s.g, s.u, mapped ? s.h : f.h, ye, stream);
   if (rc) return rc;
   const void* base = nullptr;
   if (a->F_shared > 0) {
-    rc = swiglu_train(x, nullptr, nullptr, 0, a->shared_gate, a->shared_up, a->shared_down, a->D, a->F_shared, a->T,
+    rc = swiglu_train(x, nullptr, nullptr, nullptr, 0, a->shared_gate, a->shared_up, a->shared_down, a->D, a->F_shared, a->T,
                       a->act_dtype, s.gs, s.us, f.hs, a->out, stream);
     if (rc) return rc;
     base = a->out;
   }
   if (a->residual != nullptr)
-    return fs2moe_combine_residual(s.ye, s.inv_perm, s.idx, s.w, base, a->residual, a->T, a->K, a->D,
+    return fs2moe_combine_residual(ye, s.inv_perm, s.idx, s.w, base, a->residual, a->T, a->K, a->D,
                                    a->act_dtype, a->scale_input ? 0 : 1, a->out, stream);
-  return fs2moe_combine(s.ye, s.inv_perm, s.idx, s.w, base, a->T, a->K, a->D, a->act_dtype,
+  return fs2moe_combine(ye, s.inv_perm, s.idx, s.w, base, a->T, a->K, a->D, a->act_dtype,
                         a->scale_input ? 0 : 1, a->out, stream);
 }
 
@@ -299,7 +367,8 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
   const void* x = a->normed ? s.xn : a->x;
   int rc;
   // output gradients in expert order, and with output-side weights the gradients of those
-  {
+  const bool mapped = in_token_order(*a);
+  if (!mapped) {
     const dim3 grid((unsigned)(((int64_t)T * K + 3) / 4)), block(256);
     const int weighted = a->scale_input ? 0 : 1;
     if (dt == FS2MOE_BF16)
@@ -313,7 +382,7 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
     if ((rc = check_launch("gather_backward"))) return rc;
   }
   // the experts: dh, then h, dg and du, then the rows' gradient
-  if ((rc = fs2moe_grouped_gemm(b.dye, nullptr, s.counts, s.offsets, a->w_down, FS2MOE_W_OUT_IN, E, D, F, R, dt, b.dh,
+  if ((rc = fs2moe_grouped_gemm(mapped ? a->dout : b.dye, mapped ? s.perm : nullptr, s.counts, s.offsets, a->w_down, FS2MOE_W_OUT_IN, E, D, F, R, dt, b.dh,
                                 stream)))
     return rc;
   const void *g = s.g, *u = s.u;
@@ -326,7 +395,18 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
     g = b.dg;
     u = b.du;
   }
-  if ((rc = fs2moe_swiglu_backward(g, u, b.dh, R, F, dt, b.dh, b.dg, b.du, stream))) return rc;
+  if (mapped) {
+    const uint16_t* dh = static_cast<const uint16_t*>(b.dh);
+    hipLaunchKernelGGL(swiglu_backward_pairs_kernel, dim3((unsigned)(((int64_t)T * K + 3) / 4)), dim3(256), 0, st,
+                       static_cast<const uint16_t*>(g), static_cast<const uint16_t*>(u),
+                       static_cast<const uint16_t*>(s.h), dh, s.inv_perm, s.w, T * K, F,
+                       static_cast<uint16_t*>(b.dh), static_cast<uint16_t*>(b.dg), static_cast<uint16_t*>(b.du),
+                       b.d_w);
+    rc = check_launch("swiglu_backward_pairs");
+  } else {
+    rc = fs2moe_swiglu_backward(g, u, b.dh, R, F, dt, b.dh, b.dg, b.du, stream);
+  }
+  if (rc) return rc;
   const bool want_x = a->dx != nullptr || a->d_norm_weight != nullptr;
   if (want_x || (a->scale_input && a->d_router != nullptr))
     if ((rc = gemm_sum(b.dg, a->w_gate, b.du, a->w_up, FS2MOE_W_OUT_IN, s.counts, s.offsets, E, F, D, R, dt, b.dxe,
@@ -353,7 +433,7 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
   const int n = requests(*a, s, b, r);
   if (n > 0) {
     (void)wgrad_plan(r, n, E, R, T, dt);
-    if ((rc = wgrad_all(r, n, s.counts, s.offsets, E, R, T, dt, b.wgrad, stream))) return rc;
+    if ((rc = wgrad_all(r, n, mapped ? s.perm : nullptr, s.counts, s.offsets, E, R, T, dt, b.wgrad, stream))) return rc;
     if (a->d_router != nullptr && Ep != E && (rc = copy_columns(b.d_router, Ep, a->d_router, E, D, dt, st))) return rc;
   }
   if (!want_x) return FS2MOE_OK;
