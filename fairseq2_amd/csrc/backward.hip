@@ -336,7 +336,14 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
   }
   deal.next_t = __builtin_amdgcn_readfirstlane(deal.next_t);
   deal.end = __builtin_amdgcn_readfirstlane(deal.end);
+  // (all of it is the same in every lane, but was computed from LDS: as scalars from here on, or the loops
+  // over tiles and chunks would be masked ones, whose paths meet where nothing can be known of the loads)
+  deal.rounds = __builtin_amdgcn_readfirstlane(deal.rounds);
+  deal.big = __builtin_amdgcn_readfirstlane(deal.big);
+  deal.stride = __builtin_amdgcn_readfirstlane(deal.stride);
+  by_expert = __builtin_amdgcn_readfirstlane(by_expert);
 
+  auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
   // Wave-uniform parameters of a tile.
   struct Tile {
     int job, slot, off, cnt, m0, n0;
@@ -410,7 +417,7 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     auto next_tile = [&]() {
       // (tiles without rows have no chunks)
       ld_left = 0;
-      for (int n; ld_left == 0 && (n = ld_deal.next()) >= 0;) {
+      for (int n; ld_left == 0 && (n = uniform(ld_deal.next())) >= 0;) {
         const Tile t = locate(n);
         if (t.cnt == 0) continue;
         const WgradJob& j = jobs.job[t.job];
@@ -422,16 +429,23 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
         ld_map_a = j.map_a;
         ld_map_b = j.map_b;
         ld_left = t.cnt;
-        const bool a_ok = t.m0 + ch * 8 < j.M, b_ok = t.n0 + ch * 8 < j.N;
+        // (columns past the operand's: all ones, past any buffer's end.  As selects these become branches,
+        // at whose joins the tile's parameters stop being scalars)
+        uint32_t a_out = t.m0 + ch * 8 < j.M ? 0u : 0xfffffff0u, b_out = t.n0 + ch * 8 < j.N ? 0u : 0xfffffff0u;
+        asm volatile("" : "+v"(a_out), "+v"(b_out));
 #pragma unroll
         for (int i = 0; i < PER_THREAD; ++i) {
-          oa[i] = a_ok ? (uint32_t)(((kr + 8 * i) * j.M + ch * 8) * 2) : 0xfffffff0u;
-          ob[i] = b_ok ? (uint32_t)(((kr + 8 * i) * j.N + ch * 8) * 2) : 0xfffffff0u;
+          oa[i] = (uint32_t)(((kr + 8 * i) * j.M + ch * 8) * 2) | a_out;
+          ob[i] = (uint32_t)(((kr + 8 * i) * j.N + ch * 8) * 2) | b_out;
         }
       }
     };
+    auto scalar = [&](const uint16_t* q) {
+      const uint64_t v = (uint64_t)q;
+      return (uint16_t*)((uint64_t)(uint32_t)uniform((int)(v >> 32)) << 32 | (uint32_t)uniform((int)v));
+    };
     auto look_up = [&]() {
-      if (ld_left <= 0) next_tile();
+      if (uniform(ld_left) <= 0) next_tile();
       if constexpr (MAPPED) {
 #pragma unroll
         for (int i = 0; i < PER_THREAD; ++i)
@@ -445,7 +459,8 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     };
     auto load_chunk = [&](auto set_c) {
       constexpr int set = decltype(set_c)::value;
-      loaded += ld_left > 0 ? 1 : 0;
+      // one more if ld_left > 0 (a truth value is added on the vector side, and takes the loop's end with it)
+      loaded += (int)((uint32_t)-ld_left >> 31);
       if constexpr (MAPPED) {
 #pragma unroll
         for (int i = 0; i < PER_THREAD; ++i) {
@@ -455,20 +470,22 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
           const uint64_t pa = (uint64_t)ld_a + ((uint64_t)(lane < 32 ? a0 : a1) * (uint32_t)ld_lda + ch * 8) * 2;
           const uint64_t pb = (uint64_t)ld_b + ((uint64_t)(lane < 32 ? b0 : b1) * (uint32_t)ld_ldb + ch * 8) * 2;
           // (the address chosen, by its bits: as pointers the two sides become branches)
-          ra[set][i] = *(const GlobalVec*)((in & (oa[i] != 0xfffffff0u)) ? pa : zero);
-          rb[set][i] = *(const GlobalVec*)((in & (ob[i] != 0xfffffff0u)) ? pb : zero);
+          ra[set][i] = *(const GlobalVec*)((in & (oa[i] < 0xfffffff0u)) ? pa : zero);
+          rb[set][i] = *(const GlobalVec*)((in & (ob[i] < 0xfffffff0u)) ? pb : zero);
         }
         ld_row += RK;
       } else {
         const __amdgpu_buffer_rsrc_t a_rsrc =
-            __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(ld_a), 0, 0xfffffff0u, 0x00020000);
+            __builtin_amdgcn_make_buffer_rsrc(scalar(ld_a), 0, 0xfffffff0u, 0x00020000);
         const __amdgpu_buffer_rsrc_t b_rsrc =
-            __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(ld_b), 0, 0xfffffff0u, 0x00020000);
+            __builtin_amdgcn_make_buffer_rsrc(scalar(ld_b), 0, 0xfffffff0u, 0x00020000);
 #pragma unroll
         for (int i = 0; i < PER_THREAD; ++i) {
           const bool in = kr + 8 * i < ld_left;
-          ra[set][i] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, in ? oa[i] : 0xfffffff0u, 0, 0);
-          rb[set][i] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, in ? ob[i] : 0xfffffff0u, 0, 0);
+          uint32_t at_a = in ? oa[i] : 0xfffffff0u, at_b = in ? ob[i] : 0xfffffff0u;
+          asm volatile("" : "+v"(at_a), "+v"(at_b));  // (chosen before the load, not by branches around two)
+          ra[set][i] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, at_a, 0, 0);
+          rb[set][i] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, at_b, 0, 0);
         }
         ld_a += (size_t)RK * ld_lda;
         ld_b += (size_t)RK * ld_ldb;
@@ -498,16 +515,22 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     look_up();
     store_chunk(Set0{}, 0);
     load_chunk(Set0{});
+    look_up();
     lds_barrier();
     auto step = [&](int g, auto next_set) {
-      look_up();
       store_chunk(next_set, (g + 1) & 1);
       load_chunk(next_set);
+      look_up();
       lds_barrier();  // the loads of the next chunks stay in flight
     };
-    for (int g = 0; g < loaded; g += 2) {  // (a step's load is three chunks ahead: `loaded` is final in time)
+    // Always two steps, the one past an odd last chunk with zeros that no one reads, and everything that the
+    // loop's way depends on in scalars: where a skipped step's path, or a masked lane's, joined the loop again
+    // the compiler waited for all loads in flight, in every other step.  128 experts of about 256 rows, 2048 x
+    // 768, 189 -> 178 us; 8 of 2048, 4096 x 14336, 1775 -> 1655; 60 of 300, 1096 x 1416, 116 -> 106.  (A
+    // third set of registers gives the long ones nothing more and costs launches of few chunks 1 to 2 us.)
+    for (int g = 0; g < uniform(loaded); g += 2) {  // (a step's load is three chunks ahead: `loaded` is final)
       step(g, Set1{});
-      if (g + 1 < loaded) step(g + 1, Set0{});
+      step(g + 1, Set0{});
     }
     return;  // the consumers write the tiles
   }
@@ -621,7 +644,7 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     }
   };
   bool started = false;
-  int buf = 0;
+  int buf = 0, chunks_done = 0;
   for (int n; (n = deal.next()) >= 0;) {
     const Tile tl = locate(n);
 #pragma unroll
@@ -638,10 +661,12 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     for (int i = 0; i < chunks; ++i) {
       compute_chunk(buf);
       buf ^= 1;
+      ++chunks_done;
       lds_barrier();
     }
     write_tile(tl);
   }
+  if (chunks_done % 2 != 0) lds_barrier();  // the producers' last step
 }
 
 // out[i] = sum over the segments, in order, of partial[s][i]; one rounding.
