@@ -1018,13 +1018,11 @@ def forward(
     norm: tuple[Tensor | None, float] | None = None,
     router_t: Tensor | None = None,
     act_quant: bool = False,
-    prepared: list | None = None,
 ) -> Tensor:
     """The whole layer through ``fs2moe_forward``: one call, intermediates in one workspace.
     ``router_t``: optionally the router matrix expert-major, (E, D), used where the library reads it.
     ``act_quant`` (with ``scales``, i.e. e4m3 weights): the expert products on the fp8 matrix pipe,
     the rows rounded to block-scaled e4m3 inside the call (``FS2MOE_ACT_MXFP8``).
-    ``prepared``: a list to leave the call's arguments in, for :func:`forward_again`.
     With ``residual`` ``(T, D)`` the result is ``residual + layer(x)`` from the same accumulation.
     With ``norm`` = (weight or None, eps) the rows are RMS-normalised on the way into the router
     (``fs2moe_forward_norm``): the result is ``[residual +] layer(rms_norm(x))``.
@@ -1065,25 +1063,6 @@ def forward(
         _ptr(workspace), workspace.numel(), _ptr(out),
     )
     _check(lib.fs2moe_forward_call(a, _stream()), "fs2moe_forward")
-    if prepared is not None:
-        prepared.append(a)
-    return out
-
-
-def forward_again(prepared: ForwardArgs, x: Tensor, residual: Tensor | None, router_t: Tensor | None) -> Tensor:
-    """:func:`forward` with the arguments that an earlier call has left in its ``prepared`` list, for
-    other rows (and another residual) of the same shape.  Nothing is checked here: the caller has made
-    sure that the tensors are as they were (``router_t``: given when that call was)."""
-    a = ForwardArgs.from_buffer_copy(prepared)
-    a.x = x.data_ptr()
-    if residual is not None:
-        a.residual = residual.data_ptr()
-    if a.score_fn & ROUTER_OUT_IN:
-        a.router = router_t.data_ptr()
-    workspace = torch.empty(a.workspace_bytes, dtype=torch.uint8, device=x.device)
-    out = torch.empty_like(x)
-    a.workspace, a.out = workspace.data_ptr(), out.data_ptr()
-    _check(_lib.fs2moe_forward_call(a, _stream()), "fs2moe_forward")
     return out
 
 

@@ -500,12 +500,6 @@ class MoE(FeedForwardNetwork):
         normalised inside the router kernel instead of by a pass of their own, so that
         ``layer(seqs, residual=seqs, norm=layer_norm)`` is the whole of ``_forward_ffn``
         (``decoder_layer.py:187-204``) for a pre-norm layer without dropout."""
-        if not (torch.is_grad_enabled() or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda")):
-            repeat = self.__dict__.get("_repeat")
-            state = None if repeat is None else self._call_state(seqs, residual, norm)
-            if state is not None and state == repeat.state:
-                return _abi.forward_again(repeat.prepared, seqs, residual,
-                                          self._router_expert_major() if repeat.reads_router_t else None)
         seqs = self._autocast(seqs)
         if residual is not None:
             residual = self._autocast(residual)
@@ -537,52 +531,13 @@ class MoE(FeedForwardNetwork):
         w8a8_staged = w8a8 and (self.scale_on == "input" or torch.compiler.is_compiling())
         if (type(ex) is GroupedExpertNetwork and ex.has_fused_gate and not w8a8_staged
                 and (se is None or type(se) is GLUFeedForwardNetwork)):
-            prepared = None
-            if not (torch.compiler.is_compiling() or torch.is_grad_enabled() or torch.is_autocast_enabled("cuda")):
-                prepared = []
-            out = self._single_call(x, res, norm_args, act_quant=w8a8, prepared=prepared).view(seqs.shape)
-            # (tensors that are computed on access, as parametrizations are, are none to come back to)
-            linears = () if se is None else se._modules.values()
-            held = [t for m in (ex, *linears) for t in m._parameters.values() if t is not None]
-            if (prepared and seqs.is_contiguous() and (residual is None or residual.is_contiguous())
-                    and "router" in self._parameters and len(held) == (3 if se is None else 6)
-                    and (norm is None or (isinstance(norm, Module)
-                                          and getattr(norm, "weight", None) is norm._parameters.get("weight")))):
-                object.__setattr__(self, "_repeat", _Repeat(self._call_state(seqs, residual, norm), prepared[0]))
-            return out
+            return self._single_call(x, res, norm_args, act_quant=w8a8).view(seqs.shape)
         if wants_grad:
             # (only reachable inside a compiler's trace: the staged path below records no graph)
             raise RuntimeError(
                 "fairseq2_amd.MoE: under torch.compile only the fused SiLU experts are differentiated; "
                 "train this configuration eagerly")
         return self._stages(x, res, norm_args)[0].view(seqs.shape)
-
-    def _call_state(self, seqs: Tensor, residual: Tensor | None, norm):
-        """All that the arguments of the one call depend on, the rows' addresses aside: attributes, and
-        where each tensor lies and how.  With grad mode, autocast and tracing off, a call in the state of
-        an earlier one takes that call's arguments (:class:`_Repeat`) instead of checking and collecting
-        them again, which took the host longer than a decode step takes the GPU (46 against 25 us)."""
-        ex, se = self.experts, self.shared_expert
-        if type(ex) is not GroupedExpertNetwork or not (se is None or type(se) is GLUFeedForwardNetwork):
-            return None
-        tensors = [self.router, self.router_bias, *ex._parameters.values(), *ex._buffers.values()]
-        if se is not None:
-            for layer in se._modules.values():
-                tensors += layer._parameters.values()
-        how = ()
-        if norm is not None:
-            if not isinstance(norm, Module):
-                return None
-            tensors += (norm._parameters.get("weight"), norm._parameters.get("bias"))
-            how = (norm, norm.eps, norm.__dict__.get("normalized_shape"))
-        like = None if residual is None else (
-            type(residual), residual.shape, residual.stride(), residual.dtype, residual.device)
-        return (
-            type(seqs), seqs.shape, seqs.stride(), seqs.dtype, seqs.device, like, how, ex, se, ex.activation,
-            ex.act_quant, ex.num_experts, ex.model_dim, ex.inner_dim, self.top_k, self.tile_m, self.score_fn,
-            self.renormalize, self.scale_on, self.tp_gang,
-            [t if t is None else (t.data_ptr(), t.shape, t.stride(), t.dtype, t.device) for t in tensors],
-        )
 
     def _differentiable(self, seqs: Tensor, residual: Tensor | None, norm) -> Tensor:
         """The training path: the layer as one ``torch.autograd.Function`` whose backward pass runs
@@ -667,7 +622,7 @@ class MoE(FeedForwardNetwork):
         return _abi.router_expert_major(self.router, self)
 
     def _single_call(self, x: Tensor, residual: Tensor | None = None, norm=None, *,
-                     act_quant: bool = False, prepared: list | None = None) -> Tensor:
+                     act_quant: bool = False) -> Tensor:
         """The layer through the library's whole-layer entry point: one call, one workspace
         allocation (same kernels and results as :meth:`_stages`)."""
         ex, se = self.experts, self.shared_expert
@@ -699,7 +654,7 @@ class MoE(FeedForwardNetwork):
             x, self.router.detach(), self.router_bias, *weights, ex.num_local_experts, self.top_k,
             scales=scales, shared=shared, tile_m=self.tile_m, score_fn=_SCORE_FNS[self.score_fn],
             renormalize=self.renormalize, scale_input=self.scale_on == "input", residual=residual,
-            norm=norm, router_t=self._router_expert_major(), act_quant=act_quant, prepared=prepared,
+            norm=norm, router_t=self._router_expert_major(), act_quant=act_quant,
         )
 
     @torch.no_grad()
@@ -772,20 +727,6 @@ class MoE(FeedForwardNetwork):
             f"top_k={self.top_k}, score_fn={self.score_fn}, renormalize={self.renormalize}, "
             f"scale_on={self.scale_on}, tile_m={self.tile_m}"
         )
-
-
-class _Repeat:
-    """The arguments of a module's latest whole-layer call and the state they belong to.  Copies and
-    pickles of the module start without one (they have tensors of their own)."""
-
-    __slots__ = ("state", "prepared", "reads_router_t")
-
-    def __init__(self, state=None, prepared=None) -> None:
-        self.state, self.prepared = state, prepared
-        self.reads_router_t = prepared is not None and bool(prepared.score_fn & _abi.ROUTER_OUT_IN)
-
-    def __reduce__(self):
-        return _Repeat, ()
 
 
 class GraphedForward:

@@ -453,3 +453,54 @@ def test_fp8_tile_packing_round_trip():
     # tile (e, c, k) holds channels 16 c .. 16 c + 15 (rows) x input features 64 k .. 64 k + 63
     assert tiled.view(torch.uint8)[1, 2, 1, 3, 5] == q.view(torch.uint8)[1 * 128 + 64 + 5, 2 * 16 + 3]
     assert torch.equal(_abi.unpack_fp8_weights(tiled, 3).view(torch.uint8), q.view(torch.uint8))
+
+
+class _Recorder:
+    """The library with its whole-layer launch replaced: what each call would hand to the kernels."""
+
+    def __init__(self, lib, monkeypatch):
+        self._lib, self.calls = lib, []
+        monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
+        monkeypatch.setattr(_abi, "_lib", self)
+        monkeypatch.setattr(_abi, "_stream", lambda: 0)
+
+    def __getattr__(self, name):
+        return getattr(self._lib, name)
+
+    def fs2moe_forward_call(self, a, stream):
+        # the memory behind an address is looked at here, while the call's tensors are alive
+        at = a.norm_weight
+        norm = None if at is None else torch.frombuffer(
+            bytearray(ctypes.string_at(at, 2 * a.D)), dtype=torch.int16).view(torch.bfloat16)
+        self.calls.append((a.T, a.x, a.residual, a.w_gate, norm))
+        return 0
+
+
+@pytest.mark.parametrize("form", ["contiguous", "every other element", "one element for all"])
+def test_every_call_passes_what_its_tensors_hold_now(lib, monkeypatch, form):
+    """Addresses are collected from the tensors of the call itself: other rows, other sizes, a weight that is
+    replaced, and a norm weight changed in place between the calls, also one that has to be made contiguous."""
+    d = 64
+    dt = torch.bfloat16
+    m = M.MoE(d, 32, False, 8, 1.0, 2, inner_dim_scale=1.0, auto_scale=False, score_fn="softmax", scale_on="output")
+    m.to(dt).requires_grad_(False)
+    base = {"contiguous": torch.rand(d), "every other element": torch.rand(2 * d), "one element for all": torch.rand(1)}
+    weight = base[form].to(dt)
+    norm = torch.nn.RMSNorm(d, eps=1e-6, dtype=dt)
+    norm.weight = torch.nn.Parameter(
+        weight if form == "contiguous" else weight[::2] if form == "every other element" else weight.expand(d),
+        requires_grad=False)
+    rec = _Recorder(lib, monkeypatch)
+    with torch.no_grad():
+        for step, t in enumerate((1, 1, 3, 1, 1)):
+            x = torch.rand(1, t, d).to(dt)
+            if step == 3:
+                weight.mul_(2)
+            if step == 4:
+                m.experts.gate_proj.data = torch.rand_like(m.experts.gate_proj)
+            out = m(x, residual=x, norm=norm)
+            assert out.shape == x.shape
+            got_t, got_x, got_res, got_gate, got_norm = rec.calls[step]
+            assert (got_t, got_x, got_res) == (t, x.data_ptr(), x.data_ptr())
+            assert got_gate == m.experts.gate_proj.data_ptr()
+            assert torch.equal(got_norm, norm.weight.contiguous()), f"call {step}"
