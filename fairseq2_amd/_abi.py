@@ -957,44 +957,45 @@ def rms_norm_backward(x: Tensor, weight: Tensor | None, eps: float, dy: Tensor,
     return dx, dw
 
 
-def check_layer_arguments(x, router, router_bias, w_gate, w_up, w_down, num_experts, f, scales, shared) -> None:
+def check_layer_arguments(x, router, router_bias, w_gate, w_up, w_down, num_experts, f, scales, shared) -> tuple:
     """Shapes, dtypes, devices and contiguity of everything ``fs2moe_forward`` takes as a raw pointer:
-    a mismatched tensor would otherwise be read out of bounds or with the wrong layout on the GPU."""
+    a mismatched tensor would otherwise be read out of bounds or with the wrong layout on the GPU.
+    Returns the addresses (None for what is absent) of ``router``, ``router_bias``, the three weights,
+    their three scales and the three shared matrices: what has been checked is what a call then passes,
+    on every call anew, as no address may outlive the call that has looked at its tensor."""
     e = num_experts
     if x.dim() != 2 or not x.is_cuda or not x.is_contiguous():
         raise ValueError("x must be a contiguous (T, D) tensor on the GPU")
-    t, d = x.shape
-    dev = x.device
+    d, dtype, dev = x.shape[1], x.dtype, x.device
 
     def need(name, tensor, shape, dtype):
         if tensor is None:
             raise ValueError(f"{name} is missing")
-        if tuple(tensor.shape) != tuple(shape) or tensor.dtype != dtype:
-            raise ValueError(f"{name} must be {tuple(shape)} {dtype}, got {tuple(tensor.shape)} {tensor.dtype}")
+        if tensor.shape != shape or tensor.dtype != dtype:
+            raise ValueError(f"{name} must be {shape} {dtype}, got {tuple(tensor.shape)} {tensor.dtype}")
         if tensor.device != dev or not tensor.is_contiguous():
             raise ValueError(f"{name} must be contiguous and on {dev}")
+        return tensor.data_ptr()
 
-    need("router", router, (d, e), x.dtype)
-    if router_bias is not None:
-        need("router_bias", router_bias, (e,), torch.float32)
+    at = [need("router", router, (d, e), dtype),
+          None if router_bias is None else need("router_bias", router_bias, (e,), torch.float32)]
     if scales is None:
-        need("gate weights", w_gate, (e * d, f), x.dtype)
-        need("up weights", w_up, (e * d, f), x.dtype)
-        need("down weights", w_down, (e * f, d), x.dtype)
+        at += (need("gate weights", w_gate, (e * d, f), dtype), need("up weights", w_up, (e * d, f), dtype),
+               need("down weights", w_down, (e * f, d), dtype), None, None, None)
     else:
-        if x.dtype != torch.bfloat16 or d % 64 or f % 64:
+        if dtype != torch.bfloat16 or d % 64 or f % 64:
             raise ValueError("fp8 weights need bf16 activations and D, F multiples of 64")
-        need("gate codes", w_gate, (e, f // 16, d // 64, 16, 64), torch.float8_e4m3fn)
-        need("up codes", w_up, (e, f // 16, d // 64, 16, 64), torch.float8_e4m3fn)
-        need("down codes", w_down, (e, d // 16, f // 64, 16, 64), torch.float8_e4m3fn)
-        need("gate scales", scales[0], (e, f), torch.float32)
-        need("up scales", scales[1], (e, f), torch.float32)
-        need("down scales", scales[2], (e, d), torch.float32)
-    if shared is not None:
-        fs = shared[0].shape[0]
-        need("shared gate", shared[0], (fs, d), x.dtype)
-        need("shared up", shared[1], (fs, d), x.dtype)
-        need("shared down", shared[2], (d, fs), x.dtype)
+        at += (need("gate codes", w_gate, (e, f // 16, d // 64, 16, 64), torch.float8_e4m3fn),
+               need("up codes", w_up, (e, f // 16, d // 64, 16, 64), torch.float8_e4m3fn),
+               need("down codes", w_down, (e, d // 16, f // 64, 16, 64), torch.float8_e4m3fn),
+               need("gate scales", scales[0], (e, f), torch.float32),
+               need("up scales", scales[1], (e, f), torch.float32),
+               need("down scales", scales[2], (e, d), torch.float32))
+    if shared is None:
+        return (*at, None, None, None)
+    fs = shared[0].shape[0]
+    return (*at, need("shared gate", shared[0], (fs, d), dtype), need("shared up", shared[1], (fs, d), dtype),
+            need("shared down", shared[2], (d, fs), dtype))
 
 
 def forward(
@@ -1018,11 +1019,13 @@ def forward(
     norm: tuple[Tensor | None, float] | None = None,
     router_t: Tensor | None = None,
     act_quant: bool = False,
+    out: Tensor | None = None,
 ) -> Tensor:
     """The whole layer through ``fs2moe_forward``: one call, intermediates in one workspace.
     ``router_t``: optionally the router matrix expert-major, (E, D), used where the library reads it.
     ``act_quant`` (with ``scales``, i.e. e4m3 weights): the expert products on the fp8 matrix pipe,
     the rows rounded to block-scaled e4m3 inside the call (``FS2MOE_ACT_MXFP8``).
+    ``out``: optionally where the result goes, contiguous, with as many elements as ``x`` in any shape.
     With ``residual`` ``(T, D)`` the result is ``residual + layer(x)`` from the same accumulation.
     With ``norm`` = (weight or None, eps) the rows are RMS-normalised on the way into the router
     (``fs2moe_forward_norm``): the result is ``[residual +] layer(rms_norm(x))``.
@@ -1039,28 +1042,37 @@ def forward(
     else:
         f = w_gate.shape[1] * 16
     f_shared = shared[0].shape[0] if shared is not None else 0
-    check_layer_arguments(x, router, router_bias, w_gate, w_up, w_down, num_experts, f, scales, shared)
-    sizes = (t, d, num_experts, top_k, f, f_shared, tile_m, dtype_code(x.dtype))
-    need = lib.fs2moe_forward_workspace_bytes(*sizes) if norm is None else lib.fs2moe_forward_norm_workspace_bytes(*sizes)
+    act_dtype = dtype_code(x.dtype)
+    router_at, bias_at, *weights_at = check_layer_arguments(
+        x, router, router_bias, w_gate, w_up, w_down, num_experts, f, scales, shared)
+    sizes = (t, d, num_experts, top_k, f, f_shared, tile_m)
+    need = (lib.fs2moe_forward_workspace_bytes if norm is None else lib.fs2moe_forward_norm_workspace_bytes)(
+        *sizes, act_dtype)
     if need < 0:
         raise ValueError("fs2moe_forward_workspace_bytes rejected the sizes")
     if workspace is None:
         workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+    normed, norm_weight, norm_eps = 0, None, 0.0
     if norm is not None:
         _check_norm_weight(norm[0], x)
-    if residual is not None and (residual.shape != x.shape or residual.dtype != x.dtype or not residual.is_contiguous()):
+        normed, norm_weight, norm_eps = 1, _ptr(norm[0]), float(norm[1])
+    if residual is not None and residual is not x and (
+            residual.shape != x.shape or residual.dtype != x.dtype or not residual.is_contiguous()):
         raise ValueError("residual must be a contiguous tensor of x's shape and dtype")
-    out = torch.empty_like(x)
-    sg, su, sd = scales if scales is not None else (None, None, None)
-    hg, hu, hd = shared if shared is not None else (None, None, None)
+    if out is None:
+        out = torch.empty_like(x)
+    elif out.numel() != x.numel() or out.dtype != x.dtype or out.device != x.device or not out.is_contiguous():
+        raise ValueError("out must be a contiguous tensor of x's elements")
     mat, score_fn = router_operand(lib, x, router, router_t, score_fn)
+    # Collected on every call, in as few steps as checking each tensor once allows: a one-token step of a
+    # layer of 128 experts takes the host 36 us with its five launches, whatever the call before it was (47 us
+    # with a detached view of every parameter and each check in passes of its own; the GPU takes 34).
+    # (fields in the order of ForwardArgs)
     a = ForwardArgs(
-        t, d, num_experts, top_k, f, f_shared, tile_m, dtype_code(x.dtype),
-        dtype_code(w_gate.dtype) | (ACT_MXFP8 if act_quant else 0), score_fn, int(renormalize), int(scale_input),
-        int(norm is not None), float(norm[1]) if norm is not None else 0.0,
-        _ptr(x), _ptr(norm[0]) if norm is not None else None, _ptr(residual), _ptr(mat), _ptr(router_bias),
-        _ptr(w_gate), _ptr(w_up), _ptr(w_down), _ptr(sg), _ptr(su), _ptr(sd), _ptr(hg), _ptr(hu), _ptr(hd),
-        _ptr(workspace), workspace.numel(), _ptr(out),
+        *sizes, act_dtype, act_dtype if scales is None else FP8_E4M3 | (ACT_MXFP8 if act_quant else 0), score_fn,
+        int(renormalize), int(scale_input), normed, norm_eps,
+        x.data_ptr(), norm_weight, _ptr(residual), router_at if mat is router else _ptr(mat), bias_at, *weights_at,
+        _ptr(workspace), workspace.numel(), out.data_ptr(),
     )
     _check(lib.fs2moe_forward_call(a, _stream()), "fs2moe_forward")
     return out

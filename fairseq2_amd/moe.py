@@ -58,6 +58,13 @@ def _require_device(t: Tensor) -> None:
         )
 
 
+def _held(module: Module, name: str) -> Tensor:
+    """``getattr(module, name)`` of a parameter, past ``Module.__getattr__`` (0.5 us of host time each, of
+    three to nine a call) where the module holds it; one that is computed on access is not held."""
+    p = module._parameters.get(name)
+    return getattr(module, name) if p is None else p
+
+
 class ExpertNetwork(Module, ABC):
     """Interface of an expert bank (``models/transformer/experts.py:117-154``)."""
 
@@ -134,7 +141,7 @@ class GroupedExpertNetwork(ExpertNetwork):
 
     @property
     def has_fp8_weights(self) -> bool:
-        return getattr(self, "_gate_q_bits", None) is not None
+        return self._buffers.get("_gate_q_bits") is not None
 
     def clear_fp8_weights(self) -> None:
         """Drops the derived e4m3 buffers: the next forward uses the Parameters again."""
@@ -500,21 +507,23 @@ class MoE(FeedForwardNetwork):
         normalised inside the router kernel instead of by a pass of their own, so that
         ``layer(seqs, residual=seqs, norm=layer_norm)`` is the whole of ``_forward_ffn``
         (``decoder_layer.py:187-204``) for a pre-norm layer without dropout."""
-        seqs = self._autocast(seqs)
-        if residual is not None:
-            residual = self._autocast(residual)
+        if torch.is_autocast_enabled("cuda"):
+            seqs = self._autocast(seqs)
+            if residual is not None:
+                residual = self._autocast(residual)
+        compiling = torch.compiler.is_compiling()
         wants_grad = torch.is_grad_enabled() and any(
             isinstance(t, Tensor) and t.requires_grad
             for t in (seqs, residual, getattr(norm, "weight", None), *self.parameters())
         )
-        if wants_grad and not torch.compiler.is_compiling():
+        if wants_grad and not compiling:
             return self._differentiable(seqs, residual, norm)
         # (while a compiler traces the call, training goes through the registered operator below,
         # which carries its own autograd formula)
         x = self._checked_rows(seqs, allow_grad=wants_grad)
         norm_args = self._norm_args(norm, x, allow_grad=wants_grad)
-        res = None
-        if residual is not None:
+        res = x if residual is seqs else None
+        if residual is not None and residual is not seqs:
             if residual.shape != seqs.shape or residual.dtype != seqs.dtype:
                 raise ValueError("residual must have the shape and dtype of seqs")
             _require_device(residual)
@@ -524,14 +533,17 @@ class MoE(FeedForwardNetwork):
         if x.shape[0] == 0:
             return torch.empty_like(seqs)
         ex, se = self.experts, self.shared_expert
-        w8a8 = type(ex) is GroupedExpertNetwork and ex.runs_w8a8(
+        w8a8 = type(ex) is GroupedExpertNetwork and ex.act_quant is not None and ex.runs_w8a8(
             x.dtype, x.shape[0] * self.top_k + ex.num_local_experts * (self.tile_m - 1))
         # (W8A8 inside the one call wherever the call takes it: output-side weights, not under a
         # compiler's trace, whose registered operator does not carry the option)
-        w8a8_staged = w8a8 and (self.scale_on == "input" or torch.compiler.is_compiling())
+        w8a8_staged = w8a8 and (self.scale_on == "input" or compiling)
         if (type(ex) is GroupedExpertNetwork and ex.has_fused_gate and not w8a8_staged
                 and (se is None or type(se) is GLUFeedForwardNetwork)):
-            return self._single_call(x, res, norm_args, act_quant=w8a8).view(seqs.shape)
+            if compiling:
+                return self._single_call(x, res, norm_args, act_quant=w8a8).view(seqs.shape)
+            out = torch.empty_like(seqs, memory_format=torch.contiguous_format)
+            return self._single_call(x, res, norm_args, act_quant=w8a8, out=out)
         if wants_grad:
             # (only reachable inside a compiler's trace: the staged path below records no graph)
             raise RuntimeError(
@@ -590,7 +602,7 @@ class MoE(FeedForwardNetwork):
         return out.view(seqs.shape)
 
     def _autocast(self, t: Tensor) -> Tensor:
-        if t.is_cuda and torch.is_autocast_enabled("cuda"):
+        if t.is_cuda:
             dt = torch.get_autocast_dtype("cuda")
             if t.is_floating_point() and t.dtype != dt and self.router.dtype == dt:
                 return t.to(dt)
@@ -598,8 +610,7 @@ class MoE(FeedForwardNetwork):
 
     @staticmethod
     def _norm_args(norm, x: Tensor, allow_grad: bool = False) -> tuple[Tensor | None, float] | None:
-        """(weight, eps) of an RMS normalisation module, checked against the rows ``x``; the weight
-        detached unless ``allow_grad`` (the training path differentiates it)."""
+        """(weight, eps) of an RMS normalisation module, checked against the rows ``x``."""
         if norm is None:
             return None
         if getattr(norm, "bias", None) is not None:
@@ -614,7 +625,7 @@ class MoE(FeedForwardNetwork):
                 _require_forward_only(weight)
             if weight.dtype != x.dtype or weight.shape != (x.shape[-1],):
                 raise ValueError("the norm weight must be (dim,) in the dtype of seqs")
-            weight = (weight if allow_grad else weight.detach()).contiguous()
+            weight = weight.contiguous()
         return weight, float(norm.eps)
 
     def _router_expert_major(self) -> Tensor | None:
@@ -622,7 +633,7 @@ class MoE(FeedForwardNetwork):
         return _abi.router_expert_major(self.router, self)
 
     def _single_call(self, x: Tensor, residual: Tensor | None = None, norm=None, *,
-                     act_quant: bool = False) -> Tensor:
+                     act_quant: bool = False, out: Tensor | None = None) -> Tensor:
         """The layer through the library's whole-layer entry point: one call, one workspace
         allocation (same kernels and results as :meth:`_stages`)."""
         ex, se = self.experts, self.shared_expert
@@ -630,19 +641,15 @@ class MoE(FeedForwardNetwork):
             weights = (ex.gate_q, ex.inner_q, ex.output_q)
             scales = (ex.gate_scale, ex.inner_scale, ex.output_scale)
         else:
-            weights = (ex.gate_proj.detach(), ex.inner_proj.detach(), ex.output_proj.detach())
+            weights = (_held(ex, "gate_proj"), _held(ex, "inner_proj"), _held(ex, "output_proj"))
             scales = None
         shared = None
         if se is not None:
-            shared = (se.gate_proj.weight.detach(), se.inner_proj.weight.detach(), se.output_proj.weight.detach())
+            shared = tuple(_held(p, "weight") for p in (se.gate_proj, se.inner_proj, se.output_proj))
         if torch.compiler.is_compiling():
             # under torch.compile the call goes through the registered operator, which the tracer
             # can represent (it cannot look through ctypes); it is given the parameters themselves,
             # so that its autograd formula reaches them when the trace is one of a training step
-            if not ex.has_fp8_weights:
-                weights = (ex.gate_proj, ex.inner_proj, ex.output_proj)
-            if se is not None:
-                shared = (se.gate_proj.weight, se.inner_proj.weight, se.output_proj.weight)
             return torch.ops.fairseq2_amd.moe_forward(
                 x, self.router, self.router_bias, *weights, *(scales or (None, None, None)),
                 *(shared or (None, None, None)), residual, None if norm is None else norm[0],
@@ -650,11 +657,13 @@ class MoE(FeedForwardNetwork):
                 self.renormalize, self.scale_on == "input", norm is not None,
                 0.0 if norm is None else norm[1],
             )
+        router = _held(self, "router")
         return _abi.forward(
-            x, self.router.detach(), self.router_bias, *weights, ex.num_local_experts, self.top_k,
+            x, router, self.router_bias, *weights, ex.num_local_experts, self.top_k,
             scales=scales, shared=shared, tile_m=self.tile_m, score_fn=_SCORE_FNS[self.score_fn],
             renormalize=self.renormalize, scale_input=self.scale_on == "input", residual=residual,
-            norm=norm, router_t=self._router_expert_major(), act_quant=act_quant,
+            norm=norm, router_t=_abi.router_expert_major(router, self), act_quant=act_quant,
+            out=out,
         )
 
     @torch.no_grad()
@@ -711,15 +720,16 @@ class MoE(FeedForwardNetwork):
         _require_device(seqs)
         if not allow_grad and torch.is_grad_enabled():  # (walking the parameters costs host time)
             _require_forward_only(seqs, *self.parameters())
-        if seqs.dtype != self.router.dtype:
+        router = _held(self, "router")
+        if seqs.dtype != router.dtype:
             hint = ""
             if torch.is_autocast_enabled("cuda"):
                 hint = (f" (autocast to {torch.get_autocast_dtype('cuda')} is on: hold the module's "
                         "parameters in that dtype)")
-            raise TypeError(f"seqs is {seqs.dtype} but the module holds {self.router.dtype} parameters{hint}")
+            raise TypeError(f"seqs is {seqs.dtype} but the module holds {router.dtype} parameters{hint}")
         dim = seqs.shape[-1]
-        if dim != self.router.shape[0]:
-            raise ValueError(f"last dimension of seqs is {dim}, expected {self.router.shape[0]}")
+        if dim != router.shape[0]:
+            raise ValueError(f"last dimension of seqs is {dim}, expected {router.shape[0]}")
         return seqs.reshape(-1, dim).contiguous()
 
     def extra_repr(self) -> str:

@@ -504,3 +504,32 @@ def test_every_call_passes_what_its_tensors_hold_now(lib, monkeypatch, form):
             assert (got_t, got_x, got_res) == (t, x.data_ptr(), x.data_ptr())
             assert got_gate == m.experts.gate_proj.data_ptr()
             assert torch.equal(got_norm, norm.weight.contiguous()), f"call {step}"
+
+
+def test_a_call_of_another_size_takes_the_host_no_longer(lib, monkeypatch):
+    """A server's batch changes from step to step: the interpreter's work for a call (function calls, Python's
+    and the built-in ones) is the same for alternating numbers of rows as for repeated ones."""
+    import sys
+
+    m = M.MoE(64, 32, True, 8, 1.0, 2, inner_dim_scale=1.0, auto_scale=False).bfloat16().requires_grad_(False)
+    norm = torch.nn.RMSNorm(64, eps=1e-6, dtype=torch.bfloat16).requires_grad_(False)
+    rows = [torch.rand(1, t, 64).bfloat16() for t in (1, 3)]
+    _Recorder(lib, monkeypatch)
+
+    def work(order):
+        events = [0]
+
+        def count(frame, event, arg):
+            events[0] += event in ("call", "c_call")
+
+        sys.setprofile(count)
+        try:
+            for i in order:
+                m(rows[i], residual=rows[i], norm=norm)
+        finally:
+            sys.setprofile(None)
+        return events[0]
+
+    with torch.no_grad():
+        work([0, 1])  # (the expert-major copy of the router matrix is made once)
+        assert work([0, 1] * 4) <= max(work([0] * 8), work([1] * 8))

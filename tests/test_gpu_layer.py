@@ -927,7 +927,7 @@ def test_layer_arguments_are_validated_before_the_gpu_reads_them(gpu_device):
 
 
 def test_repeated_calls_follow_the_module(gpu_device):
-    """A call in the state of an earlier one reuses its arguments: what changes between calls is seen."""
+    """What changes between calls -- rows, tensors, attributes, whole submodules -- is seen by the next."""
     import copy
 
     from fairseq2_amd import MoE
