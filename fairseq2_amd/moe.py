@@ -795,7 +795,9 @@ class GraphedForward:
                 f"graph was captured for {tuple(self._input.shape)} {self._input.dtype}, "
                 f"got {tuple(seqs.shape)} {seqs.dtype}"
             )
-        if seqs.device == self._input.device and seqs.is_contiguous() and self._input.is_contiguous():
+        # (the library launches on the current device's stream, a replay and copy_ go to the tensors' device)
+        if (seqs.device == self._input.device and seqs.device.index == torch._C._cuda_getDevice()
+                and seqs.is_contiguous() and self._input.is_contiguous()):
             _abi.copy(seqs, self._input)
         else:
             self._input.copy_(seqs)

@@ -533,3 +533,31 @@ def test_a_call_of_another_size_takes_the_host_no_longer(lib, monkeypatch):
     with torch.no_grad():
         work([0, 1])  # (the expert-major copy of the router matrix is made once)
         assert work([0, 1] * 4) <= max(work([0] * 8), work([1] * 8))
+
+
+@pytest.mark.parametrize("current, contiguous, by_kernel", [(1, True, True), (0, True, False), (1, False, False)])
+def test_graph_input_is_copied_on_the_graphs_device(monkeypatch, current, contiguous, by_kernel):
+    """A graph of device 1: the library's copy launches on the current device's stream, so with another
+    device current the copy is left to torch, which goes to the tensors' device as the replay does."""
+
+    class Rows:
+        shape, dtype, device = torch.Size([1, 8]), torch.bfloat16, torch.device("cuda:1")
+
+        def __init__(self, contiguous=True):
+            self.contiguous, self.copied = contiguous, []
+
+        def is_contiguous(self):
+            return self.contiguous
+
+        def copy_(self, src):
+            self.copied.append(src)
+
+    kernel = []
+    monkeypatch.setattr(_abi, "copy", lambda src, dst: kernel.append((src, dst)))
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: current, raising=False)
+    graph = M.GraphedForward.__new__(M.GraphedForward)
+    graph._input, graph._output = Rows(), "out"
+    graph._graph = type("Graph", (), {"replay": lambda self: None})()
+    rows = Rows(contiguous)
+    assert graph(rows) == "out"
+    assert (kernel, graph._input.copied) == (([(rows, graph._input)], []) if by_kernel else ([], [rows]))
