@@ -281,6 +281,8 @@ bool sizes_ok(const Args& a) {
          (a.F_shared == 0 || swiglu_train_applies(a.act_dtype, a.D, a.F_shared, a.T)) &&
          swiglu_train_applies(a.act_dtype, a.D, padded_experts(a), a.T);
 }
+// What the stage calls ask of their operands, before anything is launched: the kernels behind the pieces
+// that are called directly (swiglu_train, gemm_sum, wgrad_all) move 16 bytes at a time.
 int check(const Args* a, int64_t saved, int64_t scratch) {
   FS2_REQUIRE(a->x && a->router && a->w_gate && a->w_up && a->w_down && a->saved && a->workspace,
               "train: null pointer");
@@ -291,6 +293,11 @@ int check(const Args* a, int64_t saved, int64_t scratch) {
               (long long)a->saved_bytes, (long long)a->workspace_bytes, (long long)saved, (long long)scratch);
   FS2_REQUIRE(((reinterpret_cast<uintptr_t>(a->saved) | reinterpret_cast<uintptr_t>(a->workspace)) & 255u) == 0,
               "train: buffers must be 256-byte aligned");
+  FS2_REQUIRE(aligned16(a->w_gate) && aligned16(a->w_up) && aligned16(a->w_down) && aligned16(a->shared_gate) &&
+                  aligned16(a->shared_up) && aligned16(a->shared_down),
+              "train: weights must be 16-byte aligned");
+  // (rows that are normalised are read by the router alone, which looks at their address itself)
+  FS2_REQUIRE(a->normed || aligned16(a->x), "train: x must be 16-byte aligned");
   return FS2MOE_OK;
 }
 }  // namespace
@@ -314,6 +321,7 @@ extern "C" int fs2moe_train_forward(const fs2moe_train_args* a, void* stream) {
   const ForwardScratch f = carve_forward(*a, a->workspace);
   if (int rc = check(a, s.total, f.total)) return rc;
   FS2_REQUIRE(a->out && a->router_read, "train_forward: null pointer");
+  FS2_REQUIRE(aligned16(a->out) && aligned16(a->residual), "train_forward: out and residual must be 16-byte aligned");
   const int64_t R = rows_of(*a);
   const void* x = a->normed ? s.xn : a->x;
   int rc = a->normed
@@ -357,7 +365,16 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
   const Saved s = carve_saved(*a, a->saved);
   const BackwardScratch b = carve_backward(*a, a->workspace);
   if (int rc = check(a, s.total, b.total)) return rc;
-  FS2_REQUIRE(a->dout && aligned16(a->dout) && aligned16(a->x), "train_backward: dout and x must be 16-byte aligned");
+  const bool want_x = a->dx != nullptr || a->d_norm_weight != nullptr;
+  FS2_REQUIRE(a->dout && aligned16(a->dout), "train_backward: dout must be 16-byte aligned");
+  FS2_REQUIRE(!(a->normed && want_x) || (aligned16(a->x) && aligned16(a->norm_weight)),
+              "train_backward: x and the norm's weight must be 16-byte aligned");
+  FS2_REQUIRE(!want_x || padded_experts(*a) != a->E || aligned16(a->router),
+              "train_backward: router must be 16-byte aligned");
+  // (a padded router gradient is copied out element by element)
+  for (const void* p : {a->dx, padded_experts(*a) == a->E ? a->d_router : nullptr, a->d_gate, a->d_up, a->d_down, a->d_shared_gate, a->d_shared_up,
+                        a->d_shared_down, a->d_norm_weight})
+    FS2_REQUIRE(aligned16(p), "train_backward: gradients must be 16-byte aligned");
   FS2_REQUIRE(a->d_norm_weight == nullptr || (a->normed && a->norm_weight != nullptr),
               "train_backward: a gradient of a norm weight that is not there");
   hipStream_t st = static_cast<hipStream_t>(stream);
@@ -407,7 +424,6 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
     rc = fs2moe_swiglu_backward(g, u, b.dh, R, F, dt, b.dh, b.dg, b.du, stream);
   }
   if (rc) return rc;
-  const bool want_x = a->dx != nullptr || a->d_norm_weight != nullptr;
   if (want_x || (a->scale_input && a->d_router != nullptr))
     if ((rc = gemm_sum(b.dg, a->w_gate, b.du, a->w_up, FS2MOE_W_OUT_IN, s.counts, s.offsets, E, F, D, R, dt, b.dxe,
                        stream)))

@@ -561,3 +561,43 @@ def test_graph_input_is_copied_on_the_graphs_device(monkeypatch, current, contig
     rows = Rows(contiguous)
     assert graph(rows) == "out"
     assert (kernel, graph._input.copied) == (([(rows, graph._input)], []) if by_kernel else ([], [rows]))
+
+
+def _train_args_on_paper(lib, backward, **change):
+    """A training call's arguments with made-up addresses: enough for the checks in front of every launch."""
+    a = _abi.TrainArgs()
+    a.T, a.D, a.E, a.K, a.F, a.F_shared, a.tile_m, a.act_dtype = 64, 128, 8, 2, 64, 64, 16, _abi.BF16
+    a.score_fn = _abi.SCORE_SOFTMAX
+    for i, (name, kind) in enumerate(_abi.TrainArgs._fields_):
+        if kind is ctypes.c_void_p and name not in ("router_bias", "norm_weight"):
+            setattr(a, name, 0x10000 * (i + 1))
+    if not backward:
+        for name, kind in _abi.TrainArgs._fields_:
+            if name == "dout" or name.startswith("d_") or name == "dx":
+                setattr(a, name, None)
+    a.d_norm_weight = None
+    for name, value in change.items():
+        setattr(a, name, value)
+    a.saved_bytes = lib.fs2moe_train_saved_bytes(a)
+    a.workspace_bytes = lib.fs2moe_train_workspace_bytes(a, int(backward))
+    assert a.saved_bytes > 0 and a.workspace_bytes > 0
+    return a
+
+
+@pytest.mark.parametrize("dtype", [_abi.BF16, _abi.F32])
+@pytest.mark.parametrize("scale_input", [0, 1])
+def test_training_calls_refuse_unaligned_operands(lib, dtype, scale_input):
+    """As the stage calls do, and before anything is launched: in the pass that is called, not the next one."""
+    base = dict(act_dtype=dtype, scale_input=scale_input)
+    weights = ["w_gate", "w_up", "w_down", "shared_gate", "shared_up", "shared_down"]
+    gradients = ["dx", "d_router", "d_gate", "d_up", "d_down", "d_shared_gate", "d_shared_up", "d_shared_down"]
+    for name in ["x", "out", "residual", *weights]:
+        rc = lib.fs2moe_train_forward(_train_args_on_paper(lib, False, **base, **{name: 0x7000002}), None)
+        assert rc == -1 and b"16-byte aligned" in lib.fs2moe_last_error(), name
+    for name in ["x", "dout", "router", *weights, *gradients]:
+        rc = lib.fs2moe_train_backward(_train_args_on_paper(lib, True, **base, **{name: 0x7000002}), None)
+        assert rc == -1 and b"16-byte aligned" in lib.fs2moe_last_error(), name
+    for name in ["x", "norm_weight", "d_norm_weight"]:
+        change = {"normed": 1, "norm_weight": 0x7000000, name: 0x7000002}
+        rc = lib.fs2moe_train_backward(_train_args_on_paper(lib, True, **base, **change), None)
+        assert rc == -1 and b"16-byte aligned" in lib.fs2moe_last_error(), name

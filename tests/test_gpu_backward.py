@@ -204,6 +204,34 @@ def test_step_in_two_calls_against_its_stages(gpu_device, dtype, t, d, e, k, f, 
     assert torch.equal(some[4], grads[4])
 
 
+def test_rows_that_begin_anywhere_train_behind_a_norm_only(gpu_device):
+    """Rows two bytes past a 16-byte line: the router's kernel normalises them wherever they are, and the
+    weights' gradients then need nothing else of them; without a norm the forward pass refuses them."""
+    _say("unaligned rows")
+    from fairseq2_amd import MoE
+
+    t, d = 40, 128
+    torch.manual_seed(5)
+    with torch.device(gpu_device):
+        m = MoE(d, 64, False, 8, 1.0, 2, inner_dim_scale=1.0, auto_scale=False, score_fn="softmax",
+                renormalize=True, scale_on="output").bfloat16()
+        norm = torch.nn.RMSNorm(d, eps=1e-6).bfloat16().requires_grad_(False)
+        for p in m.parameters():
+            torch.nn.init.normal_(p, 0.0, 0.05)
+        buf = torch.randn(t * d + 1).bfloat16()
+        dout = torch.randn(t, d).bfloat16()
+    x = buf[1:].view(t, d)
+    assert x.data_ptr() % 16 == 2
+    params = list(m.parameters())
+    got = torch.autograd.grad(m(x, norm=norm), params, dout)
+    ref = torch.autograd.grad(m(x.clone(), norm=norm), params, dout)
+    # (the same experts; the norm's sum of squares in another order moves an element of the rows by a rounding)
+    for (name, _), a, b in zip(m.named_parameters(), got, ref):
+        assert_grad_close(a, b.cpu(), "bf16", f"d {name}")
+    with pytest.raises(_abi.Fs2MoeError, match="16-byte aligned"):
+        m(x)
+
+
 @pytest.mark.parametrize("rows,k,n", [([5, 0, 300, 64, 1, 700], 192, 128), ([130, 257], 64, 72), ([0, 0, 9], 128, 256)])
 def test_grouped_gemm_sum_adds_two_products(gpu_device, rows, k, n):
     """``a1 @ B1^T + a2 @ B2^T`` in one kernel against f64, and against the two products apart."""
