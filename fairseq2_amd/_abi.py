@@ -1087,19 +1087,23 @@ def copy(src: Tensor, dst: Tensor) -> None:
 
 def _train_args(x, router, wg, wu, wd, shared, norm_w, cfg) -> TrainArgs:
     a = TrainArgs()
+    e, f = cfg["num_experts"], wd.shape[0] // cfg["num_experts"]
+    # (of either pass: what the backward pass is given has been through autograd's saved-tensor hooks)
+    at = check_layer_arguments(x, router, cfg["router_bias"], wg, wu, wd, e, f, None,
+                               None if shared[0] is None else shared)
     a.T, a.D = x.shape
-    a.E, a.K, a.tile_m = cfg["num_experts"], cfg["top_k"], cfg["tile_m"]
-    a.F = wd.shape[0] // a.E
+    a.E, a.K, a.F, a.tile_m = e, cfg["top_k"], f, cfg["tile_m"]
     a.act_dtype = dtype_code(x.dtype)
     a.score_fn, a.renormalize, a.scale_input = cfg["score_fn"], int(cfg["renormalize"]), int(cfg["scale_input"])
     if cfg.get("norm_eps") is not None:
+        _check_norm_weight(norm_w, x)
         a.normed, a.norm_eps = 1, cfg["norm_eps"]
         a.norm_weight = _ptr(norm_w)
-    a.x, a.router, a.router_bias = _ptr(x), _ptr(router), _ptr(cfg["router_bias"])
-    a.w_gate, a.w_up, a.w_down = _ptr(wg), _ptr(wu), _ptr(wd)
+    a.x = x.data_ptr()
+    a.router, a.router_bias, a.w_gate, a.w_up, a.w_down = at[:5]
     if shared[0] is not None:
         a.F_shared = shared[0].shape[0]
-        a.shared_gate, a.shared_up, a.shared_down = map(_ptr, shared)
+        a.shared_gate, a.shared_up, a.shared_down = at[8:]
     return a
 
 
@@ -1107,15 +1111,12 @@ def train_forward(x: Tensor, residual: Tensor | None, router: Tensor, wg: Tensor
                   shared: tuple, norm_w: Tensor | None, cfg: dict) -> tuple[Tensor, Tensor] | None:
     """``(out, saved)`` of the layer's forward pass in training (``fs2moe_train_forward``), ``saved``
     the opaque buffer that :func:`train_backward` reads; None at sizes the call does not take.  ``cfg``
-    as for :class:`fairseq2_amd.autograd.MoEFunction`; the arguments are those that
-    :func:`check_layer_arguments` has passed."""
+    as for :class:`fairseq2_amd.autograd.MoEFunction`."""
     lib = load()
     a = _train_args(x, router, wg, wu, wd, shared, norm_w, cfg)
     saved_bytes = lib.fs2moe_train_saved_bytes(a)
     if saved_bytes < 0:
         return None
-    if cfg.get("norm_eps") is not None:
-        _check_norm_weight(norm_w, x)
     if residual is not None:
         _same("residual", residual, x.shape, x.dtype, x.device)
         a.residual = _ptr(residual)
@@ -1138,6 +1139,7 @@ def train_backward(x: Tensor, router: Tensor, wg: Tensor, wu: Tensor, wd: Tensor
     lib = load()
     a = _train_args(x, router, wg, wu, wd, shared, norm_w, cfg)
     _same("dout", dout, x.shape, x.dtype, x.device)
+    _same("saved", saved, saved.shape, torch.uint8, x.device)
     a.dout, a.saved, a.saved_bytes = dout.data_ptr(), saved.data_ptr(), saved.numel()
     operands = (x, router, wg, wu, wd, *shared, norm_w if cfg.get("norm_eps") is not None else None)
     grads = tuple(torch.empty_like(t) if n and t is not None else None for t, n in zip(operands, need))

@@ -583,11 +583,10 @@ class MoE(FeedForwardNetwork):
         shared = (None, None, None)
         if se is not None:
             shared = (se.gate_proj.weight, se.inner_proj.weight, se.output_proj.weight)
+        # (the module's own sizes; what the calls are given is checked again where addresses are taken)
         _abi.check_layer_arguments(
-            x.detach(), self.router.detach(), self.router_bias, ex.gate_proj.detach(),
-            ex.inner_proj.detach(), ex.output_proj.detach(), ex.num_local_experts, ex.inner_dim, None,
-            None if se is None else tuple(t.detach() for t in shared),
-        )
+            x, self.router, self.router_bias, ex.gate_proj, ex.inner_proj, ex.output_proj, ex.num_local_experts,
+            ex.inner_dim, None, None if se is None else shared)
         cfg = dict(
             num_experts=ex.num_local_experts, top_k=self.top_k, tile_m=self.tile_m,
             score_fn=_SCORE_FNS[self.score_fn], renormalize=self.renormalize,

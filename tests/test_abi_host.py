@@ -601,3 +601,48 @@ def test_training_calls_refuse_unaligned_operands(lib, dtype, scale_input):
         change = {"normed": 1, "norm_weight": 0x7000000, name: 0x7000002}
         rc = lib.fs2moe_train_backward(_train_args_on_paper(lib, True, **base, **change), None)
         assert rc == -1 and b"16-byte aligned" in lib.fs2moe_last_error(), name
+
+
+def test_training_calls_check_their_tensors(lib, monkeypatch):
+    """The registered operator calls the two passes without the module's checks: matrices that do not fit
+    together are refused by the passes themselves, and so is what a saved-tensor hook may hand back."""
+    from fairseq2_amd import autograd as A
+
+    launched = []
+    stub = type("Stub", (), {"__getattr__": lambda self, name: getattr(lib, name)})()
+    stub.fs2moe_train_forward = lambda a, s: launched.append("forward") or 0
+    stub.fs2moe_train_backward = lambda a, s: launched.append("backward") or 0
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
+    monkeypatch.setattr(_abi, "_lib", stub)
+    monkeypatch.setattr(_abi, "_stream", lambda: 0)
+    t, d, e, f = 40, 64, 8, 32
+    z = lambda *shape: torch.zeros(*shape, dtype=torch.bfloat16)  # noqa: E731
+    good = dict(x=z(t, d), router=z(d, e), wg=z(e * d, f), wu=z(e * d, f), wd=z(e * f, d), sg=z(f, d), su=z(f, d),
+                sd=z(d, f), norm_w=z(d))
+    bad = dict(router=z(d, e + 8), wg=z(e * d, f - 8), wu=z(e * d // 2, f), wd=z(e * f, d - 8), sg=z(f, d - 8),
+               su=z(f - 8, d), sd=z(d - 8, f), norm_w=z(d - 8))
+    cfg = dict(num_experts=e, top_k=2, tile_m=16, score_fn=_abi.SCORE_SOFTMAX, renormalize=True, scale_input=False,
+               router_bias=None, norm_eps=1e-5)
+
+    def forward(cfg=cfg, **change):
+        v = {**good, **change}
+        return A.layer_forward(v["x"], None, *[v[n] for n in good if n != "x"], cfg)
+
+    def backward(saved, dout=z(t, d), **change):
+        v = {**good, **change}
+        return A.layer_backward(v["x"], *[v[n] for n in good if n != "x"], cfg, saved, dout, (True,) * 9)
+
+    _, saved = forward()
+    grads = backward(saved)
+    assert launched == ["forward", "backward"] and [g.shape for g in grads] == [v.shape for v in good.values()]
+    for name, value in bad.items():
+        for other in (value, good[name].float()):
+            with pytest.raises(ValueError):
+                forward(**{name: other})
+            with pytest.raises(ValueError):
+                backward(saved, **{name: other})
+    with pytest.raises(ValueError):
+        forward({**cfg, "router_bias": torch.zeros(e + 1)})
+    with pytest.raises(ValueError):
+        backward((saved[0].float(),))
+    assert launched == ["forward", "backward"]
