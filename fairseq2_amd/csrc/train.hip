@@ -12,7 +12,7 @@
 namespace fs2moe {
 
 // One wave per (token, slot) pair p with row r = inv_perm[p]: dye[r] = dout[t] * w (w the pair's combine
-// weight where it scales the output, else 1), and then d_w[p] = <ye[r], dout[t]>.  A pair without a row
+// weight where it scales the output, else 1), and then d_w[p] = <ye[r], dout[t]> (ye is not read otherwise).  A pair without a row
 // (an expert id out of range) has a zero gradient.  Same products, sums and roundings as the row copy of
 // fs2moe_dispatch and fs2moe_pair_dot, whose passes over dout and launches it replaces.
 template <typename T>
@@ -164,6 +164,9 @@ bool streams(const Args& a) {
 // tokens, D 2048 / F 768, 128 experts, top-8: 1804 -> 1672 us (the copy of x 28 us and the gather of dout
 // 49 us gone, 17 us less in the first down product and 24 us in the weight gradients), 220 MB less kept.
 bool in_token_order(const Args& a) { return a.act_dtype == FS2MOE_BF16 && !a.scale_input && !streams(a); }
+// Whether the backward pass reads the experts' output rows: only for the gradients of weights on the output,
+// and in token order not even for those.
+bool keeps_ye(const Args& a) { return !a.scale_input && !in_token_order(a); }
 
 struct Saved {
   int32_t *idx, *counts, *offsets, *perm, *inv_perm;
@@ -184,7 +187,7 @@ Saved carve_saved(const Args& a, void* base) {
   s.inv_perm = static_cast<int32_t*>(c.take((int64_t)a.T * a.K * 4));
   s.xn = a.normed ? c.take((int64_t)a.T * a.D * sz) : nullptr;
   s.xe = in_token_order(a) ? nullptr : c.take(R * a.D * sz);
-  s.ye = in_token_order(a) ? nullptr : c.take(R * a.D * sz);
+  s.ye = keeps_ye(a) ? c.take(R * a.D * sz) : nullptr;
   const bool keep = !streams(a);
   s.g = keep ? c.take(R * a.F * sz) : nullptr;
   s.u = keep ? c.take(R * a.F * sz) : nullptr;
@@ -209,7 +212,7 @@ ForwardScratch carve_forward(const Args& a, void* base) {
   f.router = f.router_bytes > 0 ? c.take(f.router_bytes) : nullptr;
   f.h = in_token_order(a) ? nullptr : c.take(rows_of(a) * a.F * sz);
   f.hs = a.F_shared > 0 ? c.take((int64_t)a.T * a.F_shared * sz) : nullptr;
-  f.ye = in_token_order(a) ? c.take(rows_of(a) * a.D * sz) : nullptr;
+  f.ye = keeps_ye(a) ? nullptr : c.take(rows_of(a) * a.D * sz);
   f.total = c.used;
   return f;
 }
@@ -336,10 +339,10 @@ extern "C" int fs2moe_train_forward(const fs2moe_train_args* a, void* stream) {
                        s.offsets, s.perm, s.inv_perm, s.xe, f.disp, f.disp_bytes, stream);
   if (rc) return rc;
   const bool mapped = in_token_order(*a);
-  void* ye = mapped ? f.ye : s.ye;
+  void* ye = s.ye != nullptr ? s.ye : f.ye;
   if (s.g == nullptr)
     rc = fs2moe_grouped_swiglu_rows(s.xe, nullptr, s.counts, s.offsets, a->w_gate, a->w_up, a->w_down, nullptr,
-                                    nullptr, nullptr, a->E, a->D, a->F, R, a->act_dtype, a->act_dtype, f.h, s.ye,
+                                    nullptr, nullptr, a->E, a->D, a->F, R, a->act_dtype, a->act_dtype, f.h, ye,
                                     a->T, stream);
   else
     rc = swiglu_train(mapped ? x : s.xe, mapped ? s.perm : nullptr, s.counts, s.offsets, a->E, a->w_gate, a->w_up,

@@ -646,3 +646,19 @@ def test_training_calls_check_their_tensors(lib, monkeypatch):
     with pytest.raises(ValueError):
         backward((saved[0].float(),))
     assert launched == ["forward", "backward"]
+
+
+def test_what_a_training_step_keeps_between_its_passes(lib):
+    """The experts' output rows are kept only where the backward pass reads them: in expert order, for the
+    gradients of weights on the output; as scratch of the forward pass they are there in any case."""
+    t, d, e, k, f = 300, 256, 8, 2, 128
+    up = lambda n: (n + 255) // 256 * 256  # noqa: E731
+    rows = _abi.max_rows(t, k, e, 16)
+    ints = up(t * k * 4) * 3 + up(t * e * 4) + up(e * 4) + up((e + 1) * 4) + up(rows * 4)
+    for dtype, size, scale_input, row_matrices, products in (
+            (_abi.F32, 4, 0, 2, 2), (_abi.F32, 4, 1, 1, 2), (_abi.BF16, 2, 1, 1, 2), (_abi.BF16, 2, 0, 0, 3)):
+        a = _abi.TrainArgs()
+        a.T, a.D, a.E, a.K, a.F, a.tile_m, a.act_dtype, a.scale_input = t, d, e, k, f, 16, dtype, scale_input
+        want = ints + row_matrices * up(rows * d * size) + products * up(rows * f * size)
+        assert lib.fs2moe_train_saved_bytes(a) == want
+        assert lib.fs2moe_train_workspace_bytes(a, 0) >= (row_matrices < 2) * rows * d * size
