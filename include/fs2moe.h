@@ -57,7 +57,7 @@ extern "C" {
 #define FS2MOE_MAX_TOP_K 32
 
 /* bytes of the library's built-in scratch array (fs2moe_forward_static) */
-#define FS2MOE_STATIC_SCRATCH_BYTES (32 * 1024 * 1024)
+#define FS2MOE_STATIC_SCRATCH_BYTES (48 * 1024 * 1024)
 
 /* error codes */
 #define FS2MOE_OK 0

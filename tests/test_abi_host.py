@@ -662,3 +662,14 @@ def test_what_a_training_step_keeps_between_its_passes(lib):
         want = ints + row_matrices * up(rows * d * size) + products * up(rows * f * size)
         assert lib.fs2moe_train_saved_bytes(a) == want
         assert lib.fs2moe_train_workspace_bytes(a, 0) >= (row_matrices < 2) * rows * d * size
+
+
+def test_static_scratch_holds_the_sizes_that_fitted_32_mb(lib):
+    """The router's partial sums (up to 20 or 32 blocks to a token tile instead of 8, and for any number of
+    experts) and the tile counts in front of dispatch have grown within the same workspace: the sizes that
+    they take past 32 MB, the former size of the array, run as before.  (The largest of four million drawn
+    sizes that needed 32 MB or less then, for each of the two parts, up to 128 experts and above.)"""
+    for sizes in ((272683, 16, 475, 1, 8, 0, 1), (883, 4672, 106, 2, 128, 0, 1), (1583, 1152, 242, 4, 328, 0, 1),
+                  (2018, 896, 123, 1, 6504, 0, 1), (453, 6080, 253, 3, 48, 0, 1), (1864, 440, 256, 6, 32, 0, 16)):
+        need = lib.fs2moe_forward_workspace_bytes(*sizes, _abi.BF16)
+        assert (31 << 20) < need <= lib.fs2moe_forward_static_capacity(), sizes
