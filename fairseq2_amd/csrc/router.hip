@@ -207,7 +207,10 @@ __device__ __forceinline__ void rms_norm_cached_rows(const TA* x, const TA* w, f
   }
 }
 
-// LONG: rows of up to 12 chunks a lane in registers as well (for a kernel with registers to spare).
+// LONG: rows of up to 12 chunks a lane (bf16: D 6144) in registers as well, for a kernel with registers to
+// spare: 48 for the row, one row at a time, the weight's chunks fetched where they are used.  Norm and router
+// of 1024 tokens, 256 experts: D 4096 28.6 -> 27.3, D 6144 34.7 -> 32.9 us; 2048 tokens, D 5120 39.4 -> 38.6;
+// 4096 tokens the same within 1 us.
 template <typename TA, bool LONG = false>
 __device__ __forceinline__ void rms_norm_block_rows(const TA* x, const TA* w, float eps, TA* xn, int t0, int rows,
                                     int D, int k_lo, int k_hi) {
@@ -902,7 +905,12 @@ __global__ __launch_bounds__(1024) void router_mfma_t_kernel(
   if (tid < E) tile_counts[(size_t)blockIdx.x * E + tid] = (uint8_t)__popc(s_bits[tid]);
 }
 
-constexpr int kMaxSlices = 20;  // blocks sharing a token tile, at most
+// Blocks sharing a token tile, at most: every bf16 D up to 5120 takes one step a block (2560 with more than 128
+// experts), longer rows two.  The finishing kernel issues this many loads a lane whatever D, those past the
+// last block masked off.  With 32 of them D 6144 to 8192 would take one step as well (64 tokens, 16 to 128
+// experts 9.7-13.7 -> 7.9-13.4 us, with the norm 17.6-25.2 -> 12.3-19.3), but a layer's step of any smaller D
+// took longer: D 2048, 128 experts 32.7 -> 33.7 us at one token, D 576, 16 experts 60.5 -> 62.0 at 4000.
+constexpr int kMaxSlices = 20;
 
 // Second half of the split router: one wave per token adds the `slices` partial logits in
 // ascending order, then the bias, and selects.
@@ -1267,15 +1275,20 @@ using namespace fs2moe;
 // token tile to itself (unless it is the only tile), larger ones by the router blocks themselves.
 constexpr int kNormAloneMaxTokens = 4096;
 
-// How many blocks share a 32-token tile of the bf16 MFMA router: enough to put about 256 blocks on
-// the chip, each with at least one step of its k-groups, at most kMaxSlices.  1 = no split.
+// How many blocks share a 32-token tile of the bf16 MFMA router: one for every step of the k-groups (the last
+// may be part of one) up to about 256 blocks on the chip, at most kMaxSlices.  1 = no split, as where there
+// would be less than two whole steps.  A partial step has a block of its own as well, so that every block
+// takes exactly one (RouterMode::STEP) whatever D: with the steps rounded down only multiples of 256 did, and
+// D 1600 of 16 to 128 experts took 8.3-9.5 us at one token and 9.2-10.4 at 64, with the norm 10.4-11.5 and
+// 13.0-14.6, now 6.5-7.6, 7.2-8.7, 7.0-8.4 and 9.4-10.9.
 static int router_slices(int T, int D, int E, int act_dtype) {
   if (act_dtype != FS2MOE_BF16 || D % 8 != 0 || E > 256 || T < 1) return 1;
   const int tiles = (T + rmfma::BT - 1) / rmfma::BT;
   const int groups = E <= 128 ? rmfma::Shape<1>::GROUPS : rmfma::Shape<2>::GROUPS;
   const int nk = (D + 63) / 64;
   int s = 256 / tiles;
-  s = s < nk / groups ? s : nk / groups;
+  const int most = nk / groups < 2 ? 1 : (nk + groups - 1) / groups;
+  s = s < most ? s : most;
   s = s < kMaxSlices ? s : kMaxSlices;
   return s >= 2 ? s : 1;
 }

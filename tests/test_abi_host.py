@@ -664,8 +664,20 @@ def test_what_a_training_step_keeps_between_its_passes(lib):
         assert lib.fs2moe_train_workspace_bytes(a, 0) >= (row_matrices < 2) * rows * d * size
 
 
+@pytest.mark.parametrize("e, groups, top", [(16, 4, 5120), (128, 4, 5120), (129, 2, 2560), (256, 2, 2560)])
+def test_every_router_block_of_a_decode_step_takes_one_step(lib, e, groups, top):
+    """At any model dimension of a multiple of 64, as far as the finishing kernel's loads go: as many blocks
+    to a token tile as there are steps of ``groups`` chunks, the last of which may be part of one."""
+    for d in range(128 * groups, top + 1, 64):
+        for t in (1, 32, 33):
+            slices = lib.fs2moe_router_workspace_bytes(t, d, e, _abi.BF16) // (4 * t * e)
+            assert slices == -(-d // (64 * groups)), (t, d)
+    # less than two whole steps: one block, no scratch
+    assert lib.fs2moe_router_workspace_bytes(8, 128 * groups - 64, e, _abi.BF16) == 0
+
+
 def test_static_scratch_holds_the_sizes_that_fitted_32_mb(lib):
-    """The router's partial sums (up to 20 or 32 blocks to a token tile instead of 8, and for any number of
+    """The router's partial sums (up to 20 blocks to a token tile instead of 8, and for any number of
     experts) and the tile counts in front of dispatch have grown within the same workspace: the sizes that
     they take past 32 MB, the former size of the array, run as before.  (The largest of four million drawn
     sizes that needed 32 MB or less then, for each of the two parts, up to 128 experts and above.)"""

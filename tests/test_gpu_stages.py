@@ -82,6 +82,10 @@ def test_router_matches_oracle(gpu_device, dtype, tokens, d, e, k, mode, zipf):
 @pytest.mark.parametrize("tokens,d,e,k", [
     (1, 512, 60, 6), (32, 2048, 132, 32), (33, 1024, 60, 8), (257, 2048, 250, 5), (1024, 320, 9, 2),
     (1025, 2048, 60, 4), (40, 5120, 7, 3), (8200, 128, 60, 6),
+    # a last block with part of a step: of one chunk, of three, with a tail of a chunk; the most slices, one
+    # chunk more than they take at a step each, and with the experts that have two k-groups to a block
+    (33, 1600, 60, 8), (1, 576, 16, 2), (40, 2880, 128, 8), (17, 2632, 64, 5), (32, 5120, 128, 8), (3, 5184, 128, 4),
+    (9, 2496, 200, 5),
 ])
 @pytest.mark.parametrize("normed", [False, True])
 def test_router_and_bookkeeping_in_the_whole_layer_call(gpu_device, tokens, d, e, k, normed):
