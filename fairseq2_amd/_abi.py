@@ -19,11 +19,10 @@ ABI_VERSION = 15
 
 F32, BF16, FP8_E4M3 = 0, 1, 2
 SCORE_SIGMOID, SCORE_SOFTMAX = 0, 1
-ROUTER_OUT_IN = 0x100
-ACT_MXFP8 = 0x100  # OR-ed into a whole-layer call's w_dtype next to e4m3 weights: W8A8  # OR-ed into score_fn: the router argument is (E, D)
+ROUTER_OUT_IN = 0x100  # OR-ed into score_fn: the router argument is (E, D)
+ACT_MXFP8 = 0x100  # OR-ed into a whole-layer call's w_dtype next to e4m3 weights: W8A8
 W_IN_OUT, W_OUT_IN = 0, 1
 MAX_EXPERTS, MAX_TOP_K = 512, 32
-
 
 
 class ForwardArgs(ctypes.Structure):

@@ -1154,6 +1154,11 @@ extern "C" int fs2moe_grouped_wgrad(const void* a, const int32_t* a_row_map, con
   return segments > 1 ? launch_wgrad_reduce(partial, segments, (int64_t)M * N, dtype, dw, st) : FS2MOE_OK;
 }
 
+// The CUs that a plan counts on.  A constant and not the device's own number, which the launch asks for: a plan
+// sizes scratch in calls that touch no device, and must come out the same when it is launched.  With other
+// numbers of CUs (a partition of the chip) its cuts are only less even.
+constexpr int kPlanCUs = 256;
+
 int64_t fs2moe::wgrad_plan(WgradRequest* r, int n, int32_t E, int64_t grouped_rows, int64_t rows,
                            int32_t dtype) {
   if (dtype == FS2MOE_F32) {  // (one launch each: every single group is cut as in fs2moe_grouped_wgrad)
@@ -1171,14 +1176,14 @@ int64_t fs2moe::wgrad_plan(WgradRequest* r, int n, int32_t E, int64_t grouped_ro
   int64_t total = 0;
   for (int i = 0; i < n; ++i)
     total += tiles(r[i]) * (r[i].grouped ? grouped_rows / wgk::RK + (int64_t)E * wgk::kTileCost : one);
-  const int64_t fair = total / 256 + 1;
+  const int64_t fair = total / kPlanCUs + 1;
   int64_t bytes = 0;
   for (int i = 0; i < n; ++i) {
     r[i].segments = 1;
     if (r[i].grouped || one <= fair) continue;
     // at least 256 rows each, and no more than gives every CU a tile of this gradient
     int64_t s = (one + fair - 1) / fair;
-    const int64_t by_rows = rows / 256, by_cus = 256 / tiles(r[i]) + 1;
+    const int64_t by_rows = rows / 256, by_cus = kPlanCUs / tiles(r[i]) + 1;
     s = s < by_rows ? s : by_rows;
     s = s < by_cus ? s : by_cus;
     if (s < 2) continue;
@@ -1221,8 +1226,8 @@ int fs2moe::wgrad_all(const WgradRequest* r, int n, const int32_t* row_map, cons
                    q.map_a, q.map_b};
     if (!q.grouped && slots > 1) part += (int64_t)slots * q.M * q.N;
   }
-  if (int rc = launch_wgrad(jobs, any_mapped ? row_map : nullptr, any_grouped ? counts : nullptr, any_grouped ? offsets : nullptr,
-                            any_grouped ? E : 0, st))
+  if (int rc = launch_wgrad(jobs, any_mapped ? row_map : nullptr, any_grouped ? counts : nullptr,
+                            any_grouped ? offsets : nullptr, any_grouped ? E : 0, st))
     return rc;
   for (int i = 0; i < n; ++i)
     if (jobs.job[i].partial != nullptr)

@@ -222,15 +222,16 @@ struct DispatchAfterRouter {
 constexpr int kRouterTileTok = 32;   // tokens per tile of the MFMA routers
 constexpr int kIndexTilesMax = 512;  // tiles whose counts every block of dispatch_index_tiles adds up
 // The dispatch workspace as the tile-counting router fills it: per tile and expert the number of the
-// tile's tokens that chose the expert (a byte: at most 32; E up to a multiple of 8 of them), then per pair its rank among the tile's
-// pairs of the same expert.
+// tile's tokens that chose the expert (a byte: at most 32; E up to a multiple of 8 of them), then per
+// pair its rank among the tile's pairs of the same expert.
 inline uint8_t* tile_counts_of(void* ws) { return static_cast<uint8_t*>(ws); }
 inline int32_t* tile_rank_of(void* ws, int T, int E, int tile_tok) {
   const int64_t nt = (T + tile_tok - 1) / tile_tok;
   return reinterpret_cast<int32_t*>(static_cast<uint8_t*>(ws) + (nt * ((E + 7) / 8 * 8) + 255) / 256 * 256);
 }
 // The rest of dispatch after such a router: offsets, counts, perm and inv_perm as fs2moe_dispatch
-// writes them without a row copy, for tiles of tile_tok (8 or more, at most 32) tokens.  E at most 256; at most kIndexTilesMax tiles.
+// writes them without a row copy, for tiles of tile_tok (8 or more, at most 32) tokens.  E at most 256; at
+// most kIndexTilesMax tiles.
 int dispatch_index_tiles(const int32_t* topk_idx, int32_t T, int32_t K, int32_t E, int tile_tok, int32_t tile_m,
                          int64_t max_rows, const uint8_t* tile_counts, const int32_t* tile_rank,
                          int32_t* counts, int32_t* offsets, int32_t* perm, int32_t* inv_perm,

@@ -4,9 +4,9 @@
 // Python with its own buffers took the host longer (10 to 15 us a launch) than a layer of a few
 // thousand rows takes the GPU.  Both calls therefore carve every intermediate out of two buffers and
 // launch the whole pass.  What is new on the device is small: the gather of the output gradients, which
-// also takes the dot products that are the combine weights' gradients, the activation's derivative of a step
-// whose rows stay in token order, and the padding of a router matrix
-// whose number of experts is not a multiple of 8.
+// also takes the dot products that are the combine weights' gradients, the activation's derivative of a
+// step whose rows stay in token order, and the padding of a router matrix whose number of experts is not
+// a multiple of 8.
 #include "common.h"
 
 namespace fs2moe {
@@ -69,8 +69,8 @@ __global__ __launch_bounds__(256) void gather_backward_kernel(
 // two.)  Bound by memory: seven passes over [rows, F].  h may be dh's buffer.
 __global__ __launch_bounds__(256) void swiglu_backward_pairs_kernel(
     const uint16_t* __restrict__ g, const uint16_t* __restrict__ u, const uint16_t* __restrict__ h_fwd,
-    const uint16_t* dh, const int32_t* __restrict__ inv_perm, const float* __restrict__ topk_w, int pairs, int F, uint16_t* h,
-    uint16_t* __restrict__ dg, uint16_t* __restrict__ du, float* __restrict__ d_w) {
+    const uint16_t* dh, const int32_t* __restrict__ inv_perm, const float* __restrict__ topk_w, int pairs, int F,
+    uint16_t* h, uint16_t* __restrict__ dg, uint16_t* __restrict__ du, float* __restrict__ d_w) {
   const int p = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (p >= pairs) return;
   const int lane = threadIdx.x & 63;
@@ -350,8 +350,8 @@ extern "C" int fs2moe_train_forward(const fs2moe_train_args* a, void* stream) {
   if (rc) return rc;
   const void* base = nullptr;
   if (a->F_shared > 0) {
-    rc = swiglu_train(x, nullptr, nullptr, nullptr, 0, a->shared_gate, a->shared_up, a->shared_down, a->D, a->F_shared, a->T,
-                      a->act_dtype, s.gs, s.us, f.hs, a->out, stream);
+    rc = swiglu_train(x, nullptr, nullptr, nullptr, 0, a->shared_gate, a->shared_up, a->shared_down, a->D,
+                      a->F_shared, a->T, a->act_dtype, s.gs, s.us, f.hs, a->out, stream);
     if (rc) return rc;
     base = a->out;
   }
@@ -402,8 +402,8 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
     if ((rc = check_launch("gather_backward"))) return rc;
   }
   // the experts: dh, then h, dg and du, then the rows' gradient
-  if ((rc = fs2moe_grouped_gemm(mapped ? a->dout : b.dye, mapped ? s.perm : nullptr, s.counts, s.offsets, a->w_down, FS2MOE_W_OUT_IN, E, D, F, R, dt, b.dh,
-                                stream)))
+  if ((rc = fs2moe_grouped_gemm(mapped ? a->dout : b.dye, mapped ? s.perm : nullptr, s.counts, s.offsets, a->w_down,
+                                FS2MOE_W_OUT_IN, E, D, F, R, dt, b.dh, stream)))
     return rc;
   const void *g = s.g, *u = s.u;
   if (g == nullptr) {

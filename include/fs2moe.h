@@ -193,7 +193,12 @@ int fs2moe_grouped_swiglu_rows(const void* xe, const int32_t* row_map, const int
                                int64_t max_rows, int32_t act_dtype, int32_t w_dtype, void* h,
                                void* ye, int32_t rows_per_expert, void* stream);
 
-/* 1 if fs2moe_grouped_swiglu accepts a row_map for these sizes and types, else 0. */
+/*
+ * 1 if fs2moe_grouped_swiglu accepts a row_map for these sizes and types, else 0.  Like
+ * fs2moe_grouped_swiglu_keeps and fs2moe_grouped_gemm_sum_supported it says 1 for D and F in whole
+ * units of 64; the whole-layer and training calls read rows in place, keep the products and add the
+ * two sources for any multiple of 8, so at such sizes they take fewer passes than the stages do.
+ */
 int fs2moe_grouped_swiglu_fuses_gather(int32_t D, int32_t F, int32_t act_dtype, int32_t w_dtype);
 
 /*
@@ -245,9 +250,10 @@ int fs2moe_combine_residual(const void* ye, const int32_t* inv_perm, const int32
  *               0: they multiply the experts' output rows
  *   workspace   at least fs2moe_forward_workspace_bytes(...) bytes, 256-byte aligned
  *   out [T, D] act_dtype (out; must not alias x; may alias residual unless there is a shared expert)
- * With a large shared expert (192 MB of weights or more) and at most 16 tokens its kernels run on a stream of the
- * library's own, forked from `stream` and joined back to it inside the call (events; under stream
- * capture both branches are captured): to the caller the call is ordered on `stream` as before.
+ * With a large shared expert (192 MB of weights or more) and at most 16 tokens its kernels run on a
+ * stream of the library's own, forked from `stream` and joined back to it inside the call (events;
+ * under stream capture both branches are captured): to the caller the call is ordered on `stream` as
+ * before.
  */
 int64_t fs2moe_forward_workspace_bytes(int32_t T, int32_t D, int32_t E, int32_t K, int32_t F,
                                        int32_t F_shared, int32_t tile_m, int32_t act_dtype);
@@ -456,8 +462,8 @@ int fs2moe_rms_norm_backward(const void* x, const void* weight, float eps, const
                              void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
- * fs2moe_forward (normed 0) or fs2moe_forward_norm (normed 1) with their arguments in a struct, for
- * callers that prepare them once and change a few pointers from call to call.
+ * fs2moe_forward (normed 0) or fs2moe_forward_norm (normed 1) with their arguments in a struct: one
+ * pointer to pass through a foreign-function interface instead of thirty values.
  */
 typedef struct fs2moe_forward_args {
   int32_t T, D, E, K, F, F_shared, tile_m, act_dtype, w_dtype;
@@ -488,7 +494,9 @@ int fs2moe_copy(const void* src, void* dst, int64_t bytes, void* stream);
  * `saved` is written by the forward call and read by the backward call (which leaves it as it is);
  * `workspace` is scratch of either.  Both 256-byte aligned, of the bytes that
  * fs2moe_train_saved_bytes / fs2moe_train_workspace_bytes return for the sizes in the struct and, for
- * the backward pass (backward 1, else 0), the gradients whose pointers are set (-1: sizes these calls do not take -- bf16 matrices of 4 GB and more).
+ * the backward pass (backward 1, else 0), the gradients whose pointers are set (-1: sizes these calls
+ * do not take -- bf16 matrices of 4 GB and more).  Weights, rows, results and gradients are 16-byte
+ * aligned, x with a norm only where its own gradient or the norm weight's is taken.
  *   normed       the rows are RMS-normalised first (norm_weight [D] or NULL, norm_eps)
  *   router       (D, E); router_read: what the forward pass reads, the same or, with
  *                FS2MOE_ROUTER_OUT_IN or-ed into score_fn, its (E, D) copy
