@@ -1018,13 +1018,13 @@ def forward(
     norm: tuple[Tensor | None, float] | None = None,
     router_t: Tensor | None = None,
     act_quant: bool = False,
-    out: Tensor | None = None,
+    out_shape: torch.Size | None = None,
 ) -> Tensor:
     """The whole layer through ``fs2moe_forward``: one call, intermediates in one workspace.
     ``router_t``: optionally the router matrix expert-major, (E, D), used where the library reads it.
     ``act_quant`` (with ``scales``, i.e. e4m3 weights): the expert products on the fp8 matrix pipe,
     the rows rounded to block-scaled e4m3 inside the call (``FS2MOE_ACT_MXFP8``).
-    ``out``: optionally where the result goes, contiguous, with as many elements as ``x`` in any shape.
+    ``out_shape``: the result's shape where it is not that of ``x``, for as many elements.
     With ``residual`` ``(T, D)`` the result is ``residual + layer(x)`` from the same accumulation.
     With ``norm`` = (weight or None, eps) the rows are RMS-normalised on the way into the router
     (``fs2moe_forward_norm``): the result is ``[residual +] layer(rms_norm(x))``.
@@ -1058,10 +1058,9 @@ def forward(
     if residual is not None and residual is not x and (
             residual.shape != x.shape or residual.dtype != x.dtype or not residual.is_contiguous()):
         raise ValueError("residual must be a contiguous tensor of x's shape and dtype")
-    if out is None:
-        out = torch.empty_like(x)
-    elif out.numel() != x.numel() or out.dtype != x.dtype or out.device != x.device or not out.is_contiguous():
-        raise ValueError("out must be a contiguous tensor of x's elements")
+    out = torch.empty_like(x) if out_shape is None else x.new_empty(out_shape)
+    if out.numel() != x.numel():
+        raise ValueError("out_shape must be a shape of x's elements")
     mat, score_fn = router_operand(lib, x, router, router_t, score_fn)
     # Collected on every call, in as few steps as checking each tensor once allows: a one-token step of a
     # layer of 128 experts takes the host 36 us with its five launches, whatever the call before it was (47 us

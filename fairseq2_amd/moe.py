@@ -542,8 +542,7 @@ class MoE(FeedForwardNetwork):
                 and (se is None or type(se) is GLUFeedForwardNetwork)):
             if compiling:
                 return self._single_call(x, res, norm_args, act_quant=w8a8).view(seqs.shape)
-            out = torch.empty_like(seqs, memory_format=torch.contiguous_format)
-            return self._single_call(x, res, norm_args, act_quant=w8a8, out=out)
+            return self._single_call(x, res, norm_args, act_quant=w8a8, out_shape=seqs.shape)
         if wants_grad:
             # (only reachable inside a compiler's trace: the staged path below records no graph)
             raise RuntimeError(
@@ -632,7 +631,7 @@ class MoE(FeedForwardNetwork):
         return _abi.router_expert_major(self.router, self)
 
     def _single_call(self, x: Tensor, residual: Tensor | None = None, norm=None, *,
-                     act_quant: bool = False, out: Tensor | None = None) -> Tensor:
+                     act_quant: bool = False, out_shape: torch.Size | None = None) -> Tensor:
         """The layer through the library's whole-layer entry point: one call, one workspace
         allocation (same kernels and results as :meth:`_stages`)."""
         ex, se = self.experts, self.shared_expert
@@ -662,7 +661,7 @@ class MoE(FeedForwardNetwork):
             scales=scales, shared=shared, tile_m=self.tile_m, score_fn=_SCORE_FNS[self.score_fn],
             renormalize=self.renormalize, scale_input=self.scale_on == "input", residual=residual,
             norm=norm, router_t=_abi.router_expert_major(router, self), act_quant=act_quant,
-            out=out,
+            out_shape=out_shape,
         )
 
     @torch.no_grad()
