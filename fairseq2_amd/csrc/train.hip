@@ -12,9 +12,10 @@
 namespace fs2moe {
 
 // One wave per (token, slot) pair p with row r = inv_perm[p]: dye[r] = dout[t] * w (w the pair's combine
-// weight where it scales the output, else 1), and then d_w[p] = <ye[r], dout[t]> (ye is not read otherwise).  A pair without a row
-// (an expert id out of range) has a zero gradient.  Same products, sums and roundings as the row copy of
-// fs2moe_dispatch and fs2moe_pair_dot, whose passes over dout and launches it replaces.
+// weight where it scales the output, else 1), and then d_w[p] = <ye[r], dout[t]> (ye is not read otherwise).
+// A pair without a row (an expert id out of range) has a zero gradient.  Same products, sums and roundings as
+// the row copy of fs2moe_dispatch and fs2moe_pair_dot, whose passes over dout and launches it replaces.  With
+// weighted 0 it is a plain copy of rows, of x as well.
 template <typename T>
 __global__ __launch_bounds__(256) void gather_backward_kernel(
     const T* __restrict__ dout, const T* __restrict__ ye, const int32_t* __restrict__ inv_perm,
@@ -158,15 +159,24 @@ bool streams(const Args& a) {
   return a.T <= 16 && swiglu_streams_rows(a.act_dtype, a.act_dtype, a.D, a.F, a.E, a.T);
 }
 
-// Whether the rows stay where they are: every product and weight gradient reads the tokens' rows (x, and in
-// the backward pass dout) through the permutation, and nothing of K rows a token is copied, kept or gathered.
-// Needs rows that enter the experts unscaled, and the bf16 kernels, which take a row map.  A step of 4096
-// tokens, D 2048 / F 768, 128 experts, top-8: 1804 -> 1672 us (the copy of x 28 us and the gather of dout
-// 49 us gone, 17 us less in the first down product and 24 us in the weight gradients), 220 MB less kept.
+// Whether the rows stay in token order: the products read the tokens' rows (x, and in the backward pass dout)
+// through the permutation, the weights on the output are applied to dh and h in f32
+// (swiglu_backward_pairs_kernel), and nothing of K rows a token is kept.  Needs rows that enter the experts
+// unscaled, and the bf16 kernels, which take a row map.
 bool in_token_order(const Args& a) { return a.act_dtype == FS2MOE_BF16 && !a.scale_input && !streams(a); }
-// Whether the backward pass reads the experts' output rows: only for the gradients of weights on the output,
-// and in token order not even for those.
-bool keeps_ye(const Args& a) { return !a.scale_input && !in_token_order(a); }
+// Whether the weight gradients, too, read them there.  Their tiles are 256 columns of F wide, and each of them
+// gathers the rows anew: with more than four, two copies in expert order (of x, of dout) in front cost less,
+// unless an expert has so few rows (under two of a tile's chunks of 32) that a tile is mostly its results.
+// Steps without copies against with them, us: 8192 tokens, D 2048, F 512 / 768 / 1024 of 128, 128 and 64 experts
+// 1804 / 2563 / 2974 against 1938 / 2689 / 3033; F 1408 of 64 3424 against 3057, D 4096, F 4096 of 16 5368
+// against 4896, F 14336 of 8 17088 against 15710; the same layers at 3000 tokens 895 / 1302 / 1356, 1670, 2445,
+// 7089 against 991 / 1303 / 1365, 1614, 2340, 6489; 75 rows an expert (F 14336, 300 tokens) 2147 against 2080,
+// 37 rows (D 1024, F 2048 and D 4096, F 4096 of 16) 261 and 994 against 265 and 1009.
+constexpr int kMappedGradientMaxF = 1024, kMappedGradientRows = 64;
+bool gradients_in_place(const Args& a) {
+  return in_token_order(a) &&
+         (a.F <= kMappedGradientMaxF || (int64_t)a.T * a.K < (int64_t)kMappedGradientRows * a.E);
+}
 
 struct Saved {
   int32_t *idx, *counts, *offsets, *perm, *inv_perm;
@@ -177,6 +187,7 @@ struct Saved {
 Saved carve_saved(const Args& a, void* base) {
   Carver c{static_cast<uint8_t*>(base)};
   const int64_t R = rows_of(a), sz = elem_size(a.act_dtype);
+  const bool mapped = in_token_order(a);
   Saved s;
   s.idx = static_cast<int32_t*>(c.take((int64_t)a.T * a.K * 4));
   s.w = static_cast<float*>(c.take((int64_t)a.T * a.K * 4));
@@ -186,12 +197,13 @@ Saved carve_saved(const Args& a, void* base) {
   s.perm = static_cast<int32_t*>(c.take(R * 4));
   s.inv_perm = static_cast<int32_t*>(c.take((int64_t)a.T * a.K * 4));
   s.xn = a.normed ? c.take((int64_t)a.T * a.D * sz) : nullptr;
-  s.xe = in_token_order(a) ? nullptr : c.take(R * a.D * sz);
-  s.ye = keeps_ye(a) ? c.take(R * a.D * sz) : nullptr;
+  s.xe = mapped ? nullptr : c.take(R * a.D * sz);
+  // (the backward pass reads them for the gradients of weights on the output, in token order not even for those)
+  s.ye = mapped || a.scale_input ? nullptr : c.take(R * a.D * sz);
   const bool keep = !streams(a);
   s.g = keep ? c.take(R * a.F * sz) : nullptr;
   s.u = keep ? c.take(R * a.F * sz) : nullptr;
-  s.h = in_token_order(a) ? c.take(R * a.F * sz) : nullptr;
+  s.h = mapped ? c.take(R * a.F * sz) : nullptr;
   s.gs = a.F_shared > 0 ? c.take((int64_t)a.T * a.F_shared * sz) : nullptr;
   s.us = a.F_shared > 0 ? c.take((int64_t)a.T * a.F_shared * sz) : nullptr;
   s.total = c.used;
@@ -212,13 +224,13 @@ ForwardScratch carve_forward(const Args& a, void* base) {
   f.router = f.router_bytes > 0 ? c.take(f.router_bytes) : nullptr;
   f.h = in_token_order(a) ? nullptr : c.take(rows_of(a) * a.F * sz);
   f.hs = a.F_shared > 0 ? c.take((int64_t)a.T * a.F_shared * sz) : nullptr;
-  f.ye = keeps_ye(a) ? nullptr : c.take(rows_of(a) * a.D * sz);
+  f.ye = in_token_order(a) || a.scale_input ? c.take(rows_of(a) * a.D * sz) : nullptr;
   f.total = c.used;
   return f;
 }
 
 struct BackwardScratch {
-  void *dye, *dh, *dg, *du, *dxe, *dl, *router, *d_router, *dx_router, *dhs, *dgs, *dus, *dx_shared, *dxn,
+  void *xe, *dye, *dh, *dg, *du, *dxe, *dl, *router, *d_router, *dx_router, *dhs, *dgs, *dus, *dx_shared, *dxn,
       *norm, *wgrad;
   float* d_w;
   int64_t norm_bytes, total;
@@ -233,9 +245,10 @@ int requests(const Args& a, const Saved& s, const BackwardScratch& b, WgradReque
                  bool map_b = false) {
     if (dw != nullptr) r[n++] = WgradRequest{left, right, dw, M, N, grouped, 1, map_a, map_b};
   };
-  const bool mapped = in_token_order(a);
-  add(a.d_gate, mapped ? x : s.xe, b.dg, a.D, a.F, true, mapped);
-  add(a.d_up, mapped ? x : s.xe, b.du, a.D, a.F, true, mapped);
+  const bool mapped = gradients_in_place(a);
+  const void* xe = mapped ? x : in_token_order(a) ? b.xe : s.xe;
+  add(a.d_gate, xe, b.dg, a.D, a.F, true, mapped);
+  add(a.d_up, xe, b.du, a.D, a.F, true, mapped);
   add(a.d_down, b.dh, mapped ? a.dout : b.dye, a.F, a.D, true, false, mapped);  // (dh holds h by then)
   if (a.F_shared > 0) {
     add(a.d_shared_gate, b.dgs, x, a.F_shared, a.D, false);
@@ -251,7 +264,10 @@ BackwardScratch carve_backward(const Args& a, void* base) {
   const int64_t R = rows_of(a), sz = elem_size(a.act_dtype), T = a.T;
   const int Ep = padded_experts(a);
   BackwardScratch b;
-  b.dye = in_token_order(a) ? nullptr : c.take(R * a.D * sz);
+  // (in token order for the weight gradients alone, and only for those that are asked for)
+  const bool copies = !gradients_in_place(a), mapped = in_token_order(a);
+  b.xe = copies && mapped && (a.d_gate != nullptr || a.d_up != nullptr) ? c.take(R * a.D * sz) : nullptr;
+  b.dye = copies && (!mapped || a.d_down != nullptr) ? c.take(R * a.D * sz) : nullptr;
   b.dh = c.take(R * a.F * sz);
   b.dg = c.take(R * a.F * sz);
   b.du = c.take(R * a.F * sz);
@@ -375,8 +391,8 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
   FS2_REQUIRE(!want_x || padded_experts(*a) != a->E || aligned16(a->router),
               "train_backward: router must be 16-byte aligned");
   // (a padded router gradient is copied out element by element)
-  for (const void* p : {a->dx, padded_experts(*a) == a->E ? a->d_router : nullptr, a->d_gate, a->d_up, a->d_down, a->d_shared_gate, a->d_shared_up,
-                        a->d_shared_down, a->d_norm_weight})
+  for (const void* p : {a->dx, padded_experts(*a) == a->E ? a->d_router : nullptr, a->d_gate, a->d_up, a->d_down,
+                        a->d_shared_gate, a->d_shared_up, a->d_shared_down, a->d_norm_weight})
     FS2_REQUIRE(aligned16(p), "train_backward: gradients must be 16-byte aligned");
   FS2_REQUIRE(a->d_norm_weight == nullptr || (a->normed && a->norm_weight != nullptr),
               "train_backward: a gradient of a norm weight that is not there");
@@ -386,24 +402,26 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
   const int64_t R = rows_of(*a);
   const void* x = a->normed ? s.xn : a->x;
   int rc;
-  // output gradients in expert order, and with output-side weights the gradients of those
+  // rows in expert order: the output gradients, with those of output-side weights that are applied to them, and in
+  // token order the copies for the weight gradients
   const bool mapped = in_token_order(*a);
-  if (!mapped) {
+  auto gather = [&](const void* rows, void* to, bool weighted) -> int {
     const dim3 grid((unsigned)(((int64_t)T * K + 3) / 4)), block(256);
-    const int weighted = a->scale_input ? 0 : 1;
     if (dt == FS2MOE_BF16)
-      hipLaunchKernelGGL(gather_backward_kernel<uint16_t>, grid, block, 0, st, static_cast<const uint16_t*>(a->dout),
+      hipLaunchKernelGGL(gather_backward_kernel<uint16_t>, grid, block, 0, st, static_cast<const uint16_t*>(rows),
                          static_cast<const uint16_t*>(s.ye), s.inv_perm, s.w, T * K, K, D, weighted,
-                         static_cast<uint16_t*>(b.dye), b.d_w);
+                         static_cast<uint16_t*>(to), b.d_w);
     else
-      hipLaunchKernelGGL(gather_backward_kernel<float>, grid, block, 0, st, static_cast<const float*>(a->dout),
+      hipLaunchKernelGGL(gather_backward_kernel<float>, grid, block, 0, st, static_cast<const float*>(rows),
                          static_cast<const float*>(s.ye), s.inv_perm, s.w, T * K, K, D, weighted,
-                         static_cast<float*>(b.dye), b.d_w);
-    if ((rc = check_launch("gather_backward"))) return rc;
-  }
+                         static_cast<float*>(to), b.d_w);
+    return check_launch("gather_backward");
+  };
+  if (b.dye != nullptr && (rc = gather(a->dout, b.dye, !a->scale_input && !mapped))) return rc;
+  if (b.xe != nullptr && (rc = gather(x, b.xe, false))) return rc;
   // the experts: dh, then h, dg and du, then the rows' gradient
-  if ((rc = fs2moe_grouped_gemm(mapped ? a->dout : b.dye, mapped ? s.perm : nullptr, s.counts, s.offsets, a->w_down,
-                                FS2MOE_W_OUT_IN, E, D, F, R, dt, b.dh, stream)))
+  if ((rc = fs2moe_grouped_gemm(b.dye != nullptr ? b.dye : a->dout, b.dye != nullptr ? nullptr : s.perm, s.counts,
+                                s.offsets, a->w_down, FS2MOE_W_OUT_IN, E, D, F, R, dt, b.dh, stream)))
     return rc;
   const void *g = s.g, *u = s.u;
   if (g == nullptr) {
@@ -452,7 +470,9 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
   const int n = requests(*a, s, b, r);
   if (n > 0) {
     (void)wgrad_plan(r, n, E, R, T, dt);
-    if ((rc = wgrad_all(r, n, mapped ? s.perm : nullptr, s.counts, s.offsets, E, R, T, dt, b.wgrad, stream))) return rc;
+    if ((rc = wgrad_all(r, n, gradients_in_place(*a) ? s.perm : nullptr, s.counts, s.offsets, E, R, T, dt, b.wgrad,
+                        stream)))
+      return rc;
     if (a->d_router != nullptr && Ep != E && (rc = copy_columns(b.d_router, Ep, a->d_router, E, D, dt, st))) return rc;
   }
   if (!want_x) return FS2MOE_OK;

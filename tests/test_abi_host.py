@@ -685,3 +685,19 @@ def test_static_scratch_holds_the_sizes_that_fitted_32_mb(lib):
                   (2018, 896, 123, 1, 6504, 0, 1), (453, 6080, 253, 3, 48, 0, 1), (1864, 440, 256, 6, 32, 0, 16)):
         need = lib.fs2moe_forward_workspace_bytes(*sizes, _abi.BF16)
         assert (31 << 20) < need <= lib.fs2moe_forward_static_capacity(), sizes
+
+
+@pytest.mark.parametrize("t, f, copies", [(256, 1024, 0), (256, 1032, 1), (255, 1032, 0)])
+def test_rows_in_token_order_are_copied_for_wide_weight_gradients(lib, t, f, copies):
+    """Past four tiles of 256 columns, and from 64 rows an expert on, the weight gradients of a step in token order
+    read copies of the rows in expert order: scratch of the backward pass, and only for the gradients that are
+    asked for."""
+    d, e, k = 256, 8, 2
+    rows_bytes = (_abi.max_rows(t, k, e, 16) * d * 2 + 255) // 256 * 256
+    a = _abi.TrainArgs()
+    a.T, a.D, a.E, a.K, a.F, a.tile_m, a.act_dtype = t, d, e, k, f, 16, _abi.BF16
+    none = lib.fs2moe_train_workspace_bytes(a, 1)
+    for names, rows in ((("d_gate",), 1), (("d_up", "d_gate"), 1), (("d_down",), 1), (("d_down", "d_up"), 2)):
+        for name in ("d_gate", "d_up", "d_down"):
+            setattr(a, name, 0x1000 if name in names else None)
+        assert lib.fs2moe_train_workspace_bytes(a, 1) == none + rows * copies * rows_bytes, names

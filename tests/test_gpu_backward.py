@@ -235,6 +235,50 @@ def test_step_in_two_calls_against_its_stages(gpu_device, dtype, t, d, e, k, f, 
     assert torch.equal(some[4], grads[4])
 
 
+@pytest.mark.parametrize("t,d,e,k,skew,normed", [(192, 64, 3, 1, 0.0, False), (700, 264, 6, 2, 1.0, True),
+                                                 (1500, 512, 64, 4, 2.0, False), (300, 1032, 8, 8, 0.0, True)])
+def test_copied_rows_give_the_gradients_of_rows_in_place(gpu_device, t, d, e, k, skew, normed):
+    """Weights on the output, F 1024: the weight gradients gather the tokens' rows.  The same layer with eight
+    more columns of zeros, F 1032: they read copies in expert order.  Same rows, same order of sums: the same
+    bits in everything but the columns of zeros, whose gradients are zero where they are products of zeros."""
+    from fairseq2_amd import autograd as A
+
+    _say("copied rows", t, d, e, k, skew, normed)
+    f = 1024
+    g = torch.Generator().manual_seed(t + e)
+    mk = lambda *s, scale=1.0: (scale * torch.randn(*s, generator=g)).bfloat16().to(gpu_device)  # noqa: E731
+    x, dout, router, norm_w = mk(t, d), mk(t, d), mk(d, e, scale=d**-0.5), mk(d) if normed else None
+    wg, wu, wd = mk(e, d, f, scale=d**-0.5), mk(e, d, f, scale=d**-0.5), mk(e, f, d, scale=f**-0.5)
+    bias = (-skew * torch.log(1.0 + torch.arange(e))).to(gpu_device) if skew else None
+    cfg = dict(num_experts=e, top_k=k, tile_m=16, score_fn=_abi.SCORE_SOFTMAX, renormalize=True, scale_input=False,
+               router_bias=bias, norm_eps=1e-6 if normed else None)
+
+    def step(wg, wu, wd):
+        ws = [wg.reshape(e * d, -1), wu.reshape(e * d, -1), wd.reshape(-1, d), None, None, None]
+        out, saved = A.layer_forward(x, None, router, *ws, norm_w, cfg)
+        return out, A.layer_backward(x, router, *ws, norm_w, cfg, saved, dout, (True,) * 9)
+
+    out, grads = step(wg, wu, wd)
+    pad = torch.nn.functional.pad
+    out_pad, grads_pad = step(pad(wg, (0, 8)).contiguous(), pad(wu, (0, 8)).contiguous(),
+                              pad(wd, (0, 0, 0, 8)).contiguous())
+    assert torch.equal(out, out_pad)
+    for i, name in enumerate(("x", "router", "gate", "up", "down", "", "", "", "norm weight")):
+        a, b = grads[i], grads_pad[i]
+        if a is None:
+            assert b is None
+            continue
+        if name in ("gate", "up"):
+            b = b.view(e, d, f + 8)
+            assert not bool(b[:, :, f:].any())
+            b = b[:, :, :f].reshape(a.shape)
+        elif name == "down":
+            b = b.view(e, f + 8, d)
+            assert not bool(b[:, f:].any())
+            b = b[:, :f].reshape(a.shape)
+        assert torch.equal(a, b), f"d {name}"
+
+
 def test_rows_that_begin_anywhere_train_behind_a_norm_only(gpu_device):
     """Rows two bytes past a 16-byte line: the router's kernel normalises them wherever they are, and the
     weights' gradients then need nothing else of them; without a norm the forward pass refuses them."""
