@@ -965,10 +965,15 @@ __global__ __launch_bounds__(4 * kWave) void router_finish_kernel(
 // selection kernel and one or two that read the selection back from memory (8 tokens, 128 experts:
 // 9.1 -> 5.2 us; 777 tokens, 64 experts: 16.5 -> 10.5 us with the index kernel).  The partial logits of a
 // tile are one CU's reads, which favours small tiles (48 tokens in tiles of 32: 11.3 us, of 8: 5.4),
-// while the index kernel's every block adds up all tiles' counts, which favours few of them.
-constexpr int kFinishTok = 8, kFinishTokMax = 1024;  // tokens per tile up to so many tokens, then kRouterTileTok
+// while the index kernel's every block adds up all tiles' counts, which favours few of them: 8 tokens to a
+// tile up to 2048, 16 above (a layer of D 2048, experts of 256, in tiles of 32 / 16 / 8, us: 128 experts
+// 137.5 / 133.5 / 134.0 at 1030 tokens, 155.8 / 151.4 / 150.7 at 1828, 185.6 / 183.1 / 184.4 at 2500; 256 experts
+// 224.6 / 215.3 / 213.8, 239.5 / 230.8 / 231.7, 262.8 / 255.4 / 260.0, at 4096 300.5 / 297.0 / 303.6; 8 experts
+// 77.4 / 76.0 / 75.6, 79.1 / 78.0 / 78.0, 90.0 / 88.9 / 90.0).
+constexpr int kFinishTok = 8, kFinishTokMax = 2048, kFinishTokMany = 16;
 template <int TOK>
 constexpr int finish_tile_threads() { return TOK <= 16 ? TOK * kWave : 1024; }
+static_assert(finish_tile_threads<kRouterTileTok>() == finish_tile_threads<kFinishTokMany>(), "one launch for both");
 template <int J, bool ALL, int TOK>
 __global__ __launch_bounds__(finish_tile_threads<TOK>()) void router_finish_tile_kernel(
     const float* __restrict__ partial, int slices, const float* __restrict__ bias, int T, int E,
@@ -1469,7 +1474,8 @@ static int router_entry(const void* x, const void* norm_w, float norm_eps, void*
       const dim3 fgrid((T + 3) / 4), fblock(4 * kWave);
       const int j = (E + 63) / 64;
       const bool all = T <= kRouterTileTok;
-      const int tok = all || T > kFinishTokMax ? kRouterTileTok : kFinishTok, tiles = (T + tok - 1) / tok;
+      const int tok = all ? kRouterTileTok : T > kFinishTokMax ? kFinishTokMany : kFinishTok;
+      const int tiles = (T + tok - 1) / tok;
       if (disp != nullptr && logits == nullptr &&
           (all || (disp->row_w == nullptr && disp->ws != nullptr && tiles <= kIndexTilesMax &&
                    disp->ws_bytes >= fs2moe_dispatch_workspace_bytes(T, K, E)))) {
@@ -1479,9 +1485,9 @@ static int router_entry(const void* x, const void* norm_w, float norm_eps, void*
   case JJ:                                                                                         \
     hipLaunchKernelGGL((all                 ? router_finish_tile_kernel<JJ, true, kRouterTileTok>  \
                         : tok == kFinishTok ? router_finish_tile_kernel<JJ, false, kFinishTok>     \
-                                            : router_finish_tile_kernel<JJ, false, kRouterTileTok>), \
+                                            : router_finish_tile_kernel<JJ, false, kFinishTokMany>), \
                        dim3(tiles), dim3(tok == kFinishTok ? finish_tile_threads<kFinishTok>()     \
-                                                           : finish_tile_threads<kRouterTileTok>()), \
+                                                           : finish_tile_threads<kFinishTokMany>()), \
                        0, s, partial, slices, bias, T, E, K, \
                        score_fn, renormalize, topk_idx, topk_w, tile_counts, tile_rank, disp->tile_m, \
                        disp->max_rows, disp->counts, disp->offsets, disp->perm, disp->inv_perm,    \

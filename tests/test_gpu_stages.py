@@ -77,8 +77,8 @@ def test_router_matches_oracle(gpu_device, dtype, tokens, d, e, k, mode, zipf):
 
 # Numbers of experts that are no multiple of 8 on the matrix-pipe router (rows of the matrix begin anywhere, the
 # last chunk ends past it), and the bookkeeping that the router's kernels leave to the whole-layer call: in one
-# block (up to 32 tokens), in tiles of 8 (up to 1024) and of 32, with one step of the model dimension to a
-# block (normalised on the way) and with several.
+# block (up to 32 tokens), in tiles of 8 (up to 2048), of 16 and of 32, with one step of the model dimension to
+# a block (normalised on the way) and with several.
 @pytest.mark.parametrize("tokens,d,e,k", [
     (1, 512, 60, 6), (32, 2048, 132, 32), (33, 1024, 60, 8), (257, 2048, 250, 5), (1024, 320, 9, 2),
     (1025, 2048, 60, 4), (40, 5120, 7, 3), (8200, 128, 60, 6),
@@ -86,6 +86,8 @@ def test_router_matches_oracle(gpu_device, dtype, tokens, d, e, k, mode, zipf):
     # chunk more than they take at a step each, and with the experts that have two k-groups to a block
     (33, 1600, 60, 8), (1, 576, 16, 2), (40, 2880, 128, 8), (17, 2632, 64, 5), (32, 5120, 128, 8), (3, 5184, 128, 4),
     (9, 2496, 200, 5),
+    # the last tile of 8, the first and the last of 16
+    (2047, 1024, 60, 4), (2049, 512, 132, 32), (4096, 512, 250, 5),
 ])
 @pytest.mark.parametrize("normed", [False, True])
 def test_router_and_bookkeeping_in_the_whole_layer_call(gpu_device, tokens, d, e, k, normed):
