@@ -164,18 +164,25 @@ bool streams(const Args& a) {
 // (swiglu_backward_pairs_kernel), and nothing of K rows a token is kept.  Needs rows that enter the experts
 // unscaled, and the bf16 kernels, which take a row map.
 bool in_token_order(const Args& a) { return a.act_dtype == FS2MOE_BF16 && !a.scale_input && !streams(a); }
-// Whether the weight gradients, too, read them there.  Their tiles are 256 columns of F wide, and each of them
-// gathers the rows anew: with more than four, two copies in expert order (of x, of dout) in front cost less,
-// unless an expert has so few rows (under two of a tile's chunks of 32) that a tile is mostly its results.
-// Steps without copies against with them, us: 8192 tokens, D 2048, F 512 / 768 / 1024 of 128, 128 and 64 experts
-// 1804 / 2563 / 2974 against 1938 / 2689 / 3033; F 1408 of 64 3424 against 3057, D 4096, F 4096 of 16 5368
-// against 4896, F 14336 of 8 17088 against 15710; the same layers at 3000 tokens 895 / 1302 / 1356, 1670, 2445,
-// 7089 against 991 / 1303 / 1365, 1614, 2340, 6489; 75 rows an expert (F 14336, 300 tokens) 2147 against 2080,
-// 37 rows (D 1024, F 2048 and D 4096, F 4096 of 16) 261 and 994 against 265 and 1009.
-constexpr int kMappedGradientMaxF = 1024, kMappedGradientRows = 64;
+// Whether the weight gradients, too, read them there.  Copies in expert order (of x, of dout) are two passes;
+// without them each tile of 256 columns of F gathers the rows anew, and a chunk of rows takes it longer, which
+// the largest expert's tiles, chains of their chunks, pay in full.  So: in place up to four such tiles and up to
+// 768 rows an expert on average, and with so few rows (under two chunks of 32) that a tile is mostly its results.
+// Steps without copies against with them, us, experts equally loaded:
+//   8192 tokens, D 2048, F 512 / 768 of 128, 1024 of 64   1804 / 2563 / 2974 against 1938 / 2689 / 3033
+//   F 1408 of 64; D 4096, F 4096 of 16, F 14336 of 8      3424; 5368, 17088 against 3057; 4896, 15710
+//   3000 tokens, the same six                             895 / 1302 / 1356, 1670, 2445, 7089 against
+//                                                         991 / 1303 / 1365, 1614, 2340, 6489
+//   75 rows an expert, F 14336; 37, F 2048 and 4096       2147; 261, 994 against 2080; 265, 1009
+// and by a popularity law of exponent 1.2 (the largest has a fifth of the rows):
+//   512 rows an expert on average, F 512 / 768 of 128     2005 / 2850 against 1995 / 2744
+//   1024, D 2048, F 1024 of 64; D 1024, F 1024 of 32;     3335; 1013;
+//   D 4096, F 1024 of 16                                  1729 against 3020; 921; 1597
+constexpr int kMappedGradientMaxF = 1024, kMappedGradientRows = 64, kMappedGradientMaxRows = 768;
 bool gradients_in_place(const Args& a) {
-  return in_token_order(a) &&
-         (a.F <= kMappedGradientMaxF || (int64_t)a.T * a.K < (int64_t)kMappedGradientRows * a.E);
+  const int64_t pairs = (int64_t)a.T * a.K;
+  return in_token_order(a) && ((a.F <= kMappedGradientMaxF && pairs <= (int64_t)kMappedGradientMaxRows * a.E) ||
+                               pairs < (int64_t)kMappedGradientRows * a.E);
 }
 
 struct Saved {

@@ -687,11 +687,11 @@ def test_static_scratch_holds_the_sizes_that_fitted_32_mb(lib):
         assert (31 << 20) < need <= lib.fs2moe_forward_static_capacity(), sizes
 
 
-@pytest.mark.parametrize("t, f, copies", [(256, 1024, 0), (256, 1032, 1), (255, 1032, 0)])
+@pytest.mark.parametrize("t, f, copies", [(256, 1024, 0), (256, 1032, 1), (255, 1032, 0), (3072, 64, 0), (3073, 64, 1)])
 def test_rows_in_token_order_are_copied_for_wide_weight_gradients(lib, t, f, copies):
-    """Past four tiles of 256 columns, and from 64 rows an expert on, the weight gradients of a step in token order
-    read copies of the rows in expert order: scratch of the backward pass, and only for the gradients that are
-    asked for."""
+    """Past four tiles of 256 columns, from 64 rows an expert on, and past 768 rows whatever the columns, the weight
+    gradients of a step in token order read copies of the rows in expert order: scratch of the backward pass, and
+    only for the gradients that are asked for."""
     d, e, k = 256, 8, 2
     rows_bytes = (_abi.max_rows(t, k, e, 16) * d * 2 + 255) // 256 * 256
     a = _abi.TrainArgs()
