@@ -279,6 +279,20 @@ def test_copied_rows_give_the_gradients_of_rows_in_place(gpu_device, t, d, e, k,
         assert torch.equal(a, b), f"d {name}"
 
 
+def test_the_backward_operator_refuses_matrices_that_do_not_fit(gpu_device):
+    """``torch.ops.fairseq2_amd.moe_backward`` reaches the library without the module's checks."""
+    _say("operator, mismatched matrices")
+    t, d, e, f = 40, 64, 8, 32
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=gpu_device)  # noqa: E731
+    good = [z(t, d), z(t, d), z(d, e), None, z(e * d, f), z(e * d, f), z(e * f, d), z(f, d), z(f, d), z(d, f)]
+    tail = (e, 2, 16, _abi.SCORE_SOFTMAX, True, False, None, False, 0.0)
+    op = torch.ops.fairseq2_amd.moe_backward
+    assert [g.shape for g in op(*good, *tail)] == [v.shape for v in good[1:] if v is not None]
+    for i, bad in ((2, z(d, e + 8)), (4, z(e * d, f - 8)), (5, z(e * d // 2, f)), (7, z(f - 8, d)), (9, z(d, f - 8))):
+        with pytest.raises(ValueError):
+            op(*good[:i], bad, *good[i + 1 :], *tail)
+
+
 def test_rows_that_begin_anywhere_train_behind_a_norm_only(gpu_device):
     """Rows two bytes past a 16-byte line: the router's kernel normalises them wherever they are, and the
     weights' gradients then need nothing else of them; without a norm the forward pass refuses them."""
