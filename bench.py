@@ -28,20 +28,21 @@ MFMA_PEAK_TFLOPS = {"bf16": 2500.0, "fp32": 157.3, "fp8": 5000.0}  # dense, publ
 
 # HBM bytes per launch of the dominant kernel pair, from `rocprofv3 --pmc FETCH_SIZE` and
 # `--pmc WRITE_SIZE` runs of this script (see profiles/); None until measured for a workload.
-# The commit whose kernels the table below was measured on: a kernel change after it makes the
-# figures stale until the counter runs are repeated (the roofline object carries the stamp).
-MEASURED_TRAFFIC_AT = "06e32e2"
 MEASURED_TRAFFIC_BYTES: dict[str, float | None] = {
     # profiles/bench_<workload>_all_kernels.md, the two launches of the grouped experts together
     # (FETCH_SIZE scaled by 2.0, WRITE_SIZE by 1.0 against a 256 MiB copy)
     "qwen3_30b_a3b": 2.653e9,     # gate/up 1566 + 101 MB, down 717 + 269 MB
     "mixtral_8x7b": 13.402e9,     # gate/up 8792 + 470 MB, down 4006 + 134 MB
     "llama4_scout": 6.677e9,      # routed experts only: gate/up 4103 + 135 MB, down 2355 + 84 MB
-    "small_fp32": 0.866e9,        # gate/up 402 + 46 MB, down 401 + 17 MB
-    "qwen3_decode_fp8": 0.222e9,  # gate/up 143 + 1 MB, down 76 + 2 MB
+    "small_fp32": 0.377e9,        # gate/up 230 + 46 MB, down 85 + 17 MB
+    "qwen3_decode_fp8": 0.221e9,  # gate/up 143 + 1 MB, down 76 + 2 MB
     "qwen3_30b_a3b_fp8": 1.886e9,  # gate/up 1033 + 101 MB, down 484 + 269 MB
     "qwen3_30b_a3b_w8a8": 1.475e9,  # gate/up 778 + 67 MB, down 362 + 269 MB
 }
+# The commit whose kernels each figure was measured on: a kernel change after it makes the figure stale
+# until the counter runs are repeated (the roofline object carries the stamp).
+MEASURED_TRAFFIC_AT = {**dict.fromkeys(MEASURED_TRAFFIC_BYTES, "06e32e2"),
+                       **dict.fromkeys(("small_fp32", "qwen3_decode_fp8"), "3a230ec")}
 
 
 def parse_args():
@@ -520,7 +521,8 @@ def main() -> int:
         roofline = {
             "kernel": kernel, "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-            "traffic": MEASURED_TRAFFIC_BYTES.get(args.workload), "traffic_measured_at": MEASURED_TRAFFIC_AT,
+            "traffic": MEASURED_TRAFFIC_BYTES.get(args.workload),
+            "traffic_measured_at": MEASURED_TRAFFIC_AT.get(args.workload),
             "launch_ms": round(exp_ms, 4), "launch_timing": "calls queued back to back",
             "bytes_per_launch": work["experts"]["bytes"], "active_experts": active,
         }
@@ -529,7 +531,8 @@ def main() -> int:
         roofline = {
             "kernel": kernel, "bound": "mfma", "achieved": round(achieved, 2), "peak": peak_tf,
             "unit": "TFLOP/s", "frac": round(achieved / peak_tf, 4),
-            "traffic": MEASURED_TRAFFIC_BYTES.get(args.workload), "traffic_measured_at": MEASURED_TRAFFIC_AT,
+            "traffic": MEASURED_TRAFFIC_BYTES.get(args.workload),
+            "traffic_measured_at": MEASURED_TRAFFIC_AT.get(args.workload),
             "launch_ms": round(exp_ms, 4),
             "flops_per_launch": work["experts"]["flops"],
         }
