@@ -21,6 +21,7 @@
 #include "common.h"
 #include "tile_map.h"
 #include "experts_dma.h"
+#include "experts_half.h"
 #include "experts_f32.h"
 #include "experts_fp8.h"
 #include "experts_gemv.h"
@@ -227,6 +228,30 @@ static bool whole_units(int act_dtype, int D, int F) {
   return act_dtype == FS2MOE_BF16 && D % (2 * dma::BK) == 0 && F % (2 * dma::BK) == 0;
 }
 
+// One launch of the bf16 kernel on smaller tiles (experts_half.h), one block per CU.
+template <int BM, int BNV, bool DUAL, int BLAYOUT, bool KEEP_GU, bool TWO_SRC>
+static int launch_half(const void* a, const int32_t* row_map, int K, const void* b0, const void* b1,
+                       const void* s0, const void* s1, void* c, int N, const Groups& g, const char* what,
+                       int num_blocks, hipStream_t stream) {
+  auto k = glu_gemm_bf16_half_kernel<BM, BNV, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>;
+  constexpr int bytes = half_tiles::smem_bytes(BM, BNV), bn = DUAL ? BNV / 2 : BNV;
+  static bool attr_set = false;  // benign race: setting the attribute is idempotent
+  if (!attr_set) {
+    hipError_t e =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e != hipSuccess) {
+      set_error("%s: cannot reserve %d bytes of LDS: %s", what, bytes, hipGetErrorString(e));
+      return FS2MOE_ERR_LAUNCH;
+    }
+    attr_set = true;
+  }
+  hipLaunchKernelGGL(k, dim3((unsigned)num_blocks), dim3(half_tiles::THREADS), bytes, stream,
+                     static_cast<const uint16_t*>(a), row_map, K, static_cast<const uint16_t*>(b0),
+                     static_cast<const uint16_t*>(b1), static_cast<const float*>(s0), static_cast<const float*>(s1),
+                     static_cast<uint16_t*>(c), N, K, N, g, (N + bn - 1) / bn);
+  return check_launch(what);
+}
+
 // One launch of the bf16 throughput kernel on persistent blocks, one per CU (the 128 KB ring allows no
 // more), a multiple of the 8 XCDs.  `b1`, `s0` and `s1` as the kernel's variants take them.
 template <bool DUAL, int BLAYOUT, bool KEEP_GU = false, bool TWO_SRC = false>
@@ -258,6 +283,23 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
   if ((rows_bound / BM + groups + 1) * nt > 0x7fffffffll) {
     set_error("%s: too many tiles", what);
     return FS2MOE_ERR_UNSUPPORTED;
+  }
+  if constexpr (BLAYOUT != W_FP8_TILED) {
+    // (tiles of 64 x 64 are counted in 31 bits too)
+    const bool counted = (rows_bound / 64 + groups + 1) * ((N + 63) / 64) <= 0x7fffffffll;
+    switch (counted ? half_tiles::pick(DUAL, rows_bound, groups, K, N, num_blocks) : 0) {
+      case 1:
+        if constexpr (!DUAL)
+          return launch_half<64, 64, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
+                                                                      num_blocks, stream);
+        break;
+      case 2:
+        return launch_half<64, 128, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
+                                                                     num_blocks, stream);
+      case 3:
+        return launch_half<128, 128, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
+                                                                      num_blocks, stream);
+    }
   }
   hipLaunchKernelGGL(K % (2 * BK) == 0 ? whole : tail, dim3((unsigned)num_blocks), dim3(NWAVES * 64),
                      SMEM_BYTES, stream, static_cast<const uint16_t*>(a), row_map, K,

@@ -1,0 +1,398 @@
+// bf16 grouped GEMM on tiles of 128 x 128, 64 x 128 or 64 x 64 (rows x "virtual" channels: gate and up channels of
+// 64 each when DUAL), for launches whose 256 x 256 tiles (experts_dma.h) would leave CUs idle.
+//
+// What bounds it: with few tiles a CU's time is its tiles' bytes over what it takes in.  Four waves bring a CU 47 GB/s
+// through registers and 55 straight into LDS, eight 70 straight into LDS (every CU, blocks that do nothing else), so
+// all eight waves load, straight into LDS, and the ring holds as many stages of 64 k as 128 KB allow (4, 5 or 8),
+// all but one on their way.  80 rows, K 3200, N 1408: the throughput kernel's 6 tiles 42 us, 44 tiles of 64 x 64 19;
+// 8 experts of 290 rows, K 5408, N 704: 89 us, 240 tiles of 64 x 128 45 us.  Where there are several rounds of tiles
+// the throughput kernel's cost the chip less (half_tiles::pick).
+//
+// The k order of every sum is the throughput kernel's, on the same instruction: the same bits.
+//
+// In LDS a stage is its activations (rows of 128 bytes, 16-byte chunk kc of row r in place kc ^ ((r >> 1) & 7)) and
+// its weights: (out, in) matrices like the activations; (in, out) matrices as rows of one k, of 256 bytes (chunk c of
+// row k in place c ^ ((k & 3) << 2)) or 128 (c ^ (((k >> 1) & 1) << 2); with DUAL a sub-tile per matrix), so that the
+// four rows a transposing read touches lie in different banks.
+// Rows, channels and k that do not exist load zeros and touch no memory (buffer loads past the buffer's end).
+//
+// Blocks are persistent, one per CU; tile i of the list (expert-major, row block minor inside bands) goes to
+// slot i % grid, where slots 32 c .. 32 c + 31 are the blocks of XCD c: what an XCD works on at a time are
+// neighbours, which share weights and rows in its L2.  A block's tiles form one stream of stages.
+#pragma once
+
+#include <type_traits>
+
+#include "common.h"
+#include "tile_map.h"
+
+namespace fs2moe {
+namespace half_tiles {
+constexpr int BK = 64;
+constexpr int WAVES = 8, THREADS = WAVES * 64;
+constexpr int BAND = 8;                        // row blocks per band of the tile order
+constexpr int LDE = 144, EPI_BYTES = WAVES * 16 * LDE;  // epilogue: 16 rows of up to 128 bytes per wave
+constexpr int TABLE_INTS = 3 * FS2MOE_MAX_EXPERTS + 8;
+constexpr int stage_bytes(int BM, int BNV) { return (BM + BNV) * BK * 2; }
+constexpr int stages(int BM, int BNV) { return 131072 / stage_bytes(BM, BNV); }
+constexpr int smem_bytes(int BM, int BNV) {
+  return stages(BM, BNV) * stage_bytes(BM, BNV) + EPI_BYTES + TABLE_INTS * 4;
+}
+constexpr uint32_t NOWHERE = 0xfffffff0u;      // an offset past any buffer's end
+
+// Which of these tiles a launch takes: 0 none (the throughput kernel), else the smallest whose tiles are about
+// one a CU: 1 64 x 64 (single products), 2 64 x 128, 3 128 x 128.
+// us, throughput kernel and 1, 2, 3 (single products but for the last two, which are gate/up and down):
+//   80 rows, K 3200, N 1408              42 against 19, 23, 28     (5, 44, 22, 11 tiles)
+//   755 rows, K 1408, N 576              25 against 12, 14, 18
+//   8 experts of 290, K 5408, N 704      89 against 59, 45, 56     (480, 240, 144 tiles: one round of the second)
+//   3001 rows, K 1368, N 1024            28 against 27, 25, 20
+//   16 experts of 375, K 1368, N 1024    33 against 62, 50, 37     (none fits one round)
+//   32 of 35, D 1472, F 1216             90 against 79 (2), 80 (3) (the throughput kernel: 1.25 rounds)
+//   64 of 23, D 2944, F 1840             377 against 394, 400      (memory)
+inline int pick(bool dual, int64_t rows, int groups, int K, int N, int cus) {
+  // The experts' rows, which only the device knows, as the buffers' size has them: less what blocks of 16 pad
+  // them by, equally loaded.
+  const int64_t real = rows > 15ll * groups ? rows - 15ll * groups : rows;
+  const int64_t each = groups ? real / groups : real;
+  auto tiles = [&](int bm, int bn) -> int64_t {
+    const int64_t nt = (N + bn - 1) / bn;
+    if (groups == 0) return (rows + bm - 1) / bm * nt;
+    // (half of a last row block per expert)
+    const int64_t blocks = groups + (each > bm / 2 ? (real - (int64_t)groups * (bm / 2)) / bm : 0);
+    return (blocks < real ? blocks : real) * nt;
+  };
+  const int64_t room = cus - cus / 16;  // (experts are not equally loaded: a few tiles more)
+  if (!dual && tiles(64, 64) <= room) return 1;
+  if (tiles(64, dual ? 64 : 128) <= room) return 2;
+  if (tiles(128, dual ? 64 : 128) <= room) return 3;
+  // Several rounds of tiles of a few rows: rounds of the throughput kernel (1 us per 64 k and 6 per tile, us) against
+  // rounds of these (0.4 and 4), neither faster than memory delivers half of the experts' weights (5.2 TB/s; with few
+  // tokens or a skewed load not all experts have rows), and a fifth for what that leaves out.
+  if (groups > 0 && each <= 64) {
+    const int64_t units = (K + BK - 1) / BK, active = groups < real ? groups : real;
+    const int64_t memory = active * K * N * (dual ? 2 : 1) / 5200;  // ns
+    auto rounds = [&](int64_t n) { return (n + cus - 1) / cus; };
+    const int64_t whole = rounds(tiles(256, dual ? 128 : 256)) * (units * 1000 + 6000);
+    const int64_t small = rounds(tiles(64, dual ? 64 : 128)) * (units * 400 + 4000);
+    if ((small > memory ? small : memory) * 6 < (whole > memory ? whole : memory) * 5) return 2;
+  }
+  return 0;
+}
+}  // namespace half_tiles
+
+// 16 bytes per lane from a buffer to LDS, lane l's to lds + 16 l.  Written out because the compiler, which cannot
+// tell the ring's stages apart, would wait for every load in flight before each LDS read.  The caller waits
+// (vmcnt) in front of the barrier that hands the stage over.
+__device__ __forceinline__ void buffer_to_lds(const void* base, uint32_t off, uint32_t lds) {
+  const uint64_t b = (uint64_t)base;
+  const u32x4 rsrc = {(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, half_tiles::NOWHERE, 0x00020000u};
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc),
+               "s"(lds)
+               : "memory");
+}
+
+// Arguments as glu_gemm_bf16_dma_kernel takes them (KEEP_GU: the products' destinations in S0 and S1; TWO_SRC:
+// the second activations in S0, the second weights in B1).  n_tiles: of 64 (DUAL) or 128 channels.
+template <int BM, int BNV, bool DUAL, int BLAYOUT, bool KEEP_GU = false, bool TWO_SRC = false>
+__global__ __launch_bounds__(half_tiles::THREADS, 2) void glu_gemm_bf16_half_kernel(
+    const uint16_t* __restrict__ A, const int32_t* __restrict__ row_map, int lda,
+    const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1, const float* __restrict__ S0,
+    const float* __restrict__ S1, uint16_t* __restrict__ C, int ldc, int Kdim, int N, Groups g, int n_tiles) {
+  using namespace half_tiles;
+  static_assert(!KEEP_GU || DUAL, "the products are kept by the gate/up kernel only");
+  static_assert(!TWO_SRC || !DUAL, "two sources: one matrix each");
+  constexpr bool KN = BLAYOUT == FS2MOE_W_IN_OUT;
+  static_assert((BM == 64 || BM == 128) && (BNV == 128 || (BNV == 64 && !DUAL)), "tiles that the loads are cut for");
+  constexpr int A_BYTES = BM * BK * 2, B_BYTES = BNV * BK * 2, STAGE_BYTES = A_BYTES + B_BYTES;
+  constexpr int STAGES = stages(BM, BNV), RING_BYTES = STAGES * STAGE_BYTES;
+  constexpr int PA = BM / 64, PB = BNV / 64, LOADS = PA + PB;  // of a wave and stage
+  constexpr int BN = DUAL ? BNV / 2 : BNV;       // real channels per tile
+  constexpr int BROW = BN * 2;                   // bytes per LDS row of (in, out) weights
+  constexpr int NF = DUAL || BM * BNV == 128 * 128 ? 2 : 1;  // 32-channel fragments of a wave
+  constexpr int WN = BNV / 32 / NF;              // waves across the channels
+  constexpr int COLS = DUAL ? 32 : NF * 32;      // channels a wave writes
+  constexpr int TILE_STORES = COLS / 16 * (KEEP_GU ? 3 : 1);  // of a wave
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
+  int32_t* s_start = reinterpret_cast<int32_t*>(smem_raw + RING_BYTES + EPI_BYTES);  // [E + 1] row blocks
+  int32_t* s_counts = s_start + FS2MOE_MAX_EXPERTS + 4;
+  int32_t* s_offsets = s_counts + FS2MOE_MAX_EXPERTS;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // The wave's 32 rows and its share of the channels; waves past the tile only load.  (Waves w and w + 4 share a
+  // SIMD.)
+  const int wm = wave / WN, wn = wave % WN;
+  const int lr = lane & 31, lk = lane >> 5;
+
+  // ---- row blocks of the experts before each
+  const bool dense = g.counts == nullptr;
+  const int E = dense ? 1 : g.E;
+  {
+    __shared__ int s_wave_tot[WAVES];
+    const int cnt = dense ? (tid == 0 ? g.dense_rows : 0) : (tid < E ? g.counts[tid] : 0);
+    const int off = dense || tid >= E ? 0 : g.offsets[tid];
+    const int blocks = (cnt + BM - 1) / BM;
+    int incl = blocks;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, kWave);
+      if (lane >= o) incl += v;
+    }
+    if (lane == 63) s_wave_tot[wave] = incl;
+    __syncthreads();
+    int base = 0;
+    for (int w = 0; w < wave; ++w) base += s_wave_tot[w];
+    if (tid < E) {
+      s_start[tid] = base + incl - blocks;
+      s_counts[tid] = cnt;
+      s_offsets[tid] = off;
+    }
+    if (tid == E - 1) s_start[E] = base + incl;
+    __syncthreads();
+  }
+  const int slot = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3), grid = (int)gridDim.x;
+  const int tiles = s_start[E] * n_tiles;  // (the host guarantees that it fits 31 bits)
+  const int my_tiles = slot < tiles ? (tiles - slot + grid - 1) / grid : 0;
+  if (my_tiles == 0) return;
+  const int units = (Kdim + BK - 1) / BK, nu = (TWO_SRC ? 2 : 1) * units;  // stages per tile
+
+  struct Tile {
+    int e, row0, row_end, n0;
+  };
+  auto locate = [&](int j) {
+    const int t = slot + j * grid, mt = t / n_tiles;  // mt: which expert, as its tiles are contiguous
+    int found = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + lane;
+      const unsigned long long m = __ballot(e < E && s_start[e] <= mt && mt < s_start[e + 1]);
+      if (m) found = e0 + (int)__builtin_ctzll(m);
+    }
+    found = __builtin_amdgcn_readfirstlane(found);
+    const int first = s_start[found], l = t - first * n_tiles, per_band = BAND * n_tiles;
+    const int b = l / per_band, i = l - b * per_band;
+    const int left = s_start[found + 1] - first - b * BAND, high = left < BAND ? left : BAND;
+    const int nt = i / high, row = (b * BAND + i - nt * high) * BM, cnt = s_counts[found];
+    Tile r;
+    r.e = found;
+    r.row0 = __builtin_amdgcn_readfirstlane(s_offsets[found] + row);
+    r.row_end = __builtin_amdgcn_readfirstlane(s_offsets[found] + (cnt < row + BM ? cnt : row + BM));
+    r.n0 = __builtin_amdgcn_readfirstlane(nt) * BN;
+    return r;
+  };
+  const size_t wstride = (size_t)Kdim * N;
+
+  // ---- the stream of stages into LDS: stage u of the block goes to slot u % STAGES
+  const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem_raw;
+  // The wave's pieces of 1 KB: rows 8 wave .. 8 wave + 7 of the activations and, 64 further on, 8 more; of the
+  // weights likewise (with DUAL the first of the gate and the second of the up matrix).  A lane's place in piece i:
+  uint32_t pa[PA], pb[PB];
+  // chunk of the row's 128 bytes that the lane fetches (the same for both pieces), of activations and (out, in)
+  // weights; k row of (in, out) weights in the stage
+  const int kc = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);
+  constexpr int KROWS = 1024 / BROW, KCHUNKS = BROW / 16;  // rows and chunks of a piece of (in, out) weights
+  auto k_key = [](int k) { return BROW == 128 ? ((k >> 1) & 1) << 2 : (k & 3) << 2; };
+  int ld_tile = 0, ld_ku = 0, ld_slot = 0;
+  const uint16_t* ld_b[2] = {B0, B0};
+  auto setup_tile = [&]() {
+    const Tile t = locate(ld_tile);
+    ld_b[0] = B0 + (size_t)t.e * wstride;
+    ld_b[1] = DUAL || TWO_SRC ? B1 + (size_t)t.e * wstride : ld_b[0];
+#pragma unroll
+    for (int i = 0; i < PA; ++i) {
+      const int piece_row = 8 * (wave + 8 * i);  // uniform
+      int row = t.row0 + piece_row + (lane >> 3);
+      const bool in = row < t.row_end;
+      if (row_map != nullptr) {
+        // (scalar loads: a vector load would be waited for with every stage in flight; rows past the end
+        // repeat the last one's entry)
+        int entry[8];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          const int at = t.row0 + piece_row + r;
+          entry[r] = row_map[at < t.row_end ? at : t.row_end - 1];
+        }
+        row = entry[0];
+#pragma unroll
+        for (int r = 1; r < 8; ++r) row = lane >> 3 == r ? entry[r] : row;
+      }
+      pa[i] = in ? (uint32_t)row * (uint32_t)lda * 2u + (uint32_t)kc * 16u : NOWHERE;
+    }
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      if constexpr (KN) {
+        const int k = KROWS * (DUAL ? wave : wave + 8 * i) + lane / KCHUNKS, key = k_key(k);
+        const int col = t.n0 + ((lane % KCHUNKS) ^ key) * 8;
+        pb[i] = col < N ? ((uint32_t)k * (uint32_t)N + (uint32_t)col) * 2u : NOWHERE;
+      } else {
+        const int ch = t.n0 + 8 * (DUAL ? wave : wave + 8 * i) + (lane >> 3);
+        pb[i] = ch < N ? (uint32_t)ch * (uint32_t)Kdim * 2u + (uint32_t)kc * 16u : NOWHERE;
+      }
+    }
+  };
+  // Load l of the stage to load next: the activations' pieces, then the weights'.
+  auto load = [&](int l) {
+    const bool of_a = l < PA;
+    const int i = of_a ? l : l - PA;
+    const bool second = TWO_SRC && ld_ku >= units;
+    const int ku = second ? ld_ku - units : ld_ku;
+    // (behind the last tile nothing is left)
+    const int left = ld_tile < my_tiles ? Kdim - ku * BK : 0;
+    const uint32_t at = ring + (uint32_t)(ld_slot * STAGE_BYTES + (of_a ? 0 : A_BYTES) + (wave + 8 * i) * 1024);
+    if (of_a) {
+      const uint16_t* src = second ? reinterpret_cast<const uint16_t*>(S0) : A;
+      buffer_to_lds(src + (size_t)ku * BK, kc * 8 < left ? pa[i] : NOWHERE, at);
+    } else {
+      const uint16_t* src = TWO_SRC ? ld_b[second ? 1 : 0] : ld_b[DUAL ? i : 0];
+      if constexpr (KN) {
+        const int k = KROWS * (DUAL ? wave : wave + 8 * i) + lane / KCHUNKS;
+        buffer_to_lds(src + (size_t)ku * BK * N, k < left ? pb[i] : NOWHERE, at);
+      } else {
+        buffer_to_lds(src + (size_t)ku * BK, kc * 8 < left ? pb[i] : NOWHERE, at);
+      }
+    }
+  };
+  auto loaded = [&]() {
+    ld_slot = ld_slot + 1 == STAGES ? 0 : ld_slot + 1;
+    if (++ld_ku == nu) {
+      ld_ku = 0;
+      if (++ld_tile < my_tiles) setup_tile();
+    }
+  };
+
+  // ---- fragments (bytes from the start of a stage)
+  const int xrow = (wm * 32 + lr) * 128, xkey = (lr >> 1) & 7;
+  int wb[NF];
+#pragma unroll
+  for (int fn = 0; fn < NF; ++fn) {
+    if constexpr (KN) {
+      const int s = lane & 15, k = lk * 8 + (s >> 2);
+      const int col = wn * COLS + (DUAL ? 0 : fn * 32) + ((lane >> 4) & 1) * 16 + (s & 3) * 4;
+      wb[fn] = A_BYTES + (DUAL ? fn * (B_BYTES / 2) : 0) + k * BROW + (((col >> 3) ^ k_key(k)) * 16) + (col & 7) * 2;
+    } else {
+      wb[fn] = A_BYTES + (wn * COLS + (DUAL ? fn * BN : fn * 32) + lr) * 128;
+    }
+  }
+  struct Frags {
+    bf16x8 x, w[NF];
+  };
+  auto read = [&](Frags& f, int at_slot, int ks) {
+    const uint8_t* st = smem_raw + at_slot * STAGE_BYTES;
+    const int xo = ((2 * ks + lk) ^ xkey) * 16;
+    f.x = lds_read_frag(reinterpret_cast<const uint16_t*>(st + xrow + xo));
+#pragma unroll
+    for (int fn = 0; fn < NF; ++fn) {
+      if constexpr (KN)
+        f.w[fn] = lds_read_frag_tr(reinterpret_cast<const uint16_t*>(st + wb[fn] + ks * 16 * BROW),
+                                   reinterpret_cast<const uint16_t*>(st + wb[fn] + ks * 16 * BROW + 4 * BROW));
+      else
+        f.w[fn] = lds_read_frag(reinterpret_cast<const uint16_t*>(st + wb[fn] + xo));
+    }
+  };
+  f32x16 acc[NF];
+  auto multiply = [&](const Frags& f) {
+#pragma unroll
+    for (int fn = 0; fn < NF; ++fn)
+      acc[fn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[fn], f.x, acc[fn], 0, 0, 0);
+  };
+
+  // ---- epilogue: through the wave's own piece of LDS, so that a store instruction writes whole pieces of rows.
+  // 16 rows at a time of COLS columns, 144 bytes apart.  Every store is issued (what does
+  // not exist with an offset past the buffer's end): the stages' waits count them.
+  auto store_rows = [&](uint16_t* out, const Tile& t, auto value) {
+    constexpr int LPR = COLS / 8, ROWS = 64 / LPR;  // lanes per row, rows per store
+    uint8_t* buf = smem_raw + RING_BYTES + wave * 16 * LDE;
+    const int r_lane = lane / LPR, n = wn * COLS + (lane % LPR) * 8;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        out + (size_t)t.row0 * ldc + t.n0, 0, NOWHERE, 0x00020000);
+    u32x2 o[COLS / 32][4];
+#pragma unroll
+    for (int fn = 0; fn < COLS / 32; ++fn)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = value(fn, 4 * q + j);
+        o[fn][q] = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (lr >> 4 == h) {
+#pragma unroll
+        for (int fn = 0; fn < COLS / 32; ++fn)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<u32x2*>(buf + (lr & 15) * LDE + (fn * 32 + 8 * q + 4 * lk) * 2) = o[fn][q];
+      }
+      // (the wave's LDS traffic runs in order: only the compiler has to keep it)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int p = 0; p < 16 / ROWS; ++p) {
+        const int row = p * ROWS + r_lane, m = wm * 32 + h * 16 + row;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(buf + row * LDE + (lane % LPR) * 16);
+        uint32_t at = ((m < BM) & (t.row0 + m < t.row_end) & (t.n0 + n < N)) ? (uint32_t)(m * ldc + n) * 2u : NOWHERE;
+        asm volatile("" : "+v"(at));  // (chosen before the store, not by a branch around it)
+        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, at, 0, 0);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+  };
+
+  setup_tile();
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s) {
+#pragma unroll
+    for (int l = 0; l < LOADS; ++l) load(l);
+    loaded();
+  }
+  // How many of the stages to wait for were asked for in front of the last tile's stores: what was issued
+  // behind them need not have completed, the stores neither (loads and stores complete in order of issue).
+  int before_stores = 0, at_slot = 0;
+  for (int j = 0; j < my_tiles; ++j) {
+    const Tile t = locate(j);
+    const bool active = wm * 32 < BM && t.row0 + wm * 32 < t.row_end;
+#pragma unroll
+    for (int fn = 0; fn < NF; ++fn)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[fn][i] = 0.f;
+    for (int ku = 0; ku < nu; ++ku) {
+      // this wave's part of the stage, the oldest on its way, has to be there
+      if (before_stores > 0) {
+        --before_stores;
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2) * LOADS + TILE_STORES) : "memory");
+      } else {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2) * LOADS) : "memory");
+      }
+      lds_barrier();  // and the stage before has been read by everyone: its slot takes the next one to load
+      // (a load takes a wave its turn among the eight: they go out between the products)
+      if (active) {
+        Frags f[2];
+        read(f[0], at_slot, 0);
+        read(f[1], at_slot, 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ks = 0; ks < BK / 16; ++ks) {
+          if (ks < LOADS) load(ks);
+          __builtin_amdgcn_sched_barrier(0);
+          multiply(f[ks & 1]);
+          if (ks + 2 < BK / 16) read(f[ks & 1], at_slot, ks + 2);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+#pragma unroll
+        for (int l = 0; l < LOADS; ++l) load(l);
+      }
+      loaded();
+      at_slot = at_slot + 1 == STAGES ? 0 : at_slot + 1;
+    }
+    before_stores = STAGES - 1;
+    if constexpr (KEEP_GU) {
+      store_rows(reinterpret_cast<uint16_t*>(const_cast<float*>(S0)), t, [&](int, int i) { return acc[0][i]; });
+      store_rows(reinterpret_cast<uint16_t*>(const_cast<float*>(S1)), t, [&](int, int i) { return acc[1][i]; });
+    }
+    store_rows(C, t, [&](int fn, int i) { return DUAL ? silu_f32(acc[0][i]) * acc[1][i] : acc[fn][i]; });
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may arrive in LDS after the block
+}
+
+}  // namespace fs2moe

@@ -629,6 +629,84 @@ def test_grouped_swiglu_with_a_k_tail(gpu_device, d, f):
         assert ex == 3 or torch.equal(ye_nan[sl], ye[sl]), f"expert {ex} next to NaN weights"
 
 
+# The bf16 products choose their tile by how many of them a launch has (256 CUs): 64 x 64, 64 x 128, 128 x 128 and
+# the throughput kernel's 256 x 256, in this order; rows on both sides of a tile's 64 and 128, N off its channels.
+TILE_CASES = [
+    ([1, 63, 64, 65, 0, 130], 200),
+    ([128, 0, 129, 127, 200, 120], 1352),
+    ([1290, 0, 129, 1581], 712),
+    ([1290, 0, 257, 1581], 2056),
+]
+
+
+def _tile_case(counts, gen, dev):
+    counts = torch.tensor(counts, dtype=torch.int32)
+    blocks = (counts + 15) // 16 * 16
+    offsets = torch.zeros(len(counts) + 1, dtype=torch.int32)
+    offsets[1:] = blocks.cumsum(0)
+    rows = int(offsets[-1]) + 15 * len(counts)
+    return counts.to(dev), offsets.to(dev), rows, torch.randint(0, 500, (rows,), generator=gen, dtype=torch.int32).to(dev)
+
+
+def _assert_products(got, pairs, what):
+    """Every element within its rounding to bf16 and the rounding of a f32 sum of its products."""
+    ref = sum(a.double() @ b.double() for a, b in pairs)
+    size = sum(a.double().abs() @ b.double().abs() for a, b in pairs)
+    terms = sum(a.shape[1] for a, _ in pairs)
+    bound = 2.0**-8 * ref.abs() + (terms + 2) * 2.0**-24 * size + 1e-30
+    worst = float(((got.double() - ref).abs() / bound).max())
+    assert worst <= 1.0, f"{what}: {worst:.3f} of the bound"
+
+
+@pytest.mark.parametrize("counts,n", TILE_CASES)
+@pytest.mark.parametrize("k", [8, 64, 200, 328])
+@pytest.mark.parametrize("layout", [_abi.W_IN_OUT, _abi.W_OUT_IN])
+def test_products_on_every_tile_size(gpu_device, counts, n, k, layout):
+    _say("tile sizes", counts, n, k, layout)
+    g = torch.Generator().manual_seed(n + k)
+    c, off, rows, row_map = _tile_case(counts, g, gpu_device)
+    e = len(counts)
+    x = torch.randn(500, k, generator=g).to(torch.bfloat16).to(gpu_device)
+    w = torch.randn(e, k, n, generator=g).to(torch.bfloat16).to(gpu_device)
+    b = (w if layout == _abi.W_IN_OUT else w.transpose(1, 2).contiguous()).reshape(-1, n if layout == _abi.W_IN_OUT else k)
+    mapped = _abi.grouped_gemm(x, b, layout, c, off, e, row_map=row_map, rows=rows)
+    copied = _abi.grouped_gemm(x[row_map.long()].contiguous(), b, layout, c, off, e)
+    for i in range(e):
+        sl = slice(int(off[i]), int(off[i]) + counts[i])
+        if counts[i]:
+            _assert_products(mapped[sl], [(x[row_map[sl].long()], w[i])], f"expert {i}")
+            assert torch.equal(mapped[sl], copied[sl]), f"expert {i}: rows through the map"
+    # all rows of one matrix
+    _assert_products(_abi.grouped_gemm(x, b[: (k if layout == _abi.W_IN_OUT else n)], layout), [(x, w[0])], "dense")
+
+
+@pytest.mark.parametrize("counts,n", TILE_CASES)
+def test_pair_and_two_sources_on_every_tile_size(gpu_device, counts, n):
+    """The gate/up product with both products kept, and the product of two sources; the pair without keeping, bit for
+    bit the same."""
+    _say("tile sizes, pair", counts, n)
+    g = torch.Generator().manual_seed(n)
+    c, off, rows, row_map = _tile_case(counts, g, gpu_device)
+    e, k, n = len(counts), 192, (n + 63) // 64 * 64
+    make = lambda *shape: (0.1 * torch.randn(*shape, generator=g)).to(torch.bfloat16).to(gpu_device)
+    x, wg, wu, wd = make(500, k), make(e * k, n), make(e * k, n), make(e * n, k)
+    ye, h, gk, uk = _abi.grouped_swiglu_keep(x, c, off, wg, wu, wd, e, row_map=row_map)
+    ye2, h2 = _abi.grouped_swiglu(x, c, off, wg, wu, wd, e, row_map=row_map)
+    summed = _abi.grouped_gemm_sum(gk, wg, uk, wu, c, off, e)  # (gradients of the same shapes, as it happens)
+    for i in range(e):
+        sl = slice(int(off[i]), int(off[i]) + counts[i])
+        if not counts[i]:
+            continue
+        xr, ks, ns = x[row_map[sl].long()], slice(i * k, (i + 1) * k), slice(i * n, (i + 1) * n)
+        _assert_products(gk[sl], [(xr, wg[ks])], f"g of expert {i}")
+        _assert_products(uk[sl], [(xr, wu[ks])], f"u of expert {i}")
+        h_ref = torch.nn.functional.silu(xr.double() @ wg[ks].double()) * (xr.double() @ wu[ks].double())
+        assert_output_close(h[sl], h_ref.cpu(), "bf16", f"h of expert {i}")
+        _assert_products(ye[sl], [(h[sl], wd[ns])], f"ye of expert {i}")
+        _assert_products(summed[sl], [(gk[sl], wg[ks].t()), (uk[sl], wu[ks].t())], f"sum of expert {i}")
+        assert torch.equal(ye[sl], ye2[sl]) and torch.equal(h[sl], h2[sl]), f"expert {i} without keeping"
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
 @pytest.mark.parametrize(
     "t,d,f",
