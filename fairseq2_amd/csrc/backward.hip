@@ -1035,12 +1035,12 @@ static int wgrad_segments(int64_t rows, int M, int N) {
 
 // A gradient is written once and not read here, and as ordinary stores its lines push the operands' rows,
 // which other tiles read again, out of L2: 128 experts of 256 rows, 2048 x 768, 207 us with ordinary and
-// 186 us with non-temporal stores (bf16).  Rows that do not begin on a 128-byte line leave parts of lines,
-// which are better merged in the caches unless the gradient is larger than these (16 experts, 1024 x 1368:
-// 43 against 50 us).
-static int nt_stores(int64_t slots, int64_t M, int64_t N) {
-  return N % 64 == 0 || slots * M * N * 2 > (256ll << 20);
-}
+// 186 us with non-temporal stores (bf16); 8 of 71 rows, 4288 x 5504, 108 and 97.  But rows that do not begin on a
+// 128-byte line leave every piece of 128 bytes in two lines, whose halves L2 puts together unless they are marked
+// non-temporal: 8 of 71, 4288 x 5496, 131 us with ordinary and 221 with non-temporal stores; 8 of 40, 4096 x 14344,
+// 301 and 596; 64 of 220, 2880 x 808, 149 and 173; 128 of 256, 2048 x 776, 254 and 263; 8 of 2048, 4096 x 14344, 1785
+// and 1844; 16 of 375, 1024 x 1368, 43 and 50.
+static int nt_stores(int64_t N) { return N % 64 == 0; }
 
 // Rows of each of (at most) *segments segments, a multiple of 16; *segments becomes how many that makes,
 // none of them empty.
@@ -1136,7 +1136,7 @@ extern "C" int fs2moe_grouped_wgrad(const void* a, const int32_t* a_row_map, con
     jobs.n = 1;
     jobs.job[0] = {static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b),
                    static_cast<uint16_t*>(dw), partial, M, N, m_tiles, m_tiles * n_tiles,
-                   counts != nullptr, slots, seg_rows, (int)max_rows, nt_stores(slots, M, N), mapped, 0};
+                   counts != nullptr, slots, seg_rows, (int)max_rows, nt_stores(N), mapped, 0};
     // (without rows nothing is read, and the map may be empty)
     if (int rc = launch_wgrad(jobs, max_rows > 0 ? a_row_map : nullptr, counts, offsets, E, st)) return rc;
   } else {
@@ -1222,7 +1222,7 @@ int fs2moe::wgrad_all(const WgradRequest* r, int n, const int32_t* row_map, cons
     const int seg = segment_rows(rows, &segments), slots = q.grouped ? E : segments;
     jobs.job[i] = {static_cast<const uint16_t*>(q.a), static_cast<const uint16_t*>(q.b),
                    static_cast<uint16_t*>(q.dw), !q.grouped && slots > 1 ? part : nullptr, q.M, q.N, mt, mt * nt,
-                   q.grouped ? 1 : 0, slots, q.grouped ? 0 : seg, (int)rows, nt_stores(slots, q.M, q.N),
+                   q.grouped ? 1 : 0, slots, q.grouped ? 0 : seg, (int)rows, nt_stores(q.N),
                    q.map_a, q.map_b};
     if (!q.grouped && slots > 1) part += (int64_t)slots * q.M * q.N;
   }
