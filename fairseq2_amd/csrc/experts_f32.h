@@ -29,7 +29,14 @@
 
 namespace fs2moe {
 namespace f32t {
-constexpr int BK = 32, THREADS = 256;
+constexpr int BK = 32;
+// Threads of a block: four waves, or two groups of four that each take half of every chunk's k, whose sums are added
+// at the end.  Two waves to a SIMD cover each other's reads and barriers, and where a tile has up to 32 rows every SIMD
+// has one that multiplies: 16 experts of 18 rows, K 1792, N 1024, 38 -> 30 us; 1024 rows, K 4096, N 1024 (a tile a CU)
+// 80 -> 74; 60 experts of 80, the pair of D 768, F 2000, 575 -> 547.  Not for two products at once: what the sums leave
+// of registers and LDS lets two such blocks share a CU instead of three smaller ones (60 experts of 17 rows, K 576, N
+// 1760, 66 -> 80 us).
+constexpr int threads(int groups) { return 256 * groups; }
 
 // Tiles of 64 x 64 while 128 x 128 ones would give a CU fewer than two blocks (big_tiles of them in the
 // launch), or where the groups have so few rows on average that half of a 128-row tile would be padding.
@@ -42,7 +49,7 @@ static __device__ __attribute__((aligned(16))) uint32_t zero16[4] = {0u, 0u, 0u,
 
 // A chunk (32 k) of one operand: ROWS rows (or columns) x 32 k.  `base` points at the operand's first row
 // (column) of the tile in k 0; ld is the stride in floats of a row (k-contiguous) or of a k (k-major).
-template <int ROWS, bool KMAJOR>
+template <int ROWS, bool KMAJOR, int THREADS>
 struct Operand {
   static constexpr int BYTES = ROWS * BK * 4;
   static constexpr int PER = ROWS * BK / 4 / THREADS;  // 16-byte chunks per thread
@@ -120,15 +127,22 @@ struct Operand {
 // acc[b][fn][fm] is the transposed 32 x 32 tile (lane: row lr, channels 8 q + 4 lk + 0..3 in 4 q ..).
 // With two sources the second pair follows the first in the same accumulators.
 // A_MAPPED: a_map gives the rows of the k-major A.
-template <int NB, int FM, int FN, bool A_KMAJOR, bool B_KMAJOR, bool A_MAPPED = false>
+template <int NB, int FM, int FN, bool A_KMAJOR, bool B_KMAJOR, bool A_MAPPED = false, int GROUPS = 1>
 struct Walk {
-  static constexpr int BM = 64 * FM, BN = 64 * FN;
-  using OpA = Operand<BM, A_KMAJOR>;
-  using OpB = Operand<BN, B_KMAJOR>;
+  static constexpr int BM = 64 * FM, BN = 64 * FN, THREADS = threads(GROUPS);
+  using OpA = Operand<BM, A_KMAJOR, THREADS>;
+  using OpB = Operand<BN, B_KMAJOR, THREADS>;
   static constexpr int BUF_BYTES = OpA::BYTES + NB * OpB::BYTES;
   static constexpr int SMEM_BYTES = 2 * BUF_BYTES;
   static constexpr int PIECES = OpA::PER + NB * OpB::PER;  // 16-byte pieces of a chunk per thread
-  static constexpr int PRODUCTS = BK / 2 * NB * FM * FN;    // MFMAs of a chunk per wave
+  static constexpr int STEPS = BK / 8 / GROUPS;              // steps of 8 k of a chunk per wave
+  static constexpr int PRODUCTS = 4 * STEPS * NB * FM * FN;  // MFMAs of a chunk per wave
+
+  // The wave's rows and channels of the tile, and which share of a chunk's k it takes.  (Waves w and w + 4 share a
+  // SIMD: with a tile of up to 32 rows every SIMD has a wave that multiplies.)
+  static __device__ __forceinline__ int wave_m(int wave) { return GROUPS == 2 ? wave >> 2 : wave & 1; }
+  static __device__ __forceinline__ int wave_n(int wave) { return GROUPS == 2 ? wave & 1 : wave >> 1; }
+  static __device__ __forceinline__ int wave_group(int wave) { return GROUPS == 2 ? (wave >> 1) & 1 : 0; }
 
   struct Source {
     const float* a;
@@ -141,7 +155,7 @@ struct Walk {
                                              const int32_t* a_map = nullptr) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave & 1, wn = wave >> 1;
+    const int wm = wave_m(wave), wn = wave_n(wave), s0k = wave_group(wave) * STEPS;
     OpA opa;
     OpB opb;
     opa.setup(tid, lda, m_rows);
@@ -199,22 +213,29 @@ struct Walk {
           wf[set][b][fn] = OpB::frag(at + OpA::BYTES + b * OpB::BYTES, lane, (wn * FN + fn) * 32, s);
     };
     // Chunk st is multiplied from buffer st & 1, while chunk st + 1 is stored from register set
-    // (st + 1) & 1 into the other buffer (read last in chunk st - 1, whose barrier has passed) and the
-    // loads of chunk st + 3 go into the registers that frees.  A wave issues in order, and a 16-byte store
-    // takes its turn for about 80 clocks and a load for about 40: they go out one at a time, each behind
-    // a product that takes the matrix pipe 64 clocks, and each step's fragments are read a step ahead.
+    // (st + 1) & 1 into the other buffer (whose last reads, of chunk st - 1, are behind that chunk's barrier)
+    // and the loads of chunk st + 3 go into the registers that frees.  A wave issues in order, and a 16-byte
+    // store takes its turn for about 80 clocks and a load for about 40: they go out one at a time, each behind
+    // a product that takes the matrix pipe 64 clocks, and each step's fragments are read a step ahead.  The
+    // chunk's barrier stands in front of its last step, whose fragments have been read: its products cover the
+    // reading of the next chunk's first ones.
     // (The fences keep that order: left alone, the compiler moves the reads to their first use.  A wave
     // without rows walks a loop of its own: a condition around the products would make every one of them
     // wait for all LDS traffic in flight.)
     auto chunk = [&](auto multiply, auto& a, auto& b, int buf, int st) {
       const Chunk next = chunk_at(st + 3);
       if constexpr (decltype(multiply)::value) {
-        constexpr int EVERY = PRODUCTS / (2 * PIECES);
-        static_assert(EVERY >= 1 && EVERY * 2 * PIECES <= PRODUCTS, "a product per store and load");
-        read(0, buf, 0);
+        constexpr int BEHIND = PRODUCTS / STEPS * (STEPS - 1);  // products in front of the barrier
+        constexpr int EVERY = BEHIND / (2 * PIECES);
+        static_assert(EVERY >= 1 && EVERY * 2 * PIECES <= BEHIND, "a product per store and load");
 #pragma unroll
-        for (int s = 0; s < BK / 8; ++s) {
-          if (s + 1 < BK / 8) read((s + 1) & 1, buf, s + 1);
+        for (int s = 0; s < STEPS; ++s) {
+          if (s + 1 < STEPS) {
+            read((s + 1) & 1, buf, s0k + s + 1);
+          } else {
+            lds_barrier();
+            read(0, buf ^ 1, s0k);
+          }
 #pragma unroll
           for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -227,7 +248,7 @@ struct Walk {
                   acc[m][fn][fm] = __builtin_amdgcn_mfma_f32_32x32x2f32(
                       wf[s & 1][m][fn][j], xf[s & 1][fm][j], acc[m][fn][fm], 0, 0, 0);
                   const int done = (((s * 4 + j) * NB + m) * FN + fn) * FM + fm;
-                  if (done % EVERY == 0) {
+                  if (done < BEHIND && done % EVERY == 0) {
                     const int o = done / EVERY;
                     if (o < PIECES)
                       store(a, b, buf ^ 1, o);
@@ -235,14 +256,15 @@ struct Walk {
                       load(a, b, next, o - PIECES);
                   }
                 }
+          __builtin_amdgcn_sched_barrier(0);
         }
       } else {
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) store(a, b, buf ^ 1, p);
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) load(a, b, next, p);
+        lds_barrier();
       }
-      lds_barrier();
     };
     auto load_all = [&](auto& a, auto& b, int step) {
       const Chunk c = chunk_at(step);
@@ -257,6 +279,7 @@ struct Walk {
     load_all(ra[0], rb[0], 2);
     lds_barrier();
     auto walk = [&](auto multiply) {
+      if constexpr (decltype(multiply)::value) read(0, 0, s0k);
       int st = 0;
       for (; st + 1 < steps; st += 2) {
         chunk(multiply, ra[1], rb[1], 0, st);
@@ -268,29 +291,57 @@ struct Walk {
       walk(std::integral_constant<bool, true>{});
     else
       walk(std::integral_constant<bool, false>{});
+    if constexpr (GROUPS == 2) {
+      // the second group's sums onto the first's, through the chunks' LDS (the last barrier is behind every read)
+      constexpr int REGS = NB * FN * FM * 16;
+      static_assert(4 * REGS * 64 * 4 <= SMEM_BYTES, "the sums of four waves fit the chunks' buffers");
+      float* at = reinterpret_cast<float*>(smem) + (wm * 2 + wn) * (REGS * 64) + lane;
+      auto exchange = [&](auto store) {
+#pragma unroll
+        for (int m = 0; m < NB; ++m)
+#pragma unroll
+          for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+            for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+              for (int i = 0; i < 16; ++i) {
+                float& v = at[(((m * FN + fn) * FM + fm) * 16 + i) * 64];
+                if constexpr (decltype(store)::value)
+                  v = acc[m][fn][fm][i];
+                else
+                  acc[m][fn][fm][i] += v;
+              }
+      };
+      const bool second = s0k != 0;
+      if (second && active) exchange(std::integral_constant<bool, true>{});
+      lds_barrier();
+      if (!second && active) exchange(std::integral_constant<bool, false>{});
+    }
   }
+  // whether the wave holds the tile's sums after run
+  static __device__ __forceinline__ bool holds_sums(int wave) { return wave_group(wave) == 0; }
 };
 }  // namespace f32t
 
 // C = A B_e (+ A2 B2_e), or with DUAL C = SiLU(A B0_e) * (A B1_e), the two products left in g_keep and
 // u_keep where those are given.  A block per tile; BLAYOUT as for the bf16 kernels.
-template <bool DUAL, int FM, int FN, int BLAYOUT>
-__global__ __launch_bounds__(f32t::THREADS, 2) void glu_gemm_f32_kernel(
+template <bool DUAL, int FM, int FN, int BLAYOUT, int GROUPS>
+__global__ __launch_bounds__(f32t::threads(GROUPS), 2 * GROUPS) void glu_gemm_f32_kernel(
     const float* __restrict__ A, const float* __restrict__ B0, const float* __restrict__ B1,
     const float* __restrict__ A2, float* __restrict__ C, float* __restrict__ g_keep,
     float* __restrict__ u_keep, int K, int N, Groups g, int n_tiles) {
   constexpr int NB = DUAL ? 2 : 1;
   constexpr bool KN = BLAYOUT == FS2MOE_W_IN_OUT;
-  using W = f32t::Walk<NB, FM, FN, false, KN>;
+  using W = f32t::Walk<NB, FM, FN, false, KN, false, GROUPS>;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[W::SMEM_BYTES];
   int e, row0, row_end, nt;
-  if (!locate_tile_by_xcd<W::BM>(g, n_tiles, e, row0, row_end, nt)) return;
+  if (!locate_tile_by_xcd<W::BM, W::THREADS>(g, n_tiles, e, row0, row_end, nt)) return;
   e = __builtin_amdgcn_readfirstlane(e);
   row0 = __builtin_amdgcn_readfirstlane(row0);
   row_end = __builtin_amdgcn_readfirstlane(row_end);
   const int n0 = nt * W::BN;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave & 1, wn = wave >> 1, lr = lane & 31, lk = lane >> 5;
+  const int wm = W::wave_m(wave), wn = W::wave_n(wave), lr = lane & 31, lk = lane >> 5;
 
   f32x16 acc[NB][FN][FM];
 #pragma unroll
@@ -316,6 +367,7 @@ __global__ __launch_bounds__(f32t::THREADS, 2) void glu_gemm_f32_kernel(
   const int m_wave = row0 + wm * 32 * FM;
   W::run(acc, smem, s0, s1, !DUAL && A2 != nullptr ? 2 : 1, K, KN ? N : K, K, row_end - row0, N - n0,
          m_wave < row_end);
+  if (!W::holds_sums(wave)) return;
 
 #pragma unroll
   for (int fm = 0; fm < FM; ++fm) {
@@ -351,7 +403,7 @@ __global__ __launch_bounds__(f32t::THREADS, 2) void glu_gemm_f32_kernel(
 // group (slots: segments, whose sums go to `partial` where there are several).
 // MAPPED: A's rows are read through a_map.
 template <int F, bool MAPPED>
-__global__ __launch_bounds__(f32t::THREADS, 2) void grouped_wgrad_f32_kernel(
+__global__ __launch_bounds__(f32t::threads(1), 2) void grouped_wgrad_f32_kernel(
     const float* __restrict__ A, const int32_t* __restrict__ a_map, const float* __restrict__ B,
     float* __restrict__ C, int M, int N, Groups g, int m_tiles, int n_tiles, int seg_rows,
     float* __restrict__ partial) {
@@ -370,7 +422,7 @@ __global__ __launch_bounds__(f32t::THREADS, 2) void grouped_wgrad_f32_kernel(
   }
   const int m0 = mt * W::BM, n0 = nt * W::BN;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave & 1, wn = wave >> 1, lr = lane & 31, lk = lane >> 5;
+  const int wm = W::wave_m(wave), wn = W::wave_n(wave), lr = lane & 31, lk = lane >> 5;
   f32x16 acc[1][F][F];
 #pragma unroll
   for (int fn = 0; fn < F; ++fn)

@@ -388,9 +388,9 @@ __global__ __launch_bounds__(half_tiles::THREADS, 2) void glu_gemm_bf16_half_ker
     before_stores = STAGES - 1;
     if constexpr (KEEP_GU) {
       store_rows(reinterpret_cast<uint16_t*>(const_cast<float*>(S0)), t, [&](int, int i) { return acc[0][i]; });
-      store_rows(reinterpret_cast<uint16_t*>(const_cast<float*>(S1)), t, [&](int, int i) { return acc[1][i]; });
+      store_rows(reinterpret_cast<uint16_t*>(const_cast<float*>(S1)), t, [&](int, int i) { return acc[NF - 1][i]; });
     }
-    store_rows(C, t, [&](int fn, int i) { return DUAL ? silu_f32(acc[0][i]) * acc[1][i] : acc[fn][i]; });
+    store_rows(C, t, [&](int fn, int i) { return DUAL ? silu_f32(acc[0][i]) * acc[NF - 1][i] : acc[fn][i]; });
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may arrive in LDS after the block
 }

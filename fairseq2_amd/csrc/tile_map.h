@@ -60,9 +60,9 @@ __device__ __forceinline__ bool locate_tile(const Groups& g, int mt, int& e, int
 
 // The tile of block blockIdx.x when the grid's tiles (m-tiles of BM rows x n_tiles, channel block minor)
 // are cut into eight runs of neighbours, one per XCD (block b runs on XCD b % 8, each with its own L2):
-// the blocks an XCD holds at a time then share their rows and their expert's weights.  All 256 threads
-// of the block must call it; the grid is a multiple of 8.  false: no tile for this block.
-template <int BM>
+// the blocks an XCD holds at a time then share their rows and their expert's weights.  All THREADS
+// threads of the block must call it; the grid is a multiple of 8.  false: no tile for this block.
+template <int BM, int THREADS>
 __device__ __forceinline__ bool locate_tile_by_xcd(const Groups& g, int n_tiles, int& e, int& row0,
                                                    int& row_end, int& nt) {
   const int idx = blockIdx.x >> 3, xcd = blockIdx.x & 7;
@@ -76,15 +76,16 @@ __device__ __forceinline__ bool locate_tile_by_xcd(const Groups& g, int n_tiles,
     row_end = g.dense_rows;
     return true;
   }
-  __shared__ int s_wave[2][4], s_found[4];
+  constexpr int ROUNDS = FS2MOE_MAX_EXPERTS / THREADS, WAVES = THREADS / 64;
+  __shared__ int s_wave[2][WAVES], s_found[4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // tiles in all, then the one of this block (the experts 256 at a time, one per thread)
-  int cnt[FS2MOE_MAX_EXPERTS / 256], excl[FS2MOE_MAX_EXPERTS / 256], carried = 0;
+  // tiles in all, then the one of this block (the experts one per thread)
+  int cnt[ROUNDS], excl[ROUNDS], carried = 0;
 #pragma unroll
-  for (int r = 0; r < FS2MOE_MAX_EXPERTS / 256; ++r) {
+  for (int r = 0; r < ROUNDS; ++r) {
     cnt[r] = excl[r] = 0;
-    if (r * 256 >= g.E) continue;  // block-uniform
-    const int ex = r * 256 + tid;
+    if (r * THREADS >= g.E) continue;  // block-uniform
+    const int ex = r * THREADS + tid;
     cnt[r] = ex < g.E ? g.counts[ex] : 0;
     const int tiles = (cnt[r] + BM - 1) / BM;
     int incl = tiles;
@@ -98,17 +99,17 @@ __device__ __forceinline__ bool locate_tile_by_xcd(const Groups& g, int n_tiles,
     int base = carried;
     for (int w = 0; w < wave; ++w) base += s_wave[r & 1][w];
     excl[r] = base + incl - tiles;
-    for (int w = 0; w < 4; ++w) carried += s_wave[r & 1][w];
+    for (int w = 0; w < WAVES; ++w) carried += s_wave[r & 1][w];
   }
   const int total = carried * n_tiles, per = (total + 7) / 8, t = xcd * per + idx;
   if (idx >= per || t >= total) return false;  // block-uniform
   const int mt = t / n_tiles;
 #pragma unroll
-  for (int r = 0; r < FS2MOE_MAX_EXPERTS / 256; ++r) {
+  for (int r = 0; r < ROUNDS; ++r) {
     const int tiles = (cnt[r] + BM - 1) / BM;
     if (tiles > 0 && mt >= excl[r] && mt < excl[r] + tiles) {
-      const int off = g.offsets[r * 256 + tid];
-      s_found[0] = r * 256 + tid;
+      const int off = g.offsets[r * THREADS + tid];
+      s_found[0] = r * THREADS + tid;
       s_found[1] = off + (mt - excl[r]) * BM;
       s_found[2] = off + cnt[r];
     }
