@@ -236,8 +236,8 @@ template <int BM, int BNV, bool DUAL, int BLAYOUT, bool KEEP_GU, bool TWO_SRC>
 static int launch_half(const void* a, const int32_t* row_map, int K, const void* b0, const void* b1,
                        const void* s0, const void* s1, void* c, int N, const Groups& g, const char* what,
                        int num_blocks, hipStream_t stream) {
-  auto k = glu_gemm_bf16_half_kernel<BM, BNV, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>;
-  constexpr int bytes = half_tiles::smem_bytes(BM, BNV), bn = DUAL ? BNV / 2 : BNV;
+  auto k = glu_gemm_half_kernel<BM, BNV, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>;
+  constexpr int bytes = half_tiles::smem_bytes(BM, BNV, BLAYOUT), bn = DUAL ? BNV / 2 : BNV;
   static bool attr_set = false;  // benign race: setting the attribute is idempotent
   if (!attr_set) {
     hipError_t e =
@@ -249,9 +249,9 @@ static int launch_half(const void* a, const int32_t* row_map, int K, const void*
     attr_set = true;
   }
   hipLaunchKernelGGL(k, dim3((unsigned)num_blocks), dim3(half_tiles::THREADS), bytes, stream,
-                     static_cast<const uint16_t*>(a), row_map, K, static_cast<const uint16_t*>(b0),
-                     static_cast<const uint16_t*>(b1), static_cast<const float*>(s0), static_cast<const float*>(s1),
-                     static_cast<uint16_t*>(c), N, K, N, g, (N + bn - 1) / bn);
+                     static_cast<const uint8_t*>(a), row_map, K, static_cast<const uint8_t*>(b0),
+                     static_cast<const uint8_t*>(b1), static_cast<const float*>(s0), static_cast<const float*>(s1),
+                     static_cast<uint8_t*>(c), N, K, N, g, (N + bn - 1) / bn, HalfMx{});
   return check_launch(what);
 }
 
@@ -287,22 +287,21 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
     set_error("%s: too many tiles", what);
     return FS2MOE_ERR_UNSUPPORTED;
   }
-  if constexpr (BLAYOUT != W_FP8_TILED) {
-    // (tiles of 64 x 64 are counted in 31 bits too)
-    const bool counted = (rows_bound / 64 + groups + 1) * ((N + 63) / 64) <= 0x7fffffffll;
-    switch (counted ? half_tiles::pick(DUAL, rows_bound, groups, K, N, num_blocks) : 0) {
-      case 1:
-        if constexpr (!DUAL)
-          return launch_half<64, 64, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
-                                                                      num_blocks, stream);
-        break;
-      case 2:
-        return launch_half<64, 128, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
-                                                                     num_blocks, stream);
-      case 3:
-        return launch_half<128, 128, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
-                                                                      num_blocks, stream);
-    }
+  // (tiles of 64 x 64 are counted in 31 bits too)
+  const bool counted = (rows_bound / 64 + groups + 1) * ((N + 63) / 64) <= 0x7fffffffll;
+  constexpr bool SINGLE = !DUAL && CAN_TAIL;
+  switch (counted ? half_tiles::pick(DUAL, SINGLE, rows_bound, groups, K, N, num_blocks) : 0) {
+    case 1:
+      if constexpr (SINGLE)
+        return launch_half<64, 64, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
+                                                                    num_blocks, stream);
+      break;
+    case 2:
+      return launch_half<64, 128, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
+                                                                   num_blocks, stream);
+    case 3:
+      return launch_half<128, 128, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
+                                                                    num_blocks, stream);
   }
   hipLaunchKernelGGL(K % (2 * BK) == 0 ? whole : tail, dim3((unsigned)num_blocks), dim3(NWAVES * 64),
                      SMEM_BYTES, stream, static_cast<const uint16_t*>(a), row_map, K,

@@ -530,43 +530,4 @@ __global__ __launch_bounds__(mx::NWAVES * 64) void glu_gemm_mx_kernel(
   }
 }
 
-// x [T, D] bf16 -> e4m3 codes [T, D] and one scale byte per row and 32 features, k-group major:
-// [D / 128][T][4].  A lane owns a block of 32 features (64 bytes in, 32 bytes out); consecutive
-// lanes take consecutive blocks of a row, so four lanes fill a scale dword.
-__global__ __launch_bounds__(256) void mx_quantize_kernel(const uint16_t* __restrict__ x, int64_t T,
-                                                          int D, uint8_t* __restrict__ xq,
-                                                          uint8_t* __restrict__ xs) {
-  const int lane = threadIdx.x & 63;
-  const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int nb = D / 32;
-  const int64_t blocks = T * nb;
-  for (int64_t b = wave * 64 + lane; b < blocks; b += (int64_t)gridDim.x * 256) {
-    const uint16_t* src = x + b * 32;
-    u32x4 in[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) in[j] = *reinterpret_cast<const u32x4*>(src + 8 * j);
-    float v[32];
-    float amax = 0.f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[8 * j + 2 * i] = __uint_as_float(in[j][i] << 16);
-        v[8 * j + 2 * i + 1] = __uint_as_float(in[j][i] & 0xffff0000u);
-        amax = fmaxf(amax, fmaxf(fabsf(v[8 * j + 2 * i]), fabsf(v[8 * j + 2 * i + 1])));
-      }
-    const int X = mx::block_exponent(amax);
-    const float inv = __builtin_ldexpf(1.0f, -X);
-    u32x4 out[2];
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      out[j >> 2][j & 3] = mx::to_e4m3x4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3], inv);
-    *reinterpret_cast<u32x4*>(xq + b * 32) = out[0];
-    *reinterpret_cast<u32x4*>(xq + b * 32 + 16) = out[1];
-    const int64_t row = b / nb;
-    const int kb = (int)(b - row * nb);
-    xs[((int64_t)(kb >> 2) * T + row) * 4 + (kb & 3)] = (uint8_t)(X + 127);
-  }
-}
-
 }  // namespace fs2moe

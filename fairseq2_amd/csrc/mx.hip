@@ -1,7 +1,49 @@
 // W8A8 expert path: block-scaled e4m3 activations against e4m3 weights on the fp8 matrix pipe.
 // Host side of experts_mx.h.  No counterpart in the reference (its experts run in the parameters'
 // dtype, experts.py:102-112); an opt-in of this library.
+#include "experts_half.h"
 #include "experts_mx.h"
+
+namespace fs2moe {
+// x [T, D] bf16 -> e4m3 codes [T, D] and one scale byte per row and 32 features, k-group major:
+// [D / 128][T][4].  A lane owns a block of 32 features (64 bytes in, 32 bytes out); consecutive
+// lanes take consecutive blocks of a row, so four lanes fill a scale dword.
+__global__ __launch_bounds__(256) void mx_quantize_kernel(const uint16_t* __restrict__ x, int64_t T,
+                                                          int D, uint8_t* __restrict__ xq,
+                                                          uint8_t* __restrict__ xs) {
+  const int lane = threadIdx.x & 63;
+  const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int nb = D / 32;
+  const int64_t blocks = T * nb;
+  for (int64_t b = wave * 64 + lane; b < blocks; b += (int64_t)gridDim.x * 256) {
+    const uint16_t* src = x + b * 32;
+    u32x4 in[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) in[j] = *reinterpret_cast<const u32x4*>(src + 8 * j);
+    float v[32];
+    float amax = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[8 * j + 2 * i] = __uint_as_float(in[j][i] << 16);
+        v[8 * j + 2 * i + 1] = __uint_as_float(in[j][i] & 0xffff0000u);
+        amax = fmaxf(amax, fmaxf(fabsf(v[8 * j + 2 * i]), fabsf(v[8 * j + 2 * i + 1])));
+      }
+    const int X = mx::block_exponent(amax);
+    const float inv = __builtin_ldexpf(1.0f, -X);
+    u32x4 out[2];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      out[j >> 2][j & 3] = mx::to_e4m3x4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3], inv);
+    *reinterpret_cast<u32x4*>(xq + b * 32) = out[0];
+    *reinterpret_cast<u32x4*>(xq + b * 32 + 16) = out[1];
+    const int64_t row = b / nb;
+    const int kb = (int)(b - row * nb);
+    xs[((int64_t)(kb >> 2) * T + row) * 4 + (kb & 3)] = (uint8_t)(X + 127);
+  }
+}
+}  // namespace fs2moe
 
 using namespace fs2moe;
 
@@ -102,15 +144,65 @@ extern "C" int fs2moe_grouped_swiglu_w8a8(const void* xq, const void* xs, const 
     }
   }
   Groups g{counts, offsets, E, 0};
-  hipLaunchKernelGGL(k1, dim3((unsigned)num_blocks), dim3(NWAVES * 64), SMEM_BYTES, st,
-                     static_cast<const uint8_t*>(xq), static_cast<const uint8_t*>(xs), row_map,
-                     static_cast<const uint8_t*>(w_gate), static_cast<const uint8_t*>(w_up), s_gate,
-                     s_up, hq, static_cast<uint8_t*>(hs), F, D, F, g, nt1, (int)x_rows, (int)max_rows);
-  if (int rc = check_launch("glu_gemm_mx<gate,up>")) return rc;
+  // Few tiles: the smaller tiles of experts_half.h (the same bits).
+  auto half = [&](auto bm_c, auto dual_c, const void* a, const void* as, const int32_t* map, int K, const void* b0,
+                  const void* b1, const float* s0, const float* s1, void* c, void* cs, int N, int64_t a_rows,
+                  int64_t c_rows, const char* what) -> int {
+    constexpr int HBM = decltype(bm_c)::value, HBN = 128;
+    constexpr bool DUAL = decltype(dual_c)::value;
+    constexpr int bytes = half_tiles::smem_bytes(HBM, HBN, half_tiles::W_MX), bn = DUAL ? HBN / 2 : HBN;
+    auto k = glu_gemm_half_kernel<HBM, HBN, DUAL, half_tiles::W_MX>;
+    static bool half_attr_set = false;  // benign race: setting the attribute is idempotent
+    if (!half_attr_set) {
+      hipError_t e =
+          hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+      if (e != hipSuccess) {
+        set_error("%s: cannot reserve %d bytes of LDS: %s", what, bytes, hipGetErrorString(e));
+        return FS2MOE_ERR_LAUNCH;
+      }
+      half_attr_set = true;
+    }
+    hipLaunchKernelGGL(k, dim3((unsigned)num_blocks), dim3(half_tiles::THREADS), bytes, st,
+                       static_cast<const uint8_t*>(a), map, K, static_cast<const uint8_t*>(b0),
+                       static_cast<const uint8_t*>(b1), s0, s1, static_cast<uint8_t*>(c), N, K, N, g,
+                       (N + bn - 1) / bn,
+                       HalfMx{static_cast<const uint8_t*>(as), static_cast<uint8_t*>(cs), (int)a_rows, (int)c_rows});
+    return check_launch(what);
+  };
+  using I64 = std::integral_constant<int, 64>;
+  using I128 = std::integral_constant<int, 128>;
+  const bool counted = (max_rows / 64 + E + 1) * (((D > F ? D : F) + 63) / 64) <= 0x7fffffffll;
+  auto pick = [&](bool dual, int K, int N) {
+    return counted ? half_tiles::pick(dual, false, max_rows, E, K / 2, N, num_blocks) : 0;
+  };
+  const char* what = "glu_gemm_mx<gate,up>";
+  int rc;
+  switch (pick(true, D, F)) {
+    case 2:
+      rc = half(I64{}, std::true_type{}, xq, xs, row_map, D, w_gate, w_up, s_gate, s_up, hq, hs, F, x_rows, max_rows, what);
+      break;
+    case 3:
+      rc = half(I128{}, std::true_type{}, xq, xs, row_map, D, w_gate, w_up, s_gate, s_up, hq, hs, F, x_rows, max_rows, what);
+      break;
+    default:
+      hipLaunchKernelGGL(k1, dim3((unsigned)num_blocks), dim3(NWAVES * 64), SMEM_BYTES, st,
+                         static_cast<const uint8_t*>(xq), static_cast<const uint8_t*>(xs), row_map,
+                         static_cast<const uint8_t*>(w_gate), static_cast<const uint8_t*>(w_up), s_gate, s_up, hq,
+                         static_cast<uint8_t*>(hs), F, D, F, g, nt1, (int)x_rows, (int)max_rows);
+      rc = check_launch(what);
+  }
+  if (rc) return rc;
+  what = "glu_gemm_mx<down>";
+  switch (pick(false, F, D)) {
+    case 2:
+      return half(I64{}, std::false_type{}, hq, hs, nullptr, F, w_down, nullptr, s_down, nullptr, ye, nullptr, D, max_rows, 0, what);
+    case 3:
+      return half(I128{}, std::false_type{}, hq, hs, nullptr, F, w_down, nullptr, s_down, nullptr, ye, nullptr, D, max_rows, 0, what);
+  }
   hipLaunchKernelGGL(k2, dim3((unsigned)num_blocks), dim3(NWAVES * 64), SMEM_BYTES, st,
                      static_cast<const uint8_t*>(hq), static_cast<const uint8_t*>(hs),
                      static_cast<const int32_t*>(nullptr), static_cast<const uint8_t*>(w_down),
                      static_cast<const uint8_t*>(nullptr), s_down, static_cast<const float*>(nullptr),
                      ye, static_cast<uint8_t*>(nullptr), D, F, D, g, nt2, (int)max_rows, 0);
-  return check_launch("glu_gemm_mx<down>");
+  return check_launch(what);
 }

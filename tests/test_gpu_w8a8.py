@@ -120,6 +120,34 @@ def test_grouped_swiglu_w8a8_matches_oracle(gpu_device, rows, d, f, mapped):
         assert_output_close(ye[lo : lo + n], h_dev @ wd, "bf16", f"expert {ex}")
 
 
+# Rows on both sides of 64 and 128, in buffers whose size has them on tiles of 64 x 128, of 128 x 128 and on the
+# throughput kernel's: the same bits.
+@pytest.mark.parametrize("weights_only", [False, True])
+def test_e4m3_products_on_every_tile_size(gpu_device, weights_only):
+    rows, d, f = [1, 63, 64, 65, 0, 130, 129, 300], 256, 384
+    e = len(rows)
+    _say("e4m3 tiles", rows, d, f, weights_only)
+    wts = _fp8_experts(e, d, f, seed=5)
+    w = [_abi.pack_fp8_weights(wts[n][0].to(gpu_device), e) for n in ("gate", "up", "down")]
+    scales = tuple(wts[n][1].to(gpu_device) for n in ("gate", "up", "down"))
+    counts = torch.tensor(rows, dtype=torch.int32, device=gpu_device)
+    offsets = torch.zeros(e + 1, dtype=torch.int32, device=gpu_device)
+    offsets[1:] = torch.cumsum((counts + 15) // 16 * 16, 0)
+    lo = offsets.tolist()
+    x = torch.randn(16000, d, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(gpu_device)
+    want = None
+    for total in (lo[-1], 4000, 16000):
+        if weights_only:
+            out = _abi.grouped_swiglu(x[:total], counts, offsets, *w, e, scales=scales)
+        else:
+            xq, xs = _abi.mx_quantize(x[:total])
+            out = _abi.grouped_swiglu_w8a8(xq, xs, counts, offsets, *w, scales, e)
+            out = (*out[:2], _abi.mx_scales_row_major(out[2]))
+        got = [torch.cat([o[lo[i] : lo[i] + n] for i, n in enumerate(rows)]) for o in out]
+        want = want or got
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), total
+
+
 @pytest.mark.parametrize("mode,shared", [(W.RoutingMode("softmax", True, "output"), False),
                                          (W.RoutingMode("sigmoid", False, "input"), True)])
 def test_layer_with_quantised_activations_matches_oracle(gpu_device, mode, shared):
