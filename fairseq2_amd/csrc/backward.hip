@@ -889,7 +889,106 @@ __global__ __launch_bounds__(256) void rms_norm_backward_rows_kernel(
   }
 }
 
-// Weight gradient, first half: the rows are cut into gridDim.y slabs; a thread owns 16 bytes' worth
+// Rows and weight gradient in one pass, for rows of at most NC chunks of 64 x 16 bytes that a wave keeps in registers:
+// a block owns a run of rows (its eight waves every eighth of it), a lane adds up dy x r of its columns over its
+// wave's rows in ascending order, and at the end the eight waves' sums meet in LDS, a chunk at a time, in the waves'
+// order.  partial [gridDim.x][D] f32 (may be null).  dx is rms_norm_backward_rows_kernel's.
+//
+// A kernel of its own for the weight reads x and dy again, on as many blocks as there are slabs: with the rows' 17.4 us
+// at 640 rows of 1024 (20 blocks), 27.2 at 4096 of 2048 (128); together 4.8 and 13.4.
+template <typename T, int NC>
+__global__ __launch_bounds__(512) void rms_norm_backward_kernel(
+    const T* __restrict__ x, const T* __restrict__ w, float eps, const T* __restrict__ dy, int rows, int D,
+    T* __restrict__ dx, float* __restrict__ partial) {
+  constexpr int VEC = 16 / sizeof(T), COLS = 64 * VEC, WAVES = 8;
+  __shared__ __attribute__((aligned(16))) float s_sum[2][WAVES][COLS];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const float inv_d = 1.0f / (float)D;
+  const int per = (rows + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int64_t first = (int64_t)blockIdx.x * per;
+  const int t1 = (int)(first + per < rows ? first + per : rows);
+  auto get = [](u32x4 v, int j) {  // element j of 16 bytes
+    if constexpr (sizeof(T) == 2)
+      return j & 1 ? __uint_as_float(v[j >> 1] & 0xffff0000u) : __uint_as_float(v[j >> 1] << 16);
+    else
+      return __uint_as_float(v[j]);
+  };
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  u32x4 wv[NC];
+  float acc[NC][VEC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int d = i * COLS + lane * VEC;
+    wv[i] = w != nullptr && d < D ? *reinterpret_cast<const u32x4*>(w + d) : zero;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) acc[i][j] = 0.f;
+  }
+  for (int64_t t = first + wave; t < t1; t += WAVES) {
+    const T* xr = x + (size_t)t * D;
+    const T* gr = dy + (size_t)t * D;
+    T* outr = dx + (size_t)t * D;
+    u32x4 xv[NC], gv[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int d = i * COLS + lane * VEC;
+      xv[i] = d < D ? *reinterpret_cast<const u32x4*>(xr + d) : zero;
+      gv[i] = d < D ? *reinterpret_cast<const u32x4*>(gr + d) : zero;
+    }
+    float ss = 0.f, sg = 0.f;
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        const float x0 = get(xv[i], j);
+        float g0 = get(gv[i], j);
+        if (w != nullptr) g0 *= get(wv[i], j);
+        ss += x0 * x0;
+        sg += g0 * x0;
+      }
+    const float r = 1.0f / sqrtf(wave_sum_f32(ss) * inv_d + eps);
+    const float c = r * r * r * wave_sum_f32(sg) * inv_d;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      // (the row stays as 16 bits an element: the compiler would keep what it has unpacked, and spill)
+      asm volatile("" : "+v"(xv[i]), "+v"(gv[i]), "+v"(wv[i]));
+      float o[VEC];
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        const float x0 = get(xv[i], j), dy0 = get(gv[i], j);
+        const float g0 = w != nullptr ? dy0 * get(wv[i], j) : dy0;
+        o[j] = r * g0 - x0 * c;
+        acc[i][j] += dy0 * x0 * r;
+      }
+      u32x4 ov;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (sizeof(T) == 2) ov[j] = pack_bf16x2(o[2 * j], o[2 * j + 1]);
+        else ov[j] = __float_as_uint(o[j]);
+      }
+      const int d = i * COLS + lane * VEC;
+      if (d < D) *reinterpret_cast<u32x4*>(outr + d) = ov;
+    }
+  }
+  if (partial == nullptr) return;
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+#pragma unroll
+    for (int j = 0; j < VEC; j += 4)
+      *reinterpret_cast<f32x4*>(&s_sum[i & 1][wave][lane * VEC + j]) =
+          f32x4{acc[i][j], acc[i][j + 1], acc[i][j + 2], acc[i][j + 3]};
+    __syncthreads();  // (two buffers: chunk i + 2 is written after the barrier of chunk i + 1, behind every read of i)
+    const int d = i * COLS + tid;
+    if (tid < COLS && d < D) {
+      float sum = s_sum[i & 1][0][tid];
+#pragma unroll
+      for (int v = 1; v < WAVES; ++v) sum += s_sum[i & 1][v][tid];
+      partial[(size_t)blockIdx.x * D + d] = sum;
+    }
+  }
+}
+
+// Longer rows and rows of no whole 16 bytes: the weight gradient, first half.  The rows are cut into gridDim.y slabs; a thread owns 16 bytes' worth
 // of columns (one column when D does not divide that way) and adds up dy x r over the rows of its
 // slab in ascending order.  partial [slabs][D] f32.
 template <typename T>
@@ -1325,9 +1424,10 @@ int fs2moe::router_backward_ld(const float* logits, const int32_t* topk_idx, con
   return check_launch("router_backward");
 }
 
-// slabs of rows for the weight gradient of the normalisation: at least 32 rows each, at most 256
+// slabs of rows for the weight gradient of the normalisation: eight rows each (a row for each of a block's waves), at
+// most 256
 static int norm_weight_slabs(int64_t rows) {
-  const int64_t s = rows / 32;
+  const int64_t s = (rows + 7) / 8;
   return s < 1 ? 1 : (s > 256 ? 256 : (int)s);
 }
 
@@ -1362,7 +1462,30 @@ extern "C" int fs2moe_rms_norm_backward(const void* x, const void* weight, float
     partial = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) +
                                        ((int64_t)T * 4 + 15) / 16 * 16);
   }
-  if (T > 0) {
+  const int slabs = norm_weight_slabs(T);
+  const int vec = dtype == FS2MOE_BF16 ? 8 : 4;
+  const int chunks = D % vec == 0 ? (D / vec + 63) / 64 : 0;
+  // (rows whose 16-byte pieces and sums a lane holds in its registers: D up to 4096 in bf16, 2560 in f32.  With ten
+  // pieces in bf16 they spill: 2000 rows of 5120 40.1 us, the kernels of their own 28.1)
+  const bool one_pass = T > 0 && chunks >= 1 && chunks <= (dtype == FS2MOE_BF16 ? 8 : 10);
+  if (one_pass) {
+    auto launch = [&](auto type, auto nc) {
+      using E = decltype(type);
+      hipLaunchKernelGGL((rms_norm_backward_kernel<E, decltype(nc)::value>), dim3((unsigned)slabs), dim3(512), 0, st,
+                         static_cast<const E*>(x), static_cast<const E*>(weight), eps, static_cast<const E*>(dy), T, D,
+                         static_cast<E*>(dx), partial);
+    };
+    auto by_chunks = [&](auto type) {
+      if (chunks <= 1) launch(type, std::integral_constant<int, 1>{});
+      else if (chunks <= 2) launch(type, std::integral_constant<int, 2>{});
+      else if (chunks <= 4) launch(type, std::integral_constant<int, 4>{});
+      else if (chunks <= 6) launch(type, std::integral_constant<int, 6>{});
+      else launch(type, std::integral_constant<int, sizeof(type) == 2 ? 8 : 10>{});
+    };
+    if (dtype == FS2MOE_BF16) by_chunks(uint16_t{});
+    else by_chunks(float{});
+    if (int rc = check_launch("rms_norm_backward")) return rc;
+  } else if (T > 0) {
     int blocks = (T + 3) / 4;
     if (blocks > 4096) blocks = 4096;
     if (dtype == FS2MOE_BF16)
@@ -1378,19 +1501,19 @@ extern "C" int fs2moe_rms_norm_backward(const void* x, const void* weight, float
   }
   if (dweight == nullptr) return FS2MOE_OK;
   // (with no rows the one slab sums nothing and the gradient is zero)
-  const int slabs = norm_weight_slabs(T);
-  const int vec = dtype == FS2MOE_BF16 ? 8 : 4;
   const int owners = D % vec == 0 ? D / vec : D;  // threads per slab
   const dim3 grid((unsigned)((owners + 255) / 256), (unsigned)slabs);
   const unsigned sum_blocks = (unsigned)((D + 31) / 32);
   if (dtype == FS2MOE_BF16) {
-    hipLaunchKernelGGL(rms_norm_backward_weight_kernel<uint16_t>, grid, dim3(256), 0, st,
+    if (!one_pass)
+      hipLaunchKernelGGL(rms_norm_backward_weight_kernel<uint16_t>, grid, dim3(256), 0, st,
                        static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(dy), rstd, T, D,
                        partial);
     hipLaunchKernelGGL(rms_norm_backward_weight_sum_kernel<uint16_t>, dim3(sum_blocks), dim3(256), 0, st,
                        partial, slabs, D, static_cast<uint16_t*>(dweight));
   } else {
-    hipLaunchKernelGGL(rms_norm_backward_weight_kernel<float>, grid, dim3(256), 0, st,
+    if (!one_pass)
+      hipLaunchKernelGGL(rms_norm_backward_weight_kernel<float>, grid, dim3(256), 0, st,
                        static_cast<const float*>(x), static_cast<const float*>(dy), rstd, T, D,
                        partial);
     hipLaunchKernelGGL(rms_norm_backward_weight_sum_kernel<float>, dim3(sum_blocks), dim3(256), 0, st,

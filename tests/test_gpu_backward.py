@@ -824,6 +824,15 @@ def test_rms_norm_backward_matches_autograd_of_the_oracle(gpu_device, dtype, t, 
         assert none is None and torch.equal(dx2, dx)
 
 
+# One to ten chunks of a wave's 1 KB a row, the last one partly filled; a block with fewer rows than waves, the largest
+# number of blocks, and the longest rows of the one pass with the next that are past it.
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("t,d", [(9, 520), (17, 1000), (2049, 1288), (2, 2560), (33, 2564), (3, 2568),
+                                 (33, 4096), (33, 4104)])
+def test_rms_norm_backward_on_every_row_length(gpu_device, dtype, t, d):
+    test_rms_norm_backward_matches_autograd_of_the_oracle(gpu_device, dtype, t, d, True)
+
+
 class _RMSNorm(torch.nn.Module):
     """What the layer reads of ``fairseq2.nn.RMSNorm`` (``nn/normalization.py:166-254``)."""
 
