@@ -965,15 +965,16 @@ def check_layer_arguments(x, router, router_bias, w_gate, w_up, w_down, num_expe
     e = num_experts
     if x.dim() != 2 or not x.is_cuda or not x.is_contiguous():
         raise ValueError("x must be a contiguous (T, D) tensor on the GPU")
-    d, dtype, dev = x.shape[1], x.dtype, x.device
+    d, dtype, dev = x.shape[1], x.dtype, x.get_device()
 
     def need(name, tensor, shape, dtype):
         if tensor is None:
             raise ValueError(f"{name} is missing")
-        if tensor.shape != shape or tensor.dtype != dtype:
+        if tensor.shape != shape or tensor.dtype is not dtype:
             raise ValueError(f"{name} must be {shape} {dtype}, got {tuple(tensor.shape)} {tensor.dtype}")
-        if tensor.device != dev or not tensor.is_contiguous():
-            raise ValueError(f"{name} must be contiguous and on {dev}")
+        # (by the device's number, which a tensor elsewhere does not have: device objects take longer to compare)
+        if tensor.get_device() != dev or not tensor.is_contiguous():
+            raise ValueError(f"{name} must be contiguous and on {x.device}")
         return tensor.data_ptr()
 
     at = [need("router", router, (d, e), dtype),
@@ -1045,25 +1046,30 @@ def forward(
     router_at, bias_at, *weights_at = check_layer_arguments(
         x, router, router_bias, w_gate, w_up, w_down, num_experts, f, scales, shared)
     sizes = (t, d, num_experts, top_k, f, f_shared, tile_m)
-    need = (lib.fs2moe_forward_workspace_bytes if norm is None else lib.fs2moe_forward_norm_workspace_bytes)(
-        *sizes, act_dtype)
-    if need < 0:
-        raise ValueError("fs2moe_forward_workspace_bytes rejected the sizes")
     if workspace is None:
+        need = (lib.fs2moe_forward_workspace_bytes if norm is None else lib.fs2moe_forward_norm_workspace_bytes)(
+            *sizes, act_dtype)
+        if need < 0:
+            raise ValueError("fs2moe_forward_workspace_bytes rejected the sizes")
         workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
     normed, norm_weight, norm_eps = 0, None, 0.0
     if norm is not None:
-        _check_norm_weight(norm[0], x)
-        normed, norm_weight, norm_eps = 1, _ptr(norm[0]), float(norm[1])
-    if residual is not None and residual is not x and (
-            residual.shape != x.shape or residual.dtype != x.dtype or not residual.is_contiguous()):
-        raise ValueError("residual must be a contiguous tensor of x's shape and dtype")
-    out = torch.empty_like(x) if out_shape is None else x.new_empty(out_shape)
+        weight, norm_eps = norm
+        _check_norm_weight(weight, x)
+        normed, norm_weight = 1, _ptr(weight)
+    residual_at = None
+    if residual is x:
+        residual_at = x.data_ptr()
+    elif residual is not None:
+        if residual.shape != x.shape or residual.dtype != x.dtype or not residual.is_contiguous():
+            raise ValueError("residual must be a contiguous tensor of x's shape and dtype")
+        residual_at = _ptr(residual)
+    out = torch.empty_like(x) if out_shape is None else torch.empty(out_shape, dtype=x.dtype, device=x.device)
     if out.numel() != x.numel():
         raise ValueError("out_shape must be a shape of x's elements")
     mat, score_fn = router_operand(lib, x, router, router_t, score_fn)
     # Collected on every call, in as few steps as checking each tensor once allows: a one-token step of a
-    # layer of 128 experts takes the host 36 us with its five launches, whatever the call before it was (47 us
+    # layer of 128 experts takes the host 32 us with its five launches, whatever the call before it was (47 us
     # with a detached view of every parameter and each check in passes of its own; the GPU takes 34).
     # (fields in the order of ForwardArgs)
     a = ForwardArgs(

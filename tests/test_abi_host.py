@@ -445,6 +445,35 @@ def test_fp8_buffers_follow_the_parameters():
         ex.gate_q
 
 
+def test_operands_are_looked_up_as_attributes_are():
+    """What a call reads of a module past ``Module.__getattr__`` is what the attributes give: typed codes after
+    they have been replaced, and a norm's members whether they are parameters, buffers, properties or absent."""
+    ex = M.GroupedExpertNetwork(2, 64, 64).bfloat16()
+    ex.quantize_fp8_()
+    for _ in range(2):
+        for _ in range(2):
+            codes, scales = ex._fp8_operands()
+            want = [getattr(ex, n) for n in M.GroupedExpertNetwork._FP8_NAMES]
+            assert all(a is b for a, b in zip((*codes, *scales), want))
+        ex._buffers["_inner_q_bits"] = ex._buffers["_inner_q_bits"].clone()
+
+    class Norm(torch.nn.Module):
+        scale = property(lambda self: 3)
+
+        def __init__(self):
+            super().__init__()
+            self.weight, self.bias, self.plain = torch.nn.Parameter(torch.ones(2)), None, 5
+            self.register_buffer("held", torch.ones(1))
+
+    class Computed(Norm):
+        def __getattr__(self, name):
+            return 7 if name == "other" else super().__getattr__(name)
+
+    for norm in (Norm(), Computed(), torch.nn.RMSNorm(4), torch.nn.LayerNorm(4), object()):
+        for name in ("weight", "bias", "scale", "plain", "held", "other"):
+            assert M._optional(norm, name) is getattr(norm, name, None), (type(norm), name)
+
+
 def test_fp8_tile_packing_round_trip():
     g = torch.Generator().manual_seed(1)
     q = (50 * torch.randn(3 * 128, 80, generator=g)).to(torch.float8_e4m3fn)
