@@ -85,10 +85,12 @@ struct WgradJobs {
 
 // MAPPED: operands of some gradients are read through the row map (rows of the layer's input, or of its
 // output gradient, that no one has copied into expert order).  The map's entries are scalar loads, two rows
-// per wave and load, asked for before the chunk ahead is stored: vector loads would be waited for with every
-// other load of the wave, a round trip per chunk.  128 experts of about 256 rows, 2048 x 768, the three
-// gradients of a step: 594 us on copied rows, 570 through the map (fewer distinct rows to fetch).  The map
-// holds at least one entry, and one for every row of a gradient in the same launch that does not use it.
+// per wave and load, asked for a chunk ahead, right behind a barrier: vector loads would be waited for with every
+// other load of the wave, a round trip per chunk, and scalar ones in front of a barrier are waited for there, with
+// the LDS traffic, by the whole block.  128 experts of about 256 rows, 2048 x 768, one gradient: 171 us with the
+// entries asked for in front of the barrier, 163 now (150 on copied rows, whose copies cost more than that); training
+// steps of 4444 tokens, top-8 of 128, D 1280, F 704 1212 -> 1175 us, of 3771, top-8 of 64, D 1152, F 696 901 -> 879.
+// The map holds at least one entry, and one for every row of a gradient in the same launch that does not use it.
 template <bool MAPPED>
 __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     const WgradJobs jobs, const int32_t* __restrict__ row_map, const int32_t* __restrict__ counts,
@@ -411,6 +413,8 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     asm volatile("" : "+s"(zero));  // (read once)
     const int kr0 = (wave - CONSUMERS) * 2;
     int ld_row = 0, ld_map_a = 0, ld_map_b = 0, place[PER_THREAD][2], entry[PER_THREAD][2];
+    uint64_t row_a = zero, row_b = zero;    // a lane's place in row 0 of the operands, and their rows' distance
+    uint32_t pitch_a = 0, pitch_b = 0;
     Deal ld_deal = deal;
     uint32_t oa[PER_THREAD], ob[PER_THREAD];
     int loaded = 0;  // chunks so far (those past the stream's end do not count)
@@ -433,6 +437,13 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
         // at whose joins the tile's parameters stop being scalars)
         uint32_t a_out = t.m0 + ch * 8 < j.M ? 0u : 0xfffffff0u, b_out = t.n0 + ch * 8 < j.N ? 0u : 0xfffffff0u;
         asm volatile("" : "+v"(a_out), "+v"(b_out));
+        if constexpr (MAPPED) {
+          row_a = a_out == 0u ? (uint64_t)ld_a + ch * 16 : zero;
+          row_b = b_out == 0u ? (uint64_t)ld_b + ch * 16 : zero;
+          pitch_a = a_out == 0u ? (uint32_t)j.M * 2u : 0u;
+          pitch_b = b_out == 0u ? (uint32_t)j.N * 2u : 0u;
+          continue;
+        }
 #pragma unroll
         for (int i = 0; i < PER_THREAD; ++i) {
           oa[i] = (uint32_t)(((kr + 8 * i) * j.M + ch * 8) * 2) | a_out;
@@ -457,24 +468,47 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
           }
       }
     };
-    auto load_chunk = [&](auto set_c) {
-      constexpr int set = decltype(set_c)::value;
-      // one more if ld_left > 0 (a truth value is added on the vector side, and takes the loop's end with it)
-      loaded += (int)((uint32_t)-ld_left >> 31);
+    // MAPPED: where the chunk's pieces lie, and the entries of the chunk after it asked for.  In front of the stores,
+    // behind the barrier that has waited for the entries with the LDS traffic before it (one counter for both, in
+    // no order): asked for in front of a barrier, they were a round trip that every wave of the block waited for.
+    // (a lane whose column lies past the operand's reads zeros whatever the row)
+    uint64_t at_a[PER_THREAD], at_b[PER_THREAD];
+    auto place_chunk = [&]() {
       if constexpr (MAPPED) {
 #pragma unroll
         for (int i = 0; i < PER_THREAD; ++i) {
-          const bool in = kr + 8 * i < ld_left;
           const uint32_t a0 = ld_map_a ? entry[i][0] : place[i][0], a1 = ld_map_a ? entry[i][1] : place[i][1];
           const uint32_t b0 = ld_map_b ? entry[i][0] : place[i][0], b1 = ld_map_b ? entry[i][1] : place[i][1];
-          const uint64_t pa = (uint64_t)ld_a + ((uint64_t)(lane < 32 ? a0 : a1) * (uint32_t)ld_lda + ch * 8) * 2;
-          const uint64_t pb = (uint64_t)ld_b + ((uint64_t)(lane < 32 ? b0 : b1) * (uint32_t)ld_ldb + ch * 8) * 2;
-          // (the address chosen, by its bits: as pointers the two sides become branches)
-          ra[set][i] = *(const GlobalVec*)((in & (oa[i] < 0xfffffff0u)) ? pa : zero);
-          rb[set][i] = *(const GlobalVec*)((in & (ob[i] < 0xfffffff0u)) ? pb : zero);
+          at_a[i] = row_a + (uint64_t)(lane < 32 ? a0 : a1) * pitch_a;
+          at_b[i] = row_b + (uint64_t)(lane < 32 ? b0 : b1) * pitch_b;
         }
+        if (ld_left < RK) {
+#pragma unroll
+          for (int i = 0; i < PER_THREAD; ++i) {
+            const bool in = kr + 8 * i < ld_left;
+            at_a[i] = in ? at_a[i] : zero;
+            at_b[i] = in ? at_b[i] : zero;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i) asm volatile("" : "+v"(at_a[i]), "+v"(at_b[i]));
+        loaded += (int)((uint32_t)-ld_left >> 31);  // (as below)
         ld_row += RK;
+        ld_left -= RK;
+        look_up();
+      }
+    };
+    auto load_chunk = [&](auto set_c) {
+      constexpr int set = decltype(set_c)::value;
+      if constexpr (MAPPED) {
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i) {
+          ra[set][i] = *(const GlobalVec*)at_a[i];
+          rb[set][i] = *(const GlobalVec*)at_b[i];
+        }
       } else {
+        // one more if ld_left > 0 (a truth value is added on the vector side, and takes the loop's end with it)
+        loaded += (int)((uint32_t)-ld_left >> 31);
         const __amdgpu_buffer_rsrc_t a_rsrc =
             __builtin_amdgcn_make_buffer_rsrc(scalar(ld_a), 0, 0xfffffff0u, 0x00020000);
         const __amdgpu_buffer_rsrc_t b_rsrc =
@@ -489,8 +523,9 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
         }
         ld_a += (size_t)RK * ld_lda;
         ld_b += (size_t)RK * ld_ldb;
+        ld_left -= RK;
+        look_up();
       }
-      ld_left -= RK;
     };
     auto store_chunk = [&](auto set_c, int buf) {
       constexpr int set = decltype(set_c)::value;
@@ -508,19 +543,19 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     using Set0 = std::integral_constant<int, 0>;
     using Set1 = std::integral_constant<int, 1>;
     look_up();
+    place_chunk();
     load_chunk(Set0{});
     if (loaded == 0) return;  // no tile with rows: nothing for the consumers to wait for
-    look_up();
+    place_chunk();
     load_chunk(Set1{});
-    look_up();
+    place_chunk();
     store_chunk(Set0{}, 0);
     load_chunk(Set0{});
-    look_up();
     lds_barrier();
     auto step = [&](int g, auto next_set) {
+      place_chunk();
       store_chunk(next_set, (g + 1) & 1);
       load_chunk(next_set);
-      look_up();
       lds_barrier();  // the loads of the next chunks stay in flight
     };
     // Always two steps, the one past an odd last chunk with zeros that no one reads, and everything that the
