@@ -311,6 +311,101 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
   return check_launch(what);
 }
 
+// Single products of few tiles over a long K: into how many parts the sum over K goes (1: it stays whole), each a
+// round of tiles of its own.  The throughput kernel's time, in ns per unit of 64 k: a full round 2000, one that has n
+// of the chip's CUs at work 800 + 1200 n / 256 (40 tiles 1.0 us, 144 1.6, 192 1.8), neither faster than the operands
+// come in (4 TB/s); the smaller tiles' 330, 450 and 650 of one round.  Against that the parts' sums on their way out
+// and in again, and a launch.  us for two sources, whole (with the smaller tiles where they are taken) and in parts:
+//   16 experts of 424 rows, K 13800, N 640    593, 367 (5)    8 of 427, K 9472, N 2112   464, 348 (3)
+//   8 of 457, K 10560, N 512                  151, 105 (8)    8 of 880, K 8768, N 1216   443, 334 (3)
+//   16 of 214, K 5568, N 1280                 180, 163 (2)    8 of 920, K 2800, N 576     89,  91 (2)
+// and where it says 1: 16 of 552, K 7040, N 1088 365, 370 (3); 60 of 240, K 1600, N 1216 159, 202 (2); 16 of 375,
+// K 1368, N 1024 52, 63 (2).  A constant number of CUs, as the scratch is sized in calls that touch no device.
+int fs2moe::split_parts(int sources, int64_t rows, int E, int K, int N) {
+  constexpr int CUS = 256, MIN_UNITS = 16;
+  constexpr int64_t MAX_BYTES = 256ll << 20;
+  if (rows <= 0) return 1;
+  const int groups = E > 0 ? E : 1;
+  const int64_t real = E > 0 && rows > 15ll * E ? rows - 15ll * E : rows;  // (as in half_tiles::pick)
+  const int64_t each = real / groups, nt = (N + dma::BNV - 1) / dma::BNV, rest = each % dma::BM;
+  const int64_t heavy = (each / dma::BM + (rest > dma::LIGHT_ROWS)) * groups * nt;
+  const int64_t light = (rest > 0 && rest <= dma::LIGHT_ROWS ? groups : 0) * nt;
+  const int64_t units = (int64_t)sources * ((K + 63) / 64);
+  const int64_t memory = sources * ((groups < real ? groups : real) * K * N + rows * K) / 2000;  // ns
+  auto whole = [&](int64_t parts) {
+    const int64_t n = parts * (10 * heavy + 6 * light) / 10, left = n % CUS;
+    const int64_t t = (units + parts - 1) / parts * (n / CUS * 2000 + (left ? 800 + 1200 * left / CUS : 0));
+    return t > memory ? t : memory;
+  };
+  const int small = half_tiles::pick(false, true, rows, E, K, N, CUS);
+  int64_t base = whole(1);
+  if (small != 0) {
+    const int64_t t = units * (small == 1 ? 330 : small == 2 ? 450 : 650);
+    base = (t > memory ? t : memory) + 4000;
+  }
+  int best = 1;
+  for (int parts = 2; parts <= 16 && units / parts >= MIN_UNITS && parts * rows * N * 4 <= MAX_BYTES; ++parts) {
+    const int64_t t = whole(parts) + parts * rows * N / 1000 + 6000;
+    // (worth 5 % by these figures, to be taken at all)
+    if (best == 1 ? t * 20 < base * 19 : t < base) {
+      best = parts;
+      base = t;
+    }
+  }
+  // (no part without a unit)
+  const int64_t per = (units + best - 1) / best;
+  return (int)((units + per - 1) / per);
+}
+
+// C [rows][N] = the sum of the parts [parts][rows][N] in order, rounded once; a lane takes 8 columns of N, a multiple
+// of 8.  (Rows between the experts hold anything, there as here.)
+static __global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict__ from, int parts, int64_t n,
+                                                        uint16_t* __restrict__ C) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
+  if (i >= n) return;
+  f32x4 lo = *reinterpret_cast<const f32x4*>(from + i), hi = *reinterpret_cast<const f32x4*>(from + i + 4);
+#pragma unroll 4
+  for (int p = 1; p < parts; ++p) {
+    lo += *reinterpret_cast<const f32x4*>(from + (size_t)p * n + i);
+    hi += *reinterpret_cast<const f32x4*>(from + (size_t)p * n + i + 4);
+  }
+  *reinterpret_cast<u32x4*>(C + i) = u32x4{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]),
+                                           pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
+}
+
+// The product in `parts` parts (at least 2), whose sums go to scratch [parts][rows][N] f32, and their sum.
+template <int BLAYOUT, bool TWO_SRC>
+static int launch_split(const void* a, int K, const void* b0, const void* b1, const void* a2, void* c, int N,
+                        const Groups& g, int parts, void* scratch, const char* what, hipStream_t stream) {
+  using namespace dma;
+  auto k = glu_gemm_bf16_dma_kernel<false, BLAYOUT, false, TWO_SRC, true, true>;
+  static bool attr_set = false;  // benign race: setting the attribute is idempotent
+  if (!attr_set) {
+    hipError_t e =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_BYTES);
+    if (e != hipSuccess) {
+      set_error("%s: cannot reserve %d bytes of LDS: %s", what, SMEM_BYTES, hipGetErrorString(e));
+      return FS2MOE_ERR_LAUNCH;
+    }
+    attr_set = true;
+  }
+  const int num_blocks = cu_count_by_xcd();
+  if (num_blocks == 0) {
+    set_error("%s: cannot query the compute-unit count", what);
+    return FS2MOE_ERR_LAUNCH;
+  }
+  hipLaunchKernelGGL(k, dim3((unsigned)num_blocks), dim3(NWAVES * 64), SMEM_BYTES, stream,
+                     static_cast<const uint16_t*>(a), static_cast<const int32_t*>(nullptr), K,
+                     static_cast<const uint16_t*>(b0), static_cast<const uint16_t*>(b1),
+                     static_cast<const float*>(a2), static_cast<const float*>(nullptr),
+                     static_cast<uint16_t*>(scratch), parts, K, N, g, (N + 255) / 256 * parts);
+  if (int rc = check_launch(what)) return rc;
+  const int64_t n = (int64_t)g.dense_rows * N;
+  hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, stream,
+                     static_cast<const float*>(scratch), parts, n, static_cast<uint16_t*>(c));
+  return check_launch("split_sum");
+}
+
 // The bf16 throughput kernel pair (gate/up, then down); BLAYOUT as the kernel takes it, scales only
 // with dma::W_FP8_TILED.  With g_keep and u_keep the gate/up kernel also stores the two products (their
 // destinations travel in the two scale arguments).
@@ -878,9 +973,16 @@ int fs2moe::swiglu_train(const void* x, const int32_t* row_map, const int32_t* c
 
 int fs2moe::gemm_sum(const void* a1, const void* b1, const void* a2, const void* b2, int32_t layout,
                      const int32_t* counts, const int32_t* offsets, int32_t E, int32_t K, int32_t N,
-                     int64_t rows, int32_t dtype, void* c, void* stream) {
+                     int64_t rows, int32_t dtype, void* c, void* split_scratch, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
   const Groups g{E > 0 ? counts : nullptr, E > 0 ? offsets : nullptr, E > 0 ? E : 1, (int)rows};
+  const int parts = dtype == FS2MOE_BF16 && split_scratch != nullptr ? split_parts(2, rows, E, K, N) : 1;
+  if (parts > 1)
+    return layout == FS2MOE_W_IN_OUT
+               ? launch_split<FS2MOE_W_IN_OUT, true>(a1, K, b1, b2, a2, c, N, g, parts, split_scratch,
+                                                     "glu_gemm_bf16_dma<two sources, parts>", st)
+               : launch_split<FS2MOE_W_OUT_IN, true>(a1, K, b1, b2, a2, c, N, g, parts, split_scratch,
+                                                     "glu_gemm_bf16_dma<two sources, parts>", st);
   // (the second activation matrix travels in the first scale argument, the second weights in B1)
   if (dtype == FS2MOE_BF16)
     return layout == FS2MOE_W_IN_OUT

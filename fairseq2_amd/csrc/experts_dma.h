@@ -137,7 +137,10 @@ struct TileOrder {
 // for every k-step's loads) and the gathered copy it needed: D 1088, F 1392, 8 experts, 8364 rows, whole
 // layer 179 -> 134 us; D 1664, F 1312, 32 experts and a shared one, 7092 rows 339 -> 275 us; the bits
 // are the same.
-template <bool DUAL, int BLAYOUT, bool KEEP_GU = false, bool TWO_SRC = false, bool KTAIL = false>
+// SPLIT (single matrix, with KTAIL): the sum over K in parts, for launches of few tiles and a long K.  The tiles are
+// those of `ldc` parts (C's rows are N wide), part-major within a row block, n_tiles counts them all; part p of C
+// [ldc][rows][N] f32 is the sum over its units, and split_sum_kernel adds the parts.
+template <bool DUAL, int BLAYOUT, bool KEEP_GU = false, bool TWO_SRC = false, bool KTAIL = false, bool SPLIT = false>
 __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
     const uint16_t* __restrict__ A, const int32_t* __restrict__ row_map, int lda,
     const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1,
@@ -148,6 +151,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
   static_assert(!KEEP_GU || (DUAL && !FP8), "the products are kept by the bf16 gate/up kernel only");
   static_assert(!KTAIL || !FP8, "e4m3 weight tiles hold whole units");
   static_assert(!TWO_SRC || (!DUAL && !FP8), "two sources: one bf16 matrix each");
+  static_assert(!SPLIT || (!DUAL && KTAIL), "parts of a sum over K: one matrix, parts past its end");
   constexpr int BN = DUAL ? 128 : 256;    // real channels per tile
   constexpr int BROW = DUAL ? 256 : 512;  // bytes per LDS row of a weight sub-tile (in x out)
   constexpr bool KN = BLAYOUT == FS2MOE_W_IN_OUT;
@@ -237,12 +241,15 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
   const int my_heavy = slot < heavy_end ? (heavy_end - slot + grid - 1) / grid : 0;
 
   // units per tile; without KTAIL the host guarantees Kdim % 64 == 0
-  const int nu = (TWO_SRC ? 2 : 1) * ((Kdim + (KTAIL ? 2 * BK - 1 : 0)) / (2 * BK));
+  const int source_units = (Kdim + (KTAIL ? 2 * BK - 1 : 0)) / (2 * BK);
+  const int all_units = (TWO_SRC ? 2 : 1) * source_units;
+  const int nu = SPLIT ? (all_units + ldc - 1) / ldc : all_units;
+  const int part_tiles = SPLIT ? n_tiles / ldc : 0;
   const int total_units = my_tiles * nu;
 
   // Wave-uniform parameters of a tile: expert, first row, end row, first channel.
   struct Tile {
-    int e, row0, row_end, n0;
+    int e, row0, row_end, n0, part;
   };
   auto locate = [&](int j) {
     const int listed = slot + j * grid;
@@ -292,7 +299,9 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
     t.e = found;
     t.row0 = __builtin_amdgcn_readfirstlane(off + first_row);
     t.row_end = __builtin_amdgcn_readfirstlane(off + last_row);
-    t.n0 = __builtin_amdgcn_readfirstlane(nt) * BN;
+    nt = __builtin_amdgcn_readfirstlane(nt);
+    t.part = SPLIT ? nt / part_tiles : 0;
+    t.n0 = (nt - (SPLIT ? t.part * part_tiles : 0)) * BN;
     return t;
   };
 
@@ -320,7 +329,8 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
     // gather) the tokens its rows are read from.  Those come out of row_map, a load that the tile's
     // own loads depend on; asked for when the tile before it is set up, they have long arrived when
     // the tile's turn comes, and its first unit goes out without a round trip to memory in front.
-    Tile pre_t = {0, 0, 0, 0};
+    Tile pre_t = {0, 0, 0, 0, 0};
+    int ld_ku0 = 0;  // SPLIT: the first unit of the tile's part
     int pre_rows[8];
     auto lookup_ahead = [&](int j) {
       pre_t = locate(j);
@@ -336,6 +346,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
     };
     auto setup_loads = [&]() {
       const Tile t = pre_t;
+      if constexpr (SPLIT) ld_ku0 = t.part * nu;
       if constexpr (FP8) {
         // wstride counts codes = bytes here; the pointers stay typed as 16-bit
         ld_bg = reinterpret_cast<const uint16_t*>(reinterpret_cast<const uint8_t*>(B0) +
@@ -432,8 +443,9 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
     // Unit ku of the tile set up last -> registers.
     auto load_unit = [&](int ku) {
       // with two sources the second half of a tile's units comes from the second pair
-      const bool second = TWO_SRC && ku >= nu / 2;
-      if constexpr (TWO_SRC) ku = second ? ku - nu / 2 : ku;
+      if constexpr (SPLIT) ku += ld_ku0;
+      const bool second = TWO_SRC && ku >= source_units;
+      if constexpr (TWO_SRC) ku = second ? ku - source_units : ku;
       const uint16_t* a_src = second ? reinterpret_cast<const uint16_t*>(S0) : A;
       const uint8_t* abase = reinterpret_cast<const uint8_t*>(a_src + (size_t)ku * (2 * BK));
       const int left = k_left(ku);
@@ -536,9 +548,9 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
         ++ld_ku;
       }
       if constexpr (!FP8) {
-        int ku = ld_ku;
-        const bool second = TWO_SRC && ku >= nu / 2;
-        if constexpr (TWO_SRC) ku = second ? ku - nu / 2 : ku;
+        int ku = ld_ku + (SPLIT ? ld_ku0 : 0);
+        const bool second = TWO_SRC && ku >= source_units;
+        if constexpr (TWO_SRC) ku = second ? ku - source_units : ku;
         const uint16_t* a_src = second ? reinterpret_cast<const uint16_t*>(S0) : A;
         const uint8_t* abase = reinterpret_cast<const uint8_t*>(a_src + (size_t)ku * (2 * BK));
         const int left = k_left(ku);
@@ -787,6 +799,37 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
     }
   };
 
+  // SPLIT: a 32 x 32 fragment at a time, as f32 through 4 KB of the same place in the ring (alternating halves of it):
+  // rows of 128 bytes, chunk c of row r in place c ^ ((r >> 1) & 7).
+  auto store_part = [&](const Tile& t, int gu) {
+    uint8_t* buf = smem_raw + (gu & 1) * UNIT_BYTES + wave * 8192;
+    int lane_l = lane;  // (as in store_tile)
+    asm volatile("" : "+v"(lane_l));
+    const int lane = lane_l, lr = lane & 31, lk = lane >> 5;
+    const uint32_t wbase = (uint32_t)(lr * 128 + ((lk ^ ((lr >> 1) & 7)) << 4));
+    const uint32_t rbase = (uint32_t)((lane >> 3) * 128 + (((lane & 7) ^ (lane >> 4)) << 4));
+    float* out = reinterpret_cast<float*>(C) + (size_t)t.part * g.dense_rows * N;
+    const int r_lane = lane >> 3;
+#pragma unroll
+    for (int fm = 0; fm < 2; ++fm)
+#pragma unroll
+      for (int fn = 0; fn < 4; ++fn) {
+        uint8_t* half = buf + (fn & 1) * 4096;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          f32x4 o = {acc[fn][fm][4 * q], acc[fn][fm][4 * q + 1], acc[fn][fm][4 * q + 2], acc[fn][fm][4 * q + 3]};
+          *reinterpret_cast<f32x4*>(half + (wbase ^ (uint32_t)(q << 5))) = o;
+        }
+        const int n = t.n0 + wn * 128 + fn * 32 + (lane & 7) * 4;
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+          const f32x4 val = *reinterpret_cast<const f32x4*>(half + (rbase ^ (uint32_t)((it & 1) << 6)) + it * 1024);
+          const int r = t.row0 + wm * 64 + fm * 32 + it * 8 + r_lane;
+          if (n < N && r < t.row_end) *reinterpret_cast<f32x4*>(out + (size_t)r * N + n) = val;
+        }
+      }
+  };
+
   // ---- main stream -----------------------------------------------------------------------------------
   TileOrder order(my_heavy, my_tiles - my_heavy, (int)(blockIdx.x & 7));
   Tile cur = locate(order.next());
@@ -805,7 +848,11 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
     if (wave_active) compute_unit(gu);
     if (++ku == nu) {
       __syncthreads();  // every consumer is done with the ring half the epilogue borrows
-      if (wave_active) store_tile(cur, gu, tiles_done & 1);
+      if constexpr (SPLIT) {
+        if (wave_active) store_part(cur, gu);
+      } else {
+        if (wave_active) store_tile(cur, gu, tiles_done & 1);
+      }
       if constexpr (KEEP_GU)
         if (wave_active) store_products(cur, gu);
       ++tiles_done;

@@ -238,7 +238,7 @@ ForwardScratch carve_forward(const Args& a, void* base) {
 
 struct BackwardScratch {
   void *xe, *dye, *dh, *dg, *du, *dxe, *dl, *router, *d_router, *dx_router, *dhs, *dgs, *dus, *dx_shared, *dxn,
-      *norm, *wgrad;
+      *norm, *part;
   float* d_w;
   int64_t norm_bytes, total;
 };
@@ -294,7 +294,16 @@ BackwardScratch carve_backward(const Args& a, void* base) {
   b.norm = a.normed ? c.take(b.norm_bytes) : nullptr;
   WgradRequest r[8];
   const int n = requests(a, Saved{}, b, r);
-  b.wgrad = c.take(wgrad_plan(r, n, a.E, R, T, a.act_dtype));
+  // (the weight gradients' partial sums, after those of the rows' gradients)
+  int64_t part = wgrad_plan(r, n, a.E, R, T, a.act_dtype);
+  auto parts = [&](int64_t rows, int E, int F) {
+    const int n = a.act_dtype == FS2MOE_BF16 ? split_parts(2, rows, E, F, a.D) : 1;
+    const int64_t bytes = n > 1 ? (int64_t)n * rows * a.D * 4 : 0;
+    part = bytes > part ? bytes : part;
+  };
+  parts(R, a.E, a.F);
+  if (a.F_shared > 0) parts(T, 0, a.F_shared);
+  b.part = c.take(part);
   b.total = c.used;
   return b;
 }
@@ -454,7 +463,7 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
   if (rc) return rc;
   if (want_x || (a->scale_input && a->d_router != nullptr))
     if ((rc = gemm_sum(b.dg, a->w_gate, b.du, a->w_up, FS2MOE_W_OUT_IN, s.counts, s.offsets, E, F, D, R, dt, b.dxe,
-                       stream)))
+                       b.part, stream)))
       return rc;
   // combine weights -> logits
   if (want_x || a->d_router != nullptr) {
@@ -469,7 +478,7 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
         (rc = fs2moe_swiglu_backward(s.gs, s.us, b.dhs, T, Fs, dt, b.dhs, b.dgs, b.dus, stream)))
       return rc;
     if (want_x && (rc = gemm_sum(b.dgs, a->shared_gate, b.dus, a->shared_up, FS2MOE_W_IN_OUT, nullptr, nullptr, 0, Fs,
-                                 D, T, dt, b.dx_shared, stream)))
+                                 D, T, dt, b.dx_shared, b.part, stream)))
       return rc;
   }
   // all weight gradients
@@ -477,7 +486,7 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
   const int n = requests(*a, s, b, r);
   if (n > 0) {
     (void)wgrad_plan(r, n, E, R, T, dt);
-    if ((rc = wgrad_all(r, n, gradients_in_place(*a) ? s.perm : nullptr, s.counts, s.offsets, E, R, T, dt, b.wgrad,
+    if ((rc = wgrad_all(r, n, gradients_in_place(*a) ? s.perm : nullptr, s.counts, s.offsets, E, R, T, dt, b.part,
                         stream)))
       return rc;
     if (a->d_router != nullptr && Ep != E && (rc = copy_columns(b.d_router, Ep, a->d_router, E, D, dt, st))) return rc;
