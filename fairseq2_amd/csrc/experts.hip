@@ -303,7 +303,12 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
       return launch_half<128, 128, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
                                                                     num_blocks, stream);
   }
-  hipLaunchKernelGGL(K % (2 * BK) == 0 ? whole : tail, dim3((unsigned)num_blocks), dim3(NWAVES * 64),
+  // The variant for any K also stores rows that do not begin on lines as L2 wants them, which counts for more than its
+  // selects at every load where stores are a large part of the work: three results (the training step of 3395 tokens,
+  // top-2 of 16, D 640, F 13800 2049 -> 1967 us, of 3001, D 1024, F 1368 542 -> 540), or few units (forward over 8803
+  // tokens, top-2 of 16, D 4928, F 7768 3950 -> 3970, so not there).
+  const bool off_lines = N % 64 != 0 && (KEEP_GU || K <= 1024);
+  hipLaunchKernelGGL(K % (2 * BK) == 0 && !off_lines ? whole : tail, dim3((unsigned)num_blocks), dim3(NWAVES * 64),
                      SMEM_BYTES, stream, static_cast<const uint16_t*>(a), row_map, K,
                      static_cast<const uint16_t*>(b0), static_cast<const uint16_t*>(b1),
                      static_cast<const float*>(s0), static_cast<const float*>(s1),
@@ -321,7 +326,7 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
 //   16 of 214, K 5568, N 1280                 180, 163 (2)    8 of 920, K 2800, N 576     89,  91 (2)
 // and where it says 1: 16 of 552, K 7040, N 1088 365, 370 (3); 60 of 240, K 1600, N 1216 159, 202 (2); 16 of 375,
 // K 1368, N 1024 52, 63 (2).  A constant number of CUs, as the scratch is sized in calls that touch no device.
-int fs2moe::split_parts(int sources, int64_t rows, int E, int K, int N) {
+int split_parts(int sources, int64_t rows, int E, int K, int N) {
   constexpr int CUS = 256, MIN_UNITS = 16;
   constexpr int64_t MAX_BYTES = 256ll << 20;
   if (rows <= 0) return 1;

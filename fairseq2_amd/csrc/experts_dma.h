@@ -130,8 +130,8 @@ struct TileOrder {
 // TWO_SRC (single matrix, bf16 weights): C = A @ B0_e + A2 @ B1_e, the second pair
 // walked after the first into the same accumulators (Kdim is one pair's).  A2 arrives in S0, for the
 // reason given above.
-// KTAIL (bf16 weights): Kdim is a multiple of 8 but not of the unit's 64.  A tile's last unit then
-// ends inside its 64 k: the producers load zeros for the 16-byte pieces past Kdim, of both operands,
+// KTAIL (bf16 weights): Kdim is any multiple of 8.  A tile's last unit may then
+// end inside its 64 k: the producers load zeros for the 16-byte pieces past Kdim, of both operands,
 // since what lies there may be anything.  Variants of their own, so that the kernels for whole units
 // compile to what they were.  Against the 128-row kernel that such sizes took before (its blocks wait
 // for every k-step's loads) and the gathered copy it needed: D 1088, F 1392, 8 experts, 8364 rows, whole
@@ -684,6 +684,17 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
   // Chunk c of row r sits at r * ROWB + ((c ^ key(r)) << 4), key(r) = (r >> 1) & 7 when DUAL (rows are
   // 128 B: two rows span the banks) and r & 15 otherwise.  With r and c split into a per-lane part and
   // a compile-time part, every address below is one per-lane base XOR / plus constants.
+  // Streaming stores: the tile is not read again by this kernel.  But where C's rows do not begin on 128-byte lines, a
+  // piece of 128 bytes lies in two, and each would go to memory in parts: as ordinary stores L2 puts them together
+  // (KTAIL variants alone, which take such widths as well: the choice costs the others 0.5-1 % of a layer).
+  auto store_16 = [&](uint8_t* to, u32x4 v) {
+    if (!KTAIL || (ldc & 63) == 0) {
+      __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(to));
+    } else {
+      *reinterpret_cast<u32x4*>(to) = v;
+      asm volatile("" ::: "memory");  // (else the two are merged into one that is not non-temporal)
+    }
+  };
   auto store_tile = [&](const Tile& t, int gu, int scale_slot) {
     constexpr int ROWB = DUAL ? 128 : 256;  // bytes per row of the wave's output tile
     constexpr int CH = ROWB / 16;           // 16-byte chunks per row
@@ -752,9 +763,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
             buf + (rbase_l ^ (uint32_t)((it & KEYMASK) << 6)) + it * RPI * ROWB);
         const int r = m_wave + fm * 32 + it * RPI;  // uniform
         uint8_t* row_base = reinterpret_cast<uint8_t*>(C + (size_t)r * ldc);
-        if (col_ok && r + r_lane < t.row_end)
-          // streaming store: the tile is not read again by this kernel
-          __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(row_base + lane_off_l));
+        if (col_ok && r + r_lane < t.row_end) store_16(row_base + lane_off_l, val);
       }
     }
   };
@@ -792,8 +801,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
               buf + (rbase ^ (uint32_t)((it & 1) << 6)) + it * RPI * ROWB);
           const int r = m_wave + fm * 32 + it * RPI;  // uniform
           uint8_t* row_base = reinterpret_cast<uint8_t*>(out + (size_t)r * ldc);
-          if (col_ok && r + r_lane < t.row_end)
-            __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(row_base + lane_off));
+          if (col_ok && r + r_lane < t.row_end) store_16(row_base + lane_off, val);
         }
       }
     }
