@@ -65,10 +65,13 @@ constexpr int RING_BYTES = 2 * UNIT_BYTES;         // 128 KB
 #define FS2MOE_GEMM_BAND 8
 #endif
 constexpr int BAND = FS2MOE_GEMM_BAND;  // row blocks per band of the tile order (see locate)
+// Where no expert has more rows than this, one of 257 to 384 has its rows cut into two tiles of about as many (the
+// first a multiple of 64) instead of 256 and the rest: see the tile tables.
+constexpr int EVEN_ROWS = 2 * BM;
 constexpr int LIGHT_ROWS = 128;  // a last tile of at most this many rows costs about half a tile
-// after the ring: heavy-tile prefix [E + 1], light-tile prefix [E + 1], counts [E], offsets [E], each
+// after the ring: heavy-tile prefix [E + 1], light-tile prefix [E + 1], counts [E], offsets [E], rows of a heavy tile [E], each
 // sized for the library's limit on E
-constexpr int TABLE_INTS = 4 * FS2MOE_MAX_EXPERTS + 8;
+constexpr int TABLE_INTS = 5 * FS2MOE_MAX_EXPERTS + 8;
 // then, for e4m3 weights, the per-channel scales of two tiles (the one being multiplied and the one
 // whose loads are under way): [2][256] f32
 constexpr int SCALE_BYTES = 2 * BNV * 4;
@@ -160,6 +163,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
   int32_t* s_lstart = s_hstart + FS2MOE_MAX_EXPERTS + 4;                  // [E + 1]
   int32_t* s_counts = s_lstart + FS2MOE_MAX_EXPERTS + 4;
   int32_t* s_offsets = s_counts + FS2MOE_MAX_EXPERTS;
+  int32_t* s_rows = s_offsets + FS2MOE_MAX_EXPERTS;  // of a heavy tile
   float* s_scale = reinterpret_cast<float*>(smem_raw + RING_BYTES + TABLE_INTS * 4);  // [2][BNV]
 
   const int tid = threadIdx.x;
@@ -181,12 +185,18 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
   // Every block then gets the same number of heavy tiles to within one, the light tiles fill up the
   // blocks that got one heavy tile fewer, and the 32 tiles in flight on an XCD are neighbours in the
   // list, which share activation rows (same rows, next channels) and weights (same expert).
+  // The light tile of an expert with heavy ones reads its weights a second time, at another time.  Two tiles of about
+  // as many rows are neighbours in the list instead: they walk K side by side on one XCD, and the second finds the
+  // weights in L2.  128 experts of 270, 310, 350 and 384 rows, K 2048, N 1536: 323, 329, 356, 360 -> 317, 314, 325, 329
+  // us (257: 362, 368).  Not with experts of many rows beside them, whose heavy tiles hide light ones: 8192 tokens of
+  // the layer with D 2048, F 768, top-8 of 128 by a popularity law 720 us as it is, 728 with even tiles.
   {
     __shared__ int s_wave_tot[2][NWAVES];
     const int cnt = dense ? (tid == 0 ? g.dense_rows : 0) : (tid < E ? g.counts[tid] : 0);
+    const bool even = !__syncthreads_or(cnt > EVEN_ROWS) && cnt > BM;
     const int rem = cnt % BM;
-    const int heavy = cnt / BM + (rem > LIGHT_ROWS ? 1 : 0);
-    const int light = (rem > 0 && rem <= LIGHT_ROWS) ? 1 : 0;
+    const int light = (rem > 0 && rem <= LIGHT_ROWS && !even) ? 1 : 0;
+    const int heavy = (cnt + BM - 1) / BM - light;
     int hincl = heavy, lincl = light;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -210,6 +220,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
       s_hstart[tid] = hbase + hincl - heavy;
       s_lstart[tid] = lbase + lincl - light;
       s_counts[tid] = cnt;
+      s_rows[tid] = even ? ((cnt + 1) / 2 + 63) & ~63 : BM;
       s_offsets[tid] = dense ? 0 : g.offsets[tid];
     }
     if (tid == E - 1) {
@@ -259,7 +270,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
     const int half = (listed >= heavy_end && !is_light) ? ((listed - heavy_end) & 1) : -1;
     const int logical = half >= 0 ? heavy_end + ((listed - heavy_end) >> 1) : listed;
     const int in_kind = is_light ? listed - halves_end : logical;
-    int mt = in_kind / n_tiles;  // m-tile in list order: which expert
+    int mt = __builtin_amdgcn_readfirstlane(in_kind / n_tiles);  // m-tile in list order: which expert
     const int32_t* start = is_light ? s_lstart : s_hstart;
     int found = 0;
     for (int e0 = 0; e0 < E; e0 += 64) {
@@ -269,8 +280,9 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
       if (m) found = e0 + (int)__builtin_ctzll(m);
     }
     found = __builtin_amdgcn_readfirstlane(found);
-    const int off = s_offsets[found], cnt = s_counts[found];
-    int nt, first_row;
+    const int off = __builtin_amdgcn_readfirstlane(s_offsets[found]);
+    const int cnt = __builtin_amdgcn_readfirstlane(s_counts[found]);
+    int nt, first_row, last_row = cnt;
     if (is_light) {
       nt = in_kind - mt * n_tiles;
       first_row = cnt / BM * BM;
@@ -281,16 +293,17 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
       // Channel block minor, an XCD would hold one row block x 32 channel blocks, whose weight slabs
       // nobody else on the XCD reads: with wide layers every tile then streams its weights from
       // memory and the kernel is bound by that.
-      const int h0 = s_hstart[found];
+      const int h0 = __builtin_amdgcn_readfirstlane(s_hstart[found]);
       const int l = logical - h0 * n_tiles;
       const int per_band = BAND * n_tiles;
       const int b = l / per_band, t = l - b * per_band;
-      const int left = s_hstart[found + 1] - h0 - b * BAND;
+      const int left = __builtin_amdgcn_readfirstlane(s_hstart[found + 1]) - h0 - b * BAND;
       const int gm = left < BAND ? left : BAND;
       nt = t / gm;
-      first_row = (b * BAND + t - nt * gm) * BM;
+      const int rows = __builtin_amdgcn_readfirstlane(s_rows[found]);
+      first_row = (b * BAND + t - nt * gm) * rows;
+      last_row = cnt < first_row + rows ? cnt : first_row + rows;
     }
-    int last_row = cnt;
     if (half >= 0) {
       first_row += half * LIGHT_ROWS;
       last_row = last_row < first_row + LIGHT_ROWS ? last_row : first_row + LIGHT_ROWS;
@@ -617,8 +630,11 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
   //                (r >> 1) & 7 == (lr >> 1) & 7, so fm only adds 32 rows.
   //   weights: k = 16*ks + 8*lk + (s >> 2) (+4 for the upper half) and k & 3 == (s >> 2) & 3, so ks
   //            adds 16 rows and the upper half 4 rows of BROW bytes: compile-time immediates.
-  const int xrow = (wm * 64 + lr) * 128;
-  const int xr3 = (lr >> 1) & 7;
+  // chunk[2 h + ks]: chunk kc of row lr of a 32-row fragment (row and chunk in one register each, for the
+  // fragments of activations and (out, in) weights alike: with one more the loop reloads it from scratch)
+  int chunk[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) chunk[i] = lr * 128 + (((2 * i + lk) ^ ((lr >> 1) & 7)) << 4);
   int wb[4];
   {
     const int s = lane & 15, half = (lane >> 4) & 1;
@@ -633,8 +649,8 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
         wb[fn] = A_BYTES + mat * (B_BYTES / 2) + k * BROW + (((col >> 3) ^ ((k & 3) << 2)) * 16) +
                  (col & 7) * 2;
       } else {
-        // row (channel) mat * 128 + cbase + lr of the weight block; its swizzle key is xr3 again
-        wb[fn] = A_BYTES + (mat * 128 + cbase + lr) * 128;
+        // row (channel) mat * 128 + cbase + lr of the weight block; its swizzle key is the activations'
+        wb[fn] = A_BYTES + (mat * 128 + cbase) * 128;
       }
     }
   }
@@ -642,14 +658,14 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
   f32x16 acc[4][2];  // [fn][fm]
   auto compute_unit = [&](int gu) {
     const uint8_t* su = smem_raw + (gu & 1) * UNIT_BYTES;
-    const uint8_t* sa = su + xrow;
+    const uint8_t* sa = su + wm * 64 * 128;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const uint8_t* sb = su + h * B_BYTES;
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
         bf16x8 xf[2], wf[4];
-        const int xo = ((4 * h + 2 * ks + lk) ^ xr3) * 16;
+        const int xo = chunk[2 * h + ks];
 #pragma unroll
         for (int fm = 0; fm < 2; ++fm)
           xf[fm] = lds_read_frag(reinterpret_cast<const uint16_t*>(sa + xo + fm * 4096));

@@ -96,7 +96,13 @@ def _groups(rows_per_expert, pad=16):
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
 @pytest.mark.parametrize("layout", ["in_out", "out_in"])
-@pytest.mark.parametrize("rows,k,n", [([5, 0, 300, 64, 1], 64, 96), ([130, 257], 128, 64), ([40, 3, 0, 77], 72, 40)])
+@pytest.mark.parametrize("rows,k,n", [
+    ([5, 0, 300, 64, 1], 64, 96), ([130, 257], 128, 64), ([40, 3, 0, 77], 72, 40),
+    # enough tiles for the throughput kernel: two even tiles from 257 rows to 384, unless an expert has more than 512
+    ([257, 270, 320, 384, 385, 512, 129, 100, 64, 300, 0, 256, 1, 383, 330, 290], 128, 2048),
+    ([257, 270, 320, 384, 385, 512, 129, 100, 64, 300, 0, 256, 1, 383, 330, 290], 72, 1992),
+    ([257, 270, 320, 384, 385, 513, 129, 100, 64, 300, 0, 256, 1, 383, 330, 290], 64, 2048),
+])
 def test_grouped_gemm_both_orientations(gpu_device, dtype, layout, rows, k, n):
     _say("grouped_gemm", dtype, layout, rows, k, n)
     dt = TORCH_DTYPE[dtype]
