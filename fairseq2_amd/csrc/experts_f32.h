@@ -399,6 +399,45 @@ __global__ __launch_bounds__(f32t::threads(GROUPS), 2 * GROUPS) void glu_gemm_f3
   }
 }
 
+// The n-th of the experts, those of more than four times the mean's rows first, then those of more than twice, then the
+// rest, by their numbers within each.  Wave-uniform, every wave for itself; without such experts it is n.
+// A block is one tile's walk over an expert's rows, and the hardware starts blocks in order: where the tiles of the
+// largest expert begin last, the launch waits for their walks alone.  Training step of 2439 tokens, top-2 of 16, D 1024,
+// F 1472 by a popularity law 1926 -> 1591 us; of 2153 evenly, top-1 of 8, D 640, F 2048 1220, 1221; 1000 tokens, top-2 of
+// 8, D 512, F 1408, whose tiles are small, 397 without and 404 with it.
+__device__ __forceinline__ int nth_expert_by_size(const int32_t* __restrict__ counts, int total, int E, int n) {
+  static_assert(FS2MOE_MAX_EXPERTS <= 512, "eight counts a lane");
+  const int lane = threadIdx.x & 63;
+  const float twice = 2.f * (float)total / (float)E;
+  float c[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int i = 64 * j + lane;
+    c[j] = 64 * j < E && i < E ? (float)counts[i] : -1.f;
+  }
+  unsigned long long large = 0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    if (64 * j < E) large |= __ballot(c[j] > twice);
+  if (large == 0) return n;
+  int e = 0, seen = 0;
+#pragma unroll
+  for (int size = 2; size >= 0; --size) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (64 * j >= E) continue;  // uniform
+      const bool in = size == 2 ? c[j] > 2.f * twice : size == 1 ? c[j] > twice && !(c[j] > 2.f * twice)
+                                                                 : c[j] >= 0.f && !(c[j] > twice);
+      const unsigned long long m = __ballot(in);
+      const int before = seen + __popcll(m & ((1ull << lane) - 1ull));
+      const unsigned long long hit = __ballot(in && before == n);
+      if (hit != 0ull) e = 64 * j + (int)__builtin_ctzll(hit);
+      seen += __popcll(m);
+    }
+  }
+  return e;
+}
+
 // dW_e = A_e^T B_e over the rows of an expert (slots: the experts), or over seg_rows rows each of one
 // group (slots: segments, whose sums go to `partial` where there are several).
 // MAPPED: A's rows are read through a_map.
@@ -410,13 +449,19 @@ __global__ __launch_bounds__(f32t::threads(1), 2) void grouped_wgrad_f32_kernel(
   using W = f32t::Walk<1, F, F, true, true, MAPPED>;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[W::SMEM_BYTES];
   const int per = m_tiles * n_tiles;
-  const int slot = blockIdx.x / per, rem = blockIdx.x - slot * per;
+  int slot = blockIdx.x / per;
+  const int rem = blockIdx.x - slot * per;
   const int mt = rem / n_tiles, nt = rem - mt * n_tiles;
   int off, cnt;
   if (g.counts == nullptr) {
     off = slot * seg_rows;
     cnt = g.dense_rows - off < seg_rows ? g.dense_rows - off : seg_rows;
   } else {
+    // (small tiles have short walks, several to a CU side by side: looking costs them 2 % of the step below)
+    if constexpr (F == 2) {
+      const int total = g.offsets[g.E];
+      slot = __builtin_amdgcn_readfirstlane(nth_expert_by_size(g.counts, total, g.E, slot));
+    }
     off = __builtin_amdgcn_readfirstlane(g.offsets[slot]);
     cnt = __builtin_amdgcn_readfirstlane(g.counts[slot]);
   }

@@ -555,6 +555,8 @@ def test_backward_twice_gives_the_same_gradients(gpu_device):
     # (1024 / 256 row blocks here, then 4 column blocks); an odd count leaves the last one alone
     ([(7 * i) % 90 for i in range(33)], 1024, 264), ([(11 * i) % 70 for i in range(35)], 72, 1024),
     ([40 + i for i in range(32)], 520, 520),
+    # enough tiles and rows for the large f32 tiles, experts of more than twice and four times the mean's rows last
+    ([100, 3, 60, 120, 0, 100, 120, 130, 700, 1100], 1032, 1000), ([90] * 66 + [300, 20, 500], 520, 264),
 ])
 def test_grouped_wgrad_matches_torch(gpu_device, dtype, rows, m, n):
     _say("grouped_wgrad", dtype, rows, m, n)
