@@ -270,8 +270,8 @@ bool swiglu_train_applies(int32_t dtype, int32_t D, int32_t F, int64_t rows);
 int swiglu_train(const void* x, const int32_t* row_map, const int32_t* counts, const int32_t* offsets, int32_t E,
                  const void* w_gate, const void* w_up, const void* w_down, int32_t D, int32_t F,
                  int64_t rows, int32_t dtype, void* g, void* u, void* h, void* y, void* stream);
-// Into how many parts the sum over K of a product of `sources` pairs of bf16 matrices goes (1: it stays whole).
-int split_parts(int sources, int64_t rows, int E, int K, int N);
+// Into how many parts the sum over K of a product of `sources` pairs of matrices goes (1: it stays whole).
+int split_parts(int sources, int64_t rows, int E, int K, int N, int dtype);
 // c = a1 @ B1 + a2 @ B2 (fs2moe_grouped_gemm's layouts and groups; E 0: one group), one rounding.  Split where there
 // is scratch for [split_parts(2, ..)][rows][N] f32.
 int gemm_sum(const void* a1, const void* b1, const void* a2, const void* b2, int32_t layout,

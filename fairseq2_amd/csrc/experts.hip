@@ -194,7 +194,7 @@ __global__ __launch_bounds__(256, 2) void glu_gemm_bf16_kernel(
 template <bool DUAL, int BLAYOUT>
 static int launch_f32(const void* a, const void* b0, const void* b1, const void* a2, void* c,
                       void* g_keep, void* u_keep, int K, int N, const Groups& g, int64_t rows_bound,
-                      const char* what, hipStream_t stream) {
+                      const char* what, hipStream_t stream, int parts = 1) {
   const int groups = g.counts ? g.E : 0;
   const int big_n = DUAL ? 64 : 128;
   const bool small = f32t::small_tiles((rows_bound / 128 + groups + 1) * ((N + big_n - 1) / big_n),
@@ -210,7 +210,8 @@ static int launch_f32(const void* a, const void* b0, const void* b1, const void*
   constexpr int groups_small = DUAL ? 1 : 2;
   auto k = small ? glu_gemm_f32_kernel<DUAL, 1, 1, BLAYOUT, groups_small>
                  : glu_gemm_f32_kernel<DUAL, 2, DUAL ? 1 : 2, BLAYOUT, 1>;
-  hipLaunchKernelGGL(k, dim3((unsigned)((m_tiles * nt + 7) / 8 * 8)), dim3(f32t::threads(small ? groups_small : 1)), 0, stream,
+  hipLaunchKernelGGL(k, dim3((unsigned)((m_tiles * nt + 7) / 8 * 8), (unsigned)parts),
+                     dim3(f32t::threads(small ? groups_small : 1)), 0, stream,
                      static_cast<const float*>(a), static_cast<const float*>(b0),
                      static_cast<const float*>(b1), static_cast<const float*>(a2),
                      static_cast<float*>(c), static_cast<float*>(g_keep), static_cast<float*>(u_keep), K,
@@ -326,12 +327,34 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
 //   16 of 214, K 5568, N 1280                 180, 163 (2)    8 of 920, K 2800, N 576     89,  91 (2)
 // and where it says 1: 16 of 552, K 7040, N 1088 365, 370 (3); 60 of 240, K 1600, N 1216 159, 202 (2); 16 of 375,
 // K 1368, N 1024 52, 63 (2).  A constant number of CUs, as the scratch is sized in calls that touch no device.
-int split_parts(int sources, int64_t rows, int E, int K, int N) {
+// f32 tiles (experts_f32.h): a CU multiplies no faster with several, so a part's time is its rounds of tiles, 0.53 us
+// per 32 k and tile of 64 x 64.  8 experts of 250 rows, two sources of K 1408, N 512 (280 tiles): the step of 1000 tokens
+// 394 -> 372 us in four parts.
+int split_parts(int sources, int64_t rows, int E, int K, int N, int dtype) {
   constexpr int CUS = 256, MIN_UNITS = 16;
   constexpr int64_t MAX_BYTES = 256ll << 20;
   if (rows <= 0) return 1;
   const int groups = E > 0 ? E : 1;
   const int64_t real = E > 0 && rows > 15ll * E ? rows - 15ll * E : rows;  // (as in half_tiles::pick)
+  if (dtype == FS2MOE_F32) {
+    const int64_t big = (rows / 128 + E + 1) * ((N + 127) / 128);  // (as in launch_f32)
+    if (!f32t::small_tiles(big, rows / groups)) return 1;
+    const int64_t each = real / groups, chunks = sources * ((K + f32t::BK - 1) / f32t::BK);
+    // (half of a last row block per expert)
+    const int64_t tiles = (groups + (each > 32 ? (real - 32 * groups) / 64 : 0)) * ((N + 63) / 64);
+    auto time = [&](int64_t parts) { return (tiles * parts + CUS - 1) / CUS * ((chunks + parts - 1) / parts) * 530; };
+    int best = 1;
+    int64_t base = time(1);
+    for (int parts = 2; parts <= 8 && chunks / parts >= MIN_UNITS && parts * rows * N * 4 <= MAX_BYTES; ++parts) {
+      const int64_t t = time(parts) + parts * rows * N / 500 + 6000;
+      if (best == 1 ? t * 10 < base * 9 : t < base) {
+        best = parts;
+        base = t;
+      }
+    }
+    const int64_t per = (chunks + best - 1) / best;
+    return (int)((chunks + per - 1) / per);
+  }
   const int64_t each = real / groups, nt = (N + dma::BNV - 1) / dma::BNV, rest = each % dma::BM;
   const int64_t heavy = (each / dma::BM + (rest > dma::LIGHT_ROWS)) * groups * nt;
   const int64_t light = (rest > 0 && rest <= dma::LIGHT_ROWS ? groups : 0) * nt;
@@ -364,8 +387,9 @@ int split_parts(int sources, int64_t rows, int E, int K, int N) {
 
 // C [rows][N] = the sum of the parts [parts][rows][N] in order, rounded once; a lane takes 8 columns of N, a multiple
 // of 8.  (Rows between the experts hold anything, there as here.)
+template <typename T>
 static __global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict__ from, int parts, int64_t n,
-                                                        uint16_t* __restrict__ C) {
+                                                               T* __restrict__ C) {
   const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
   if (i >= n) return;
   f32x4 lo = *reinterpret_cast<const f32x4*>(from + i), hi = *reinterpret_cast<const f32x4*>(from + i + 4);
@@ -374,8 +398,19 @@ static __global__ __launch_bounds__(256) void split_sum_kernel(const float* __re
     lo += *reinterpret_cast<const f32x4*>(from + (size_t)p * n + i);
     hi += *reinterpret_cast<const f32x4*>(from + (size_t)p * n + i + 4);
   }
-  *reinterpret_cast<u32x4*>(C + i) = u32x4{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]),
-                                           pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
+  if constexpr (sizeof(T) == 2) {
+    *reinterpret_cast<u32x4*>(C + i) = u32x4{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]),
+                                             pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
+  } else {
+    *reinterpret_cast<f32x4*>(C + i) = lo;
+    *reinterpret_cast<f32x4*>(C + i + 4) = hi;
+  }
+}
+template <typename T>
+static int launch_split_sum(const void* scratch, int parts, int64_t n, void* c, hipStream_t stream) {
+  hipLaunchKernelGGL(split_sum_kernel<T>, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, stream,
+                     static_cast<const float*>(scratch), parts, n, static_cast<T*>(c));
+  return check_launch("split_sum");
 }
 
 // The product in `parts` parts (at least 2), whose sums go to scratch [parts][rows][N] f32, and their sum.
@@ -405,10 +440,7 @@ static int launch_split(const void* a, int K, const void* b0, const void* b1, co
                      static_cast<const float*>(a2), static_cast<const float*>(nullptr),
                      static_cast<uint16_t*>(scratch), parts, K, N, g, (N + 255) / 256 * parts);
   if (int rc = check_launch(what)) return rc;
-  const int64_t n = (int64_t)g.dense_rows * N;
-  hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, stream,
-                     static_cast<const float*>(scratch), parts, n, static_cast<uint16_t*>(c));
-  return check_launch("split_sum");
+  return launch_split_sum<uint16_t>(scratch, parts, (int64_t)g.dense_rows * N, c, stream);
 }
 
 // The bf16 throughput kernel pair (gate/up, then down); BLAYOUT as the kernel takes it, scales only
@@ -981,7 +1013,15 @@ int fs2moe::gemm_sum(const void* a1, const void* b1, const void* a2, const void*
                      int64_t rows, int32_t dtype, void* c, void* split_scratch, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
   const Groups g{E > 0 ? counts : nullptr, E > 0 ? offsets : nullptr, E > 0 ? E : 1, (int)rows};
-  const int parts = dtype == FS2MOE_BF16 && split_scratch != nullptr ? split_parts(2, rows, E, K, N) : 1;
+  const int parts = split_scratch != nullptr ? split_parts(2, rows, E, K, N, dtype) : 1;
+  if (parts > 1 && dtype == FS2MOE_F32) {
+    const int rc = layout == FS2MOE_W_IN_OUT
+                       ? launch_f32<false, FS2MOE_W_IN_OUT>(a1, b1, b2, a2, split_scratch, nullptr, nullptr, K, N, g,
+                                                            rows, "glu_gemm_f32<two sources, parts>", st, parts)
+                       : launch_f32<false, FS2MOE_W_OUT_IN>(a1, b1, b2, a2, split_scratch, nullptr, nullptr, K, N, g,
+                                                            rows, "glu_gemm_f32<two sources, parts>", st, parts);
+    return rc ? rc : launch_split_sum<float>(split_scratch, parts, rows * N, c, st);
+  }
   if (parts > 1)
     return layout == FS2MOE_W_IN_OUT
                ? launch_split<FS2MOE_W_IN_OUT, true>(a1, K, b1, b2, a2, c, N, g, parts, split_scratch,

@@ -148,11 +148,12 @@ struct Walk {
     const float* a;
     const float* b[NB];
   };
-  // m_rows, n_cols: how many of the tile's rows and channels exist; `active`: this wave's rows do
+  // m_rows, n_cols: how many of the tile's rows and channels exist; `active`: this wave's rows do.  The walk is the
+  // part-th of `parts`, each as many chunks but the last.
   static __device__ __forceinline__ void run(f32x16 (&acc)[NB][FN][FM], uint8_t* smem, const Source& s0,
                                              const Source& s1, int sources, int lda, int ldb, int K,
                                              int m_rows, int n_cols, bool active,
-                                             const int32_t* a_map = nullptr) {
+                                             const int32_t* a_map = nullptr, int part = 0, int parts = 1) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave_m(wave), wn = wave_n(wave), s0k = wave_group(wave) * STEPS;
@@ -160,7 +161,8 @@ struct Walk {
     OpB opb;
     opa.setup(tid, lda, m_rows);
     opb.setup(tid, ldb, n_cols);
-    const int nk = (K + BK - 1) / BK, steps = sources * nk;
+    const int nk = (K + BK - 1) / BK, all = sources * nk, per = (all + parts - 1) / parts, first = part * per;
+    const int steps = all - first < per ? all - first : per;
     u32x4 ra[2][OpA::PER], rb[2][NB][OpB::PER];
     // piece p of a chunk's PIECES: A's first, then each matrix's
     struct Chunk {
@@ -169,8 +171,9 @@ struct Walk {
       int k0, left;
     };
     auto chunk_at = [&](int step) {
-      const bool second = step >= nk;
-      const int k0 = (second ? step - nk : step) * BK;
+      const int at = first + step;
+      const bool second = at >= nk;
+      const int k0 = (second ? at - nk : at) * BK;
       const int left = step < steps ? K - k0 : 0;
       Chunk c;
       c.k0 = k0;
@@ -324,7 +327,8 @@ struct Walk {
 }  // namespace f32t
 
 // C = A B_e (+ A2 B2_e), or with DUAL C = SiLU(A B0_e) * (A B1_e), the two products left in g_keep and
-// u_keep where those are given.  A block per tile; BLAYOUT as for the bf16 kernels.
+// u_keep where those are given.  A block per tile; BLAYOUT as for the bf16 kernels.  With several rows of blocks
+// (single products) each takes a part of the sum over K, and C is [gridDim.y][rows][N].
 template <bool DUAL, int FM, int FN, int BLAYOUT, int GROUPS>
 __global__ __launch_bounds__(f32t::threads(GROUPS), 2 * GROUPS) void glu_gemm_f32_kernel(
     const float* __restrict__ A, const float* __restrict__ B0, const float* __restrict__ B1,
@@ -366,8 +370,9 @@ __global__ __launch_bounds__(f32t::threads(GROUPS), 2 * GROUPS) void glu_gemm_f3
   }
   const int m_wave = row0 + wm * 32 * FM;
   W::run(acc, smem, s0, s1, !DUAL && A2 != nullptr ? 2 : 1, K, KN ? N : K, K, row_end - row0, N - n0,
-         m_wave < row_end);
+         m_wave < row_end, nullptr, DUAL ? 0 : (int)blockIdx.y, DUAL ? 1 : (int)gridDim.y);
   if (!W::holds_sums(wave)) return;
+  if constexpr (!DUAL) C += (size_t)blockIdx.y * g.dense_rows * N;
 
 #pragma unroll
   for (int fm = 0; fm < FM; ++fm) {

@@ -297,7 +297,7 @@ BackwardScratch carve_backward(const Args& a, void* base) {
   // (the weight gradients' partial sums, after those of the rows' gradients)
   int64_t part = wgrad_plan(r, n, a.E, R, T, a.act_dtype);
   auto parts = [&](int64_t rows, int E, int F) {
-    const int n = a.act_dtype == FS2MOE_BF16 ? split_parts(2, rows, E, F, a.D) : 1;
+    const int n = split_parts(2, rows, E, F, a.D, a.act_dtype);
     const int64_t bytes = n > 1 ? (int64_t)n * rows * a.D * 4 : 0;
     part = bytes > part ? bytes : part;
   };
