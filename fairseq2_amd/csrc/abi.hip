@@ -264,8 +264,8 @@ int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_
                                         b.inv_perm, b.disp_ws,  b.disp_ws_bytes, b.row_w,   false};
     if (int rc = fs2moe::router_then_dispatch(
             x, normed ? norm_weight : nullptr, normed ? norm_eps : 0.f, normed ? b.xn : nullptr, router,
-            router_bias, T, D, E, K, act_dtype, score_fn, renormalize, b.topk_idx, b.topk_w, b.router_ws,
-            b.router_ws_bytes, b.xe == nullptr ? &disp : nullptr, stream))
+            router_bias, T, D, E, K, act_dtype, score_fn, renormalize, b.topk_idx, b.topk_w, nullptr,
+            b.router_ws, b.router_ws_bytes, b.xe == nullptr ? &disp : nullptr, stream))
       return rc;
     if (normed) x = b.xn;
     if (beside && normed) {

@@ -236,11 +236,11 @@ int dispatch_index_tiles(const int32_t* topk_idx, int32_t T, int32_t K, int32_t 
                          int64_t max_rows, const uint8_t* tile_counts, const int32_t* tile_rank,
                          int32_t* counts, int32_t* offsets, int32_t* perm, int32_t* inv_perm,
                          void* stream);
-// fs2moe_router_topk (xn null) or fs2moe_router_topk_norm, without the logits output
+// fs2moe_router_topk (xn null) or fs2moe_router_topk_norm; logits may be null
 int router_then_dispatch(const void* x, const void* norm_w, float norm_eps, void* xn,
                          const void* router, const float* bias, int32_t T, int32_t D, int32_t E,
                          int32_t K, int32_t act_dtype, int32_t score_fn, int32_t renormalize,
-                         int32_t* topk_idx, float* topk_w, void* workspace, int64_t workspace_bytes,
+                         int32_t* topk_idx, float* topk_w, float* logits, void* workspace, int64_t workspace_bytes,
                          DispatchAfterRouter* disp, void* stream);
 
 // fs2moe_dispatch without a row copy that also writes row_w[row] = topk_w[pair] (see

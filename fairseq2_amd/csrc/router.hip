@@ -978,8 +978,8 @@ template <int J, bool ALL, int TOK>
 __global__ __launch_bounds__(finish_tile_threads<TOK>()) void router_finish_tile_kernel(
     const float* __restrict__ partial, int slices, const float* __restrict__ bias, int T, int E,
     int K, int score_fn, int renorm, int32_t* __restrict__ topk_idx, float* __restrict__ topk_w,
-    uint8_t* __restrict__ tile_counts, int32_t* __restrict__ tile_rank, int tile_m, int64_t max_rows,
-    int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ perm,
+    float* __restrict__ logits, uint8_t* __restrict__ tile_counts, int32_t* __restrict__ tile_rank, int tile_m,
+    int64_t max_rows, int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ perm,
     int32_t* __restrict__ inv_perm, float* __restrict__ row_w) {
   constexpr int THREADS = finish_tile_threads<TOK>(), NW = THREADS / kWave, TPW = TOK / NW;
   __shared__ uint32_t s_bits[64 * J];
@@ -996,7 +996,7 @@ __global__ __launch_bounds__(finish_tile_threads<TOK>()) void router_finish_tile
     const int tl = wave + NW * i;
     chosen[i] = 0;
     if (t0 + tl >= T) continue;  // wave-uniform
-    finish_token<J>(partial, slices, bias, t0 + tl, T, E, K, score_fn, renorm, topk_idx, topk_w, nullptr,
+    finish_token<J>(partial, slices, bias, t0 + tl, T, E, K, score_fn, renorm, topk_idx, topk_w, logits,
                     &chosen[i]);
     if (lane < K) atomicOr(&s_bits[chosen[i]], 1u << tl);
   }
@@ -1476,7 +1476,7 @@ static int router_entry(const void* x, const void* norm_w, float norm_eps, void*
       const bool all = T <= kRouterTileTok;
       const int tok = all ? kRouterTileTok : T > kFinishTokMax ? kFinishTokMany : kFinishTok;
       const int tiles = (T + tok - 1) / tok;
-      if (disp != nullptr && logits == nullptr &&
+      if (disp != nullptr &&
           (all || (disp->row_w == nullptr && disp->ws != nullptr && tiles <= kIndexTilesMax &&
                    disp->ws_bytes >= fs2moe_dispatch_workspace_bytes(T, K, E)))) {
         uint8_t* tile_counts = all ? nullptr : tile_counts_of(disp->ws);
@@ -1489,7 +1489,7 @@ static int router_entry(const void* x, const void* norm_w, float norm_eps, void*
                        dim3(tiles), dim3(tok == kFinishTok ? finish_tile_threads<kFinishTok>()     \
                                                            : finish_tile_threads<kFinishTokMany>()), \
                        0, s, partial, slices, bias, T, E, K, \
-                       score_fn, renormalize, topk_idx, topk_w, tile_counts, tile_rank, disp->tile_m, \
+                       score_fn, renormalize, topk_idx, topk_w, logits, tile_counts, tile_rank, disp->tile_m, \
                        disp->max_rows, disp->counts, disp->offsets, disp->perm, disp->inv_perm,    \
                        disp->row_w);                                                               \
     break;
@@ -1561,7 +1561,7 @@ extern "C" int fs2moe_router_topk_norm(const void* x, const void* norm_weight, f
 int fs2moe::router_then_dispatch(const void* x, const void* norm_w, float norm_eps, void* xn,
                                  const void* router, const float* bias, int32_t T, int32_t D,
                                  int32_t E, int32_t K, int32_t act_dtype, int32_t score_fn,
-                                 int32_t renormalize, int32_t* topk_idx, float* topk_w,
+                                 int32_t renormalize, int32_t* topk_idx, float* topk_w, float* logits,
                                  void* workspace, int64_t workspace_bytes,
                                  DispatchAfterRouter* disp, void* stream) {
   FS2_REQUIRE(xn == nullptr || norm_eps >= 0.f, "router: norm_eps %g is negative", (double)norm_eps);
@@ -1572,7 +1572,7 @@ int fs2moe::router_then_dispatch(const void* x, const void* norm_w, float norm_e
     disp->done = false;
   }
   return router_entry(x, norm_w, norm_eps, xn, router, bias, T, D, E, K, act_dtype, score_fn,
-                      renormalize, topk_idx, topk_w, nullptr, workspace, workspace_bytes, disp,
+                      renormalize, topk_idx, topk_w, logits, workspace, workspace_bytes, disp,
                       stream);
 }
 

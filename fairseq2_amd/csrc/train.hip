@@ -359,17 +359,18 @@ extern "C" int fs2moe_train_forward(const fs2moe_train_args* a, void* stream) {
   FS2_REQUIRE(aligned16(a->out) && aligned16(a->residual), "train_forward: out and residual must be 16-byte aligned");
   const int64_t R = rows_of(*a);
   const void* x = a->normed ? s.xn : a->x;
-  int rc = a->normed
-               ? fs2moe_router_topk_norm(a->x, a->norm_weight, a->norm_eps, s.xn, a->router_read, a->router_bias,
-                                         a->T, a->D, a->E, a->K, a->act_dtype, a->score_fn, a->renormalize, s.idx,
-                                         s.w, s.logits, f.router, f.router_bytes, stream)
-               : fs2moe_router_topk(a->x, a->router_read, a->router_bias, a->T, a->D, a->E, a->K, a->act_dtype,
-                                    a->score_fn, a->renormalize, s.idx, s.w, s.logits, f.router, f.router_bytes,
-                                    stream);
+  // (rows that stay in token order need no copy: the router's last kernel counts for the dispatch, a launch fewer; 4096
+  // tokens, top-8 of 128, D 2048, F 768 1580 -> 1573 us, 4444, D 1280, F 704 1094 -> 1087)
+  DispatchAfterRouter disp{a->tile_m, R, s.counts, s.offsets, s.perm, s.inv_perm, f.disp, f.disp_bytes, nullptr, false};
+  int rc = router_then_dispatch(a->x, a->normed ? a->norm_weight : nullptr, a->normed ? a->norm_eps : 0.f,
+                                a->normed ? s.xn : nullptr, a->router_read, a->router_bias, a->T, a->D, a->E, a->K,
+                                a->act_dtype, a->score_fn, a->renormalize, s.idx, s.w, s.logits, f.router,
+                                f.router_bytes, s.xe == nullptr ? &disp : nullptr, stream);
   if (rc) return rc;
-  rc = fs2moe_dispatch(s.idx, s.w, x, a->T, a->K, a->E, a->D, a->tile_m, a->act_dtype, a->scale_input, R, s.counts,
-                       s.offsets, s.perm, s.inv_perm, s.xe, f.disp, f.disp_bytes, stream);
-  if (rc) return rc;
+  if (!disp.done &&
+      (rc = fs2moe_dispatch(s.idx, s.w, x, a->T, a->K, a->E, a->D, a->tile_m, a->act_dtype, a->scale_input, R,
+                            s.counts, s.offsets, s.perm, s.inv_perm, s.xe, f.disp, f.disp_bytes, stream)))
+    return rc;
   const bool mapped = in_token_order(*a);
   void* ye = s.ye != nullptr ? s.ye : f.ye;
   if (s.g == nullptr)
