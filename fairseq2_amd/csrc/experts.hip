@@ -198,7 +198,8 @@ static int launch_f32(const void* a, const void* b0, const void* b1, const void*
   const int groups = g.counts ? g.E : 0;
   const int big_n = DUAL ? 64 : 128;
   const bool small = f32t::small_tiles((rows_bound / 128 + groups + 1) * ((N + big_n - 1) / big_n),
-                                       groups ? rows_bound / groups : rows_bound);
+                                       groups ? rows_bound / groups : rows_bound) ||
+                     f32t::small_rounds(DUAL, rows_bound, groups, N, 256);
   const int bm = small ? 64 : 128, bn = small ? 64 : big_n;
   const int64_t m_tiles = rows_bound / bm + groups + 1;
   const int nt = (N + bn - 1) / bn;
@@ -338,7 +339,7 @@ int split_parts(int sources, int64_t rows, int E, int K, int N, int dtype) {
   const int64_t real = E > 0 && rows > 15ll * E ? rows - 15ll * E : rows;  // (as in half_tiles::pick)
   if (dtype == FS2MOE_F32) {
     const int64_t big = (rows / 128 + E + 1) * ((N + 127) / 128);  // (as in launch_f32)
-    if (!f32t::small_tiles(big, rows / groups)) return 1;
+    if (!f32t::small_tiles(big, rows / groups) && !f32t::small_rounds(false, rows, E, N, CUS)) return 1;
     const int64_t each = real / groups, chunks = sources * ((K + f32t::BK - 1) / f32t::BK);
     // (half of a last row block per expert)
     const int64_t tiles = (groups + (each > 32 ? (real - 32 * groups) / 64 : 0)) * ((N + 63) / 64);

@@ -43,6 +43,20 @@ constexpr int threads(int groups) { return 256 * groups; }
 inline bool small_tiles(int64_t big_tiles, int64_t rows_per_group) {
   return big_tiles < 512 || rows_per_group <= 96;
 }
+// Or where their rounds of tiles (of the experts' rows, half of a last row block each) take less time than those of the
+// large ones, 64 rows x N as small tiles or 128 rows x N as large ones of 64 (two products) or 128 columns: 0.53 us per
+// 32 k and small tile, 0.44 per 64 x 64 of a large one.
+// 1356 tokens, top-1 of 16, D 1024, F 2048 by a popularity law 283 -> 225 us; the training step of 2439, top-2 of 16, D
+// 1024, F 1472 1596 -> 1534.
+inline bool small_rounds(bool dual, int64_t rows, int groups, int N, int cus) {
+  const int64_t real = groups > 0 && rows > 15ll * groups ? rows - 15ll * groups : rows;  // (less the blocks' padding)
+  const int g = groups > 0 ? groups : 1;
+  auto blocks = [&](int bm) { return g + (real > (int64_t)g * (bm / 2) ? (real - (int64_t)g * (bm / 2)) / bm : 0); };
+  auto rounds = [&](int64_t tiles) { return (tiles + cus - 1) / cus; };
+  const int64_t small = rounds(blocks(64) * ((N + 63) / 64)) * 53;
+  const int64_t large = dual ? rounds(blocks(128) * ((N + 63) / 64)) * 88 : rounds(blocks(128) * ((N + 127) / 128)) * 176;
+  return small * 12 < large * 11;
+}
 
 // what a load through a row map reads past the end (not const: a global address)
 static __device__ __attribute__((aligned(16))) uint32_t zero16[4] = {0u, 0u, 0u, 0u};

@@ -132,6 +132,8 @@ def test_grouped_gemm_both_orientations(gpu_device, dtype, layout, rows, k, n):
 @pytest.mark.parametrize("rows,k,n", [
     ([63, 64, 65, 0, 1], 8, 56), ([129, 31, 32, 33], 40, 64), ([97], 96, 136),
     ([700, 127, 128, 1, 1300], 40, 4104), ([400] * 6, 1000, 1032),
+    # small tiles for their rounds (of 1230 by the rule's count, against 399 large ones)
+    ([450, 200, 120, 33, 65, 65, 65, 97, 49, 33, 113, 33, 1, 33, 65, 49], 40, 2624),
 ])
 def test_f32_products_at_the_edges_of_their_tiles(gpu_device, rows, k, n):
     _say("f32 products", rows, k, n)
