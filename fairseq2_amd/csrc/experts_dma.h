@@ -193,11 +193,14 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
   {
     __shared__ int s_wave_tot[2][NWAVES];
     const int cnt = dense ? (tid == 0 ? g.dense_rows : 0) : (tid < E ? g.counts[tid] : 0);
-    const bool even = !__syncthreads_or(cnt > EVEN_ROWS) && cnt > BM;
     const int rem = cnt % BM;
-    const int light = (rem > 0 && rem <= LIGHT_ROWS && !even) ? 1 : 0;
-    const int heavy = (cnt + BM - 1) / BM - light;
-    int hincl = heavy, lincl = light;
+    int heavy = cnt / BM + (rem > LIGHT_ROWS ? 1 : 0);
+    int light = (rem > 0 && rem <= LIGHT_ROWS) ? 1 : 0;
+    // what even tiles change: an expert of 257 to 384 rows has two heavy tiles instead of one of each
+    const int moved = (light && cnt > BM && cnt <= EVEN_ROWS) ? 1 : 0;
+    constexpr int MOVED = 1 << 12, MANY = 1 << 24;  // (next to the light tiles, at most FS2MOE_MAX_EXPERTS of each)
+    static_assert(FS2MOE_MAX_EXPERTS < MOVED, "light tiles, moved ones and a flag in one word");
+    int hincl = heavy, lincl = light + moved * MOVED;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
       const int hv = __shfl_up(hincl, off, kWave), lv = __shfl_up(lincl, off, kWave);
@@ -206,26 +209,37 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
         lincl += lv;
       }
     }
+    const bool many = __ballot(cnt > EVEN_ROWS) != 0ull;
     if (lane == 63) {
       s_wave_tot[0][wave] = hincl;
-      s_wave_tot[1][wave] = lincl;
+      s_wave_tot[1][wave] = lincl + (many ? MANY : 0);
     }
     __syncthreads();
-    int hbase = 0, lbase = 0;
-    for (int w = 0; w < wave; ++w) {
-      hbase += s_wave_tot[0][w];
-      lbase += s_wave_tot[1][w];
+    int hbase = 0, lbase = 0, any = 0;
+    for (int w = 0; w < NWAVES; ++w) {
+      const int v = s_wave_tot[1][w];
+      any |= v;
+      if (w < wave) {
+        hbase += s_wave_tot[0][w];
+        lbase += v & (MANY - 1);
+      }
     }
+    const bool even = (any & MANY) == 0;
+    lincl += lbase;
+    hincl += hbase + (even ? lincl / MOVED : 0);
+    lincl = lincl % MOVED - (even ? lincl / MOVED : 0);
+    heavy += even ? moved : 0;
+    light -= even ? moved : 0;
     if (tid < E) {
-      s_hstart[tid] = hbase + hincl - heavy;
-      s_lstart[tid] = lbase + lincl - light;
+      s_hstart[tid] = hincl - heavy;
+      s_lstart[tid] = lincl - light;
       s_counts[tid] = cnt;
-      s_rows[tid] = even ? ((cnt + 1) / 2 + 63) & ~63 : BM;
+      s_rows[tid] = even && cnt > BM ? ((cnt + 1) / 2 + 63) & ~63 : BM;
       s_offsets[tid] = dense ? 0 : g.offsets[tid];
     }
     if (tid == E - 1) {
-      s_hstart[E] = hbase + hincl;
-      s_lstart[E] = lbase + lincl;
+      s_hstart[E] = hincl;
+      s_lstart[E] = lincl;
     }
     __syncthreads();
   }
