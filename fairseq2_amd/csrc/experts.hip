@@ -309,7 +309,8 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
   // selects at every load where stores are a large part of the work: three results (the training step of 3395 tokens,
   // top-2 of 16, D 640, F 13800 2049 -> 1967 us, of 3001, D 1024, F 1368 542 -> 540), or few units (forward over 8803
   // tokens, top-2 of 16, D 4928, F 7768 3950 -> 3970, so not there).
-  const bool off_lines = N % 64 != 0 && (KEEP_GU || K <= 1024);
+  const bool off_lines =
+      off_lines_variant(DUAL, BLAYOUT, TWO_SRC, CAN_TAIL) && N % 64 != 0 && (KEEP_GU || K <= 1024);
   hipLaunchKernelGGL(K % (2 * BK) == 0 && !off_lines ? whole : tail, dim3((unsigned)num_blocks), dim3(NWAVES * 64),
                      SMEM_BYTES, stream, static_cast<const uint16_t*>(a), row_map, K,
                      static_cast<const uint16_t*>(b0), static_cast<const uint16_t*>(b1),

@@ -80,6 +80,11 @@ constexpr int SMEM_BYTES = RING_BYTES + TABLE_INTS * 4 + SCALE_BYTES;
 // output channels x 64 in-features, [expert][channel / 16][feature / 64][16][64], with one f32 scale
 // per output channel (the layout of the decode kernel in experts_fp8.h).
 constexpr int W_FP8_TILED = 2;
+// Whether a variant stores rows that do not begin on lines as ordinary stores (store_16 in the kernel): those that
+// write the experts' inner width, gate/up and the product with the down projection's transpose.
+constexpr bool off_lines_variant(bool dual, int layout, bool two_src, bool ktail) {
+  return ktail && (dual || (layout == FS2MOE_W_OUT_IN && !two_src));
+}
 }  // namespace dma
 
 // Which of a 1 KB e4m3 weight tile's 16 channel rows lane l of a producer takes (it takes the 16
@@ -716,9 +721,10 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
   // a compile-time part, every address below is one per-lane base XOR / plus constants.
   // Streaming stores: the tile is not read again by this kernel.  But where C's rows do not begin on 128-byte lines, a
   // piece of 128 bytes lies in two, and each would go to memory in parts: as ordinary stores L2 puts them together
-  // (KTAIL variants alone, which take such widths as well: the choice costs the others 0.5-1 % of a layer).
+  // (KTAIL variants alone, which take such widths as well: the choice costs the others 0.5-1 % of a layer; and of those
+  // not the ones whose C has the layer's width: 1074 tokens, top-2 of 16, D 3776, F 1872 210.6 us with it, 209.5 without).
   auto store_16 = [&](uint8_t* to, u32x4 v) {
-    if (!KTAIL || (ldc & 63) == 0) {
+    if (!off_lines_variant(DUAL, BLAYOUT, TWO_SRC, KTAIL) || (ldc & 63) == 0) {
       __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(to));
     } else {
       *reinterpret_cast<u32x4*>(to) = v;
