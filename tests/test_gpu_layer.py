@@ -174,6 +174,17 @@ def test_deterministic_and_tile_size_independent(gpu_device):
         assert torch.equal(o, outs[0]), "output must not depend on the run or on the padding granularity"
 
 
+@pytest.mark.parametrize("shared", [False, True])
+def test_f32_layer_does_not_depend_on_the_padding(gpu_device, shared):
+    """Sizes at which the padding alone decides between the two tile sizes of the f32 products."""
+    spec = W.small_spec(tokens=3300, model_dim=1024, num_experts=8, top_k=2, inner_dim=192, dtype="fp32",
+                        shared=shared, seed=11)
+    wl = W.make_workload_from_spec(spec)
+    outs = [_run(wl, gpu_device, tile_m)[2].cpu() for tile_m in (16, 1, 128)]
+    for o in outs[1:]:
+        assert torch.equal(o, outs[0])
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
 @pytest.mark.parametrize("shared", [False, True])
 def test_other_expert_activation(gpu_device, dtype, shared):

@@ -707,6 +707,40 @@ def test_pair_and_two_sources_on_every_tile_size(gpu_device, counts, n):
         assert torch.equal(ye[sl], ye2[sl]) and torch.equal(h[sl], h2[sl]), f"expert {i} without keeping"
 
 
+# The f32 products take tiles of 64 x 64 or 128 x 128 (the pair 128 x 64) by the size of the buffers: the same bits.  Rows
+# on both sides of 32, 64 and 128, K within a chunk of 32, past its quarters and over several, N off the tiles' channels.
+@pytest.mark.parametrize("k", [8, 24, 40, 200])
+@pytest.mark.parametrize("n", [1024, 1000])
+@pytest.mark.parametrize("layout", [_abi.W_IN_OUT, _abi.W_OUT_IN])
+def test_f32_products_are_the_same_on_every_tile_size(gpu_device, k, n, layout):
+    rows = [1, 16, 17, 33, 65, 0, 130, 700]
+    _say("f32 tiles", k, n, layout)
+    e, g = len(rows), torch.Generator().manual_seed(k + n)
+    counts = torch.tensor(rows, dtype=torch.int32, device=gpu_device)
+    offsets = torch.zeros(e + 1, dtype=torch.int32, device=gpu_device)
+    offsets[1:] = torch.cumsum((counts + 15) // 16 * 16, 0)
+    lo = offsets.tolist()
+    x, w, wu = torch.randn(20000, k, generator=g), torch.randn(e, k, n, generator=g), torch.zeros(e, k, n)
+    # the pair's h is its gate product: a product of 20 and more with an up product of one
+    x[:, -1], w[:, -1], wu[:, -1] = 1.0, 20.0 + 16 * k**0.5, 1.0
+    x, w, wu = x.to(gpu_device), w.to(gpu_device), wu.to(gpu_device)
+    b = (w if layout == _abi.W_IN_OUT else w.transpose(1, 2).contiguous()).reshape(-1, n if layout == _abi.W_IN_OUT else k)
+    wd = torch.zeros(e * n, k, device=gpu_device)
+    got = []
+    for total in (lo[-1], 20000):
+        out = [_abi.grouped_gemm(x[:total], b, layout, counts, offsets, e)]
+        if layout == _abi.W_IN_OUT:
+            out.append(_abi.grouped_swiglu(x[:total], counts, offsets, b, wu.reshape(-1, n), wd, e)[1])
+        got += [torch.cat([o[lo[i] : lo[i] + r] for i, r in enumerate(rows)]) for o in out]
+    for i, o in enumerate(got[1:], 1):
+        assert torch.equal(o, got[0]), i
+    ref = torch.cat([x[lo[i] : lo[i] + r].double() @ w[i].double() for i, r in enumerate(rows)])
+    assert_output_close(got[0], ref.cpu(), "fp32")
+    # all rows of one matrix: every group of rows in a launch of its own size
+    dense = [_abi.grouped_gemm(x[:r].contiguous(), b[: (k if layout == _abi.W_IN_OUT else n)], layout) for r in (33, 9000)]
+    assert torch.equal(dense[0], dense[1][:33])
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
 @pytest.mark.parametrize(
     "t,d,f",
