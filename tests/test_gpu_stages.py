@@ -707,13 +707,14 @@ def test_pair_and_two_sources_on_every_tile_size(gpu_device, counts, n):
         assert torch.equal(ye[sl], ye2[sl]) and torch.equal(h[sl], h2[sl]), f"expert {i} without keeping"
 
 
-# The f32 products take tiles of 64 x 64 or 128 x 128 (the pair 128 x 64) by the size of the buffers: the same bits.  Rows
-# on both sides of 32, 64 and 128, K within a chunk of 32, past its quarters and over several, N off the tiles' channels.
+# The f32 products take tiles of 64 x 64, of eight waves or four, or of 128 x 128 (the pair 128 x 64) by the size of the
+# buffers: the same bits.  Rows on both sides of 32, 64 and 128, experts without any, K within a chunk of 32, past its
+# quarters and over several, N off the tiles' channels.
 @pytest.mark.parametrize("k", [8, 24, 40, 200])
 @pytest.mark.parametrize("n", [1024, 1000])
 @pytest.mark.parametrize("layout", [_abi.W_IN_OUT, _abi.W_OUT_IN])
 def test_f32_products_are_the_same_on_every_tile_size(gpu_device, k, n, layout):
-    rows = [1, 16, 17, 33, 65, 0, 130, 700]
+    rows = [1, 16, 17, 33, 65, 0, 130, 700] + [0] * 16
     _say("f32 tiles", k, n, layout)
     e, g = len(rows), torch.Generator().manual_seed(k + n)
     counts = torch.tensor(rows, dtype=torch.int32, device=gpu_device)
@@ -727,7 +728,7 @@ def test_f32_products_are_the_same_on_every_tile_size(gpu_device, k, n, layout):
     b = (w if layout == _abi.W_IN_OUT else w.transpose(1, 2).contiguous()).reshape(-1, n if layout == _abi.W_IN_OUT else k)
     wd = torch.zeros(e * n, k, device=gpu_device)
     got = []
-    for total in (lo[-1], 20000):
+    for total in (lo[-1], 3000, 20000):
         out = [_abi.grouped_gemm(x[:total], b, layout, counts, offsets, e)]
         if layout == _abi.W_IN_OUT:
             out.append(_abi.grouped_swiglu(x[:total], counts, offsets, b, wu.reshape(-1, n), wd, e)[1])
@@ -737,8 +738,9 @@ def test_f32_products_are_the_same_on_every_tile_size(gpu_device, k, n, layout):
     ref = torch.cat([x[lo[i] : lo[i] + r].double() @ w[i].double() for i, r in enumerate(rows)])
     assert_output_close(got[0], ref.cpu(), "fp32")
     # all rows of one matrix: every group of rows in a launch of its own size
-    dense = [_abi.grouped_gemm(x[:r].contiguous(), b[: (k if layout == _abi.W_IN_OUT else n)], layout) for r in (33, 9000)]
-    assert torch.equal(dense[0], dense[1][:33])
+    first = b[: (k if layout == _abi.W_IN_OUT else n)]
+    dense = [_abi.grouped_gemm(x[:r].contiguous(), first, layout) for r in (32, 33, 9000)]
+    assert torch.equal(dense[0], dense[2][:32]) and torch.equal(dense[1], dense[2][:33])
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
