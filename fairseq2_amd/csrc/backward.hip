@@ -1293,7 +1293,7 @@ extern "C" int fs2moe_grouped_wgrad(const void* a, const int32_t* a_row_map, con
 // numbers of CUs (a partition of the chip) its cuts are only less even.
 constexpr int kPlanCUs = 256;
 
-int64_t fs2moe::wgrad_plan(WgradRequest* r, int n, int32_t E, int64_t grouped_rows, int64_t rows,
+int64_t fs2moe::wgrad_plan(WgradRequest* r, int n, int32_t E, int64_t planned, int64_t rows,
                            int32_t dtype) {
   if (dtype == FS2MOE_F32) {  // (one launch each: every single group is cut as in fs2moe_grouped_wgrad)
     int64_t most = 0;
@@ -1309,7 +1309,7 @@ int64_t fs2moe::wgrad_plan(WgradRequest* r, int n, int32_t E, int64_t grouped_ro
   const int64_t one = rows / wgk::RK + wgk::kTileCost;
   int64_t total = 0;
   for (int i = 0; i < n; ++i)
-    total += tiles(r[i]) * (r[i].grouped ? grouped_rows / wgk::RK + (int64_t)E * wgk::kTileCost : one);
+    total += tiles(r[i]) * (r[i].grouped ? planned / wgk::RK + (int64_t)E * wgk::kTileCost : one);
   const int64_t fair = total / kPlanCUs + 1;
   int64_t bytes = 0;
   for (int i = 0; i < n; ++i) {

@@ -270,13 +270,17 @@ bool swiglu_train_applies(int32_t dtype, int32_t D, int32_t F, int64_t rows);
 int swiglu_train(const void* x, const int32_t* row_map, const int32_t* counts, const int32_t* offsets, int32_t E,
                  const void* w_gate, const void* w_up, const void* w_down, int32_t D, int32_t F,
                  int64_t rows, int32_t dtype, void* g, void* u, void* h, void* y, void* stream);
-// Into how many parts the sum over K of a product of `sources` pairs of matrices goes (1: it stays whole).
-int split_parts(int sources, int64_t rows, int E, int K, int N, int dtype);
-// c = a1 @ B1 + a2 @ B2 (fs2moe_grouped_gemm's layouts and groups; E 0: one group), one rounding.  Split where there
-// is scratch for [split_parts(2, ..)][rows][N] f32.
+// The experts' rows that a plan goes by: as many as `pairs` rows take in blocks of 16, whatever granularity the buffers
+// have.  Where the plan decides how sums are cut, results then do not depend on the padding.
+inline int64_t planned_rows(int64_t pairs, int E) { return pairs + 15ll * E; }
+// Into how many parts the sum over K of a product of `sources` pairs of matrices goes (1: it stays whole), by the
+// planned rows (E 0: the rows).
+int split_parts(int sources, int64_t planned, int E, int K, int N, int dtype);
+// c = a1 @ B1 + a2 @ B2 (fs2moe_grouped_gemm's layouts and groups; E 0: one group), one rounding: in split_parts(2,
+// planned, ..) parts, for whose sums there is scratch [parts][rows][N] f32.
 int gemm_sum(const void* a1, const void* b1, const void* a2, const void* b2, int32_t layout,
              const int32_t* counts, const int32_t* offsets, int32_t E, int32_t K, int32_t N,
-             int64_t rows, int32_t dtype, void* c, void* split_scratch, void* stream);
+             int64_t rows, int64_t planned, int32_t dtype, void* c, void* split_scratch, void* stream);
 // One of several weight gradients taken together: grouped (over the experts' rows) or over all `rows` of
 // one group.
 struct WgradRequest {
@@ -287,9 +291,9 @@ struct WgradRequest {
   int segments;  // set by wgrad_plan: of a group's rows, each with its own partial sums
   bool map_a = false, map_b = false;  // bf16: the operand's rows are read through the row map
 };
-// Cuts the rows of single groups whose tiles would take longer than the others together; returns the
-// bytes of scratch that the partial sums need.
-int64_t wgrad_plan(WgradRequest* r, int n, int32_t E, int64_t grouped_rows, int64_t rows, int32_t dtype);
+// Cuts the rows of single groups whose tiles would take longer than the others together (the experts' `planned`
+// rows); returns the bytes of scratch that the partial sums need.
+int64_t wgrad_plan(WgradRequest* r, int n, int32_t E, int64_t planned, int64_t rows, int32_t dtype);
 int wgrad_all(const WgradRequest* r, int n, const int32_t* row_map, const int32_t* counts, const int32_t* offsets,
               int32_t E, int64_t grouped_rows, int64_t rows, int32_t dtype, void* scratch, void* stream);
 // fs2moe_router_backward into rows of ld >= E elements, those past E zero

@@ -332,23 +332,25 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
 // f32 tiles (experts_f32.h): a CU multiplies no faster with several, so a part's time is its rounds of tiles, 0.53 us
 // per 32 k and tile of 64 x 64.  8 experts of 250 rows, two sources of K 1408, N 512 (280 tiles): the step of 1000 tokens
 // 394 -> 372 us in four parts.
-int split_parts(int sources, int64_t rows, int E, int K, int N, int dtype) {
+int split_parts(int sources, int64_t planned, int E, int K, int N, int dtype) {
   constexpr int CUS = 256, MIN_UNITS = 16;
   constexpr int64_t MAX_BYTES = 256ll << 20;
-  if (rows <= 0) return 1;
   const int groups = E > 0 ? E : 1;
-  const int64_t real = E > 0 && rows > 15ll * E ? rows - 15ll * E : rows;  // (as in half_tiles::pick)
+  const int64_t real = planned - 15ll * E;  // (the experts' rows, equally loaded)
+  if (real <= 0) return 1;
+  // (the sums of buffers padded to 128 rows an expert have room in it)
+  const int64_t part_bytes = (real + 127ll * E) * N * 4;
   if (dtype == FS2MOE_F32) {
-    const int64_t big = (rows / 128 + E + 1) * ((N + 127) / 128);  // (as in launch_f32)
-    if (!f32t::small_tiles(big, rows / groups) && !f32t::small_rounds(false, rows, E, N, CUS)) return 1;
+    const int64_t big = (planned / 128 + E + 1) * ((N + 127) / 128);  // (as in launch_f32)
+    if (!f32t::small_tiles(big, planned / groups) && !f32t::small_rounds(false, planned, E, N, CUS)) return 1;
     const int64_t each = real / groups, chunks = sources * ((K + f32t::BK - 1) / f32t::BK);
     // (half of a last row block per expert)
     const int64_t tiles = (groups + (each > 32 ? (real - 32 * groups) / 64 : 0)) * ((N + 63) / 64);
     auto time = [&](int64_t parts) { return (tiles * parts + CUS - 1) / CUS * ((chunks + parts - 1) / parts) * 530; };
     int best = 1;
     int64_t base = time(1);
-    for (int parts = 2; parts <= 8 && chunks / parts >= MIN_UNITS && parts * rows * N * 4 <= MAX_BYTES; ++parts) {
-      const int64_t t = time(parts) + parts * rows * N / 500 + 6000;
+    for (int parts = 2; parts <= 8 && chunks / parts >= MIN_UNITS && parts * part_bytes <= MAX_BYTES; ++parts) {
+      const int64_t t = time(parts) + parts * planned * N / 500 + 6000;
       if (best == 1 ? t * 10 < base * 9 : t < base) {
         best = parts;
         base = t;
@@ -361,21 +363,21 @@ int split_parts(int sources, int64_t rows, int E, int K, int N, int dtype) {
   const int64_t heavy = (each / dma::BM + (rest > dma::LIGHT_ROWS)) * groups * nt;
   const int64_t light = (rest > 0 && rest <= dma::LIGHT_ROWS ? groups : 0) * nt;
   const int64_t units = (int64_t)sources * ((K + 63) / 64);
-  const int64_t memory = sources * ((groups < real ? groups : real) * K * N + rows * K) / 2000;  // ns
+  const int64_t memory = sources * ((groups < real ? groups : real) * K * N + planned * K) / 2000;  // ns
   auto whole = [&](int64_t parts) {
     const int64_t n = parts * (10 * heavy + 6 * light) / 10, left = n % CUS;
     const int64_t t = (units + parts - 1) / parts * (n / CUS * 2000 + (left ? 800 + 1200 * left / CUS : 0));
     return t > memory ? t : memory;
   };
-  const int small = half_tiles::pick(false, true, rows, E, K, N, CUS);
+  const int small = half_tiles::pick(false, true, planned, E, K, N, CUS);
   int64_t base = whole(1);
   if (small != 0) {
     const int64_t t = units * (small == 1 ? 330 : small == 2 ? 450 : 650);
     base = (t > memory ? t : memory) + 4000;
   }
   int best = 1;
-  for (int parts = 2; parts <= 16 && units / parts >= MIN_UNITS && parts * rows * N * 4 <= MAX_BYTES; ++parts) {
-    const int64_t t = whole(parts) + parts * rows * N / 1000 + 6000;
+  for (int parts = 2; parts <= 16 && units / parts >= MIN_UNITS && parts * part_bytes <= MAX_BYTES; ++parts) {
+    const int64_t t = whole(parts) + parts * planned * N / 1000 + 6000;
     // (worth 5 % by these figures, to be taken at all)
     if (best == 1 ? t * 20 < base * 19 : t < base) {
       best = parts;
@@ -387,38 +389,44 @@ int split_parts(int sources, int64_t rows, int E, int K, int N, int dtype) {
   return (int)((units + per - 1) / per);
 }
 
-// C [rows][N] = the sum of the parts [parts][rows][N] in order, rounded once; a lane takes 8 columns of N, a multiple
-// of 8.  (Rows between the experts hold anything, there as here.)
+// C [rows][N] = the sum of the parts [parts][rows][N] in order, rounded once, over the rows of group blockIdx.y (rows
+// between the experts are left alone, there as here); a lane takes 8 columns of N, a multiple of 8.
 template <typename T>
-static __global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict__ from, int parts, int64_t n,
-                                                               T* __restrict__ C) {
-  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
-  if (i >= n) return;
-  f32x4 lo = *reinterpret_cast<const f32x4*>(from + i), hi = *reinterpret_cast<const f32x4*>(from + i + 4);
+static __global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict__ from, int parts, int N,
+                                                               Groups g, T* __restrict__ C) {
+  const bool dense = g.counts == nullptr;
+  const int64_t first = dense ? 0 : (int64_t)g.offsets[blockIdx.y] * N, all = (int64_t)g.dense_rows * N;
+  const int64_t end = first + (int64_t)(dense ? g.dense_rows : g.counts[blockIdx.y]) * N;
+  for (int64_t i = first + ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8; i < end; i += (int64_t)gridDim.x * 2048) {
+    f32x4 lo = *reinterpret_cast<const f32x4*>(from + i), hi = *reinterpret_cast<const f32x4*>(from + i + 4);
 #pragma unroll 4
-  for (int p = 1; p < parts; ++p) {
-    lo += *reinterpret_cast<const f32x4*>(from + (size_t)p * n + i);
-    hi += *reinterpret_cast<const f32x4*>(from + (size_t)p * n + i + 4);
-  }
-  if constexpr (sizeof(T) == 2) {
-    *reinterpret_cast<u32x4*>(C + i) = u32x4{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]),
-                                             pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
-  } else {
-    *reinterpret_cast<f32x4*>(C + i) = lo;
-    *reinterpret_cast<f32x4*>(C + i + 4) = hi;
+    for (int p = 1; p < parts; ++p) {
+      lo += *reinterpret_cast<const f32x4*>(from + (size_t)p * all + i);
+      hi += *reinterpret_cast<const f32x4*>(from + (size_t)p * all + i + 4);
+    }
+    if constexpr (sizeof(T) == 2) {
+      *reinterpret_cast<u32x4*>(C + i) = u32x4{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]),
+                                               pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
+    } else {
+      *reinterpret_cast<f32x4*>(C + i) = lo;
+      *reinterpret_cast<f32x4*>(C + i + 4) = hi;
+    }
   }
 }
+// (as many blocks a group as its planned rows have pieces of 2048, equally loaded)
 template <typename T>
-static int launch_split_sum(const void* scratch, int parts, int64_t n, void* c, hipStream_t stream) {
-  hipLaunchKernelGGL(split_sum_kernel<T>, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, stream,
-                     static_cast<const float*>(scratch), parts, n, static_cast<T*>(c));
+static int launch_split_sum(const void* scratch, int parts, int64_t planned, int N, const Groups& g, void* c,
+                            hipStream_t stream) {
+  const int64_t each = g.E * 2048ll, blocks = (planned * N + each - 1) / each;
+  hipLaunchKernelGGL(split_sum_kernel<T>, dim3((unsigned)blocks, (unsigned)g.E), dim3(256), 0, stream,
+                     static_cast<const float*>(scratch), parts, N, g, static_cast<T*>(c));
   return check_launch("split_sum");
 }
 
 // The product in `parts` parts (at least 2), whose sums go to scratch [parts][rows][N] f32, and their sum.
 template <int BLAYOUT, bool TWO_SRC>
 static int launch_split(const void* a, int K, const void* b0, const void* b1, const void* a2, void* c, int N,
-                        const Groups& g, int parts, void* scratch, const char* what, hipStream_t stream) {
+                        const Groups& g, int64_t planned, int parts, void* scratch, const char* what, hipStream_t stream) {
   using namespace dma;
   auto k = glu_gemm_bf16_dma_kernel<false, BLAYOUT, false, TWO_SRC, true, true>;
   static bool attr_set = false;  // benign race: setting the attribute is idempotent
@@ -442,7 +450,7 @@ static int launch_split(const void* a, int K, const void* b0, const void* b1, co
                      static_cast<const float*>(a2), static_cast<const float*>(nullptr),
                      static_cast<uint16_t*>(scratch), parts, K, N, g, (N + 255) / 256 * parts);
   if (int rc = check_launch(what)) return rc;
-  return launch_split_sum<uint16_t>(scratch, parts, (int64_t)g.dense_rows * N, c, stream);
+  return launch_split_sum<uint16_t>(scratch, parts, planned, N, g, c, stream);
 }
 
 // The bf16 throughput kernel pair (gate/up, then down); BLAYOUT as the kernel takes it, scales only
@@ -1012,23 +1020,23 @@ int fs2moe::swiglu_train(const void* x, const int32_t* row_map, const int32_t* c
 
 int fs2moe::gemm_sum(const void* a1, const void* b1, const void* a2, const void* b2, int32_t layout,
                      const int32_t* counts, const int32_t* offsets, int32_t E, int32_t K, int32_t N,
-                     int64_t rows, int32_t dtype, void* c, void* split_scratch, void* stream) {
+                     int64_t rows, int64_t planned, int32_t dtype, void* c, void* split_scratch, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
   const Groups g{E > 0 ? counts : nullptr, E > 0 ? offsets : nullptr, E > 0 ? E : 1, (int)rows};
-  const int parts = split_scratch != nullptr ? split_parts(2, rows, E, K, N, dtype) : 1;
+  const int parts = split_parts(2, planned, E, K, N, dtype);
   if (parts > 1 && dtype == FS2MOE_F32) {
     const int rc = layout == FS2MOE_W_IN_OUT
                        ? launch_f32<false, FS2MOE_W_IN_OUT>(a1, b1, b2, a2, split_scratch, nullptr, nullptr, K, N, g,
                                                             rows, "glu_gemm_f32<two sources, parts>", st, parts)
                        : launch_f32<false, FS2MOE_W_OUT_IN>(a1, b1, b2, a2, split_scratch, nullptr, nullptr, K, N, g,
                                                             rows, "glu_gemm_f32<two sources, parts>", st, parts);
-    return rc ? rc : launch_split_sum<float>(split_scratch, parts, rows * N, c, st);
+    return rc ? rc : launch_split_sum<float>(split_scratch, parts, planned, N, g, c, st);
   }
   if (parts > 1)
     return layout == FS2MOE_W_IN_OUT
-               ? launch_split<FS2MOE_W_IN_OUT, true>(a1, K, b1, b2, a2, c, N, g, parts, split_scratch,
+               ? launch_split<FS2MOE_W_IN_OUT, true>(a1, K, b1, b2, a2, c, N, g, planned, parts, split_scratch,
                                                      "glu_gemm_bf16_dma<two sources, parts>", st)
-               : launch_split<FS2MOE_W_OUT_IN, true>(a1, K, b1, b2, a2, c, N, g, parts, split_scratch,
+               : launch_split<FS2MOE_W_OUT_IN, true>(a1, K, b1, b2, a2, c, N, g, planned, parts, split_scratch,
                                                      "glu_gemm_bf16_dma<two sources, parts>", st);
   // (the second activation matrix travels in the first scale argument, the second weights in B1)
   if (dtype == FS2MOE_BF16)

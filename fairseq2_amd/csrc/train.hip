@@ -152,6 +152,7 @@ struct Carver {
 using Args = fs2moe_train_args;
 
 int64_t rows_of(const Args& a) { return FS2MOE_MAX_ROWS(a.T, a.K, a.E, a.tile_m); }
+int64_t planned_rows(const Args& a) { return fs2moe::planned_rows((int64_t)a.T * a.K, a.E); }
 int padded_experts(const Args& a) { return (a.E + 7) / 8 * 8; }
 // With up to 16 bf16 tokens the experts run as streams over their weights, as in the inference call, and
 // keep no products: the backward pass computes them again.
@@ -295,14 +296,14 @@ BackwardScratch carve_backward(const Args& a, void* base) {
   WgradRequest r[8];
   const int n = requests(a, Saved{}, b, r);
   // (the weight gradients' partial sums, after those of the rows' gradients)
-  int64_t part = wgrad_plan(r, n, a.E, R, T, a.act_dtype);
-  auto parts = [&](int64_t rows, int E, int F) {
-    const int n = split_parts(2, rows, E, F, a.D, a.act_dtype);
+  int64_t part = wgrad_plan(r, n, a.E, planned_rows(a), T, a.act_dtype);
+  auto parts = [&](int64_t rows, int64_t planned, int E, int F) {
+    const int n = split_parts(2, planned, E, F, a.D, a.act_dtype);
     const int64_t bytes = n > 1 ? (int64_t)n * rows * a.D * 4 : 0;
     part = bytes > part ? bytes : part;
   };
-  parts(R, a.E, a.F);
-  if (a.F_shared > 0) parts(T, 0, a.F_shared);
+  parts(R, planned_rows(a), a.E, a.F);
+  if (a.F_shared > 0) parts(T, T, 0, a.F_shared);
   b.part = c.take(part);
   b.total = c.used;
   return b;
@@ -463,8 +464,8 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
   }
   if (rc) return rc;
   if (want_x || (a->scale_input && a->d_router != nullptr))
-    if ((rc = gemm_sum(b.dg, a->w_gate, b.du, a->w_up, FS2MOE_W_OUT_IN, s.counts, s.offsets, E, F, D, R, dt, b.dxe,
-                       b.part, stream)))
+    if ((rc = gemm_sum(b.dg, a->w_gate, b.du, a->w_up, FS2MOE_W_OUT_IN, s.counts, s.offsets, E, F, D, R,
+                       planned_rows(*a), dt, b.dxe, b.part, stream)))
       return rc;
   // combine weights -> logits
   if (want_x || a->d_router != nullptr) {
@@ -479,14 +480,14 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
         (rc = fs2moe_swiglu_backward(s.gs, s.us, b.dhs, T, Fs, dt, b.dhs, b.dgs, b.dus, stream)))
       return rc;
     if (want_x && (rc = gemm_sum(b.dgs, a->shared_gate, b.dus, a->shared_up, FS2MOE_W_IN_OUT, nullptr, nullptr, 0, Fs,
-                                 D, T, dt, b.dx_shared, b.part, stream)))
+                                 D, T, T, dt, b.dx_shared, b.part, stream)))
       return rc;
   }
   // all weight gradients
   WgradRequest r[8];
   const int n = requests(*a, s, b, r);
   if (n > 0) {
-    (void)wgrad_plan(r, n, E, R, T, dt);
+    (void)wgrad_plan(r, n, E, planned_rows(*a), T, dt);
     if ((rc = wgrad_all(r, n, gradients_in_place(*a) ? s.perm : nullptr, s.counts, s.offsets, E, R, T, dt, b.part,
                         stream)))
       return rc;

@@ -248,6 +248,35 @@ def test_step_in_two_calls_against_its_stages(gpu_device, dtype, t, d, e, k, f, 
     assert torch.equal(some[4], grads[4])
 
 
+# Sizes at which a count of rows with their padding would cut the rows' gradients, or the router's and the shared
+# expert's weight gradients, into another number of parts.
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("t,d,e,k,f,f_shared,scale_input", [
+    (600, 264, 3, 1, 4104, 4104, True), (500, 264, 4, 1, 6152, 0, False), (700, 520, 4, 2, 4104, 0, False),
+    (1000, 512, 8, 2, 1408, 0, True), (2500, 520, 60, 4, 256, 512, False), (900, 512, 16, 2, 2048, 0, False),
+    (300, 512, 16, 2, 4096, 0, False), (3000, 640, 8, 1, 2048, 1024, True),
+])
+def test_gradients_do_not_depend_on_the_padding(gpu_device, dtype, t, d, e, k, f, f_shared, scale_input):
+    from fairseq2_amd import autograd as A
+
+    _say("padding", dtype, t, d, e, k, f, f_shared, scale_input)
+    g = torch.Generator().manual_seed(t)
+    mk = lambda *s, scale=1.0: (scale * torch.randn(*s, generator=g)).to(TORCH_DTYPE[dtype]).to(gpu_device)  # noqa: E731
+    x, dout, router = mk(t, d), mk(t, d), mk(d, e, scale=d**-0.5)
+    ws = [mk(e * d, f, scale=d**-0.5), mk(e * d, f, scale=d**-0.5), mk(e * f, d, scale=f**-0.5)]
+    ws += [mk(f_shared, d, scale=d**-0.5), mk(f_shared, d, scale=d**-0.5), mk(d, f_shared, scale=f_shared**-0.5)] \
+        if f_shared else [None] * 3
+    want = None
+    for tile_m in (16, 1, 128):
+        cfg = dict(num_experts=e, top_k=k, tile_m=tile_m, score_fn=_abi.SCORE_SIGMOID if scale_input else _abi.SCORE_SOFTMAX,
+                   renormalize=False, scale_input=scale_input, router_bias=None, norm_eps=None)
+        out, saved = A.layer_forward(x, None, router, *ws, None, cfg)
+        grads = A.layer_backward(x, router, *ws, None, cfg, saved, dout, (True,) * 9)
+        got = [out, *(v for v in grads if v is not None)]
+        want = want or got
+        assert [torch.equal(a, b) for a, b in zip(got, want)] == [True] * len(want), tile_m
+
+
 @pytest.mark.parametrize("t,d,e,k,skew,normed", [(192, 64, 3, 1, 0.0, False), (700, 264, 6, 2, 1.0, True),
                                                  (1500, 512, 64, 4, 2.0, False), (300, 1032, 8, 8, 0.0, True)])
 def test_copied_rows_give_the_gradients_of_rows_in_place(gpu_device, t, d, e, k, skew, normed):
