@@ -252,6 +252,7 @@ int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_
     }
     return FS2MOE_OK;
   };
+  const int64_t planned = fs2moe::planned_rows((int64_t)T * K, E);
   bool forked = false;
   // router, dispatch and the routed experts, with the shared expert forked off on the way
   auto routed_path = [&]() -> int {
@@ -287,17 +288,17 @@ int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_
     if (act_q) {
       // the token rows to block-scaled e4m3 once; both products read codes (the first through perm)
       if (int rc = fs2moe_mx_quantize(x, T, D, b.xq, b.xs, stream)) return rc;
-      return fs2moe_grouped_swiglu_w8a8(b.xq, b.xs, b.perm, b.counts, b.offsets, w_gate, w_up, w_down,
-                                        s_gate, s_up, s_down, E, D, F, T, b.max_rows, b.hq, b.hs, b.ye,
-                                        stream);
+      return fs2moe::grouped_swiglu_w8a8_planned(b.xq, b.xs, b.perm, b.counts, b.offsets, w_gate, w_up, w_down,
+                                                 s_gate, s_up, s_down, E, D, F, T, b.max_rows, planned, b.hq, b.hs,
+                                                 b.ye, stream);
     }
     if (scaled_stream)
       return fs2moe::grouped_swiglu_scaled_rows(x, b.perm, b.row_w, b.counts, b.offsets, w_gate, w_up,
                                                 w_down, E, D, F, b.max_rows, b.h, b.ye, T, stream);
     // (a token takes an expert at most once: with up to 16 tokens no expert has more rows than that)
-    return fs2moe_grouped_swiglu_rows(fused ? x : b.xe, fused ? b.perm : nullptr, b.counts, b.offsets,
-                                      w_gate, w_up, w_down, s_gate, s_up, s_down, E, D, F, b.max_rows,
-                                      act_dtype, w_dtype, b.h, b.ye, T <= 16 ? T : 0, stream);
+    return fs2moe::grouped_swiglu_planned(fused ? x : b.xe, fused ? b.perm : nullptr, b.counts, b.offsets,
+                                          w_gate, w_up, w_down, s_gate, s_up, s_down, E, D, F, b.max_rows,
+                                          planned, act_dtype, w_dtype, b.h, b.ye, T <= 16 ? T : 0, stream);
   };
   int rc_routed = routed_path();
   if (forked) {

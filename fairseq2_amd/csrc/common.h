@@ -249,6 +249,24 @@ int dispatch_with_row_weights(const int32_t* topk_idx, const float* topk_w, int3
                               int32_t E, int32_t tile_m, int64_t max_rows, int32_t* counts,
                               int32_t* offsets, int32_t* perm, int32_t* inv_perm, float* row_w,
                               void* stream);
+// The experts' rows that a plan goes by: as many as `pairs` rows take in blocks of 16, whatever granularity the buffers
+// have.  Where the plan decides how sums are cut, results then do not depend on the padding.
+inline int64_t planned_rows(int64_t pairs, int E) { return pairs + 15ll * E; }
+// fs2moe_grouped_swiglu_rows, fs2moe_grouped_swiglu_w8a8 and fs2moe_grouped_gemm for callers that know the planned rows
+// (the stage calls know the buffers' size alone, and plan by that).
+int grouped_swiglu_planned(const void* xe, const int32_t* row_map, const int32_t* counts, const int32_t* offsets,
+                           const void* w_gate, const void* w_up, const void* w_down, const float* s_gate,
+                           const float* s_up, const float* s_down, int32_t E, int32_t D, int32_t F, int64_t max_rows,
+                           int64_t planned, int32_t act_dtype, int32_t w_dtype, void* h, void* ye,
+                           int32_t rows_per_expert, void* stream);
+int grouped_swiglu_w8a8_planned(const void* xq, const void* xs, const int32_t* row_map, const int32_t* counts,
+                                const int32_t* offsets, const void* w_gate, const void* w_up, const void* w_down,
+                                const float* s_gate, const float* s_up, const float* s_down, int32_t E, int32_t D,
+                                int32_t F, int64_t x_rows, int64_t max_rows, int64_t planned, void* hq, void* hs,
+                                void* ye, void* stream);
+int grouped_gemm_planned(const void* a, const int32_t* row_map, const int32_t* counts, const int32_t* offsets,
+                         const void* b, int32_t b_layout, int32_t E, int32_t K, int32_t N, int64_t max_rows,
+                         int64_t planned, int32_t dtype, void* c, void* stream);
 // Whether the grouped SwiGLU pair of these sizes reads its rows through a row map (no gathered copy).
 bool swiglu_gathers_rows(int32_t act_dtype, int32_t w_dtype, int32_t D, int32_t F, int64_t max_rows);
 // Whether the grouped SwiGLU pair of these sizes runs on the kernels that stream the weights past a
@@ -269,10 +287,7 @@ int grouped_swiglu_scaled_rows(const void* x, const int32_t* row_map, const floa
 bool swiglu_train_applies(int32_t dtype, int32_t D, int32_t F, int64_t rows);
 int swiglu_train(const void* x, const int32_t* row_map, const int32_t* counts, const int32_t* offsets, int32_t E,
                  const void* w_gate, const void* w_up, const void* w_down, int32_t D, int32_t F,
-                 int64_t rows, int32_t dtype, void* g, void* u, void* h, void* y, void* stream);
-// The experts' rows that a plan goes by: as many as `pairs` rows take in blocks of 16, whatever granularity the buffers
-// have.  Where the plan decides how sums are cut, results then do not depend on the padding.
-inline int64_t planned_rows(int64_t pairs, int E) { return pairs + 15ll * E; }
+                 int64_t rows, int64_t planned, int32_t dtype, void* g, void* u, void* h, void* y, void* stream);
 // Into how many parts the sum over K of a product of `sources` pairs of matrices goes (1: it stays whole), by the
 // planned rows (E 0: the rows).
 int split_parts(int sources, int64_t planned, int E, int K, int N, int dtype);

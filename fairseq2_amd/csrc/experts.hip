@@ -197,9 +197,10 @@ static int launch_f32(const void* a, const void* b0, const void* b1, const void*
                       const char* what, hipStream_t stream, int parts = 1) {
   const int groups = g.counts ? g.E : 0;
   const int big_n = DUAL ? 64 : 128;
-  const bool small = f32t::small_tiles((rows_bound / 128 + groups + 1) * ((N + big_n - 1) / big_n),
-                                       groups ? rows_bound / groups : rows_bound) ||
-                     f32t::small_rounds(DUAL, rows_bound, groups, N, 256);
+  const int64_t planned = g.rows_to_plan(rows_bound);
+  const bool small = f32t::small_tiles((planned / 128 + groups + 1) * ((N + big_n - 1) / big_n),
+                                       groups ? planned / groups : planned) ||
+                     f32t::small_rounds(DUAL, planned, groups, N, 256);
   const int bm = small ? 64 : 128, bn = small ? 64 : big_n;
   const int64_t m_tiles = rows_bound / bm + groups + 1;
   const int nt = (N + bn - 1) / bn;
@@ -207,7 +208,7 @@ static int launch_f32(const void* a, const void* b0, const void* b1, const void*
     set_error("%s: grid too large", what);
     return FS2MOE_ERR_UNSUPPORTED;
   }
-  const bool eight = !DUAL && small && f32t::eight_waves(rows_bound, groups);
+  const bool eight = !DUAL && small && f32t::eight_waves(planned, groups);
   auto k = eight   ? glu_gemm_f32_kernel<DUAL, 1, 1, BLAYOUT, DUAL ? 4 : 8>
            : small ? glu_gemm_f32_kernel<DUAL, 1, 1, BLAYOUT, 4>
                    : glu_gemm_f32_kernel<DUAL, 2, DUAL ? 1 : 2, BLAYOUT, 4>;
@@ -292,7 +293,7 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
   // (tiles of 64 x 64 are counted in 31 bits too)
   const bool counted = (rows_bound / 64 + groups + 1) * ((N + 63) / 64) <= 0x7fffffffll;
   constexpr bool SINGLE = !DUAL && CAN_TAIL;
-  switch (counted ? half_tiles::pick(DUAL, SINGLE, rows_bound, groups, K, N, num_blocks) : 0) {
+  switch (counted ? half_tiles::pick(DUAL, SINGLE, g.rows_to_plan(rows_bound), groups, K, N, num_blocks) : 0) {
     case 1:
       if constexpr (SINGLE)
         return launch_half<64, 64, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
@@ -732,8 +733,8 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
                                const int32_t* offsets, const void* w_gate, const void* w_up,
                                const void* w_down, const float* s_gate, const float* s_up,
                                const float* s_down, int32_t E, int32_t D, int32_t F,
-                               int64_t max_rows, int32_t act_dtype, int32_t w_dtype, void* h,
-                               void* ye, int32_t rows_hint, void* stream,
+                               int64_t max_rows, int64_t planned, int32_t act_dtype, int32_t w_dtype,
+                               void* h, void* ye, int32_t rows_hint, void* stream,
                                const float* row_w = nullptr) {
   FS2_REQUIRE(xe && counts && offsets && w_gate && w_up && w_down && h && ye,
               "grouped_swiglu: null pointer");
@@ -768,7 +769,7 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
     // buffers are sized for.
     // (the streaming kernels build their item table with a thread per expert: up to 256 experts)
     if ((max_rows / E >= kFp8GemmMinRowsPerExpert || E > 256) && dma_offsets_fit(max_rows, D, F)) {
-      Groups g{counts, offsets, E, 0};
+      Groups g{counts, offsets, E, 0, (int)planned};
       return launch_dma_pair<dma::W_FP8_TILED>(xe, row_map, g, max_rows, w_gate, w_up, w_down, s_gate,
                                                s_up, s_down, D, F, h, ye, st);
     }
@@ -826,7 +827,7 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
     return FS2MOE_ERR_UNSUPPORTED;
   }
   if (max_rows == 0) return FS2MOE_OK;
-  Groups g{counts, offsets, E, 0};
+  Groups g{counts, offsets, E, 0, (int)planned};
   return launch_glu<FS2MOE_W_IN_OUT>(xe, row_map, g, max_rows, w_gate, w_up, w_down, D, F, act_dtype,
                                      h, ye, static_cast<hipStream_t>(stream), rows_hint, row_w);
 }
@@ -856,7 +857,7 @@ int fs2moe::grouped_swiglu_scaled_rows(const void* x, const int32_t* row_map, co
               "grouped_swiglu: internal: D=%d F=%d E=%d with %d rows an expert do not stream", D, F, E,
               rows_per_expert);
   return grouped_swiglu_impl(x, row_map, counts, offsets, w_gate, w_up, w_down, nullptr, nullptr,
-                             nullptr, E, D, F, max_rows, FS2MOE_BF16, FS2MOE_BF16, h, ye,
+                             nullptr, E, D, F, max_rows, 0, FS2MOE_BF16, FS2MOE_BF16, h, ye,
                              rows_per_expert, stream, row_w);
 }
 
@@ -867,7 +868,7 @@ extern "C" int fs2moe_grouped_swiglu(const void* xe, const int32_t* row_map, con
                                      int64_t max_rows, int32_t act_dtype, int32_t w_dtype, void* h,
                                      void* ye, void* stream) {
   return grouped_swiglu_impl(xe, row_map, counts, offsets, w_gate, w_up, w_down, s_gate, s_up, s_down,
-                             E, D, F, max_rows, act_dtype, w_dtype, h, ye, 0, stream);
+                             E, D, F, max_rows, 0, act_dtype, w_dtype, h, ye, 0, stream);
 }
 
 extern "C" int fs2moe_grouped_swiglu_rows(const void* xe, const int32_t* row_map,
@@ -878,7 +879,16 @@ extern "C" int fs2moe_grouped_swiglu_rows(const void* xe, const int32_t* row_map
                                           int64_t max_rows, int32_t act_dtype, int32_t w_dtype,
                                           void* h, void* ye, int32_t rows_per_expert, void* stream) {
   return grouped_swiglu_impl(xe, row_map, counts, offsets, w_gate, w_up, w_down, s_gate, s_up, s_down,
-                             E, D, F, max_rows, act_dtype, w_dtype, h, ye, rows_per_expert, stream);
+                             E, D, F, max_rows, 0, act_dtype, w_dtype, h, ye, rows_per_expert, stream);
+}
+
+int fs2moe::grouped_swiglu_planned(const void* xe, const int32_t* row_map, const int32_t* counts,
+                                   const int32_t* offsets, const void* w_gate, const void* w_up, const void* w_down,
+                                   const float* s_gate, const float* s_up, const float* s_down, int32_t E, int32_t D,
+                                   int32_t F, int64_t max_rows, int64_t planned, int32_t act_dtype, int32_t w_dtype,
+                                   void* h, void* ye, int32_t rows_per_expert, void* stream) {
+  return grouped_swiglu_impl(xe, row_map, counts, offsets, w_gate, w_up, w_down, s_gate, s_up, s_down, E, D, F,
+                             max_rows, planned, act_dtype, w_dtype, h, ye, rows_per_expert, stream);
 }
 
 // One grouped (or dense) GEMM, C = A @ B_e, on the kernels of the SwiGLU pair's second half.
@@ -911,10 +921,9 @@ static int launch_gemm(const void* a, const int32_t* row_map, const Groups& g, i
                                     "glu_gemm_f32<single>", stream);
 }
 
-extern "C" int fs2moe_grouped_gemm(const void* a, const int32_t* row_map, const int32_t* counts,
-                                   const int32_t* offsets, const void* b, int32_t b_layout,
-                                   int32_t E, int32_t K, int32_t N, int64_t max_rows, int32_t dtype,
-                                   void* c, void* stream) {
+int fs2moe::grouped_gemm_planned(const void* a, const int32_t* row_map, const int32_t* counts, const int32_t* offsets,
+                                 const void* b, int32_t b_layout, int32_t E, int32_t K, int32_t N, int64_t max_rows,
+                                 int64_t planned, int32_t dtype, void* c, void* stream) {
   FS2_REQUIRE(a && b && c, "grouped_gemm: null pointer");
   FS2_REQUIRE((counts == nullptr) == (offsets == nullptr), "grouped_gemm: counts without offsets");
   FS2_REQUIRE(E >= 1 && E <= FS2MOE_MAX_EXPERTS && (counts != nullptr || E == 1),
@@ -929,11 +938,18 @@ extern "C" int fs2moe_grouped_gemm(const void* a, const int32_t* row_map, const 
   FS2_REQUIRE(aligned16(a) && aligned16(b) && aligned16(c),
               "grouped_gemm: buffers must be 16-byte aligned");
   if (max_rows == 0) return FS2MOE_OK;
-  Groups g{counts, offsets, E, (int)max_rows};
+  Groups g{counts, offsets, E, (int)max_rows, (int)planned};
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (b_layout == FS2MOE_W_IN_OUT)
     return launch_gemm<FS2MOE_W_IN_OUT>(a, row_map, g, max_rows, b, K, N, dtype, c, st);
   return launch_gemm<FS2MOE_W_OUT_IN>(a, row_map, g, max_rows, b, K, N, dtype, c, st);
+}
+
+extern "C" int fs2moe_grouped_gemm(const void* a, const int32_t* row_map, const int32_t* counts,
+                                   const int32_t* offsets, const void* b, int32_t b_layout,
+                                   int32_t E, int32_t K, int32_t N, int64_t max_rows, int32_t dtype,
+                                   void* c, void* stream) {
+  return grouped_gemm_planned(a, row_map, counts, offsets, b, b_layout, E, K, N, max_rows, 0, dtype, c, stream);
 }
 
 extern "C" int fs2moe_dense_swiglu_keep(const void* x, const void* w_gate, const void* w_up,
@@ -996,10 +1012,10 @@ bool fs2moe::swiglu_train_applies(int32_t dtype, int32_t D, int32_t F, int64_t r
 int fs2moe::swiglu_train(const void* x, const int32_t* row_map, const int32_t* counts,
                          const int32_t* offsets, int32_t E,
                          const void* w_gate, const void* w_up, const void* w_down, int32_t D,
-                         int32_t F, int64_t rows, int32_t dtype, void* g, void* u, void* h, void* y,
-                         void* stream) {
+                         int32_t F, int64_t rows, int64_t planned, int32_t dtype, void* g, void* u, void* h,
+                         void* y, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const Groups grp{E > 0 ? counts : nullptr, E > 0 ? offsets : nullptr, E > 0 ? E : 1, (int)rows};
+  const Groups grp{E > 0 ? counts : nullptr, E > 0 ? offsets : nullptr, E > 0 ? E : 1, (int)rows, (int)planned};
   if (dtype == FS2MOE_BF16) {
     if (E > 0)
       return launch_dma_pair<FS2MOE_W_IN_OUT>(x, row_map, grp, rows, w_gate, w_up, w_down, nullptr, nullptr,
@@ -1022,7 +1038,7 @@ int fs2moe::gemm_sum(const void* a1, const void* b1, const void* a2, const void*
                      const int32_t* counts, const int32_t* offsets, int32_t E, int32_t K, int32_t N,
                      int64_t rows, int64_t planned, int32_t dtype, void* c, void* split_scratch, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const Groups g{E > 0 ? counts : nullptr, E > 0 ? offsets : nullptr, E > 0 ? E : 1, (int)rows};
+  const Groups g{E > 0 ? counts : nullptr, E > 0 ? offsets : nullptr, E > 0 ? E : 1, (int)rows, (int)planned};
   const int parts = split_parts(2, planned, E, K, N, dtype);
   if (parts > 1 && dtype == FS2MOE_F32) {
     const int rc = layout == FS2MOE_W_IN_OUT

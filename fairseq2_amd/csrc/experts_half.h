@@ -71,8 +71,8 @@ constexpr uint32_t NOWHERE = 0xfffffff0u;      // an offset past any buffer's en
 //   64 of 23, D 2944, F 1840             377 against 394, 400      (memory)
 // single: the launch is one product of bf16 matrices.
 inline int pick(bool dual, bool single, int64_t rows, int groups, int K, int N, int cus) {
-  // The experts' rows, which only the device knows, as the buffers' size has them: less what blocks of 16 pad
-  // them by, equally loaded.
+  // Of the experts' rows only the device knows how they are spread: the planned ones (Groups), less what blocks of 16
+  // pad them by, equally loaded.
   const int64_t real = rows > 15ll * groups ? rows - 15ll * groups : rows;
   const int64_t each = groups ? real / groups : real;
   auto tiles = [&](int bm, int bn) -> int64_t {

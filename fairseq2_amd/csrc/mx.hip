@@ -84,13 +84,12 @@ extern "C" int fs2moe_grouped_swiglu_w8a8_supported(int32_t D, int32_t F, int64_
              : 0;
 }
 
-extern "C" int fs2moe_grouped_swiglu_w8a8(const void* xq, const void* xs, const int32_t* row_map,
-                                          const int32_t* counts, const int32_t* offsets,
-                                          const void* w_gate, const void* w_up, const void* w_down,
-                                          const float* s_gate, const float* s_up,
-                                          const float* s_down, int32_t E, int32_t D, int32_t F,
-                                          int64_t x_rows, int64_t max_rows, void* hq, void* hs,
-                                          void* ye, void* stream) {
+int fs2moe::grouped_swiglu_w8a8_planned(const void* xq, const void* xs, const int32_t* row_map, const int32_t* counts,
+                                        const int32_t* offsets, const void* w_gate, const void* w_up,
+                                        const void* w_down, const float* s_gate, const float* s_up,
+                                        const float* s_down, int32_t E, int32_t D, int32_t F, int64_t x_rows,
+                                        int64_t max_rows, int64_t planned, void* hq, void* hs, void* ye,
+                                        void* stream) {
   using namespace mx;
   FS2_REQUIRE(xq && xs && counts && offsets && w_gate && w_up && w_down && s_gate && s_up && s_down &&
                   hq && hs && ye,
@@ -143,7 +142,7 @@ extern "C" int fs2moe_grouped_swiglu_w8a8(const void* xq, const void* xs, const 
       return FS2MOE_ERR_UNSUPPORTED;
     }
   }
-  Groups g{counts, offsets, E, 0};
+  Groups g{counts, offsets, E, 0, (int)planned};
   // Few tiles: the smaller tiles of experts_half.h (the same bits).
   auto half = [&](auto bm_c, auto dual_c, const void* a, const void* as, const int32_t* map, int K, const void* b0,
                   const void* b1, const float* s0, const float* s1, void* c, void* cs, int N, int64_t a_rows,
@@ -173,7 +172,7 @@ extern "C" int fs2moe_grouped_swiglu_w8a8(const void* xq, const void* xs, const 
   using I128 = std::integral_constant<int, 128>;
   const bool counted = (max_rows / 64 + E + 1) * (((D > F ? D : F) + 63) / 64) <= 0x7fffffffll;
   auto pick = [&](bool dual, int K, int N) {
-    return counted ? half_tiles::pick(dual, false, max_rows, E, K / 2, N, num_blocks) : 0;
+    return counted ? half_tiles::pick(dual, false, g.rows_to_plan(max_rows), E, K / 2, N, num_blocks) : 0;
   };
   const char* what = "glu_gemm_mx<gate,up>";
   int rc;
@@ -205,4 +204,15 @@ extern "C" int fs2moe_grouped_swiglu_w8a8(const void* xq, const void* xs, const 
                      static_cast<const uint8_t*>(nullptr), s_down, static_cast<const float*>(nullptr),
                      ye, static_cast<uint8_t*>(nullptr), D, F, D, g, nt2, (int)max_rows, 0);
   return check_launch(what);
+}
+
+extern "C" int fs2moe_grouped_swiglu_w8a8(const void* xq, const void* xs, const int32_t* row_map,
+                                          const int32_t* counts, const int32_t* offsets,
+                                          const void* w_gate, const void* w_up, const void* w_down,
+                                          const float* s_gate, const float* s_up,
+                                          const float* s_down, int32_t E, int32_t D, int32_t F,
+                                          int64_t x_rows, int64_t max_rows, void* hq, void* hs,
+                                          void* ye, void* stream) {
+  return grouped_swiglu_w8a8_planned(xq, xs, row_map, counts, offsets, w_gate, w_up, w_down, s_gate, s_up, s_down, E, D,
+                                     F, x_rows, max_rows, 0, hq, hs, ye, stream);
 }

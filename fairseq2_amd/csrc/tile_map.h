@@ -10,6 +10,10 @@ struct Groups {
   const int32_t* offsets;  // [E + 1] first row of each expert
   int E;
   int dense_rows;
+  // host: the planned rows (common.h) where the caller knows them, else 0 and the buffers' size stands for them; the
+  // choice of tiles goes by them, while grids and addresses go by the buffers
+  int planned = 0;
+  int64_t rows_to_plan(int64_t bound) const { return counts != nullptr && planned > 0 ? planned : bound; }
 };
 
 // Finds the (expert, row range) of m-tile `mt`.  All 256 threads of the block must call it.

@@ -375,17 +375,18 @@ extern "C" int fs2moe_train_forward(const fs2moe_train_args* a, void* stream) {
   const bool mapped = in_token_order(*a);
   void* ye = s.ye != nullptr ? s.ye : f.ye;
   if (s.g == nullptr)
-    rc = fs2moe_grouped_swiglu_rows(s.xe, nullptr, s.counts, s.offsets, a->w_gate, a->w_up, a->w_down, nullptr,
-                                    nullptr, nullptr, a->E, a->D, a->F, R, a->act_dtype, a->act_dtype, f.h, ye,
-                                    a->T, stream);
+    rc = grouped_swiglu_planned(s.xe, nullptr, s.counts, s.offsets, a->w_gate, a->w_up, a->w_down, nullptr, nullptr,
+                                nullptr, a->E, a->D, a->F, R, planned_rows(*a), a->act_dtype, a->act_dtype, f.h, ye,
+                                a->T, stream);
   else
     rc = swiglu_train(mapped ? x : s.xe, mapped ? s.perm : nullptr, s.counts, s.offsets, a->E, a->w_gate, a->w_up,
-                      a->w_down, a->D, a->F, R, a->act_dtype, s.g, s.u, mapped ? s.h : f.h, ye, stream);
+                      a->w_down, a->D, a->F, R, planned_rows(*a), a->act_dtype, s.g, s.u, mapped ? s.h : f.h, ye,
+                      stream);
   if (rc) return rc;
   const void* base = nullptr;
   if (a->F_shared > 0) {
     rc = swiglu_train(x, nullptr, nullptr, nullptr, 0, a->shared_gate, a->shared_up, a->shared_down, a->D,
-                      a->F_shared, a->T, a->act_dtype, s.gs, s.us, f.hs, a->out, stream);
+                      a->F_shared, a->T, a->T, a->act_dtype, s.gs, s.us, f.hs, a->out, stream);
     if (rc) return rc;
     base = a->out;
   }
@@ -438,15 +439,16 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
   if (b.dye != nullptr && (rc = gather(a->dout, b.dye, !a->scale_input && !mapped))) return rc;
   if (b.xe != nullptr && (rc = gather(x, b.xe, false))) return rc;
   // the experts: dh, then h, dg and du, then the rows' gradient
-  if ((rc = fs2moe_grouped_gemm(b.dye != nullptr ? b.dye : a->dout, b.dye != nullptr ? nullptr : s.perm, s.counts,
-                                s.offsets, a->w_down, FS2MOE_W_OUT_IN, E, D, F, R, dt, b.dh, stream)))
+  const int64_t planned = planned_rows(*a);
+  if ((rc = grouped_gemm_planned(b.dye != nullptr ? b.dye : a->dout, b.dye != nullptr ? nullptr : s.perm, s.counts,
+                                 s.offsets, a->w_down, FS2MOE_W_OUT_IN, E, D, F, R, planned, dt, b.dh, stream)))
     return rc;
   const void *g = s.g, *u = s.u;
   if (g == nullptr) {
-    if ((rc = fs2moe_grouped_gemm(s.xe, nullptr, s.counts, s.offsets, a->w_gate, FS2MOE_W_IN_OUT, E, D, F, R, dt, b.dg,
-                                  stream)) ||
-        (rc = fs2moe_grouped_gemm(s.xe, nullptr, s.counts, s.offsets, a->w_up, FS2MOE_W_IN_OUT, E, D, F, R, dt, b.du,
-                                  stream)))
+    if ((rc = grouped_gemm_planned(s.xe, nullptr, s.counts, s.offsets, a->w_gate, FS2MOE_W_IN_OUT, E, D, F, R, planned,
+                                   dt, b.dg, stream)) ||
+        (rc = grouped_gemm_planned(s.xe, nullptr, s.counts, s.offsets, a->w_up, FS2MOE_W_IN_OUT, E, D, F, R, planned,
+                                   dt, b.du, stream)))
       return rc;
     g = b.dg;
     u = b.du;
@@ -464,8 +466,8 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
   }
   if (rc) return rc;
   if (want_x || (a->scale_input && a->d_router != nullptr))
-    if ((rc = gemm_sum(b.dg, a->w_gate, b.du, a->w_up, FS2MOE_W_OUT_IN, s.counts, s.offsets, E, F, D, R,
-                       planned_rows(*a), dt, b.dxe, b.part, stream)))
+    if ((rc = gemm_sum(b.dg, a->w_gate, b.du, a->w_up, FS2MOE_W_OUT_IN, s.counts, s.offsets, E, F, D, R, planned,
+                       dt, b.dxe, b.part, stream)))
       return rc;
   // combine weights -> logits
   if (want_x || a->d_router != nullptr) {
@@ -487,7 +489,7 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
   WgradRequest r[8];
   const int n = requests(*a, s, b, r);
   if (n > 0) {
-    (void)wgrad_plan(r, n, E, planned_rows(*a), T, dt);
+    (void)wgrad_plan(r, n, E, planned, T, dt);
     if ((rc = wgrad_all(r, n, gradients_in_place(*a) ? s.perm : nullptr, s.counts, s.offsets, E, R, T, dt, b.part,
                         stream)))
       return rc;
