@@ -321,18 +321,25 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
 }
 
 // Single products of few tiles over a long K: into how many parts the sum over K goes (1: it stays whole), each a
-// round of tiles of its own.  The throughput kernel's time, in ns per unit of 64 k: a full round 2000, one that has n
-// of the chip's CUs at work 800 + 1200 n / 256 (40 tiles 1.0 us, 144 1.6, 192 1.8), neither faster than the operands
-// come in (4 TB/s); the smaller tiles' 330, 450 and 650 of one round.  Against that the parts' sums on their way out
-// and in again, and a launch.  us for two sources, whole (with the smaller tiles where they are taken) and in parts:
-//   16 experts of 424 rows, K 13800, N 640    593, 367 (5)    8 of 427, K 9472, N 2112   464, 348 (3)
-//   8 of 457, K 10560, N 512                  151, 105 (8)    8 of 880, K 8768, N 1216   443, 334 (3)
-//   16 of 214, K 5568, N 1280                 180, 163 (2)    8 of 920, K 2800, N 576     89,  91 (2)
-// and where it says 1: 16 of 552, K 7040, N 1088 365, 370 (3); 60 of 240, K 1600, N 1216 159, 202 (2); 16 of 375,
-// K 1368, N 1024 52, 63 (2).  A constant number of CUs, as the scratch is sized in calls that touch no device.
+// round of tiles of its own.  The throughput kernel's time, in ns per unit of 64 k: a full round of heavy tiles 1950;
+// a last one 1420 to 1820 with the CUs at work, a light tile counted as 0.6 of a heavy one; or, where it is dealt as
+// halves, 1200 to 1400 with the light tiles (a whole launch of halves up to K 6000 1100), of light tiles alone 1000 to
+// 1350; none faster than the operands come in (5 TB/s for both sources).  The smaller tiles' 300, 460 and 580 of one
+// round.  Against that the parts' sums on their way out and in again, and a launch.  The figures are those that lose
+// least over 229 products of 8 to 128 experts or one group, loaded evenly, at random or by a popularity law.  226 others
+// take, whole, 1.094 times as long as by this rule, and 1.130 times as long as in the best number of parts; eleven are
+// slower than whole by this rule, eight of them loaded by the law, which the host does not know.  us for two sources,
+// whole (with the smaller tiles where they are taken) and in parts:
+//   16 experts of 424 rows, K 13800, N 640    523, 360 (5)    8 of 427, K 9472, N 2112   439, 335 (3)
+//   8 of 457, K 10560, N 512                  197, 104 (8)    8 of 880, K 8768, N 1216   427, 341 (3)
+//   16 of 214, K 5568, N 1280                 181, 140 (3), with two 164
+// and where it says 1: 16 of 552, K 7040, N 1088 355, 365 (3); 60 of 240, K 1600, N 1216 160, 192 (2); 16 of 375,
+// K 1368, N 1024 46, 56 (2); 8 of 920, K 2800, N 576 88, 91 (2) and 87 (4).  A constant number of CUs, as the scratch is
+// sized in calls that touch no device.
 // f32 tiles (experts_f32.h): a CU multiplies no faster with several, so a part's time is its rounds of tiles, 0.53 us
 // per 32 k and tile of 64 x 64.  8 experts of 250 rows, two sources of K 1408, N 512 (280 tiles): the step of 1000 tokens
-// 394 -> 372 us in four parts.
+// 394 -> 372 us in four parts, its loads at random (with 250 rows each the product is one round whole: 51 us, 53 in
+// parts).  147 products, whole, 1.13 times as long as by this rule and 1.24 as in the best number of parts.
 int split_parts(int sources, int64_t planned, int E, int K, int N, int dtype) {
   constexpr int CUS = 256, MIN_UNITS = 16;
   constexpr int64_t MAX_BYTES = 256ll << 20;
@@ -364,23 +371,32 @@ int split_parts(int sources, int64_t planned, int E, int K, int N, int dtype) {
   const int64_t heavy = (each / dma::BM + (rest > dma::LIGHT_ROWS)) * groups * nt;
   const int64_t light = (rest > 0 && rest <= dma::LIGHT_ROWS ? groups : 0) * nt;
   const int64_t units = (int64_t)sources * ((K + 63) / 64);
-  const int64_t memory = sources * ((groups < real ? groups : real) * K * N + planned * K) / 2000;  // ns
+  const int64_t memory = sources * ((groups < real ? groups : real) * K * N + planned * K) / 2500;  // ns
   auto whole = [&](int64_t parts) {
-    const int64_t n = parts * (10 * heavy + 6 * light) / 10, left = n % CUS;
-    const int64_t t = (units + parts - 1) / parts * (n / CUS * 2000 + (left ? 800 + 1200 * left / CUS : 0));
+    const int64_t left = heavy * parts % CUS, lights = light * parts, halves = 2 * left + lights;
+    int64_t t = heavy * parts / CUS * 1950;  // of a unit
+    if (halves > CUS) {
+      const int64_t n = left + lights * 6 / 10;
+      t += n / CUS * 1950 + (n % CUS ? 1420 + 400 * (n % CUS) / CUS : 0);
+    } else if (left > 0) {
+      t += (heavy < CUS && lights == 0 && parts == 1 && K < 6000 ? 1100 : 1200) + 200 * lights / CUS;
+    } else if (lights > 0) {
+      t += 1000 + 350 * lights / CUS;
+    }
+    t *= (units + parts - 1) / parts;
     return t > memory ? t : memory;
   };
   const int small = half_tiles::pick(false, true, planned, E, K, N, CUS);
   int64_t base = whole(1);
   if (small != 0) {
-    const int64_t t = units * (small == 1 ? 330 : small == 2 ? 450 : 650);
+    const int64_t t = units * (small == 1 ? 300 : small == 2 ? 460 : 580);
     base = (t > memory ? t : memory) + 4000;
   }
   int best = 1;
   for (int parts = 2; parts <= 16 && units / parts >= MIN_UNITS && parts * part_bytes <= MAX_BYTES; ++parts) {
-    const int64_t t = whole(parts) + parts * planned * N / 1000 + 6000;
-    // (worth 5 % by these figures, to be taken at all)
-    if (best == 1 ? t * 20 < base * 19 : t < base) {
+    const int64_t t = whole(parts) + parts * planned * N / 665 + 5000;
+    // (worth 7.5 % by these figures, to be taken at all)
+    if (best == 1 ? t * 40 < base * 37 : t < base) {
       best = parts;
       base = t;
     }

@@ -203,7 +203,7 @@ def _exact_step(x, router, ws, norm_w, cfg, dout, idx, xn_device):
     (1100, 1024, 4, 2, 1032, 1024, 3.0, True, False),
     # rows in token order: the fewest rows that do not stream; most experts without rows, F past one piece a lane
     (17, 64, 3, 1, 40, 0, 0.0, False, False), (40, 72, 64, 2, 1032, 0, 3.0, False, True),
-    # few tiles over a long K: the rows' gradients in parts (8 and 8, 12, 8 and 12, 16 and 16, 7 and 13), tiles of
+    # few tiles over a long K: the rows' gradients in parts (8 and 8, 12, 7 and 12, 16 and 16, 7 and 15), tiles of
     # up to 128 rows and more, fewer columns than a tile has and a few more, the last part shorter than the others
     (600, 264, 3, 1, 4104, 4104, 0.0, True, False), (500, 264, 4, 1, 6152, 0, 3.0, False, False),
     (700, 520, 4, 2, 4104, 6152, 0.0, False, True), (390, 72, 3, 1, 8200, 8200, 1.0, True, False),
