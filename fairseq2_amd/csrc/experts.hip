@@ -307,11 +307,17 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
                                                                     num_blocks, stream);
   }
   // The variant for any K also stores rows that do not begin on lines as L2 wants them, which counts for more than its
-  // selects at every load where stores are a large part of the work: three results (the training step of 3395 tokens,
-  // top-2 of 16, D 640, F 13800 2049 -> 1967 us, of 3001, D 1024, F 1368 542 -> 540), or few units (forward over 8803
-  // tokens, top-2 of 16, D 4928, F 7768 3950 -> 3970, so not there).
+  // selects at every load where stores are a large part of the work: three results, or few units.  us with the variant
+  // for whole units and with this one, 8 experts of 2000 rows, N 2728 and 60 of 300, N 712:
+  //   K                            512        1024       1536       2048       3072       4096       5120
+  //   three results (of 1500, pair) 165, 154  245, 240   354, 338   419, 398   595, 585   739, 725   913, 911
+  //                                 82,  77   136, 130   187, 180   244, 240   349, 352   456, 459   564, 563
+  //   gate/up (pair)               151, 149   249, 248   371, 372   468, 474   686, 696   916, 927  1133, 1154
+  //                                 74,  73   127, 123   182, 175   234, 230   346, 345   455, 458   569, 572
+  //   down's transpose              64,  60    98,  95   132, 128   168, 166   237, 239   317, 316   394, 393
+  //                                 28,  29    45,  45    65,  62    81,  81   120, 124   155, 166   196, 205
   const bool off_lines =
-      off_lines_variant(DUAL, BLAYOUT, TWO_SRC, CAN_TAIL) && N % 64 != 0 && (KEEP_GU || K <= 1024);
+      off_lines_variant(DUAL, BLAYOUT, TWO_SRC, CAN_TAIL) && N % 64 != 0 && (KEEP_GU || K <= 1536);
   hipLaunchKernelGGL(K % (2 * BK) == 0 && !off_lines ? whole : tail, dim3((unsigned)num_blocks), dim3(NWAVES * 64),
                      SMEM_BYTES, stream, static_cast<const uint16_t*>(a), row_map, K,
                      static_cast<const uint16_t*>(b0), static_cast<const uint16_t*>(b1),
