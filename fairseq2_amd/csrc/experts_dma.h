@@ -65,9 +65,9 @@ constexpr int RING_BYTES = 2 * UNIT_BYTES;         // 128 KB
 #define FS2MOE_GEMM_BAND 8
 #endif
 constexpr int BAND = FS2MOE_GEMM_BAND;  // row blocks per band of the tile order (see locate)
-// Where no expert has more rows than this, one of 257 to 384 has its rows cut into two tiles of about as many (the
-// first a multiple of 64) instead of 256 and the rest: see the tile tables.
-constexpr int EVEN_ROWS = 2 * BM;
+// Where no expert has more rows than EVEN_ROWS, one of 257 to 384 has its rows cut into two tiles of EVEN_FIRST and the
+// rest instead of 256 and the rest: see the tile tables.
+constexpr int EVEN_ROWS = 2 * BM, EVEN_FIRST = 192;
 constexpr int LIGHT_ROWS = 128;  // a last tile of at most this many rows costs about half a tile
 // after the ring: heavy-tile prefix [E + 1], light-tile prefix [E + 1], counts [E], offsets [E], rows of a heavy tile [E], each
 // sized for the library's limit on E
@@ -190,11 +190,17 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
   // Every block then gets the same number of heavy tiles to within one, the light tiles fill up the
   // blocks that got one heavy tile fewer, and the 32 tiles in flight on an XCD are neighbours in the
   // list, which share activation rows (same rows, next channels) and weights (same expert).
-  // The light tile of an expert with heavy ones reads its weights a second time, at another time.  Two tiles of about
-  // as many rows are neighbours in the list instead: they walk K side by side on one XCD, and the second finds the
-  // weights in L2.  128 experts of 270, 310, 350 and 384 rows, K 2048, N 1536: 323, 329, 356, 360 -> 317, 314, 325, 329
-  // us (257: 362, 368).  Not with experts of many rows beside them, whose heavy tiles hide light ones: 8192 tokens of
-  // the layer with D 2048, F 768, top-8 of 128 by a popularity law 720 us as it is, 728 with even tiles.
+  // The light tile of an expert with heavy ones reads its weights a second time, at another time.  Two tiles of 192 rows
+  // and the rest are neighbours in the list instead: they walk K side by side on one XCD, and the second finds the
+  // weights in L2.  Up to 320 rows the second takes half of the first's products, as the light tile of 256 rows; the
+  // grid is even, so that without locate's exchange every other block would have the long ones alone.  us of the SwiGLU
+  // pair with light tiles, without and with that exchange, every expert of 257, 300, 350 and 384 rows:
+  //   128 of D 2048, F 768    477, 490, 441   491, 489, 449   535, 508, 502   544, 512, 512
+  //   128 of D 2048, F 1536   920, 981, 847   943, 982, 859  1017, 964, 959  1034, 972, 967
+  //   60 of D 1280, F 704     167, 150, 142   (304) 169, 151, 142     (352) 174, 160, 159
+  // and at random, 262 rows on average, the first 428, 433, 419; its training step of 4096 tokens 2217, 2153, 2153.  Not
+  // with experts of many rows beside them, whose heavy tiles hide light ones: 65536 rows by a popularity law of exponent
+  // 0.6 over the first 677 us as it is, 688 with even tiles.
   {
     __shared__ int s_wave_tot[2][NWAVES];
     const int cnt = dense ? (tid == 0 ? g.dense_rows : 0) : (tid < E ? g.counts[tid] : 0);
@@ -239,7 +245,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
       s_hstart[tid] = hincl - heavy;
       s_lstart[tid] = lincl - light;
       s_counts[tid] = cnt;
-      s_rows[tid] = even && cnt > BM ? ((cnt + 1) / 2 + 63) & ~63 : BM;
+      s_rows[tid] = even && moved ? EVEN_FIRST : BM;
       s_offsets[tid] = dense ? 0 : g.offsets[tid];
     }
     if (tid == E - 1) {
@@ -320,7 +326,11 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
       const int gm = left < BAND ? left : BAND;
       nt = t / gm;
       const int rows = __builtin_amdgcn_readfirstlane(s_rows[found]);
-      first_row = (b * BAND + t - nt * gm) * rows;
+      int block = b * BAND + t - nt * gm;
+      // (of an even pair the first tile is the longer one: every other round of the deal has them the other way round, so
+      // that no block gets long ones alone)
+      if (rows != BM) block ^= (h0 * n_tiles + (l & ~1)) / grid & 1;
+      first_row = block * rows;
       last_row = cnt < first_row + rows ? cnt : first_row + rows;
     }
     if (half >= 0) {

@@ -102,6 +102,8 @@ def _groups(rows_per_expert, pad=16):
     ([257, 270, 320, 384, 385, 512, 129, 100, 64, 300, 0, 256, 1, 383, 330, 290], 128, 2048),
     ([257, 270, 320, 384, 385, 512, 129, 100, 64, 300, 0, 256, 1, 383, 330, 290], 72, 1992),
     ([257, 270, 320, 384, 385, 513, 129, 100, 64, 300, 0, 256, 1, 383, 330, 290], 64, 2048),
+    # several rounds of the deal, whose even pairs begin with either tile, at any place in a round
+    ([257, 384, 200, 300, 320, 130, 321, 0, 290, 260] * 6, 64, 1544),
 ])
 def test_grouped_gemm_both_orientations(gpu_device, dtype, layout, rows, k, n):
     _say("grouped_gemm", dtype, layout, rows, k, n)
