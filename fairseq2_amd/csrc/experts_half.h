@@ -104,6 +104,9 @@ inline int pick(bool dual, bool single, int64_t rows, int groups, int K, int N, 
 // 16 bytes per lane from a buffer to LDS, lane l's to lds + 16 l.  Written out because the compiler, which cannot
 // tell the ring's stages apart, would wait for every load in flight before each LDS read.  The caller waits
 // (vmcnt) in front of the barrier that hands the stage over.  BYTES 4: lane l's four to lds + 4 l.
+// (m0 is named because the other kernels' loads to LDS set it as well; the compiler warns that it reserves it.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 template <int BYTES>
 __device__ __forceinline__ void buffer_to_lds(const void* base, uint32_t off, uint32_t lds) {
   const uint64_t b = (uint64_t)base;
@@ -111,12 +114,13 @@ __device__ __forceinline__ void buffer_to_lds(const void* base, uint32_t off, ui
   if constexpr (BYTES == 16)
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc),
                  "s"(lds)
-                 : "memory");
+                 : "memory", "m0");
   else
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc),
                  "s"(lds)
-                 : "memory");
+                 : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 // The block-scaled e4m3 kernels' further operands: scale bytes of the rows in and (gate/up) out, k-group major
 // ([K / 128][rows][4]), and how many rows each array has.
