@@ -1468,7 +1468,8 @@ static int norm_weight_slabs(int64_t rows) {
 
 extern "C" int64_t fs2moe_rms_norm_backward_workspace_bytes(int32_t T, int32_t D) {
   if (T < 0 || D < 1) return -1;
-  // rstd [T] (padded to 16 bytes), then the slabs' partial sums
+  // rstd [T] (padded to 16 bytes), then the slabs' partial sums.  (rstd is for rows past the one pass alone; how long
+  // those are depends on the type, which this size does not)
   return ((int64_t)T * 4 + 15) / 16 * 16 + (int64_t)norm_weight_slabs(T) * D * 4;
 }
 
