@@ -279,6 +279,46 @@ def test_gradients_do_not_depend_on_the_padding(gpu_device, dtype, t, d, e, k, f
         assert [torch.equal(a, b) for a, b in zip(got, want)] == [True] * len(want), tile_m
 
 
+# Sums over K in parts (8 in bf16, 5 in f32) and whole on small tiles, both past K in their last unit: what is infinite
+# or no number stays in its row, with its expert.
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("t,f", [(600, 4104), (100, 200)])
+def test_infinities_and_nan_stay_in_their_rows(gpu_device, dtype, t, f):
+    from fairseq2_amd import autograd as A
+
+    _say("poisoned rows", dtype, t, f)
+    d, e = 264, 3
+    g = torch.Generator().manual_seed(t)
+    mk = lambda *s, scale=1.0: (scale * torch.randn(*s, generator=g)).to(TORCH_DTYPE[dtype]).to(gpu_device)  # noqa: E731
+    x, dout, router = mk(t, d), mk(t, d), mk(d, e, scale=d**-0.5)
+    ws = [mk(e * d, f, scale=d**-0.5), mk(e * d, f, scale=d**-0.5), mk(e * f, d, scale=f**-0.5)]
+    ws += [mk(f, d, scale=d**-0.5), mk(f, d, scale=d**-0.5), mk(d, f, scale=f**-0.5)]
+    cfg = dict(num_experts=e, top_k=1, tile_m=16, score_fn=_abi.SCORE_SIGMOID, renormalize=False, scale_input=True,
+               router_bias=None, norm_eps=None)
+
+    def dx_of(ws, dout):
+        _, saved = A.layer_forward(x, None, router, *ws, None, cfg)
+        return A.layer_backward(x, router, *ws, None, cfg, saved, dout, (True,) * 9)[0]
+
+    clean = dx_of(ws, dout)
+    assert torch.isfinite(clean.float()).all()
+    for value in (float("inf"), float("nan")):
+        rows = [0, 7, t // 2, t - 1]
+        bad = dout.clone()
+        bad[rows, 5] = value
+        got = dx_of(ws, bad)
+        keep = torch.ones(t, dtype=torch.bool, device=gpu_device)
+        keep[rows] = False
+        assert torch.equal(got[keep], clean[keep]) and not torch.isfinite(got[rows].float()).any(), value
+        of_expert = (x.float() @ router.float()).argmax(1) == 1
+        poisoned = [w.clone() for w in ws]
+        for w in poisoned[:2]:
+            w[d : 2 * d] = value
+        got = dx_of(poisoned, dout)
+        assert torch.equal(got[~of_expert], clean[~of_expert]), value
+        assert not torch.isfinite(got[of_expert].float()).any(), value
+
+
 @pytest.mark.parametrize("t,d,e,k,skew,normed", [(192, 64, 3, 1, 0.0, False), (700, 264, 6, 2, 1.0, True),
                                                  (1500, 512, 64, 4, 2.0, False), (300, 1032, 8, 8, 0.0, True)])
 def test_copied_rows_give_the_gradients_of_rows_in_place(gpu_device, t, d, e, k, skew, normed):
