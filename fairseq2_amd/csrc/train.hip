@@ -302,8 +302,9 @@ BackwardScratch carve_backward(const Args& a, void* base) {
     const int64_t bytes = n > 1 ? (int64_t)n * rows * a.D * 4 : 0;
     part = bytes > part ? bytes : part;
   };
-  parts(R, planned_rows(a), a.E, a.F);
-  if (a.F_shared > 0) parts(T, T, 0, a.F_shared);
+  const bool want_x = a.dx != nullptr || a.d_norm_weight != nullptr;
+  if (want_x || (a.scale_input && a.d_router != nullptr)) parts(R, planned_rows(a), a.E, a.F);
+  if (want_x && a.F_shared > 0) parts(T, T, 0, a.F_shared);
   b.part = c.take(part);
   b.total = c.used;
   return b;

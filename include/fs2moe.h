@@ -497,6 +497,13 @@ int fs2moe_copy(const void* src, void* dst, int64_t bytes, void* stream);
  * the backward pass (backward 1, else 0), the gradients whose pointers are set (-1: sizes these calls
  * do not take -- bf16 matrices of 4 GB and more).  Weights, rows, results and gradients are 16-byte
  * aligned, x with a norm only where its own gradient or the norm weight's is taken.
+ *
+ * Results do not depend on tile_m.  Where the products that give the rows'
+ * gradients (dxe = dg Wg^T + du Wu^T, and the shared expert's) have few tiles over a long inner size, their
+ * sums are taken in parts, in f32 and in a fixed order, and rounded once: the workspace then holds the parts,
+ * at most 256 MB with a tile_m of up to 128 (in proportion to the padded rows beyond), and dx agrees with the
+ * stage calls' (fs2moe_grouped_gemm_sum, which has no scratch and takes the sum whole) to f32 rounding
+ * instead of bit for bit.
  *   normed       the rows are RMS-normalised first (norm_weight [D] or NULL, norm_eps)
  *   router       (D, E); router_read: what the forward pass reads, the same or, with
  *                FS2MOE_ROUTER_OUT_IN or-ed into score_fn, its (E, D) copy

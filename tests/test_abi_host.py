@@ -730,3 +730,26 @@ def test_rows_in_token_order_are_copied_for_wide_weight_gradients(lib, t, f, cop
         for name in ("d_gate", "d_up", "d_down"):
             setattr(a, name, 0x1000 if name in names else None)
         assert lib.fs2moe_train_workspace_bytes(a, 1) == none + rows * copies * rows_bytes, names
+
+
+@pytest.mark.parametrize("dtype", [_abi.BF16, _abi.F32])
+@pytest.mark.parametrize("t,d,e,k,f,split", [
+    (500, 264, 4, 1, 6152, (True, True)), (1000, 512, 8, 2, 1408, (False, True)), (300, 512, 16, 2, 4096, (True, True)),
+    (4000, 2048, 8, 1, 14336, (True, False)), (8192, 2048, 128, 8, 768, (False, False)),
+])
+def test_train_scratch_for_sums_in_parts(lib, dtype, t, d, e, k, f, split):
+    """As many parts whatever the padding, 256 MB at most with blocks of up to 128 rows, and only for a call that takes
+    the rows' gradients."""
+    parts = set()
+    for tile_m in (1, 16, 128, 512):
+        a = _abi.TrainArgs(T=t, D=d, E=e, K=k, F=f, tile_m=tile_m, act_dtype=dtype, score_fn=_abi.SCORE_SIGMOID,
+                           scale_input=1)
+        without = lib.fs2moe_train_workspace_bytes(a, 1)
+        a.dx = 0x1000
+        taken = lib.fs2moe_train_workspace_bytes(a, 1) - without
+        a.dx, a.d_norm_weight = None, 0x1000
+        assert lib.fs2moe_train_workspace_bytes(a, 1) - without == taken
+        row = (t * k + e * (tile_m - 1)) * d * 4
+        assert taken % 256 == 0 and taken % row < 256 and (tile_m > 128 or taken <= 256 << 20)
+        parts.add(taken // row)
+    assert len(parts) == 1 and (parts.pop() > 1) == split[dtype == _abi.F32]
