@@ -47,8 +47,8 @@ inline bool small_tiles(int64_t big_tiles, int64_t rows_per_group) {
 // Or where their rounds of tiles (of the experts' rows, half of a last row block each) take less time than those of the
 // large ones, 64 rows x N as small tiles or 128 rows x N as large ones of 64 (two products) or 128 columns: 0.53 us per
 // 32 k and small tile, 0.44 per 64 x 64 of a large one.
-// 1356 tokens, top-1 of 16, D 1024, F 2048 by a popularity law 283 -> 225 us; the training step of 2439, top-2 of 16, D
-// 1024, F 1472 1596 -> 1534.
+// 1356 tokens, top-1 of 16, D 1024, F 2048 by a popularity law 285 -> 228 us; the training step of 2439, top-2 of 16, D
+// 1024, F 1472 1604 -> 1538.
 inline bool small_rounds(bool dual, int64_t rows, int groups, int N, int cus) {
   const int64_t real = groups > 0 && rows > 15ll * groups ? rows - 15ll * groups : rows;  // (less the blocks' padding)
   const int g = groups > 0 ? groups : 1;
@@ -432,7 +432,7 @@ __global__ __launch_bounds__(f32t::threads(WAVES), WAVES / 2) void glu_gemm_f32_
 // rest, by their numbers within each.  Wave-uniform, every wave for itself; without such experts it is n.
 // A block is one tile's walk over an expert's rows, and the hardware starts blocks in order: where the tiles of the
 // largest expert begin last, the launch waits for their walks alone.  Training step of 2439 tokens, top-2 of 16, D 1024,
-// F 1472 by a popularity law 1926 -> 1591 us; of 2153 evenly, top-1 of 8, D 640, F 2048 1220, 1221; 1000 tokens, top-2 of
+// F 1472 by a popularity law 1899 -> 1538 us; of 2153 evenly, top-1 of 8, D 640, F 2048 1220, 1221; 1000 tokens, top-2 of
 // 8, D 512, F 1408, whose tiles are small, 397 without and 404 with it.
 __device__ __forceinline__ int nth_expert_by_size(const int32_t* __restrict__ counts, int total, int E, int n) {
   static_assert(FS2MOE_MAX_EXPERTS <= 512, "eight counts a lane");
