@@ -69,6 +69,8 @@ constexpr uint32_t NOWHERE = 0xfffffff0u;      // an offset past any buffer's en
 //   16 experts of 375, K 1368, N 1024    33 against 62, 50, 37     (none fits one round)
 //   32 of 35, D 1472, F 1216             90 against 79 (2), 80 (3) (the throughput kernel: 1.25 rounds)
 //   64 of 23, D 2944, F 1840             377 against 394, 400      (memory)
+// All are even loads, which the rounds' model further down assumes.  Where a few rows reach a part of the experts it is
+// far off: 48 tokens, top-8 of 128 by a popularity law, K 768, N 2048 36 us with the throughput kernel, 18 by the model.
 // single: the launch is one product of bf16 matrices.
 inline int pick(bool dual, bool single, int64_t rows, int groups, int K, int N, int cus) {
   // Of the experts' rows only the device knows how they are spread: the planned ones (Groups), less what blocks of 16
