@@ -576,10 +576,15 @@ def test_residual_is_added_in_the_same_accumulation(gpu_device, dtype, shared):
     assert torch.equal(res_d, res.to(gpu_device)), "the residual is left untouched"
     assert_output_close(got, ref.out + res.double(), dtype, "residual + layer")
     # the separate addition rounds the layer output and then the sum, the fused one only the sum:
-    # they differ by at most those roundings
+    # they differ by at most those roundings, and by those of the sums' k and k + 1 additions in f32, half a step each of
+    # a partial sum, which is at most the terms' sizes together.  (Without the latter the bound is not one in f32, where
+    # they count as much: half of 40 seeds had an element outside, by up to 3.8.)
     eps = 2.0 ** -8 if dtype == "bf16" else 2.0 ** -23
     two_step = out.double() + res_d.double()
+    pairs = torch.from_numpy(ref.routing.inv_perm).long()
+    terms = ref.base.abs() + ref.ye[pairs].abs().sum(1) + res.reshape(ref.base.shape).double().abs()
     bound = eps * (out.double().abs() + two_step.abs() + got.double().abs())
+    bound += (2 * pairs.shape[1] + 1) * 2.0**-24 * terms.reshape(got.shape).to(gpu_device)
     assert bool(((got.double() - two_step).abs() <= bound).all())
 
 
