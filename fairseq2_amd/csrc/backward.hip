@@ -1280,7 +1280,7 @@ extern "C" int fs2moe_grouped_wgrad(const void* a, const int32_t* a_row_map, con
     FS2_REQUIRE((int64_t)slots * mt * nt <= 0x7fffffffll, "grouped_wgrad: too many tiles");
     auto k = small ? (mapped ? grouped_wgrad_f32_kernel<1, true> : grouped_wgrad_f32_kernel<1, false>)
                    : (mapped ? grouped_wgrad_f32_kernel<2, true> : grouped_wgrad_f32_kernel<2, false>);
-    hipLaunchKernelGGL(k, dim3((unsigned)(slots * mt * nt)), dim3(f32t::threads(4)), 0, st,
+    hipLaunchKernelGGL(k, dim3((unsigned)(slots * mt * nt)), dim3(f32t::threads(1)), 0, st,
                        static_cast<const float*>(a), a_row_map, static_cast<const float*>(b),
                        static_cast<float*>(dw), M, N, g, mt, nt, seg_rows, partial);
   }

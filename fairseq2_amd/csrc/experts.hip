@@ -208,12 +208,12 @@ static int launch_f32(const void* a, const void* b0, const void* b1, const void*
     set_error("%s: grid too large", what);
     return FS2MOE_ERR_UNSUPPORTED;
   }
-  const bool eight = !DUAL && small && f32t::eight_waves(planned, groups);
-  auto k = eight   ? glu_gemm_f32_kernel<DUAL, 1, 1, BLAYOUT, DUAL ? 4 : 8>
-           : small ? glu_gemm_f32_kernel<DUAL, 1, 1, BLAYOUT, 4>
-                   : glu_gemm_f32_kernel<DUAL, 2, DUAL ? 1 : 2, BLAYOUT, 4>;
+  // (small tiles of one product: two groups of waves, f32t::threads)
+  constexpr int groups_small = DUAL ? 1 : 2;
+  auto k = small ? glu_gemm_f32_kernel<DUAL, 1, 1, BLAYOUT, groups_small>
+                 : glu_gemm_f32_kernel<DUAL, 2, DUAL ? 1 : 2, BLAYOUT, 1>;
   hipLaunchKernelGGL(k, dim3((unsigned)((m_tiles * nt + 7) / 8 * 8), (unsigned)parts),
-                     dim3(f32t::threads(eight ? 8 : 4)), 0, stream,
+                     dim3(f32t::threads(small ? groups_small : 1)), 0, stream,
                      static_cast<const float*>(a), static_cast<const float*>(b0),
                      static_cast<const float*>(b1), static_cast<const float*>(a2),
                      static_cast<float*>(c), static_cast<float*>(g_keep), static_cast<float*>(u_keep), K,

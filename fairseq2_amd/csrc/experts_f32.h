@@ -15,16 +15,15 @@
 //
 // k slots.  Lanes 0..31 carry one k of an instruction and lanes 32..63 the other, and which k they are is
 // free as long as both operands agree: instruction j of step s takes k 8 s + j and 8 s + 4 + j, so that a
-// lane's four values of a k-contiguous operand are one 16-byte LDS read.  Fragments of 16 x 16 take the same k in the same
-// order, four an instruction: an instruction of either shape adds its k one after the other, each as a fused multiply-add
-// (2 million sums of either against fmaf, bit for bit).  Instruction j of step s, of 16 k, has in its lanes 16 q ..
-// 16 q + 15 k 16 s + 8 (j / 2) + 2 (j % 2) + 4 (q % 2) + q / 2, so a row has the same bits on every tile.
+// lane's four values of a k-contiguous operand are one 16-byte LDS read.  Products add the first halves of all chunks
+// (steps 0 and 1) in one sum, the second ones (2 and 3) in another, and the two at the end, on every tile: on some
+// two groups of waves take a half each, and a row's bits do not depend on the tile.  Two sums of half the length also
+// round less (K 1408 4.8e-7 of the result instead of 6.7e-7); on large tiles, which keep both in a wave's registers,
+// they take the same time (8192 x 2048 by 2048 x 4096 971, 972 us).
 //
 // LDS layouts (16-byte chunks).  k-contiguous operand: rows of 128 bytes, chunk c of row r in slot
-// c ^ ((r >> 1) & 7); for fragments of 16 x 16 slot 4 s + q has the four values of q's lanes in step s instead, so that
-// they, too, are one read.  k-major operand: a row per k, chunk c of row k in slot c ^ (((k >> 2) & 1) << 3), so
-// that the two half waves, which read rows 4 apart, use different banks; for fragments of 16 x 16, whose quarters also
-// read neighbouring rows, c ^ (((k >> 2) & 1) << 3) ^ ((k & 1) << 2).
+// c ^ ((r >> 1) & 7).  k-major operand: a row per k, chunk c of row k in slot c ^ (((k >> 2) & 1) << 3), so
+// that the two half waves, which read rows 4 apart, use different banks.
 #pragma once
 
 #include <type_traits>
@@ -35,9 +34,13 @@
 namespace fs2moe {
 namespace f32t {
 constexpr int BK = 32;
-// Waves of a block: four of 32 x 32 fragments each, or on the small tile of one product eight, each 32 rows x 16
-// channels in fragments of 16 x 16 (eight_waves).
-constexpr int threads(int waves) { return 64 * waves; }
+// Threads of a block: four waves, or two groups of four that each take half of every chunk's k, whose sums are added
+// at the end.  Two waves to a SIMD cover each other's reads and barriers, and where a tile has up to 32 rows every SIMD
+// has one that multiplies: 16 experts of 18 rows, K 1792, N 1024, 38 -> 30 us; 1024 rows, K 4096, N 1024 (a tile a CU)
+// 80 -> 74; 60 experts of 80, the pair of D 768, F 2000, 575 -> 547.  Not for two products at once: what the sums leave
+// of registers and LDS lets two such blocks share a CU instead of three smaller ones (60 experts of 17 rows, K 576, N
+// 1760, 66 -> 80 us).
+constexpr int threads(int groups) { return 256 * groups; }
 
 // Tiles of 64 x 64 while 128 x 128 ones would give a CU fewer than two blocks (big_tiles of them in the
 // launch), or where the groups have so few rows on average that half of a 128-row tile would be padding.
@@ -59,28 +62,12 @@ inline bool small_rounds(bool dual, int64_t rows, int groups, int N, int cus) {
   return small * 12 < large * 11;
 }
 
-// Small tiles of one product: eight waves where a group's last tile has up to 32 rows and is a large part of its work.
-// Of four waves the two of such a tile's rows 32 .. 63 idle, and with them two of the CU's SIMDs; of eight every SIMD
-// has one that multiplies.  Elsewhere they cost more, as their smaller fragments read LDS 1.5 times as often.  K 1408, N
-// 640, us with four and with eight, (in, out) and (out, in) weights; evenly, as random routing spreads them, or by a
-// popularity law of exponent 1.1:
-//   60 experts of 96 rows 121, 104; 120, 106   of 64  69, 70; 68, 69     of 20 at random 50, 44; 48, 43
-//   of 80 at random       122, 106; 122, 108   of 30  68, 69; 66, 68     of 80 by the law 112, 113; 110, 114
-//   32 of 96               67, 62;   66, 61    of 112 69, 70; 67, 69     of 192           90, 91; 88, 93
-// and 16 of 18 rows, K 1792, N 1024 36, 27; 33, 26.
-inline bool eight_waves(int64_t rows, int groups) {
-  const int64_t real = groups > 0 && rows > 15ll * groups ? rows - 15ll * groups : rows;  // (less the blocks' padding)
-  const int64_t each = real / (groups > 0 ? groups : 1);
-  return each <= 32 || (each > 64 && each <= 96);
-}
-
 // what a load through a row map reads past the end (not const: a global address)
 static __device__ __attribute__((aligned(16))) uint32_t zero16[4] = {0u, 0u, 0u, 0u};
 
 // A chunk (32 k) of one operand: ROWS rows (or columns) x 32 k.  `base` points at the operand's first row
 // (column) of the tile in k 0; ld is the stride in floats of a row (k-contiguous) or of a k (k-major).
-// FRAG: rows of a fragment.
-template <int ROWS, bool KMAJOR, int THREADS, int FRAG>
+template <int ROWS, bool KMAJOR, int THREADS>
 struct Operand {
   static constexpr int BYTES = ROWS * BK * 4;
   static constexpr int PER = ROWS * BK / 4 / THREADS;  // 16-byte chunks per thread
@@ -137,61 +124,48 @@ struct Operand {
   }
   static __device__ __forceinline__ void store(u32x4 reg, int tid, int i, uint8_t* lds) {
     const int c = tid + THREADS * i;
-    if constexpr (KMAJOR) {
-      const int k = c / CPK, key = (k >> 2 & 1) << 3 | (FRAG == 16 ? (k & 1) << 2 : 0);
-      *reinterpret_cast<u32x4*>(lds + (k * CPK + ((c % CPK) ^ key)) * 16) = reg;
-    } else if constexpr (FRAG == 16) {
-      // (chunk c of k 4 c .. 4 c + 3: the even ones for quarter c % 2, the odd ones for 2 more)
-      const int row = (c >> 3) * 8, key = (c >> 4) & 7, slot = (c & 4) | (c & 1);
-      uint8_t* to = lds + (c >> 1 & 1) * 8;
-      *reinterpret_cast<u32x2*>(to + (row + (slot ^ key)) * 16) = u32x2{reg[0], reg[2]};
-      *reinterpret_cast<u32x2*>(to + (row + ((slot | 2) ^ key)) * 16) = u32x2{reg[1], reg[3]};
-    } else {
-      *reinterpret_cast<u32x4*>(lds + ((c >> 3) * 8 + ((c & 7) ^ ((c >> 4) & 7))) * 16) = reg;
-    }
+    const int at = KMAJOR ? (c / CPK) * CPK + ((c % CPK) ^ (((c / CPK) >> 2 & 1) << 3))
+                          : (c >> 3) * 8 + ((c & 7) ^ ((c >> 4) & 7));
+    *reinterpret_cast<u32x4*>(lds + at * 16) = reg;
   }
-  // the lane's four values of step s of the FRAG rows from r0 on
+  // the lane's four values of step s (k 8 s + 4 (lane / 32) + 0..3) of the 32 rows from r0 on
   static __device__ __forceinline__ f32x4 frag(const uint8_t* lds, int lane, int r0, int s) {
-    const int r = r0 + lane % FRAG, q = lane / FRAG;
-    if constexpr (KMAJOR && FRAG == 16) {
-      const float* p = reinterpret_cast<const float*>(lds) + (16 * s + 4 * (q & 1) + (q >> 1)) * ROWS +
-                       (r ^ ((q & 1) << 5) ^ ((q >> 1) << 4));
-      return f32x4{p[0], p[2 * ROWS], p[8 * ROWS], p[10 * ROWS]};
-    } else if constexpr (KMAJOR) {
-      const float* p = reinterpret_cast<const float*>(lds) + (8 * s + 4 * q) * ROWS + (r ^ (q << 5));
+    const int lr = lane & 31, lk = lane >> 5;
+    if constexpr (KMAJOR) {
+      const float* p = reinterpret_cast<const float*>(lds) + (8 * s + 4 * lk) * ROWS + ((r0 + lr) ^ (lk << 5));
       return f32x4{p[0], p[ROWS], p[2 * ROWS], p[3 * ROWS]};
     } else {
-      const int slot = FRAG == 16 ? 4 * s + q : 2 * s + q;
-      return *reinterpret_cast<const f32x4*>(lds + r * 128 + ((slot ^ ((r >> 1) & 7)) << 4));
+      const int r = r0 + lr;
+      return *reinterpret_cast<const f32x4*>(lds + r * 128 + (((2 * s + lk) ^ ((r >> 1) & 7)) << 4));
     }
   }
 };
 
-// The walk over k of one tile: waves 2 x 2, each 32 FM rows x 32 FN channels of each of NB matrices, in fragments of
-// 32 x 32; or, with WAVES 8, waves 2 x 4, each 32 rows x 16 channels in fragments of 16 x 16.
-// acc[b][fn][fm] is the transposed fragment (lane: row lane % FRAG, channels 8 q + 4 (lane / FRAG) + 0..3 in 4 q ..).
+// The walk over k of one tile: waves 2 x 2, each 32 FM rows x 32 FN channels of each of NB matrices.
+// acc[b][fn][fm] is the transposed 32 x 32 tile (lane: row lr, channels 8 q + 4 lk + 0..3 in 4 q ..).
 // With two sources the second pair follows the first in the same accumulators.
 // A_MAPPED: a_map gives the rows of the k-major A.
-template <int NB, int FM, int FN, bool A_KMAJOR, bool B_KMAJOR, bool A_MAPPED = false, int WAVES = 4>
+// HALVES: two sums, over the first and the second half of every chunk's k, added at the end; the groups' (GROUPS 2), or
+// both of each wave.
+template <int NB, int FM, int FN, bool A_KMAJOR, bool B_KMAJOR, bool A_MAPPED = false, int GROUPS = 1,
+          bool HALVES = true>
 struct Walk {
-  static constexpr int BM = 64 * FM, BN = 64 * FN, THREADS = threads(WAVES);
-  static_assert(WAVES == 4 || (WAVES == 8 && NB == 1 && FM == 1 && FN == 1), "eight waves on the small tile");
-  static constexpr int FRAG = WAVES == 8 ? 16 : 32;
-  static constexpr int XF = WAVES == 8 ? 2 : FM, WF = WAVES == 8 ? 1 : FN;  // a wave's fragments of rows and channels
-  static constexpr int REGS = FRAG * FRAG / 64;                             // of a fragment's sums
-  using Sums = std::conditional_t<WAVES == 8, f32x4, f32x16>;
-  using OpA = Operand<BM, A_KMAJOR, THREADS, FRAG>;
-  using OpB = Operand<BN, B_KMAJOR, THREADS, FRAG>;
+  static_assert(HALVES || GROUPS == 1, "two groups of waves take a half each");
+  static constexpr int CHAINS = HALVES && GROUPS == 1 ? 2 : 1;  // sums that a wave keeps
+  static constexpr int BM = 64 * FM, BN = 64 * FN, THREADS = threads(GROUPS);
+  using OpA = Operand<BM, A_KMAJOR, THREADS>;
+  using OpB = Operand<BN, B_KMAJOR, THREADS>;
   static constexpr int BUF_BYTES = OpA::BYTES + NB * OpB::BYTES;
   static constexpr int SMEM_BYTES = 2 * BUF_BYTES;
   static constexpr int PIECES = OpA::PER + NB * OpB::PER;  // 16-byte pieces of a chunk per thread
-  static constexpr int STEPS = BK / (WAVES == 8 ? 16 : 8);   // steps of a chunk, four MFMAs per pair of fragments each
-  static constexpr int PRODUCTS = 4 * STEPS * NB * XF * WF;  // MFMAs of a chunk per wave
+  static constexpr int STEPS = BK / 8 / GROUPS;              // steps of 8 k of a chunk per wave
+  static constexpr int PRODUCTS = 4 * STEPS * NB * FM * FN;  // MFMAs of a chunk per wave
 
-  // The wave's rows and channels of the tile.  (Waves w and w + 4 share a SIMD: with a tile of up to 32 rows every
-  // SIMD has a wave that multiplies.)
-  static __device__ __forceinline__ int wave_m(int wave) { return WAVES == 8 ? wave >> 2 : wave & 1; }
-  static __device__ __forceinline__ int wave_n(int wave) { return WAVES == 8 ? wave & 3 : wave >> 1; }
+  // The wave's rows and channels of the tile, and which share of a chunk's k it takes.  (Waves w and w + 4 share a
+  // SIMD: with a tile of up to 32 rows every SIMD has a wave that multiplies.)
+  static __device__ __forceinline__ int wave_m(int wave) { return GROUPS == 2 ? wave >> 2 : wave & 1; }
+  static __device__ __forceinline__ int wave_n(int wave) { return GROUPS == 2 ? wave & 1 : wave >> 1; }
+  static __device__ __forceinline__ int wave_group(int wave) { return GROUPS == 2 ? (wave >> 1) & 1 : 0; }
 
   struct Source {
     const float* a;
@@ -199,13 +173,24 @@ struct Walk {
   };
   // m_rows, n_cols: how many of the tile's rows and channels exist; `active`: this wave's rows do.  The walk is the
   // part-th of `parts`, each as many chunks but the last.
-  static __device__ __forceinline__ void run(Sums (&acc)[NB][WF][XF], uint8_t* smem, const Source& s0,
+  static __device__ __forceinline__ void run(f32x16 (&sums)[NB][FN][FM], uint8_t* smem, const Source& s0,
                                              const Source& s1, int sources, int lda, int ldb, int K,
                                              int m_rows, int n_cols, bool active,
                                              const int32_t* a_map = nullptr, int part = 0, int parts = 1) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave_m(wave), wn = wave_n(wave);
+    const int wm = wave_m(wave), wn = wave_n(wave), s0k = wave_group(wave) * STEPS;
+    f32x16 acc[CHAINS][NB][FN][FM];
+#pragma unroll
+    for (int c = 0; c < CHAINS; ++c)
+#pragma unroll
+      for (int m = 0; m < NB; ++m)
+#pragma unroll
+        for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+          for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[c][m][fn][fm][i] = 0.f;
     OpA opa;
     OpB opb;
     opa.setup(tid, lda, m_rows);
@@ -253,16 +238,16 @@ struct Walk {
         OpB::store(b[i][j], tid, j, at + OpA::BYTES + i * OpB::BYTES);
       }
     };
-    f32x4 xf[2][XF], wf[2][NB][WF];
+    f32x4 xf[2][FM], wf[2][NB][FN];
     auto read = [&](int set, int buf, int s) {
       const uint8_t* at = smem + buf * BUF_BYTES;
 #pragma unroll
-      for (int fm = 0; fm < XF; ++fm) xf[set][fm] = OpA::frag(at, lane, (wm * XF + fm) * FRAG, s);
+      for (int fm = 0; fm < FM; ++fm) xf[set][fm] = OpA::frag(at, lane, (wm * FM + fm) * 32, s);
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int fn = 0; fn < WF; ++fn)
-          wf[set][b][fn] = OpB::frag(at + OpA::BYTES + b * OpB::BYTES, lane, (wn * WF + fn) * FRAG, s);
+        for (int fn = 0; fn < FN; ++fn)
+          wf[set][b][fn] = OpB::frag(at + OpA::BYTES + b * OpB::BYTES, lane, (wn * FN + fn) * 32, s);
     };
     // Chunk st is multiplied from buffer st & 1, while chunk st + 1 is stored from register set
     // (st + 1) & 1 into the other buffer (whose last reads, of chunk st - 1, are behind that chunk's barrier)
@@ -283,27 +268,23 @@ struct Walk {
 #pragma unroll
         for (int s = 0; s < STEPS; ++s) {
           if (s + 1 < STEPS) {
-            read((s + 1) & 1, buf, s + 1);
+            read((s + 1) & 1, buf, s0k + s + 1);
           } else {
             lds_barrier();
-            read(0, buf ^ 1, 0);
+            read(0, buf ^ 1, s0k);
           }
 #pragma unroll
           for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int m = 0; m < NB; ++m)
 #pragma unroll
-              for (int fn = 0; fn < WF; ++fn)
+              for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
-                for (int fm = 0; fm < XF; ++fm) {
+                for (int fm = 0; fm < FM; ++fm) {
                   __builtin_amdgcn_sched_barrier(0);
-                  if constexpr (WAVES == 8)
-                    acc[m][fn][fm] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                        wf[s & 1][m][fn][j], xf[s & 1][fm][j], acc[m][fn][fm], 0, 0, 0);
-                  else
-                    acc[m][fn][fm] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                        wf[s & 1][m][fn][j], xf[s & 1][fm][j], acc[m][fn][fm], 0, 0, 0);
-                  const int done = (((s * 4 + j) * NB + m) * WF + fn) * XF + fm;
+                  f32x16& sum = acc[CHAINS == 2 ? s / (STEPS / 2) : 0][m][fn][fm];
+                  sum = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[s & 1][m][fn][j], xf[s & 1][fm][j], sum, 0, 0, 0);
+                  const int done = (((s * 4 + j) * NB + m) * FN + fn) * FM + fm;
                   if (done < BEHIND && done % EVERY == 0) {
                     const int o = done / EVERY;
                     if (o < PIECES)
@@ -335,7 +316,7 @@ struct Walk {
     load_all(ra[0], rb[0], 2);
     lds_barrier();
     auto walk = [&](auto multiply) {
-      if constexpr (decltype(multiply)::value) read(0, 0, 0);
+      if constexpr (decltype(multiply)::value) read(0, 0, s0k);
       int st = 0;
       for (; st + 1 < steps; st += 2) {
         chunk(multiply, ra[1], rb[1], 0, st);
@@ -347,21 +328,60 @@ struct Walk {
       walk(std::integral_constant<bool, true>{});
     else
       walk(std::integral_constant<bool, false>{});
+    if constexpr (GROUPS == 2) {
+      // the second group's sums onto the first's, through the chunks' LDS (the barrier: each chunk's last step reads the
+      // next one's first fragments, the last chunk's too)
+      constexpr int REGS = NB * FN * FM * 16;
+      static_assert(4 * REGS * 64 * 4 <= SMEM_BYTES, "the sums of four waves fit the chunks' buffers");
+      float* at = reinterpret_cast<float*>(smem) + (wm * 2 + wn) * (REGS * 64) + lane;
+      auto exchange = [&](auto store) {
+#pragma unroll
+        for (int m = 0; m < NB; ++m)
+#pragma unroll
+          for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+            for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+              for (int i = 0; i < 16; ++i) {
+                float& v = at[(((m * FN + fn) * FM + fm) * 16 + i) * 64];
+                if constexpr (decltype(store)::value)
+                  v = acc[0][m][fn][fm][i];
+                else
+                  acc[0][m][fn][fm][i] += v;
+              }
+      };
+      const bool second = s0k != 0;
+      lds_barrier();
+      if (second && active) exchange(std::integral_constant<bool, true>{});
+      lds_barrier();
+      if (!second && active) exchange(std::integral_constant<bool, false>{});
+    }
+#pragma unroll
+    for (int m = 0; m < NB; ++m)
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+        for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            sums[m][fn][fm][i] = CHAINS == 2 ? acc[0][m][fn][fm][i] + acc[CHAINS - 1][m][fn][fm][i] : acc[0][m][fn][fm][i];
   }
+  // whether the wave holds the tile's sums after run
+  static __device__ __forceinline__ bool holds_sums(int wave) { return wave_group(wave) == 0; }
 };
 }  // namespace f32t
 
 // C = A B_e (+ A2 B2_e), or with DUAL C = SiLU(A B0_e) * (A B1_e), the two products left in g_keep and
 // u_keep where those are given.  A block per tile; BLAYOUT as for the bf16 kernels.  With several rows of blocks
 // (single products) each takes a part of the sum over K, and C is [gridDim.y][rows][N].
-template <bool DUAL, int FM, int FN, int BLAYOUT, int WAVES>
-__global__ __launch_bounds__(f32t::threads(WAVES), WAVES / 2) void glu_gemm_f32_kernel(
+template <bool DUAL, int FM, int FN, int BLAYOUT, int GROUPS>
+__global__ __launch_bounds__(f32t::threads(GROUPS), 2 * GROUPS) void glu_gemm_f32_kernel(
     const float* __restrict__ A, const float* __restrict__ B0, const float* __restrict__ B1,
     const float* __restrict__ A2, float* __restrict__ C, float* __restrict__ g_keep,
     float* __restrict__ u_keep, int K, int N, Groups g, int n_tiles) {
   constexpr int NB = DUAL ? 2 : 1;
   constexpr bool KN = BLAYOUT == FS2MOE_W_IN_OUT;
-  using W = f32t::Walk<NB, FM, FN, false, KN, false, WAVES>;
+  using W = f32t::Walk<NB, FM, FN, false, KN, false, GROUPS>;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[W::SMEM_BYTES];
   int e, row0, row_end, nt;
   if (!locate_tile_by_xcd<W::BM, W::THREADS>(g, n_tiles, e, row0, row_end, nt)) return;
@@ -370,17 +390,9 @@ __global__ __launch_bounds__(f32t::threads(WAVES), WAVES / 2) void glu_gemm_f32_
   row_end = __builtin_amdgcn_readfirstlane(row_end);
   const int n0 = nt * W::BN;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = W::wave_m(wave), wn = W::wave_n(wave), lr = lane % W::FRAG, lk = lane / W::FRAG;
+  const int wm = W::wave_m(wave), wn = W::wave_n(wave), lr = lane & 31, lk = lane >> 5;
 
-  typename W::Sums acc[NB][W::WF][W::XF];
-#pragma unroll
-  for (int b = 0; b < NB; ++b)
-#pragma unroll
-    for (int fn = 0; fn < W::WF; ++fn)
-#pragma unroll
-      for (int fm = 0; fm < W::XF; ++fm)
-#pragma unroll
-        for (int i = 0; i < W::REGS; ++i) acc[b][fn][fm][i] = 0.f;
+  f32x16 acc[NB][FN][FM];
 
   const size_t at = (size_t)e * K * N + (KN ? (size_t)n0 : (size_t)n0 * K);
   typename W::Source s0, s1;
@@ -396,17 +408,18 @@ __global__ __launch_bounds__(f32t::threads(WAVES), WAVES / 2) void glu_gemm_f32_
   const int m_wave = row0 + wm * 32 * FM;
   W::run(acc, smem, s0, s1, !DUAL && A2 != nullptr ? 2 : 1, K, KN ? N : K, K, row_end - row0, N - n0,
          m_wave < row_end, nullptr, DUAL ? 0 : (int)blockIdx.y, DUAL ? 1 : (int)gridDim.y);
+  if (!W::holds_sums(wave)) return;
   if constexpr (!DUAL) C += (size_t)blockIdx.y * g.dense_rows * N;
 
 #pragma unroll
-  for (int fm = 0; fm < W::XF; ++fm) {
-    const int m = m_wave + fm * W::FRAG + lr;
+  for (int fm = 0; fm < FM; ++fm) {
+    const int m = m_wave + fm * 32 + lr;
     if (m >= row_end) continue;
 #pragma unroll
-    for (int fn = 0; fn < W::WF; ++fn)
+    for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
-      for (int q = 0; q < W::REGS / 4; ++q) {
-        const int n = n0 + (wn * W::WF + fn) * W::FRAG + 8 * q + 4 * lk;
+      for (int q = 0; q < 4; ++q) {
+        const int n = n0 + (wn * FN + fn) * 32 + 8 * q + 4 * lk;
         if (n >= N) continue;
         const size_t to = (size_t)m * N + n;
         f32x4 v, u;
@@ -471,11 +484,11 @@ __device__ __forceinline__ int nth_expert_by_size(const int32_t* __restrict__ co
 // group (slots: segments, whose sums go to `partial` where there are several).
 // MAPPED: A's rows are read through a_map.
 template <int F, bool MAPPED>
-__global__ __launch_bounds__(f32t::threads(4), 2) void grouped_wgrad_f32_kernel(
+__global__ __launch_bounds__(f32t::threads(1), 2) void grouped_wgrad_f32_kernel(
     const float* __restrict__ A, const int32_t* __restrict__ a_map, const float* __restrict__ B,
     float* __restrict__ C, int M, int N, Groups g, int m_tiles, int n_tiles, int seg_rows,
     float* __restrict__ partial) {
-  using W = f32t::Walk<1, F, F, true, true, MAPPED>;
+  using W = f32t::Walk<1, F, F, true, true, MAPPED, 1, false>;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[W::SMEM_BYTES];
   const int per = m_tiles * n_tiles;
   int slot = blockIdx.x / per;

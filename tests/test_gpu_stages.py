@@ -707,9 +707,9 @@ def test_pair_and_two_sources_on_every_tile_size(gpu_device, counts, n):
         assert torch.equal(ye[sl], ye2[sl]) and torch.equal(h[sl], h2[sl]), f"expert {i} without keeping"
 
 
-# The f32 products take tiles of 64 x 64, of eight waves or four, or of 128 x 128 (the pair 128 x 64) by the size of the
-# buffers: the same bits.  Rows on both sides of 32, 64 and 128, experts without any, K within a chunk of 32, past its
-# quarters and over several, N off the tiles' channels.
+# The f32 products take tiles of 64 x 64, on which two groups of waves share the sum over K (the pair one), or of 128 x
+# 128 (the pair 128 x 64) by the size of the buffers: the same bits.  Rows on both sides of 32, 64 and 128, experts
+# without any, K within a chunk of 32, past its quarters and over several, N off the tiles' channels.
 @pytest.mark.parametrize("k", [8, 24, 40, 200])
 @pytest.mark.parametrize("n", [1024, 1000])
 @pytest.mark.parametrize("layout", [_abi.W_IN_OUT, _abi.W_OUT_IN])
