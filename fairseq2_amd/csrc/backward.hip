@@ -61,7 +61,6 @@ constexpr int SMEM_BYTES = RING_BYTES + EPI_BYTES + TABLE_INTS * 4;
 constexpr int kTileCost = 5;
 constexpr int BAND = 8;
 constexpr int MAX_JOBS = 8;
-constexpr int kNonTemporal = 2;                         // in a buffer instruction's cache policy
 }  // namespace wgk
 // what a load through a row map reads past the end (not const: a global address, so the loads stay global
 // loads)

@@ -235,11 +235,11 @@ static bool whole_units(int act_dtype, int D, int F) {
 }
 
 // One launch of the bf16 kernel on smaller tiles (experts_half.h), one block per CU.
-template <int BM, int BNV, bool DUAL, int BLAYOUT, bool KEEP_GU, bool TWO_SRC>
-static int launch_half(const void* a, const int32_t* row_map, int K, const void* b0, const void* b1,
+template <int BM, int BNV, bool DUAL, int BLAYOUT, bool KEEP_GU, bool TWO_SRC, bool ONCE>
+static int launch_half_as(const void* a, const int32_t* row_map, int K, const void* b0, const void* b1,
                        const void* s0, const void* s1, void* c, int N, const Groups& g, const char* what,
                        int num_blocks, hipStream_t stream) {
-  auto k = glu_gemm_half_kernel<BM, BNV, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>;
+  auto k = glu_gemm_half_kernel<BM, BNV, DUAL, BLAYOUT, KEEP_GU, TWO_SRC, ONCE>;
   constexpr int bytes = half_tiles::smem_bytes(BM, BNV, BLAYOUT), bn = DUAL ? BNV / 2 : BNV;
   static bool attr_set = false;  // benign race: setting the attribute is idempotent
   if (!attr_set) {
@@ -258,19 +258,32 @@ static int launch_half(const void* a, const int32_t* row_map, int K, const void*
   return check_launch(what);
 }
 
+template <int BM, int BNV, bool DUAL, int BLAYOUT, bool KEEP_GU, bool TWO_SRC>
+static int launch_half(const void* a, const int32_t* row_map, int K, const void* b0, const void* b1,
+                       const void* s0, const void* s1, void* c, int N, const Groups& g, const char* what,
+                       int num_blocks, int64_t mean_rows, hipStream_t stream) {
+  auto launch = g.once_past_cache && mean_rows <= half_tiles::once_rows(BM)
+                    ? launch_half_as<BM, BNV, DUAL, BLAYOUT, KEEP_GU, TWO_SRC, true>
+                    : launch_half_as<BM, BNV, DUAL, BLAYOUT, KEEP_GU, TWO_SRC, false>;
+  return launch(a, row_map, K, b0, b1, s0, s1, c, N, g, what, num_blocks, stream);
+}
+
 // One launch of the bf16 throughput kernel on persistent blocks, one per CU (the 128 KB ring allows no
 // more), a multiple of the 8 XCDs.  `b1`, `s0` and `s1` as the kernel's variants take them.
 template <bool DUAL, int BLAYOUT, bool KEEP_GU = false, bool TWO_SRC = false>
 static int launch_dma(const void* a, const int32_t* row_map, int K, const void* b0, const void* b1,
-                      const void* s0, const void* s1, void* c, int N, const Groups& g,
+                      const void* s0, const void* s1, void* c, int N, Groups g,
                       int64_t rows_bound, const char* what, hipStream_t stream) {
   using namespace dma;
   constexpr bool CAN_TAIL = BLAYOUT != W_FP8_TILED;
   auto whole = glu_gemm_bf16_dma_kernel<DUAL, BLAYOUT, KEEP_GU, TWO_SRC>;
   auto tail = glu_gemm_bf16_dma_kernel<DUAL, BLAYOUT, KEEP_GU, TWO_SRC, CAN_TAIL>;
+  auto whole_once = glu_gemm_bf16_dma_kernel<DUAL, BLAYOUT, KEEP_GU, TWO_SRC, false, false, true>;
+  auto tail_once = glu_gemm_bf16_dma_kernel<DUAL, BLAYOUT, KEEP_GU, TWO_SRC, CAN_TAIL, false, true>;
   static bool attr_set = false;  // benign race: setting the attribute is idempotent
   if (!attr_set) {
-    for (const void* k : {reinterpret_cast<const void*>(whole), reinterpret_cast<const void*>(tail)}) {
+    for (const void* k : {reinterpret_cast<const void*>(whole), reinterpret_cast<const void*>(tail),
+                          reinterpret_cast<const void*>(whole_once), reinterpret_cast<const void*>(tail_once)}) {
       hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_BYTES);
       if (e != hipSuccess) {
         set_error("%s: cannot reserve %d bytes of LDS: %s", what, SMEM_BYTES, hipGetErrorString(e));
@@ -285,11 +298,16 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
     return FS2MOE_ERR_LAUNCH;
   }
   const int groups = g.counts ? g.E : 0;
+  // (rows that do not begin on lines share lines with the tiles beside: 16 experts of D 2048, F 3000, 512 tokens 174 us
+  // without, 176 with)
+  const bool on_lines = !CAN_TAIL || (BLAYOUT == FS2MOE_W_IN_OUT ? N : K) % 64 == 0;
+  g.once_past_cache = on_lines && weights_past_cache(groups, pairs_of(g, rows_bound), K, N, CAN_TAIL ? 2 : 1);
   const int nt = (N + (DUAL ? 127 : 255)) / (DUAL ? 128 : 256);
   if ((rows_bound / BM + groups + 1) * nt > 0x7fffffffll) {
     set_error("%s: too many tiles", what);
     return FS2MOE_ERR_UNSUPPORTED;
   }
+  const int64_t rows = pairs_of(g, rows_bound), mean_rows = groups ? rows / groups : rows;
   // (tiles of 64 x 64 are counted in 31 bits too)
   const bool counted = (rows_bound / 64 + groups + 1) * ((N + 63) / 64) <= 0x7fffffffll;
   constexpr bool SINGLE = !DUAL && CAN_TAIL;
@@ -297,14 +315,14 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
     case 1:
       if constexpr (SINGLE)
         return launch_half<64, 64, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
-                                                                    num_blocks, stream);
+                                                                    num_blocks, mean_rows, stream);
       break;
     case 2:
       return launch_half<64, 128, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
-                                                                   num_blocks, stream);
+                                                                   num_blocks, mean_rows, stream);
     case 3:
       return launch_half<128, 128, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
-                                                                    num_blocks, stream);
+                                                                    num_blocks, mean_rows, stream);
   }
   // The variant for any K also stores rows that do not begin on lines as L2 wants them, which counts for more than its
   // selects at every load where stores are a large part of the work: three results, or few units.  us with the variant
@@ -318,7 +336,20 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
   //                                 28,  29    45,  45    65,  62    81,  81   120, 124   155, 166   196, 205
   const bool off_lines =
       off_lines_variant(DUAL, BLAYOUT, TWO_SRC, CAN_TAIL) && N % 64 != 0 && (KEEP_GU || K <= 1536);
-  hipLaunchKernelGGL(K % (2 * BK) == 0 && !off_lines ? whole : tail, dim3((unsigned)num_blocks), dim3(NWAVES * 64),
+  // Weights past the caches where most tiles are their expert's only row block, by the mean of the experts' rows.  (By
+  // the expert, as the kernels do that load straight to LDS, it costs more than it gives: two kinds of loads into the
+  // same registers meet behind a branch, where the compiler waits for all of them.)  us without and with, experts loaded
+  // evenly and by a popularity law of exponent 1.2; forward passes, then training steps with these rows on average:
+  //   128 of D 2048, F 768    3  222, 204  102, 97    32  246, 227  181, 177    94  274, 257  259, 260
+  //                         128  294, 283  319, 319  188  344, 336  393, 401   256  457, 475  456, 465
+  //   8 of D 4096, F 8192   175  412, 431  467, 478
+  //   128 of D 2048, F 768   64  908, 788  829, 776   128 1119, 980 1125, 1060  192 1321, 1227 1395, 1355
+  //                         256 1535, 1586 1647, 1674
+  //   64 of D 2048, F 1408  187  1170, 1116 1296, 1257  281 1531, 1607 1586, 1577
+  const bool once =
+      g.once_past_cache && mean_rows <= (KEEP_GU || BLAYOUT == FS2MOE_W_OUT_IN ? kOnceRowsTraining : kOnceRows);
+  const bool units = K % (2 * BK) == 0 && !off_lines;
+  hipLaunchKernelGGL(once ? (units ? whole_once : tail_once) : (units ? whole : tail), dim3((unsigned)num_blocks), dim3(NWAVES * 64),
                      SMEM_BYTES, stream, static_cast<const uint16_t*>(a), row_map, K,
                      static_cast<const uint16_t*>(b0), static_cast<const uint16_t*>(b1),
                      static_cast<const float*>(s0), static_cast<const float*>(s1),
@@ -535,15 +566,15 @@ static unsigned stream_experts(int blocks, int col_blocks, int E) {
   return (unsigned)(n < E ? n : E);
 }
 
-template <int R>
+template <int R, bool NT>
 static int launch_gemv_pair_r(const void* x, const int32_t* row_map, const float* row_w,
                               const Groups& g, const void* w_gate, const void* w_up,
                               const void* w_down, int D, int F, void* h, void* y,
                               hipStream_t stream) {
   using namespace gemv;
-  auto k1 = glu_gemv_bf16_kernel<true, R>;
-  auto k2 = glu_gemv_bf16_kernel<false, R>;
-  auto k2d = glu_gemv_bf16_kernel<false, R, true>;  // more loads in flight over a long K
+  auto k1 = glu_gemv_bf16_kernel<true, R, NT>;
+  auto k2 = glu_gemv_bf16_kernel<false, R, NT>;
+  auto k2d = glu_gemv_bf16_kernel<false, R, NT, true>;  // more loads in flight over a long K
   static bool attr_set = false;  // benign race: setting the attribute is idempotent
   if (!attr_set) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(k1),
@@ -593,14 +624,14 @@ static int gemv16_rows(int D, int F, int rows_hint) {
   return rows_hint > 8 && gemv16::fits(D > F ? D : F, 16) ? 16 : 8;
 }
 
-template <int XR>
+template <int XR, bool NT>
 static int launch_gemv16_pair(const void* x, const int32_t* row_map, const float* row_w,
                               const Groups& g, const void* w_gate, const void* w_up,
                               const void* w_down, int D, int F, void* h, void* y,
                               hipStream_t stream) {
   using namespace gemv16;
-  auto k1 = glu_gemv16_bf16_kernel<true, XR>;
-  auto k2 = glu_gemv16_bf16_kernel<false, XR>;
+  auto k1 = glu_gemv16_bf16_kernel<true, XR, NT>;
+  auto k2 = glu_gemv16_bf16_kernel<false, XR, NT>;
   static bool attr_set = false;  // benign race: setting the attribute is idempotent
   if (!attr_set) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(k1),
@@ -632,15 +663,16 @@ static int launch_gemv16_pair(const void* x, const int32_t* row_map, const float
 static bool dense_gemv_applies(int act_dtype, const Groups& g, int64_t rows) {
   return act_dtype == FS2MOE_BF16 && g.counts == nullptr && rows >= 1 && rows <= dgemv::MAX_ROWS;
 }
+template <bool NT>
 static int launch_dense_gemv_pair(const void* x, int T, const void* w_gate, const void* w_up,
                                   const void* w_down, int D, int F, void* h, void* y,
                                   hipStream_t stream) {
   using namespace dgemv;
-  hipLaunchKernelGGL(dense_gemv_bf16_kernel<true>, dim3((unsigned)((F + 15) / 16)), dim3(THREADS), 0,
+  hipLaunchKernelGGL((dense_gemv_bf16_kernel<true, NT>), dim3((unsigned)((F + 15) / 16)), dim3(THREADS), 0,
                      stream, static_cast<const uint16_t*>(x), D, static_cast<const uint16_t*>(w_gate),
                      static_cast<const uint16_t*>(w_up), static_cast<uint16_t*>(h), F, D, F, T);
   if (int rc = check_launch("dense_gemv_bf16<gate,up>")) return rc;
-  hipLaunchKernelGGL(dense_gemv_bf16_kernel<false>, dim3((unsigned)((D + 15) / 16)), dim3(THREADS), 0,
+  hipLaunchKernelGGL((dense_gemv_bf16_kernel<false, NT>), dim3((unsigned)((D + 15) / 16)), dim3(THREADS), 0,
                      stream, static_cast<const uint16_t*>(h), F, static_cast<const uint16_t*>(w_down),
                      static_cast<const uint16_t*>(nullptr), static_cast<uint16_t*>(y), D, F, D, T);
   return check_launch("dense_gemv_bf16<down>");
@@ -654,20 +686,26 @@ static int launch_glu(const void* x, const int32_t* row_map, const Groups& g, in
                       int act_dtype, void* h, void* y, hipStream_t stream, int rows_hint = 0,
                       const float* row_w = nullptr) {
   const int groups = g.counts ? g.E : 0;
+  const bool past = (BLAYOUT == FS2MOE_W_OUT_IN || (D % 64 == 0 && F % 64 == 0)) &&
+                    weights_past_cache(groups, pairs_of(g, rows_bound), D, F, 2);  // (lines: as in launch_dma)
   if constexpr (BLAYOUT == FS2MOE_W_OUT_IN) {
-    if (row_map == nullptr && dense_gemv_applies(act_dtype, g, rows_bound))
-      return launch_dense_gemv_pair(x, (int)rows_bound, w_gate, w_up, w_down, D, F, h, y, stream);
+    if (row_map == nullptr && dense_gemv_applies(act_dtype, g, rows_bound)) {
+      auto launch = past ? launch_dense_gemv_pair<true> : launch_dense_gemv_pair<false>;
+      return launch(x, (int)rows_bound, w_gate, w_up, w_down, D, F, h, y, stream);
+    }
   }
   if constexpr (BLAYOUT == FS2MOE_W_IN_OUT) {
     if (gemv_applies(act_dtype, D, F, g, rows_hint)) {
-      if (rows_hint <= 1) return launch_gemv_pair_r<1>(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream);
-      if (rows_hint <= 2) return launch_gemv_pair_r<2>(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream);
-      return launch_gemv_pair_r<4>(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream);
+      auto launch = rows_hint <= 1   ? (past ? launch_gemv_pair_r<1, true> : launch_gemv_pair_r<1, false>)
+                    : rows_hint <= 2 ? (past ? launch_gemv_pair_r<2, true> : launch_gemv_pair_r<2, false>)
+                                     : (past ? launch_gemv_pair_r<4, true> : launch_gemv_pair_r<4, false>);
+      return launch(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream);
     }
     if (gemv16_applies(act_dtype, D, F, g, rows_hint)) {
-      if (gemv16_rows(D, F, rows_hint) == 8)
-        return launch_gemv16_pair<8>(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream);
-      return launch_gemv16_pair<16>(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream);
+      auto launch = gemv16_rows(D, F, rows_hint) == 8
+                        ? (past ? launch_gemv16_pair<8, true> : launch_gemv16_pair<8, false>)
+                        : (past ? launch_gemv16_pair<16, true> : launch_gemv16_pair<16, false>);
+      return launch(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream);
     }
   }
   if (row_w != nullptr) {
@@ -817,10 +855,15 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
         return FS2MOE_ERR_UNSUPPORTED;
       }
     }
-    auto launch = [&](auto dual_tag, const void* a, const int32_t* map, int lda, const void* w0,
+    const Groups grp{counts, offsets, E, 0, (int)planned};
+    // (chunks of 16 rows share an expert's weights in L2: 126 rows of 8 experts, D 1344, F 14080 140 us with them there,
+    // 151 past it; 14 rows, D 4864, F 11136 260, 236; 64 tokens, top-8 of 128, D 2048, F 768 73.5, 70.4)
+    const int64_t pairs = pairs_of(grp, max_rows);
+    const bool past = pairs <= 8ll * E && weights_past_cache(E, pairs, D, F, 1);
+    auto launch = [&](auto dual_tag, auto nt_tag, const void* a, const int32_t* map, int lda, const void* w0,
                       const void* w1, const float* s0, const float* s1, void* c, int ldc, int kdim,
                       int n) {
-      constexpr bool DUAL = decltype(dual_tag)::value;
+      constexpr bool DUAL = decltype(dual_tag)::value, NT = decltype(nt_tag)::value;
       const uint16_t* ap = static_cast<const uint16_t*>(a);
       const uint8_t* w0p = static_cast<const uint8_t*>(w0);
       const uint8_t* w1p = static_cast<const uint8_t*>(w1);
@@ -828,20 +871,23 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
       const unsigned grid = (DUAL ? 4u : 3u) * cu_blocks;  // the kernels' launch bounds
       if (kdim >= 512) {
         constexpr int CGW = DUAL ? 2 : 4;
-        hipLaunchKernelGGL((glu_gemm_fp8w_kernel<DUAL, 4, CGW>), dim3(grid), dim3(256), 0, st, ap,
+        hipLaunchKernelGGL((glu_gemm_fp8w_kernel<DUAL, 4, CGW, NT>), dim3(grid), dim3(256), 0, st, ap,
                            map, lda, w0p, w1p, s0, s1, cp, ldc, kdim, n, counts, offsets, E,
                            n / 16 / CGW);
       } else {
         constexpr int CGW = DUAL ? 1 : 2;
-        hipLaunchKernelGGL((glu_gemm_fp8w_kernel<DUAL, 2, CGW>), dim3(grid), dim3(256), 0, st, ap,
+        hipLaunchKernelGGL((glu_gemm_fp8w_kernel<DUAL, 2, CGW, NT>), dim3(grid), dim3(256), 0, st, ap,
                            map, lda, w0p, w1p, s0, s1, cp, ldc, kdim, n, counts, offsets, E,
                            n / 16 / (2 * CGW));
       }
     };
-    launch(std::true_type{}, xe, row_map, D, w_gate, w_up, s_gate, s_up, h, F, D, F);
-    if (int rc = check_launch("glu_gemm_fp8w<gate,up>")) return rc;
-    launch(std::false_type{}, h, nullptr, F, w_down, nullptr, s_down, nullptr, ye, D, F, D);
-    return check_launch("glu_gemm_fp8w<down>");
+    auto pair = [&](auto nt) -> int {
+      launch(std::true_type{}, nt, xe, row_map, D, w_gate, w_up, s_gate, s_up, h, F, D, F);
+      if (int rc = check_launch("glu_gemm_fp8w<gate,up>")) return rc;
+      launch(std::false_type{}, nt, h, nullptr, F, w_down, nullptr, s_down, nullptr, ye, D, F, D);
+      return check_launch("glu_gemm_fp8w<down>");
+    };
+    return past ? pair(std::true_type{}) : pair(std::false_type{});
   }
   if (w_dtype != act_dtype) {
     set_error("grouped_swiglu: weight dtype %d with activation dtype %d has no kernel", w_dtype,

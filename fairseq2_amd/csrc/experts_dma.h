@@ -50,6 +50,8 @@
 //     touches land 64 B apart.
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 #include "tile_map.h"
 
@@ -148,7 +150,9 @@ struct TileOrder {
 // SPLIT (single matrix, with KTAIL): the sum over K in parts, for launches of few tiles and a long K.  The tiles are
 // those of `ldc` parts (C's rows are N wide), part-major within a row block, n_tiles counts them all; part p of C
 // [ldc][rows][N] f32 is the sum over its units, and split_sum_kernel adds the parts.
-template <bool DUAL, int BLAYOUT, bool KEEP_GU = false, bool TWO_SRC = false, bool KTAIL = false, bool SPLIT = false>
+// ONCE: the weights are loaded past the caches (load_once), for launches most of whose experts have one row block.
+template <bool DUAL, int BLAYOUT, bool KEEP_GU = false, bool TWO_SRC = false, bool KTAIL = false, bool SPLIT = false,
+          bool ONCE = false>
 __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
     const uint16_t* __restrict__ A, const int32_t* __restrict__ row_map, int lda,
     const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1,
@@ -471,16 +475,19 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
       const int p = q + 4 * i;
       return ROWS * (DUAL ? (p & 7) : p) + lane / CHUNKS;
     };
-    auto piece = [&](bool in_k, const uint8_t* base, uint32_t off) -> u32x4 {
+    auto piece = [&](auto once, bool in_k, const uint8_t* base, uint32_t off) -> u32x4 {
+      constexpr bool PAST = decltype(once)::value;
       if constexpr (KTAIL) {
         // (the host keeps every valid offset below 2^32 - 16)
         const __amdgpu_buffer_rsrc_t rsrc =
             __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), 0, 0xfffffff0u, 0x00020000);
-        return __builtin_amdgcn_raw_buffer_load_b128(rsrc, in_k ? off : 0xfffffff0u, 0, 0);
+        return __builtin_amdgcn_raw_buffer_load_b128(rsrc, in_k ? off : 0xfffffff0u, 0, PAST ? kNonTemporal : 0);
       } else {
-        return *reinterpret_cast<const u32x4*>(base + off);
+        return load_weights<PAST>(base + off);
       }
     };
+    const std::false_type shared{};                       // rows: other tiles of their row block read them
+    const std::integral_constant<bool, ONCE> weights{};
     auto k_left = [&](int ku) { return Kdim - ku * (2 * BK); };  // k of unit ku and those after it
     // Unit ku of the tile set up last -> registers.
     auto load_unit = [&](int ku) {
@@ -494,13 +501,13 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
       const bool kc_ok = tail_kc * 8 < left;
 #pragma unroll
       for (int jj = 0; jj < 8; ++jj)
-        if (jj < a_pieces) stage[jj] = piece(kc_ok, abase, pa[jj]);
+        if (jj < a_pieces) stage[jj] = piece(shared, kc_ok, abase, pa[jj]);
       if constexpr (FP8) {
         const uint8_t* bg = reinterpret_cast<const uint8_t*>(ld_bg) + (size_t)ku * 1024;
         const uint8_t* bu = reinterpret_cast<const uint8_t*>(ld_bu) + (size_t)ku * 1024;
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj)
-          stage[8 + jj] = *reinterpret_cast<const u32x4*>((jj < 2 ? bg : bu) + pb[jj]);
+          stage[8 + jj] = load_weights<ONCE>((jj < 2 ? bg : bu) + pb[jj]);
         stage_scale_slot = ku == 0 ? ((ld_tiles - 1) & 1) : -1;
         stage_scale = ld_scale;
       } else if constexpr (KN) {
@@ -512,7 +519,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
           // pieces q, q+4 (gate when DUAL) and q+8, q+12 (up when DUAL)
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            stage[8 + 4 * h + i] = piece(h * BK + tail_row(i) < left, i < 2 ? bg : bu, pb[i]);
+            stage[8 + 4 * h + i] = piece(weights, h * BK + tail_row(i) < left, i < 2 ? bg : bu, pb[i]);
         }
       } else {
         const uint8_t* bg =
@@ -521,7 +528,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
             TWO_SRC ? bg : reinterpret_cast<const uint8_t*>(ld_bu + (size_t)ku * (2 * BK));
         // pieces q + 4 jj: jj < 4 lie in rows 0..127 (gate when DUAL), the rest in rows 128..255
 #pragma unroll
-        for (int jj = 0; jj < 8; ++jj) stage[8 + jj] = piece(kc_ok, jj < 4 ? bg : bu, pb[jj]);
+        for (int jj = 0; jj < 8; ++jj) stage[8 + jj] = piece(weights, kc_ok, jj < 4 ? bg : bu, pb[jj]);
       }
       stage_pieces = a_pieces;
     };
@@ -601,7 +608,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
 #pragma unroll
         for (int jj = 0; jj < 8; ++jj) {
           if (jj < stage_pieces) *reinterpret_cast<u32x4*>(dst + jj * 4096) = stage[jj];
-          if (jj < a_pieces) stage[jj] = piece(kc_ok, abase, pa[jj]);
+          if (jj < a_pieces) stage[jj] = piece(shared, kc_ok, abase, pa[jj]);
         }
         if constexpr (KN) {
 #pragma unroll
@@ -612,7 +619,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               *reinterpret_cast<u32x4*>(dst + A_BYTES + (4 * h + i) * 4096) = stage[8 + 4 * h + i];
-              stage[8 + 4 * h + i] = piece(h * BK + tail_row(i) < left, i < 2 ? bg : bu, pb[i]);
+              stage[8 + 4 * h + i] = piece(weights, h * BK + tail_row(i) < left, i < 2 ? bg : bu, pb[i]);
             }
           }
         } else {
@@ -623,7 +630,7 @@ __global__ __launch_bounds__(dma::NWAVES * 64) void glu_gemm_bf16_dma_kernel(
 #pragma unroll
           for (int jj = 0; jj < 8; ++jj) {
             *reinterpret_cast<u32x4*>(dst + A_BYTES + jj * 4096) = stage[8 + jj];
-            stage[8 + jj] = piece(kc_ok, jj < 4 ? bg : bu, pb[jj]);
+            stage[8 + jj] = piece(weights, kc_ok, jj < 4 ? bg : bu, pb[jj]);
           }
         }
         stage_pieces = a_pieces;

@@ -39,7 +39,7 @@ namespace fs2moe {
 // channels (the groups share the activation loads).  K is walked 4 blocks of 64 at a time with all
 // of a step's loads issued before any conversion or MFMA: every step is one round trip to memory,
 // with 4 * (CW * (DUAL ? 2 : 1) + 2) loads of 1 KB in flight per wave.
-template <bool DUAL, int CW>
+template <bool DUAL, int CW, bool NT>
 __device__ __forceinline__ void fp8w_partial(const uint16_t* __restrict__ xr,
                                              const uint8_t* __restrict__ wg,
                                              const uint8_t* __restrict__ wu, size_t group_stride,
@@ -54,8 +54,8 @@ __device__ __forceinline__ void fp8w_partial(const uint16_t* __restrict__ xr,
 #pragma unroll
       for (int c = 0; c < CW; ++c) {
         const size_t off = c * group_stride + (size_t)(kb0 + u) * 1024;
-        qg[u][c] = *reinterpret_cast<const u32x4*>(wg + off);
-        if (DUAL) qu[u][c] = *reinterpret_cast<const u32x4*>(wu + off);
+        qg[u][c] = load_weights<NT>(wg + off);
+        if (DUAL) qu[u][c] = load_weights<NT>(wu + off);
       }
       const u32x4* p = reinterpret_cast<const u32x4*>(xr + (size_t)(kb0 + u) * 64);
       xa[u][0] = p[0];
@@ -96,9 +96,10 @@ __device__ __forceinline__ void fp8w_partial(const uint16_t* __restrict__ xr,
 
 // row_map (may be null): activation row r is read from A[row_map[r]] instead of A[r].
 // A [rows, Kdim] bf16; W0/W1 tiled e4m3 [E][N/16][Kdim/64][16][64]; S0/S1 [E, N] f32; C [rows, N] bf16.
+// NT: the weights are loaded past the caches (load_once), for launches most of whose experts have one chunk.
 // n_blocks = N / (16 * CGW * (4 / KS)) channel blocks per expert (the host picks KS and CGW so that
 // this divides); any grid size works, E <= 256 = the block size.
-template <bool DUAL, int KS, int CGW>
+template <bool DUAL, int KS, int CGW, bool NT>
 __global__ __launch_bounds__(256, DUAL ? 4 : 3) void glu_gemm_fp8w_kernel(
     const uint16_t* __restrict__ A, const int32_t* __restrict__ row_map, int lda,
     const uint8_t* __restrict__ W0, const uint8_t* __restrict__ W1,
@@ -187,8 +188,8 @@ __global__ __launch_bounds__(256, DUAL ? 4 : 3) void glu_gemm_fp8w_kernel(
       accg[c] = f32x4{0.f, 0.f, 0.f, 0.f};
       accu[c] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    fp8w_partial<DUAL, CGW>(A + (size_t)src * lda + 16 * g, W0 + wrow, DUAL ? W1 + wrow : W0,
-                            group_stride, kb_lo, kb_hi, accg, accu);
+    fp8w_partial<DUAL, CGW, NT>(A + (size_t)src * lda + 16 * g, W0 + wrow, DUAL ? W1 + wrow : W0,
+                                group_stride, kb_lo, kb_hi, accg, accu);
     if (item != (int)blockIdx.x) __syncthreads();  // the last item's partial sums have been consumed
 #pragma unroll
     for (int c = 0; c < CGW; ++c) {

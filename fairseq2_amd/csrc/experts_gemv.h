@@ -87,7 +87,8 @@ __device__ __forceinline__ int nth_active_expert(const int32_t* __restrict__ cou
 // and multiplied by row_w[offset + r] on the way into LDS when that is given (rounded to bf16: the
 // bits dispatch's scaled row copy would have held).
 // grid: (ceil(N / 64), as many experts at a time as fill the chip).  K a multiple of 4, N a multiple of 8.
-template <bool DUAL, int R, bool DEEP = false>
+// NT: the weights are loaded past the caches (load_once).
+template <bool DUAL, int R, bool NT, bool DEEP = false>
 __global__ __launch_bounds__(gemv::threads(R)) void glu_gemv_bf16_kernel(
     const uint16_t* __restrict__ A, const int32_t* __restrict__ row_map,
     const float* __restrict__ row_w, int lda,
@@ -130,7 +131,7 @@ __global__ __launch_bounds__(gemv::threads(R)) void glu_gemv_bf16_kernel(
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int m = 0; m < M; ++m) wv[set][m][j] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc[m], at, j * N * 2, 0);
+      for (int m = 0; m < M; ++m) wv[set][m][j] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc[m], at, j * N * 2, NT ? kNonTemporal : 0);
     at += (uint32_t)KSTEP * (uint32_t)N * 2u;
   };
   const int steps = (K + KSTEP - 1) / KSTEP;
@@ -328,7 +329,7 @@ inline bool fits(int K, int XR) { return lds_bytes(K, XR, true) <= (size_t)MAX_L
 // (The second launch bound is waves per SIMD: the single product is held to 128 registers so that
 // two blocks share a CU -- the down projection of 20 active experts is 320 blocks, which at one block
 // per CU ran as a full round and a quarter-full one: 4 us of 75 at 8 tokens.)
-template <bool DUAL, int XR>
+template <bool DUAL, int XR, bool NT>
 __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16_kernel(
     const uint16_t* __restrict__ A, const int32_t* __restrict__ row_map,
     const float* __restrict__ row_w, int lda,
@@ -376,7 +377,7 @@ __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16
         for (int j = 0; j < 4; ++j)
 #pragma unroll
           for (int m = 0; m < M; ++m)
-            wq[set][h][m][j] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc[m], at, j * N * 2, 0);
+            wq[set][h][m][j] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc[m], at, j * N * 2, NT ? kNonTemporal : 0);
         at += (uint32_t)KSTEP * (uint32_t)N * 2u;
       }
     };
@@ -558,7 +559,7 @@ constexpr int MAX_ROWS = 16;
 
 // DUAL: C[r, n] = SiLU(A[r] . B0[n]) * (A[r] . B1[n]); else C[r, n] = A[r] . B0[n].
 // A [T][lda], B0/B1 [N][K], C [T][ldc]; T <= 16; K and N multiples of 8.  grid: ceil(N / 16).
-template <bool DUAL>
+template <bool DUAL, bool NT>
 __global__ __launch_bounds__(dgemv::THREADS) void dense_gemv_bf16_kernel(
     const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, uint16_t* __restrict__ C, int ldc, int K, int N, int T) {
@@ -584,8 +585,8 @@ __global__ __launch_bounds__(dgemv::THREADS) void dense_gemv_bf16_kernel(
     for (int u = 0; u < U; ++u) {
       const int k = (s0 + u * WAVES) * 32 + g * 8;
       const int kk = k < K ? k : 0;  // K is a multiple of 8: the lane's eight k are in or out together
-      wq[u][0] = *reinterpret_cast<const u32x4*>(w0 + kk);
-      if (DUAL) wq[u][M - 1] = *reinterpret_cast<const u32x4*>(w1 + kk);
+      wq[u][0] = load_weights<NT>(w0 + kk);
+      if (DUAL) wq[u][M - 1] = load_weights<NT>(w1 + kk);
       xq[u] = *reinterpret_cast<const u32x4*>(xr + kk);
     }
     // (all the loads are issued before the first is waited for)

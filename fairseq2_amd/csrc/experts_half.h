@@ -57,6 +57,10 @@ constexpr int stages(int BM, int BNV, int layout) {
 constexpr int smem_bytes(int BM, int BNV, int layout) {
   return stages(BM, BNV, layout) * stage_bytes(BM, BNV, layout) + EPI_BYTES + TABLE_INTS * 4;
 }
+// Up to how many rows an expert has on average the weights are loaded past the caches (twice as many: the same times).
+// us without and with: 89 tokens, top-4 of 60, D 2048, F 1152 183, 171; 26, top-8 of 32, D 960, F 1536 99, 93; a training
+// step of 494, top-1 of 16, D 2176, F 8320 1212, 1178.
+inline int64_t once_rows(int BM) { return BM / 2; }
 constexpr uint32_t NOWHERE = 0xfffffff0u;      // an offset past any buffer's end
 
 // Which of these tiles a launch takes: 0 none (the throughput kernel), else the smallest whose tiles are about
@@ -105,15 +109,20 @@ inline int pick(bool dual, bool single, int64_t rows, int groups, int K, int N, 
 
 // 16 bytes per lane from a buffer to LDS, lane l's to lds + 16 l.  Written out because the compiler, which cannot
 // tell the ring's stages apart, would wait for every load in flight before each LDS read.  The caller waits
-// (vmcnt) in front of the barrier that hands the stage over.  BYTES 4: lane l's four to lds + 4 l.
+// (vmcnt) in front of the barrier that hands the stage over.  BYTES 4: lane l's four to lds + 4 l.  PAST: past the
+// caches (load_once).
 // (m0 is named because the other kernels' loads to LDS set it as well; the compiler warns that it reserves it.)
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-template <int BYTES>
+template <int BYTES, bool PAST = false>
 __device__ __forceinline__ void buffer_to_lds(const void* base, uint32_t off, uint32_t lds) {
   const uint64_t b = (uint64_t)base;
   const u32x4 rsrc = {(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, half_tiles::NOWHERE, 0x00020000u};
-  if constexpr (BYTES == 16)
+  if constexpr (BYTES == 16 && PAST)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen nt lds" ::"v"(off), "s"(rsrc),
+                 "s"(lds)
+                 : "memory", "m0");
+  else if constexpr (BYTES == 16)
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc),
                  "s"(lds)
                  : "memory", "m0");
@@ -135,7 +144,8 @@ struct HalfMx {
 // Arguments as glu_gemm_bf16_dma_kernel takes them (KEEP_GU: the products' destinations in S0 and S1; TWO_SRC:
 // the second activations in S0, the second weights in B1), or for W_MX as glu_gemm_mx_kernel does.  n_tiles: of 64
 // (DUAL) or 128 channels.
-template <int BM, int BNV, bool DUAL, int BLAYOUT, bool KEEP_GU = false, bool TWO_SRC = false>
+// ONCE: the weights are loaded past the caches, for launches most of whose experts have one row block.
+template <int BM, int BNV, bool DUAL, int BLAYOUT, bool KEEP_GU = false, bool TWO_SRC = false, bool ONCE = false>
 __global__ __launch_bounds__(half_tiles::THREADS, 2) void glu_gemm_half_kernel(
     const uint8_t* __restrict__ A, const int32_t* __restrict__ row_map, int lda,
     const uint8_t* __restrict__ B0, const uint8_t* __restrict__ B1, const float* __restrict__ S0,
@@ -323,14 +333,14 @@ __global__ __launch_bounds__(half_tiles::THREADS, 2) void glu_gemm_half_kernel(
     } else {
       const uint8_t* src = TWO_SRC ? ld_b[second ? 1 : 0] : ld_b[DUAL ? (FP8 ? wave >> 2 : i) : 0];
       if constexpr (FP8) {
-        buffer_to_lds<16>(src + (size_t)ku * 1024, left > 0 ? pb[i] : NOWHERE, at);
+        buffer_to_lds<16, ONCE>(src + (size_t)ku * 1024, left > 0 ? pb[i] : NOWHERE, at);
       } else if constexpr (MX) {
-        buffer_to_lds<16>(src + (size_t)ku * 2048, left > 0 ? pb[i] : NOWHERE, at);
+        buffer_to_lds<16, ONCE>(src + (size_t)ku * 2048, left > 0 ? pb[i] : NOWHERE, at);
       } else if constexpr (KN) {
         const int k = KROWS * (DUAL ? wave : wave + 8 * i) + lane / KCHUNKS;
-        buffer_to_lds<16>(src + (size_t)ku * KU * N * 2, k < left ? pb[i] : NOWHERE, at);
+        buffer_to_lds<16, ONCE>(src + (size_t)ku * KU * N * 2, k < left ? pb[i] : NOWHERE, at);
       } else {
-        buffer_to_lds<16>(src + (size_t)ku * ROW_BYTES, kc * 8 < left ? pb[i] : NOWHERE, at);
+        buffer_to_lds<16, ONCE>(src + (size_t)ku * ROW_BYTES, kc * 8 < left ? pb[i] : NOWHERE, at);
       }
     }
   };

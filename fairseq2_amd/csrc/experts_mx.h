@@ -81,7 +81,8 @@ __device__ __forceinline__ int mx_tile_row(int lane) {
 // work removed).  This way consecutive rows are consecutive dwords: expert-major rows (the gated
 // product) always are, and token rows read through the permutation mostly are for the experts
 // that take most tokens, whose rows are dense runs of token numbers.
-template <bool DUAL>
+// ONCE: the weights are loaded past the caches, as in experts_dma.h.
+template <bool DUAL, bool ONCE = false>
 __global__ __launch_bounds__(mx::NWAVES * 64) void glu_gemm_mx_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ As,
     const int32_t* __restrict__ row_map, const uint8_t* __restrict__ B0,
@@ -304,12 +305,13 @@ __global__ __launch_bounds__(mx::NWAVES * 64) void glu_gemm_mx_kernel(
       const __amdgpu_buffer_rsrc_t bg = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(ld_b[0]), 0, -1, 0x00020000);
       const __amdgpu_buffer_rsrc_t bu = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(ld_b[1]), 0, -1, 0x00020000);
       const uint32_t koff_w = (uint32_t)ku * 2048u;  // two tiles along k per unit
+      constexpr int WEIGHTS = ONCE ? kNonTemporal : 0;
 #pragma unroll
       for (int jj = 0; jj < 8; ++jj) {
         if (DUAL && jj >= 4)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(bu, (lds_ptr)(base + A_BYTES + (q + 4 * jj) * 1024), 16, pb[jj], koff_w, 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(bu, (lds_ptr)(base + A_BYTES + (q + 4 * jj) * 1024), 16, pb[jj], koff_w, 0, WEIGHTS);
         else
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(bg, (lds_ptr)(base + A_BYTES + (q + 4 * jj) * 1024), 16, pb[jj], koff_w, 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(bg, (lds_ptr)(base + A_BYTES + (q + 4 * jj) * 1024), 16, pb[jj], koff_w, 0, WEIGHTS);
       }
       if (ku == 0) s_wscale[((ld_tiles - 1) & 1) * BNV + 64 * q + lane] = ld_scale;
     };

@@ -114,12 +114,19 @@ int fs2moe::grouped_swiglu_w8a8_planned(const void* xq, const void* xs, const in
   if (max_rows == 0) return FS2MOE_OK;
   FS2_REQUIRE(x_rows * (int64_t)D <= 0xffffffffll, "grouped_swiglu_w8a8: xq is addressed with 32-bit byte offsets");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  auto k1 = glu_gemm_mx_kernel<true>;
-  auto k2 = glu_gemm_mx_kernel<false>;
+  Groups g{counts, offsets, E, 0, (int)planned};
+  g.once_past_cache = weights_past_cache(E, pairs_of(g, max_rows), D, F, 1);
+  // (us without and with, loaded evenly and by a popularity law: 1100 tokens, top-8 of 128, D 2048, F 768 181, 172 and 170,
+  // 166; 2000 202, 193 and 215, 214; 1100, top-2 of 16, D 4096, F 4096 219, 208 and 278, 275)
+  const bool once = g.once_past_cache && pairs_of(g, max_rows) <= kOnceRows * E;
+  auto k1 = once ? glu_gemm_mx_kernel<true, true> : glu_gemm_mx_kernel<true>;
+  auto k2 = once ? glu_gemm_mx_kernel<false, true> : glu_gemm_mx_kernel<false>;
   static bool attr_set = false;  // benign race: setting the attribute is idempotent
   if (!attr_set) {
-    const void* ks[2] = {reinterpret_cast<const void*>(k1), reinterpret_cast<const void*>(k2)};
-    for (const void* k : ks) {
+    for (const void* k : {reinterpret_cast<const void*>(glu_gemm_mx_kernel<true>),
+                          reinterpret_cast<const void*>(glu_gemm_mx_kernel<false>),
+                          reinterpret_cast<const void*>(glu_gemm_mx_kernel<true, true>),
+                          reinterpret_cast<const void*>(glu_gemm_mx_kernel<false, true>)}) {
       hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_BYTES);
       if (e != hipSuccess) {
         set_error("grouped_swiglu_w8a8: cannot reserve %d bytes of LDS: %s", SMEM_BYTES,
@@ -142,7 +149,6 @@ int fs2moe::grouped_swiglu_w8a8_planned(const void* xq, const void* xs, const in
       return FS2MOE_ERR_UNSUPPORTED;
     }
   }
-  Groups g{counts, offsets, E, 0, (int)planned};
   // Few tiles: the smaller tiles of experts_half.h (the same bits).
   auto half = [&](auto bm_c, auto dual_c, const void* a, const void* as, const int32_t* map, int K, const void* b0,
                   const void* b1, const float* s0, const float* s1, void* c, void* cs, int N, int64_t a_rows,
@@ -150,17 +156,20 @@ int fs2moe::grouped_swiglu_w8a8_planned(const void* xq, const void* xs, const in
     constexpr int HBM = decltype(bm_c)::value, HBN = 128;
     constexpr bool DUAL = decltype(dual_c)::value;
     constexpr int bytes = half_tiles::smem_bytes(HBM, HBN, half_tiles::W_MX), bn = DUAL ? HBN / 2 : HBN;
-    auto k = glu_gemm_half_kernel<HBM, HBN, DUAL, half_tiles::W_MX>;
+    auto shared = glu_gemm_half_kernel<HBM, HBN, DUAL, half_tiles::W_MX>;
+    auto past = glu_gemm_half_kernel<HBM, HBN, DUAL, half_tiles::W_MX, false, false, true>;
     static bool half_attr_set = false;  // benign race: setting the attribute is idempotent
     if (!half_attr_set) {
-      hipError_t e =
-          hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-      if (e != hipSuccess) {
-        set_error("%s: cannot reserve %d bytes of LDS: %s", what, bytes, hipGetErrorString(e));
-        return FS2MOE_ERR_LAUNCH;
+      for (const void* k : {reinterpret_cast<const void*>(shared), reinterpret_cast<const void*>(past)}) {
+        hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+        if (e != hipSuccess) {
+          set_error("%s: cannot reserve %d bytes of LDS: %s", what, bytes, hipGetErrorString(e));
+          return FS2MOE_ERR_LAUNCH;
+        }
       }
       half_attr_set = true;
     }
+    auto k = g.once_past_cache && pairs_of(g, max_rows) / E <= half_tiles::once_rows(HBM) ? past : shared;
     hipLaunchKernelGGL(k, dim3((unsigned)num_blocks), dim3(half_tiles::THREADS), bytes, st,
                        static_cast<const uint8_t*>(a), map, K, static_cast<const uint8_t*>(b0),
                        static_cast<const uint8_t*>(b1), s0, s1, static_cast<uint8_t*>(c), N, K, N, g,

@@ -13,8 +13,30 @@ struct Groups {
   // host: the planned rows (common.h) where the caller knows them, else 0 and the buffers' size stands for them; the
   // choice of tiles goes by them, while grids and addresses go by the buffers
   int planned = 0;
+  // whether weights that one tile alone reads are loaded past the caches (load_once)
+  int once_past_cache = 0;
   int64_t rows_to_plan(int64_t bound) const { return counts != nullptr && planned > 0 ? planned : bound; }
 };
+
+// Whether the weights that a call's `pairs` rows can reach are more than the last-level cache (256 MB) holds: what is read
+// once is then loaded past the caches, where otherwise some of it may still lie there from the call before.  D 2048,
+// F 768, 128 experts, top-8 (9.4 MB an expert), us of the layer without and with the hint: one token (75 MB) 36.1, 40.1
+// where its experts' weights are in that cache, 42.1, 41.2 where they are not; 8 tokens (at most 604 MB) 79.6, 75.2.
+// Whole layers of 262 MB, by a popularity law, which leaves some experts out: 60 of D 704, F 1088, 720 tokens 66.0, 69.5;
+// of 288 MB 62.9, 64.5 (128 of D 768, F 512), 86.8, 84.3 (64 of D 1024, F 768); of 432 MB 125, 121.  One group, the
+// shared expert, counts for more: the routed ones' weights go by beside it.
+inline bool weights_past_cache(int groups, int64_t pairs, int64_t D, int64_t F, int weight_bytes) {
+  const int64_t reached = groups == 0 ? 1 : pairs < groups ? pairs : groups;
+  return reached * 3 * D * F * weight_bytes > (groups == 0 ? 128ll << 20 : 320ll << 20);
+}
+// (the rows of experts that are not planned: as many as the buffers hold)
+inline int64_t pairs_of(const Groups& g, int64_t rows_bound) {
+  return g.counts != nullptr && g.planned > 15ll * g.E ? g.planned - 15ll * g.E : rows_bound;
+}
+
+// Up to how many rows an expert has on average most tiles of 256 rows are their expert's only row block (launch_dma has
+// the times).
+constexpr int64_t kOnceRows = 128, kOnceRowsTraining = 192;
 
 // Finds the (expert, row range) of m-tile `mt`.  All 256 threads of the block must call it.
 template <int BM>

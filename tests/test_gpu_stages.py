@@ -743,6 +743,57 @@ def test_f32_products_are_the_same_on_every_tile_size(gpu_device, k, n, layout):
     assert torch.equal(dense[0], dense[2][:32]) and torch.equal(dense[1], dense[2][:33])
 
 
+# Weights of more than half of the last-level cache are loaded past the caches where one block reads them (128 experts),
+# others through them (the first 8 of these experts alone): the same bits from every kernel that has both kinds of loads,
+# with K and N of whole units and lines, K off the units, and N off the lines.
+@pytest.mark.parametrize("d,f", [(1024, 512), (1000, 512), (1024, 520)])
+def test_weights_past_the_caches_give_the_same_bits(gpu_device, d, f):
+    _say("past the caches", d, f)
+    many, few, dev, bf = 128, 8, gpu_device, torch.bfloat16
+    assert 3 * d * f * 2 * few < 2**27 < 3 * d * f * 2 * 100
+    g = torch.Generator(dev).manual_seed(d + f)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(bf)
+    x, mid = rnd(4608, d), rnd(4608, f)
+    wg, wu, wd = rnd(many * d, f) * 0.05, rnd(many * d, f) * 0.05, rnd(many * f, d) * 0.05
+
+    def both(rows, total, run):
+        """``run(counts, offsets, experts, total)`` with all experts and with the first few."""
+        out = []
+        for e in (many, few):
+            counts = torch.tensor(rows + [0] * (e - few), dtype=torch.int32, device=dev)
+            offsets = torch.zeros(e + 1, dtype=torch.int32, device=dev)
+            offsets[1:] = torch.cumsum((counts + 15) // 16 * 16, 0)
+            lo = offsets.tolist()
+            got = run(counts, offsets, e, total)
+            out.append([torch.cat([o[lo[i] : lo[i] + n] for i, n in enumerate(rows)]) for o in got])
+        assert all(torch.equal(a, b) for a, b in zip(*out))
+        return out[0]
+
+    w = lambda e: (wg[: e * d], wu[: e * d], wd[: e * f])
+    swiglu = lambda total, **kw: lambda c, o, e, t: _abi.grouped_swiglu(x[:t], c, o, *w(e), e, **kw)
+    for bound, rows in ((1, [1] * 8), (2, [2, 1, 2, 0, 2, 2, 2, 2]), (4, [4, 1, 3, 4, 4, 2, 4, 4]),
+                        (8, [8, 1, 5, 0, 7, 8, 8, 3]), (16, [16, 9, 1, 0, 12, 16, 5, 16])):
+        both(rows, 128, swiglu(128, rows_per_expert=bound))
+    rows = [300, 17, 0, 256, 257, 129, 1, 64]
+    total = sum((n + 15) // 16 * 16 for n in rows)
+    both(rows, total, swiglu(total))
+    if _abi.keeps_products(d, f, total, bf):
+        both(rows, total, lambda c, o, e, t: _abi.grouped_swiglu_keep(x[:t], c, o, *w(e), e))
+        both(rows, total, lambda c, o, e, t: [_abi.grouped_gemm_sum(mid[:t], w(e)[0], mid[1000 : 1000 + t], w(e)[1], c, o, e)])
+    both(rows, total, lambda c, o, e, t: [_abi.grouped_gemm(x[:t], w(e)[2], _abi.W_OUT_IN, c, o, e)])
+    if d % 64 or f % 64:
+        return
+    packed = [_abi.pack_fp8_weights(t.to(torch.float8_e4m3fn), many) for t in (wg, wu, wd)]
+    scales = [torch.rand(many, n, generator=g, device=dev) + 0.5 for n in (f, f, d)]
+    both([16, 17, 1, 0, 33, 2, 9, 16], 160, lambda c, o, e, t: _abi.grouped_swiglu(
+        x[:t], c, o, *(q[:e] for q in packed), e, scales=tuple(s[:e] for s in scales)))
+    both(rows, 4608, lambda c, o, e, t: _abi.grouped_swiglu(
+        x[:t], c, o, *(q[:e] for q in packed), e, scales=tuple(s[:e] for s in scales)))
+    xq, xs = _abi.mx_quantize(x[:total].contiguous())
+    both(rows, total, lambda c, o, e, t: _abi.grouped_swiglu_w8a8(
+        xq, xs, c, o, *(q[:e] for q in packed), tuple(s[:e] for s in scales), e)[:2])
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
 @pytest.mark.parametrize(
     "t,d,f",
