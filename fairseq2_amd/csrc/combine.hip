@@ -47,9 +47,9 @@ struct Chunk<uint16_t> {
 };
 
 // KMAX: compile-time bound on K (slots beyond K carry row -1).  WPT: waves per token; the token's
-// 16-byte chunks are dealt round-robin to its waves (WPT = 4 when there are too few tokens to fill
-// the GPU with one wave each).
-template <typename TA, int KMAX, int WPT>
+// 16-byte chunks are dealt round-robin to its waves.  NT: the rows are loaded past the caches (load_once).
+// Bound by memory: 8192 tokens, top-8, D 2048, 302 MB in 53 us, 5.7 TB/s.
+template <typename TA, int KMAX, int WPT, bool NT>
 __global__ __launch_bounds__(kCombWaves* kWave) void combine_kernel(
     const TA* __restrict__ ye, const int32_t* __restrict__ inv_perm,
     const int32_t* __restrict__ topk_idx, const float* __restrict__ topk_w, const TA* base,
@@ -67,21 +67,14 @@ __global__ __launch_bounds__(kCombWaves* kWave) void combine_kernel(
     row = inv_perm[(size_t)t * K + lane];
     w = weight_output ? topk_w[(size_t)t * K + lane] : 1.0f;
   }
-  int pos = 0;
+  // (lanes K and up keep their places behind the list)
+  int pos = lane < K ? 0 : lane;
   for (int i = 0; i < K; ++i) {
-    int ei = __shfl(e, i, kWave);
-    pos += (ei < e || (ei == e && i < lane)) ? 1 : 0;
+    const int ei = __builtin_amdgcn_readlane(e, i);
+    if (lane < K) pos += (ei < e || (ei == e && i < lane)) ? 1 : 0;
   }
-  // Invert: lane s takes the slot whose position is s, so lanes 0..K-1 hold the sorted list.
-  int src = 0;
-  for (int i = 0; i < K; ++i) {
-    int pi = __shfl(pos, i, kWave);
-    if (pi == lane) src = i;
-  }
-  // lanes K .. KMAX-1 found no slot (src = 0): they must contribute nothing
-  const int picked_row = __shfl(row, src, kWave);
-  const int sorted_row = lane < K ? picked_row : -1;
-  const float sorted_w = __shfl(w, src, kWave);
+  const int sorted_row = __builtin_amdgcn_ds_permute(pos << 2, row);
+  const float sorted_w = __int_as_float(__builtin_amdgcn_ds_permute(pos << 2, __float_as_int(w)));
   // Wave-uniform copies of the sorted list (lanes >= K contributed row -1).
   int rj[KMAX];
   float wj[KMAX];
@@ -97,13 +90,14 @@ __global__ __launch_bounds__(kCombWaves* kWave) void combine_kernel(
   const u32x4* base4 = reinterpret_cast<const u32x4*>(base);
   const u32x4* res4 = reinterpret_cast<const u32x4*>(residual);
   u32x4* out4 = reinterpret_cast<u32x4*>(out);
-  const u32x4 zero4 = {0u, 0u, 0u, 0u};
+  const int rj0 = rj[0] >= 0 ? rj[0] : 0;
   for (int c = lane + kWave * part; c < chunks; c += kWave * WPT) {
-    // all of the chunk's loads are issued before the first add
+    // all of the chunk's loads are issued before the first add (a slot without a row loads the first one's: a condition
+    // would be a branch around each); no one else reads them
     u32x4 v[KMAX];
 #pragma unroll
-    for (int j = 0; j < KMAX; ++j)
-      v[j] = rj[j] >= 0 ? ye4[(size_t)rj[j] * chunks + c] : zero4;
+    for (int j = 0; j < KMAX; ++j) v[j] = load_weights<NT>(ye4 + (size_t)(rj[j] >= 0 ? rj[j] : rj0) * chunks + c);
+    __builtin_amdgcn_sched_barrier(0);
     float acc[N];
     if (base != nullptr) {
       Chunk<TA>::unpack(base4[(size_t)t * chunks + c], acc);
@@ -134,25 +128,31 @@ template <typename TA>
 static int launch_combine(const void* ye, const int32_t* inv_perm, const int32_t* topk_idx,
                           const float* topk_w, const void* base, const void* residual, int T, int K,
                           int D, int weight_output, void* out, hipStream_t s) {
-  const int wpt = T < 2048 ? 4 : 1;
+  // Two pieces of 64 chunks a wave where there are enough tokens: what a wave does before its first load counts for less,
+  // and more waves than run at once begin theirs under others' loads.  Rows of more than 64 MB are past what L2 keeps, and
+  // are loaded past it (less: 777 tokens, top-8, D 2048 10.2 us with the hint, 9.0 without).  us with one, two and four
+  // waves a token: 8192 tokens, top-8, D 2048 55.3, 53.0, 53.8 (without the hint and with the list sorted by exchanges
+  // 60.5); 2500, top-6, D 4096 30.6, 28.9, 27.4; 6000, top-8, D 1024 20.8, 21.5, 23.5.
+  const int chunks = D / Chunk<TA>::N;
+  const int wpt = T < 2048 || chunks >= 512 ? 4 : chunks >= 256 ? 2 : 1;
+  const bool past = (int64_t)T * K * D * (int64_t)sizeof(TA) > (64ll << 20);
   dim3 grid(((size_t)T * wpt + kCombWaves - 1) / kCombWaves), block(kCombWaves * kWave);
   const TA* yp = static_cast<const TA*>(ye);
   const TA* bp = static_cast<const TA*>(base);
   const TA* rp = static_cast<const TA*>(residual);
   TA* op = static_cast<TA*>(out);
-#define FS2_COMBINE_CASE(KM)                                                                      \
-  if (K <= KM) {                                                                                  \
-    if (wpt == 4)                                                                                 \
-      hipLaunchKernelGGL((combine_kernel<TA, KM, 4>), grid, block, 0, s, yp, inv_perm, topk_idx,  \
-                         topk_w, bp, rp, T, K, D, weight_output, op);                             \
-    else                                                                                          \
-      hipLaunchKernelGGL((combine_kernel<TA, KM, 1>), grid, block, 0, s, yp, inv_perm, topk_idx,  \
-                         topk_w, bp, rp, T, K, D, weight_output, op);                             \
-    return check_launch("combine");                                                               \
+#define FS2_COMBINE_CASE(KM)                                                                                \
+  if (K <= KM) {                                                                                            \
+    auto k = wpt == 4 ? (past ? combine_kernel<TA, KM, 4, true> : combine_kernel<TA, KM, 4, false>)         \
+             : wpt == 2 ? (past ? combine_kernel<TA, KM, 2, true> : combine_kernel<TA, KM, 2, false>)       \
+                        : (past ? combine_kernel<TA, KM, 1, true> : combine_kernel<TA, KM, 1, false>);      \
+    hipLaunchKernelGGL(k, grid, block, 0, s, yp, inv_perm, topk_idx, topk_w, bp, rp, T, K, D, weight_output, op); \
+    return check_launch("combine");                                                                         \
   }
   FS2_COMBINE_CASE(1)
   FS2_COMBINE_CASE(2)
   FS2_COMBINE_CASE(4)
+  FS2_COMBINE_CASE(6)
   FS2_COMBINE_CASE(8)
   FS2_COMBINE_CASE(16)
   FS2_COMBINE_CASE(32)

@@ -84,9 +84,7 @@ __global__ __launch_bounds__(256) void swiglu_backward_pairs_kernel(
   const size_t base = (size_t)row * F;
   float dot = 0.f;
   for (int c = lane * 8; c < F; c += 512) {
-    const u32x4 gv = *reinterpret_cast<const u32x4*>(g + base + c);
-    const u32x4 uv = *reinterpret_cast<const u32x4*>(u + base + c);
-    const u32x4 fv = *reinterpret_cast<const u32x4*>(h_fwd + base + c);
+    const u32x4 gv = load_once(g + base + c), uv = load_once(u + base + c), fv = load_once(h_fwd + base + c);
     const u32x4 dv = *reinterpret_cast<const u32x4*>(dh + base + c);
     u32x4 hv, gov, uov;
 #pragma unroll

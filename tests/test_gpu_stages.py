@@ -912,6 +912,24 @@ def test_combine_matches_oracle(gpu_device, dtype, weight_output, with_base, k):
         assert float((got - want).abs().max()) <= float(want.abs().max()) * (2**-7 if dtype == "bf16" else 2**-22)
 
 
+# One, two and four waves a token, through the caches and past them, rows off a wave's pieces, lists shorter than the
+# compile-time one: without weights the sum is bit-exact.
+@pytest.mark.parametrize("t,d,k,dtype", [(2048, 512, 3, "bf16"), (2049, 2056, 6, "bf16"), (2300, 2048, 8, "bf16"),
+                                         (4100, 1032, 9, "bf16"), (2048, 4096, 5, "bf16"), (2050, 1028, 4, "fp32"),
+                                         (2047, 4096, 2, "bf16")])
+def test_combine_by_rows_and_tokens(gpu_device, t, d, k, dtype):
+    _say("combine", t, d, k, dtype)
+    g, dev, dt = torch.Generator(gpu_device).manual_seed(t + d), gpu_device, TORCH_DTYPE[dtype]
+    idx = torch.rand(t, 32, generator=g, device=dev).argsort(dim=1)[:, :k]
+    inv = torch.randperm(t * k, generator=g, device=dev).view(t, k)
+    ye, base = (torch.randn(n, d, generator=g, device=dev).to(dt) for n in (t * k, t))
+    out = _abi.combine(ye, inv.to(torch.int32), idx.to(torch.int32).contiguous(), torch.rand(t, k, device=dev), base, False)
+    acc, order = base.float(), idx.argsort(dim=1)
+    for j in range(k):
+        acc = acc + ye[inv.gather(1, order[:, j : j + 1])[:, 0]].float()
+    assert torch.equal(out, acc.to(dt))
+
+
 # ------------------------------------------------------------------------ experts, fp8 weights
 @pytest.mark.parametrize(
     "rows_per_expert,d,f",
