@@ -1166,6 +1166,13 @@ static int wgrad_segments(int64_t rows, int M, int N) {
   return s >= 2 ? (int)s : 1;
 }
 
+// (the f32 tiles are smaller: enough segments for two blocks to a CU)
+static int wgrad_segments_f32(int64_t rows, int M, int N) {
+  const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64), enough = (511 + tiles) / tiles;
+  const int segments = wgrad_segments(rows, M, N);
+  return segments < enough ? segments : (int)enough;
+}
+
 // A gradient is written once and not read here, and as ordinary stores its lines push the operands' rows,
 // which other tiles read again, out of L2: 128 experts of 256 rows, 2048 x 768, 207 us with ordinary and
 // 186 us with non-temporal stores (bf16); 8 of 71 rows, 4288 x 5504, 108 and 97.  But rows that do not begin on a
@@ -1196,6 +1203,23 @@ static int launch_wgrad_reduce(const float* partial, int segments, int64_t n, in
 }
 
 // One launch for all gradients of `jobs`; the grouped ones share counts and offsets.
+// The f32 gradients of one call.
+static int launch_wgrad_f32(F32WgradJobs& jobs, const int32_t* a_map, const int32_t* counts, const int32_t* offsets, int E,
+                            hipStream_t st) {
+  int64_t blocks = 0;
+  for (int i = 0; i < jobs.n; ++i) {
+    F32WgradJob& j = jobs.job[i];
+    j.m_tiles = (j.M + 63) / 64;
+    j.n_tiles = (j.N + 63) / 64;
+    j.first = (int)blocks;
+    blocks += (int64_t)(j.grouped ? E : j.segments) * j.m_tiles * j.n_tiles;
+    FS2_REQUIRE(blocks <= 0x7fffffffll, "grouped_wgrad: too many tiles");
+  }
+  const Groups g{counts, offsets, E, 0};
+  auto k = a_map != nullptr ? grouped_wgrad_f32_kernel<true> : grouped_wgrad_f32_kernel<false>;
+  hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(f32t::threads(1)), 0, st, jobs, a_map, g);
+  return check_launch("grouped_wgrad");
+}
 static int launch_wgrad(const WgradJobs& jobs, const int32_t* row_map, const int32_t* counts,
                         const int32_t* offsets, int E, hipStream_t st) {
   auto k = row_map != nullptr ? grouped_wgrad_kernel<true> : grouped_wgrad_kernel<false>;
@@ -1249,19 +1273,13 @@ extern "C" int fs2moe_grouped_wgrad(const void* a, const int32_t* a_row_map, con
   // one group: segments of its rows (each a slot of the grid) when there is scratch for their sums
   int segments = 1;
   if (counts == nullptr) {
-    segments = wgrad_segments(max_rows, M, N);
-    if (dtype == FS2MOE_F32) {
-      // (the f32 tiles are smaller: enough segments for two blocks to a CU)
-      const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64), enough = (511 + tiles) / tiles;
-      if (segments > enough) segments = (int)enough;
-    }
+    segments = dtype == FS2MOE_F32 ? wgrad_segments_f32(max_rows, M, N) : wgrad_segments(max_rows, M, N);
     if (workspace == nullptr || workspace_bytes < (int64_t)segments * M * N * 4) segments = 1;
   }
   const int seg_rows = segment_rows(max_rows, &segments);
   const int slots = counts != nullptr ? E : segments;
   float* partial = segments > 1 ? static_cast<float*>(workspace) : nullptr;
   FS2_REQUIRE((int64_t)slots * m_tiles * n_tiles <= 0x7fffffffll, "grouped_wgrad: too many tiles");
-  Groups g{counts, offsets, E, (int)max_rows};
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool mapped = a_row_map != nullptr;
   if (dtype == FS2MOE_BF16) {
@@ -1273,17 +1291,12 @@ extern "C" int fs2moe_grouped_wgrad(const void* a, const int32_t* a_row_map, con
     // (without rows nothing is read, and the map may be empty)
     if (int rc = launch_wgrad(jobs, max_rows > 0 ? a_row_map : nullptr, counts, offsets, E, st)) return rc;
   } else {
-    const int64_t big = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-    const bool small = f32t::small_tiles(big * slots, 128);
-    const int t = small ? 64 : 128, mt = (M + t - 1) / t, nt = (N + t - 1) / t;
-    FS2_REQUIRE((int64_t)slots * mt * nt <= 0x7fffffffll, "grouped_wgrad: too many tiles");
-    auto k = small ? (mapped ? grouped_wgrad_f32_kernel<1, true> : grouped_wgrad_f32_kernel<1, false>)
-                   : (mapped ? grouped_wgrad_f32_kernel<2, true> : grouped_wgrad_f32_kernel<2, false>);
-    hipLaunchKernelGGL(k, dim3((unsigned)(slots * mt * nt)), dim3(f32t::threads(1)), 0, st,
-                       static_cast<const float*>(a), a_row_map, static_cast<const float*>(b),
-                       static_cast<float*>(dw), M, N, g, mt, nt, seg_rows, partial);
+    F32WgradJobs jobs;
+    jobs.n = 1;
+    jobs.job[0] = {static_cast<const float*>(a), static_cast<const float*>(b), static_cast<float*>(dw), partial, M, N, 0, 0,
+                   segments, seg_rows, (int)max_rows, counts != nullptr, 0};
+    if (int rc = launch_wgrad_f32(jobs, a_row_map, counts, offsets, E, st)) return rc;
   }
-  if (int rc = check_launch("grouped_wgrad")) return rc;
   return segments > 1 ? launch_wgrad_reduce(partial, segments, (int64_t)M * N, dtype, dw, st) : FS2MOE_OK;
 }
 
@@ -1294,13 +1307,13 @@ constexpr int kPlanCUs = 256;
 
 int64_t fs2moe::wgrad_plan(WgradRequest* r, int n, int32_t E, int64_t planned, int64_t rows,
                            int32_t dtype) {
-  if (dtype == FS2MOE_F32) {  // (one launch each: every single group is cut as in fs2moe_grouped_wgrad)
-    int64_t most = 0;
+  if (dtype == FS2MOE_F32) {  // every single group is cut as in fs2moe_grouped_wgrad
+    int64_t bytes = 0;
     for (int i = 0; i < n; ++i) {
-      const int64_t b = r[i].grouped ? 0 : fs2moe_grouped_wgrad_workspace_bytes(0, r[i].M, r[i].N, rows);
-      most = b > most ? b : most;
+      r[i].segments = r[i].grouped ? 1 : wgrad_segments_f32(rows, r[i].M, r[i].N);
+      if (r[i].segments > 1) bytes += (int64_t)r[i].segments * r[i].M * r[i].N * 4;
     }
-    return most;
+    return bytes;
   }
   auto tiles = [](const WgradRequest& q) {
     return (int64_t)((q.M + wgk::TM - 1) / wgk::TM) * ((q.N + wgk::TN - 1) / wgk::TN);
@@ -1330,13 +1343,28 @@ int fs2moe::wgrad_all(const WgradRequest* r, int n, const int32_t* row_map, cons
                       const int32_t* offsets, int32_t E, int64_t grouped_rows, int64_t rows, int32_t dtype,
                       void* scratch, void* stream) {
   if (dtype == FS2MOE_F32) {
-    for (int i = 0; i < n; ++i) {
-      const bool g = r[i].grouped;
-      const int64_t ws = g ? 0 : fs2moe_grouped_wgrad_workspace_bytes(0, r[i].M, r[i].N, rows);
-      if (int rc = fs2moe_grouped_wgrad(r[i].a, nullptr, r[i].b, g ? counts : nullptr, g ? offsets : nullptr,
-                                        g ? E : 1, r[i].M, r[i].N, g ? grouped_rows : rows, dtype, r[i].dw,
-                                        ws > 0 ? scratch : nullptr, ws, stream))
-        return rc;
+    F32WgradJobs jobs;
+    FS2_REQUIRE(n <= F32WgradJobs::MAX, "wgrad: internal: %d gradients", n);
+    jobs.n = 0;
+    float* part = static_cast<float*>(scratch);
+    // (those of one group first: their segments are the longer walks)
+    for (const bool grouped : {false, true})
+      for (int i = 0; i < n; ++i) {
+        const WgradRequest& q = r[i];
+        if (q.grouped != grouped) continue;
+        int segments = grouped ? 1 : q.segments;
+        const int seg = segment_rows(rows, &segments);
+        jobs.job[jobs.n] = {static_cast<const float*>(q.a), static_cast<const float*>(q.b), static_cast<float*>(q.dw),
+                            segments > 1 ? part : nullptr, q.M, q.N, 0, 0, segments, seg, (int)rows, grouped, 0};
+        if (segments > 1) part += (int64_t)segments * q.M * q.N;
+        ++jobs.n;
+      }
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (int rc = launch_wgrad_f32(jobs, nullptr, counts, offsets, E, st)) return rc;
+    for (int i = 0; i < jobs.n; ++i) {
+      const F32WgradJob& j = jobs.job[i];
+      if (j.partial != nullptr)
+        if (int rc = launch_wgrad_reduce(j.partial, j.segments, (int64_t)j.M * j.N, dtype, j.C, st)) return rc;
     }
     return FS2MOE_OK;
   }

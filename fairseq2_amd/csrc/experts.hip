@@ -196,12 +196,8 @@ static int launch_f32(const void* a, const void* b0, const void* b1, const void*
                       void* g_keep, void* u_keep, int K, int N, const Groups& g, int64_t rows_bound,
                       const char* what, hipStream_t stream, int parts = 1) {
   const int groups = g.counts ? g.E : 0;
-  const int big_n = DUAL ? 64 : 128;
-  const int64_t planned = g.rows_to_plan(rows_bound);
-  const bool small = f32t::small_tiles((planned / 128 + groups + 1) * ((N + big_n - 1) / big_n),
-                                       groups ? planned / groups : planned) ||
-                     f32t::small_rounds(DUAL, planned, groups, N, 256);
-  const int bm = small ? 64 : 128, bn = small ? 64 : big_n;
+  const bool small = !f32t::large_tiles(DUAL, g.rows_to_plan(rows_bound), groups, N, 256);
+  const int bm = small ? 64 : 128, bn = small || DUAL ? 64 : 128;
   const int64_t m_tiles = rows_bound / bm + groups + 1;
   const int nt = (N + bn - 1) / bn;
   if (m_tiles * nt > 0x7ffffff0ll) {
@@ -386,8 +382,7 @@ int split_parts(int sources, int64_t planned, int E, int K, int N, int dtype) {
   // (the sums of buffers padded to 128 rows an expert have room in it)
   const int64_t part_bytes = (real + 127ll * E) * N * 4;
   if (dtype == FS2MOE_F32) {
-    const int64_t big = (planned / 128 + E + 1) * ((N + 127) / 128);  // (as in launch_f32)
-    if (!f32t::small_tiles(big, planned / groups) && !f32t::small_rounds(false, planned, E, N, CUS)) return 1;
+    if (f32t::large_tiles(false, planned, E, N, CUS)) return 1;
     const int64_t each = real / groups, chunks = sources * ((K + f32t::BK - 1) / f32t::BK);
     // (half of a last row block per expert)
     const int64_t tiles = (groups + (each > 32 ? (real - 32 * groups) / 64 : 0)) * ((N + 63) / 64);

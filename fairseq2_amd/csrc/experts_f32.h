@@ -4,8 +4,8 @@
 // What bounds them: the matrix pipe (64 clocks per instruction and SIMD, 157 TFLOP/s nominal, 154 in a
 // large product of the vendor's library), and, with few tiles, their number against 256 CUs.  A chunk is
 // 32 k; two chunks are on their way from memory in two register sets while a third is multiplied, LDS
-// holds two (one barrier per chunk), and a block is 4 waves (or 8) on a 64 x 64 or 4 on a 128 x 128 tile: the
-// small one, several blocks to a CU, where 128 x 128 tiles would not fill the chip twice (f32t::small_tiles).  What a
+// holds two (one barrier per chunk), and a block is 4 waves (or 8) on a 64 x 64 or 4 on a 128 x 128 tile, several of the
+// small ones' blocks to a CU (f32t::large_tiles).  What a
 // wave does besides multiplying is dealt out one instruction behind each product (Walk::run): as phases,
 // i.e. stores, barrier, loads, reads, products, the same tiles reach 132 TFLOP/s with every SIMD full
 // and 95 with one wave on each, whether one chunk or four are in flight; dealt out 149-154 and 107.
@@ -42,24 +42,28 @@ constexpr int BK = 32;
 // 1760, 66 -> 80 us).
 constexpr int threads(int groups) { return 256 * groups; }
 
-// Tiles of 64 x 64 while 128 x 128 ones would give a CU fewer than two blocks (big_tiles of them in the
-// launch), or where the groups have so few rows on average that half of a 128-row tile would be padding.
-inline bool small_tiles(int64_t big_tiles, int64_t rows_per_group) {
-  return big_tiles < 512 || rows_per_group <= 96;
-}
-// Or where their rounds of tiles (of the experts' rows, half of a last row block each) take less time than those of the
-// large ones, 64 rows x N as small tiles or 128 rows x N as large ones of 64 (two products) or 128 columns: 0.53 us per
-// 32 k and small tile, 0.44 per 64 x 64 of a large one.
-// 1356 tokens, top-1 of 16, D 1024, F 2048 by a popularity law 285 -> 228 us; the training step of 2439, top-2 of 16, D
-// 1024, F 1472 1604 -> 1538.
-inline bool small_rounds(bool dual, int64_t rows, int groups, int N, int cus) {
+// Products on tiles of 128 x 128 (two products at once: 128 rows x 64 channels of each) instead of 64 x 64: where their
+// rounds of tiles take less time.  In hundredths of a us per 32 k, on full rounds: a small tile 54, of two products 103, a
+// large one 195; so full rounds of large ones take a tenth less (two products a twentieth), and whatever part of a last
+// round is empty decides most cases.  us, small and large tiles, one product and two:
+//   8192 rows, N 2048, K 4096; N 4096, K 2048                 1108, 996; 2116, 1998    (4 and 16 rounds of large ones)
+//   8 experts of 2048, the same                               2500, 2379; 4829, 4404
+//   4 of 2048, N 1024, K 2048; N 2048, K 1024                  320, 393; 602, 610      (2.1 and 8.3 rounds)
+//   8 of 1024, N 2048, K 2048                                  597, 651; 1164, 1169
+//   16 of 500, D 768, F 1536, the layer                        521, 539
+//   128 of 256, D 1024, F 1024                                 1896, 1971
+// rows: the experts' rows, half of a last row block each.  One round of large tiles leaves a SIMD one wave, and few rounds of experts' tiles are as uneven as their loads:
+// 8 of 187 rows, D 1024, F 2048, the layer 227, 224 loaded evenly and 227, 256 by a popularity law.
+// (The weight gradients' tiles are small ones: 16 of 12 rows, 768 x 1024 44 us for the three of a step, 52 on large
+// ones; 128 of 256, 1024 x 1024 1755, 1777.)
+inline bool large_tiles(bool dual, int64_t rows, int groups, int N, int cus) {
   const int64_t real = groups > 0 && rows > 15ll * groups ? rows - 15ll * groups : rows;  // (less the blocks' padding)
   const int g = groups > 0 ? groups : 1;
   auto blocks = [&](int bm) { return g + (real > (int64_t)g * (bm / 2) ? (real - (int64_t)g * (bm / 2)) / bm : 0); };
   auto rounds = [&](int64_t tiles) { return (tiles + cus - 1) / cus; };
-  const int64_t small = rounds(blocks(64) * ((N + 63) / 64)) * 53;
-  const int64_t large = dual ? rounds(blocks(128) * ((N + 63) / 64)) * 88 : rounds(blocks(128) * ((N + 127) / 128)) * 176;
-  return small * 12 < large * 11;
+  const int64_t small = rounds(blocks(64) * ((N + 63) / 64)) * (dual ? 103 : 54);
+  const int64_t large = rounds(blocks(128) * (dual ? (N + 63) / 64 : (N + 127) / 128));
+  return large * 195 < small && large >= (groups == 0 ? 2 : 4);
 }
 
 // what a load through a row map reads past the end (not const: a global address)
@@ -441,103 +445,67 @@ __global__ __launch_bounds__(f32t::threads(GROUPS), 2 * GROUPS) void glu_gemm_f3
   }
 }
 
-// The n-th of the experts, those of more than four times the mean's rows first, then those of more than twice, then the
-// rest, by their numbers within each.  Wave-uniform, every wave for itself; without such experts it is n.
-// A block is one tile's walk over an expert's rows, and the hardware starts blocks in order: where the tiles of the
-// largest expert begin last, the launch waits for their walks alone.  Training step of 2439 tokens, top-2 of 16, D 1024,
-// F 1472 by a popularity law 1899 -> 1538 us; of 2153 evenly, top-1 of 8, D 640, F 2048 1220, 1221; 1000 tokens, top-2 of
-// 8, D 512, F 1408, whose tiles are small, 397 without and 404 with it.
-__device__ __forceinline__ int nth_expert_by_size(const int32_t* __restrict__ counts, int total, int E, int n) {
-  static_assert(FS2MOE_MAX_EXPERTS <= 512, "eight counts a lane");
-  const int lane = threadIdx.x & 63;
-  const float twice = 2.f * (float)total / (float)E;
-  float c[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int i = 64 * j + lane;
-    c[j] = 64 * j < E && i < E ? (float)counts[i] : -1.f;
-  }
-  unsigned long long large = 0;
-#pragma unroll
-  for (int j = 0; j < 8; ++j)
-    if (64 * j < E) large |= __ballot(c[j] > twice);
-  if (large == 0) return n;
-  int e = 0, seen = 0;
-#pragma unroll
-  for (int size = 2; size >= 0; --size) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (64 * j >= E) continue;  // uniform
-      const bool in = size == 2 ? c[j] > 2.f * twice : size == 1 ? c[j] > twice && !(c[j] > 2.f * twice)
-                                                                 : c[j] >= 0.f && !(c[j] > twice);
-      const unsigned long long m = __ballot(in);
-      const int before = seen + __popcll(m & ((1ull << lane) - 1ull));
-      const unsigned long long hit = __ballot(in && before == n);
-      if (hit != 0ull) e = 64 * j + (int)__builtin_ctzll(hit);
-      seen += __popcll(m);
-    }
-  }
-  return e;
-}
+// One weight gradient: dW_e = A_e^T B_e over the rows of an expert (slots: the experts), or over seg_rows rows each of
+// one group (slots: segments, whose sums go to `partial` where there are several).
+struct F32WgradJob {
+  const float *A, *B;
+  float *C, *partial;
+  int M, N, m_tiles, n_tiles, segments, seg_rows, rows;
+  int grouped, first;  // first: its first block
+};
+// Those of a step in one launch: each alone ends with a round of tiles that leaves CUs idle.  1000 tokens, top-2 of 8,
+// D 512, F 1408: three launches and the router's 113 us, one 89.
+struct F32WgradJobs {
+  static constexpr int MAX = 8;
+  F32WgradJob job[MAX];
+  int n;
+};
 
-// dW_e = A_e^T B_e over the rows of an expert (slots: the experts), or over seg_rows rows each of one
-// group (slots: segments, whose sums go to `partial` where there are several).
 // MAPPED: A's rows are read through a_map.
-template <int F, bool MAPPED>
+template <bool MAPPED>
 __global__ __launch_bounds__(f32t::threads(1), 2) void grouped_wgrad_f32_kernel(
-    const float* __restrict__ A, const int32_t* __restrict__ a_map, const float* __restrict__ B,
-    float* __restrict__ C, int M, int N, Groups g, int m_tiles, int n_tiles, int seg_rows,
-    float* __restrict__ partial) {
-  using W = f32t::Walk<1, F, F, true, true, MAPPED, 1, false>;
+    const F32WgradJobs jobs, const int32_t* __restrict__ a_map, Groups g) {
+  using W = f32t::Walk<1, 1, 1, true, true, MAPPED, 1, false>;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[W::SMEM_BYTES];
-  const int per = m_tiles * n_tiles;
-  int slot = blockIdx.x / per;
-  const int rem = blockIdx.x - slot * per;
-  const int mt = rem / n_tiles, nt = rem - mt * n_tiles;
+  int at = 0;
+  for (int i = 1; i < jobs.n; ++i)
+    if ((int)blockIdx.x >= jobs.job[i].first) at = i;
+  const F32WgradJob& job = jobs.job[at];
+  const float *A = job.A, *B = job.B;
+  const int M = job.M, N = job.N, per = job.m_tiles * job.n_tiles;
+  int slot = ((int)blockIdx.x - job.first) / per;
+  const int rem = (int)blockIdx.x - job.first - slot * per;
+  const int mt = rem / job.n_tiles, nt = rem - mt * job.n_tiles;
   int off, cnt;
-  if (g.counts == nullptr) {
-    off = slot * seg_rows;
-    cnt = g.dense_rows - off < seg_rows ? g.dense_rows - off : seg_rows;
+  if (!job.grouped) {
+    off = slot * job.seg_rows;
+    cnt = job.rows - off < job.seg_rows ? job.rows - off : job.seg_rows;
   } else {
-    // (small tiles have short walks, several to a CU side by side: looking costs them 2 % of the step below)
-    if constexpr (F == 2) {
-      const int total = g.offsets[g.E];
-      slot = __builtin_amdgcn_readfirstlane(nth_expert_by_size(g.counts, total, g.E, slot));
-    }
     off = __builtin_amdgcn_readfirstlane(g.offsets[slot]);
     cnt = __builtin_amdgcn_readfirstlane(g.counts[slot]);
   }
   const int m0 = mt * W::BM, n0 = nt * W::BN;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = W::wave_m(wave), wn = W::wave_n(wave), lr = lane & 31, lk = lane >> 5;
-  f32x16 acc[1][F][F];
+  f32x16 acc[1][1][1];
 #pragma unroll
-  for (int fn = 0; fn < F; ++fn)
-#pragma unroll
-    for (int fm = 0; fm < F; ++fm)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[0][fn][fm][i] = 0.f;
+  for (int i = 0; i < 16; ++i) acc[0][0][0][i] = 0.f;
   typename W::Source s;
   s.a = (MAPPED ? A : A + (size_t)off * M) + m0;
   s.b[0] = B + (size_t)off * N + n0;
-  const int m_wave = m0 + wm * 32 * F;
+  const int m_wave = m0 + wm * 32;
   if (cnt > 0) W::run(acc, smem, s, s, 1, M, N, cnt, M - m0, N - n0, m_wave < M,
                      MAPPED ? a_map + off : nullptr);
-  float* to = partial != nullptr ? partial : C;
+  float* to = job.partial != nullptr ? job.partial : job.C;
   to += (size_t)slot * M * N;
+  const int m = m_wave + lr;
+  if (m >= M) return;
 #pragma unroll
-  for (int fm = 0; fm < F; ++fm) {
-    const int m = m_wave + fm * 32 + lr;
-    if (m >= M) continue;
-#pragma unroll
-    for (int fn = 0; fn < F; ++fn)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = n0 + (wn * F + fn) * 32 + 8 * q + 4 * lk;
-        if (n >= N) continue;
-        const f32x16& a = acc[0][fn][fm];
-        *reinterpret_cast<f32x4*>(to + (size_t)m * N + n) = f32x4{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
-      }
+  for (int q = 0; q < 4; ++q) {
+    const int n = n0 + wn * 32 + 8 * q + 4 * lk;
+    if (n >= N) continue;
+    const f32x16& a = acc[0][0][0];
+    *reinterpret_cast<f32x4*>(to + (size_t)m * N + n) = f32x4{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
   }
 }
 

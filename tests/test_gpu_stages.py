@@ -794,6 +794,26 @@ def test_weights_past_the_caches_give_the_same_bits(gpu_device, d, f):
         xq, xs, c, o, *(q[:e] for q in packed), tuple(s[:e] for s in scales), e)[:2])
 
 
+# f32 products of many rounds take large tiles; rows and channels past them, one product, its transpose and two at once:
+# the bits of launches of a few rows, which take small ones.
+def test_f32_products_on_large_tiles(gpu_device):
+    rows, k, n = 8190, 40, 2040
+    _say("f32 large tiles", rows, k, n)
+    g = torch.Generator(gpu_device).manual_seed(1)
+    x, w, wu = (torch.randn(*s, generator=g, device=gpu_device) for s in ((rows, k), (k, n), (k, n)))
+    wd = torch.zeros(n, k, device=gpu_device)
+    group = lambda m: (torch.tensor([m], dtype=torch.int32, device=gpu_device),
+                       torch.tensor([0, m], dtype=torch.int32, device=gpu_device))
+    runs = (lambda a: _abi.grouped_gemm(a, w, _abi.W_IN_OUT),
+            lambda a: _abi.grouped_gemm(a, w.t().contiguous(), _abi.W_OUT_IN),
+            lambda a: _abi.grouped_swiglu(a, *group(a.shape[0]), w, wu, wd, 1)[1])
+    for run in runs:
+        whole = run(x)
+        for lo in (0, 4096, 8126):
+            assert torch.equal(run(x[lo : lo + 64].contiguous()), whole[lo : lo + 64])
+    assert_output_close(runs[0](x[:300]), (x[:300].double() @ w.double()).cpu(), "fp32")
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
 @pytest.mark.parametrize(
     "t,d,f",
