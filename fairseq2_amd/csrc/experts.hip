@@ -307,7 +307,7 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
   // (tiles of 64 x 64 are counted in 31 bits too)
   const bool counted = (rows_bound / 64 + groups + 1) * ((N + 63) / 64) <= 0x7fffffffll;
   constexpr bool SINGLE = !DUAL && CAN_TAIL;
-  switch (counted ? half_tiles::pick(DUAL, SINGLE, g.rows_to_plan(rows_bound), groups, K, N, num_blocks) : 0) {
+  switch (counted ? half_tiles::pick(DUAL, CAN_TAIL, g.rows_to_plan(rows_bound), groups, K, N, num_blocks) : 0) {
     case 1:
       if constexpr (SINGLE)
         return launch_half<64, 64, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,

@@ -73,10 +73,16 @@ constexpr uint32_t NOWHERE = 0xfffffff0u;      // an offset past any buffer's en
 //   16 experts of 375, K 1368, N 1024    33 against 62, 50, 37     (none fits one round)
 //   32 of 35, D 1472, F 1216             90 against 79 (2), 80 (3) (the throughput kernel: 1.25 rounds)
 //   64 of 23, D 2944, F 1840             377 against 394, 400      (memory)
-// All are even loads, which the rounds' model further down assumes.  Where a few rows reach a part of the experts it is
-// far off: 48 tokens, top-8 of 128 by a popularity law, K 768, N 2048 36 us with the throughput kernel, 18 by the model.
-// single: the launch is one product of bf16 matrices.
-inline int pick(bool dual, bool single, int64_t rows, int groups, int K, int N, int cus) {
+// All are even loads.  Where a few rows reach a part of the experts, or most of the rows one, the tiles that count are
+// few as well and these win by more: the margins below are what even loads lose and skewed ones gain, us of the layer
+// with the margin of e4m3 weights for all, with bf16's:
+//   20 and 200 tokens, top-4 of 60 by a popularity law, D 1024, F 1408       60.3, 51.1; 73.0, 57.5
+//   20 and 100, top-2 of 8, D 2048, F 12800                                  308, 243; 324, 260
+//   48 and 100, top-8 of 128, D 2048, F 768                                  96.2, 90.4; 130, 125.5
+//   a training step of 260, top-1 of 8, D 640, F 6400                        271, 235
+//   200 evenly, top-6 of 64, D 3072, F 1024; a training step of 260, skewed  217.8, 221.3; 706, 718
+// bf16: matrices and rows of bf16, not codes (which take longer than the model's rounds to convert).
+inline int pick(bool dual, bool bf16, int64_t rows, int groups, int K, int N, int cus) {
   // Of the experts' rows only the device knows how they are spread: the planned ones (Groups), less what blocks of 16
   // pad them by, equally loaded.
   const int64_t real = rows > 15ll * groups ? rows - 15ll * groups : rows;
@@ -88,20 +94,22 @@ inline int pick(bool dual, bool single, int64_t rows, int groups, int K, int N, 
     const int64_t blocks = groups + (each > bm / 2 ? (real - (int64_t)groups * (bm / 2)) / bm : 0);
     return (blocks < real ? blocks : real) * nt;
   };
-  const int64_t room = cus - cus / 16;  // (experts are not equally loaded: a few tiles more)
-  if (single && tiles(64, 64) <= room) return 1;
+  // (experts of many rows are not equally loaded: a few tiles more; of those of one row block some have none)
+  const int64_t room = bf16 && each <= 32 ? cus : cus - cus / 16;
+  if (bf16 && !dual && tiles(64, 64) <= room) return 1;
   if (tiles(64, dual ? 64 : 128) <= room) return 2;
   if (tiles(128, dual ? 64 : 128) <= room) return 3;
   // Several rounds of tiles of a few rows: rounds of the throughput kernel (1 us per 64 k and 6 per tile, us) against
   // rounds of these (0.4 and 4), neither faster than memory delivers half of the experts' weights (5.2 TB/s; with few
-  // tokens or a skewed load not all experts have rows), and a fifth for what that leaves out.
+  // tokens or a skewed load not all experts have rows), and a margin for what that leaves out.
   if (groups > 0 && each <= 64) {
     const int64_t units = (K + 63) / 64, active = groups < real ? groups : real;
     const int64_t memory = active * K * N * (dual ? 2 : 1) / 5200;  // ns
     auto rounds = [&](int64_t n) { return (n + cus - 1) / cus; };
     const int64_t whole = rounds(tiles(256, dual ? 128 : 256)) * (units * 1000 + 6000);
     const int64_t small = rounds(tiles(64, dual ? 64 : 128)) * (units * 400 + 4000);
-    if ((small > memory ? small : memory) * 6 < (whole > memory ? whole : memory) * 5) return 2;
+    const int64_t percent = !bf16 ? 83 : dual ? 70 : 100 - each / 4;
+    if ((small > memory ? small : memory) * 100 < (whole > memory ? whole : memory) * percent) return 2;
   }
   return 0;
 }

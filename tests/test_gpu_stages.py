@@ -794,6 +794,36 @@ def test_weights_past_the_caches_give_the_same_bits(gpu_device, d, f):
         xq, xs, c, o, *(q[:e] for q in packed), tuple(s[:e] for s in scales), e)[:2])
 
 
+# Which tiles products of bf16 take follows from the size of the buffers (one round of small ones, several rounds of
+# few rows, the throughput kernel): the same bits, with few experts' tiles about one a compute unit and several a unit,
+# rows on both sides of a tile's 64 in one expert, K and N off the units.
+@pytest.mark.parametrize("e,d,f", [(8, 1024, 2048), (32, 1000, 1416)])
+def test_products_of_few_rows_are_the_same_on_every_tile_size(gpu_device, e, d, f):
+    _say("tiles of few rows", e, d, f)
+    dev, bf = gpu_device, torch.bfloat16
+    g = torch.Generator(dev).manual_seed(e)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(bf)
+    rows = [130, 1, 0, 64, 65, 17, 0, 33] + [0, 2] * (e // 2 - 4)
+    counts = torch.tensor(rows, dtype=torch.int32, device=dev)
+    offsets = torch.zeros(e + 1, dtype=torch.int32, device=dev)
+    offsets[1:] = torch.cumsum((counts + 15) // 16 * 16, 0)
+    lo = offsets.tolist()
+    x, wg, wu, wd = rnd(400 * e, d), rnd(e * d, f) * 0.05, rnd(e * d, f) * 0.05, rnd(e * f, d) * 0.05
+    got = []
+    for total in (lo[-1], 24 * e + lo[-1], 48 * e + lo[-1], 80 * e + lo[-1], 400 * e):
+        out = list(_abi.grouped_swiglu(x[:total], counts, offsets, wg, wu, wd, e))
+        out.append(_abi.grouped_gemm(x[:total], wd, _abi.W_OUT_IN, counts, offsets, e))
+        got.append([torch.cat([o[lo[i] : lo[i] + n] for i, n in enumerate(rows)]) for o in out])
+    assert all(torch.equal(a, b) for o in got[:-1] for a, b in zip(o, got[-1]))
+    for i, n in enumerate(rows):
+        if n == 0:
+            continue
+        ref = O.glu_expert(*(t.double() for t in (x[lo[i] : lo[i] + n], wg[i * d : (i + 1) * d], wu[i * d : (i + 1) * d],
+                                                  wd[i * f : (i + 1) * f])))
+        at = sum(rows[:i])
+        assert_output_close(got[0][0][at : at + n], ref.cpu(), "bf16", f"expert {i}")
+
+
 # f32 products of many rounds take large tiles; rows and channels past them, one product, its transpose and two at once:
 # the bits of launches of a few rows, which take small ones.
 def test_f32_products_on_large_tiles(gpu_device):
