@@ -180,17 +180,15 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// 8 e4m3 codes (two dwords) -> 8 bf16 values.
+// 8 e4m3 codes (two dwords) -> 8 bf16 values, all exact.  One instruction for two (two to f32 and one to join their upper
+// halves before: 1000 tokens, top-2 of 8, D 2048, F 12800 463, 434 us; 150, top-8 of 32, D 4096, F 1152 172, 149).
 __device__ __forceinline__ bf16x8 fp8x8_to_bf16x8(uint32_t lo, uint32_t hi) {
-  typedef __attribute__((ext_vector_type(2))) float f32x2;
   u32x4 out;
-  const uint32_t w[2] = {lo, hi};
+  const int w[2] = {(int)lo, (int)hi};
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[i], false);  // bytes 0, 1
-    const f32x2 b = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[i], true);   // bytes 2, 3
-    out[2 * i] = (__float_as_uint(a[0]) >> 16) | (__float_as_uint(a[1]) & 0xffff0000u);
-    out[2 * i + 1] = (__float_as_uint(b[0]) >> 16) | (__float_as_uint(b[1]) & 0xffff0000u);
+    out[2 * i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[i], 1.f, false));
+    out[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[i], 1.f, true));
   }
   return __builtin_bit_cast(bf16x8, out);
 }
