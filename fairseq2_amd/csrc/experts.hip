@@ -217,9 +217,15 @@ static int launch_f32(const void* a, const void* b0, const void* b1, const void*
   return check_launch(what);
 }
 
-// e4m3 weights go to the throughput kernel from this many rows per expert on (mean over all experts)
+// e4m3 weights go to the throughput kernels from this many rows per expert on (mean over all experts, of the rows
+// planned, 15 of which may be padding).  us of the layer, streamed against there:
+//   20 rows an expert on average   (D 1024, F 1408, top-4 of 60) 83, 102; (4096, 6400, 2 of 16) 261, 286
+//   25                             (4096, 1152, 8 of 32) 129, 142; (2048, 768, 8 of 128) 172, 184; (4096, 6400) 307,
+//                                  294
+//   27, 28                         (1024, 1408) 95, 103; (3072, 1024, 6 of 64) 179, 174
+//   37                             (3072, 1024) 246, 176; (2048, 12800, 2 of 8) 243, 204
 #ifndef FS2MOE_FP8_GEMM_MIN_ROWS
-#define FS2MOE_FP8_GEMM_MIN_ROWS 32
+#define FS2MOE_FP8_GEMM_MIN_ROWS 42
 #endif
 constexpr int64_t kFp8GemmMinRowsPerExpert = FS2MOE_FP8_GEMM_MIN_ROWS;
 
@@ -829,60 +835,59 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
                                                s_up, s_down, D, F, h, ye, st);
     }
     FS2_REQUIRE(E <= 256, "grouped_swiglu: the e4m3 streaming kernels take up to 256 experts (E=%d)", E);
-    // Persistent blocks, three or four per CU (what the kernels' registers allow), walking work
+    // Persistent blocks, three to five per CU (what the kernels' registers allow), walking work
     // items.
     // A long K is split over the 4 waves of a block (the chain of dependent loads per wave sets the
     // time of an item), a short one over 2 with two sets of channel groups per block.  A wave takes
     // 2 (gate/up) or 4 (down) groups of 16 channels when K is long, half that when it is short;
-    // N / 16 is a multiple of 4, so the channel blocks tile N exactly.
+    // N / 16 is a multiple of 4, so the channel blocks tile N exactly.  Figures with the kernel.
+    // Chunks of 32 rows from 8 rows an expert on (6 rows: 1-4 % slower evenly, 3-8 % faster skewed; 9 and more:
+    // 0-22 % faster); one group for gate/up up to 3 (1.5 rows: 0-15 % faster; 4 rows, skewed: 8 % slower).
     const int cus = cu_count_by_xcd();
     if (cus == 0) {
       set_error("experts: cannot query the compute-unit count");
       return FS2MOE_ERR_LAUNCH;
     }
-    const unsigned cu_blocks = (unsigned)cus;
-    {
-      // work items (16-row chunks x channel blocks of at least 32 channels) are counted in 31 bits
-      const int64_t chunks = max_rows / 16 + E;
-      const int64_t most_blocks = (D > F ? D : F) / 32;
-      if (chunks * most_blocks > 0x7fffffffll) {
-        set_error("experts: too many work items");
-        return FS2MOE_ERR_UNSUPPORTED;
-      }
+    // work items (chunks of at least 16 rows x channel blocks of at least 32 channels) are counted in 31 bits
+    const int64_t chunks = max_rows / 16 + E;
+    if (chunks * ((D > F ? D : F) / 32) > 0x7fffffffll) {
+      set_error("experts: too many work items");
+      return FS2MOE_ERR_UNSUPPORTED;
     }
+    const bool fine_items = chunks * (F / 16) <= 0x7fffffffll;
     const Groups grp{counts, offsets, E, 0, (int)planned};
-    // (chunks of 16 rows share an expert's weights in L2: 126 rows of 8 experts, D 1344, F 14080 140 us with them there,
-    // 151 past it; 14 rows, D 4864, F 11136 260, 236; 64 tokens, top-8 of 128, D 2048, F 768 73.5, 70.4)
+    // (past the caches: chunks share an expert's weights in L2: 126 rows of 8 experts, D 1344, F 14080 140 us with them
+    // there, 151 past it; 14 rows, D 4864, F 11136 260, 236; 64 tokens, top-8 of 128, D 2048, F 768 73.5, 70.4)
     const int64_t pairs = pairs_of(grp, max_rows);
-    const bool past = pairs <= 8ll * E && weights_past_cache(E, pairs, D, F, 1);
-    auto launch = [&](auto dual_tag, auto nt_tag, const void* a, const int32_t* map, int lda, const void* w0,
-                      const void* w1, const float* s0, const float* s1, void* c, int ldc, int kdim,
+    const bool few = pairs <= 3ll * E && fine_items;
+    auto launch = [&](auto dual_tag, auto fr_tag, auto nt_tag, const void* a, const int32_t* map, int lda,
+                      const void* w0, const void* w1, const float* s0, const float* s1, void* c, int ldc, int kdim,
                       int n) {
       constexpr bool DUAL = decltype(dual_tag)::value, NT = decltype(nt_tag)::value;
-      const uint16_t* ap = static_cast<const uint16_t*>(a);
-      const uint8_t* w0p = static_cast<const uint8_t*>(w0);
-      const uint8_t* w1p = static_cast<const uint8_t*>(w1);
-      uint16_t* cp = static_cast<uint16_t*>(c);
-      const unsigned grid = (DUAL ? 4u : 3u) * cu_blocks;  // the kernels' launch bounds
-      if (kdim >= 512) {
-        constexpr int CGW = DUAL ? 2 : 4;
-        hipLaunchKernelGGL((glu_gemm_fp8w_kernel<DUAL, 4, CGW, NT>), dim3(grid), dim3(256), 0, st, ap,
-                           map, lda, w0p, w1p, s0, s1, cp, ldc, kdim, n, counts, offsets, E,
-                           n / 16 / CGW);
-      } else {
-        constexpr int CGW = DUAL ? 1 : 2;
-        hipLaunchKernelGGL((glu_gemm_fp8w_kernel<DUAL, 2, CGW, NT>), dim3(grid), dim3(256), 0, st, ap,
-                           map, lda, w0p, w1p, s0, s1, cp, ldc, kdim, n, counts, offsets, E,
-                           n / 16 / (2 * CGW));
-      }
+      constexpr int FR = decltype(fr_tag)::value;
+      auto go = [&](auto ks_tag, auto groups_tag) {
+        constexpr int KS = decltype(ks_tag)::value, CGW = decltype(groups_tag)::value;
+        const unsigned grid = (unsigned)(fp8w::blocks(DUAL, CGW, FR) * cus);
+        hipLaunchKernelGGL((glu_gemm_fp8w_kernel<DUAL, KS, CGW, FR, NT>), dim3(grid), dim3(256), 0, st,
+                           static_cast<const uint16_t*>(a), map, lda, static_cast<const uint8_t*>(w0),
+                           static_cast<const uint8_t*>(w1), s0, s1, static_cast<uint16_t*>(c), ldc, kdim, n, counts,
+                           offsets, E, n / (16 * CGW * (4 / KS)));
+      };
+      if (kdim < 512)
+        return go(std::integral_constant<int, 2>{}, std::integral_constant<int, DUAL ? 1 : 2>{});
+      if constexpr (DUAL && FR == 1)
+        if (few) return go(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
+      go(std::integral_constant<int, 4>{}, std::integral_constant<int, DUAL ? 2 : 4>{});
     };
-    auto pair = [&](auto nt) -> int {
-      launch(std::true_type{}, nt, xe, row_map, D, w_gate, w_up, s_gate, s_up, h, F, D, F);
+    auto pair = [&](auto fr, auto nt) -> int {
+      launch(std::true_type{}, fr, nt, xe, row_map, D, w_gate, w_up, s_gate, s_up, h, F, D, F);
       if (int rc = check_launch("glu_gemm_fp8w<gate,up>")) return rc;
-      launch(std::false_type{}, nt, h, nullptr, F, w_down, nullptr, s_down, nullptr, ye, D, F, D);
+      launch(std::false_type{}, fr, nt, h, nullptr, F, w_down, nullptr, s_down, nullptr, ye, D, F, D);
       return check_launch("glu_gemm_fp8w<down>");
     };
-    return past ? pair(std::true_type{}) : pair(std::false_type{});
+    if (pairs > 8ll * E) return pair(std::integral_constant<int, 2>{}, std::false_type{});
+    if (weights_past_cache(E, pairs, D, F, 1)) return pair(std::integral_constant<int, 1>{}, std::true_type{});
+    return pair(std::integral_constant<int, 1>{}, std::false_type{});
   }
   if (w_dtype != act_dtype) {
     set_error("grouped_swiglu: weight dtype %d with activation dtype %d has no kernel", w_dtype,

@@ -138,9 +138,9 @@ class GroupedExpertNetwork(ExpertNetwork):
     def has_fused_gate(self) -> bool:
         return isinstance(_part(self, "activation"), nn.SiLU)
 
-    # e4m3 weights go to the GEMM kernels from this many rows per expert on (mean over all experts,
-    # the library's own rule for its bf16-pipe path); below that the experts are a weight stream,
-    # which activations of one byte would not make faster.
+    # Rows go to the fp8 matrix pipe from this many per expert on (mean over all experts; the library
+    # takes its bf16-pipe GEMMs for e4m3 weights from about 27 on); below that the experts are a weight
+    # stream, which activations of one byte would not make faster.
     _W8A8_MIN_ROWS_PER_EXPERT = 32
 
     def runs_w8a8(self, act_dtype: torch.dtype, rows: int) -> bool:

@@ -753,7 +753,7 @@ def test_weights_past_the_caches_give_the_same_bits(gpu_device, d, f):
     assert 3 * d * f * 2 * few < 2**27 < 3 * d * f * 2 * 100
     g = torch.Generator(dev).manual_seed(d + f)
     rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(bf)
-    x, mid = rnd(4608, d), rnd(4608, f)
+    x, mid = rnd(5632, d), rnd(5632, f)
     wg, wu, wd = rnd(many * d, f) * 0.05, rnd(many * d, f) * 0.05, rnd(many * f, d) * 0.05
 
     def both(rows, total, run):
@@ -787,7 +787,7 @@ def test_weights_past_the_caches_give_the_same_bits(gpu_device, d, f):
     scales = [torch.rand(many, n, generator=g, device=dev) + 0.5 for n in (f, f, d)]
     both([16, 17, 1, 0, 33, 2, 9, 16], 160, lambda c, o, e, t: _abi.grouped_swiglu(
         x[:t], c, o, *(q[:e] for q in packed), e, scales=tuple(s[:e] for s in scales)))
-    both(rows, 4608, lambda c, o, e, t: _abi.grouped_swiglu(
+    both(rows, 5632, lambda c, o, e, t: _abi.grouped_swiglu(
         x[:t], c, o, *(q[:e] for q in packed), e, scales=tuple(s[:e] for s in scales)))
     xq, xs = _abi.mx_quantize(x[:total].contiguous())
     both(rows, total, lambda c, o, e, t: _abi.grouped_swiglu_w8a8(
@@ -820,6 +820,37 @@ def test_products_of_few_rows_are_the_same_on_every_tile_size(gpu_device, e, d, 
             continue
         ref = O.glu_expert(*(t.double() for t in (x[lo[i] : lo[i] + n], wg[i * d : (i + 1) * d], wu[i * d : (i + 1) * d],
                                                   wd[i * f : (i + 1) * f])))
+        at = sum(rows[:i])
+        assert_output_close(got[0][0][at : at + n], ref.cpu(), "bf16", f"expert {i}")
+
+
+# How many rows and channels a piece of the e4m3 stream's work has follows from the size of the buffers: the same bits,
+# for rows on both sides of 16 and 32, K within a step, past one and split over two waves, against the oracle.
+@pytest.mark.parametrize("d,f", [(512, 1024), (448, 704), (1088, 64)])
+def test_e4m3_streams_of_every_chunk_are_the_same(gpu_device, d, f):
+    _say("e4m3 stream", d, f)
+    e, dev, bf = 64, gpu_device, torch.bfloat16
+    g = torch.Generator(dev).manual_seed(d)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(bf)
+    rows = [33, 32, 17, 16, 1, 0, 48, 31] + [0] * (e - 8)
+    counts = torch.tensor(rows, dtype=torch.int32, device=dev)
+    offsets = torch.zeros(e + 1, dtype=torch.int32, device=dev)
+    offsets[1:] = torch.cumsum((counts + 15) // 16 * 16, 0)
+    lo = offsets.tolist()
+    x = rnd(24 * e, d)
+    codes = [(rnd(e * i, o) * 0.05).to(torch.float8_e4m3fn) for i, o in ((d, f), (d, f), (f, d))]
+    packed = [_abi.pack_fp8_weights(c, e) for c in codes]
+    scales = [torch.rand(e, n, generator=g, device=dev) + 0.5 for n in (f, f, d)]
+    got = []
+    for total in (18 * e, 20 * e, 24 * e):
+        out = _abi.grouped_swiglu(x[:total], counts, offsets, *packed, e, scales=tuple(scales))
+        got.append([torch.cat([o[lo[i] : lo[i] + n] for i, n in enumerate(rows)]) for o in out])
+    assert all(torch.equal(a, b) for o in got[1:] for a, b in zip(o, got[0]))
+    for i, n in enumerate(rows):
+        if n == 0:
+            continue
+        w = [c[i * k : (i + 1) * k].double() * s[i].double() for c, s, k in zip(codes, scales, (d, d, f))]
+        ref = O.glu_expert(x[lo[i] : lo[i] + n].double(), *w)
         at = sum(rows[:i])
         assert_output_close(got[0][0][at : at + n], ref.cpu(), "bf16", f"expert {i}")
 
