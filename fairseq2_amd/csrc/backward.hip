@@ -83,12 +83,13 @@ struct WgradJobs {
 };
 
 // MAPPED: operands of some gradients are read through the row map (rows of the layer's input, or of its
-// output gradient, that no one has copied into expert order).  The map's entries are scalar loads, two rows
-// per wave and load, asked for a chunk ahead, right behind a barrier: vector loads would be waited for with every
-// other load of the wave, a round trip per chunk, and scalar ones in front of a barrier are waited for there, with
-// the LDS traffic, by the whole block.  128 experts of about 256 rows, 2048 x 768, one gradient: 171 us with the
-// entries asked for in front of the barrier, 163 now (150 on copied rows, whose copies cost more than that); training
-// steps of 4444 tokens, top-8 of 128, D 1280, F 704 1212 -> 1175 us, of 3771, top-8 of 64, D 1152, F 696 901 -> 879.
+// output gradient, that no one has copied into expert order).  The map's entries are asked for two chunks ahead, by one
+// load per wave right behind those of the chunk before the last, with which they arrive: nothing waits for them alone.
+// (As scalar loads a chunk ahead every barrier waited for them with the LDS traffic.)  That, and a way out of a tile
+// without branches and waits around its stores, us of the gradients of a training step: 4096 tokens, top-8 of 128
+// skewed, 2048 x 768 648 -> 617; top-6 of 64, 2048 x 1024 465 -> 449; 2000, top-4 of 60 skewed, 1024 x 1408 181 -> 173;
+// 300 of the first 246 -> 236; 4096 evenly, top-8 of 128 554 -> 553, which memory bounds (2.3 GB; 478 without the
+// products, 420 without memory).
 // The map holds at least one entry, and one for every row of a gradient in the same launch that does not use it.
 template <bool MAPPED>
 __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
@@ -405,15 +406,20 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     const uint16_t* ld_a = nullptr;
     const uint16_t* ld_b = nullptr;
     int ld_left = 0, ld_lda = 0, ld_ldb = 0;
-    // MAPPED: the chunk's first row in expert order, which operands go through the map, and the rows of the
-    // wave's eight pieces (two to a load instruction) in expert order and behind the map
+    // MAPPED: the chunk's first row in expert order, which operands go through the map, a lane's place in row 0 of the
+    // operands, and their rows' distance
     typedef u32x4 __attribute__((address_space(1))) GlobalVec;
     uint64_t zero = (uint64_t)kZero16;
     asm volatile("" : "+s"(zero));  // (read once)
-    const int kr0 = (wave - CONSUMERS) * 2;
-    int ld_row = 0, ld_map_a = 0, ld_map_b = 0, place[PER_THREAD][2], entry[PER_THREAD][2];
-    uint64_t row_a = zero, row_b = zero;    // a lane's place in row 0 of the operands, and their rows' distance
+    int ld_row = 0, ld_map_a = 0, ld_map_b = 0;
+    uint64_t row_a = zero, row_b = zero;
     uint32_t pitch_a = 0, pitch_b = 0;
+    // and the same of the next chunk to load into each register set, with its rows' entries: lane l holds row kr + 8 (l & 3)'s
+    struct Ahead {
+      uint64_t row_a, row_b;
+      uint32_t pitch_a, pitch_b;
+      int row, left, map_a, map_b, entry;
+    } next_up[2];
     Deal ld_deal = deal;
     uint32_t oa[PER_THREAD], ob[PER_THREAD];
     int loaded = 0;  // chunks so far (those past the stream's end do not count)
@@ -454,47 +460,43 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
       const uint64_t v = (uint64_t)q;
       return (uint16_t*)((uint64_t)(uint32_t)uniform((int)(v >> 32)) << 32 | (uint32_t)uniform((int)v));
     };
-    auto look_up = [&]() {
-      if (uniform(ld_left) <= 0) next_tile();
+    // MAPPED: the stream's next chunk becomes the register set's, and its entries are asked for.
+    auto look_up = [&](auto set_c) {
       if constexpr (MAPPED) {
-#pragma unroll
-        for (int i = 0; i < PER_THREAD; ++i)
-#pragma unroll
-          for (int r = 0; r < 2; ++r) {
-            const int k = kr0 + 8 * i + r, last = ld_left - 1;
-            place[i][r] = last >= 0 ? ld_row + (k < last ? k : last) : 0;
-            entry[i][r] = row_map[place[i][r]];
-          }
+        if (uniform(ld_left) <= 0) next_tile();
+        const int k = kr + 8 * (lane & 3), last = ld_left - 1;
+        const int entry = row_map[last >= 0 ? ld_row + (k < last ? k : last) : 0];
+        next_up[decltype(set_c)::value] = {row_a, row_b, pitch_a, pitch_b, ld_row, ld_left, ld_map_a, ld_map_b, entry};
+        loaded += (int)((uint32_t)-ld_left >> 31);  // (as below)
+        ld_row += RK;
+        ld_left -= RK;
       }
     };
-    // MAPPED: where the chunk's pieces lie, and the entries of the chunk after it asked for.  In front of the stores,
-    // behind the barrier that has waited for the entries with the LDS traffic before it (one counter for both, in
-    // no order): asked for in front of a barrier, they were a round trip that every wave of the block waited for.
+    // MAPPED: where the chunk's pieces lie.
     // (a lane whose column lies past the operand's reads zeros whatever the row)
     uint64_t at_a[PER_THREAD], at_b[PER_THREAD];
-    auto place_chunk = [&]() {
+    auto place_chunk = [&](auto set_c) {
       if constexpr (MAPPED) {
+        const Ahead& up = next_up[decltype(set_c)::value];
+        const int left = uniform(up.left), last = left - 1;
 #pragma unroll
         for (int i = 0; i < PER_THREAD; ++i) {
-          const uint32_t a0 = ld_map_a ? entry[i][0] : place[i][0], a1 = ld_map_a ? entry[i][1] : place[i][1];
-          const uint32_t b0 = ld_map_b ? entry[i][0] : place[i][0], b1 = ld_map_b ? entry[i][1] : place[i][1];
-          at_a[i] = row_a + (uint64_t)(lane < 32 ? a0 : a1) * pitch_a;
-          at_b[i] = row_b + (uint64_t)(lane < 32 ? b0 : b1) * pitch_b;
+          const uint32_t e0 = __builtin_amdgcn_readlane(up.entry, i), e1 = __builtin_amdgcn_readlane(up.entry, 32 + i);
+          const int k = kr + 8 * i;
+          const uint32_t mapped = lane < 32 ? e0 : e1, place = last >= 0 ? up.row + (k < last ? k : last) : 0;
+          at_a[i] = up.row_a + (uint64_t)(up.map_a ? mapped : place) * up.pitch_a;
+          at_b[i] = up.row_b + (uint64_t)(up.map_b ? mapped : place) * up.pitch_b;
         }
-        if (ld_left < RK) {
+        if (left < RK) {
 #pragma unroll
           for (int i = 0; i < PER_THREAD; ++i) {
-            const bool in = kr + 8 * i < ld_left;
+            const bool in = kr + 8 * i < left;
             at_a[i] = in ? at_a[i] : zero;
             at_b[i] = in ? at_b[i] : zero;
           }
         }
 #pragma unroll
         for (int i = 0; i < PER_THREAD; ++i) asm volatile("" : "+v"(at_a[i]), "+v"(at_b[i]));
-        loaded += (int)((uint32_t)-ld_left >> 31);  // (as below)
-        ld_row += RK;
-        ld_left -= RK;
-        look_up();
       }
     };
     auto load_chunk = [&](auto set_c) {
@@ -523,7 +525,7 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
         ld_a += (size_t)RK * ld_lda;
         ld_b += (size_t)RK * ld_ldb;
         ld_left -= RK;
-        look_up();
+        if (uniform(ld_left) <= 0) next_tile();
       }
     };
     auto store_chunk = [&](auto set_c, int buf) {
@@ -541,20 +543,29 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     };
     using Set0 = std::integral_constant<int, 0>;
     using Set1 = std::integral_constant<int, 1>;
-    look_up();
-    place_chunk();
+    if constexpr (MAPPED) {
+      look_up(Set0{});
+      look_up(Set1{});
+    } else {
+      next_tile();
+    }
+    place_chunk(Set0{});
     load_chunk(Set0{});
     if (loaded == 0) return;  // no tile with rows: nothing for the consumers to wait for
-    place_chunk();
+    look_up(Set0{});
+    place_chunk(Set1{});
     load_chunk(Set1{});
-    place_chunk();
+    look_up(Set1{});
     store_chunk(Set0{}, 0);
+    place_chunk(Set0{});
     load_chunk(Set0{});
+    look_up(Set0{});
     lds_barrier();
     auto step = [&](int g, auto next_set) {
-      place_chunk();
       store_chunk(next_set, (g + 1) & 1);
+      place_chunk(next_set);
       load_chunk(next_set);
+      look_up(next_set);
       lds_barrier();  // the loads of the next chunks stay in flight
     };
     // Always two steps, the one past an odd last chunk with zeros that no one reads, and everything that the
@@ -621,42 +632,47 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
       // Through the wave's own piece of LDS, so that a store instruction writes 8 rows of 128 contiguous
       // bytes instead of 32 rows of 16: a 32 (m) x 64 (n) fragment row as bf16, rows 136 bytes apart,
       // read back 16 bytes per lane.
-      const __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-          j.C + (size_t)tl.slot * M * N + (size_t)tl.m0 * N + tl.n0, 0, 0xfffffff0u, 0x00020000);
+      // (rows past the matrix lie past the buffer's end, and lanes whose columns do are given an offset there: N is a
+      // multiple of 8, so the eight columns are in or out together)
+      const int rows = M - tl.m0 < TM ? M - tl.m0 : TM;
+      const __amdgpu_buffer_rsrc_t c_rsrc =
+          __builtin_amdgcn_make_buffer_rsrc(j.C + (size_t)tl.slot * M * N + (size_t)tl.m0 * N + tl.n0, 0,
+                                            (int)(((uint32_t)rows * N - tl.n0) * 2u), 0x00020000);
       uint8_t* sw = smem + RING_BYTES + wave * 32 * LDE;
-      const int rrow = lane >> 3, rcol = lane & 7;
+      const int rrow = lane >> 3, rcol = lane & 7, col = wn * 64 + rcol * 8;
+      const uint32_t at = tl.n0 + col < N ? (uint32_t)((wm * 128 + rrow) * N + col) * 2u : 0x80000000u;
+      auto write = [&](auto past) {
 #pragma unroll
-      for (int tm = 0; tm < 4; ++tm) {
+        for (int tm = 0; tm < 4; ++tm) {
 #pragma unroll
-        for (int tn = 0; tn < 2; ++tn)
+          for (int tn = 0; tn < 2; ++tn)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            u32x2 o = {pack_bf16x2(acc[tn][tm][4 * q], acc[tn][tm][4 * q + 1]),
-                       pack_bf16x2(acc[tn][tm][4 * q + 2], acc[tn][tm][4 * q + 3])};
-            *reinterpret_cast<u32x2*>(sw + lr * LDE + (tn * 32 + 8 * q + 4 * lk) * 2) = o;
+            for (int q = 0; q < 4; ++q) {
+              u32x2 o = {pack_bf16x2(acc[tn][tm][4 * q], acc[tn][tm][4 * q + 1]),
+                         pack_bf16x2(acc[tn][tm][4 * q + 2], acc[tn][tm][4 * q + 3])};
+              *reinterpret_cast<u32x2*>(sw + lr * LDE + (tn * 32 + 8 * q + 4 * lk) * 2) = o;
+            }
+          // the wave's own LDS traffic runs in order; the compiler must not move the reads (other
+          // lanes' data) above the writes, nor the next round's writes above these reads
+          asm volatile("" ::: "memory");
+          u32x4 o[4];
+#pragma unroll
+          for (int p8 = 0; p8 < 4; ++p8) {
+            const uint8_t* from = sw + (p8 * 8 + rrow) * LDE + rcol * 16;
+            const u32x2 lo = *reinterpret_cast<const u32x2*>(from), hi = *reinterpret_cast<const u32x2*>(from + 8);
+            o[p8] = u32x4{lo[0], lo[1], hi[0], hi[1]};
           }
-        // the wave's own LDS traffic runs in order; the compiler must not move the reads (other
-        // lanes' data) above the writes, nor the next round's writes above these reads
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        const int n = tl.n0 + wn * 64 + rcol * 8;
+          asm volatile("" ::: "memory");
 #pragma unroll
-        for (int p8 = 0; p8 < 4; ++p8) {
-          const int row = p8 * 8 + rrow;
-          const u32x2 lo = *reinterpret_cast<const u32x2*>(sw + row * LDE + rcol * 16);
-          const u32x2 hi = *reinterpret_cast<const u32x2*>(sw + row * LDE + rcol * 16 + 8);
-          const int m = tl.m0 + wm * 128 + tm * 32 + row;
-          if (m < M && n < N) {  // N is a multiple of 8: the eight columns are in or out together
-            u32x4 o = {lo[0], lo[1], hi[0], hi[1]};
-            // (two plain stores of which one is marked non-temporal the compiler merges into one that is not)
-            const int at = ((m - tl.m0) * N + n - tl.n0) * 2;
-            if (j.past_cache)
-              __builtin_amdgcn_raw_buffer_store_b128(o, c_rsrc, at, 0, kNonTemporal);
-            else
-              __builtin_amdgcn_raw_buffer_store_b128(o, c_rsrc, at, 0, 0);
-          }
+          for (int p8 = 0; p8 < 4; ++p8)
+            __builtin_amdgcn_raw_buffer_store_b128(o[p8], c_rsrc, (int)(at + (uint32_t)((tm * 32 + p8 * 8) * N) * 2u), 0,
+                                                   decltype(past)::value ? kNonTemporal : 0);
         }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      }
+      };
+      if (j.past_cache)
+        write(std::true_type{});
+      else
+        write(std::false_type{});
       return;
     }
     float* Pe = j.partial + (size_t)tl.slot * M * N;
