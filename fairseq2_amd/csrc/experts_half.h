@@ -74,14 +74,14 @@ constexpr uint32_t NOWHERE = 0xfffffff0u;      // an offset past any buffer's en
 //   32 of 35, D 1472, F 1216             90 against 79 (2), 80 (3) (the throughput kernel: 1.25 rounds)
 //   64 of 23, D 2944, F 1840             377 against 394, 400      (memory)
 // All are even loads.  Where a few rows reach a part of the experts, or most of the rows one, the tiles that count are
-// few as well and these win by more: the margins below are what even loads lose and skewed ones gain, us of the layer
-// with the margin of e4m3 weights for all, with bf16's:
+// few as well and these win by more.  So single products of bf16 take them on a smaller margin than a sixth, which codes
+// need (they take longer to convert than the model's rounds say), us of the layer with that margin and with bf16's:
 //   20 and 200 tokens, top-4 of 60 by a popularity law, D 1024, F 1408       60.3, 51.1; 73.0, 57.5
-//   20 and 100, top-2 of 8, D 2048, F 12800                                  308, 243; 324, 260
-//   48 and 100, top-8 of 128, D 2048, F 768                                  96.2, 90.4; 130, 125.5
-//   a training step of 260, top-1 of 8, D 640, F 6400                        271, 235
-//   200 evenly, top-6 of 64, D 3072, F 1024; a training step of 260, skewed  217.8, 221.3; 706, 718
-// bf16: matrices and rows of bf16, not codes (which take longer than the model's rounds to convert).
+//   48 and 100, top-8 of 128 by one, D 2048, F 768                           96.2, 90.4; 130, 117
+//   a training step of 2240 D, 960 F, 715 tokens, top-4 of 64 by one         610, 557
+// Gate/up within 70 to 83 % of the model's time: evenly 11 % faster to 2 % slower on small tiles (24 shapes), by a
+// popularity law 15 % faster to 18 % slower; within 85 to 88 % 1 % faster to 12 % slower at D 2048 and above.
+// bf16: matrices and rows of bf16, not codes.
 inline int pick(bool dual, bool bf16, int64_t rows, int groups, int K, int N, int cus) {
   // Of the experts' rows only the device knows how they are spread: the planned ones (Groups), less what blocks of 16
   // pad them by, equally loaded.
@@ -108,7 +108,7 @@ inline int pick(bool dual, bool bf16, int64_t rows, int groups, int K, int N, in
     auto rounds = [&](int64_t n) { return (n + cus - 1) / cus; };
     const int64_t whole = rounds(tiles(256, dual ? 128 : 256)) * (units * 1000 + 6000);
     const int64_t small = rounds(tiles(64, dual ? 64 : 128)) * (units * 400 + 4000);
-    const int64_t percent = !bf16 ? 83 : dual ? 70 : 100 - each / 4;
+    const int64_t percent = bf16 && !dual ? 100 - each / 4 : 83;
     if ((small > memory ? small : memory) * 100 < (whole > memory ? whole : memory) * percent) return 2;
   }
   return 0;
