@@ -78,7 +78,6 @@ constexpr uint32_t NOWHERE = 0xfffffff0u;      // an offset past any buffer's en
 // need (they take longer to convert than the model's rounds say), us of the layer with that margin and with bf16's:
 //   20 and 200 tokens, top-4 of 60 by a popularity law, D 1024, F 1408       60.3, 51.1; 73.0, 57.5
 //   48 and 100, top-8 of 128 by one, D 2048, F 768                           96.2, 90.4; 130, 117
-//   a training step of 2240 D, 960 F, 715 tokens, top-4 of 64 by one         610, 557
 // Gate/up within 70 to 83 % of the model's time: evenly 11 % faster to 2 % slower on small tiles (24 shapes), by a
 // popularity law 15 % faster to 18 % slower; within 85 to 88 % 1 % faster to 12 % slower at D 2048 and above.
 // bf16: matrices and rows of bf16, not codes.
