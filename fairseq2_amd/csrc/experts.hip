@@ -842,7 +842,9 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
     // 2 (gate/up) or 4 (down) groups of 16 channels when K is long, half that when it is short;
     // N / 16 is a multiple of 4, so the channel blocks tile N exactly.  Figures with the kernel.
     // Chunks of 32 rows from 8 rows an expert on (6 rows: 1-4 % slower evenly, 3-8 % faster skewed; 9 and more:
-    // 0-22 % faster); one group for gate/up up to 3 (1.5 rows: 0-15 % faster; 4 rows, skewed: 8 % slower).
+    // 0-22 % faster); one group for gate/up up to 3 and 96 in all (16 experts 3-9 % faster, 128 1-8 %; more rows in
+    // all, where those of the busy experts are read once more per group, by a popularity law: 60 tokens, top-8 of 256,
+    // D 2048, F 1024 79 -> 89 us, 69, top-4 of 128, D 2496, F 1600 98 -> 102).
     const int cus = cu_count_by_xcd();
     if (cus == 0) {
       set_error("experts: cannot query the compute-unit count");
@@ -859,7 +861,7 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
     // (past the caches: chunks share an expert's weights in L2: 126 rows of 8 experts, D 1344, F 14080 140 us with them
     // there, 151 past it; 14 rows, D 4864, F 11136 260, 236; 64 tokens, top-8 of 128, D 2048, F 768 73.5, 70.4)
     const int64_t pairs = pairs_of(grp, max_rows);
-    const bool few = pairs <= 3ll * E && fine_items;
+    const bool few = pairs <= 3ll * E && pairs <= 96 && fine_items;
     auto launch = [&](auto dual_tag, auto fr_tag, auto nt_tag, const void* a, const int32_t* map, int lda,
                       const void* w0, const void* w1, const float* s0, const float* s1, void* c, int ldc, int kdim,
                       int n) {

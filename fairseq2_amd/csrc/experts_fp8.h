@@ -23,7 +23,7 @@
 //   50, top-2 of 8, D 2048, F 12800                  166       148   180
 //   64, top-8 of 128 skewed, D 2048, F 768            69        67   75
 //   50, top-1 of 16, D 5120, F 2048                  107       116   103
-//   24, top-8 of 128, D 2048, F 768                  107       111   99
+//   24, top-2 of 16, D 4096, F 6400                  222       223   214
 //   6, top-2 of 8, D 2048, F 12800                   101       101   92
 // (Loads that run ahead over the ends of items, two blocks of 64 k of each of up to 32 rows in flight: 5-20 % slower,
 // 3 blocks per CU and shorter bursts of loads against 4.)
