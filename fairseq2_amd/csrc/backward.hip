@@ -632,15 +632,16 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
       // Through the wave's own piece of LDS, so that a store instruction writes 8 rows of 128 contiguous
       // bytes instead of 32 rows of 16: a 32 (m) x 64 (n) fragment row as bf16, rows 136 bytes apart,
       // read back 16 bytes per lane.
-      // (rows past the matrix lie past the buffer's end, and lanes whose columns do are given an offset there: N is a
-      // multiple of 8, so the eight columns are in or out together)
+      // (rows past the matrix lie past the buffer's end, and lanes whose columns do stay at an offset there: N is a
+      // multiple of 8, so the eight columns are in or out together.  The host keeps every offset of a tile's rows below)
       const int rows = M - tl.m0 < TM ? M - tl.m0 : TM;
       const __amdgpu_buffer_rsrc_t c_rsrc =
           __builtin_amdgcn_make_buffer_rsrc(j.C + (size_t)tl.slot * M * N + (size_t)tl.m0 * N + tl.n0, 0,
                                             (int)(((uint32_t)rows * N - tl.n0) * 2u), 0x00020000);
       uint8_t* sw = smem + RING_BYTES + wave * 32 * LDE;
       const int rrow = lane >> 3, rcol = lane & 7, col = wn * 64 + rcol * 8;
-      const uint32_t at = tl.n0 + col < N ? (uint32_t)((wm * 128 + rrow) * N + col) * 2u : 0x80000000u;
+      const bool in = tl.n0 + col < N;
+      const uint32_t at = in ? ((uint32_t)(wm * 128 + rrow) * N + col) * 2u : 0xfffffff0u, rows8 = in ? N * 16u : 0u;
       auto write = [&](auto past) {
 #pragma unroll
         for (int tm = 0; tm < 4; ++tm) {
@@ -665,7 +666,7 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
           asm volatile("" ::: "memory");
 #pragma unroll
           for (int p8 = 0; p8 < 4; ++p8)
-            __builtin_amdgcn_raw_buffer_store_b128(o[p8], c_rsrc, (int)(at + (uint32_t)((tm * 32 + p8 * 8) * N) * 2u), 0,
+            __builtin_amdgcn_raw_buffer_store_b128(o[p8], c_rsrc, (int)(at + (uint32_t)(tm * 4 + p8) * rows8), 0,
                                                    decltype(past)::value ? kNonTemporal : 0);
         }
       };
@@ -1238,6 +1239,11 @@ static int launch_wgrad_f32(F32WgradJobs& jobs, const int32_t* a_map, const int3
 }
 static int launch_wgrad(const WgradJobs& jobs, const int32_t* row_map, const int32_t* counts,
                         const int32_t* offsets, int E, hipStream_t st) {
+  for (int i = 0; i < jobs.n; ++i) {
+    const WgradJob& j = jobs.job[i];
+    FS2_REQUIRE((int64_t)(j.M < wgk::TM ? j.M : wgk::TM) * j.N * 2 <= 0xfffffff0ll,
+                "grouped_wgrad: M=%d, N=%d: rows of a tile are addressed with 32-bit byte offsets", j.M, j.N);
+  }
   auto k = row_map != nullptr ? grouped_wgrad_kernel<true> : grouped_wgrad_kernel<false>;
   static bool attr_set = false;  // benign race: setting the attribute is idempotent
   if (!attr_set) {

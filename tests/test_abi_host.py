@@ -206,6 +206,9 @@ def test_backward_entry_points_report_argument_errors_without_touching_the_gpu(l
     assert rc == -1 and b"multiples of 8" in err()
     rc = lib.fs2moe_grouped_wgrad(fake, None, fake, fake, fake, 4, 64, 64, 128, 9, fake, None, 0, None)
     assert rc == -1 and b"dtype 9" in err()
+    # (a tile's rows past 32-bit offsets)
+    rc = lib.fs2moe_grouped_wgrad(fake, None, fake, None, None, 1, 256, 1 << 23, 16, _abi.BF16, fake, None, 0, None)
+    assert rc == -1 and b"32-bit byte offsets" in err()
     assert lib.fs2moe_grouped_wgrad_workspace_bytes(1, 2048, 128, 8192) == 0
     assert lib.fs2moe_grouped_wgrad_workspace_bytes(0, 2048, 128, 8192) > 0  # the router's gradient: segments
     assert lib.fs2moe_grouped_wgrad_workspace_bytes(0, 0, 128, 8192) == -1

@@ -628,7 +628,7 @@ def test_backward_twice_gives_the_same_gradients(gpu_device):
     # (1024 / 256 row blocks here, then 4 column blocks); an odd count leaves the last one alone
     ([(7 * i) % 90 for i in range(33)], 1024, 264), ([(11 * i) % 70 for i in range(35)], 72, 1024),
     ([40 + i for i in range(32)], 520, 520),
-    # enough tiles and rows for the large f32 tiles, experts of more than twice and four times the mean's rows last
+    # many tiles and rows, experts of more than twice and four times the mean's rows last
     ([100, 3, 60, 120, 0, 100, 120, 130, 700, 1100], 1032, 1000), ([90] * 66 + [300, 20, 500], 520, 264),
 ])
 def test_grouped_wgrad_matches_torch(gpu_device, dtype, rows, m, n):
@@ -659,6 +659,22 @@ def test_grouped_wgrad_matches_torch(gpu_device, dtype, rows, m, n):
     assert torch.equal(dw2, dw), "row map"
     one = _abi.grouped_wgrad(a.to(dev), b.to(dev))
     assert_grad_close(one, a.double().T @ b.double(), dtype, "one group")
+
+
+def test_wgrad_of_very_wide_rows(gpu_device):
+    """A tile's rows reach over half of the 32-bit offsets, the last tile's columns past the matrix."""
+    m, n, rows = 256, 4_300_000, 16
+    assert m * n * 2 > 2**31 and n % 256
+    _say("wgrad of wide rows", m, n)
+    g = torch.Generator(gpu_device).manual_seed(0)
+    a, b = (torch.randn(rows, c, generator=g, device=gpu_device).bfloat16() for c in (m, n))
+    dw = _abi.grouped_wgrad(a, b)
+    for lo in range(0, n, 1 << 20):
+        x, y, got = a.float(), b[:, lo : lo + (1 << 20)].float(), dw[:, lo : lo + (1 << 20)].float()
+        ref = x.T @ y
+        # the result's rounding, and those of two sums of 16 products
+        bound = ref.abs() * 2**-8 + (x.abs().T @ y.abs()) * (2 * rows * 2**-24)
+        assert bool(((got - ref).abs() <= bound).all()), lo
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
