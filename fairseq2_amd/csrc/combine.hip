@@ -90,13 +90,18 @@ __global__ __launch_bounds__(kCombWaves* kWave) void combine_kernel(
   const u32x4* base4 = reinterpret_cast<const u32x4*>(base);
   const u32x4* res4 = reinterpret_cast<const u32x4*>(residual);
   u32x4* out4 = reinterpret_cast<u32x4*>(out);
-  const int rj0 = rj[0] >= 0 ? rj[0] : 0;
+  // what slots without a row load: one of the token's rows, or, where it has none, its row of the output (as long, and there
+  // whatever the size of ye)
+  int some = rj[0];
+#pragma unroll
+  for (int j = 1; j < KMAX; ++j) some = some > rj[j] ? some : rj[j];
+  const u32x4* none = some >= 0 ? ye4 + (size_t)some * chunks : out4 + (size_t)__builtin_amdgcn_readfirstlane(t) * chunks;
   for (int c = lane + kWave * part; c < chunks; c += kWave * WPT) {
-    // all of the chunk's loads are issued before the first add (a slot without a row loads the first one's: a condition
-    // would be a branch around each); no one else reads them
+    // all of the chunk's loads are issued before the first add (a condition on a slot's row would be a branch around each);
+    // no one else reads them
     u32x4 v[KMAX];
 #pragma unroll
-    for (int j = 0; j < KMAX; ++j) v[j] = load_weights<NT>(ye4 + (size_t)(rj[j] >= 0 ? rj[j] : rj0) * chunks + c);
+    for (int j = 0; j < KMAX; ++j) v[j] = load_weights<NT>((rj[j] >= 0 ? ye4 + (size_t)rj[j] * chunks : none) + c);
     __builtin_amdgcn_sched_barrier(0);
     float acc[N];
     if (base != nullptr) {
@@ -133,6 +138,9 @@ static int launch_combine(const void* ye, const int32_t* inv_perm, const int32_t
   // are loaded past it (less: 777 tokens, top-8, D 2048 10.2 us with the hint, 9.0 without).  us with one, two and four
   // waves a token: 8192 tokens, top-8, D 2048 55.3, 53.0, 53.8 (without the hint and with the list sorted by exchanges
   // 60.5); 2500, top-6, D 4096 30.6, 28.9, 27.4; 6000, top-8, D 1024 20.8, 21.5, 23.5.
+  // Lists in between the compile-time ones load a row again for each slot left over, and are no slower for it up to eight
+  // slots than with those skipped behind branches: in the layer, D 2048, 8192 tokens, top-3 27.3, 25.0, top-7 54.5, 48.3;
+  // beyond, one more of a list in between pays: 3000 tokens, top-9 by 16 slots 28.0, by 10 23.4; 64, top-12 by 16 4.6.
   const int chunks = D / Chunk<TA>::N;
   const int wpt = T < 2048 || chunks >= 512 ? 4 : chunks >= 256 ? 2 : 1;
   const bool past = (int64_t)T * K * D * (int64_t)sizeof(TA) > (64ll << 20);
@@ -154,6 +162,7 @@ static int launch_combine(const void* ye, const int32_t* inv_perm, const int32_t
   FS2_COMBINE_CASE(4)
   FS2_COMBINE_CASE(6)
   FS2_COMBINE_CASE(8)
+  FS2_COMBINE_CASE(10)
   FS2_COMBINE_CASE(16)
   FS2_COMBINE_CASE(32)
 #undef FS2_COMBINE_CASE

@@ -1011,6 +1011,34 @@ def test_combine_by_rows_and_tokens(gpu_device, t, d, k, dtype):
     assert torch.equal(out, acc.to(dt))
 
 
+# Pairs without a row (-1), first, in between, last and all of a token's, in lists of every compile-time length: what they
+# load in a row's place is not ye's first row, and adds nothing.
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("t", [3, 2100])
+@pytest.mark.parametrize("k", [1, 2, 3, 5, 8, 9, 10, 11, 17])
+def test_combine_of_pairs_without_rows(gpu_device, t, k, dtype):
+    _say("combine without rows", t, k, dtype)
+    d, dev, dt = 520, gpu_device, TORCH_DTYPE[dtype]
+    g = torch.Generator(dev).manual_seed(t + k)
+    idx = torch.rand(t, 32, generator=g, device=dev).argsort(dim=1)[:, :k].to(torch.int32).contiguous()
+    inv = 1 + torch.randperm(t * k, generator=g, device=dev).view(t, k).to(torch.int32)
+    order = idx.argsort(dim=1)
+    inv[0] = -1
+    inv[1, order[1, 0]] = -1
+    inv[2::2, order[2, k // 2]] = -1
+    ye = torch.randn(t * k + 1, d, generator=g, device=dev).to(dt)
+    ye[0] = float("nan")
+    base = torch.randn(t, d, generator=g, device=dev).to(dt)
+    out = _abi.combine(ye, inv, idx, torch.rand(t, k, device=dev), base, False)
+    acc = base.float()
+    for j in range(k):
+        row = inv.gather(1, order[:, j : j + 1])
+        acc = acc + torch.where(row >= 0, ye[row[:, 0].clamp(min=0)].float(), 0.0)
+    assert torch.equal(out, acc.to(dt))
+    assert torch.equal(_abi.combine(ye[1:2], torch.full_like(inv, -1), idx, None, base, False), base)
+    assert float(_abi.combine(ye[1:2], torch.full_like(inv, -1), idx, None, None, False).float().abs().max()) == 0.0
+
+
 # ------------------------------------------------------------------------ experts, fp8 weights
 @pytest.mark.parametrize(
     "rows_per_expert,d,f",
