@@ -294,7 +294,7 @@ int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_
     }
     if (scaled_stream)
       return fs2moe::grouped_swiglu_scaled_rows(x, b.perm, b.row_w, b.counts, b.offsets, w_gate, w_up,
-                                                w_down, E, D, F, b.max_rows, b.h, b.ye, T, stream);
+                                                w_down, E, D, F, b.max_rows, planned, b.h, b.ye, T, stream);
     // (a token takes an expert at most once: with up to 16 tokens no expert has more rows than that)
     return fs2moe::grouped_swiglu_planned(fused ? x : b.xe, fused ? b.perm : nullptr, b.counts, b.offsets,
                                           w_gate, w_up, w_down, s_gate, s_up, s_down, E, D, F, b.max_rows,

@@ -290,8 +290,8 @@ bool swiglu_streams_rows(int32_t act_dtype, int32_t w_dtype, int32_t D, int32_t 
 int grouped_swiglu_scaled_rows(const void* x, const int32_t* row_map, const float* row_w,
                                const int32_t* counts, const int32_t* offsets, const void* w_gate,
                                const void* w_up, const void* w_down, int32_t E, int32_t D, int32_t F,
-                               int64_t max_rows, void* h, void* ye, int32_t rows_per_expert,
-                               void* stream);
+                               int64_t max_rows, int64_t planned, void* h, void* ye,
+                               int32_t rows_per_expert, void* stream);
 
 // ---- pieces of a training step (fs2moe_train_forward / fs2moe_train_backward)
 // Whether the SwiGLU pair keeps its two products at these sizes, and that pair (E 0: one group of `rows`

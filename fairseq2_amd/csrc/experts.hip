@@ -920,14 +920,14 @@ bool fs2moe::swiglu_streams_rows(int32_t act_dtype, int32_t w_dtype, int32_t D, 
 int fs2moe::grouped_swiglu_scaled_rows(const void* x, const int32_t* row_map, const float* row_w,
                                        const int32_t* counts, const int32_t* offsets,
                                        const void* w_gate, const void* w_up, const void* w_down,
-                                       int32_t E, int32_t D, int32_t F, int64_t max_rows, void* h,
-                                       void* ye, int32_t rows_per_expert, void* stream) {
+                                       int32_t E, int32_t D, int32_t F, int64_t max_rows, int64_t planned,
+                                       void* h, void* ye, int32_t rows_per_expert, void* stream) {
   FS2_REQUIRE(row_map && row_w, "grouped_swiglu: null pointer");
   FS2_REQUIRE(swiglu_streams_rows(FS2MOE_BF16, FS2MOE_BF16, D, F, E, rows_per_expert),
               "grouped_swiglu: internal: D=%d F=%d E=%d with %d rows an expert do not stream", D, F, E,
               rows_per_expert);
   return grouped_swiglu_impl(x, row_map, counts, offsets, w_gate, w_up, w_down, nullptr, nullptr,
-                             nullptr, E, D, F, max_rows, 0, FS2MOE_BF16, FS2MOE_BF16, h, ye,
+                             nullptr, E, D, F, max_rows, planned, FS2MOE_BF16, FS2MOE_BF16, h, ye,
                              rows_per_expert, stream, row_w);
 }
 

@@ -2,6 +2,8 @@
 
 from __future__ import annotations
 
+import re
+
 import numpy as np
 import torch
 
@@ -122,3 +124,18 @@ def assert_routing_equal(idx_gpu, disp, r: O.Routing, what: str = ""):
     np.testing.assert_array_equal(perm[: r.num_rows], r.perm, err_msg=f"{what} perm")
     assert (perm[r.num_rows :] == -1).all(), f"{what} perm tail"
     np.testing.assert_array_equal(disp.inv_perm.cpu().numpy(), r.inv_perm, err_msg=f"{what} inv_perm")
+
+
+def launched(run) -> list[str]:
+    """The library's kernels that ``run()`` launches, as ``name<template arguments>`` in order.  Which variant a rule
+    takes does not show in results that are the same bits from all of them."""
+    from torch.profiler import ProfilerActivity, profile
+
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        run()
+        torch.cuda.synchronize()
+    kernels = sorted((e for e in prof.events() if "fs2moe::" in e.name), key=lambda e: e.time_range.start)
+    names = [re.search(r"fs2moe::(\w+(?:<[^()]*(?:\([^()]*\)[^()]*)*>)?)\(", e.name) for e in kernels]
+    assert names and all(names), [e.name for e in kernels]
+    return [n.group(1).replace("fs2moe::", "") for n in names]

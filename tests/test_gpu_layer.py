@@ -13,7 +13,7 @@ from fairseq2_amd import _abi
 import workloads as W
 from oracle import moe_oracle as O
 from tests._util import (
-    TORCH_DTYPE, assert_output_close, assert_routing_equal, build_module, oracle_forward, oracle_routing,
+    TORCH_DTYPE, assert_output_close, assert_routing_equal, build_module, launched, oracle_forward, oracle_routing,
 )
 
 pytestmark = pytest.mark.gpu
@@ -129,6 +129,27 @@ def test_decode_steps_in_the_reference_mode_without_a_row_copy(gpu_device, token
     torch.cuda.synchronize()
     assert torch.equal(single, out)
     assert torch.equal(single_res, staged_res)
+
+
+# Expert weights are loaded past the caches where those that the tokens can reach are more than the last-level cache
+# holds (128 experts of 3.1 MB here): one token reaches 4 and 40 reach them all, whichever routing mode reads the rows.
+@pytest.mark.parametrize("tokens,past", [(1, False), (12, False), (16, False), (40, True)])
+@pytest.mark.parametrize("mode", ["reference", "softmax"])
+def test_decode_steps_count_the_experts_that_their_tokens_reach(gpu_device, tokens, past, mode):
+    _say("reached experts", tokens, mode)
+    how = (W.RoutingMode("sigmoid", False, "input") if mode == "reference" else W.RoutingMode("softmax", True, "output"))
+    spec = W.small_spec(tokens=tokens, model_dim=1024, num_experts=128, top_k=4, inner_dim=512, mode=how, seed=1)
+    wl = W.make_workload_from_spec(spec)
+    m, x = build_module(wl, gpu_device), wl.x.bfloat16().to(gpu_device)
+    with torch.no_grad():
+        m(x)
+        names = launched(lambda: m(x))
+    if tokens <= 16:  # <two products, rows, past the caches>
+        streams = [n for n in names if n.startswith("glu_gemv")]
+        assert len(streams) == 2 and all(n.rstrip(">").split(", ")[2] == str(past).lower() for n in streams), names
+    else:
+        assert any(n.startswith(("glu_gemm_half_kernel", "glu_gemm_bf16_dma_kernel")) and n.endswith(str(past).lower() + ">")
+                   for n in names), names
 
 
 def test_empty_input(gpu_device):
