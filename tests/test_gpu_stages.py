@@ -7,7 +7,7 @@ import torch
 from fairseq2_amd import _abi
 import workloads as W
 from oracle import moe_oracle as O
-from tests._util import TORCH_DTYPE, assert_output_close, assert_routing_equal, oracle_routing
+from tests._util import TORCH_DTYPE, assert_output_close, assert_routing_equal, launched, oracle_routing
 
 pytestmark = pytest.mark.gpu
 
@@ -792,6 +792,17 @@ def test_weights_past_the_caches_give_the_same_bits(gpu_device, d, f):
     xq, xs = _abi.mx_quantize(x[:total].contiguous())
     both(rows, total, lambda c, o, e, t: _abi.grouped_swiglu_w8a8(
         xq, xs, c, o, *(q[:e] for q in packed), tuple(s[:e] for s in scales), e)[:2])
+
+
+# The shared expert's weights are loaded past the caches where their rows begin on lines: off them a line is read twice.
+@pytest.mark.parametrize("d,f,past", [(4096, 8192, True), (4104, 8192, False), (4096, 8200, False), (5160, 8232, False)])
+def test_shared_expert_off_the_lines_goes_through_the_caches(gpu_device, d, f, past):
+    _say("shared expert on lines", d, f)
+    x = torch.randn(3, d, device=gpu_device).bfloat16()
+    w = [torch.randn(*s, device=gpu_device).bfloat16() * 0.02 for s in ((f, d), (f, d), (d, f))]
+    names = launched(lambda: _abi.dense_swiglu(x, *w))
+    flag = str(past).lower()
+    assert names == [f"dense_gemv_bf16_kernel<true, {flag}>", f"dense_gemv_bf16_kernel<false, {flag}>"]
 
 
 # Which tiles products of bf16 take follows from the size of the buffers (one round of small ones, several rounds of
