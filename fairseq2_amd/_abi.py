@@ -94,6 +94,12 @@ _PROTOTYPES = {
          c_void_p, c_int32, c_int32, c_int32, c_int64, c_int32, c_int32, c_void_p, c_void_p,
          c_int32, c_void_p],
     ),
+    "fs2moe_grouped_swiglu_pairs": (
+        c_int32,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+         c_void_p, c_int32, c_int32, c_int32, c_int64, c_int32, c_int32, c_void_p, c_void_p,
+         c_int32, c_int64, c_void_p],
+    ),
     "fs2moe_grouped_swiglu_fuses_gather": (c_int32, [c_int32, c_int32, c_int32, c_int32]),
     "fs2moe_grouped_swiglu_keeps": (c_int32, [c_int32, c_int32, c_int64, c_int32]),
     "fs2moe_dense_swiglu_keep": (c_int32, [c_void_p] * 4 + [c_int32] * 4 + [c_void_p] * 5),
@@ -492,12 +498,15 @@ def grouped_swiglu(
     scales: tuple[Tensor, Tensor, Tensor] | None = None,
     row_map: Tensor | None = None,
     rows_per_expert: int = 0,
+    pairs: int = 0,
 ) -> tuple[Tensor, Tensor]:
     """Returns ``(ye, h)`` for the rows of ``xe`` (rows, D).
 
     ``rows_per_expert``: an upper bound on the rows of any one expert when the caller knows one
     (the number of tokens is one), else 0; with 1..16 and bf16 weights the products run as streams
-    over the weights instead of as GEMM tiles (``fs2moe_grouped_swiglu_rows``).
+    over the weights instead of as GEMM tiles (``fs2moe_grouped_swiglu_rows``).  ``pairs``: how many rows
+    the experts have in all, without padding, when the caller knows it (tokens times experts per token),
+    else 0: the kernels are chosen by it (``fs2moe_grouped_swiglu_pairs``).
 
     With ``row_map`` (int32, one entry per row: ``Dispatched.perm``) ``xe`` is the token matrix
     ``(T, D)`` and row ``r`` of the experts' input is ``xe[row_map[r]]``: the gather is fused into
@@ -538,12 +547,12 @@ def grouped_swiglu(
     h = torch.empty((rows, f), dtype=xe.dtype, device=xe.device)
     ye = torch.empty((rows, d), dtype=xe.dtype, device=xe.device)
     sg, su, sd = scales if scales is not None else (None, None, None)
-    rc = lib.fs2moe_grouped_swiglu_rows(
+    rc = lib.fs2moe_grouped_swiglu_pairs(
         _ptr(xe), _ptr(row_map), _ptr(counts), _ptr(offsets), _ptr(w_gate), _ptr(w_up),
         _ptr(w_down), _ptr(sg), _ptr(su), _ptr(sd), num_experts, d, f, rows, dtype_code(xe.dtype),
-        dtype_code(w_gate.dtype), _ptr(h), _ptr(ye), int(rows_per_expert), _stream(),
+        dtype_code(w_gate.dtype), _ptr(h), _ptr(ye), int(rows_per_expert), int(pairs), _stream(),
     )
-    _check(rc, "fs2moe_grouped_swiglu_rows")
+    _check(rc, "fs2moe_grouped_swiglu_pairs")
     return ye, h
 
 

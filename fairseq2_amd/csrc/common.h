@@ -265,7 +265,7 @@ int dispatch_with_row_weights(const int32_t* topk_idx, const float* topk_w, int3
 // have.  Where the plan decides how sums are cut, results then do not depend on the padding.
 inline int64_t planned_rows(int64_t pairs, int E) { return pairs + 15ll * E; }
 // fs2moe_grouped_swiglu_rows, fs2moe_grouped_swiglu_w8a8 and fs2moe_grouped_gemm for callers that know the planned rows
-// (the stage calls know the buffers' size alone, and plan by that).
+// (most stage calls know the buffers' size alone, and plan by that).
 int grouped_swiglu_planned(const void* xe, const int32_t* row_map, const int32_t* counts, const int32_t* offsets,
                            const void* w_gate, const void* w_up, const void* w_down, const float* s_gate,
                            const float* s_up, const float* s_down, int32_t E, int32_t D, int32_t F, int64_t max_rows,

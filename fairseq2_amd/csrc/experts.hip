@@ -217,17 +217,22 @@ static int launch_f32(const void* a, const void* b0, const void* b1, const void*
   return check_launch(what);
 }
 
-// e4m3 weights go to the throughput kernels from this many rows per expert on (mean over all experts, of the rows
-// planned, 15 of which may be padding).  us of the layer, streamed against there:
-//   20 rows an expert on average   (D 1024, F 1408, top-4 of 60) 83, 102; (4096, 6400, 2 of 16) 261, 286
-//   25                             (4096, 1152, 8 of 32) 129, 142; (2048, 768, 8 of 128) 172, 184; (4096, 6400) 307,
-//                                  294
-//   27, 28                         (1024, 1408) 95, 103; (3072, 1024, 6 of 64) 179, 174
-//   37                             (3072, 1024) 246, 176; (2048, 12800, 2 of 8) 243, 204
-#ifndef FS2MOE_FP8_GEMM_MIN_ROWS
-#define FS2MOE_FP8_GEMM_MIN_ROWS 42
-#endif
-constexpr int64_t kFp8GemmMinRowsPerExpert = FS2MOE_FP8_GEMM_MIN_ROWS;
+// e4m3 weights go to the throughput kernels from this many rows per expert on (mean over all experts).  us of the layer,
+// streamed against there, loaded evenly and by a popularity law of exponent 1.2:
+//                                          20 rows             25                  28                  37
+//   D 1024, F 1408, top-4 of 60      77, 98    68, 78    84, 99    76, 83    92, 99    80, 85   120, 101   93, 94
+//   2048, 768, 8 of 128             166, 186  134, 146  178, 187  151, 157  188, 187  162, 159  236, 191  198, 172
+//   4096, 6400, 2 of 16             273, 296  311, 310  305, 299  326, 337  325, 300  342, 353  432, 312  398, 372
+//   4096, 1152, 8 of 32             123, 144  135, 146  130, 145  145, 147  145, 146  155, 148  193, 152  174, 155
+//   3072, 1024, 6 of 64             158, 172  162, 192  174, 173  179, 198  183, 174  188, 198  244, 177  217, 203
+//   2048, 12800, 2 of 8             163, 190  183, 213  179, 196  198, 217  200, 206  205, 220  247, 215  232, 230
+//   5120, 2048, 1 of 16             133, 141  145, 153  152, 146  156, 165  156, 148  164, 173  201, 153  188, 192
+//   1024, 4096, 2 of 16              70,  83   69,  91   78,  86   79,  96   84,  88   82,  97   104,  88   89,  97
+// (from 25 on the large experts of an even load lose 1 to 6 % and all others gain up to 17; no size tells them apart
+// from a skewed load, which the host does not see)
+constexpr int64_t kFp8GemmMinRowsPerExpert = 27;
+// Of a caller that does not say how many rows the experts have: so many of the buffers', which may have no padding.
+constexpr int64_t kFp8GemmMinBufferRows = 32;
 
 // The bf16 throughput kernel takes any D and F that are multiples of 8 (its KTAIL variants where a K is
 // not a multiple of the unit's 64).  The entry points that exist for whole units only (the fused
@@ -829,11 +834,13 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
     // Two regimes.  With many rows per expert the layer is a GEMM: the bf16 throughput kernel, its
     // producers turning the codes into bf16 on the way to LDS (half the weight bytes of bf16, the
     // same matrix rate).  With few (decode) it is a stream over the weights: the kernels below.  The
-    // row counts live on the device, so the choice goes by the mean number of rows per expert the
-    // buffers are sized for.
+    // row counts live on the device, so the choice goes by the mean number of rows per expert, whatever
+    // the buffers are padded to; only where the caller does not say them by the buffers' rows.
     // (the streaming kernels build their item table with a thread per expert: up to 256 experts)
-    if ((max_rows / E >= kFp8GemmMinRowsPerExpert || E > 256) && dma_offsets_fit(max_rows, D, F)) {
-      Groups g{counts, offsets, E, 0, (int)planned};
+    Groups g{counts, offsets, E, 0, (int)planned};
+    const int64_t pairs = pairs_of(g, max_rows);
+    const bool many = g.planned > 0 ? pairs >= kFp8GemmMinRowsPerExpert * E : max_rows >= kFp8GemmMinBufferRows * E;
+    if ((many || E > 256) && dma_offsets_fit(max_rows, D, F)) {
       return launch_dma_pair<dma::W_FP8_TILED>(xe, row_map, g, max_rows, w_gate, w_up, w_down, s_gate,
                                                s_up, s_down, D, F, h, ye, st);
     }
@@ -847,7 +854,8 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
     // Chunks of 32 rows from 8 rows an expert on (6 rows: 1-4 % slower evenly, 3-8 % faster skewed; 9 and more:
     // 0-22 % faster); one group for gate/up up to 3 and 96 in all (16 experts 3-9 % faster, 128 1-8 %; more rows in
     // all, where those of the busy experts are read once more per group, by a popularity law: 60 tokens, top-8 of 256,
-    // D 2048, F 1024 79 -> 89 us, 69, top-4 of 128, D 2496, F 1600 98 -> 102).
+    // D 2048, F 1024 79 -> 89 us, 69, top-4 of 128, D 2496, F 1600 98 -> 102).  Of a caller that does not say the rows
+    // neither, unless the buffers hold more than 8 rows an expert besides the padding to 16.
     const int cus = cu_count_by_xcd();
     if (cus == 0) {
       set_error("experts: cannot query the compute-unit count");
@@ -860,11 +868,9 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
       return FS2MOE_ERR_UNSUPPORTED;
     }
     const bool fine_items = chunks * (F / 16) <= 0x7fffffffll;
-    const Groups grp{counts, offsets, E, 0, (int)planned};
     // (past the caches: chunks share an expert's weights in L2: 126 rows of 8 experts, D 1344, F 14080 140 us with them
     // there, 151 past it; 14 rows, D 4864, F 11136 260, 236; 64 tokens, top-8 of 128, D 2048, F 768 73.5, 70.4)
-    const int64_t pairs = pairs_of(grp, max_rows);
-    const bool few = pairs <= 3ll * E && pairs <= 96 && fine_items;
+    const bool few = g.planned > 0 && pairs <= 3ll * E && pairs <= 96 && fine_items;
     auto launch = [&](auto dual_tag, auto fr_tag, auto nt_tag, const void* a, const int32_t* map, int lda,
                       const void* w0, const void* w1, const float* s0, const float* s1, void* c, int ldc, int kdim,
                       int n) {
@@ -890,8 +896,9 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
       launch(std::false_type{}, fr, nt, h, nullptr, F, w_down, nullptr, s_down, nullptr, ye, D, F, D);
       return check_launch("glu_gemm_fp8w<down>");
     };
-    if (pairs > 8ll * E) return pair(std::integral_constant<int, 2>{}, std::false_type{});
-    if (weights_past_cache(E, pairs, D, F, 1)) return pair(std::integral_constant<int, 1>{}, std::true_type{});
+    if ((g.planned > 0 ? pairs : max_rows - 15ll * E) > 8ll * E)
+      return pair(std::integral_constant<int, 2>{}, std::false_type{});
+    if (g.planned > 0 && weights_past_cache(E, pairs, D, F, 1)) return pair(std::integral_constant<int, 1>{}, std::true_type{});
     return pair(std::integral_constant<int, 1>{}, std::false_type{});
   }
   if (w_dtype != act_dtype) {
@@ -900,7 +907,7 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
     return FS2MOE_ERR_UNSUPPORTED;
   }
   if (max_rows == 0) return FS2MOE_OK;
-  Groups g{counts, offsets, E, 0, (int)planned};
+  const Groups g{counts, offsets, E, 0, (int)planned};
   return launch_glu<FS2MOE_W_IN_OUT>(xe, row_map, g, max_rows, w_gate, w_up, w_down, D, F, act_dtype,
                                      h, ye, static_cast<hipStream_t>(stream), rows_hint, row_w);
 }
@@ -953,6 +960,21 @@ extern "C" int fs2moe_grouped_swiglu_rows(const void* xe, const int32_t* row_map
                                           void* h, void* ye, int32_t rows_per_expert, void* stream) {
   return grouped_swiglu_impl(xe, row_map, counts, offsets, w_gate, w_up, w_down, s_gate, s_up, s_down,
                              E, D, F, max_rows, 0, act_dtype, w_dtype, h, ye, rows_per_expert, stream);
+}
+
+extern "C" int fs2moe_grouped_swiglu_pairs(const void* xe, const int32_t* row_map,
+                                           const int32_t* counts, const int32_t* offsets,
+                                           const void* w_gate, const void* w_up, const void* w_down,
+                                           const float* s_gate, const float* s_up,
+                                           const float* s_down, int32_t E, int32_t D, int32_t F,
+                                           int64_t max_rows, int32_t act_dtype, int32_t w_dtype,
+                                           void* h, void* ye, int32_t rows_per_expert, int64_t pairs,
+                                           void* stream) {
+  FS2_REQUIRE(pairs >= 0 && pairs <= (max_rows > 0 ? max_rows : 0),
+              "grouped_swiglu: %lld rows of experts in buffers of %lld", (long long)pairs, (long long)max_rows);
+  return grouped_swiglu_impl(xe, row_map, counts, offsets, w_gate, w_up, w_down, s_gate, s_up, s_down, E, D, F,
+                             max_rows, pairs > 0 ? planned_rows(pairs, E) : 0, act_dtype, w_dtype, h, ye,
+                             rows_per_expert, stream);
 }
 
 int fs2moe::grouped_swiglu_planned(const void* xe, const int32_t* row_map, const int32_t* counts,

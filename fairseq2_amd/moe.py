@@ -139,7 +139,7 @@ class GroupedExpertNetwork(ExpertNetwork):
         return isinstance(_part(self, "activation"), nn.SiLU)
 
     # Rows go to the fp8 matrix pipe from this many per expert on (mean over all experts; the library
-    # takes its bf16-pipe GEMMs for e4m3 weights from about 27 on); below that the experts are a weight
+    # takes its bf16-pipe GEMMs for e4m3 weights from 27 on); below that the experts are a weight
     # stream, which activations of one byte would not make faster.
     _W8A8_MIN_ROWS_PER_EXPERT = 32
 
@@ -272,12 +272,13 @@ class GroupedExpertNetwork(ExpertNetwork):
 
     def forward_rows(
         self, xe: Tensor, counts: Tensor, offsets: Tensor, row_map: Tensor | None = None,
-        rows_per_expert: int = 0,
+        rows_per_expert: int = 0, pairs: int = 0,
     ) -> Tensor:
         """Runs every expert on its block of rows of ``xe`` (rows, D); with ``row_map``, row ``r``
         is ``xe[row_map[r]]`` and ``xe`` is the token matrix.  ``rows_per_expert``: an upper bound
         on any expert's rows when the caller knows one (the number of tokens is one), else 0; up to 16
-        the bf16 experts run as streams over their weights.  Inference only (the training paths are
+        the bf16 experts run as streams over their weights.  ``pairs``: how many rows the experts have in
+        all when the caller knows it, else 0: the kernels are then chosen by it.  Inference only (the training paths are
         :meth:`forward` and the layer's)."""
         _require_forward_only(xe, self.gate_proj, self.inner_proj, self.output_proj)
         if not self.has_fused_gate:
@@ -305,13 +306,13 @@ class GroupedExpertNetwork(ExpertNetwork):
             ye, _ = _abi.grouped_swiglu(
                 xe, counts, offsets, self.gate_q, self.inner_q, self.output_q,
                 self.num_local_experts,
-                scales=(self.gate_scale, self.inner_scale, self.output_scale), row_map=row_map,
+                scales=(self.gate_scale, self.inner_scale, self.output_scale), row_map=row_map, pairs=pairs,
             )
             return ye
         ye, _ = _abi.grouped_swiglu(
             xe, counts, offsets, self.gate_proj.detach(), self.inner_proj.detach(),
             self.output_proj.detach(), self.num_local_experts, row_map=row_map,
-            rows_per_expert=rows_per_expert,
+            rows_per_expert=rows_per_expert, pairs=pairs,
         )
         return ye
 
@@ -340,7 +341,14 @@ class GroupedExpertNetwork(ExpertNetwork):
             return ye.view(e, n, d)
         # (every expert has exactly n rows: a bound the library can use when it is small)
         return self.forward_rows(x.reshape(e * n, d).contiguous(), counts, offsets,
-                                 rows_per_expert=n if n <= 16 else 0).view(e, n, d)
+                                 **self._row_hints(n if n <= 16 else 0, e * n)).view(e, n, d)
+
+    def _row_hints(self, rows_per_expert: int, pairs: int) -> dict[str, int]:
+        """What is known of the rows, for :meth:`forward_rows` (an override of it may not take ``pairs``)."""
+        hints = {"rows_per_expert": rows_per_expert} if rows_per_expert else {}
+        if type(self).forward_rows is GroupedExpertNetwork.forward_rows:
+            hints["pairs"] = pairs
+        return hints
 
     def _uniform_groups(self, n: int, device: torch.device) -> tuple[Tensor, Tensor]:
         """counts / offsets of ``n`` rows for every expert, built once per (n, device) so that the
@@ -720,7 +728,9 @@ class MoE(FeedForwardNetwork):
         )
         # a token takes an expert at most once: with up to 16 tokens no expert has more rows than that
         # (what the whole-layer call passes on as well)
-        hint = dict(rows_per_expert=x.shape[0]) if isinstance(ex, GroupedExpertNetwork) and x.shape[0] <= 16 else {}
+        hint = {}
+        if isinstance(ex, GroupedExpertNetwork):
+            hint = ex._row_hints(x.shape[0] if x.shape[0] <= 16 else 0, idx.numel())
         if fused:
             ye = ex.forward_rows(x, disp.counts, disp.offsets, row_map=disp.perm, **hint)
         else:

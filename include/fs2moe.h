@@ -194,6 +194,19 @@ int fs2moe_grouped_swiglu_rows(const void* xe, const int32_t* row_map, const int
                                void* ye, int32_t rows_per_expert, void* stream);
 
 /*
+ * fs2moe_grouped_swiglu_rows for a caller that knows how many rows the experts have in all (pairs: T * K
+ * after fs2moe_dispatch, at most max_rows; 0: not known, then this is fs2moe_grouped_swiglu_rows).  The
+ * kernels are chosen by them instead of by the buffers, of which padding may be any part: the choice of
+ * the whole-layer calls, whose results then have the same bits.
+ */
+int fs2moe_grouped_swiglu_pairs(const void* xe, const int32_t* row_map, const int32_t* counts,
+                                const int32_t* offsets, const void* w_gate, const void* w_up,
+                                const void* w_down, const float* s_gate, const float* s_up,
+                                const float* s_down, int32_t E, int32_t D, int32_t F,
+                                int64_t max_rows, int32_t act_dtype, int32_t w_dtype, void* h,
+                                void* ye, int32_t rows_per_expert, int64_t pairs, void* stream);
+
+/*
  * 1 if fs2moe_grouped_swiglu accepts a row_map for these sizes and types, else 0.  Like
  * fs2moe_grouped_swiglu_keeps and fs2moe_grouped_gemm_sum_supported it says 1 for D and F in whole
  * units of 64; the whole-layer and training calls read rows in place, keep the products and add the

@@ -106,6 +106,10 @@ def test_argument_errors_are_reported_without_touching_the_gpu(lib):
     rc = lib.fs2moe_grouped_swiglu_rows(fake, None, fake, fake, fake, fake, fake, None, None, None, 4, 64, 64, 128, _abi.BF16, _abi.BF16, fake, fake, -1, None)
     assert rc == -1 and b"rows_per_expert" in lib.fs2moe_last_error()
     assert lib.fs2moe_grouped_swiglu_rows(fake, None, fake, fake, fake, fake, fake, None, None, None, 4, 64, 64, 0, _abi.BF16, _abi.BF16, fake, fake, 2, None) == 0
+    # the rows that experts have are at most those of the buffers
+    for rows, want in ((129, -1), (-1, -1), (128, None)):
+        rc = lib.fs2moe_grouped_swiglu_pairs(fake, None, fake, fake, fake, fake, fake, None, None, None, 4, 60, 64, 128, _abi.BF16, _abi.BF16, fake, fake, 2, rows, None)
+        assert rc == -1 and (b"in buffers of 128" if want else b"multiples of 8") in lib.fs2moe_last_error()
     # the fused gather exists for bf16 activations with D and F multiples of 64 (bf16 or e4m3
     # weights), and nowhere else
     assert lib.fs2moe_grouped_swiglu_fuses_gather(2048, 768, _abi.BF16, _abi.BF16) == 1

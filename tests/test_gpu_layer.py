@@ -152,6 +152,44 @@ def test_decode_steps_count_the_experts_that_their_tokens_reach(gpu_device, toke
                    for n in names), names
 
 
+# Whether e4m3 experts run as a stream over their weights or on GEMM tiles, and by which pieces, goes by the rows that the
+# experts have and not by the buffers' padding: the same kernels, and so the same bits, in one call and by stages.
+# <two products, waves along K, channel groups, sixteens of rows, past the caches>
+@pytest.mark.parametrize("tokens,gate_up", [
+    (12, "4, 1, 1"), (16, "4, 2, 1"), (32, "4, 2, 1"), (33, "4, 2, 2"), (80, "4, 2, 2"), (107, "4, 2, 2"), (108, None),
+    (148, None)])
+def test_e4m3_kernels_go_by_the_rows_whatever_the_padding(gpu_device, tokens, gate_up):
+    _say("e4m3 by rows", tokens)
+    spec = W.small_spec(tokens=tokens, model_dim=512, num_experts=8, top_k=2, inner_dim=576, weight_dtype="fp8",
+                        mode=W.RoutingMode("softmax", True, "output"), seed=tokens)
+    wl = W.make_workload_from_spec(spec)
+    x, outs = wl.x.bfloat16().to(gpu_device), []
+    for tile_m in (1, 16, 32, 128):
+        m = build_module(wl, gpu_device, tile_m)
+        for call in (m, lambda v: m.forward_with_routing(v)[0]):
+            with torch.no_grad():
+                names = launched(lambda: outs.append(call(x)))
+            streams = [n for n in names if n.startswith("glu_gemm_fp8w_kernel")]
+            tiles = [n for n in names if n.startswith(("glu_gemm_half", "glu_gemm_bf16_dma"))]
+            if gate_up:
+                assert len(streams) == 2 and not tiles and f"<true, {gate_up}, " in streams[0], names
+            else:
+                assert len(tiles) == 2 and not streams, names
+    assert all(torch.equal(o, outs[0]) for o in outs)
+
+
+def test_e4m3_experts_alone_go_by_their_rows(gpu_device):
+    _say("e4m3 experts alone")
+    for n, kind in ((2, "fp8w_kernel<true, 4, 1, 1"), (9, "fp8w_kernel<true, 4, 2, 2"), (26, "fp8w_kernel<true, 4, 2, 2"),
+                    (27, "half")):
+        spec = W.small_spec(model_dim=512, num_experts=8, top_k=2, inner_dim=576, weight_dtype="fp8", seed=n)
+        ex = build_module(W.make_workload_from_spec(spec), gpu_device).experts
+        xe = torch.randn(8, n, 512, device=gpu_device).bfloat16()
+        with torch.no_grad():
+            names = launched(lambda: ex(xe))
+        assert names[0].startswith("glu_gemm_" + kind), names
+
+
 def test_empty_input(gpu_device):
     wl = W.make_workload_from_spec(W.small_spec(tokens=4, dtype="bf16"))
     m = build_module(wl, gpu_device)

@@ -835,27 +835,34 @@ def test_products_of_few_rows_are_the_same_on_every_tile_size(gpu_device, e, d, 
         assert_output_close(got[0][0][at : at + n], ref.cpu(), "bf16", f"expert {i}")
 
 
-# How many rows and channels a piece of the e4m3 stream's work has follows from the size of the buffers: the same bits,
-# for rows on both sides of 16 and 32, K within a step, past one and split over two waves, against the oracle.
+# How many rows and channels a piece of the e4m3 stream's work has follows from the rows that the caller says: the same
+# bits, for rows on both sides of 16 and 32, K within a step, past one and split over two waves, against the oracle.
 @pytest.mark.parametrize("d,f", [(512, 1024), (448, 704), (1088, 64)])
 def test_e4m3_streams_of_every_chunk_are_the_same(gpu_device, d, f):
     _say("e4m3 stream", d, f)
     e, dev, bf = 32, gpu_device, torch.bfloat16
     g = torch.Generator(dev).manual_seed(d)
     rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(bf)
-    rows = [33, 32, 17, 16, 1, 0, 48, 31] + [0] * (e - 8)
+    rows = [33, 32, 17, 16, 1, 0, 48, 31] + [0] * (e - 10) + [40, 5]
     counts = torch.tensor(rows, dtype=torch.int32, device=dev)
     offsets = torch.zeros(e + 1, dtype=torch.int32, device=dev)
     offsets[1:] = torch.cumsum((counts + 15) // 16 * 16, 0)
     lo = offsets.tolist()
-    x = rnd(24 * e, d)
+    x = rnd(lo[-1], d)
     codes = [(rnd(e * i, o) * 0.05).to(torch.float8_e4m3fn) for i, o in ((d, f), (d, f), (f, d))]
     packed = [_abi.pack_fp8_weights(c, e) for c in codes]
     scales = [torch.rand(e, n, generator=g, device=dev) + 0.5 for n in (f, f, d)]
-    got = []
-    for total in (18 * e, 20 * e, 24 * e):
-        out = _abi.grouped_swiglu(x[:total], counts, offsets, *packed, e, scales=tuple(scales))
-        got.append([torch.cat([o[lo[i] : lo[i] + n] for i, n in enumerate(rows)]) for o in out])
+    got, variants = [], []
+    for pairs in (3 * e, 5 * e, lo[-1], 0):
+        def run():
+            out = _abi.grouped_swiglu(x, counts, offsets, *packed, e, scales=tuple(scales), pairs=pairs)
+            got.append([torch.cat([o[lo[i] : lo[i] + n] for i, n in enumerate(rows)]) for o in out])
+        variants.append([n.split("<")[1] for n in launched(run) if n.startswith("glu_gemm_fp8w_kernel")])
+    assert 8 * e < lo[-1] <= 23 * e  # (0: what such buffers hold besides padding to 16 may be few rows)
+    up, down = (4 if d >= 512 else 2), (4 if f >= 512 else 2)  # waves along K
+    groups = (1, 2, 2, 2) if d >= 512 else (1, 1, 1, 1)
+    assert variants == [[f"true, {up}, {c}, {fr}, false>", f"false, {down}, {4 if f >= 512 else 2}, {fr}, false>"]
+                        for c, fr in zip(groups, (1, 1, 2, 1))]
     assert all(torch.equal(a, b) for o in got[1:] for a, b in zip(o, got[0]))
     for i, n in enumerate(rows):
         if n == 0:
