@@ -743,55 +743,101 @@ def test_f32_products_are_the_same_on_every_tile_size(gpu_device, k, n, layout):
     assert torch.equal(dense[0], dense[2][:32]) and torch.equal(dense[1], dense[2][:33])
 
 
-# Weights of more than half of the last-level cache are loaded past the caches where one block reads them (128 experts),
-# others through them (the first 8 of these experts alone): the same bits from every kernel that has both kinds of loads,
-# with K and N of whole units and lines, K off the units, and N off the lines.
+# Weights of more than 320 MB are loaded past the caches where one block reads them (all experts), others through them (the
+# first 8 of these experts alone): the same bits from every kernel that has both kinds of loads.  Which kernels a call
+# takes, and which loads, is asked for: where "past the caches" stands among their template arguments, by name.
+_PAST = {"glu_gemv_bf16_kernel": 2, "glu_gemv16_bf16_kernel": 2, "glu_gemm_half_kernel": 6, "glu_gemm_bf16_dma_kernel": 6,
+         "glu_gemm_fp8w_kernel": 4, "glu_gemm_mx_kernel": 1}
+
+
+class _PastTheCaches:
+    def __init__(self, many, few, device):
+        self.many, self.few, self.device, self.seen = many, few, device, set()
+
+    def both(self, rows, total, run, everywhere=True):
+        """``run(counts, offsets, experts, total)`` with all experts and with the first few: the same bits; past the
+        caches with all of them (in every kernel, or in one) and never with a few."""
+        out = []
+        for e in (self.many, self.few):
+            counts = torch.tensor(rows + [0] * (e - len(rows)), dtype=torch.int32, device=self.device)
+            offsets = torch.zeros(e + 1, dtype=torch.int32, device=self.device)
+            offsets[1:] = torch.cumsum((counts + 15) // 16 * 16, 0)
+            lo, got = offsets.tolist(), []
+            assert lo[-1] <= total
+            names = [n.rstrip(">").split("<") for n in launched(lambda: got.extend(run(counts, offsets, e, total)))]
+            loads = [(n, a.split(", ")) for n, a in (m for m in names if m[0] in _PAST)]
+            past = [a[_PAST[n]] == "true" for n, a in loads]
+            assert past and ((all if everywhere else any)(past) if e == self.many else not any(past)), (e, loads)
+            self.seen |= {(n, ", ".join(a[2:4]) if n == "glu_gemm_half_kernel" else a[0]) for (n, a), p in zip(loads, past) if p}
+            out.append([torch.cat([o[lo[i] : lo[i] + n] for i, n in enumerate(rows)]) for o in got])
+        assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
+# K and N of whole units and lines, K off the units, and N off the lines (whose weights go through the caches)
 @pytest.mark.parametrize("d,f", [(1024, 512), (1000, 512), (1024, 520)])
 def test_weights_past_the_caches_give_the_same_bits(gpu_device, d, f):
     _say("past the caches", d, f)
     many, few, dev, bf = 128, 8, gpu_device, torch.bfloat16
-    assert 3 * d * f * 2 * few < 2**27 < 3 * d * f * 2 * 100
+    assert 3 * d * f * 2 * few < 320 << 20 < 3 * d * f * 2 * many
     g = torch.Generator(dev).manual_seed(d + f)
     rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(bf)
-    x, mid = rnd(5632, d), rnd(5632, f)
+    x, mid = rnd(100 * many, d), rnd(102 * many, f)
     wg, wu, wd = rnd(many * d, f) * 0.05, rnd(many * d, f) * 0.05, rnd(many * f, d) * 0.05
-
-    def both(rows, total, run):
-        """``run(counts, offsets, experts, total)`` with all experts and with the first few."""
-        out = []
-        for e in (many, few):
-            counts = torch.tensor(rows + [0] * (e - few), dtype=torch.int32, device=dev)
-            offsets = torch.zeros(e + 1, dtype=torch.int32, device=dev)
-            offsets[1:] = torch.cumsum((counts + 15) // 16 * 16, 0)
-            lo = offsets.tolist()
-            got = run(counts, offsets, e, total)
-            out.append([torch.cat([o[lo[i] : lo[i] + n] for i, n in enumerate(rows)]) for o in got])
-        assert all(torch.equal(a, b) for a, b in zip(*out))
-        return out[0]
-
+    check, whole = _PastTheCaches(many, few, dev), d % 64 == 0 and f % 64 == 0
     w = lambda e: (wg[: e * d], wu[: e * d], wd[: e * f])
-    swiglu = lambda total, **kw: lambda c, o, e, t: _abi.grouped_swiglu(x[:t], c, o, *w(e), e, **kw)
-    for bound, rows in ((1, [1] * 8), (2, [2, 1, 2, 0, 2, 2, 2, 2]), (4, [4, 1, 3, 4, 4, 2, 4, 4]),
-                        (8, [8, 1, 5, 0, 7, 8, 8, 3]), (16, [16, 9, 1, 0, 12, 16, 5, 16])):
-        both(rows, 128, swiglu(128, rows_per_expert=bound))
+    swiglu = lambda **kw: lambda c, o, e, t: _abi.grouped_swiglu(x[:t], c, o, *w(e), e, **kw)
+    if whole:
+        for bound, rows in ((1, [1] * 8), (2, [2, 1, 2, 0, 2, 2, 2, 2]), (4, [4, 1, 3, 4, 4, 2, 4, 4]),
+                            (8, [8, 1, 5, 0, 7, 8, 8, 3]), (16, [16, 9, 1, 0, 12, 16, 5, 16])):
+            check.both(rows, 128, swiglu(rows_per_expert=bound))
     rows = [300, 17, 0, 256, 257, 129, 1, 64]
-    total = sum((n + 15) // 16 * 16 for n in rows)
-    both(rows, total, swiglu(total))
-    if _abi.keeps_products(d, f, total, bf):
-        both(rows, total, lambda c, o, e, t: _abi.grouped_swiglu_keep(x[:t], c, o, *w(e), e))
-        both(rows, total, lambda c, o, e, t: [_abi.grouped_gemm_sum(mid[:t], w(e)[0], mid[1000 : 1000 + t], w(e)[1], c, o, e)])
-    both(rows, total, lambda c, o, e, t: [_abi.grouped_gemm(x[:t], w(e)[2], _abi.W_OUT_IN, c, o, e)])
-    if d % 64 or f % 64:
-        return
-    packed = [_abi.pack_fp8_weights(t.to(torch.float8_e4m3fn), many) for t in (wg, wu, wd)]
+    # buffers that may hold 32 rows besides padding, of a few rows an expert (small tiles), and of more (large ones)
+    for total in (32 + 15 * many, 100 * many):
+        check.both(rows, total, swiglu(), whole)
+        if _abi.keeps_products(d, f, total, bf):
+            check.both(rows, total, lambda c, o, e, t: _abi.grouped_swiglu_keep(x[:t], c, o, *w(e), e), whole)
+            check.both(rows, total, lambda c, o, e, t: [
+                _abi.grouped_gemm_sum(mid[:t], w(e)[0], mid[200 : 200 + t], w(e)[1], c, o, e)], whole)
+        if d % 64 == 0:
+            check.both(rows, total, lambda c, o, e, t: [_abi.grouped_gemm(x[:t], w(e)[2], _abi.W_OUT_IN, c, o, e)], whole)
+    # (small tiles: two products, and the matrices' orientation)
+    single = {("glu_gemm_half_kernel", "false, 0"), ("glu_gemm_bf16_dma_kernel", "false")}
+    dual = {("glu_gemm_half_kernel", "true, 0"), ("glu_gemm_bf16_dma_kernel", "true")}
+    streams = {(n, two) for n in ("glu_gemv_bf16_kernel", "glu_gemv16_bf16_kernel") for two in ("true", "false")}
+    assert check.seen >= (single | dual | streams | {("glu_gemm_half_kernel", "false, 1")} if whole else
+                          single if f % 64 else dual), check.seen
+
+
+# The same of e4m3 weights, with rows of bf16 and block-scaled ones: many experts, whose launches take the stream and large
+# tiles, and fewer with a long K, whose gate/up takes small ones.
+@pytest.mark.parametrize("many,d,f", [(128, 2048, 768), (32, 9216, 384)])
+def test_e4m3_weights_past_the_caches_give_the_same_bits(gpu_device, many, d, f):
+    _say("e4m3 past the caches", many, d, f)
+    few, dev, bf = 8, gpu_device, torch.bfloat16
+    assert 3 * d * f * few < 320 << 20 < 3 * d * f * many
+    g = torch.Generator(dev).manual_seed(d + f)
+    codes = lambda k, n: (torch.randn(many * k, n, generator=g, device=dev) * 0.05).to(torch.float8_e4m3fn)
+    packed = [_abi.pack_fp8_weights(codes(k, n), many) for k, n in ((d, f), (d, f), (f, d))]
     scales = [torch.rand(many, n, generator=g, device=dev) + 0.5 for n in (f, f, d)]
-    both([16, 17, 1, 0, 33, 2, 9, 16], 160, lambda c, o, e, t: _abi.grouped_swiglu(
-        x[:t], c, o, *(q[:e] for q in packed), e, scales=tuple(s[:e] for s in scales)))
-    both(rows, 5632, lambda c, o, e, t: _abi.grouped_swiglu(
-        x[:t], c, o, *(q[:e] for q in packed), e, scales=tuple(s[:e] for s in scales)))
-    xq, xs = _abi.mx_quantize(x[:total].contiguous())
-    both(rows, total, lambda c, o, e, t: _abi.grouped_swiglu_w8a8(
-        xq, xs, c, o, *(q[:e] for q in packed), tuple(s[:e] for s in scales), e)[:2])
+    w = lambda e: dict(scales=tuple(s[:e] for s in scales))
+    x = torch.randn(5632, d, generator=g, device=dev).to(bf)
+    check = _PastTheCaches(many, few, dev)
+    swiglu = lambda pairs: lambda c, o, e, t: _abi.grouped_swiglu(
+        x[:t], c, o, *(q[:e] for q in packed), e, pairs=pairs(e), **w(e))
+    if many == 128:
+        for pairs in (96, 480):  # pieces of one and of two groups of channels
+            check.both([16, 17, 1, 0, 33, 2, 9, 16], 480, swiglu(lambda e: min(pairs, 26 * e)))
+        rows, mx_total = [300, 17, 0, 256, 257, 129, 1, 64], 44 * many
+    else:
+        rows, mx_total = [60, 17, 0, 100, 64, 129, 1, 65], 31 * many
+    check.both(rows, 27 * many + 600, swiglu(lambda e: 27 * many))
+    xq, xs = _abi.mx_quantize(x[:mx_total].contiguous())
+    check.both(rows, mx_total, lambda c, o, e, t: _abi.grouped_swiglu_w8a8(
+        xq, xs, c, o, *(q[:e] for q in packed), w(e)["scales"], e)[:2])
+    duals = lambda *names: {(n, dual) for n in names for dual in ("true", "false")}
+    assert check.seen >= (duals("glu_gemm_fp8w_kernel", "glu_gemm_bf16_dma_kernel", "glu_gemm_mx_kernel") if many == 128 else
+                          {("glu_gemm_half_kernel", "true, 2"), ("glu_gemm_half_kernel", "true, 3"),
+                           ("glu_gemm_bf16_dma_kernel", "false"), ("glu_gemm_mx_kernel", "false")}), check.seen
 
 
 # The shared expert's weights are loaded past the caches where their rows begin on lines: off them a line is read twice.
