@@ -1219,8 +1219,7 @@ static int launch_wgrad_reduce(const float* partial, int segments, int64_t n, in
   return check_launch("wgrad_reduce");
 }
 
-// One launch for all gradients of `jobs`; the grouped ones share counts and offsets.
-// The f32 gradients of one call.
+// The f32 gradients of one call, in one launch.
 static int launch_wgrad_f32(F32WgradJobs& jobs, const int32_t* a_map, const int32_t* counts, const int32_t* offsets, int E,
                             hipStream_t st) {
   int64_t blocks = 0;
@@ -1237,6 +1236,8 @@ static int launch_wgrad_f32(F32WgradJobs& jobs, const int32_t* a_map, const int3
   hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(f32t::threads(1)), 0, st, jobs, a_map, g);
   return check_launch("grouped_wgrad");
 }
+
+// One launch for all gradients of `jobs`; the grouped ones share counts and offsets.
 static int launch_wgrad(const WgradJobs& jobs, const int32_t* row_map, const int32_t* counts,
                         const int32_t* offsets, int E, hipStream_t st) {
   for (int i = 0; i < jobs.n; ++i) {

@@ -343,9 +343,9 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
   //                                 28,  29    45,  45    65,  62    81,  81   120, 124   155, 166   196, 205
   const bool off_lines =
       off_lines_variant(DUAL, BLAYOUT, TWO_SRC, CAN_TAIL) && N % 64 != 0 && (KEEP_GU || K <= 1536);
-  // Weights past the caches where most tiles are their expert's only row block, by the mean of the experts' rows.  (By
-  // the expert, as the kernels do that load straight to LDS, it costs more than it gives: two kinds of loads into the
-  // same registers meet behind a branch, where the compiler waits for all of them.)  us without and with, experts loaded
+  // Weights past the caches where most tiles are their expert's only row block, by the mean of the experts' rows: a
+  // choice for the launch, as in all kernels.  (By the expert, within the kernel, it costs more than it gives: two kinds
+  // of loads into the same registers meet behind a branch, where the compiler waits for all of them.)  us without and with, experts loaded
   // evenly and by a popularity law of exponent 1.2; forward passes, then training steps with these rows on average:
   //   128 of D 2048, F 768    3  222, 204  102, 97    32  246, 227  181, 177    94  274, 257  259, 260
   //                         128  294, 283  319, 319  188  344, 336  393, 401   256  457, 475  456, 465
@@ -356,8 +356,8 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
   const bool once =
       g.once_past_cache && mean_rows <= (KEEP_GU || BLAYOUT == FS2MOE_W_OUT_IN ? kOnceRowsTraining : kOnceRows);
   const bool units = K % (2 * BK) == 0 && !off_lines;
-  hipLaunchKernelGGL(once ? (units ? whole_once : tail_once) : (units ? whole : tail), dim3((unsigned)num_blocks), dim3(NWAVES * 64),
-                     SMEM_BYTES, stream, static_cast<const uint16_t*>(a), row_map, K,
+  hipLaunchKernelGGL(once ? (units ? whole_once : tail_once) : (units ? whole : tail), dim3((unsigned)num_blocks),
+                     dim3(NWAVES * 64), SMEM_BYTES, stream, static_cast<const uint16_t*>(a), row_map, K,
                      static_cast<const uint16_t*>(b0), static_cast<const uint16_t*>(b1),
                      static_cast<const float*>(s0), static_cast<const float*>(s1),
                      static_cast<uint16_t*>(c), N, K, N, g, nt);
@@ -898,7 +898,8 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
     };
     if ((g.planned > 0 ? pairs : max_rows - 15ll * E) > 8ll * E)
       return pair(std::integral_constant<int, 2>{}, std::false_type{});
-    if (g.planned > 0 && weights_past_cache(E, pairs, D, F, 1)) return pair(std::integral_constant<int, 1>{}, std::true_type{});
+    if (g.planned > 0 && weights_past_cache(E, pairs, D, F, 1))
+      return pair(std::integral_constant<int, 1>{}, std::true_type{});
     return pair(std::integral_constant<int, 1>{}, std::false_type{});
   }
   if (w_dtype != act_dtype) {

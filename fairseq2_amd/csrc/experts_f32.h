@@ -52,10 +52,22 @@ constexpr int threads(int groups) { return 256 * groups; }
 //   8 of 1024, N 2048, K 2048                                  597, 651; 1164, 1169
 //   16 of 500, D 768, F 1536, the layer                        521, 539
 //   128 of 256, D 1024, F 1024                                 1896, 1971
-// rows: the experts' rows, half of a last row block each.  One round of large tiles leaves a SIMD one wave, and few rounds of experts' tiles are as uneven as their loads:
-// 8 of 187 rows, D 1024, F 2048, the layer 227, 224 loaded evenly and 227, 256 by a popularity law.
-// (The weight gradients' tiles are small ones: 16 of 12 rows, 768 x 1024 44 us for the three of a step, 52 on large
-// ones; 128 of 256, 1024 x 1024 1755, 1777.)
+// rows: the experts' rows, half of a last row block each.  One round of large tiles leaves a SIMD one wave, and few rounds
+// of experts' tiles are as uneven as their loads: 8 of 187 rows, D 1024, F 2048, the layer 227, 224 loaded evenly and 227,
+// 256 by a popularity law.
+// The weight gradients' tiles are small ones.  Large ones give a step up to 2.5 % where their rounds are many and full
+// (with the largest experts first, and one gradient up to 15 % by a skewed load) and cost up to 8 % elsewhere; no size
+// tells these apart from the load.  us on small and on large tiles, of one gradient and of whole training steps:
+//   8192 rows, 2048 x 4096                999, 990       8 experts of 512            554, 548, by a law of 1.2 527, 541
+//   8192 rows, 1024 x 2048                277, 510       16 of 500, 1024 x 2048      262, 267                  315, 275
+//   64 of 256, 1024 x 1024                296, 304; 331, 407 by a law      32 of 100, 2048 x 2048  319, 381
+//   4096 tokens, top-2 of 8, D 1024, F 2048      2615, 2588; by a law of 1.2 2698, 2736
+//   4096, top-4 of 64, D 1024, F 1024            2902, 2862                  2923, 2961
+//   4096, top-4 of 32, D 1024, F 2048            by laws of 1.1, three of them 5952, 5808; 5827, 5800; 5871, 5819
+//   4096, top-8 of 128, D 1024, F 768            4376, 4351; 4633, 4625; 4657, 4644; 4666, 4623
+//   4000, top-2 of 16, D 1024, F 2048            by the law 2994, 3038; 2931, 2948; 2934, 3005
+//   1500, top-1 of 8, D 1024, F 2048             by the law 663, 715
+//   1000, top-2 of 8, D 512, F 1408              365, 385
 inline bool large_tiles(bool dual, int64_t rows, int groups, int N, int cus) {
   const int64_t real = groups > 0 && rows > 15ll * groups ? rows - 15ll * groups : rows;  // (less the blocks' padding)
   const int g = groups > 0 ? groups : 1;

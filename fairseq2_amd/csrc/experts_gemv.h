@@ -131,7 +131,8 @@ __global__ __launch_bounds__(gemv::threads(R)) void glu_gemv_bf16_kernel(
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int m = 0; m < M; ++m) wv[set][m][j] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc[m], at, j * N * 2, NT ? kNonTemporal : 0);
+      for (int m = 0; m < M; ++m)
+        wv[set][m][j] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc[m], at, j * N * 2, NT ? kNonTemporal : 0);
     at += (uint32_t)KSTEP * (uint32_t)N * 2u;
   };
   const int steps = (K + KSTEP - 1) / KSTEP;

@@ -309,9 +309,11 @@ __global__ __launch_bounds__(mx::NWAVES * 64) void glu_gemm_mx_kernel(
 #pragma unroll
       for (int jj = 0; jj < 8; ++jj) {
         if (DUAL && jj >= 4)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(bu, (lds_ptr)(base + A_BYTES + (q + 4 * jj) * 1024), 16, pb[jj], koff_w, 0, WEIGHTS);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(bu, (lds_ptr)(base + A_BYTES + (q + 4 * jj) * 1024), 16, pb[jj], koff_w,
+                                                   0, WEIGHTS);
         else
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(bg, (lds_ptr)(base + A_BYTES + (q + 4 * jj) * 1024), 16, pb[jj], koff_w, 0, WEIGHTS);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(bg, (lds_ptr)(base + A_BYTES + (q + 4 * jj) * 1024), 16, pb[jj], koff_w,
+                                                   0, WEIGHTS);
       }
       if (ku == 0) s_wscale[((ld_tiles - 1) & 1) * BNV + 64 * q + lane] = ld_scale;
     };

@@ -13,15 +13,25 @@ struct Groups {
   // host: the planned rows (common.h) where the caller knows them, else 0 and the buffers' size stands for them; the
   // choice of tiles goes by them, while grids and addresses go by the buffers
   int planned = 0;
-  // whether weights that one tile alone reads are loaded past the caches (load_once)
+  // host: whether the launch may load its weights past the caches (load_once); it does where few rows an expert make
+  // most tiles their expert's only row block
   int once_past_cache = 0;
   int64_t rows_to_plan(int64_t bound) const { return counts != nullptr && planned > 0 ? planned : bound; }
 };
 
-// Whether the weights that a call's `pairs` rows can reach are more than the last-level cache (256 MB) holds: what is read
-// once is then loaded past the caches, where otherwise some of it may still lie there from the call before.  D 2048,
-// F 768, 128 experts, top-8 (9.4 MB an expert), us of the layer without and with the hint: one token (75 MB) 36.1, 40.1
-// where its experts' weights are in that cache, 42.1, 41.2 where they are not; 8 tokens (at most 604 MB) 79.6, 75.2.
+// Whether the weights that a call's `pairs` rows can reach, each row an expert of its own, are more than the last-level
+// cache (256 MB) holds: what is read once is then loaded past the caches, where otherwise some of it may still lie there
+// from the call before.  A skewed load reaches fewer, and its weights may fit: that costs a call 3 % whose own weights
+// still lie there, and gives 17 % to one with other layers' calls in between.  D 2048, F 768, 128 experts, top-8 (9.4 MB an
+// expert), us of the layer under a graph without and with the hint, on the same input again, on 24 inputs in turn, and with
+// 1.3 GB of other memory read and written in between:
+//   1 token (75 MB at most)                                44.1, 46.8    48.2, 47.8    61.2, 55.3
+//   4, by a popularity law (302 MB at most)                59.9, 61.2    63.2, 64.4    83.0, 69.4
+//   8 by one (604 at most, 210)                            71.2, 73.5    72.0, 73.9    98.7, 81.4
+//   8 evenly (470)                                        140.0, 128.7  139.2, 129.1  170.0, 135.8
+//   16 by a law                                            80.6, 80.7    80.4, 81.0   110.5, 87.2
+// 64 tokens by a law with e4m3 weights (without a graph)   63.3, 67.5    62.0, 67.1    82.7, 71.1
+// (What fits even so, up to 320 MB, is left in the caches: a program of one layer.)
 // Whole layers of 262 MB, by a popularity law, which leaves some experts out: 60 of D 704, F 1088, 720 tokens 66.0, 69.5;
 // of 288 MB 62.9, 64.5 (128 of D 768, F 512), 86.8, 84.3 (64 of D 1024, F 768); of 432 MB 125, 121.  One group, the
 // shared expert, counts for more: the routed ones' weights go by beside it.

@@ -67,7 +67,10 @@ __global__ __launch_bounds__(256) void gather_backward_kernel(
 // whose right one is the unweighted output gradient), dg and du, and from the forward pass' h the combine
 // weight's gradient d_w[p] = <ye[r], dout[t]> = <h[r], dh[r]>, which so needs neither ye nor dout.  (With an
 // h from the rounded g and u the router's gradient is 15% further from 64 bits: three roundings instead of
-// two.)  Bound by memory: seven passes over [rows, F].  h may be dh's buffer.
+// two.)  Bound by memory: seven passes over [rows, F].  h may be dh's buffer.  What the forward pass kept is read here for
+// the last time, past the caches (load_once), which changes little: us of a training step without and with the hint, 260
+// tokens, top-1 of 8, F 6400 243, 243; 2048, top-4 of 32, F 512 237, 237; 4096, top-8 of 128, F 768 1514, 1513; 8000,
+// top-2 of 16, F 1024 357, 353; 700, top-2 of 8, F 8192 1350, 1357.
 __global__ __launch_bounds__(256) void swiglu_backward_pairs_kernel(
     const uint16_t* __restrict__ g, const uint16_t* __restrict__ u, const uint16_t* __restrict__ h_fwd,
     const uint16_t* dh, const int32_t* __restrict__ inv_perm, const float* __restrict__ topk_w, int pairs, int F,
