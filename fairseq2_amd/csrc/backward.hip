@@ -40,9 +40,14 @@ namespace fs2moe {
 //     XCD (block b runs on XCD b % 8) take the share's tiles in turn, so that at any time they work on
 //     neighbours, which share operand slabs in the XCD's L2 (shares of neighbours per block instead: 2170
 //     against 1750 us at 8 experts of 2048 rows, M 4096, N 14336);
-//   * larger (a few experts or one group hold most rows): the experts are sorted by their rows, the tiles
-//     above that quarter go out one per block in rounds that reverse direction, and the rest are cut into
-//     shares that fill each block up to a common level.
+//   * larger (a few experts or one group hold most rows): the tiles above that quarter go out one per block in rounds that
+//     reverse direction, those of experts with the experts sorted by their rows, and the rest fill the blocks up to a
+//     common level: each XCD gets a share as large as its blocks' room, and its blocks take the share's tiles in turn, each
+//     from the round on that its large tiles last to.  As a share of neighbours for each block, a block for itself, every
+//     tile read its operands from memory: 4096 tokens, top-8 of 128, 2048 x 768, evenly loaded with the router's gradient
+//     2.37 GB for 2.42 that the tiles take in, now 0.55.  us of that training step 1552 -> 1517, by a popularity law 1594
+//     -> 1541; 8192 tokens 2444 -> 2355 and 2516 -> 2416; 2000, top-6 of 32 by a law with a shared expert, 1600 x 1000
+//     813 -> 795.  Sorted only where experts have large tiles: in the gradients' order two operands share L2, not six.
 // The chunks of a block's tiles form one stream: while the consumers write a tile out, the producers have
 // the next one's first three chunks on their way.  (A block per tile, started by the hardware, paid about
 // 10 us around its chunks.)
@@ -88,8 +93,7 @@ struct WgradJobs {
 // (As scalar loads a chunk ahead every barrier waited for them with the LDS traffic.)  That, and a way out of a tile
 // without branches and waits around its stores, us of the gradients of a training step: 4096 tokens, top-8 of 128
 // skewed, 2048 x 768 648 -> 617; top-6 of 64, 2048 x 1024 465 -> 449; 2000, top-4 of 60 skewed, 1024 x 1408 181 -> 173;
-// 300 of the first 246 -> 236; 4096 evenly, top-8 of 128 554 -> 553, which memory bounds (2.3 GB; 478 without the
-// products, 420 without memory).
+// 300 of the first 246 -> 236; 4096 evenly, top-8 of 128 554 -> 553 (where memory then bound them, see the deal above).
 // The map holds at least one entry, and one for every row of a gradient in the same launch that does not use it.
 template <bool MAPPED>
 __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
@@ -224,38 +228,44 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     const int64_t t = divide(2 * x + cost - 1, 2 * (int64_t)cost);
     return tiles + (int)(t < tiles_of ? t : tiles_of);
   };
-  // The block's tiles: `rounds` of one of the first `big` tiles each, then first, first + stride, ..
+  // The block's tiles: `rounds` of one of the first `big` tiles each, then its XCD's tiles [next_t, end) in turn with the
+  // XCD's other blocks: in rounds of one tile each, of which block i misses the first skip_i.  Of the tiles that go out
+  // before the block's round n those of lane i's block are max(0, n + ahead).
   struct Deal {
-    int slot, grid, rounds, big, round, next_t, end, stride;
+    int slot, grid, rounds, big, round, next_t, end, turn, ahead;
     __device__ int next() {  // -1: no more
       while (round < rounds) {
         const int r = round++, p = r * grid + ((r & 1) ? grid - 1 - slot : slot);
         if (p < big) return p;
       }
-      if (next_t >= end) return -1;
-      const int t = next_t;
-      next_t += stride;
-      return t;
+      const int of_lane = turn + ahead, t = next_t + wave_sum_i32(of_lane > 0 ? of_lane : 0);
+      ++turn;
+      return t < end ? t : -1;
     }
   };
   Deal deal;
   deal.grid = (int)gridDim.x;
   const int xcd = blockIdx.x & 7;
   deal.slot = xcd * (deal.grid >> 3) + (int)(blockIdx.x >> 3);
-  deal.round = deal.rounds = deal.big = 0;
+  deal.round = deal.rounds = deal.big = deal.turn = 0;
+  // (nothing skipped: the blocks before this one are a tile ahead; lanes without a block never count)
+  constexpr int NEVER = -(1 << 29);
+  const int xcd_blocks = deal.grid >> 3, rank = (int)(blockIdx.x >> 3);
+  deal.ahead = lane < xcd_blocks ? (lane < rank ? 1 : 0) : NEVER;
   const int64_t fair = divide(total, deal.grid);
   if (dense + (int64_t)E * per <= deal.grid) {
     deal.big = dense + E * per;  // at most one tile each
     deal.rounds = 1;
     deal.next_t = deal.end = 0;
-    deal.stride = 1;
   } else if (most * 4ll <= fair) {
-    deal.next_t = tiles_before(total * xcd / 8) + (int)(blockIdx.x >> 3);
+    deal.next_t = tiles_before(total * xcd / 8);
     deal.end = tiles_before(total * (xcd + 1) / 8);
-    deal.stride = deal.grid >> 3;
   } else {
-    by_expert = true;
-    if (per > 0) {
+    int expert_most = 0;
+    for (int w = 0; per > 0 && w < WAVES; ++w) expert_most = s_wave_max[w] > expert_most ? s_wave_max[w] : expert_most;
+    // (where only the gradients of one group have large tiles, the others stay in the order that shares operands best)
+    by_expert = expert_most * 4ll > fair;
+    if (by_expert) {
       // sort the experts by their rows, largest first (ties: lower index first)
       int rank = 0;
       for (int j = 0; j < E; ++j) {
@@ -268,7 +278,7 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
     // the large tiles: all of one group (as large as any expert's, mostly), and the experts whose tiles
     // are above a quarter of the fair share
     int large = 0;
-    if (per > 0) {
+    if (by_expert) {
       for (int e0 = 0; e0 < E; e0 += 64) {
         const int e = e0 + lane;
         large += __popcll(__ballot(e < E && (s_pre[e + 1] - s_pre[e]) * 4ll > fair));
@@ -324,17 +334,56 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
       below = n;
       level = (int)divide(rest + wave_sum_i32(sum) + n - 1, n);
     }
-    int mine = 0, before = 0;  // room of this lane's slots, and of those before this block's
+    // the XCD's part of it: the room of its blocks behind that of the XCDs before
+    const int first_slot = xcd * xcd_blocks;
+    int mine = 0, before = 0;
 #pragma unroll
     for (int i = 0; i < PL; ++i) {
-      const int r = load[i] <= level ? level - load[i] : 0;
-      if (PL * lane + i < deal.slot) before += r;
-      if (PL * lane + i == deal.slot) mine = r;
+      const int r = load[i] <= level ? level - load[i] : 0, sl = PL * lane + i;
+      if (sl < first_slot) before += r;
+      if (sl >= first_slot && sl < first_slot + xcd_blocks) mine += r;
     }
-    const int64_t from = wave_sum_i32(before), to = from + wave_sum_i32(mine);
-    deal.next_t = tiles_before(big_cost + (from < rest ? from : rest));
+    const int64_t from = wave_sum_i32(before), room = wave_sum_i32(mine), to = from + room;
+    const int64_t first_cost = big_cost + (from < rest ? from : rest);
+    deal.next_t = tiles_before(first_cost);
     deal.end = tiles_before(big_cost + (to < rest ? to : rest));
-    deal.stride = 1;
+    // A block joins the XCD's rounds when the others have been filled to its load: as many rounds as tiles of that cost
+    // lie at the share's beginning, for the number of blocks that take part on average.
+    const int my_load = lane < xcd_blocks ? s_cap[first_slot + lane] : 0x7fffffff;
+    const int least = -(int)wave_max_u32((uint32_t)(0x7fffffff - my_load)) + 0x7fffffff, height = level - least;
+    const int part = height > 0 ? (int)divide(room + height - 1, height) : 0;  // blocks
+    int skip = 0;
+    if (my_load >= level) {
+      skip = -NEVER;
+    } else if (per > 0 && my_load > least) {
+      int64_t y = first_cost - dense_cost + (int64_t)part * (my_load - least);
+      int tiles = dense, tiles_of = per;
+      if (!by_expert)
+        for (int i = 0; i < jobs.n; ++i) {
+          const WgradJob& j = jobs.job[i];
+          if (!j.grouped) continue;
+          tiles_of = j.tiles;
+          const int64_t all = (int64_t)s_pre[E] * tiles_of;
+          if (y < all) break;
+          y -= all;
+          tiles += E * tiles_of;
+        }
+      int lo = 0, hi = E;  // the expert of cost y
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if ((int64_t)s_pre[mid] * tiles_of <= y) lo = mid;
+        else hi = mid;
+      }
+      const int64_t in = y - (int64_t)s_pre[lo] * tiles_of;
+      tiles += lo * tiles_of + (int)divide(in, s_pre[lo + 1] - s_pre[lo]) - deal.next_t;
+      skip = tiles > 0 ? (2 * tiles + part) / (2 * part) : 0;
+    }
+    if (lane < xcd_blocks) {
+      const int own = __builtin_amdgcn_readlane(skip, rank);
+      deal.ahead = skip == -NEVER || own == -NEVER ? NEVER : own - skip + (lane < rank ? 1 : 0);
+      if (own == -NEVER) deal.end = deal.next_t;
+    }
+    deal.end = __builtin_amdgcn_readfirstlane(deal.end);
   }
   deal.next_t = __builtin_amdgcn_readfirstlane(deal.next_t);
   deal.end = __builtin_amdgcn_readfirstlane(deal.end);
@@ -342,7 +391,6 @@ __global__ __launch_bounds__(wgk::WAVES * 64) void grouped_wgrad_kernel(
   // over tiles and chunks would be masked ones, whose paths meet where nothing can be known of the loads)
   deal.rounds = __builtin_amdgcn_readfirstlane(deal.rounds);
   deal.big = __builtin_amdgcn_readfirstlane(deal.big);
-  deal.stride = __builtin_amdgcn_readfirstlane(deal.stride);
   by_expert = __builtin_amdgcn_readfirstlane(by_expert);
 
   auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };

@@ -250,6 +250,35 @@ def test_step_in_two_calls_against_its_stages(gpu_device, dtype, t, d, e, k, f, 
     assert torch.equal(some[4], grads[4])
 
 
+# A step's weight gradients in one launch against each of them alone, whose tiles are dealt otherwise: the experts' tiles
+# behind large ones of the gradients of one group, which some blocks have (evenly loaded, in the order of the gradients);
+# the same in the order of the experts' sizes, with large ones dealt one by one; no expert with room left behind one;
+# and as many experts as there may be.
+@pytest.mark.parametrize("t,d,e,k,f,f_shared,skew", [
+    (1500, 512, 64, 4, 520, 0, 0.0), (1500, 512, 64, 4, 520, 512, 0.0), (1500, 512, 64, 4, 520, 0, 2.0),
+    (2500, 520, 60, 4, 256, 264, 1.2), (3000, 264, 2, 1, 264, 1032, 3.0), (1200, 264, 512, 2, 264, 0, 1.0),
+])
+def test_weight_gradients_whatever_is_dealt_with_them(gpu_device, t, d, e, k, f, f_shared, skew):
+    from fairseq2_amd import autograd as A
+
+    _say("dealt together", t, d, e, k, f, f_shared, skew)
+    g = torch.Generator().manual_seed(t + e)
+    mk = lambda *s, scale=1.0: (scale * torch.randn(*s, generator=g)).to(torch.bfloat16).to(gpu_device)  # noqa: E731
+    x, dout, router = mk(t, d), mk(t, d), mk(d, e, scale=d**-0.5)
+    ws = [mk(e * d, f, scale=d**-0.5), mk(e * d, f, scale=d**-0.5), mk(e * f, d, scale=f**-0.5)]
+    ws += [mk(f_shared, d, scale=d**-0.5), mk(f_shared, d, scale=d**-0.5), mk(d, f_shared, scale=f_shared**-0.5)] \
+        if f_shared else [None] * 3
+    bias = (-skew * torch.log(1.0 + torch.arange(e))).to(gpu_device) if skew else None
+    cfg = dict(num_experts=e, top_k=k, tile_m=16, score_fn=_abi.SCORE_SOFTMAX, renormalize=False, scale_input=False,
+               router_bias=bias, norm_eps=None)
+    _, saved = A.layer_forward(x, None, router, *ws, None, cfg)
+    together = A.layer_backward(x, router, *ws, None, cfg, saved, dout, (True,) * 9)
+    for i in (2, 3, 4):
+        wants = tuple(j == i for j in range(9))
+        alone = A.layer_backward(x, router, *ws, None, cfg, saved, dout, wants)[i]
+        assert torch.equal(together[i], alone), i
+
+
 # Sizes at which a count of rows with their padding would cut the rows' gradients, or the router's and the shared
 # expert's weight gradients, into another number of parts.
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
