@@ -214,6 +214,18 @@ inline int cu_count_by_xcd() {
 
 inline int elem_size(int dtype) { return dtype == FS2MOE_F32 ? 4 : dtype == FS2MOE_BF16 ? 2 : 1; }
 
+// What is left of router and dispatch where the experts' first kernel does it itself (swiglu_selects): the partial logits
+// [slices][T][E], and where its results go.
+struct Selection {
+  const float *partial, *bias;
+  int slices, T, K, score_fn, renormalize, tile_m;
+  int64_t max_rows;
+  int32_t* topk_idx;
+  float* topk_w;
+  int32_t *counts, *offsets, *perm, *inv_perm;
+  float* row_w;
+};
+
 // Where the whole-layer call wants its dispatch (no rows copied): with at most 32 bf16 tokens the
 // router's finishing kernel ends with it; with more the finishing kernel, or the block that routes a
 // whole tile of 32 tokens from an (E, D) matrix, also counts its tile's pairs per expert and ranks them
@@ -229,6 +241,9 @@ struct DispatchAfterRouter {
   // optional (bf16 decode sizes, rows scaled by the routing weight on their way into the experts
   // instead of by a copy): per expert row the weight of its pair, written next to perm
   float* row_w;
+  // optional: may take the selection instead (partial is set then) where the router leaves partial logits of at most
+  // kRouterTileTok tokens and is not asked for logits; `done` is set as well
+  Selection* later;
   bool done;
 };
 constexpr int kRouterTileTok = 32;   // tokens per tile of the MFMA routers
@@ -287,6 +302,12 @@ bool swiglu_gathers_rows(int32_t act_dtype, int32_t w_dtype, int32_t D, int32_t 
 // multiplied by row_w[row] (rounded to bf16, as dispatch's scaled copy rounds them).
 bool swiglu_streams_rows(int32_t act_dtype, int32_t w_dtype, int32_t D, int32_t F, int32_t E,
                          int32_t rows_per_expert);
+// Whether the pair may begin with the selection itself (grouped_swiglu_selecting): up to 16 tokens on these kernels, with room
+// for its tables in LDS; and that pair, whose rows are those of `sel`, read from x.
+bool swiglu_selects(int32_t act_dtype, int32_t w_dtype, int32_t D, int32_t F, int32_t E, int32_t T);
+int grouped_swiglu_selecting(const void* x, const Selection& sel, const void* w_gate, const void* w_up, const void* w_down,
+                             int32_t E, int32_t D, int32_t F, int64_t max_rows, int64_t planned, void* h, void* ye,
+                             void* stream);
 int grouped_swiglu_scaled_rows(const void* x, const int32_t* row_map, const float* row_w,
                                const int32_t* counts, const int32_t* offsets, const void* w_gate,
                                const void* w_up, const void* w_down, int32_t E, int32_t D, int32_t F,

@@ -572,41 +572,54 @@ static unsigned stream_experts(int blocks, int col_blocks, int E) {
   return (unsigned)(n < E ? n : E);
 }
 
+// A kernel that begins with the selection has a block a CU (its registers allow no more), which take (expert, channel block)
+// pairs in turn, so that each selects once; and no more than there may be pairs.
+static dim3 selecting_grid(const Selection& sel, int col_blocks, int E) {
+  const int64_t pairs = (int64_t)sel.T * sel.K, most = (pairs < E ? pairs : E) * col_blocks;
+  return dim3((unsigned)(most < 256 ? most : 256));
+}
+
 template <int R, bool NT>
 static int launch_gemv_pair_r(const void* x, const int32_t* row_map, const float* row_w,
                               const Groups& g, const void* w_gate, const void* w_up,
                               const void* w_down, int D, int F, void* h, void* y,
-                              hipStream_t stream) {
+                              hipStream_t stream, const Selection* sel) {
   using namespace gemv;
   auto k1 = glu_gemv_bf16_kernel<true, R, NT>;
+  auto k1s2 = glu_gemv_bf16_kernel<true, R, NT, false, 2>;
+  auto k1s4 = glu_gemv_bf16_kernel<true, R, NT, false, 4>;
   auto k2 = glu_gemv_bf16_kernel<false, R, NT>;
   auto k2d = glu_gemv_bf16_kernel<false, R, NT, true>;  // more loads in flight over a long K
   static bool attr_set = false;  // benign race: setting the attribute is idempotent
   if (!attr_set) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(k1),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, MAX_LDS_BYTES) != hipSuccess ||
-        hipFuncSetAttribute(reinterpret_cast<const void*>(k2d),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, MAX_LDS_BYTES) != hipSuccess ||
-        hipFuncSetAttribute(reinterpret_cast<const void*>(k2),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, MAX_LDS_BYTES) != hipSuccess) {
-      set_error("experts: cannot reserve %d bytes of LDS", MAX_LDS_BYTES);
-      return FS2MOE_ERR_LAUNCH;
+    for (const void* k : {reinterpret_cast<const void*>(k1), reinterpret_cast<const void*>(k1s2),
+                          reinterpret_cast<const void*>(k1s4), reinterpret_cast<const void*>(k2),
+                          reinterpret_cast<const void*>(k2d)}) {
+      const int bytes = k == reinterpret_cast<const void*>(k1s2) || k == reinterpret_cast<const void*>(k1s4)
+                            ? MAX_LDS_SELECT : MAX_LDS_BYTES;
+      if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
+        set_error("experts: cannot reserve %d bytes of LDS", bytes);
+        return FS2MOE_ERR_LAUNCH;
+      }
     }
     attr_set = true;
   }
+  if (sel != nullptr) k1 = g.E <= 128 ? k1s2 : k1s4;
+  const Selection selection = sel != nullptr ? *sel : Selection{};
   const uint16_t* xp = static_cast<const uint16_t*>(x);
   const int f_blocks = (F + COLS - 1) / COLS, d_blocks = (D + COLS - 1) / COLS;
-  hipLaunchKernelGGL(k1, dim3((unsigned)f_blocks, stream_experts(256 * (R + 1), f_blocks, g.E)), dim3(threads(R)),
+  hipLaunchKernelGGL(k1, sel != nullptr ? selecting_grid(*sel, f_blocks, g.E)
+                                        : dim3((unsigned)f_blocks, stream_experts(256 * (R + 1), f_blocks, g.E)), dim3(threads(R)),
                      (size_t)R * D * 2, stream, xp, row_map, row_w, D, static_cast<const uint16_t*>(w_gate),
                      static_cast<const uint16_t*>(w_up), static_cast<uint16_t*>(h), F, D, F,
-                     g.counts, g.offsets, g.E);
+                     g.counts, g.offsets, g.E, selection);
   if (int rc = check_launch("glu_gemv_bf16<gate,up>")) return rc;
   hipLaunchKernelGGL(deep_applies(F, R) ? k2d : k2, dim3((unsigned)d_blocks, stream_experts(256 * (R + 1), d_blocks, g.E)),
                      dim3(threads(R)), (size_t)R * F * 2, stream, static_cast<const uint16_t*>(h),
                      static_cast<const int32_t*>(nullptr), static_cast<const float*>(nullptr), F,
                      static_cast<const uint16_t*>(w_down),
                      static_cast<const uint16_t*>(nullptr), static_cast<uint16_t*>(y), D, F, D,
-                     g.counts, g.offsets, g.E);
+                     g.counts, g.offsets, g.E, Selection{});
   return check_launch("glu_gemv_bf16<down>");
 }
 
@@ -634,33 +647,40 @@ template <int XR, bool NT>
 static int launch_gemv16_pair(const void* x, const int32_t* row_map, const float* row_w,
                               const Groups& g, const void* w_gate, const void* w_up,
                               const void* w_down, int D, int F, void* h, void* y,
-                              hipStream_t stream) {
+                              hipStream_t stream, const Selection* sel) {
   using namespace gemv16;
   auto k1 = glu_gemv16_bf16_kernel<true, XR, NT>;
+  auto k1s2 = glu_gemv16_bf16_kernel<true, XR, NT, 2>;
+  auto k1s4 = glu_gemv16_bf16_kernel<true, XR, NT, 4>;
   auto k2 = glu_gemv16_bf16_kernel<false, XR, NT>;
   static bool attr_set = false;  // benign race: setting the attribute is idempotent
   if (!attr_set) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(k1),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, MAX_LDS_BYTES) != hipSuccess ||
-        hipFuncSetAttribute(reinterpret_cast<const void*>(k2),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, MAX_LDS_BYTES) != hipSuccess) {
-      set_error("experts: cannot reserve %d bytes of LDS", MAX_LDS_BYTES);
-      return FS2MOE_ERR_LAUNCH;
+    for (const void* k : {reinterpret_cast<const void*>(k1), reinterpret_cast<const void*>(k1s2),
+                          reinterpret_cast<const void*>(k1s4), reinterpret_cast<const void*>(k2)}) {
+      const int bytes = k == reinterpret_cast<const void*>(k1s2) || k == reinterpret_cast<const void*>(k1s4)
+                            ? MAX_LDS_SELECT : MAX_LDS_BYTES;
+      if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
+        set_error("experts: cannot reserve %d bytes of LDS", bytes);
+        return FS2MOE_ERR_LAUNCH;
+      }
     }
     attr_set = true;
   }
+  if (sel != nullptr) k1 = g.E <= 128 ? k1s2 : k1s4;
+  const Selection selection = sel != nullptr ? *sel : Selection{};
   const int f_blocks = (F + COLS - 1) / COLS, d_blocks = (D + COLS - 1) / COLS;
-  hipLaunchKernelGGL(k1, dim3((unsigned)f_blocks, stream_experts(2048, f_blocks, g.E)), dim3(THREADS),
+  hipLaunchKernelGGL(k1, sel != nullptr ? selecting_grid(*sel, f_blocks, g.E)
+                                        : dim3((unsigned)f_blocks, stream_experts(2048, f_blocks, g.E)), dim3(THREADS),
                      lds_bytes(D, XR, true), stream, static_cast<const uint16_t*>(x), row_map, row_w, D,
                      static_cast<const uint16_t*>(w_gate), static_cast<const uint16_t*>(w_up),
-                     static_cast<uint16_t*>(h), F, D, F, g.counts, g.offsets, g.E);
+                     static_cast<uint16_t*>(h), F, D, F, g.counts, g.offsets, g.E, selection);
   if (int rc = check_launch("glu_gemv16_bf16<gate,up>")) return rc;
   hipLaunchKernelGGL(k2, dim3((unsigned)d_blocks, stream_experts(2048, d_blocks, g.E)), dim3(THREADS),
                      lds_bytes(F, XR, false), stream, static_cast<const uint16_t*>(h),
                      static_cast<const int32_t*>(nullptr), static_cast<const float*>(nullptr), F,
                      static_cast<const uint16_t*>(w_down),
                      static_cast<const uint16_t*>(nullptr), static_cast<uint16_t*>(y), D, F, D,
-                     g.counts, g.offsets, g.E);
+                     g.counts, g.offsets, g.E, Selection{});
   return check_launch("glu_gemv16_bf16<down>");
 }
 
@@ -690,7 +710,7 @@ template <int BLAYOUT>
 static int launch_glu(const void* x, const int32_t* row_map, const Groups& g, int64_t rows_bound,
                       const void* w_gate, const void* w_up, const void* w_down, int D, int F,
                       int act_dtype, void* h, void* y, hipStream_t stream, int rows_hint = 0,
-                      const float* row_w = nullptr) {
+                      const float* row_w = nullptr, const Selection* sel = nullptr) {
   const int groups = g.counts ? g.E : 0;
   // (rows off the lines share them with the rows beside, in both orientations: nn.Linear's of D 4096, F 8192 42.8 us
   // without and 48.1 with the hint on the same weights again, 64.6 and 53.2 with other memory read in between; of D 5160,
@@ -708,17 +728,17 @@ static int launch_glu(const void* x, const int32_t* row_map, const Groups& g, in
       auto launch = rows_hint <= 1   ? (past ? launch_gemv_pair_r<1, true> : launch_gemv_pair_r<1, false>)
                     : rows_hint <= 2 ? (past ? launch_gemv_pair_r<2, true> : launch_gemv_pair_r<2, false>)
                                      : (past ? launch_gemv_pair_r<4, true> : launch_gemv_pair_r<4, false>);
-      return launch(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream);
+      return launch(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream, sel);
     }
     if (gemv16_applies(act_dtype, D, F, g, rows_hint)) {
       auto launch = gemv16_rows(D, F, rows_hint) == 8
                         ? (past ? launch_gemv16_pair<8, true> : launch_gemv16_pair<8, false>)
                         : (past ? launch_gemv16_pair<16, true> : launch_gemv16_pair<16, false>);
-      return launch(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream);
+      return launch(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream, sel);
     }
   }
-  if (row_w != nullptr) {
-    set_error("experts: internal: row weights given to kernels that do not scale rows");
+  if (row_w != nullptr || sel != nullptr) {
+    set_error("experts: internal: row weights or a selection given to kernels that do not scale rows");
     return FS2MOE_ERR_UNSUPPORTED;
   }
   if (act_dtype == FS2MOE_BF16 && dma_offsets_fit(rows_bound, D, F))
@@ -926,6 +946,24 @@ bool fs2moe::swiglu_streams_rows(int32_t act_dtype, int32_t w_dtype, int32_t D, 
   static const int32_t some = 0;  // (the predicates only ask whether the groups have counts)
   const Groups g{&some, &some, E, 0};
   return gemv_applies(act_dtype, D, F, g, rows_per_expert) || gemv16_applies(act_dtype, D, F, g, rows_per_expert);
+}
+
+bool fs2moe::swiglu_selects(int32_t act_dtype, int32_t w_dtype, int32_t D, int32_t F, int32_t E, int32_t T) {
+  if (T < 1 || T > 16 || !swiglu_streams_rows(act_dtype, w_dtype, D, F, E, T)) return false;
+  if (T <= FS2MOE_GEMV_MAX_ROWS) return (int64_t)D * (T <= 2 ? T : 4) * 2 <= gemv::MAX_LDS_SELECT;
+  return gemv16::lds_bytes(D, gemv16_rows(D, F, T), true) <= (size_t)gemv16::MAX_LDS_SELECT;
+}
+
+int fs2moe::grouped_swiglu_selecting(const void* x, const Selection& sel, const void* w_gate, const void* w_up,
+                                     const void* w_down, int32_t E, int32_t D, int32_t F, int64_t max_rows, int64_t planned,
+                                     void* h, void* ye, void* stream) {
+  FS2_REQUIRE(swiglu_selects(FS2MOE_BF16, FS2MOE_BF16, D, F, E, sel.T),
+              "grouped_swiglu: internal: D=%d F=%d E=%d of %d tokens do not select", D, F, E, sel.T);
+  FS2_REQUIRE(aligned16(x) && aligned16(w_gate) && aligned16(w_up) && aligned16(w_down) && aligned16(h) && aligned16(ye),
+              "grouped_swiglu: buffers must be 16-byte aligned");
+  const Groups g{sel.counts, sel.offsets, E, 0, (int)planned};
+  return launch_glu<FS2MOE_W_IN_OUT>(x, sel.perm, g, max_rows, w_gate, w_up, w_down, D, F, FS2MOE_BF16, h, ye,
+                                     static_cast<hipStream_t>(stream), sel.T, sel.row_w, &sel);
 }
 
 int fs2moe::grouped_swiglu_scaled_rows(const void* x, const int32_t* row_map, const float* row_w,

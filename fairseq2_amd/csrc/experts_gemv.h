@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "router_select.h"
 
 namespace fs2moe {
 namespace gemv {
@@ -31,6 +32,7 @@ constexpr int COLS = 64;          // channels per block
 constexpr int waves(int R) { return 8; }
 constexpr int threads(int R) { return 64 * waves(R); }
 constexpr int MAX_LDS_BYTES = 144 * 1024;  // (160 KB less the kernel's own partial sums, 16 KB at most)
+constexpr int MAX_LDS_SELECT = MAX_LDS_BYTES - 6 * 1024;  // (less what a kernel that selects keeps of it)
 inline bool fits(int K, int R) { return (int64_t)K * R * 2 <= MAX_LDS_BYTES; }
 // Steps of K (256 rows a block) whose loads a wave has in flight: 4 with one or two rows, 2 with four
 // (registers).  DEEP: 8, for the single product with one or two rows over a
@@ -82,19 +84,103 @@ __device__ __forceinline__ int nth_active_expert(const int32_t* __restrict__ cou
   return e;
 }
 
+// SELECT 2 or 4 (gate/up): the kernel begins with what router_finish_tile_kernel does, for at most 16 tokens and 64 SELECT
+// experts.  Every block adds the partial logits, selects and keeps a word per expert with a bit per token in LDS, from which
+// its experts, their rows and those rows' tokens follow without a look at memory; the last block of the grid, which has the
+// least to stream, writes what the kernels behind it read.  A launch of one block is a boundary and a chain of round trips
+// while the chip waits (6 to 7 us); here it is 2 us in front of the stream, as its three look-ups (counts, offsets, tokens)
+// are gone.  Each block pays them, so there is one a CU, which takes (expert, channel block) pairs in turn: with a block for
+// every pair 4 tokens took 70 us.  us of the layer under a graph, D 2048, F 768, top-8 of 128, with the launch and without:
+//   1 token 43.7, 40.6    2 53.4, 49.7    4 63.5, 59.6    8 75.3, 72.2    12 78.3, 76.5    16 81.6, 79.7
+// 3 of D 1024, F 1408, top-4 of 60, rows scaled 47.5, 44.0; 1 of D 4096, F 14336, top-2 of 8 173.3, 169.8.
+struct Selected {
+  uint32_t bits[256];
+  float weight[16][FS2MOE_MAX_TOP_K];  // by token and slot, and their experts
+  int16_t expert[16][FS2MOE_MAX_TOP_K];
+  int32_t off[257], wave_tot[4];
+};
+template <int SELECT, int THREADS>
+__device__ __forceinline__ void select_for_block(Selected& s, const Selection& sel, int E, bool writes) {
+  constexpr int NW = THREADS / kWave, TPW = 16 / NW;
+  const int tid = threadIdx.x, lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  static_assert(64 * SELECT <= THREADS && SELECT <= 4, "a thread per expert");
+  if (tid < 64 * SELECT) s.bits[tid] = 0u;
+  __syncthreads();
+  int chosen[TPW];
+  float weight[TPW];
+#pragma unroll
+  for (int i = 0; i < TPW; ++i) {
+    const int t = wave + NW * i;
+    chosen[i] = 0;
+    weight[i] = 0.f;
+    if (t >= sel.T) continue;  // wave-uniform
+    float v[SELECT];
+    finish_logits<SELECT>(sel.partial, sel.slices, sel.bias, t, sel.T, E, v);
+    select_experts<SELECT>(v, lane, E, sel.K, sel.score_fn, sel.renormalize, chosen[i], weight[i]);
+    if (lane < sel.K) {
+      atomicOr(&s.bits[chosen[i]], 1u << t);
+      s.weight[t][lane] = weight[i];
+      s.expert[t][lane] = (int16_t)chosen[i];
+      if (writes) {
+        sel.topk_idx[(size_t)t * sel.K + lane] = chosen[i];
+        sel.topk_w[(size_t)t * sel.K + lane] = weight[i];
+      }
+    }
+  }
+  __syncthreads();
+  if (writes)
+    dispatch_finished<SELECT, THREADS, TPW>(s.bits, s.off, s.wave_tot, chosen, weight, sel.T, E, sel.K, sel.tile_m,
+                                            sel.max_rows, sel.counts, sel.offsets, sel.perm, sel.inv_perm, sel.row_w);
+}
+// The n-th expert with rows (-1: there is none) with its number of rows and its first row.
+template <int SELECT>
+__device__ __forceinline__ int nth_selected_expert(const Selected& s, int tile_m, int n, int& cnt, int& off) {
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));  // (as in nth_active_expert)
+  int e = -1, seen = 0, c[SELECT];
+#pragma unroll
+  for (int j = 0; j < SELECT; ++j) {
+    c[j] = __popc(s.bits[lane + 64 * j]);
+    const unsigned long long act = __ballot(c[j] > 0);
+    const int before = __popcll(act & ((1ull << lane) - 1ull));
+    const unsigned long long hit = __ballot(((act >> lane) & 1ull) != 0ull && seen + before == n);
+    if (e < 0 && hit != 0ull) e = 64 * j + (int)__builtin_ctzll(hit);
+    seen += __popcll(act);
+  }
+  if (e < 0) return e;
+  int rows = 0;
+#pragma unroll
+  for (int j = 0; j < SELECT; ++j) rows += lane + 64 * j < e ? (c[j] + tile_m - 1) / tile_m * tile_m : 0;
+  off = wave_sum_i32(rows);
+  cnt = __builtin_amdgcn_readfirstlane(__popc(s.bits[e]));
+  return e;
+}
+static_assert(sizeof(Selected) <= 6 * 1024, "left out of MAX_LDS_SELECT");
+// The token of the expert's r-th row, and the weight of that pair.
+__device__ __forceinline__ int selected_token(uint32_t bits, int r) {
+  for (int i = 0; i < r; ++i) bits &= bits - 1u;
+  return (int)__builtin_ctz(bits);
+}
+__device__ __forceinline__ float selected_weight(const Selected& s, int t, int e, int K) {
+  const int lane = lane_id(), k = lane < K ? lane : 0;
+  const unsigned long long hit = __ballot(s.expert[t][k] == e);
+  return s.weight[t][(int)__builtin_ctzll(hit)];
+}
+
 // DUAL: C[r, n] = SiLU(A[r] . B0[:, n]) * (A[r] . B1[:, n]); else C[r, n] = A[r] . B0[:, n].
 // A rows are read through row_map when it is given (row r of the expert is A[row_map[offset + r]]),
 // and multiplied by row_w[offset + r] on the way into LDS when that is given (rounded to bf16: the
 // bits dispatch's scaled row copy would have held).
 // grid: (ceil(N / 64), as many experts at a time as fill the chip).  K a multiple of 4, N a multiple of 8.
 // NT: the weights are loaded past the caches (load_once).
-template <bool DUAL, int R, bool NT, bool DEEP = false>
+template <bool DUAL, int R, bool NT, bool DEEP = false, int SELECT = 0>
 __global__ __launch_bounds__(gemv::threads(R)) void glu_gemv_bf16_kernel(
     const uint16_t* __restrict__ A, const int32_t* __restrict__ row_map,
     const float* __restrict__ row_w, int lda,
     const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1, uint16_t* __restrict__ C,
     int ldc, int K, int N, const int32_t* __restrict__ counts,
-    const int32_t* __restrict__ offsets, int E) {
+    const int32_t* __restrict__ offsets, int E, const Selection sel) {
   using namespace gemv;
   constexpr int M = DUAL ? 2 : 1;
   constexpr int NW = waves(R), THREADS = threads(R);
@@ -106,13 +192,27 @@ __global__ __launch_bounds__(gemv::threads(R)) void glu_gemv_bf16_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ks = lane >> 3, cc = lane & 7;
-  const int col = blockIdx.x * COLS + cc * 8;
-  const bool col_ok = col < N;  // N is a multiple of 8: the lane's eight channels are in or out together
-  for (int nth = blockIdx.y;; nth += (int)gridDim.y) {
-  const int e = nth_active_expert(counts, E, nth);
-  if (e < 0) return;
-  const int cnt = counts[e], off = offsets[e];
+  __shared__ std::conditional_t<SELECT != 0, Selected, char> chosen;
+  if constexpr (SELECT != 0)
+    select_for_block<SELECT, THREADS>(chosen, sel, E, blockIdx.x == gridDim.x - 1);
+  const int col_blocks = (N + COLS - 1) / COLS;
+  for (int item = SELECT != 0 ? blockIdx.x : blockIdx.y;; item += (int)(SELECT != 0 ? gridDim.x : gridDim.y)) {
+  int e, cnt, off, col_block;
+  if constexpr (SELECT != 0) {
+    const int nth = item / col_blocks;
+    col_block = item - nth * col_blocks;
+    e = nth_selected_expert<SELECT>(chosen, sel.tile_m, nth, cnt, off);
+    if (e < 0) return;
+  } else {
+    col_block = (int)blockIdx.x;
+    e = nth_active_expert(counts, E, item);
+    if (e < 0) return;
+    cnt = counts[e];
+    off = offsets[e];
+  }
   const __amdgpu_buffer_rsrc_t w_rsrc[2] = {expert_matrix(B0, e, K, N), expert_matrix(DUAL ? B1 : B0, e, K, N)};
+  const int col = col_block * COLS + cc * 8;
+  const bool col_ok = col < N;  // N is a multiple of 8: the lane's eight channels are in or out together
   // U steps of K are in flight, each loaded into the registers of the one U before it as soon as that has
   // been multiplied.  The first of them are issued before the rows are even looked up: they need only the
   // expert's number, and a decode step's block is a chain of round trips (one token, D 2048 / F 768: the
@@ -155,6 +255,12 @@ __global__ __launch_bounds__(gemv::threads(R)) void glu_gemv_bf16_kernel(
     float rw[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
+      if constexpr (SELECT != 0) {
+        const int t = selected_token(__builtin_amdgcn_readfirstlane(chosen.bits[e]), r0 + (r < rcnt ? r : 0));
+        src[r] = (size_t)t * lda;
+        rw[r] = row_w != nullptr ? selected_weight(chosen, t, e, sel.K) : 1.f;
+        continue;
+      }
       const int row = off + r0 + (r < rcnt ? r : 0);
       src[r] = (size_t)(row_map != nullptr ? row_map[row] : row) * lda;
       rw[r] = row_w != nullptr ? row_w[row] : 1.f;
@@ -279,7 +385,7 @@ __global__ __launch_bounds__(gemv::threads(R)) void glu_gemv_bf16_kernel(
     __syncthreads();
     for (int i = tid; i < R * COLS; i += THREADS) {
       const int r = i / COLS, c = i - r * COLS;
-      const int n = blockIdx.x * COLS + c;
+      const int n = col_block * COLS + c;
       if (r0 + r >= cnt || n >= N) continue;
       float g = 0.f, u = 0.f;
 #pragma unroll
@@ -316,7 +422,7 @@ namespace gemv16 {
 constexpr int COLS = 128;     // channels per block: 16 lanes x 8
 constexpr int WAVES = 8, THREADS = WAVES * 64;
 constexpr int KSTEP = WAVES * 16;  // k rows per step of the block: waves x 4 lane groups x 4
-constexpr int MAX_LDS_BYTES = 160 * 1024;
+constexpr int MAX_LDS_BYTES = 160 * 1024, MAX_LDS_SELECT = MAX_LDS_BYTES - 6 * 1024;
 __host__ __device__ inline int stride(int K) { return K + 4; }
 inline size_t lds_bytes(int K, int XR, bool dual) {
   const size_t xs = ((size_t)XR * stride(K) + 4) * 2;
@@ -330,13 +436,13 @@ inline bool fits(int K, int XR) { return lds_bytes(K, XR, true) <= (size_t)MAX_L
 // (The second launch bound is waves per SIMD: the single product is held to 128 registers so that
 // two blocks share a CU -- the down projection of 20 active experts is 320 blocks, which at one block
 // per CU ran as a full round and a quarter-full one: 4 us of 75 at 8 tokens.)
-template <bool DUAL, int XR, bool NT>
+template <bool DUAL, int XR, bool NT, int SELECT = 0>
 __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16_kernel(
     const uint16_t* __restrict__ A, const int32_t* __restrict__ row_map,
     const float* __restrict__ row_w, int lda,
     const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1, uint16_t* __restrict__ C,
     int ldc, int K, int N, const int32_t* __restrict__ counts,
-    const int32_t* __restrict__ offsets, int E) {
+    const int32_t* __restrict__ offsets, int E, const Selection sel) {
   using namespace gemv16;
   constexpr int M = DUAL ? 2 : 1;
   constexpr int SETS = 2;  // pairs of steps in flight: 32 (DUAL) or 16 loads per lane
@@ -346,10 +452,24 @@ __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ldx = stride(K);
-  for (int nth = blockIdx.y;; nth += (int)gridDim.y) {
-  const int e = nth_active_expert(counts, E, nth);
-  if (e < 0) return;
-  const int cnt = counts[e], off = offsets[e];
+  __shared__ std::conditional_t<SELECT != 0, Selected, char> chosen;
+  if constexpr (SELECT != 0)
+    select_for_block<SELECT, THREADS>(chosen, sel, E, blockIdx.x == gridDim.x - 1);
+  const int col_blocks = (N + COLS - 1) / COLS;
+  for (int item = SELECT != 0 ? blockIdx.x : blockIdx.y;; item += (int)(SELECT != 0 ? gridDim.x : gridDim.y)) {
+  int e, cnt, off, col_block;
+  if constexpr (SELECT != 0) {
+    const int nth = item / col_blocks;
+    col_block = item - nth * col_blocks;
+    e = nth_selected_expert<SELECT>(chosen, sel.tile_m, nth, cnt, off);
+    if (e < 0) return;
+  } else {
+    col_block = (int)blockIdx.x;
+    e = nth_active_expert(counts, E, item);
+    if (e < 0) return;
+    cnt = counts[e];
+    off = offsets[e];
+  }
   // the expert's matrices as buffers, a lane's place in them as a 32-bit byte offset (one register per
   // address, shared by gate and up)
   const __amdgpu_buffer_rsrc_t w_rsrc[2] = {expert_matrix(B0, e, K, N), expert_matrix(DUAL ? B1 : B0, e, K, N)};
@@ -361,7 +481,7 @@ __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, c16 = lane & 15, g = lane >> 4;
-    const int col = blockIdx.x * COLS + c16 * 8;
+    const int col = col_block * COLS + c16 * 8;
     // (N is a multiple of 8: the lane's eight channels are in or out together)
     const uint32_t lane_col = (uint32_t)(col < N ? col : 0);
     const bool row_ok = c16 < XR;  // row m = c16 of the pass, if it is staged; else, and past K, zeros
@@ -402,6 +522,12 @@ __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16
 #pragma unroll
       for (int i = 0; i < RPW; ++i) {
         const int rr = r0 + wave * RPW + i, row = off + (rr < cnt ? rr : 0);
+        if constexpr (SELECT != 0) {
+          const int t = selected_token(__builtin_amdgcn_readfirstlane(chosen.bits[e]), rr < cnt ? rr : 0);
+          place[i] = (size_t)t * lda;
+          weight[i] = row_w != nullptr ? selected_weight(chosen, t, e, sel.K) : 1.f;
+          continue;
+        }
         place[i] = (size_t)(row_map != nullptr ? row_map[row] : row) * lda;
         weight[i] = row_w != nullptr ? row_w[row] : 1.f;
       }
@@ -524,7 +650,7 @@ __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16
     if (wave == 0 && row_ok && r0 + c16 < cnt) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int n = blockIdx.x * COLS + (4 * g + i) * 8;
+        const int n = col_block * COLS + (4 * g + i) * 8;
         if (n >= N) continue;
         u32x4 o;
 #pragma unroll

@@ -364,7 +364,7 @@ extern "C" int fs2moe_train_forward(const fs2moe_train_args* a, void* stream) {
   const void* x = a->normed ? s.xn : a->x;
   // (rows that stay in token order need no copy: the router's last kernel counts for the dispatch, a launch fewer; 4096
   // tokens, top-8 of 128, D 2048, F 768 1580 -> 1573 us, 4444, D 1280, F 704 1094 -> 1087)
-  DispatchAfterRouter disp{a->tile_m, R, s.counts, s.offsets, s.perm, s.inv_perm, f.disp, f.disp_bytes, nullptr, false};
+  DispatchAfterRouter disp{a->tile_m, R, s.counts, s.offsets, s.perm, s.inv_perm, f.disp, f.disp_bytes, nullptr, nullptr, false};
   int rc = router_then_dispatch(a->x, a->normed ? a->norm_weight : nullptr, a->normed ? a->norm_eps : 0.f,
                                 a->normed ? s.xn : nullptr, a->router_read, a->router_bias, a->T, a->D, a->E, a->K,
                                 a->act_dtype, a->score_fn, a->renormalize, s.idx, s.w, s.logits, f.router,

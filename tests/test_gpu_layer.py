@@ -577,6 +577,54 @@ def test_single_call_dispatches_like_the_dispatch_call(gpu_device, tokens, e, k,
     assert torch.equal(out, _abi.combine(ye, dsp.inv_perm, idx, w, None, True))
 
 
+# Up to 16 tokens, whose experts' first kernel selects and dispatches itself: either stream, one and two tokens a wave,
+# experts at the edges of a word per lane (64), of the two variants (128) and of the form (256), as many slots as there may
+# be, no padding rows, ties, experts that no one takes, and a row of NaN; rows as they are and scaled.
+@pytest.mark.parametrize("tokens,e,k,tile_m", [
+    (1, 3, 1, 16), (1, 128, 8, 16), (2, 65, 2, 1), (4, 129, 4, 16), (5, 64, 8, 8), (8, 256, 32, 16), (9, 128, 3, 16),
+    (16, 33, 5, 1), (16, 256, 8, 16),
+])
+@pytest.mark.parametrize("scale_input", [False, True])
+def test_decode_steps_select_in_the_experts_first_kernel(gpu_device, tokens, e, k, tile_m, scale_input):
+    _say("selects in the experts' kernel", tokens, e, k, tile_m, scale_input)
+    d, f = 640, 200
+    g = torch.Generator().manual_seed(tokens + e)
+    x = torch.randn(tokens, d, generator=g).bfloat16().to(gpu_device)
+    if tokens > 1:
+        x[tokens // 2] = float("nan")
+    router = (torch.randn(d, e, generator=g) * 0.3).bfloat16().to(gpu_device)
+    router[:, 1] = router[:, 0]
+    bias = torch.zeros(e)
+    bias[e // 2:: 5] = -30.0
+    bias = bias.to(gpu_device)
+    wg, wu, wd = ((torch.randn(e * a, b, generator=g) * 0.1).bfloat16().to(gpu_device) for a, b in ((d, f), (d, f), (f, d)))
+    score = _abi.SCORE_SIGMOID if scale_input else _abi.SCORE_SOFTMAX
+    lib = _abi.load()
+    ws = torch.zeros(lib.fs2moe_forward_workspace_bytes(tokens, d, e, k, f, 0, tile_m, _abi.BF16),
+                     dtype=torch.uint8, device=gpu_device)
+
+    def call():
+        return _abi.forward(x, router, bias, wg, wu, wd, e, k, tile_m=tile_m, score_fn=score, renormalize=not scale_input,
+                            scale_input=scale_input, workspace=ws)
+
+    out = call()
+    idx, w, _ = _abi.router_topk(x, router, bias, k, score, not scale_input)
+    dsp = _abi.dispatch(idx, w, x, e, tile_m, scale_input, gather=scale_input)
+    torch.cuda.synchronize()
+    rows, at, parts = _abi.max_rows(tokens, k, e, tile_m), 0, []
+    for n in (tokens * k, tokens * k, e, e + 1, rows, tokens * k):
+        parts.append(ws[at: at + 4 * n].view(torch.int32))
+        at += (4 * n + 255) // 256 * 256
+    for got, want in zip(parts, (idx, w.view(torch.int32), dsp.counts, dsp.offsets, dsp.perm, dsp.inv_perm)):
+        assert torch.equal(got, want.reshape(-1))
+    ye, _ = _abi.grouped_swiglu(dsp.xe if scale_input else x, dsp.counts, dsp.offsets, wg, wu, wd, e,
+                                row_map=None if scale_input else dsp.perm, rows_per_expert=tokens)
+    want = _abi.combine(ye, dsp.inv_perm, idx, w, None, not scale_input)
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    names = launched(call)
+    assert len(names) == 4 and names[1].startswith("glu_gemv"), names
+
+
 def test_expert_major_copy_of_the_router_follows_the_parameter(gpu_device):
     """The derived (E, D) copy the bf16 router reads: made once, made again after an in-place update,
     after a move and for another tensor (also one that reuses a freed tensor's address), and kept
