@@ -253,7 +253,7 @@ int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_
     return FS2MOE_OK;
   };
   const int64_t planned = fs2moe::planned_rows((int64_t)T * K, E);
-  bool forked = false;
+  bool forked = false, shared_done = false;
   // router, dispatch and the routed experts, with the shared expert forked off on the way
   auto routed_path = [&]() -> int {
     if (beside && !normed) {
@@ -278,9 +278,13 @@ int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_
       forked = true;
       if (int rc = shared_beside()) return rc;
     }
-    if (later.partial != nullptr)
+    if (later.partial != nullptr) {
+      // (the shared expert's products go into the routed ones' launches)
+      const fs2moe::SharedBeside with = {shared_gate, shared_up, shared_down, F_shared, b.shared_h, out};
+      shared_done = shared && fs2moe::shared_goes_with_rows(D, F_shared, T);
       return fs2moe::grouped_swiglu_selecting(x, later, w_gate, w_up, w_down, E, D, F, b.max_rows, planned, b.h, b.ye,
-                                              stream);
+                                              shared_done ? &with : nullptr, stream);
+    }
     if (!disp.done) {
       if (scaled_stream) {
         if (int rc = fs2moe::dispatch_with_row_weights(b.topk_idx, b.topk_w, T, K, E, tile_m,
@@ -316,7 +320,7 @@ int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_
   if (rc_routed != FS2MOE_OK) return rc_routed;
   const void* base = nullptr;
   if (shared) {
-    if (!beside)
+    if (!beside && !shared_done)
       if (int rc = shared_on(stream, x)) return rc;
     base = out;
   }

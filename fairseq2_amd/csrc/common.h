@@ -304,10 +304,18 @@ bool swiglu_streams_rows(int32_t act_dtype, int32_t w_dtype, int32_t D, int32_t 
                          int32_t rows_per_expert);
 // Whether the pair may begin with the selection itself (grouped_swiglu_selecting): up to 16 tokens on these kernels, with room
 // for its tables in LDS; and that pair, whose rows are those of `sel`, read from x.
+// (shared: optionally a shared expert, computed in the same launches)
+struct SharedBeside {
+  const void *gate, *up, *down;
+  int F;
+  void *h, *out;
+};
 bool swiglu_selects(int32_t act_dtype, int32_t w_dtype, int32_t D, int32_t F, int32_t E, int32_t T);
 int grouped_swiglu_selecting(const void* x, const Selection& sel, const void* w_gate, const void* w_up, const void* w_down,
                              int32_t E, int32_t D, int32_t F, int64_t max_rows, int64_t planned, void* h, void* ye,
-                             void* stream);
+                             const SharedBeside* shared, void* stream);
+// Whether a shared expert of F features can go with it, for at most 16 tokens.
+bool shared_goes_with_rows(int32_t D, int32_t F, int32_t T);
 int grouped_swiglu_scaled_rows(const void* x, const int32_t* row_map, const float* row_w,
                                const int32_t* counts, const int32_t* offsets, const void* w_gate,
                                const void* w_up, const void* w_down, int32_t E, int32_t D, int32_t F,

@@ -572,10 +572,25 @@ static unsigned stream_experts(int blocks, int col_blocks, int E) {
   return (unsigned)(n < E ? n : E);
 }
 
+// The shared expert's product that goes with the routed ones' gate/up or down product (shared null: none).
+static DenseBeside dense_beside(const SharedBeside* shared, bool dual, const void* x, int D, const Selection* sel) {
+  if (shared == nullptr || sel == nullptr) return DenseBeside{};
+  auto in = [](const void* p) { return static_cast<const uint16_t*>(p); };
+  if (dual)
+    return {in(x), in(shared->gate), in(shared->up), static_cast<uint16_t*>(shared->h), D, shared->F, sel->T, (shared->F + 15) / 16};
+  return {in(shared->h), in(shared->down), nullptr, static_cast<uint16_t*>(shared->out), shared->F, D, sel->T, (D + 15) / 16};
+}
+static unsigned beside_rows(const DenseBeside& dense, int col_blocks) {
+  return (unsigned)((dense.blocks + col_blocks - 1) / col_blocks);
+}
+static size_t beside_lds(size_t bytes, const DenseBeside& dense, bool dual) {
+  return dense.blocks > 0 && bytes < (size_t)dgemv::red_bytes(dual) ? (size_t)dgemv::red_bytes(dual) : bytes;
+}
+
 // A kernel that begins with the selection has a block a CU (its registers allow no more), which take (expert, channel block)
-// pairs in turn, so that each selects once; and no more than there may be pairs.
-static dim3 selecting_grid(const Selection& sel, int col_blocks, int E) {
-  const int64_t pairs = (int64_t)sel.T * sel.K, most = (pairs < E ? pairs : E) * col_blocks;
+// pairs in turn, so that each selects once; and no more than there may be pairs (and blocks of the shared expert).
+static dim3 selecting_grid(const Selection& sel, int col_blocks, int E, const DenseBeside& dense) {
+  const int64_t pairs = (int64_t)sel.T * sel.K, most = (pairs < E ? pairs : E) * col_blocks + dense.blocks;
   return dim3((unsigned)(most < 256 ? most : 256));
 }
 
@@ -583,7 +598,7 @@ template <int R, bool NT>
 static int launch_gemv_pair_r(const void* x, const int32_t* row_map, const float* row_w,
                               const Groups& g, const void* w_gate, const void* w_up,
                               const void* w_down, int D, int F, void* h, void* y,
-                              hipStream_t stream, const Selection* sel) {
+                              hipStream_t stream, const Selection* sel, const SharedBeside* shared) {
   using namespace gemv;
   auto k1 = glu_gemv_bf16_kernel<true, R, NT>;
   auto k1s2 = glu_gemv_bf16_kernel<true, R, NT, false, 2>;
@@ -606,20 +621,22 @@ static int launch_gemv_pair_r(const void* x, const int32_t* row_map, const float
   }
   if (sel != nullptr) k1 = g.E <= 128 ? k1s2 : k1s4;
   const Selection selection = sel != nullptr ? *sel : Selection{};
+  const DenseBeside up_beside = dense_beside(shared, true, x, D, sel), down_beside = dense_beside(shared, false, x, D, sel);
   const uint16_t* xp = static_cast<const uint16_t*>(x);
   const int f_blocks = (F + COLS - 1) / COLS, d_blocks = (D + COLS - 1) / COLS;
-  hipLaunchKernelGGL(k1, sel != nullptr ? selecting_grid(*sel, f_blocks, g.E)
+  hipLaunchKernelGGL(k1, sel != nullptr ? selecting_grid(*sel, f_blocks, g.E, up_beside)
                                         : dim3((unsigned)f_blocks, stream_experts(256 * (R + 1), f_blocks, g.E)), dim3(threads(R)),
-                     (size_t)R * D * 2, stream, xp, row_map, row_w, D, static_cast<const uint16_t*>(w_gate),
+                     beside_lds((size_t)R * D * 2, up_beside, true), stream, xp, row_map, row_w, D, static_cast<const uint16_t*>(w_gate),
                      static_cast<const uint16_t*>(w_up), static_cast<uint16_t*>(h), F, D, F,
-                     g.counts, g.offsets, g.E, selection);
+                     g.counts, g.offsets, g.E, selection, up_beside);
   if (int rc = check_launch("glu_gemv_bf16<gate,up>")) return rc;
-  hipLaunchKernelGGL(deep_applies(F, R) ? k2d : k2, dim3((unsigned)d_blocks, stream_experts(256 * (R + 1), d_blocks, g.E)),
-                     dim3(threads(R)), (size_t)R * F * 2, stream, static_cast<const uint16_t*>(h),
+  hipLaunchKernelGGL(deep_applies(F, R) ? k2d : k2,
+                     dim3((unsigned)d_blocks, stream_experts(256 * (R + 1), d_blocks, g.E) + beside_rows(down_beside, d_blocks)),
+                     dim3(threads(R)), beside_lds((size_t)R * F * 2, down_beside, false), stream, static_cast<const uint16_t*>(h),
                      static_cast<const int32_t*>(nullptr), static_cast<const float*>(nullptr), F,
                      static_cast<const uint16_t*>(w_down),
                      static_cast<const uint16_t*>(nullptr), static_cast<uint16_t*>(y), D, F, D,
-                     g.counts, g.offsets, g.E, Selection{});
+                     g.counts, g.offsets, g.E, Selection{}, down_beside);
   return check_launch("glu_gemv_bf16<down>");
 }
 
@@ -647,7 +664,7 @@ template <int XR, bool NT>
 static int launch_gemv16_pair(const void* x, const int32_t* row_map, const float* row_w,
                               const Groups& g, const void* w_gate, const void* w_up,
                               const void* w_down, int D, int F, void* h, void* y,
-                              hipStream_t stream, const Selection* sel) {
+                              hipStream_t stream, const Selection* sel, const SharedBeside* shared) {
   using namespace gemv16;
   auto k1 = glu_gemv16_bf16_kernel<true, XR, NT>;
   auto k1s2 = glu_gemv16_bf16_kernel<true, XR, NT, 2>;
@@ -668,19 +685,20 @@ static int launch_gemv16_pair(const void* x, const int32_t* row_map, const float
   }
   if (sel != nullptr) k1 = g.E <= 128 ? k1s2 : k1s4;
   const Selection selection = sel != nullptr ? *sel : Selection{};
+  const DenseBeside up_beside = dense_beside(shared, true, x, D, sel), down_beside = dense_beside(shared, false, x, D, sel);
   const int f_blocks = (F + COLS - 1) / COLS, d_blocks = (D + COLS - 1) / COLS;
-  hipLaunchKernelGGL(k1, sel != nullptr ? selecting_grid(*sel, f_blocks, g.E)
+  hipLaunchKernelGGL(k1, sel != nullptr ? selecting_grid(*sel, f_blocks, g.E, up_beside)
                                         : dim3((unsigned)f_blocks, stream_experts(2048, f_blocks, g.E)), dim3(THREADS),
-                     lds_bytes(D, XR, true), stream, static_cast<const uint16_t*>(x), row_map, row_w, D,
+                     beside_lds(lds_bytes(D, XR, true), up_beside, true), stream, static_cast<const uint16_t*>(x), row_map, row_w, D,
                      static_cast<const uint16_t*>(w_gate), static_cast<const uint16_t*>(w_up),
-                     static_cast<uint16_t*>(h), F, D, F, g.counts, g.offsets, g.E, selection);
+                     static_cast<uint16_t*>(h), F, D, F, g.counts, g.offsets, g.E, selection, up_beside);
   if (int rc = check_launch("glu_gemv16_bf16<gate,up>")) return rc;
-  hipLaunchKernelGGL(k2, dim3((unsigned)d_blocks, stream_experts(2048, d_blocks, g.E)), dim3(THREADS),
-                     lds_bytes(F, XR, false), stream, static_cast<const uint16_t*>(h),
+  hipLaunchKernelGGL(k2, dim3((unsigned)d_blocks, stream_experts(2048, d_blocks, g.E) + beside_rows(down_beside, d_blocks)),
+                     dim3(THREADS), beside_lds(lds_bytes(F, XR, false), down_beside, false), stream, static_cast<const uint16_t*>(h),
                      static_cast<const int32_t*>(nullptr), static_cast<const float*>(nullptr), F,
                      static_cast<const uint16_t*>(w_down),
                      static_cast<const uint16_t*>(nullptr), static_cast<uint16_t*>(y), D, F, D,
-                     g.counts, g.offsets, g.E, Selection{});
+                     g.counts, g.offsets, g.E, Selection{}, down_beside);
   return check_launch("glu_gemv16_bf16<down>");
 }
 
@@ -710,7 +728,7 @@ template <int BLAYOUT>
 static int launch_glu(const void* x, const int32_t* row_map, const Groups& g, int64_t rows_bound,
                       const void* w_gate, const void* w_up, const void* w_down, int D, int F,
                       int act_dtype, void* h, void* y, hipStream_t stream, int rows_hint = 0,
-                      const float* row_w = nullptr, const Selection* sel = nullptr) {
+                      const float* row_w = nullptr, const Selection* sel = nullptr, const SharedBeside* shared = nullptr) {
   const int groups = g.counts ? g.E : 0;
   // (rows off the lines share them with the rows beside, in both orientations: nn.Linear's of D 4096, F 8192 42.8 us
   // without and 48.1 with the hint on the same weights again, 64.6 and 53.2 with other memory read in between; of D 5160,
@@ -728,13 +746,13 @@ static int launch_glu(const void* x, const int32_t* row_map, const Groups& g, in
       auto launch = rows_hint <= 1   ? (past ? launch_gemv_pair_r<1, true> : launch_gemv_pair_r<1, false>)
                     : rows_hint <= 2 ? (past ? launch_gemv_pair_r<2, true> : launch_gemv_pair_r<2, false>)
                                      : (past ? launch_gemv_pair_r<4, true> : launch_gemv_pair_r<4, false>);
-      return launch(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream, sel);
+      return launch(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream, sel, shared);
     }
     if (gemv16_applies(act_dtype, D, F, g, rows_hint)) {
       auto launch = gemv16_rows(D, F, rows_hint) == 8
                         ? (past ? launch_gemv16_pair<8, true> : launch_gemv16_pair<8, false>)
                         : (past ? launch_gemv16_pair<16, true> : launch_gemv16_pair<16, false>);
-      return launch(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream, sel);
+      return launch(x, row_map, row_w, g, w_gate, w_up, w_down, D, F, h, y, stream, sel, shared);
     }
   }
   if (row_w != nullptr || sel != nullptr) {
@@ -956,14 +974,20 @@ bool fs2moe::swiglu_selects(int32_t act_dtype, int32_t w_dtype, int32_t D, int32
 
 int fs2moe::grouped_swiglu_selecting(const void* x, const Selection& sel, const void* w_gate, const void* w_up,
                                      const void* w_down, int32_t E, int32_t D, int32_t F, int64_t max_rows, int64_t planned,
-                                     void* h, void* ye, void* stream) {
+                                     void* h, void* ye, const SharedBeside* shared, void* stream) {
   FS2_REQUIRE(swiglu_selects(FS2MOE_BF16, FS2MOE_BF16, D, F, E, sel.T),
               "grouped_swiglu: internal: D=%d F=%d E=%d of %d tokens do not select", D, F, E, sel.T);
   FS2_REQUIRE(aligned16(x) && aligned16(w_gate) && aligned16(w_up) && aligned16(w_down) && aligned16(h) && aligned16(ye),
               "grouped_swiglu: buffers must be 16-byte aligned");
   const Groups g{sel.counts, sel.offsets, E, 0, (int)planned};
   return launch_glu<FS2MOE_W_IN_OUT>(x, sel.perm, g, max_rows, w_gate, w_up, w_down, D, F, FS2MOE_BF16, h, ye,
-                                     static_cast<hipStream_t>(stream), sel.T, sel.row_w, &sel);
+                                     static_cast<hipStream_t>(stream), sel.T, sel.row_w, &sel, shared);
+}
+
+bool fs2moe::shared_goes_with_rows(int32_t D, int32_t F, int32_t T) {
+  // (not where its weights are loaded past the caches, which these kernels choose for the routed ones)
+  return T >= 1 && T <= dgemv::MAX_ROWS && D % 8 == 0 && F % 8 == 0 &&
+         !(D % 64 == 0 && F % 64 == 0 && weights_past_cache(0, 0, D, F, 2));
 }
 
 int fs2moe::grouped_swiglu_scaled_rows(const void* x, const int32_t* row_map, const float* row_w,

@@ -84,6 +84,109 @@ __device__ __forceinline__ int nth_active_expert(const int32_t* __restrict__ cou
   return e;
 }
 
+// ---------------------------------------------------------------------------------------------------
+// The shared expert (a dense SwiGLU, weights as nn.Linear holds them: (N, K) with K contiguous) for
+// up to 16 rows: at a decode step its three matrices are streamed once like an expert's, and the
+// GEMM tiles make that a chain of K / 64 round trips per tile (Llama-4 Scout, one token: 172 us for
+// 252 MB).  Here 16 bytes of a weight row ARE eight k of one channel, which is what
+// v_mfma_f32_16x16x32_bf16 takes from lane (n = l % 16, g = l / 16) as it stands; the matching lane
+// (m = l % 16, g) loads the same eight k of row m straight from memory (the rows stay in L2; a row
+// the call does not have repeats the last one, its results are not stored).  A block owns 16
+// channels, its eight waves split K in steps of 32 and add their sums in LDS in ascending order.
+namespace dgemv {
+constexpr int WAVES = 8, THREADS = WAVES * 64;
+constexpr int U = 8;  // steps of 32 k a wave has in flight
+constexpr int MAX_ROWS = 16;
+constexpr int red_bytes(bool dual) { return WAVES * (dual ? 2 : 1) * 64 * 16; }
+}  // namespace dgemv
+
+// DUAL: C[r, n] = SiLU(A[r] . B0[n]) * (A[r] . B1[n]); else C[r, n] = A[r] . B0[n].
+// A [T][lda], B0/B1 [N][K], C [T][ldc]; T <= 16; K and N multiples of 8.  grid: ceil(N / 16).
+// red: LDS of red_bytes(DUAL).
+template <bool DUAL, bool NT>
+__device__ __forceinline__ void dense_gemv_block(
+    const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ B0,
+    const uint16_t* __restrict__ B1, uint16_t* __restrict__ C, int ldc, int K, int N, int T, int block, uint8_t* lds) {
+  using namespace dgemv;
+  constexpr int M = DUAL ? 2 : 1;
+  f32x4(*red)[M][64] = reinterpret_cast<f32x4(*)[M][64]>(lds);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  const int n0 = block * 16;
+  const int n = n0 + r16 < N ? n0 + r16 : N - 1;  // a channel past N repeats the last one: not stored
+  const int row = r16 < T ? r16 : T - 1;
+  const uint16_t* w0 = B0 + (size_t)n * K;
+  const uint16_t* w1 = DUAL ? B1 + (size_t)n * K : w0;
+  const uint16_t* xr = A + (size_t)row * lda;
+  f32x4 acc[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // step s of the block is the 32 k from 32 s; wave w takes the steps w, w + 8, ..
+  for (int s0 = wave; s0 * 32 < K; s0 += WAVES * U) {
+    u32x4 wq[U][M], xq[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = (s0 + u * WAVES) * 32 + g * 8;
+      const int kk = k < K ? k : 0;  // K is a multiple of 8: the lane's eight k are in or out together
+      wq[u][0] = load_weights<NT>(w0 + kk);
+      if (DUAL) wq[u][M - 1] = load_weights<NT>(w1 + kk);
+      xq[u] = *reinterpret_cast<const u32x4*>(xr + kk);
+    }
+    // (all the loads are issued before the first is waited for)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = (s0 + u * WAVES) * 32 + g * 8;
+      u32x4 xv = xq[u];
+      if (k >= K) xv = u32x4{0u, 0u, 0u, 0u};
+      const bf16x8 xop = __builtin_bit_cast(bf16x8, xv);
+#pragma unroll
+      for (int m = 0; m < M; ++m)
+        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wq[u][m]), xop,
+                                                         acc[m], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < M; ++m) red[wave][m][lane] = acc[m];
+  __syncthreads();
+  if (wave != 0) return;
+  // lane (row m = l % 16, q = l / 16) holds channels n0 + 4 q + i, i = 0..3
+  f32x4 sum[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    sum[m] = red[0][m][lane];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) sum[m] += red[w][m][lane];
+  }
+  const int nc = n0 + 4 * g;
+  if (r16 < T && nc < N) {  // N is a multiple of 8: four channels are in or out together
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = DUAL ? silu_f32(sum[0][i]) * sum[M - 1][i] : sum[0][i];
+    u32x2 o = {(uint32_t)f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16),
+               (uint32_t)f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16)};
+    *reinterpret_cast<u32x2*>(C + (size_t)r16 * ldc + nc) = o;
+  }
+}
+template <bool DUAL, bool NT>
+__global__ __launch_bounds__(dgemv::THREADS) void dense_gemv_bf16_kernel(
+    const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ B0,
+    const uint16_t* __restrict__ B1, uint16_t* __restrict__ C, int ldc, int K, int N, int T) {
+  __shared__ __attribute__((aligned(16))) uint8_t red[dgemv::red_bytes(DUAL)];
+  dense_gemv_block<DUAL, NT>(A, lda, B0, B1, C, ldc, K, N, T, (int)blockIdx.x, red);
+}
+// The same product of the shared expert in the launch of the routed ones: `blocks` blocks of it (0: none).
+struct DenseBeside {
+  const uint16_t *A, *B0, *B1;
+  uint16_t* C;
+  int K, N, T, blocks;
+};
+template <bool DUAL>
+__device__ __forceinline__ void dense_beside_block(const DenseBeside& d, int block, uint8_t* lds) {
+  dense_gemv_block<DUAL, false>(d.A, d.K, d.B0, d.B1, d.C, d.N, d.K, d.N, d.T, block, lds);
+}
+
 // SELECT 2 or 4 (gate/up): the kernel begins with what router_finish_tile_kernel does, for at most 16 tokens and 64 SELECT
 // experts.  Every block adds the partial logits, selects and keeps a word per expert with a bit per token in LDS, from which
 // its experts, their rows and those rows' tokens follow without a look at memory; the last block of the grid, which has the
@@ -157,6 +260,34 @@ __device__ __forceinline__ int nth_selected_expert(const Selected& s, int tile_m
   return e;
 }
 static_assert(sizeof(Selected) <= 6 * 1024, "left out of MAX_LDS_SELECT");
+// The shared expert's product in the routed ones' launch: its own two launches had each a boundary and a round trip or two
+// while most of the chip waited, and the routed ones' blocks do not fill it either.  us of the layer under a graph with the
+// launches and without: 1 and 8 tokens of D 2048, F 768, top-8 of 128 53.8, 41.2 and 85.5, 70.6; 2 and 12 of D 1024, F 1408,
+// top-4 of 60 53.3, 42.8 and 101.9, 85.8; 6 of D 4096, F 4096, top-2 of 16 242, 233.  (One whose weights are loaded past the
+// caches has launches of its own, as has one of 192 MB and more, which runs beside the whole routed path.)
+// What a block has to do of it, in front of its own.  SELECT (blocks that stay): blocks d, d + grid,
+// .. of it, and the routed experts' pairs go on where those end; returns the block's first pair.  Else the first rows of the
+// grid are theirs; returns how many, or -1 in such a block.
+template <bool DUAL, bool SELECT>
+__device__ __forceinline__ int dense_of_grid(const DenseBeside& dense, uint8_t* lds) {
+  const int grid = (int)gridDim.x;
+  if constexpr (SELECT) {
+    int b = (int)blockIdx.x;
+    for (; b < dense.blocks; b += grid) {
+      if (b >= grid) __syncthreads();  // (the sums of the block before)
+      dense_beside_block<DUAL>(dense, b, lds);
+    }
+    return b - dense.blocks;
+  } else if constexpr (DUAL) {
+    return 0;  // (gate/up goes with the selection only)
+  } else {
+    const int rows = (dense.blocks + grid - 1) / grid;
+    if ((int)blockIdx.y >= rows) return rows;
+    const int b = (int)blockIdx.y * grid + (int)blockIdx.x;
+    if (b < dense.blocks) dense_beside_block<DUAL>(dense, b, lds);
+    return -1;
+  }
+}
 // The token of the expert's r-th row, and the weight of that pair.
 __device__ __forceinline__ int selected_token(uint32_t bits, int r) {
   for (int i = 0; i < r; ++i) bits &= bits - 1u;
@@ -180,7 +311,7 @@ __global__ __launch_bounds__(gemv::threads(R)) void glu_gemv_bf16_kernel(
     const float* __restrict__ row_w, int lda,
     const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1, uint16_t* __restrict__ C,
     int ldc, int K, int N, const int32_t* __restrict__ counts,
-    const int32_t* __restrict__ offsets, int E, const Selection sel) {
+    const int32_t* __restrict__ offsets, int E, const Selection sel, const DenseBeside dense) {
   using namespace gemv;
   constexpr int M = DUAL ? 2 : 1;
   constexpr int NW = waves(R), THREADS = threads(R);
@@ -192,11 +323,14 @@ __global__ __launch_bounds__(gemv::threads(R)) void glu_gemv_bf16_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ks = lane >> 3, cc = lane & 7;
+  const int dense_rows = dense_of_grid<DUAL, SELECT != 0>(dense, gemv_smem);
+  if (dense_rows < 0) return;
   __shared__ std::conditional_t<SELECT != 0, Selected, char> chosen;
   if constexpr (SELECT != 0)
     select_for_block<SELECT, THREADS>(chosen, sel, E, blockIdx.x == gridDim.x - 1);
   const int col_blocks = (N + COLS - 1) / COLS;
-  for (int item = SELECT != 0 ? blockIdx.x : blockIdx.y;; item += (int)(SELECT != 0 ? gridDim.x : gridDim.y)) {
+  const int items_at_once = SELECT != 0 ? (int)gridDim.x : (int)gridDim.y - dense_rows;
+  for (int item = SELECT != 0 ? dense_rows : (int)blockIdx.y - dense_rows;; item += items_at_once) {
   int e, cnt, off, col_block;
   if constexpr (SELECT != 0) {
     const int nth = item / col_blocks;
@@ -442,7 +576,7 @@ __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16
     const float* __restrict__ row_w, int lda,
     const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1, uint16_t* __restrict__ C,
     int ldc, int K, int N, const int32_t* __restrict__ counts,
-    const int32_t* __restrict__ offsets, int E, const Selection sel) {
+    const int32_t* __restrict__ offsets, int E, const Selection sel, const DenseBeside dense) {
   using namespace gemv16;
   constexpr int M = DUAL ? 2 : 1;
   constexpr int SETS = 2;  // pairs of steps in flight: 32 (DUAL) or 16 loads per lane
@@ -452,11 +586,14 @@ __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ldx = stride(K);
+  const int dense_rows = dense_of_grid<DUAL, SELECT != 0>(dense, gemv16_smem);
+  if (dense_rows < 0) return;
   __shared__ std::conditional_t<SELECT != 0, Selected, char> chosen;
   if constexpr (SELECT != 0)
     select_for_block<SELECT, THREADS>(chosen, sel, E, blockIdx.x == gridDim.x - 1);
   const int col_blocks = (N + COLS - 1) / COLS;
-  for (int item = SELECT != 0 ? blockIdx.x : blockIdx.y;; item += (int)(SELECT != 0 ? gridDim.x : gridDim.y)) {
+  const int items_at_once = SELECT != 0 ? (int)gridDim.x : (int)gridDim.y - dense_rows;
+  for (int item = SELECT != 0 ? dense_rows : (int)blockIdx.y - dense_rows;; item += items_at_once) {
   int e, cnt, off, col_block;
   if constexpr (SELECT != 0) {
     const int nth = item / col_blocks;
@@ -666,90 +803,6 @@ __global__ __launch_bounds__(gemv16::THREADS, DUAL ? 2 : 4) void glu_gemv16_bf16
       }
     }
   }
-  }
-}
-
-// ---------------------------------------------------------------------------------------------------
-// The shared expert (a dense SwiGLU, weights as nn.Linear holds them: (N, K) with K contiguous) for
-// up to 16 rows: at a decode step its three matrices are streamed once like an expert's, and the
-// GEMM tiles make that a chain of K / 64 round trips per tile (Llama-4 Scout, one token: 172 us for
-// 252 MB).  Here 16 bytes of a weight row ARE eight k of one channel, which is what
-// v_mfma_f32_16x16x32_bf16 takes from lane (n = l % 16, g = l / 16) as it stands; the matching lane
-// (m = l % 16, g) loads the same eight k of row m straight from memory (the rows stay in L2; a row
-// the call does not have repeats the last one, its results are not stored).  A block owns 16
-// channels, its eight waves split K in steps of 32 and add their sums in LDS in ascending order.
-namespace dgemv {
-constexpr int WAVES = 8, THREADS = WAVES * 64;
-constexpr int U = 8;  // steps of 32 k a wave has in flight
-constexpr int MAX_ROWS = 16;
-}  // namespace dgemv
-
-// DUAL: C[r, n] = SiLU(A[r] . B0[n]) * (A[r] . B1[n]); else C[r, n] = A[r] . B0[n].
-// A [T][lda], B0/B1 [N][K], C [T][ldc]; T <= 16; K and N multiples of 8.  grid: ceil(N / 16).
-template <bool DUAL, bool NT>
-__global__ __launch_bounds__(dgemv::THREADS) void dense_gemv_bf16_kernel(
-    const uint16_t* __restrict__ A, int lda, const uint16_t* __restrict__ B0,
-    const uint16_t* __restrict__ B1, uint16_t* __restrict__ C, int ldc, int K, int N, int T) {
-  using namespace dgemv;
-  constexpr int M = DUAL ? 2 : 1;
-  __shared__ f32x4 red[WAVES][M][64];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r16 = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16;
-  const int n = n0 + r16 < N ? n0 + r16 : N - 1;  // a channel past N repeats the last one: not stored
-  const int row = r16 < T ? r16 : T - 1;
-  const uint16_t* w0 = B0 + (size_t)n * K;
-  const uint16_t* w1 = DUAL ? B1 + (size_t)n * K : w0;
-  const uint16_t* xr = A + (size_t)row * lda;
-  f32x4 acc[M];
-#pragma unroll
-  for (int m = 0; m < M; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // step s of the block is the 32 k from 32 s; wave w takes the steps w, w + 8, ..
-  for (int s0 = wave; s0 * 32 < K; s0 += WAVES * U) {
-    u32x4 wq[U][M], xq[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = (s0 + u * WAVES) * 32 + g * 8;
-      const int kk = k < K ? k : 0;  // K is a multiple of 8: the lane's eight k are in or out together
-      wq[u][0] = load_weights<NT>(w0 + kk);
-      if (DUAL) wq[u][M - 1] = load_weights<NT>(w1 + kk);
-      xq[u] = *reinterpret_cast<const u32x4*>(xr + kk);
-    }
-    // (all the loads are issued before the first is waited for)
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = (s0 + u * WAVES) * 32 + g * 8;
-      u32x4 xv = xq[u];
-      if (k >= K) xv = u32x4{0u, 0u, 0u, 0u};
-      const bf16x8 xop = __builtin_bit_cast(bf16x8, xv);
-#pragma unroll
-      for (int m = 0; m < M; ++m)
-        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wq[u][m]), xop,
-                                                         acc[m], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int m = 0; m < M; ++m) red[wave][m][lane] = acc[m];
-  __syncthreads();
-  if (wave != 0) return;
-  // lane (row m = l % 16, q = l / 16) holds channels n0 + 4 q + i, i = 0..3
-  f32x4 sum[M];
-#pragma unroll
-  for (int m = 0; m < M; ++m) {
-    sum[m] = red[0][m][lane];
-#pragma unroll
-    for (int w = 1; w < WAVES; ++w) sum[m] += red[w][m][lane];
-  }
-  const int nc = n0 + 4 * g;
-  if (r16 < T && nc < N) {  // N is a multiple of 8: four channels are in or out together
-    float v[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = DUAL ? silu_f32(sum[0][i]) * sum[M - 1][i] : sum[0][i];
-    u32x2 o = {(uint32_t)f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16),
-               (uint32_t)f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16)};
-    *reinterpret_cast<u32x2*>(C + (size_t)r16 * ldc + nc) = o;
   }
 }
 

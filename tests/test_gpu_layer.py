@@ -625,6 +625,29 @@ def test_decode_steps_select_in_the_experts_first_kernel(gpu_device, tokens, e, 
     assert len(names) == 4 and names[1].startswith("glu_gemv"), names
 
 
+# A shared expert in the launches of the routed ones: fewer features than a block's, a few blocks of which the last holds
+# half, and more blocks than the grid has, on either stream.
+@pytest.mark.parametrize("tokens,e,k", [(1, 3, 1), (4, 24, 3), (5, 200, 4), (16, 24, 8)])
+@pytest.mark.parametrize("f_shared", [8, 200, 8200])
+def test_decode_steps_with_a_shared_expert_in_the_same_launches(gpu_device, tokens, e, k, f_shared):
+    _say("shared expert in the routed launches", tokens, e, k, f_shared)
+    d, f = 648, 200
+    g = torch.Generator().manual_seed(tokens + f_shared)
+    mk = lambda *s, scale=1.0: (scale * torch.randn(*s, generator=g)).bfloat16().to(gpu_device)  # noqa: E731
+    x, router = mk(tokens, d), mk(d, e, scale=0.3)
+    wg, wu, wd = mk(e * d, f, scale=0.1), mk(e * d, f, scale=0.1), mk(e * f, d, scale=0.1)
+    sh = (mk(f_shared, d, scale=0.1), mk(f_shared, d, scale=0.1), mk(d, f_shared, scale=0.1))
+
+    def call():
+        return _abi.forward(x, router, None, wg, wu, wd, e, k, shared=sh, score_fn=_abi.SCORE_SOFTMAX, scale_input=False)
+
+    idx, w, _ = _abi.router_topk(x, router, None, k, _abi.SCORE_SOFTMAX)
+    dsp = _abi.dispatch(idx, w, x, e, 16, False, gather=False)
+    ye, _ = _abi.grouped_swiglu(x, dsp.counts, dsp.offsets, wg, wu, wd, e, row_map=dsp.perm, rows_per_expert=tokens)
+    assert torch.equal(call(), _abi.combine(ye, dsp.inv_perm, idx, w, _abi.dense_swiglu(x, *sh), True))
+    assert len(launched(call)) == 4
+
+
 def test_expert_major_copy_of_the_router_follows_the_parameter(gpu_device):
     """The derived (E, D) copy the bf16 router reads: made once, made again after an in-place update,
     after a move and for another tensor (also one that reuses a freed tensor's address), and kept
