@@ -114,44 +114,92 @@ extern "C" int64_t fs2moe_forward_norm_workspace_bytes(int32_t T, int32_t D, int
   return carve_forward(nullptr, T, D, E, K, F, F_shared, tile_m, act_dtype, true, true).total;
 }
 
-namespace {
+namespace fs2moe {
 
-// A stream of the library's own per device, for the shared expert of a decode step.  The shared
-// expert depends on the rows only, and with a handful of tokens the routed path (the router's two
-// small kernels, the dispatch, one or a few experts' weight streams) leaves most of the chip idle
-// while it runs: the shared expert's two kernels go onto this stream, forked from the caller's
-// stream by an event and joined back by another before the combine, so a caller sees one stream's
-// worth of ordering (and a capturing stream captures both branches).  Default priority, created
-// on the first use on a device and kept; the events are reused, which is why the record-and-wait
-// pairs are taken under a lock: between one thread's record and its wait another thread's
-// record of the same event would replace what is waited for.
+// Streams of the library's own, two per device: one for callers' streams that run their work, one for those that capture
+// it, so that a capture never finds another thread's work on the stream.  Default priority, created on the first use on a
+// device and kept; the events are reused, which is why the record-and-wait pairs are taken under a lock: between one
+// thread's record and its wait another thread's record of the same event would replace what is waited for.
 struct SideStream {
   hipStream_t stream = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
+};
+namespace {
+constexpr int kSideDevices = 64;
+struct SideStreams {
+  SideStream of[2];
   bool tried = false;
 };
-constexpr int kSideDevices = 64;
-SideStream g_side[kSideDevices];
+SideStreams g_side[kSideDevices];
 std::mutex g_side_mu;
 
-// null: no such stream on this device (creation failed once); the caller then runs everything on
-// its own stream.
-SideStream* side_stream() {
+// null: no such stream on this device (creation failed once, or the caller's stream is one)
+SideStream* side_stream(hipStream_t main) {
   int dev = -1;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kSideDevices) return nullptr;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(main, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
   std::lock_guard<std::mutex> lock(g_side_mu);
-  SideStream& s = g_side[dev];
+  SideStreams& s = g_side[dev];
   if (!s.tried) {
     s.tried = true;
-    if (hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&s.fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&s.join, hipEventDisableTiming) != hipSuccess) {
-      (void)hipGetLastError();  // the failure is handled here: nothing for the next call to find
-      s.stream = nullptr;
-    }
+    for (SideStream& side : s.of)
+      if (hipStreamCreateWithFlags(&side.stream, hipStreamNonBlocking) != hipSuccess ||
+          hipEventCreateWithFlags(&side.fork, hipEventDisableTiming) != hipSuccess ||
+          hipEventCreateWithFlags(&side.join, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();  // the failure is handled here: nothing for the next call to find
+        side.stream = nullptr;
+      }
   }
-  return s.stream != nullptr ? &s : nullptr;
+  SideStream& side = s.of[status == hipStreamCaptureStatusNone ? 0 : 1];
+  return side.stream != nullptr && s.of[0].stream != main && s.of[1].stream != main ? &side : nullptr;
 }
+}  // namespace
+
+bool branch_pays(int T, int K, int E, int D, int F, int F_shared, int act_dtype, int w_dtype, bool train) {
+  const int64_t reached = (int64_t)T * K < E ? (int64_t)T * K : E;
+  const double features = 6.0 * D * T * ((double)K * F + F_shared);
+  const double weights = 3.0 * D * ((double)reached * F * elem_size(w_dtype) + (double)F_shared * elem_size(act_dtype));
+  const double memory_us = weights / 5e6, products_us = 1.6 * features / (act_dtype == FS2MOE_F32 ? 153e6 : 1200e6);
+  return train ? 2.0 * memory_us + 3.0 * products_us >= 280.0 : memory_us + products_us >= 130.0;
+}
+
+Branch::Branch(bool wanted, void* stream) : main_(stream) {
+  if (wanted) side_ = side_stream(static_cast<hipStream_t>(stream));
+}
+
+void* Branch::stream() const { return side_ != nullptr ? side_->stream : main_; }
+
+int Branch::fork() {
+  if (side_ == nullptr) return FS2MOE_OK;
+  std::lock_guard<std::mutex> lock(g_side_mu);
+  if (hipEventRecord(side_->fork, static_cast<hipStream_t>(main_)) != hipSuccess ||
+      hipStreamWaitEvent(side_->stream, side_->fork, 0) != hipSuccess) {
+    set_error("cannot fork a stream: %s", hipGetErrorString(hipGetLastError()));
+    return FS2MOE_ERR_LAUNCH;
+  }
+  forked_ = true;
+  return FS2MOE_OK;
+}
+
+int Branch::join() {
+  if (!forked_) return FS2MOE_OK;
+  forked_ = false;
+  std::lock_guard<std::mutex> lock(g_side_mu);
+  if (hipEventRecord(side_->join, side_->stream) != hipSuccess ||
+      hipStreamWaitEvent(static_cast<hipStream_t>(main_), side_->join, 0) != hipSuccess) {
+    set_error("cannot join a stream: %s", hipGetErrorString(hipGetLastError()));
+    return FS2MOE_ERR_LAUNCH;
+  }
+  return FS2MOE_OK;
+}
+
+}  // namespace fs2moe
+
+namespace {
 
 // normed: the rows are RMS-normalised on the way into the router (norm_weight may be null), and
 // every stage reads the normalised copy in the workspace.
@@ -212,54 +260,31 @@ int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_
                                          act_dtype, !fused && !act_q && !scaled_stream, normed, act_q,
                                          scaled_stream);
   FS2_REQUIRE(b.total <= need, "forward: internal: the buffers do not fit the workspace");
-  // The shared expert's output is the row the routed outputs are added onto (moe.py:143-150).  With
-  // at most 16 tokens it runs beside the routed path (see SideStream): from the start when it
-  // reads the caller's rows, after the router when it reads the rows the router normalises.
+  // The shared expert's output is the row the routed outputs are added onto (moe.py:143-150).  It depends on the rows
+  // only, so it runs beside the routed path where that pays: from the start when it reads the caller's rows, after the
+  // router when it reads the rows the router normalises.
   // (forking and joining cost the host four calls, about as long as a whole step of a small layer
   // takes it to launch: D 2048 / F 4096, 16 experts, one token 53 -> 100 us with them, where D 4096 /
   // F 8192 goes 137 -> 129 and Scout's D 5120 / F 8192 173 -> 156; so only where the shared expert
   // streams at least 192 MB of weights)
   const bool big_shared = (int64_t)3 * D * F_shared * fs2moe::elem_size(act_dtype) >= (192ll << 20);
-  SideStream* side = (shared && may_fork && T <= 16 && big_shared) ? side_stream() : nullptr;
-  const bool beside = side != nullptr && side->stream != static_cast<hipStream_t>(stream);
+  fs2moe::Branch branch(shared && may_fork && (T <= 16 ? big_shared : fs2moe::branch_pays(T, K, E, D, F, F_shared, act_dtype,
+                                                                                          w_dtype, false)), stream);
+  const bool beside = branch.beside();
   auto shared_on = [&](void* s, const void* rows) {
     return fs2moe_dense_swiglu(rows, shared_gate, shared_up, shared_down, T, D, F_shared, act_dtype,
                                b.shared_h, out, s);
   };
   auto shared_beside = [&]() -> int {
-    hipStream_t main = static_cast<hipStream_t>(stream);
-    {
-      std::lock_guard<std::mutex> lock(g_side_mu);
-      if (hipEventRecord(side->fork, main) != hipSuccess ||
-          hipStreamWaitEvent(side->stream, side->fork, 0) != hipSuccess) {
-        fs2moe::set_error("forward: cannot fork the shared expert's stream: %s",
-                          hipGetErrorString(hipGetLastError()));
-        return FS2MOE_ERR_LAUNCH;
-      }
-    }
-    return shared_on(side->stream, normed ? b.xn : x_in);
-  };
-  // the caller's stream goes on only when the side stream has come this far (called once the
-  // routed experts are on their way, in front of the combine; and on every way out after a fork,
-  // so that the side stream never stays forked from a capturing stream)
-  auto shared_joins = [&]() -> int {
-    std::lock_guard<std::mutex> lock(g_side_mu);
-    if (hipEventRecord(side->join, side->stream) != hipSuccess ||
-        hipStreamWaitEvent(static_cast<hipStream_t>(stream), side->join, 0) != hipSuccess) {
-      fs2moe::set_error("forward: cannot join the shared expert's stream: %s",
-                        hipGetErrorString(hipGetLastError()));
-      return FS2MOE_ERR_LAUNCH;
-    }
-    return FS2MOE_OK;
+    if (int rc = branch.fork()) return rc;
+    return shared_on(branch.stream(), normed ? b.xn : x_in);
   };
   const int64_t planned = fs2moe::planned_rows((int64_t)T * K, E);
-  bool forked = false, shared_done = false;
+  bool shared_done = false;
   // router, dispatch and the routed experts, with the shared expert forked off on the way
   auto routed_path = [&]() -> int {
-    if (beside && !normed) {
-      forked = true;
+    if (beside && !normed)
       if (int rc = shared_beside()) return rc;
-    }
     // (with a few tokens and no rows to copy the router's kernel dispatches as well)
     // (and where the experts stream past up to 16 tokens' rows, their first kernel begins with the selection.  Not beside a
     // shared expert: there the selection's own launch costs nothing, D 5120, F 8192, 16 experts, 5 tokens 238.7 us, 239.2)
@@ -274,10 +299,8 @@ int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_
             b.router_ws, b.router_ws_bytes, b.xe == nullptr ? &disp : nullptr, stream))
       return rc;
     if (normed) x = b.xn;
-    if (beside && normed) {
-      forked = true;
+    if (beside && normed)
       if (int rc = shared_beside()) return rc;
-    }
     if (later.partial != nullptr) {
       // (the shared expert's products go into the routed ones' launches)
       const fs2moe::SharedBeside with = {shared_gate, shared_up, shared_down, F_shared, b.shared_h, out};
@@ -312,12 +335,8 @@ int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_
                                           w_gate, w_up, w_down, s_gate, s_up, s_down, E, D, F, b.max_rows,
                                           planned, act_dtype, w_dtype, b.h, b.ye, T <= 16 ? T : 0, stream);
   };
-  int rc_routed = routed_path();
-  if (forked) {
-    const int rc_join = shared_joins();
-    if (rc_routed == FS2MOE_OK) rc_routed = rc_join;
-  }
-  if (rc_routed != FS2MOE_OK) return rc_routed;
+  if (int rc = routed_path()) return rc;
+  if (int rc = branch.join()) return rc;
   const void* base = nullptr;
   if (shared) {
     if (!beside && !shared_done)

@@ -329,6 +329,40 @@ bool swiglu_train_applies(int32_t dtype, int32_t D, int32_t F, int64_t rows);
 int swiglu_train(const void* x, const int32_t* row_map, const int32_t* counts, const int32_t* offsets, int32_t E,
                  const void* w_gate, const void* w_up, const void* w_down, int32_t D, int32_t F,
                  int64_t rows, int64_t planned, int32_t dtype, void* g, void* u, void* h, void* y, void* stream);
+// Work beside the caller's stream: from fork() on what is given to stream() runs on a stream of the library's own, and
+// join() has the caller's wait for it, so that a caller sees one stream's worth of ordering (and a capturing stream
+// captures both branches).  Where `wanted` is false, or there is no such stream, stream() is the caller's and the other
+// two do nothing.  A branch that is forked is joined on every way out.
+class Branch {
+ public:
+  Branch(bool wanted, void* stream);
+  Branch(const Branch&) = delete;
+  Branch& operator=(const Branch&) = delete;
+  ~Branch() {
+    if (forked_) (void)join();
+  }
+  bool beside() const { return side_ != nullptr; }
+  void* stream() const;
+  int fork();
+  int join();
+
+ private:
+  struct SideStream* side_ = nullptr;
+  void* main_;
+  bool forked_ = false;
+};
+// Whether more than 16 tokens' shared expert pays as a branch beside the routed experts.  What it gains is the ends of the
+// other's launches, where CUs run out of tiles, and its small ones: 2 to 10 % of a call.  What it costs is the host's time
+// for two pairs of record and wait, 30 us a pass: a loss wherever the host is what a call waits for.  So by what the call
+// should take the GPU: the weights at 5 TB/s and the products at 60 % of the pipes' rate, 130 us of them forward; a training
+// step reads them a second time and multiplies three times, 280 us.  us without and with the branch (which estimate):
+//   forward 56, 90 (26: 137 tokens, D 576, F 576, top-4 of 32); 92, 101 (60); 100, 110 (75); 120, 129 (117: 1122, D 704, F
+//   1408, top-4 of 60); 164, 172 (116); 177, 164 (132: 349 of f32, D 768, F 2048, 16); 181, 162 (185: 100, D 2048, F 4096,
+//   16); 192, 179 (179); 280, 276 (253); 421, 394; 782, 747; 2734, 2627 (6000, D 5120, F 8192, 8)
+//   training 342, 422 (255: 256 tokens, D 1024, F 1408, top-4 of 60); 328, 337 (102); 365, 372 (214); 301, 284 (170); 440,
+//   420 (282: 241 of f32); 525, 508 (360: 3001, D 1024, F 1368, top-2 of 16); 440, 419 (347); 771, 741; 1964, 1847; 8602,
+//   8455; and 2950, 2996 (3686, D 4224, F 896, top-4 of 128), the only larger one that lost more than 1 % of forty
+bool branch_pays(int T, int K, int E, int D, int F, int F_shared, int act_dtype, int w_dtype, bool train);
 // Into how many parts the sum over K of a product of `sources` pairs of matrices goes (1: it stays whole), by the
 // planned rows (E 0: the rows).
 int split_parts(int sources, int64_t planned, int E, int K, int N, int dtype);

@@ -7,6 +7,8 @@
 // also takes the dot products that are the combine weights' gradients, the activation's derivative of a
 // step whose rows stay in token order, and the padding of a router matrix whose number of experts is not
 // a multiple of 8.
+#include <algorithm>
+
 #include "common.h"
 
 namespace fs2moe {
@@ -240,7 +242,7 @@ ForwardScratch carve_forward(const Args& a, void* base) {
 
 struct BackwardScratch {
   void *xe, *dye, *dh, *dg, *du, *dxe, *dl, *router, *d_router, *dx_router, *dhs, *dgs, *dus, *dx_shared, *dxn,
-      *norm, *part;
+      *norm, *part, *part_shared;
   float* d_w;
   int64_t norm_bytes, total;
 };
@@ -300,15 +302,19 @@ BackwardScratch carve_backward(const Args& a, void* base) {
   int64_t part = wgrad_plan(r, n, a.E, planned_rows(a), T, a.act_dtype);
   auto parts = [&](int64_t rows, int64_t planned, int E, int F) {
     const int n = split_parts(2, planned, E, F, a.D, a.act_dtype);
-    const int64_t bytes = n > 1 ? (int64_t)n * rows * a.D * 4 : 0;
-    part = bytes > part ? bytes : part;
+    return n > 1 ? (int64_t)n * rows * a.D * 4 : 0;
   };
   const bool want_x = a.dx != nullptr || a.d_norm_weight != nullptr;
-  if (want_x || (a.scale_input && a.d_router != nullptr)) parts(R, planned_rows(a), a.E, a.F);
-  if (want_x && a.F_shared > 0) parts(T, T, 0, a.F_shared);
+  if (want_x || (a.scale_input && a.d_router != nullptr)) part = std::max(part, parts(R, planned_rows(a), a.E, a.F));
   b.part = c.take(part);
+  // (the shared expert's may be at work beside them)
+  b.part_shared = want_x && a.F_shared > 0 ? c.take(parts(T, T, 0, a.F_shared)) : nullptr;
   b.total = c.used;
   return b;
+}
+
+bool beside(const Args& a) {
+  return a.F_shared > 0 && a.T > 16 && branch_pays(a.T, a.K, a.E, a.D, a.F, a.F_shared, a.act_dtype, a.act_dtype, true);
 }
 
 bool sizes_ok(const Args& a) {
@@ -362,14 +368,23 @@ extern "C" int fs2moe_train_forward(const fs2moe_train_args* a, void* stream) {
   FS2_REQUIRE(aligned16(a->out) && aligned16(a->residual), "train_forward: out and residual must be 16-byte aligned");
   const int64_t R = rows_of(*a);
   const void* x = a->normed ? s.xn : a->x;
+  Branch branch(beside(*a), stream);
+  auto shared = [&]() -> int {
+    if (int rc = branch.fork()) return rc;
+    return swiglu_train(x, nullptr, nullptr, nullptr, 0, a->shared_gate, a->shared_up, a->shared_down, a->D,
+                        a->F_shared, a->T, a->T, a->act_dtype, s.gs, s.us, f.hs, a->out, branch.stream());
+  };
+  int rc;
+  if (branch.beside() && !a->normed && (rc = shared())) return rc;
   // (rows that stay in token order need no copy: the router's last kernel counts for the dispatch, a launch fewer; 4096
   // tokens, top-8 of 128, D 2048, F 768 1580 -> 1573 us, 4444, D 1280, F 704 1094 -> 1087)
   DispatchAfterRouter disp{a->tile_m, R, s.counts, s.offsets, s.perm, s.inv_perm, f.disp, f.disp_bytes, nullptr, nullptr, false};
-  int rc = router_then_dispatch(a->x, a->normed ? a->norm_weight : nullptr, a->normed ? a->norm_eps : 0.f,
+  rc = router_then_dispatch(a->x, a->normed ? a->norm_weight : nullptr, a->normed ? a->norm_eps : 0.f,
                                 a->normed ? s.xn : nullptr, a->router_read, a->router_bias, a->T, a->D, a->E, a->K,
                                 a->act_dtype, a->score_fn, a->renormalize, s.idx, s.w, s.logits, f.router,
                                 f.router_bytes, s.xe == nullptr ? &disp : nullptr, stream);
   if (rc) return rc;
+  if (branch.beside() && a->normed && (rc = shared())) return rc;
   if (!disp.done &&
       (rc = fs2moe_dispatch(s.idx, s.w, x, a->T, a->K, a->E, a->D, a->tile_m, a->act_dtype, a->scale_input, R,
                             s.counts, s.offsets, s.perm, s.inv_perm, s.xe, f.disp, f.disp_bytes, stream)))
@@ -385,13 +400,9 @@ extern "C" int fs2moe_train_forward(const fs2moe_train_args* a, void* stream) {
                       a->w_down, a->D, a->F, R, planned_rows(*a), a->act_dtype, s.g, s.u, mapped ? s.h : f.h, ye,
                       stream);
   if (rc) return rc;
-  const void* base = nullptr;
-  if (a->F_shared > 0) {
-    rc = swiglu_train(x, nullptr, nullptr, nullptr, 0, a->shared_gate, a->shared_up, a->shared_down, a->D,
-                      a->F_shared, a->T, a->T, a->act_dtype, s.gs, s.us, f.hs, a->out, stream);
-    if (rc) return rc;
-    base = a->out;
-  }
+  if ((rc = branch.join())) return rc;
+  if (a->F_shared > 0 && !branch.beside() && (rc = shared())) return rc;
+  const void* base = a->F_shared > 0 ? a->out : nullptr;
   if (a->residual != nullptr)
     return fs2moe_combine_residual(ye, s.inv_perm, s.idx, s.w, base, a->residual, a->T, a->K, a->D,
                                    a->act_dtype, a->scale_input ? 0 : 1, a->out, stream);
@@ -423,6 +434,20 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
   const int64_t R = rows_of(*a);
   const void* x = a->normed ? s.xn : a->x;
   int rc;
+  // the shared expert, which depends on what the forward pass kept and on dout only
+  Branch branch(beside(*a), stream);
+  auto shared = [&]() -> int {
+    if (int rc = branch.fork()) return rc;
+    void* on = branch.stream();
+    if (int rc = fs2moe_grouped_gemm(a->dout, nullptr, nullptr, nullptr, a->shared_down, FS2MOE_W_IN_OUT, 1, D, Fs, T, dt,
+                                     b.dhs, on))
+      return rc;
+    if (int rc = fs2moe_swiglu_backward(s.gs, s.us, b.dhs, T, Fs, dt, b.dhs, b.dgs, b.dus, on)) return rc;
+    if (!want_x) return FS2MOE_OK;
+    return gemm_sum(b.dgs, a->shared_gate, b.dus, a->shared_up, FS2MOE_W_IN_OUT, nullptr, nullptr, 0, Fs, D, T, T, dt,
+                    b.dx_shared, b.part_shared, on);
+  };
+  if (branch.beside() && (rc = shared())) return rc;
   // rows in expert order: the output gradients, with those of output-side weights that are applied to them, and in
   // token order the copies for the weight gradients
   const bool mapped = in_token_order(*a);
@@ -477,16 +502,8 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
     if ((rc = router_backward_ld(s.logits, s.idx, s.w, b.d_w, T, E, K, score_fn, a->renormalize, dt, b.dl, Ep, stream)))
       return rc;
   }
-  // the shared expert
-  if (Fs > 0) {
-    if ((rc = fs2moe_grouped_gemm(a->dout, nullptr, nullptr, nullptr, a->shared_down, FS2MOE_W_IN_OUT, 1, D, Fs, T, dt,
-                                  b.dhs, stream)) ||
-        (rc = fs2moe_swiglu_backward(s.gs, s.us, b.dhs, T, Fs, dt, b.dhs, b.dgs, b.dus, stream)))
-      return rc;
-    if (want_x && (rc = gemm_sum(b.dgs, a->shared_gate, b.dus, a->shared_up, FS2MOE_W_IN_OUT, nullptr, nullptr, 0, Fs,
-                                 D, T, T, dt, b.dx_shared, b.part, stream)))
-      return rc;
-  }
+  if ((rc = branch.join())) return rc;
+  if (Fs > 0 && !branch.beside() && (rc = shared())) return rc;
   // all weight gradients
   WgradRequest r[8];
   const int n = requests(*a, s, b, r);

@@ -5,6 +5,8 @@ routing artefact bit for bit and the output on a sample of tokens (a token costs
 the CPU), plus properties that do not depend on size.
 """
 
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -646,6 +648,59 @@ def test_decode_steps_with_a_shared_expert_in_the_same_launches(gpu_device, toke
     ye, _ = _abi.grouped_swiglu(x, dsp.counts, dsp.offsets, wg, wu, wd, e, row_map=dsp.perm, rows_per_expert=tokens)
     assert torch.equal(call(), _abi.combine(ye, dsp.inv_perm, idx, w, _abi.dense_swiglu(x, *sh), True))
     assert len(launched(call)) == 4
+
+
+@pytest.mark.parametrize("normed", [False, True])
+def test_shared_expert_on_a_stream_beside_the_routed_ones(gpu_device, normed):
+    """A call large enough for the branch: the stages' bits, from two threads with streams of their own at once, and
+    replayed from a graph with calls in between."""
+    _say("shared expert beside", normed)
+    t, d, f, e, k = 400, 768, 2048, 8, 2
+    g = torch.Generator().manual_seed(3)
+    mk = lambda *s, scale=1.0: (scale * torch.randn(*s, generator=g)).to(gpu_device)  # noqa: E731
+    xs, router, norm_w = [mk(t, d) for _ in range(3)], mk(d, e, scale=0.3), mk(d)
+    wg, wu, wd = mk(e * d, f, scale=0.05), mk(e * d, f, scale=0.05), mk(e * f, d, scale=0.05)
+    sh = (mk(f, d, scale=0.05), mk(f, d, scale=0.05), mk(d, f, scale=0.05))
+
+    def call(x):
+        return _abi.forward(x, router, None, wg, wu, wd, e, k, shared=sh, score_fn=_abi.SCORE_SOFTMAX, scale_input=False,
+                            norm=(norm_w, 1e-6) if normed else None)
+
+    def stages(x):
+        if normed:
+            x, idx, w, _ = _abi.router_topk_norm(x, norm_w, 1e-6, router, None, k, _abi.SCORE_SOFTMAX)
+        else:
+            idx, w, _ = _abi.router_topk(x, router, None, k, _abi.SCORE_SOFTMAX)
+        dsp = _abi.dispatch(idx, w, x, e, 16, False, gather=True)
+        ye, _ = _abi.grouped_swiglu(dsp.xe, dsp.counts, dsp.offsets, wg, wu, wd, e)
+        return _abi.combine(ye, dsp.inv_perm, idx, w, _abi.dense_swiglu(x, *sh), True)
+
+    want = [stages(x) for x in xs]
+    torch.cuda.synchronize()
+    results = {}
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            results[i] = [call(xs[i]) for _ in range(20)]
+            torch.cuda.current_stream().synchronize()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    for i in range(2):
+        assert all(torch.equal(out, want[i]) for out in results[i]), i
+    buf = xs[2].clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call(buf)
+    for i in (2, 0, 1, 2):
+        buf.copy_(xs[i])
+        graph.replay()
+        eager = call(xs[i])
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[i]) and torch.equal(eager, want[i]), i
 
 
 def test_expert_major_copy_of_the_router_follows_the_parameter(gpu_device):
