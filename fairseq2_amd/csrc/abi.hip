@@ -330,10 +330,10 @@ int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_
     if (scaled_stream)
       return fs2moe::grouped_swiglu_scaled_rows(x, b.perm, b.row_w, b.counts, b.offsets, w_gate, w_up,
                                                 w_down, E, D, F, b.max_rows, planned, b.h, b.ye, T, stream);
-    // (a token takes an expert at most once: with up to 16 tokens no expert has more rows than that)
+    // (a token takes an expert at most once, so no expert has more rows than that)
     return fs2moe::grouped_swiglu_planned(fused ? x : b.xe, fused ? b.perm : nullptr, b.counts, b.offsets,
                                           w_gate, w_up, w_down, s_gate, s_up, s_down, E, D, F, b.max_rows,
-                                          planned, act_dtype, w_dtype, b.h, b.ye, T <= 16 ? T : 0, stream);
+                                          planned, act_dtype, w_dtype, b.h, b.ye, T, stream);
   };
   if (int rc = routed_path()) return rc;
   if (int rc = branch.join()) return rc;

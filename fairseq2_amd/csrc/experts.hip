@@ -318,7 +318,10 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
   // (tiles of 64 x 64 are counted in 31 bits too)
   const bool counted = (rows_bound / 64 + groups + 1) * ((N + 63) / 64) <= 0x7fffffffll;
   constexpr bool SINGLE = !DUAL && CAN_TAIL;
-  switch (counted ? half_tiles::pick(DUAL, CAN_TAIL, g.rows_to_plan(rows_bound), groups, K, N, num_blocks) : 0) {
+  constexpr bool WHOLE_ROWS = DUAL && CAN_TAIL && !KEEP_GU && BLAYOUT == FS2MOE_W_IN_OUT;
+  switch (counted ? half_tiles::pick(DUAL, CAN_TAIL, g.rows_to_plan(rows_bound), groups, K, N, num_blocks,
+                                     WHOLE_ROWS ? g.most : 0)
+                  : 0) {
     case 1:
       if constexpr (SINGLE)
         return launch_half<64, 64, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
@@ -330,6 +333,11 @@ static int launch_dma(const void* a, const int32_t* row_map, int K, const void* 
     case 3:
       return launch_half<128, 128, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
                                                                     num_blocks, mean_rows, stream);
+    case 4:
+      if constexpr (WHOLE_ROWS)
+        return launch_half<64, 256, DUAL, BLAYOUT, KEEP_GU, TWO_SRC>(a, row_map, K, b0, b1, s0, s1, c, N, g, what,
+                                                                     num_blocks, mean_rows, stream);
+      break;
   }
   // The variant for any K also stores rows that do not begin on lines as L2 wants them, which counts for more than its
   // selects at every load where stores are a large part of the work: three results, or few units.  us with the variant
@@ -946,7 +954,8 @@ static int grouped_swiglu_impl(const void* xe, const int32_t* row_map, const int
     return FS2MOE_ERR_UNSUPPORTED;
   }
   if (max_rows == 0) return FS2MOE_OK;
-  const Groups g{counts, offsets, E, 0, (int)planned};
+  Groups g{counts, offsets, E, 0, (int)planned};
+  g.most = rows_hint;
   return launch_glu<FS2MOE_W_IN_OUT>(xe, row_map, g, max_rows, w_gate, w_up, w_down, D, F, act_dtype,
                                      h, ye, static_cast<hipStream_t>(stream), rows_hint, row_w);
 }

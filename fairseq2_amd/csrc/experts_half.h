@@ -1,5 +1,5 @@
-// Grouped GEMM on tiles of 128 x 128, 64 x 128 or 64 x 64 (rows x "virtual" channels: gate and up channels of 64
-// each when DUAL), for launches whose 256 x 256 tiles (experts_dma.h, experts_mx.h) would leave CUs idle: bf16 rows
+// Grouped GEMM on tiles of 128 x 128, 64 x 128, 64 x 64 or 64 x 256 (rows x "virtual" channels: gate and up channels of
+// half as many each when DUAL), for launches whose 256 x 256 tiles (experts_dma.h, experts_mx.h) would leave CUs idle: bf16 rows
 // against bf16 or e4m3 weights, block-scaled e4m3 rows against e4m3 weights.
 //
 // What bounds it: with few tiles a CU's time is its tiles' bytes over what it takes in.  Four waves bring a CU 47 GB/s
@@ -63,8 +63,23 @@ constexpr int smem_bytes(int BM, int BNV, int layout) {
 inline int64_t once_rows(int BM) { return BM / 2; }
 constexpr uint32_t NOWHERE = 0xfffffff0u;      // an offset past any buffer's end
 
+// Gate/up of several rounds of tiles where no expert has more than 64 rows: tiles of 64 x 256, as many as the throughput
+// kernel's and of the same weights, in pieces of rows as long (256 bytes).  A CU that takes weights for a few rows waits
+// for memory: here two of three stages of 40 KB are on their way, loaded by every wave, there one unit of as much, loaded by four.
+// Narrower tiles would fill more CUs, but their pieces of 128 bytes cost memory 10 % of its rate (64 tokens, top-6 of 64,
+// D 4096, F 1024 281 -> 314 us).  Experts of more rows would have their weights read once for each row block (200 tokens of
+// that layer by a popularity law 300 -> 335), and long sums stay where they were (40 tokens, top-1 of 16, D 5120, F 8192
+// 674 -> 682).  us of the layer on the throughput kernel and on these, three layers and inputs in turn, evenly loaded and by
+// a popularity law:
+//   24 tokens, top-8 of 128, D 2048, F 768   194, 190; 83.4, 82.4      64       215, 212; 110.6, 106.9
+//   48, top-4 of 60, D 1024, F 1408          110, 105; 58.1, 55.6      33, top-6 of 60, D 640, F 1600  86.5, 83.6; 49.6, 48.7
+//   60, top-8 of 64, D 768, F 2048           131, 128; 79.6, 77.1      64, top-6 of 32, D 1280, F 704  66.5, 64.4; 68.7, 66.2
+//   64, top-6 of 64, D 4096, F 1024          281, 282; 238, 238        20, top-2 of 8, D 4096, F 14336 497, 494; 480, 463
+// (the last and 33 tokens: 64 x 128 by the model of rounds instead of the throughput kernel)
+inline bool whole_rows(int most_rows, int K) { return most_rows >= 1 && most_rows <= 64 && K <= 4096; }
+
 // Which of these tiles a launch takes: 0 none (the throughput kernel), else the smallest whose tiles are about
-// one a CU: 1 64 x 64 (single products), 2 64 x 128, 3 128 x 128.
+// one a CU: 1 64 x 64 (single products), 2 64 x 128, 3 128 x 128; 4 64 x 256 (whole_rows).
 // us, throughput kernel and 1, 2, 3 (single products but for the last two, which are gate/up and down):
 //   80 rows, K 3200, N 1408              42 against 19, 23, 28     (5, 44, 22, 11 tiles)
 //   755 rows, K 1408, N 576              25 against 12, 14, 18
@@ -80,8 +95,8 @@ constexpr uint32_t NOWHERE = 0xfffffff0u;      // an offset past any buffer's en
 //   48 and 100, top-8 of 128 by one, D 2048, F 768                           96.2, 90.4; 130, 117
 // Gate/up within 70 to 83 % of the model's time: evenly 11 % faster to 2 % slower on small tiles (24 shapes), by a
 // popularity law 15 % faster to 18 % slower; within 85 to 88 % 1 % faster to 12 % slower at D 2048 and above.
-// bf16: matrices and rows of bf16, not codes.
-inline int pick(bool dual, bool bf16, int64_t rows, int groups, int K, int N, int cus) {
+// bf16: matrices and rows of bf16, not codes.  most: as for whole_rows.
+inline int pick(bool dual, bool bf16, int64_t rows, int groups, int K, int N, int cus, int most = 0) {
   // Of the experts' rows only the device knows how they are spread: the planned ones (Groups), less what blocks of 16
   // pad them by, equally loaded.
   const int64_t real = rows > 15ll * groups ? rows - 15ll * groups : rows;
@@ -98,6 +113,7 @@ inline int pick(bool dual, bool bf16, int64_t rows, int groups, int K, int N, in
   if (bf16 && !dual && tiles(64, 64) <= room) return 1;
   if (tiles(64, dual ? 64 : 128) <= room) return 2;
   if (tiles(128, dual ? 64 : 128) <= room) return 3;
+  if (dual && groups > 0 && whole_rows(most, K)) return 4;
   // Several rounds of tiles of a few rows: rounds of the throughput kernel (1 us per 64 k and 6 per tile, us) against
   // rounds of these (0.4 and 4), neither faster than memory delivers half of the experts' weights (5.2 TB/s; with few
   // tokens or a skewed load not all experts have rows), and a margin for what that leaves out.
@@ -163,7 +179,8 @@ __global__ __launch_bounds__(half_tiles::THREADS, 2) void glu_gemm_half_kernel(
   constexpr bool CODES = FP8 || MX;        // weights as e4m3 tiles with channel scales S0, S1
   static_assert(!KEEP_GU || (DUAL && !CODES), "the products are kept by the bf16 gate/up kernel only");
   static_assert(!TWO_SRC || (!DUAL && !CODES), "two sources: one bf16 matrix each");
-  static_assert((BM == 64 || BM == 128) && (BNV == 128 || (BNV == 64 && !DUAL && !CODES)),
+  static_assert((BM == 64 || BM == 128) && (BNV == 128 || (BNV == 64 && !DUAL && !CODES) ||
+                                            (BNV == 256 && BM == 64 && DUAL && !CODES)),
                 "tiles that the loads are cut for");
   constexpr int A_BYTES = BM * ROW_BYTES, B_BYTES = weight_bytes(BNV, BLAYOUT);
   constexpr int STAGE_BYTES = stage_bytes(BM, BNV, BLAYOUT);
@@ -250,12 +267,15 @@ __global__ __launch_bounds__(half_tiles::THREADS, 2) void glu_gemm_half_kernel(
   // ---- the stream of stages into LDS: stage u of the block goes to slot u % STAGES
   const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem_raw;
   // The wave's pieces of 1 KB: rows 8 wave .. 8 wave + 7 of the activations and, 64 further on, 8 more; of the
-  // weights likewise (with DUAL the first of the gate and the second of the up matrix).  A lane's place in piece i:
+  // weights likewise (with DUAL the first half of them of the gate, the second of the up matrix).  A lane's place in piece i:
   uint32_t pa[PA], pb[PB];
   // chunk of the row's 128 bytes that the lane fetches (the same for both pieces), of activations and (out, in)
   // weights; k row of (in, out) weights in the stage
   const int kc = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);
   constexpr int KROWS = 1024 / BROW, KCHUNKS = BROW / 16;  // rows and chunks of a piece of (in, out) weights
+  // (piece i is the wave's i % PM-th of matrix i / PM)
+  constexpr int PM = DUAL && !FP8 ? PB / 2 : PB;
+  auto piece = [&](int i) { return wave + 8 * (i % PM); };
   auto k_key = [](int k) { return BROW == 128 ? ((k >> 1) & 1) << 2 : (k & 3) << 2; };
   int ld_tile = 0, ld_ku = 0, ld_slot = 0;
   const uint8_t* ld_b[2] = {B0, B0};
@@ -305,18 +325,18 @@ __global__ __launch_bounds__(half_tiles::THREADS, 2) void glu_gemm_half_kernel(
           pb[i] = group < N / 16 ? (uint32_t)group * (uint32_t)nkb * 1024u + (uint32_t)(r * 64 + c * 16) : NOWHERE;
         } else {
           // a piece is 8 channel rows of 128 k, from two tiles
-          const int P = DUAL ? wave : wave + 8 * i, r = 8 * (P & 1) + (lane >> 3);
+          const int P = piece(i), r = 8 * (P & 1) + (lane >> 3);
           const int group = t.n0 / 16 + (P >> 1);
           pb[i] = group < N / 16 ? ((uint32_t)group * (uint32_t)nkb + (uint32_t)(kc >> 2)) * 1024u +
                                        (uint32_t)(r * 64 + (kc & 3) * 16)
                                  : NOWHERE;
         }
       } else if constexpr (KN) {
-        const int k = KROWS * (DUAL ? wave : wave + 8 * i) + lane / KCHUNKS, key = k_key(k);
+        const int k = KROWS * piece(i) + lane / KCHUNKS, key = k_key(k);
         const int col = t.n0 + ((lane % KCHUNKS) ^ key) * 8;
         pb[i] = col < N ? ((uint32_t)k * (uint32_t)N + (uint32_t)col) * 2u : NOWHERE;
       } else {
-        const int ch = t.n0 + 8 * (DUAL ? wave : wave + 8 * i) + (lane >> 3);
+        const int ch = t.n0 + 8 * piece(i) + (lane >> 3);
         pb[i] = ch < N ? (uint32_t)ch * (uint32_t)Kdim * 2u + (uint32_t)kc * 16u : NOWHERE;
       }
     }
@@ -338,13 +358,13 @@ __global__ __launch_bounds__(half_tiles::THREADS, 2) void glu_gemm_half_kernel(
       const uint8_t* src = second ? reinterpret_cast<const uint8_t*>(S0) : A;
       buffer_to_lds<16>(src + (size_t)ku * ROW_BYTES, kc * (16 / ASIZE) < left ? pa[i] : NOWHERE, at);
     } else {
-      const uint8_t* src = TWO_SRC ? ld_b[second ? 1 : 0] : ld_b[DUAL ? (FP8 ? wave >> 2 : i) : 0];
+      const uint8_t* src = TWO_SRC ? ld_b[second ? 1 : 0] : ld_b[DUAL ? (FP8 ? wave >> 2 : i / PM) : 0];
       if constexpr (FP8) {
         buffer_to_lds<16, ONCE>(src + (size_t)ku * 1024, left > 0 ? pb[i] : NOWHERE, at);
       } else if constexpr (MX) {
         buffer_to_lds<16, ONCE>(src + (size_t)ku * 2048, left > 0 ? pb[i] : NOWHERE, at);
       } else if constexpr (KN) {
-        const int k = KROWS * (DUAL ? wave : wave + 8 * i) + lane / KCHUNKS;
+        const int k = KROWS * piece(i) + lane / KCHUNKS;
         buffer_to_lds<16, ONCE>(src + (size_t)ku * KU * N * 2, k < left ? pb[i] : NOWHERE, at);
       } else {
         buffer_to_lds<16, ONCE>(src + (size_t)ku * ROW_BYTES, kc * 8 < left ? pb[i] : NOWHERE, at);

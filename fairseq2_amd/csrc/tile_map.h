@@ -16,6 +16,8 @@ struct Groups {
   // host: whether the launch may load its weights past the caches (load_once); it does where few rows an expert make
   // most tiles their expert's only row block
   int once_past_cache = 0;
+  // host: how many rows an expert has at most, where the caller knows it (0: it does not)
+  int most = 0;
   int64_t rows_to_plan(int64_t bound) const { return counts != nullptr && planned > 0 ? planned : bound; }
 };
 

@@ -707,6 +707,32 @@ def test_pair_and_two_sources_on_every_tile_size(gpu_device, counts, n):
         assert torch.equal(ye[sl], ye2[sl]) and torch.equal(h[sl], h2[sl]), f"expert {i} without keeping"
 
 
+# Gate/up of experts that are known to have at most 64 rows, on tiles as wide as the throughput kernel's: the same bits as
+# from that kernel.  One stage of 64 k and fewer, as many as the ring's and more with a remainder; channels within a
+# tile, past its half and past its end.
+@pytest.mark.parametrize("d", [8, 64, 136, 200, 840])
+@pytest.mark.parametrize("f", [1032, 1096, 1408])
+def test_pair_of_experts_of_at_most_64_rows(gpu_device, d, f):
+    _say("at most 64 rows", d, f)
+    counts = [1, 32, 0, 33, 64, 63, 17, 5] + [3] * 72
+    g = torch.Generator().manual_seed(d + f)
+    c, off, rows, row_map = _tile_case(counts, g, gpu_device)
+    e = len(counts)
+    make = lambda *shape: (0.1 * torch.randn(*shape, generator=g)).to(torch.bfloat16).to(gpu_device)  # noqa: E731
+    x, wg, wu, wd = make(500, d), make(e * d, f), make(e * d, f), make(e * f, d)
+
+    def call(hint):
+        return _abi.grouped_swiglu(x, c, off, wg, wu, wd, e, row_map=row_map, rows_per_expert=hint)
+
+    (ye, h), (ye0, h0) = call(64), call(0)
+    for i in range(e):
+        sl = slice(int(off[i]), int(off[i]) + counts[i])
+        assert torch.equal(h[sl], h0[sl]) and torch.equal(ye[sl], ye0[sl]), f"expert {i}"
+    names = launched(lambda: call(64)), launched(lambda: call(0))
+    assert names[0][0].startswith("glu_gemm_half_kernel<64, 256"), names
+    assert names[1][0].startswith("glu_gemm_bf16_dma_kernel"), names
+
+
 # The f32 products take tiles of 64 x 64, on which two groups of waves share the sum over K (the pair one), or of 128 x
 # 128 (the pair 128 x 64) by the size of the buffers: the same bits.  Rows on both sides of 32, 64 and 128, experts
 # without any, K within a chunk of 32, past its quarters and over several, N off the tiles' channels.
