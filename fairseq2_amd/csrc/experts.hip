@@ -197,19 +197,21 @@ static int launch_f32(const void* a, const void* b0, const void* b1, const void*
                       const char* what, hipStream_t stream, int parts = 1) {
   const int groups = g.counts ? g.E : 0;
   const bool small = !f32t::large_tiles(DUAL, g.rows_to_plan(rows_bound), groups, N, 256);
-  const int bm = small ? 64 : 128, bn = small || DUAL ? 64 : 128;
+  const bool flat = small && f32t::flat_tiles(DUAL, g.rows_to_plan(rows_bound), groups, N, parts, 256);
+  const int bm = flat ? 32 : small ? 64 : 128, bn = small || DUAL ? 64 : 128;
   const int64_t m_tiles = rows_bound / bm + groups + 1;
   const int nt = (N + bn - 1) / bn;
   if (m_tiles * nt > 0x7ffffff0ll) {
     set_error("%s: grid too large", what);
     return FS2MOE_ERR_UNSUPPORTED;
   }
-  // (small tiles of one product: two groups of waves, f32t::threads)
+  // (small tiles of one product and flat ones: two groups of waves, f32t::threads)
   constexpr int groups_small = DUAL ? 1 : 2;
-  auto k = small ? glu_gemm_f32_kernel<DUAL, 1, 1, BLAYOUT, groups_small>
-                 : glu_gemm_f32_kernel<DUAL, 2, DUAL ? 1 : 2, BLAYOUT, 1>;
+  auto k = flat    ? glu_gemm_f32_kernel<DUAL, 1, 1, BLAYOUT, 2, 1>
+           : small ? glu_gemm_f32_kernel<DUAL, 1, 1, BLAYOUT, groups_small>
+                   : glu_gemm_f32_kernel<DUAL, 2, DUAL ? 1 : 2, BLAYOUT, 1>;
   hipLaunchKernelGGL(k, dim3((unsigned)((m_tiles * nt + 7) / 8 * 8), (unsigned)parts),
-                     dim3(f32t::threads(small ? groups_small : 1)), 0, stream,
+                     dim3(flat ? f32t::threads(2, 1) : f32t::threads(small ? groups_small : 1)), 0, stream,
                      static_cast<const float*>(a), static_cast<const float*>(b0),
                      static_cast<const float*>(b1), static_cast<const float*>(a2),
                      static_cast<float*>(c), static_cast<float*>(g_keep), static_cast<float*>(u_keep), K,

@@ -4,8 +4,8 @@
 // What bounds them: the matrix pipe (64 clocks per instruction and SIMD, 157 TFLOP/s nominal, 154 in a
 // large product of the vendor's library), and, with few tiles, their number against 256 CUs.  A chunk is
 // 32 k; two chunks are on their way from memory in two register sets while a third is multiplied, LDS
-// holds two (one barrier per chunk), and a block is 4 waves (or 8) on a 64 x 64 or 4 on a 128 x 128 tile, several of the
-// small ones' blocks to a CU (f32t::large_tiles).  What a
+// holds two (one barrier per chunk), and a block is 4 waves (or 8) on a 64 x 64, 4 on a 32 x 64 or 4 on a 128 x 128 tile,
+// several of the smaller ones' blocks to a CU (f32t::large_tiles, flat_tiles).  What a
 // wave does besides multiplying is dealt out one instruction behind each product (Walk::run): as phases,
 // i.e. stores, barrier, loads, reads, products, the same tiles reach 132 TFLOP/s with every SIMD full
 // and 95 with one wave on each, whether one chunk or four are in flight; dealt out 149-154 and 107.
@@ -40,7 +40,7 @@ constexpr int BK = 32;
 // 80 -> 74; 60 experts of 80, the pair of D 768, F 2000, 575 -> 547.  Not for two products at once: what the sums leave
 // of registers and LDS lets two such blocks share a CU instead of three smaller ones (60 experts of 17 rows, K 576, N
 // 1760, 66 -> 80 us).
-constexpr int threads(int groups) { return 256 * groups; }
+constexpr int threads(int groups, int wm = 2) { return 128 * wm * groups; }
 
 // Products on tiles of 128 x 128 (two products at once: 128 rows x 64 channels of each) instead of 64 x 64: where their
 // rounds of tiles take less time.  In hundredths of a us per 32 k, on full rounds: a small tile 54, of two products 103, a
@@ -76,6 +76,28 @@ inline bool large_tiles(bool dual, int64_t rows, int groups, int N, int cus) {
   const int64_t small = rounds(blocks(64) * ((N + 63) / 64)) * (dual ? 103 : 54);
   const int64_t large = rounds(blocks(128) * (dual ? (N + 63) / 64 : (N + 127) / 128));
   return large * 195 < small && large >= (groups == 0 ? 2 : 4);
+}
+
+// Where large_tiles says no: products on tiles of 32 x 64 (two groups of two waves), whose rounds are half as long, so that
+// what is empty of a last one costs less, and an expert's last row block is half as empty.  In hundredths of a us per 32 k
+// on full rounds: 29, of two products 58 (their weights go through LDS for half as many rows).  Experts of up to 32 rows
+// have as many tiles of either kind: one product takes the flat ones where a CU has at most one, as the busiest experts
+// have two, two products where there are more, since a tile of 64 rows then leaves half of its waves idle.  us on tiles of
+// 64 x 64 and on these, the layer and (last) a training step:
+//   1000 tokens, top-2 of 8, D 512, F 1408, training          356, 332    (280 tiles on 256 CUs down, 790 gate/up)
+//   1000, top-1 of 8, D 1024, F 2048                          188, 171, 496, 482    4000, top-1 of 8, D 576, F 640 340, 329
+//   100, top-2 of 8 by a law of 1.1, D 512, F 1408            67.3, 59.1            300, 16, D 768, F 2048 91.9, 80.8
+//   64, top-4 of 60, D 1024, F 1024                           200, 185, 653, 639    200, top-6 of 128, D 1024, F 1792 586, 561
+// and where the rule says no: gate/up of 1500, top-6 of 64, D 640, F 1728 569, 595; of 2000, top-2 of 8, D 1024, F 1408
+// 331, 345; down of 200, top-6 of 128 586, 593.
+inline bool flat_tiles(bool dual, int64_t rows, int groups, int N, int parts, int cus) {
+  const int64_t real = groups > 0 && rows > 15ll * groups ? rows - 15ll * groups : rows;
+  const int g = groups > 0 ? groups : 1;
+  const int64_t nt = (int64_t)((N + 63) / 64) * parts;
+  if (real <= 32ll * g) return dual ? g * nt > cus : g * nt <= cus;
+  auto blocks = [&](int bm) { return g + (real - (int64_t)g * (bm / 2)) / bm; };
+  auto rounds = [&](int64_t tiles) { return (tiles + cus - 1) / cus; };
+  return rounds(blocks(32) * nt) * (dual ? 58 : 29) < rounds(blocks(64) * nt) * (dual ? 103 : 54);
 }
 
 // what a load through a row map reads past the end (not const: a global address)
@@ -157,18 +179,18 @@ struct Operand {
   }
 };
 
-// The walk over k of one tile: waves 2 x 2, each 32 FM rows x 32 FN channels of each of NB matrices.
+// The walk over k of one tile: waves WM x 2, each 32 FM rows x 32 FN channels of each of NB matrices.
 // acc[b][fn][fm] is the transposed 32 x 32 tile (lane: row lr, channels 8 q + 4 lk + 0..3 in 4 q ..).
 // With two sources the second pair follows the first in the same accumulators.
 // A_MAPPED: a_map gives the rows of the k-major A.
 // HALVES: two sums, over the first and the second half of every chunk's k, added at the end; the groups' (GROUPS 2), or
 // both of each wave.
 template <int NB, int FM, int FN, bool A_KMAJOR, bool B_KMAJOR, bool A_MAPPED = false, int GROUPS = 1,
-          bool HALVES = true>
+          bool HALVES = true, int WM = 2>
 struct Walk {
   static_assert(HALVES || GROUPS == 1, "two groups of waves take a half each");
   static constexpr int CHAINS = HALVES && GROUPS == 1 ? 2 : 1;  // sums that a wave keeps
-  static constexpr int BM = 64 * FM, BN = 64 * FN, THREADS = threads(GROUPS);
+  static constexpr int BM = 32 * WM * FM, BN = 64 * FN, THREADS = threads(GROUPS, WM);
   using OpA = Operand<BM, A_KMAJOR, THREADS>;
   using OpB = Operand<BN, B_KMAJOR, THREADS>;
   static constexpr int BUF_BYTES = OpA::BYTES + NB * OpB::BYTES;
@@ -179,8 +201,8 @@ struct Walk {
 
   // The wave's rows and channels of the tile, and which share of a chunk's k it takes.  (Waves w and w + 4 share a
   // SIMD: with a tile of up to 32 rows every SIMD has a wave that multiplies.)
-  static __device__ __forceinline__ int wave_m(int wave) { return GROUPS == 2 ? wave >> 2 : wave & 1; }
-  static __device__ __forceinline__ int wave_n(int wave) { return GROUPS == 2 ? wave & 1 : wave >> 1; }
+  static __device__ __forceinline__ int wave_m(int wave) { return WM == 1 ? 0 : GROUPS == 2 ? wave >> 2 : wave & 1; }
+  static __device__ __forceinline__ int wave_n(int wave) { return WM == 1 || GROUPS == 2 ? wave & 1 : wave >> 1; }
   static __device__ __forceinline__ int wave_group(int wave) { return GROUPS == 2 ? (wave >> 1) & 1 : 0; }
 
   struct Source {
@@ -279,8 +301,10 @@ struct Walk {
       const Chunk next = chunk_at(st + 3);
       if constexpr (decltype(multiply)::value) {
         constexpr int BEHIND = PRODUCTS / STEPS * (STEPS - 1);  // products in front of the barrier
-        constexpr int EVERY = BEHIND / (2 * PIECES);
-        static_assert(EVERY >= 1 && EVERY * 2 * PIECES <= BEHIND, "a product per store and load");
+        // (with too few products for both in front of it the loads go on behind it)
+        constexpr bool BOTH = BEHIND >= 2 * PIECES;
+        constexpr int EVERY = BOTH ? BEHIND / (2 * PIECES) : 1;
+        static_assert(BOTH || (PIECES <= BEHIND && 2 * PIECES <= PRODUCTS), "a product per store and load");
 #pragma unroll
         for (int s = 0; s < STEPS; ++s) {
           if (s + 1 < STEPS) {
@@ -301,7 +325,7 @@ struct Walk {
                   f32x16& sum = acc[CHAINS == 2 ? s / (STEPS / 2) : 0][m][fn][fm];
                   sum = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[s & 1][m][fn][j], xf[s & 1][fm][j], sum, 0, 0, 0);
                   const int done = (((s * 4 + j) * NB + m) * FN + fn) * FM + fm;
-                  if (done < BEHIND && done % EVERY == 0) {
+                  if ((!BOTH || done < BEHIND) && done % EVERY == 0) {
                     const int o = done / EVERY;
                     if (o < PIECES)
                       store(a, b, buf ^ 1, o);
@@ -348,7 +372,7 @@ struct Walk {
       // the second group's sums onto the first's, through the chunks' LDS (the barrier: each chunk's last step reads the
       // next one's first fragments, the last chunk's too)
       constexpr int REGS = NB * FN * FM * 16;
-      static_assert(4 * REGS * 64 * 4 <= SMEM_BYTES, "the sums of four waves fit the chunks' buffers");
+      static_assert(2 * WM * REGS * 64 * 4 <= SMEM_BYTES, "the second group's sums fit the chunks' buffers");
       float* at = reinterpret_cast<float*>(smem) + (wm * 2 + wn) * (REGS * 64) + lane;
       auto exchange = [&](auto store) {
 #pragma unroll
@@ -390,17 +414,17 @@ struct Walk {
 // C = A B_e (+ A2 B2_e), or with DUAL C = SiLU(A B0_e) * (A B1_e), the two products left in g_keep and
 // u_keep where those are given.  A block per tile; BLAYOUT as for the bf16 kernels.  With several rows of blocks
 // (single products) each takes a part of the sum over K, and C is [gridDim.y][rows][N].
-template <bool DUAL, int FM, int FN, int BLAYOUT, int GROUPS>
-__global__ __launch_bounds__(f32t::threads(GROUPS), 2 * GROUPS) void glu_gemm_f32_kernel(
+template <bool DUAL, int FM, int FN, int BLAYOUT, int GROUPS, int WM = 2>
+__global__ __launch_bounds__(f32t::threads(GROUPS, WM), 2 * GROUPS) void glu_gemm_f32_kernel(
     const float* __restrict__ A, const float* __restrict__ B0, const float* __restrict__ B1,
     const float* __restrict__ A2, float* __restrict__ C, float* __restrict__ g_keep,
     float* __restrict__ u_keep, int K, int N, Groups g, int n_tiles) {
   constexpr int NB = DUAL ? 2 : 1;
   constexpr bool KN = BLAYOUT == FS2MOE_W_IN_OUT;
-  using W = f32t::Walk<NB, FM, FN, false, KN, false, GROUPS>;
+  using W = f32t::Walk<NB, FM, FN, false, KN, false, GROUPS, true, WM>;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[W::SMEM_BYTES];
   int e, row0, row_end, nt;
-  if (!locate_tile_by_xcd<W::BM, W::THREADS>(g, n_tiles, e, row0, row_end, nt)) return;
+  if (!locate_tile_by_xcd<W::BM, W::THREADS>(g, n_tiles, reinterpret_cast<int32_t*>(smem), e, row0, row_end, nt)) return;
   e = __builtin_amdgcn_readfirstlane(e);
   row0 = __builtin_amdgcn_readfirstlane(row0);
   row_end = __builtin_amdgcn_readfirstlane(row_end);

@@ -99,9 +99,10 @@ __device__ __forceinline__ bool locate_tile(const Groups& g, int mt, int& e, int
 // The tile of block blockIdx.x when the grid's tiles (m-tiles of BM rows x n_tiles, channel block minor)
 // are cut into eight runs of neighbours, one per XCD (block b runs on XCD b % 8, each with its own L2):
 // the blocks an XCD holds at a time then share their rows and their expert's weights.  All THREADS
-// threads of the block must call it; the grid is a multiple of 8.  false: no tile for this block.
+// threads of the block must call it; the grid is a multiple of 8.  scratch: 4 + THREADS / 32 words of LDS, free again
+// afterwards.  false: no tile for this block.
 template <int BM, int THREADS>
-__device__ __forceinline__ bool locate_tile_by_xcd(const Groups& g, int n_tiles, int& e, int& row0,
+__device__ __forceinline__ bool locate_tile_by_xcd(const Groups& g, int n_tiles, int32_t* scratch, int& e, int& row0,
                                                    int& row_end, int& nt) {
   const int idx = blockIdx.x >> 3, xcd = blockIdx.x & 7;
   if (g.counts == nullptr) {
@@ -115,7 +116,8 @@ __device__ __forceinline__ bool locate_tile_by_xcd(const Groups& g, int n_tiles,
     return true;
   }
   constexpr int ROUNDS = FS2MOE_MAX_EXPERTS / THREADS, WAVES = THREADS / 64;
-  __shared__ int s_wave[2][WAVES], s_found[4];
+  int32_t* s_found = scratch;
+  int32_t(*s_wave)[WAVES] = reinterpret_cast<int32_t(*)[WAVES]>(scratch + 4);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // tiles in all, then the one of this block (the experts one per thread)
   int cnt[ROUNDS], excl[ROUNDS], carried = 0;
@@ -157,6 +159,7 @@ __device__ __forceinline__ bool locate_tile_by_xcd(const Groups& g, int n_tiles,
   row0 = s_found[1];
   row_end = s_found[2];
   nt = t - mt * n_tiles;
+  __syncthreads();  // (scratch has been read)
   return true;
 }
 

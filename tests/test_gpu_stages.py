@@ -769,6 +769,40 @@ def test_f32_products_are_the_same_on_every_tile_size(gpu_device, k, n, layout):
     assert torch.equal(dense[0], dense[2][:32]) and torch.equal(dense[1], dense[2][:33])
 
 
+# Tiles of 32 x 64 and of 64 x 64 by the rows and experts of a launch: the same bits, in both orientations of a matrix, for
+# one product and two.
+@pytest.mark.parametrize("k", [8, 32, 40, 72, 200])
+@pytest.mark.parametrize("n", [1024, 1000])
+def test_f32_products_on_flat_tiles(gpu_device, k, n):
+    rows = [1, 16, 17, 33, 65, 0, 130, 31]
+    _say("f32 flat tiles", k, n)
+    g, many = torch.Generator(gpu_device).manual_seed(k + n), 128
+    rnd = lambda *s: torch.randn(*s, generator=g, device=gpu_device)  # noqa: E731
+    x, w, wu, wd = rnd(3000, k), rnd(many * k, n), rnd(many * k, n), rnd(many * n, k)
+    wt = w.reshape(many, k, n).transpose(1, 2).contiguous().reshape(-1, k)
+    kind = lambda name: name.rsplit(", ", 2)[-1] == "1>"  # noqa: E731
+    seen, first = set(), None
+    for e, total in ((8, 368), (8, 1000), (many, 3000)):
+        counts = torch.tensor(rows + [0] * (e - 8), dtype=torch.int32, device=gpu_device)
+        offsets = torch.zeros(e + 1, dtype=torch.int32, device=gpu_device)
+        offsets[1:] = torch.cumsum((counts + 15) // 16 * 16, 0)
+        lo, got = offsets.tolist(), []
+        assert lo[-1] <= total
+        names = launched(lambda: got.extend([
+            _abi.grouped_gemm(x[:total], w[: e * k], _abi.W_IN_OUT, counts, offsets, e),
+            _abi.grouped_gemm(x[:total], wt[: e * n], _abi.W_OUT_IN, counts, offsets, e),
+            _abi.grouped_swiglu(x[:total], counts, offsets, w[: e * k], wu[: e * k], wd[: e * n], e)[1]]))
+        assert all(m.startswith("glu_gemm_f32_kernel<") for m in names), names
+        seen |= {(m.split("<")[1].split(",")[0], kind(m)) for m in names[:3]}
+        out = [torch.cat([o[lo[i] : lo[i] + r] for i, r in enumerate(rows)]) for o in got]
+        first = first or out
+        assert all(torch.equal(a, b) for a, b in zip(out, first)), (e, total)
+        assert torch.equal(out[0], out[1])
+    assert seen == {(dual, flat) for dual in ("true", "false") for flat in (True, False)}, seen
+    ref = torch.cat([x[lo[i] : lo[i] + r].double() @ w[i * k : (i + 1) * k].double() for i, r in enumerate(rows)])
+    assert_output_close(first[0], ref.cpu(), "fp32")
+
+
 # Weights of more than 320 MB are loaded past the caches where one block reads them (all experts), others through them (the
 # first 8 of these experts alone): the same bits from every kernel that has both kinds of loads.  Which kernels a call
 # takes, and which loads, is asked for: where "past the caches" stands among their template arguments, by name.
