@@ -171,11 +171,25 @@ Branch::Branch(bool wanted, void* stream) : main_(stream) {
   if (wanted) side_ = side_stream(static_cast<hipStream_t>(stream));
 }
 
-void* Branch::stream() const { return side_ != nullptr ? side_->stream : main_; }
+void* Branch::stream() const { return forked_ ? side_->stream : main_; }
+
+namespace {
+// The capture that a stream is part of, 0 where it captures nothing.
+unsigned long long capture_of(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) (void)hipGetLastError();
+  return status == hipStreamCaptureStatusNone ? 0 : id;
+}
+}  // namespace
 
 int Branch::fork() {
   if (side_ == nullptr) return FS2MOE_OK;
   std::lock_guard<std::mutex> lock(g_side_mu);
+  // (a stream that one capture has forked to stays part of it until that capture ends, so that another one under way at
+  // the same time cannot have it: its branch is then work of the caller's stream)
+  const unsigned long long held = capture_of(side_->stream);
+  if (held != 0 && held != capture_of(static_cast<hipStream_t>(main_))) return FS2MOE_OK;
   if (hipEventRecord(side_->fork, static_cast<hipStream_t>(main_)) != hipSuccess ||
       hipStreamWaitEvent(side_->stream, side_->fork, 0) != hipSuccess) {
     set_error("cannot fork a stream: %s", hipGetErrorString(hipGetLastError()));

@@ -5,6 +5,7 @@ routing artefact bit for bit and the output on a sample of tokens (a token costs
 the CPU), plus properties that do not depend on size.
 """
 
+import ctypes
 import threading
 
 import numpy as np
@@ -701,6 +702,54 @@ def test_shared_expert_on_a_stream_beside_the_routed_ones(gpu_device, normed):
         eager = call(xs[i])
         torch.cuda.synchronize()
         assert torch.equal(out, want[i]) and torch.equal(eager, want[i]), i
+
+
+def test_two_captures_at_once_of_layers_with_a_branch(gpu_device):
+    """The second of two captures under way at the same time cannot fork to the stream that the first one holds: its
+    shared expert is recorded on its own stream (a chain of nodes), the first one's beside the routed experts."""
+    _say("two captures")
+    with open("/proc/self/maps") as maps:  # the copy of the runtime that this process runs on
+        hip = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    t, d, f, e, k = 400, 768, 2048, 8, 2
+    g = torch.Generator().manual_seed(3)
+    mk = lambda *s, scale=1.0: (scale * torch.randn(*s, generator=g)).to(gpu_device)  # noqa: E731
+    xs, router = [mk(t, d) for _ in range(2)], mk(d, e, scale=0.3)
+    wg, wu, wd = mk(e * d, f, scale=0.05), mk(e * d, f, scale=0.05), mk(e * f, d, scale=0.05)
+    sh = (mk(f, d, scale=0.05), mk(f, d, scale=0.05), mk(d, f, scale=0.05))
+    call = lambda x: _abi.forward(x, router, None, wg, wu, wd, e, k, shared=sh, score_fn=_abi.SCORE_SOFTMAX,  # noqa: E731
+                                  scale_input=False)
+    want = [call(x) for x in xs]
+    streams = [torch.cuda.Stream() for _ in xs]
+    handle = lambda s: ctypes.c_void_p(s.cuda_stream)  # noqa: E731
+    relaxed = 2
+    torch.cuda.synchronize()
+    for s, x in zip(streams, xs):  # memory for the captures
+        with torch.cuda.stream(s):
+            call(x), call(x)
+    torch.cuda.synchronize()
+    got, graphs, edges = [], [ctypes.c_void_p() for _ in xs], []
+    for s, x in zip(streams, xs):
+        assert hip.hipStreamBeginCapture(handle(s), relaxed) == 0
+        with torch.cuda.stream(s):
+            got.append([call(x), call(x)])
+    for s, graph in zip(streams, graphs):
+        assert hip.hipStreamEndCapture(handle(s), ctypes.byref(graph)) == 0
+        nodes, links = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0
+        assert hip.hipGraphGetEdges(graph, None, None, ctypes.byref(links)) == 0
+        edges.append(links.value - (nodes.value - 1))
+    assert edges[0] > 0 == edges[1], "edges beyond those of a chain of its nodes"
+    for s, graph, outs, right in zip(streams, graphs, got, want):
+        runs = ctypes.c_void_p()
+        assert hip.hipGraphInstantiate(ctypes.byref(runs), graph, None, None, ctypes.c_size_t(0)) == 0
+        for out in outs:
+            out.zero_()
+        torch.cuda.synchronize()
+        for _ in range(2):
+            assert hip.hipGraphLaunch(runs, handle(s)) == 0
+            s.synchronize()
+            assert all(torch.equal(out, right) for out in outs)
+        assert hip.hipGraphExecDestroy(runs) == 0 and hip.hipGraphDestroy(graph) == 0
 
 
 def test_expert_major_copy_of_the_router_follows_the_parameter(gpu_device):
