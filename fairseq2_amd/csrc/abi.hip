@@ -159,12 +159,12 @@ SideStream* side_stream(hipStream_t main) {
 }
 }  // namespace
 
-bool branch_pays(int T, int K, int E, int D, int F, int F_shared, int act_dtype, int w_dtype, bool train) {
+bool branch_pays(int T, int K, int E, int D, int F, int F_shared, int act_dtype, int w_dtype, bool late, bool backward) {
   const int64_t reached = (int64_t)T * K < E ? (int64_t)T * K : E;
   const double features = 6.0 * D * T * ((double)K * F + F_shared);
   const double weights = 3.0 * D * ((double)reached * F * elem_size(w_dtype) + (double)F_shared * elem_size(act_dtype));
   const double memory_us = weights / 5e6, products_us = 1.6 * features / (act_dtype == FS2MOE_F32 ? 153e6 : 1200e6);
-  return train ? 2.0 * memory_us + 3.0 * products_us >= 280.0 : memory_us + products_us >= 130.0;
+  return backward ? memory_us + 2.0 * products_us >= 200.0 : memory_us + products_us >= (late ? 350.0 : 130.0);
 }
 
 Branch::Branch(bool wanted, void* stream) : main_(stream) {
@@ -283,7 +283,7 @@ int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_
   // streams at least 192 MB of weights)
   const bool big_shared = (int64_t)3 * D * F_shared * fs2moe::elem_size(act_dtype) >= (192ll << 20);
   fs2moe::Branch branch(shared && may_fork && (T <= 16 ? big_shared : fs2moe::branch_pays(T, K, E, D, F, F_shared, act_dtype,
-                                                                                          w_dtype, false)), stream);
+                                                                                          w_dtype, normed, false)), stream);
   const bool beside = branch.beside();
   auto shared_on = [&](void* s, const void* rows) {
     return fs2moe_dense_swiglu(rows, shared_gate, shared_up, shared_down, T, D, F_shared, act_dtype,

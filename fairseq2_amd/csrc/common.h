@@ -354,16 +354,23 @@ class Branch {
 };
 // Whether more than 16 tokens' shared expert pays as a branch beside the routed experts.  What it gains is the ends of the
 // other's launches, where CUs run out of tiles, and its small ones: 2 to 10 % of a call.  What it costs is the host's time
-// for two pairs of record and wait, 30 us a pass: a loss wherever the host is what a call waits for.  So by what the call
-// should take the GPU: the weights at 5 TB/s and the products at 60 % of the pipes' rate, 130 us of them forward; a training
-// step reads them a second time and multiplies three times, 280 us.  us without and with the branch (which estimate):
+// for two pairs of record and wait, 30 us a pass and more after other work: a loss wherever the host is what a call waits
+// for.  So by what the pass should take the GPU: the weights at 5 TB/s and the products at 60 % of the pipes' rate, 130 us of
+// them forward, 200 backward, which multiplies twice.  us without and with the branch (which estimate):
 //   forward 56, 90 (26: 137 tokens, D 576, F 576, top-4 of 32); 92, 101 (60); 100, 110 (75); 120, 129 (117: 1122, D 704, F
 //   1408, top-4 of 60); 164, 172 (116); 177, 164 (132: 349 of f32, D 768, F 2048, 16); 181, 162 (185: 100, D 2048, F 4096,
 //   16); 192, 179 (179); 280, 276 (253); 421, 394; 782, 747; 2734, 2627 (6000, D 5120, F 8192, 8)
-//   training 342, 422 (255: 256 tokens, D 1024, F 1408, top-4 of 60); 328, 337 (102); 365, 372 (214); 301, 284 (170); 440,
-//   420 (282: 241 of f32); 525, 508 (360: 3001, D 1024, F 1368, top-2 of 16); 440, 419 (347); 771, 741; 1964, 1847; 8602,
-//   8455; and 2950, 2996 (3686, D 4224, F 896, top-4 of 128), the only larger one that lost more than 1 % of forty
-bool branch_pays(int T, int K, int E, int D, int F, int F_shared, int act_dtype, int w_dtype, bool train);
+//   training, backward pass 520, 508 (230: 3001 tokens, D 1024, F 1368, top-2 of 16); 526, 492 (252: 263 of f32, D 1024, F
+//   2048, top-2 of 8); 409, 416 (185: 700, D 1024, F 4096, top-2 of 8, both passes; as a first pass 520, 590)
+// late: a pass whose branch brings less or costs more, 350 us forward.  That is one behind a router that normalises the
+// rows, whose branch begins with the experts' launches, which stream weights as fast alone where a call is mostly that:
+//   199.6, 203.4 (191: 100 tokens, D 2048, F 4096, top-2 of 16); 205.6, 207.5 (211: 200); 249.6, 256.1 (322: 600, D 2048, F
+//   1408, top-6 of 64); 372, 366 (395: 40, D 4096, F 8192, top-2 of 8); 375, 363 (453: 577 of f32, D 640, F 1728, top-6 of
+//   64); 506, 491 (600: 1854, D 2496, F 4352, top-2 of 8); 475, 462 (549: 5000, D 1024, F 4096, top-2 of 8); 838, 819 (1194)
+// and the forward pass of a training step, whose host time is not hidden in a first pass or where a program waits:
+//   508, 496, but as a first pass 620, 665 (129: the 3001 tokens above); 775, 764 and 862, 903 (267: 1800, D 2048, F 2048,
+//   top-2 of 16); 493, 489 and 617, 705 (152: 900, D 1536, F 3072, top-2 of 8); 495, 467 and 596, 621 (149: 263 of f32)
+bool branch_pays(int T, int K, int E, int D, int F, int F_shared, int act_dtype, int w_dtype, bool late, bool backward);
 // Into how many parts the sum over K of a product of `sources` pairs of matrices goes (1: it stays whole), by the
 // planned rows (E 0: the rows).
 int split_parts(int sources, int64_t planned, int E, int K, int N, int dtype);

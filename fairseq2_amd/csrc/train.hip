@@ -270,6 +270,11 @@ int requests(const Args& a, const Saved& s, const BackwardScratch& b, WgradReque
   if (a.d_router != nullptr && Ep != a.E) r[n - 1].dw = b.d_router;
   return n;
 }
+bool beside(const Args& a, bool backward) {
+  return a.F_shared > 0 && a.T > 16 &&
+         branch_pays(a.T, a.K, a.E, a.D, a.F, a.F_shared, a.act_dtype, a.act_dtype, true, backward);
+}
+
 BackwardScratch carve_backward(const Args& a, void* base) {
   Carver c{static_cast<uint8_t*>(base)};
   const int64_t R = rows_of(a), sz = elem_size(a.act_dtype), T = a.T;
@@ -306,15 +311,13 @@ BackwardScratch carve_backward(const Args& a, void* base) {
   };
   const bool want_x = a.dx != nullptr || a.d_norm_weight != nullptr;
   if (want_x || (a.scale_input && a.d_router != nullptr)) part = std::max(part, parts(R, planned_rows(a), a.E, a.F));
-  b.part = c.take(part);
-  // (the shared expert's may be at work beside them)
-  b.part_shared = want_x && a.F_shared > 0 ? c.take(parts(T, T, 0, a.F_shared)) : nullptr;
+  // (the shared expert's have a place of their own where they may be at work beside the others)
+  const int64_t part_shared = want_x && a.F_shared > 0 ? parts(T, T, 0, a.F_shared) : 0;
+  const bool apart = beside(a, true);
+  b.part = c.take(apart ? part : std::max(part, part_shared));
+  b.part_shared = apart ? c.take(part_shared) : b.part;
   b.total = c.used;
   return b;
-}
-
-bool beside(const Args& a) {
-  return a.F_shared > 0 && a.T > 16 && branch_pays(a.T, a.K, a.E, a.D, a.F, a.F_shared, a.act_dtype, a.act_dtype, true);
 }
 
 bool sizes_ok(const Args& a) {
@@ -368,7 +371,7 @@ extern "C" int fs2moe_train_forward(const fs2moe_train_args* a, void* stream) {
   FS2_REQUIRE(aligned16(a->out) && aligned16(a->residual), "train_forward: out and residual must be 16-byte aligned");
   const int64_t R = rows_of(*a);
   const void* x = a->normed ? s.xn : a->x;
-  Branch branch(beside(*a), stream);
+  Branch branch(beside(*a, false), stream);
   auto shared = [&]() -> int {
     if (int rc = branch.fork()) return rc;
     return swiglu_train(x, nullptr, nullptr, nullptr, 0, a->shared_gate, a->shared_up, a->shared_down, a->D,
@@ -435,7 +438,7 @@ extern "C" int fs2moe_train_backward(const fs2moe_train_args* a, void* stream) {
   const void* x = a->normed ? s.xn : a->x;
   int rc;
   // the shared expert, which depends on what the forward pass kept and on dout only
-  Branch branch(beside(*a), stream);
+  Branch branch(beside(*a, true), stream);
   auto shared = [&]() -> int {
     if (int rc = branch.fork()) return rc;
     void* on = branch.stream();

@@ -264,10 +264,11 @@ int fs2moe_combine_residual(const void* ye, const int32_t* inv_perm, const int32
  *   workspace   at least fs2moe_forward_workspace_bytes(...) bytes, 256-byte aligned
  *   out [T, D] act_dtype (out; must not alias x; may alias residual unless there is a shared expert)
  * With a large shared expert (192 MB of weights or more) and at most 16 tokens, or with more tokens
- * where the whole call should take about 150 us or more, its kernels run on a stream of the library's
- * own, forked from `stream` and joined back to it inside the call (events; under stream capture both
- * branches are captured): to the caller the call is ordered on `stream` as before.  The training calls
- * do the same from about 400 us a step on.
+ * where the whole call should take about 150 us or more (350 with rows that it normalises), its
+ * kernels run on a stream of the library's own, forked from `stream` and joined back to it inside the
+ * call (events; under stream capture both branches are captured, unless another capture under way at
+ * the same time has the library's stream): to the caller the call is ordered on `stream` as before.
+ * The training calls do the same, forward from about 350 us on, backward from about 250.
  */
 int64_t fs2moe_forward_workspace_bytes(int32_t T, int32_t D, int32_t E, int32_t K, int32_t F,
                                        int32_t F_shared, int32_t tile_m, int32_t act_dtype);

@@ -656,7 +656,7 @@ def test_shared_expert_on_a_stream_beside_the_routed_ones(gpu_device, normed):
     """A call large enough for the branch: the stages' bits, from two threads with streams of their own at once, and
     replayed from a graph with calls in between."""
     _say("shared expert beside", normed)
-    t, d, f, e, k = 400, 768, 2048, 8, 2
+    t, d, f, e, k = 1200 if normed else 400, 768, 2048, 8, 2
     g = torch.Generator().manual_seed(3)
     mk = lambda *s, scale=1.0: (scale * torch.randn(*s, generator=g)).to(gpu_device)  # noqa: E731
     xs, router, norm_w = [mk(t, d) for _ in range(3)], mk(d, e, scale=0.3), mk(d)
