@@ -250,6 +250,10 @@ int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_
   FS2_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0,
               "forward: workspace must be 256-byte aligned");
   if (T == 0) return FS2MOE_OK;
+  // (here for all of its kernels: those of a decode step may be the routed experts' own launches)
+  FS2_REQUIRE(!shared || (fs2moe::aligned16(shared_gate) && fs2moe::aligned16(shared_up) &&
+                          fs2moe::aligned16(shared_down) && fs2moe::aligned16(out)),
+              "forward: the shared expert's matrices and out must be 16-byte aligned");
 
   // rows are read through the permutation where the expert kernels can (see fs2moe_grouped_swiglu)
   const bool fused = !scale_input && fs2moe::swiglu_gathers_rows(act_dtype, w_dtype, D, F,

@@ -182,6 +182,25 @@ def test_argument_errors_are_reported_without_touching_the_gpu(lib):
     assert lib.fs2moe_dispatch_workspace_bytes(-1, 8, 128) == -1
 
 
+@pytest.mark.parametrize("tokens", [1, 5, 16, 17])
+@pytest.mark.parametrize("normed", [0, 1])
+@pytest.mark.parametrize("name", ["shared_gate", "shared_up", "shared_down", "out"])
+def test_layer_calls_refuse_an_unaligned_shared_expert(lib, name, normed, tokens):
+    """Whichever launches its products go into, and before anything is launched."""
+    a = _abi.ForwardArgs()
+    a.T, a.D, a.E, a.K, a.F, a.F_shared, a.tile_m = tokens, 640, 8, 2, 256, 256, 16
+    a.act_dtype = a.w_dtype = _abi.BF16
+    a.score_fn, a.normed = _abi.SCORE_SOFTMAX, normed
+    for i, field in enumerate(("x", "router", "w_gate", "w_up", "w_down", "shared_gate", "shared_up", "shared_down",
+                               "workspace", "out")):
+        setattr(a, field, 0x1000000 * (i + 1))
+    need = lib.fs2moe_forward_norm_workspace_bytes if normed else lib.fs2moe_forward_workspace_bytes
+    a.workspace_bytes = need(a.T, a.D, a.E, a.K, a.F, a.F_shared, a.tile_m, a.act_dtype)
+    setattr(a, name, getattr(a, name) + 8)
+    rc = lib.fs2moe_forward_call(a, None)
+    assert rc == -1 and b"16-byte aligned" in lib.fs2moe_last_error(), lib.fs2moe_last_error()
+
+
 def test_backward_entry_points_report_argument_errors_without_touching_the_gpu(lib):
     fake, other = ctypes.c_void_p(0x1000), ctypes.c_void_p(0x2000)
     err = lib.fs2moe_last_error
