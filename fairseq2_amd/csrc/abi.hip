@@ -118,11 +118,19 @@ namespace fs2moe {
 
 // Streams of the library's own, two per device: one for callers' streams that run their work, one for those that capture
 // it, so that a capture never finds another thread's work on the stream.  Default priority, created on the first use on a
-// device and kept; the events are reused, which is why the record-and-wait pairs are taken under a lock: between one
-// thread's record and its wait another thread's record of the same event would replace what is waited for.
+// device and kept.  Callers' streams that are independent stay so: what a side stream waits for, everything behind it on
+// that stream waits for too, so a caller's stream gets it only where nothing of another one's is left on it, and a call has
+// it for itself from its branch's beginning to its end; another's shared expert then runs on its own stream.  (Handed to
+// whoever came next: of 7 and 9 pairs of streams that one did not have to wait for the other on, no call on one ended before
+// a call queued on the other, which was held up for 40 ms; now on 6 and 6, the side stream being in one queue of the hardware
+// with the others.)
 struct SideStream {
   hipStream_t stream = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
+  // the caller's stream of the last branch, whose order covers all that is on this one; where its handle is another
+  // stream's by now, a branch of that one may wait for what the destroyed one had left to do
+  hipStream_t owner = nullptr;
+  bool taken = false;
 };
 namespace {
 constexpr int kSideDevices = 64;
@@ -133,15 +141,41 @@ struct SideStreams {
 SideStreams g_side[kSideDevices];
 std::mutex g_side_mu;
 
-// null: no such stream on this device (creation failed once, or the caller's stream is one)
-SideStream* side_stream(hipStream_t main) {
-  int dev = -1;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kSideDevices) return nullptr;
+// The capture that a stream is part of, 0 where it captures nothing.
+unsigned long long capture_of(hipStream_t stream) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(main, &status) != hipSuccess) {
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) (void)hipGetLastError();
+  return status == hipStreamCaptureStatusNone ? 0 : id;
+}
+
+// Whether all work of a stream is done.  (Asked for in the relaxed mode: another thread's capture may forbid it.)
+bool idle(hipStream_t stream) {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  const bool done = hipStreamQuery(stream) == hipSuccess;
+  if (!done) (void)hipGetLastError();
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  return done;
+}
+
+// For a branch of the caller's stream `main`, until given back; null: there is none to have (creation failed once, it would
+// order callers' streams, or the caller's stream is one).
+SideStream* take_side_stream(hipStream_t main) {
+  if (main == hipStreamPerThread) return nullptr;  // (one handle for a stream of each thread)
+  int dev = -1, of = -1;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipGetDevice(&dev) != hipSuccess || hipStreamGetDevice(main, &of) != hipSuccess ||
+      hipStreamIsCapturing(main, &status) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
+  // (the events would be of the current device, which a launch on another one's stream does not need)
+  if (dev != of || dev < 0 || dev >= kSideDevices) return nullptr;
+  const bool captures = status != hipStreamCaptureStatusNone;
   std::lock_guard<std::mutex> lock(g_side_mu);
   SideStreams& s = g_side[dev];
   if (!s.tried) {
@@ -154,8 +188,19 @@ SideStream* side_stream(hipStream_t main) {
         side.stream = nullptr;
       }
   }
-  SideStream& side = s.of[status == hipStreamCaptureStatusNone ? 0 : 1];
-  return side.stream != nullptr && s.of[0].stream != main && s.of[1].stream != main ? &side : nullptr;
+  SideStream& side = s.of[captures ? 1 : 0];
+  if (side.stream == nullptr || side.taken || s.of[0].stream == main || s.of[1].stream == main) return nullptr;
+  if (captures) {
+    // (a stream that a capture has forked to stays part of it until that capture ends, and another stream of the same
+    // capture is a chain of nodes of its own)
+    const unsigned long long held = capture_of(side.stream);
+    if (held != 0 && (side.owner != main || held != capture_of(main))) return nullptr;
+  } else if (side.owner != main && !idle(side.stream)) {
+    return nullptr;
+  }
+  side.owner = main;
+  side.taken = true;
+  return &side;
 }
 }  // namespace
 
@@ -168,28 +213,20 @@ bool branch_pays(int T, int K, int E, int D, int F, int F_shared, int act_dtype,
 }
 
 Branch::Branch(bool wanted, void* stream) : main_(stream) {
-  if (wanted) side_ = side_stream(static_cast<hipStream_t>(stream));
+  if (wanted) side_ = take_side_stream(static_cast<hipStream_t>(stream));
+}
+
+Branch::~Branch() {
+  (void)join();
+  if (side_ == nullptr) return;
+  std::lock_guard<std::mutex> lock(g_side_mu);
+  side_->taken = false;
 }
 
 void* Branch::stream() const { return forked_ ? side_->stream : main_; }
 
-namespace {
-// The capture that a stream is part of, 0 where it captures nothing.
-unsigned long long capture_of(hipStream_t stream) {
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  unsigned long long id = 0;
-  if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) (void)hipGetLastError();
-  return status == hipStreamCaptureStatusNone ? 0 : id;
-}
-}  // namespace
-
 int Branch::fork() {
   if (side_ == nullptr) return FS2MOE_OK;
-  std::lock_guard<std::mutex> lock(g_side_mu);
-  // (a stream that one capture has forked to stays part of it until that capture ends, so that another one under way at
-  // the same time cannot have it: its branch is then work of the caller's stream)
-  const unsigned long long held = capture_of(side_->stream);
-  if (held != 0 && held != capture_of(static_cast<hipStream_t>(main_))) return FS2MOE_OK;
   if (hipEventRecord(side_->fork, static_cast<hipStream_t>(main_)) != hipSuccess ||
       hipStreamWaitEvent(side_->stream, side_->fork, 0) != hipSuccess) {
     set_error("cannot fork a stream: %s", hipGetErrorString(hipGetLastError()));
@@ -202,7 +239,6 @@ int Branch::fork() {
 int Branch::join() {
   if (!forked_) return FS2MOE_OK;
   forked_ = false;
-  std::lock_guard<std::mutex> lock(g_side_mu);
   if (hipEventRecord(side_->join, side_->stream) != hipSuccess ||
       hipStreamWaitEvent(static_cast<hipStream_t>(main_), side_->join, 0) != hipSuccess) {
     set_error("cannot join a stream: %s", hipGetErrorString(hipGetLastError()));
@@ -217,8 +253,8 @@ namespace {
 
 // normed: the rows are RMS-normalised on the way into the router (norm_weight may be null), and
 // every stage reads the normalised copy in the workspace.
-// may_fork: the shared expert of a few tokens may run on the library's side stream (not for the
-// entry point that must create nothing).
+// may_fork: the shared expert may run on the library's side stream (not for the entry point that must
+// create nothing).
 int forward_impl(bool may_fork, bool normed, const void* x_in, const void* norm_weight, float norm_eps,
                  const void* residual, const void* router, const float* router_bias,
                  const void* w_gate, const void* w_up, const void* w_down, const float* s_gate,

@@ -331,17 +331,15 @@ int swiglu_train(const void* x, const int32_t* row_map, const int32_t* counts, c
                  int64_t rows, int64_t planned, int32_t dtype, void* g, void* u, void* h, void* y, void* stream);
 // Work beside the caller's stream: from fork() on what is given to stream() runs on a stream of the library's own, and
 // join() has the caller's wait for it, so that a caller sees one stream's worth of ordering (and a capturing stream
-// captures both branches).  Where `wanted` is false, or there is no such stream, stream() is the caller's and the other
-// two do nothing.  A branch that is forked is joined on every way out.  beside() is what decides where in the order of
-// calls its work stands; stream() is asked for behind fork(), which leaves it the caller's where another capture has ours.
+// captures both branches).  Where `wanted` is false, or there is no such stream to have without ordering callers' streams,
+// stream() is the caller's and the other two do nothing: which it is, beside() says from the beginning, so that it decides
+// where in the order of calls the branch's work stands.  A branch that is forked is joined on every way out.
 class Branch {
  public:
   Branch(bool wanted, void* stream);
   Branch(const Branch&) = delete;
   Branch& operator=(const Branch&) = delete;
-  ~Branch() {
-    if (forked_) (void)join();
-  }
+  ~Branch();
   bool beside() const { return side_ != nullptr; }
   void* stream() const;
   int fork();

@@ -263,12 +263,16 @@ int fs2moe_combine_residual(const void* ye, const int32_t* inv_perm, const int32
  *               0: they multiply the experts' output rows
  *   workspace   at least fs2moe_forward_workspace_bytes(...) bytes, 256-byte aligned
  *   out [T, D] act_dtype (out; must not alias x; may alias residual unless there is a shared expert)
- * With a large shared expert (192 MB of weights or more) and at most 16 tokens, or with more tokens
- * where the whole call should take about 150 us or more (350 with rows that it normalises), its
- * kernels run on a stream of the library's own, forked from `stream` and joined back to it inside the
- * call (events; under stream capture both branches are captured, unless another capture under way at
- * the same time has the library's stream): to the caller the call is ordered on `stream` as before.
- * The training calls do the same, forward from about 350 us on, backward from about 250.
+ * The kernels of a shared expert may run on a stream of the library's own, forked from `stream` and
+ * joined back to it inside the call (events; under stream capture both branches are captured): with at
+ * most 16 tokens where it has 192 MB of weights or more, with more tokens where the pass is estimated
+ * (weights at 5 TB/s and products at 60 % of the matrix pipes' rate) at 130 us or more, 350 with rows
+ * that it normalises.  The training calls do the same, forward from an estimated 350 us on, backward
+ * from 200.  To the caller the call is ordered on `stream` as before, and it orders no other streams:
+ * where another stream's call still has the library's stream (or another capture has, or another stream
+ * of the same capture), or `stream` is hipStreamPerThread or not of the current device, all kernels run
+ * on `stream`, with the same results.  (As any stream, the library's may share one of the runtime's few
+ * hardware queues with others, which then run in turn with it.)
  */
 int64_t fs2moe_forward_workspace_bytes(int32_t T, int32_t D, int32_t E, int32_t K, int32_t F,
                                        int32_t F_shared, int32_t tile_m, int32_t act_dtype);

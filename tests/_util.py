@@ -139,3 +139,36 @@ def launched(run) -> list[str]:
     names = [re.search(r"fs2moe::(\w+(?:<[^()]*(?:\([^()]*\)[^()]*)*>)?)\(", e.name) for e in kernels]
     assert names and all(names), [e.name for e in kernels]
     return [n.group(1).replace("fs2moe::", "") for n in names]
+
+
+def hip_runtime():
+    """The copy of the HIP runtime that this process runs on."""
+    import ctypes
+
+    with open("/proc/self/maps") as maps:
+        return ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+
+
+def recorded(stream, run):
+    """``run()`` recorded on ``stream`` instead of run: the graph's handle, its nodes and its edges.  What it allocates has
+    to be there already (a call before, its results dropped)."""
+    import ctypes
+
+    hip, graph = hip_runtime(), ctypes.c_void_p()
+    handle = ctypes.c_void_p(stream.cuda_stream)
+    relaxed = 2
+    torch.cuda.synchronize()
+    assert hip.hipStreamBeginCapture(handle, relaxed) == 0
+    try:
+        with torch.cuda.stream(stream):
+            run()
+    finally:
+        status = hip.hipStreamEndCapture(handle, ctypes.byref(graph))
+    assert status == 0, status
+    n, m = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    assert hip.hipGraphGetEdges(graph, None, None, ctypes.byref(m)) == 0
+    nodes, tails, heads = ((ctypes.c_void_p * max(1, k.value))() for k in (n, m, m))
+    assert hip.hipGraphGetNodes(graph, nodes, ctypes.byref(n)) == 0
+    assert m.value == 0 or hip.hipGraphGetEdges(graph, tails, heads, ctypes.byref(m)) == 0
+    return graph, list(nodes)[: n.value], list(zip(tails, heads))[: m.value]

