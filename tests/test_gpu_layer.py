@@ -808,6 +808,52 @@ def test_branches_leave_callers_streams_independent(gpu_device, t, d, f, dtype):
     assert apart and beside
 
 
+@pytest.mark.parametrize("what", ["normalised rows", "training forward", "training backward"])
+def test_calls_that_have_a_branch(gpu_device, what):
+    """The passes for which the rule says so fork (a node of a graph of one waits for two others), and have the same bits
+    replayed."""
+    from fairseq2_amd import autograd as A
+
+    _say("has a branch", what)
+    # (backward: both rows' gradients in parts, each with scratch of its own)
+    t, d, f = (300, 512, 4096) if what == "training backward" else (1200, 768, 2048)
+    e, k = 8, 2
+    g = torch.Generator(gpu_device).manual_seed(5)
+    mk = lambda *s, scale=1.0: scale * torch.randn(*s, generator=g, device=gpu_device)  # noqa: E731
+    x, dout, router, norm_w = mk(t, d), mk(t, d), mk(d, e, scale=0.3), mk(d)
+    ws = [mk(e * d, f, scale=0.05), mk(e * d, f, scale=0.05), mk(e * f, d, scale=0.05)]
+    sh = [mk(f, d, scale=0.05), mk(f, d, scale=0.05), mk(d, f, scale=0.05)]
+    cfg = dict(num_experts=e, top_k=k, tile_m=16, score_fn=_abi.SCORE_SOFTMAX, renormalize=False, scale_input=False,
+               router_bias=None, norm_eps=None)
+    _, saved = A.layer_forward(x, None, router, *ws, *sh, None, cfg)
+    assert len(saved) == 1, "the whole pass in one library call"
+    call = {
+        "normalised rows": lambda: [_abi.forward(x, router, None, *ws, e, k, shared=tuple(sh), score_fn=_abi.SCORE_SOFTMAX,
+                                                 scale_input=False, norm=(norm_w, 1e-6))],
+        "training forward": lambda: [A.layer_forward(x, None, router, *ws, *sh, None, cfg)[0]],
+        "training backward": lambda: list(A.layer_backward(x, router, *ws, *sh, None, cfg, saved, dout,
+                                                           (True,) * 8 + (False,)))[:8],
+    }[what]
+    if what == "training backward":
+        assert sum(name.startswith("split_sum_kernel") for name in launched(call)) == 2
+    want, outs, stream = call(), [], torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):  # memory for the capture
+        call()
+    graph, nodes, edges = recorded(stream, lambda: outs.extend(call()))
+    assert len({b for _, b in edges}) < len(edges)
+    hip, runs = hip_runtime(), ctypes.c_void_p()
+    assert hip.hipGraphInstantiate(ctypes.byref(runs), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        for out in outs:
+            out.zero_()
+        torch.cuda.synchronize()
+        assert hip.hipGraphLaunch(runs, ctypes.c_void_p(stream.cuda_stream)) == 0
+        stream.synchronize()
+        assert all(torch.equal(out, right) for out, right in zip(outs, want))
+    assert hip.hipGraphExecDestroy(runs) == 0 and hip.hipGraphDestroy(graph) == 0
+
+
 @pytest.mark.skip(reason="ended in a segmentation fault in hipStreamEndCapture when both streams had forked to the library's "
                   "stream; the second one no longer does, but the fault's cause has not been shown")
 def test_streams_of_one_capture_with_branches_stay_independent(gpu_device):
