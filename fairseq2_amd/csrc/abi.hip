@@ -117,26 +117,26 @@ extern "C" int64_t fs2moe_forward_norm_workspace_bytes(int32_t T, int32_t D, int
 namespace fs2moe {
 
 // Streams of the library's own, two per device: one for callers' streams that run their work, one for those that capture
-// it, so that a capture never finds another thread's work on the stream.  Default priority, created on the first use on a
-// device and kept.  Callers' streams that are independent stay so: what a side stream waits for, everything behind it on
-// that stream waits for too, so a caller's stream gets it only where nothing of another one's is left on it, and a call has
-// it for itself from its branch's beginning to its end; another's shared expert then runs on its own stream.  (Handed to
-// whoever came next: of 7 and 9 pairs of streams that one did not have to wait for the other on, no call on one ended before
-// a call queued on the other, which was held up for 40 ms; now on 6 and 6, the side stream being in one queue of the hardware
-// with the others.)
+// it, so that a capture never finds another thread's work on the stream.  Default priority, created on the first use of its
+// kind on a device and kept (a process with three streams, the caller's among them, runs 5 tokens of D 5120, F 8192, 16
+// experts and a shared one in 323.5 us, one with two or four in 320.5: none is there that is not used).
+// Callers' streams that are independent stay so: what a side stream waits for, everything behind it on that stream waits
+// for too, so a caller's stream gets it only where nothing of another one's is left on it, and a call has it for itself from
+// its branch's beginning to its end; another's shared expert then runs on its own stream.  (Handed to whoever came next: of 7
+// and 9 pairs of streams that one did not have to wait for the other on, no call on one ended before a call queued on the
+// other, which was held up for 40 ms; now on 6 and 6, the side stream being in one queue of the hardware with the others.)
 struct SideStream {
   hipStream_t stream = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
   // the caller's stream of the last branch, whose order covers all that is on this one; where its handle is another
   // stream's by now, a branch of that one may wait for what the destroyed one had left to do
   hipStream_t owner = nullptr;
-  bool taken = false;
+  bool taken = false, tried = false;
 };
 namespace {
 constexpr int kSideDevices = 64;
 struct SideStreams {
   SideStream of[2];
-  bool tried = false;
 };
 SideStreams g_side[kSideDevices];
 std::mutex g_side_mu;
@@ -149,16 +149,28 @@ unsigned long long capture_of(hipStream_t stream) {
   return status == hipStreamCaptureStatusNone ? 0 : id;
 }
 
-// Whether all work of a stream is done.  (Asked for in the relaxed mode: another thread's capture may forbid it.)
-bool idle(hipStream_t stream) {
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
+// This thread's calls in the relaxed mode of capturing: a capture, its own or another thread's, may forbid them else.
+class Relaxed {
+ public:
+  Relaxed() : set_(hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess) {
+    if (!set_) (void)hipGetLastError();
   }
+  Relaxed(const Relaxed&) = delete;
+  Relaxed& operator=(const Relaxed&) = delete;
+  ~Relaxed() {
+    if (set_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+  }
+
+ private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+  const bool set_;
+};
+
+// Whether all work of a stream is done.
+bool idle(hipStream_t stream) {
+  const Relaxed relaxed;
   const bool done = hipStreamQuery(stream) == hipSuccess;
   if (!done) (void)hipGetLastError();
-  (void)hipThreadExchangeStreamCaptureMode(&mode);
   return done;
 }
 
@@ -178,18 +190,20 @@ SideStream* take_side_stream(hipStream_t main) {
   const bool captures = status != hipStreamCaptureStatusNone;
   std::lock_guard<std::mutex> lock(g_side_mu);
   SideStreams& s = g_side[dev];
-  if (!s.tried) {
-    s.tried = true;
-    for (SideStream& side : s.of)
-      if (hipStreamCreateWithFlags(&side.stream, hipStreamNonBlocking) != hipSuccess ||
-          hipEventCreateWithFlags(&side.fork, hipEventDisableTiming) != hipSuccess ||
-          hipEventCreateWithFlags(&side.join, hipEventDisableTiming) != hipSuccess) {
-        (void)hipGetLastError();  // the failure is handled here: nothing for the next call to find
-        side.stream = nullptr;
-      }
-  }
   SideStream& side = s.of[captures ? 1 : 0];
-  if (side.stream == nullptr || side.taken || s.of[0].stream == main || s.of[1].stream == main) return nullptr;
+  if (!side.tried) {
+    const Relaxed relaxed;
+    side.tried = true;
+    if (hipStreamCreateWithFlags(&side.stream, hipStreamNonBlocking) != hipSuccess ||
+        hipEventCreateWithFlags(&side.fork, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&side.join, hipEventDisableTiming) != hipSuccess) {
+      (void)hipGetLastError();  // the failure is handled here: nothing for the next call to find
+      side.stream = nullptr;
+    }
+  }
+  if (side.stream == nullptr || side.taken) return nullptr;
+  for (const SideStream& one : s.of)  // (one that is not there is no caller's null stream)
+    if (one.stream != nullptr && one.stream == main) return nullptr;
   if (captures) {
     // (a stream that a capture has forked to stays part of it until that capture ends, and another stream of the same
     // capture is a chain of nodes of its own)
