@@ -1078,8 +1078,8 @@ def forward(
         raise ValueError("out_shape must be a shape of x's elements")
     mat, score_fn = router_operand(lib, x, router, router_t, score_fn)
     # Collected on every call, in as few steps as checking each tensor once allows: a one-token step of a
-    # layer of 128 experts takes the host 32 us with its five launches, whatever the call before it was (47 us
-    # with a detached view of every parameter and each check in passes of its own; the GPU takes 34).
+    # layer of 128 experts takes the host 30 us with its four launches, whatever the call before it was (47 us
+    # with a detached view of every parameter and each check in passes of its own; the GPU takes as long).
     # (fields in the order of ForwardArgs)
     a = ForwardArgs(
         *sizes, act_dtype, act_dtype if scales is None else FP8_E4M3 | (ACT_MXFP8 if act_quant else 0), score_fn,

@@ -45,9 +45,9 @@ namespace fs2moe {
 //     common level: each XCD gets a share as large as its blocks' room, and its blocks take the share's tiles in turn, each
 //     from the round on that its large tiles last to.  As a share of neighbours for each block, a block for itself, every
 //     tile read its operands from memory: 4096 tokens, top-8 of 128, 2048 x 768, evenly loaded with the router's gradient
-//     2.37 GB for 2.42 that the tiles take in, now 0.55.  us of that training step 1552 -> 1517, by a popularity law 1594
-//     -> 1541; 8192 tokens 2444 -> 2355 and 2516 -> 2416; 2000, top-6 of 32 by a law with a shared expert, 1600 x 1000
-//     813 -> 795.  Sorted only where experts have large tiles: in the gradients' order two operands share L2, not six.
+//     2.37 GB for 2.42 that the tiles take in, now 0.55 (FETCH_SIZE 1.18 and 0.27, which counts requests of 128 bytes as
+//     64), the launch under that counter 556 -> 523 us.  us of that training step with a norm 1581 -> 1549, by a popularity
+//     law 1670 -> 1632; 8192 tokens 2526 -> 2444 and 2618 -> 2561.  Sorted only where experts have large tiles: in the gradients' order two operands share L2, not six.
 // The chunks of a block's tiles form one stream: while the consumers write a tile out, the producers have
 // the next one's first three chunks on their way.  (A block per tile, started by the hardware, paid about
 // 10 us around its chunks.)
