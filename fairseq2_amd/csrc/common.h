@@ -329,10 +329,10 @@ bool swiglu_train_applies(int32_t dtype, int32_t D, int32_t F, int64_t rows);
 int swiglu_train(const void* x, const int32_t* row_map, const int32_t* counts, const int32_t* offsets, int32_t E,
                  const void* w_gate, const void* w_up, const void* w_down, int32_t D, int32_t F,
                  int64_t rows, int64_t planned, int32_t dtype, void* g, void* u, void* h, void* y, void* stream);
-// Work beside the caller's stream: from fork() on what is given to stream() runs on a stream of the library's own, and
-// join() has the caller's wait for it, so that a caller sees one stream's worth of ordering (and a capturing stream
-// captures both branches).  Where `wanted` is false, or there is no such stream to have without ordering callers' streams,
-// stream() is the caller's and the other two do nothing: which it is, beside() says from the beginning, so that it decides
+// Work beside the caller's stream: from fork() on what is given to stream() runs on a stream of the library's own, behind
+// what the caller's had at mark() (or, without one, at fork()), and join() has the caller's wait for it, so that a caller sees one stream's worth of
+// ordering (and a capturing stream captures both branches).  Where `wanted` is false, or there is no such stream to have without ordering callers' streams,
+// stream() is the caller's and the other three do nothing: which it is, beside() says from the beginning, so that it decides
 // where in the order of calls the branch's work stands.  A branch that is forked is joined on every way out.
 class Branch {
  public:
@@ -342,13 +342,14 @@ class Branch {
   ~Branch();
   bool beside() const { return side_ != nullptr; }
   void* stream() const;
+  int mark();
   int fork();
   int join();
 
  private:
   struct SideStream* side_ = nullptr;
   void* main_;
-  bool forked_ = false;
+  bool marked_ = false, forked_ = false;
 };
 // Whether more than 16 tokens' shared expert pays as a branch beside the routed experts.  What it gains is the ends of the
 // other's launches, where CUs run out of tiles, and its small ones: 2 to 10 % of a call.  What it costs is the host's time
@@ -368,9 +369,10 @@ class Branch {
 // and the forward pass of a training step, whose host time is not hidden in a first pass or where a program waits:
 //   508, 496, but as a first pass 620, 665 (129: the 3001 tokens above); 775, 764 and 862, 903 (267: 1800, D 2048, F 2048,
 //   top-2 of 16); 493, 489 and 617, 705 (152: 900, D 1536, F 3072, top-2 of 8); 495, 467 and 596, 621 (149: 263 of f32)
-// Time with the branch over time without it in 70 drawn calls, queued behind others, then with the host waiting for each: where the rule says yes, forward 17 calls 0.96 (0.91 to 1.02), 1.00 (0.93 to 1.07: the host's part is in front
-// of the routed path's first launch), behind a router that normalises 6 0.96 (0.90 to 1.00), 0.97; training steps 18 0.98
-// (0.93 to 1.03), 0.97; where it says no and the branch was forced, 5 1.27, 1.08; 13 1.06, 1.02; 11 1.17, 1.09.
+// Time with the branch over time without it in 70 drawn calls, queued behind others, then with the host waiting for each:
+// where the rule says yes, forward 17 calls 0.96 (0.91 to 1.01), 0.97 (0.91 to 1.02), behind a router that normalises 6 0.96
+// (0.91 to 0.99), 0.96; training steps 18 0.98 (0.93 to 1.03), 0.97 (0.92 to 1.02).  Where it says no and a branch was
+// forced, in front of the router: 5 1.27, 1.08; 13 1.06, 1.02; 11 1.17, 1.09.
 bool branch_pays(int T, int K, int E, int D, int F, int F_shared, int act_dtype, int w_dtype, bool late, bool backward);
 // Into how many parts the sum over K of a product of `sources` pairs of matrices goes (1: it stays whole), by the
 // planned rows (E 0: the rows).

@@ -808,6 +808,16 @@ def test_branches_leave_callers_streams_independent(gpu_device, t, d, f, dtype):
     assert apart and beside
 
 
+@pytest.mark.parametrize("t,d,f,dtype", [(400, 768, 2048, torch.float32), (4, 4096, 8192, torch.bfloat16)])
+def test_a_call_with_a_branch_begins_with_the_router(gpu_device, t, d, f, dtype):
+    """Also where the branch may begin beside it: what the host does for the branch is not what an idle GPU waits for."""
+    _say("begins with the router", t, d, f, dtype)
+    x, call = _layer_with_a_branch(gpu_device, t, d, f, dtype)
+    call(x)
+    names = launched(lambda: call(x))
+    assert names[0].startswith("router"), names
+
+
 @pytest.mark.parametrize("what", ["normalised rows", "training forward", "training backward"])
 def test_calls_that_have_a_branch(gpu_device, what):
     """The passes for which the rule says so fork (a node of a graph of one waits for two others), and have the same bits
